@@ -55,11 +55,10 @@ struct Knobs {
     int lds_min_wgs = 128;
     int lds_min_groups = 8;
     // layered models (tiled_gemm.hip, latent_attention.hip, grouped_attention.hip, linear_attention.hip, rglru.hip)
-    int tiled_big_min_tiles = 64;     // 16-bit projections of > 64 rows take the 128 × 128 tile kernel from this many tiles
-    int tiled_wide_min_tiles = 192;   // … and its 256 × 256 form from this many of those tiles
-    int tiled_wide_min_k = 512;       // … and this many columns of input
+    int tiled_big_min_tiles = 128;    // 16-bit projections of > 64 rows take the tile kernel from this many tiles of 64 × 64
+    int tiled_wide_min_tiles = 257;   // … and its 128 × 256 form from this many tiles of that size
     int tiled_min_tiles = 128;        // few-row kernel: 16-row tiles until there are this many row × 16-column tiles
-    int tiled_half_max_tiles = 128;   // … its 64 × 128 form up to this many tiles of 128 × 128
+    int tiled_half_max_tiles = 255;   // … its 128 × 64 and 64 × 64 forms up to this many tiles of 128 × 128
     int moe_rows_block = 0;           // > 0: forced rows per block of the sorted expert rows
     int tiled_nw = 0, tiled_kw = 0, tiled_j = 0;      // > 0: forced waves per workgroup, K parts, 16-column tiles per wave of the few-row kernel
     int layer_overlap_max_tokens = 64;   // parallel blocks: experts on a stream of their own beside the mixer up to this many tokens (0 = never)
@@ -132,8 +131,8 @@ enum Form : int {
     FORM_CHAIN_QKV_WIDE,        // decode chain with 128-column q|k|v blocks (the narrow ones + attention exceed the resident workgroups)
     FORM_ROUTE_GEMM_TOPK,       // prefill router: logits (MFMA) + softmax + top-k in one launch (moe_route_gemm_topk_kernel)
     FORM_TILED_GEMM,            // layered models: projection with K split over the waves of a workgroup
-    FORM_TILED_GEMM_BIG,        // … 128 × 128 tiles, operands copied to LDS as fragments
-    FORM_TILED_GEMM_256,        // … 256 × 256 tiles
+    FORM_TILED_GEMM_BIG,        // … tiles of up to 128 × 256, operands copied to LDS
+    FORM_TILED_GEMM_256,        // … 128 × 256 tiles
     FORM_TILED_GEMM_GROUPED,    // … rows sorted by expert
     FORM_TILED_GEMM_GROUPED_BIG,
     FORM_MOE_ROUTE_SORT,        // … router's top-k and the sorted rows in one workgroup

@@ -610,7 +610,7 @@ private:
     static int moe_block(int pairs, int experts) {
         const int mean = pairs / experts, forced = knobs().moe_rows_block;
         if (forced > 0 && (sizeof(E) == 2 || forced <= 64)) return forced;
-        if (sizeof(E) == 2 && mean >= 48) return mean >= 384 ? 256 : 128;
+        if (sizeof(E) == 2 && mean >= 48) return 128;
         return mean >= 32 ? 64 : mean >= 12 ? 32 : 16;
     }
 

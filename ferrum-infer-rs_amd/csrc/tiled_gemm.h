@@ -13,6 +13,8 @@ namespace fh {
 typedef __bf16 bf16;
 typedef bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef float floatx8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
@@ -20,7 +22,13 @@ typedef short shortx4 __attribute__((ext_vector_type(4)));
 template <typename E> struct Frag;
 template <> struct Frag<bf16> {
     typedef bf16x8 v8;
+    typedef bf16x4 v4;
     static __device__ __forceinline__ floatx4 mma(v8 a, v8 b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+};
+template <> struct Frag<_Float16> {
+    typedef f16x8 v8;
+    typedef f16x4 v4;
+    static __device__ __forceinline__ floatx4 mma(v8 a, v8 b, floatx4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 };
 template <> struct Frag<float> {
     typedef floatx8 v8;
@@ -100,6 +108,7 @@ template <> struct ActMath<bf16> {
         return added > 0.f ? __logf(u) * (e * __builtin_amdgcn_rcpf(added)) : e;
     }
 };
+template <> struct ActMath<_Float16> : ActMath<bf16> {};
 template <typename E>
 __device__ __forceinline__ float gelu_tanh_f32(float z) {
     return 0.5f * z * (1.0f + ActMath<E>::tanh(0.7978845608028654f * (z + 0.044715f * z * z * z)));

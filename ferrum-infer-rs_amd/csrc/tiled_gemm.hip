@@ -1,7 +1,8 @@
 // Dense projections of the layered models (tiled_gemm.h): one kernel for few rows (K split over the waves of a workgroup, summed in
-// LDS, no second launch) and one for prompts (128 × 128 tiles, both operands copied to LDS as fragments by the load unit itself).
+// LDS, no second launch) and one for prompts (tiles of up to 128 × 256, both operands copied to LDS by the load unit itself).
 // Every activation, bias and per-row factor of a projection is applied to the fp32 accumulator in the epilogue.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 #include "knobs.h"
@@ -207,22 +208,25 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(TiledGemm<E> p, int kw)
     }
 }
 
-// Prompts, 16-bit: WM × WN waves hold MI × NJ tiles of 16 × 16 each, 64 of K per stage, a ring of S stages.  A fragment (16 rows × 32 of K, or 16
-// columns × 32 of K) is one 1-KiB load straight into LDS in lane order, read back as one conflict-free ds_read_b128.
-__device__ const bf16 zero_fragment[512] = {};
-template <int WM, int WN, int MI, int NJ, int S>
+// Prompts, 16-bit: 2 × 2 waves hold MI × NJ tiles of 16 × 16 each.  Both operands go through LDS, copied there by the load unit itself:
+//  * weights in stages of 32 of K, a ring of 2G − 1; a fragment (16 columns × 32 of K) is one 1-KiB load in lane order;
+//  * rows in granules of 64 of K, a ring of G; a load takes 128 bytes (a cache line) of each of 8 rows, and the 16-byte pieces of row r lie in
+//    the order 0 … 7 xor r, so that the 16 lanes that read one piece of 16 rows touch every bank alike.
+__device__ const uint16_t zero_fragment[512] = {};
+template <int MI, int NJ, int G>
 struct BigTile {
-    static constexpr int WAVES = WM * WN, RT = WM * MI, CT = WN * NJ, ROWS = 16 * RT, COLS = 16 * CT, FRAGS = 2 * (RT + CT);
-    static constexpr size_t LDS = (size_t)S * FRAGS * 1024;
-    static_assert(RT % WAVES == 0 && CT % WAVES == 0 && MI % 2 == 0 && NJ == 4, "every wave copies whole tiles");
-    static_assert(LDS >= (size_t)WAVES * 32 * 68 * 4, "the epilogue's rows fit the stages");
+    static constexpr int RT = 2 * MI, CT = 2 * NJ, ROWS = 16 * RT, COLS = 16 * CT, STAGES = 2 * G - 1;
+    static constexpr int GRANULE = RT * 1024, STAGE = CT * 512;         // elements
+    static constexpr size_t LDS = ((size_t)G * GRANULE + STAGES * STAGE) * 2;
+    static_assert(MI % 2 == 0 && (NJ == 2 || NJ == 4 || NJ == 8), "every wave copies whole fragments");
+    static_assert(LDS >= (size_t)4 * 32 * (16 * NJ + 4) * 4, "the epilogue's rows fit the stages");
 };
-template <int WM, int WN, int MI, int NJ, int S>
-__global__ __launch_bounds__(64 * WM * WN, 2) void tiled_gemm_big_kernel(TiledGemm<bf16> p, int mtiles, int ntiles) {
-    typedef BigTile<WM, WN, MI, NJ, S> T;
+template <typename E, int MI, int NJ, int G, int PER_CU>
+__global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E> p, int mtiles, int ntiles) {
+    typedef BigTile<MI, NJ, G> T;
+    typedef typename Frag<E>::v8 v8;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    bf16* lds = reinterpret_cast<bf16*>(smem);                          // per stage: A fragments, then B fragments
-    constexpr int STAGE = T::FRAGS * 512, AT = T::RT / T::WAVES, BT = T::CT / T::WAVES;
+    E *const rows_lds = reinterpret_cast<E*>(smem), *const w_lds = rows_lds + G * T::GRANULE;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
     // workgroups go round-robin over 8 XCDs: give each XCD a contiguous run of tiles, and walk 8 row tiles per column tile
@@ -231,30 +235,33 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void tiled_gemm_big_kernel(TiledGe
     if (l >= total) return;
     const int q8 = total / 8, r8 = total % 8, xcd = l % 8;
     const int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + l / 8;
-    const int band = id / (8 * ntiles), rows_in = min(8, mtiles - band * 8), in = id - band * 8 * ntiles;
-    const int mt = band * 8 + in % rows_in, m0 = mt * T::ROWS, n0 = (in / rows_in) * T::COLS;
-    const int ksteps = p.k >> 5, ntl = p.n >> 4, g = p.rows.id ? p.rows.group[mt] : blockIdx.z;
-    const int wm = wave / WN, wn = wave % WN;
-    // this wave's fragments of a stage: AT row tiles and BT column tiles, two k-steps each
-    const bf16 *ap[AT], *bp[BT];
+    const int band = id / (8 * ntiles), rows_in = min(8, mtiles - band * 8), in_band = id - band * 8 * ntiles;
+    const int mt = band * 8 + in_band % rows_in, m0 = mt * T::ROWS, n0 = (in_band / rows_in) * T::COLS;
+    const int n = p.k >> 5, ntl = p.n >> 4, g = p.rows.id ? p.rows.group[m0 / p.rows.block] : blockIdx.z;
+    const int wm = wave >> 1, wn = wave & 1;
+    // this wave's loads: MI of a granule (8 rows each), NJ / 2 of a weight stage
+    const E *ap[MI], *bp[NJ / 2];
+    const int piece = (lane & 7) ^ (lane >> 3);
 #pragma unroll
-    for (int i = 0; i < AT; i++) ap[i] = gemm_row(p, (m0 >> 4) + AT * wave + i, g, a, b);
-#pragma unroll
-    for (int i = 0; i < BT; i++) {
-        const int t = (n0 >> 4) + BT * wave + i;
-        bp[i] = p.w + ((long)g * ntl + (t < ntl ? t : ntl - 1)) * ksteps * 512 + lane * 8;
+    for (int i = 0; i < MI; i++) {
+        const int r = (MI * wave + i) * 8 + (lane >> 3);
+        ap[i] = gemm_row(p, (m0 + r) >> 4, g, piece, r & 15);
     }
-    const int xs = gemm_row_step(p);
+#pragma unroll
+    for (int i = 0; i < NJ / 2; i++) {
+        const int t = (n0 >> 4) + NJ / 2 * wave + i;
+        bp[i] = p.w + ((long)g * ntl + (t < ntl ? t : ntl - 1)) * n * 512 + lane * 8;
+    }
+    const int xs = 2 * gemm_row_step(p);
+    const E* none = reinterpret_cast<const E*>(zero_fragment) + lane * 8;        // (past the end of K)
 #define BIG_COPY(src, dst) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src), (__attribute__((address_space(3))) void*)(dst), 16, 0, 0)
-    auto issue = [&](int st, int ks) {
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const int kk = ks + h < ksteps ? ks + h : ksteps - 1;         // (past the end of an odd count: rows of zeros)
-#pragma unroll
-            for (int i = 0; i < AT; i++) BIG_COPY(ks + h < ksteps ? ap[i] + (long)kk * xs : zero_fragment + lane * 8, lds + st * STAGE + ((AT * wave + i) * 2 + h) * 512);
-#pragma unroll
-            for (int i = 0; i < BT; i++) BIG_COPY(bp[i] + (long)kk * 512, lds + st * STAGE + ((T::RT + BT * wave + i) * 2 + h) * 512);
-        }
+    auto issue_rows = [&](int i, int place, bool in) {
+        BIG_COPY(in ? ap[i] : none, rows_lds + place * T::GRANULE + (MI * wave + i) * 512);
+        ap[i] += xs;
+    };
+    auto issue_w = [&](int i, int place, bool in) {
+        BIG_COPY(in ? bp[i] : none, w_lds + place * T::STAGE + (NJ / 2 * wave + i) * 512);
+        bp[i] += 512;
     };
 #undef BIG_COPY
     floatx4 acc[MI][NJ];
@@ -262,47 +269,80 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void tiled_gemm_big_kernel(TiledGe
     for (int i = 0; i < MI; i++)
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    struct Operands { v8 x[MI], w[NJ]; };
+    constexpr int READS = MI + NJ;
+    const E* my_w = w_lds + wn * NJ * 512 + lane * 8;
+    const E* my_rows[2];
 #pragma unroll
-    for (int i = 0; i < S - 1; i++)
-        if (2 * i < ksteps) issue(i, 2 * i);
-    auto multiply = [&](const bf16* la, const bf16* lb, int h) {
-        bf16x8 af[MI], bf[NJ];
-#pragma unroll
-        for (int j = 0; j < NJ; j++) bf[j] = *reinterpret_cast<const bf16x8*>(lb + (j * 2 + h) * 512);
-#pragma unroll
-        for (int i = 0; i < MI; i++) af[i] = *reinterpret_cast<const bf16x8*>(la + (i * 2 + h) * 512);
-#pragma unroll
-        for (int i = 0; i < MI; i++)
-#pragma unroll
-            for (int j = 0; j < NJ; j++) acc[i][j] = Frag<bf16>::mma(af[i], bf[j], acc[i][j]);
+    for (int h = 0; h < 2; h++) my_rows[h] = rows_lds + wm * MI * 1024 + b * 64 + ((4 * h + a) ^ (b & 7)) * 8;
+    // fragment f of a k-step: half h of the granule at `gran`, the weight stage at `stage`
+    auto read = [&](Operands& o, int f, int h, int gran, int stage) {
+        if (f < NJ) o.w[f] = *reinterpret_cast<const v8*>(my_w + stage * T::STAGE + f * 512);
+        else o.x[f - NJ] = *reinterpret_cast<const v8*>(my_rows[h] + gran * T::GRANULE + (f - NJ) * 1024);
     };
-    int st = 0;
-    for (int ks = 0; ks < ksteps; ks += 2) {
-        // this stage has arrived (the S − 2 after it may be on their way) and every wave is done with the one before it, whose place the
-        // next request takes
-        if (S > 2 && ks + 2 * (S - 2) < ksteps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * 2 * (AT + BT)) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        if (ks + 2 * (S - 1) < ksteps) issue(st ? st - 1 : S - 1, ks + 2 * (S - 1));
-        const bf16 *la = lds + st * STAGE + wm * MI * 1024 + lane * 8, *lb = lds + st * STAGE + (T::RT + wn * NJ) * 1024 + lane * 8;
-        multiply(la, lb, 0);
-        multiply(la, lb, 1);
-        // operands a few MFMAs ahead of their use
-        constexpr int AHEAD = NJ + 2, LEFT = 2 * (MI + NJ) - AHEAD, PER = 2 * MI * NJ / (LEFT + 2);
-        __builtin_amdgcn_sched_group_barrier(0x100, AHEAD, 0);
+    // every load but this wave's last `left` has arrived, for all waves
+#define BIG_WAIT(left)                                                          \
+    do {                                                                        \
+        constexpr int vm = (left);                                              \
+        asm volatile("" ::: "memory");                                          \
+        __builtin_amdgcn_s_waitcnt((vm & 15) | 0x70 | (vm >> 4) << 14);         \
+        __builtin_amdgcn_s_barrier();                                           \
+        asm volatile("" ::: "memory");                                          \
+        __builtin_amdgcn_sched_barrier(0);                                      \
+    } while (0)
+    // Step t multiplies the operands that step t − 1 read and meanwhile reads those of t + 1.  At its start all that was requested up to step
+    // t − (2G − 2) has arrived: weight stage t + 1, and the granule of t + 1.  Stage t is free then, its operands being in registers, and
+    // t + 2G − 1 takes its place; so is, at odd t, the granule of t.  The weights are the first operand: a lane holds four neighbouring columns
+    // of one row.
+    auto stage_after = [](int i) { return i + 1 < T::STAGES ? i + 1 : 0; };
+    auto granule_after = [](int i) { return i + 1 < G ? i + 1 : 0; };
+    auto step = [&](const Operands& now, Operands& then, auto odd, int t, int stage, int gran) {
+        constexpr bool ODD = decltype(odd)::value;
+        constexpr int LOADS = NJ / 2 + (ODD ? MI : 0), PER = MI * NJ / (READS + READS / 4);
+        BIG_WAIT((T::STAGES - 2) * (NJ / 2) + (ODD ? G - 2 : G - 1) * MI);
+        const bool in = t + T::STAGES < n, rows_in_k = 32 * (t + T::STAGES) + 8 * piece < p.k;
+        const int to = stage_after(stage), from = ODD ? granule_after(gran) : gran;
 #pragma unroll
-        for (int i = 0; i < LEFT; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, PER, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        for (int q = 0; q <= READS; q++) {
+            if (q < READS) read(then, q, ODD ? 0 : 1, from, to);
+            if (q < NJ / 2) issue_w(q, stage, in);
+            else if (ODD && q < LOADS) issue_rows(q - NJ / 2, gran, rows_in_k);
+#pragma unroll
+            for (int m = q * PER; m < (q < READS ? (q + 1) * PER : MI * NJ); m++) acc[m / NJ][m % NJ] = Frag<E>::mma(now.w[m % NJ], now.x[m / NJ], acc[m / NJ][m % NJ]);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, 2 * MI * NJ - LEFT * PER, 0);
-        st = st + 1 < S ? st + 1 : 0;
+    };
+    // (as the steps before the first would have requested it)
+#pragma unroll
+    for (int i = 0; i < T::STAGES; i++) {
+#pragma unroll
+        for (int f = 0; f < NJ / 2; f++) issue_w(f, i, i < n);
+        if (i % 2 == 0) {
+#pragma unroll
+            for (int f = 0; f < MI; f++) issue_rows(f, i / 2, 32 * i + 8 * piece < p.k);
+        }
     }
-    __syncthreads();
+    Operands even, odd;
+    BIG_WAIT((T::STAGES - 1) * (NJ / 2) + (G - 1) * MI);
+#pragma unroll
+    for (int f = 0; f < READS; f++) read(even, f, 0, 0, 0);
+    int stage = 0, gran = 0;
+    for (int t = 0; t < n; t += 2) {
+        step(even, odd, std::false_type{}, t, stage, gran);
+        stage = stage_after(stage);
+        step(odd, even, std::true_type{}, t + 1, stage, gran);
+        stage = stage_after(stage);
+        gran = granule_after(gran);
+    }
+#undef BIG_WAIT
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                    // (the requests past the end have landed: the epilogue reuses the ring)
     // epilogue: 32 rows of a wave's accumulators at a time through LDS (the stages are free, the rows its own, LDS operations of a wave
     // complete in order), then a lane finishes 8 columns of a row: bias, activation and factors, and rows leave in 16-byte pieces.  In a
     // gated section the lanes of the up tiles have nothing to do, those of the gate tiles read both.
-    float* lf = reinterpret_cast<float*>(smem) + wave * 32 * 68;
-    const int cl = (lane & 7) * 8, col = n0 + wn * 64 + cl;
+    __syncthreads();
+    constexpr int LD = 16 * NJ + 4, LANES = 2 * NJ, ROUND = 64 / LANES;          // lanes of a row, rows of a round
+    float* lf = reinterpret_cast<float*>(smem) + wave * 32 * LD;
+    const int cl = (lane % LANES) * 8, col = n0 + wn * 16 * NJ + cl;
     const GemmSection sec = gemm_section(p, min(col, p.n - 1));
     const bool gated = gemm_gated_act(sec.act), vec = p.n_store % 8 == 0 && p.ldo % 8 == 0 && p.out_group % 8 == 0;
     const bool active = gated ? col < p.n && !(col & 16) : col < p.n_store;
@@ -318,23 +358,21 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void tiled_gemm_big_kernel(TiledGe
 #pragma unroll
         for (int i = 0; i < 2; i++)
 #pragma unroll
-            for (int j = 0; j < NJ; j++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) lf[(i * 16 + 4 * a + r) * 68 + j * 16 + b] = acc[2 * ch + i][j][r];
+            for (int j = 0; j < NJ; j++) *reinterpret_cast<floatx4*>(lf + (i * 16 + b) * LD + j * 16 + 4 * a) = acc[2 * ch + i][j];
         const int row0 = m0 + (wm * MI + 2 * ch) * 16;
 #pragma unroll 1
-        for (int q = 0; q < 4; q++) {
-            const int row = q * 8 + (lane >> 3), gr = gemm_out_row(p, row0 + row);
+        for (int q = 0; q < 32 / ROUND; q++) {
+            const int row = q * ROUND + lane / LANES, gr = gemm_out_row(p, row0 + row);
             if (gr < 0 || !active) continue;
             float v[8];
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = lf[row * 68 + cl + e] * sec.mul + bias[e];
+            for (int e = 0; e < 8; e++) v[e] = lf[row * LD + cl + e] * sec.mul + bias[e];
             if (gated) {
 #pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = gemm_glu<bf16>(sec, v[e], lf[row * 68 + cl + 16 + e] * sec.mul + bias_up[e]);
+                for (int e = 0; e < 8; e++) v[e] = gemm_glu<E>(sec, v[e], lf[row * LD + cl + 16 + e] * sec.mul + bias_up[e]);
             } else if (sec.act != GEMM_ACT_NONE) {
 #pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = gemm_act<bf16, true>(sec, v[e]);
+                for (int e = 0; e < 8; e++) v[e] = gemm_act<E, true>(sec, v[e]);
             }
             if (!vec) {
                 for (int e = 0; e < 8; e++)
@@ -347,7 +385,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void tiled_gemm_big_kernel(TiledGe
                 for (int e = 0; e < 8; e++) v[e] *= f;
             }
             if (p.col_scale) {
-                const bf16x8 f = *reinterpret_cast<const bf16x8*>(p.col_scale + p.col_scale_row[gr] * p.ld_col_scale + oc);
+                const v8 f = *reinterpret_cast<const v8*>(p.col_scale + p.col_scale_row[gr] * p.ld_col_scale + oc);
 #pragma unroll
                 for (int e = 0; e < 8; e++) v[e] *= (float)f[e];
             }
@@ -356,42 +394,51 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void tiled_gemm_big_kernel(TiledGe
                 *reinterpret_cast<floatx4*>(p.out_f32 + o) = (floatx4){v[0], v[1], v[2], v[3]};
                 *reinterpret_cast<floatx4*>(p.out_f32 + o + 4) = (floatx4){v[4], v[5], v[6], v[7]};
             } else {
-                bf16x8 y;
+                v8 y;
 #pragma unroll
-                for (int e = 0; e < 8; e++) y[e] = (bf16)v[e];
-                *reinterpret_cast<bf16x8*>(p.out + o) = y;
+                for (int e = 0; e < 8; e++) y[e] = (E)v[e];
+                *reinterpret_cast<v8*>(p.out + o) = y;
             }
         }
     }
 }
 
-template <int WM, int WN, int MI, int NJ, int S>
-static int launch_big(const TiledGemm<bf16>& g, hipStream_t s) {
-    typedef BigTile<WM, WN, MI, NJ, S> T;
+template <typename E, int MI, int NJ, int G, int PER_CU>
+static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
+    typedef BigTile<MI, NJ, G> T;
     static bool attr = false;
     if (!attr) {
-        FH_CHECK_HIP(hipFuncSetAttribute((const void*)tiled_gemm_big_kernel<WM, WN, MI, NJ, S>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::LDS));
+        FH_CHECK_HIP(hipFuncSetAttribute((const void*)tiled_gemm_big_kernel<E, MI, NJ, G, PER_CU>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::LDS));
         attr = true;
     }
-    const int mtiles = g.rows.id ? g.rows.max_blocks : cdiv(g.m, T::ROWS), ntiles = cdiv(g.n, T::COLS);
+    const int mtiles = g.rows.id ? g.rows.max_blocks * (g.rows.block / T::ROWS) : cdiv(g.m, T::ROWS), ntiles = cdiv(g.n, T::COLS);
     form_hit(g.rows.id ? FORM_TILED_GEMM_GROUPED_BIG : FORM_TILED_GEMM_BIG);
-    if (T::ROWS == 256) form_hit(FORM_TILED_GEMM_256);
-    hipLaunchKernelGGL((tiled_gemm_big_kernel<WM, WN, MI, NJ, S>), dim3(mtiles * ntiles, 1, g.groups), dim3(64 * T::WAVES), T::LDS, s, g, mtiles, ntiles);
+    if (T::COLS == 256) form_hit(FORM_TILED_GEMM_256);
+    hipLaunchKernelGGL((tiled_gemm_big_kernel<E, MI, NJ, G, PER_CU>), dim3(mtiles * ntiles, 1, g.groups), dim3(256), T::LDS, s, g, mtiles, ntiles);
     FH_CHECK_LAUNCH();
     return 0;
 }
-static int launch_big(const TiledGemm<bf16>& g, hipStream_t s) {
-    // one 256 × 256 tile per CU, or two of 128 × 128: the large one halves the bytes per product, as long as there are enough of them
-    const long tiles = (long)cdiv(g.m, 256) * cdiv(g.n, 256) * g.groups;
-    // (few stages: the epilogues are most of the work, and two workgroups per CU hide one's behind the other's)
-    const bool wide = g.rows.id ? g.rows.block == 256 : tiles >= knobs().tiled_wide_min_tiles && g.k >= knobs().tiled_wide_min_k;
-    if (wide) return launch_big<2, 4, 8, 4, 2>(g, s);
-    // few tiles: rows in halves so that every CU has one, or one workgroup per CU, and a deeper ring in place of the second workgroup
-    const long tiles128 = (long)cdiv(g.m, 128) * cdiv(g.n, 128) * g.groups;
-    if (!g.rows.id && tiles128 <= knobs().tiled_half_max_tiles) return launch_big<2, 2, 2, 4, 5>(g, s);
-    return !g.rows.id && tiles128 <= 256 ? launch_big<2, 2, 4, 4, 4>(g, s) : launch_big<2, 2, 4, 4, 2>(g, s);
+// Tile sizes, µs of bf16 launches (rows × columns × K):
+//                          128 × 256   128 × 128   128 × 64   64 × 64   before (64 of K a stage, the rows' lines fetched by halves)
+//   8192 × 10240 × 2048        277         326        396        500      322
+//   8192 × 8192 × 8192         831         980       1255       1486      933
+//   4096 × 6144 × 2048          91         104        119        148      119
+//   4002 × 2048 × 2048          39          36         46         55       49
+//   2048 × 4096 × 1024          26          23         28         33       28
+//   256 × 8192 × 2048           34          24         17         19       20
+//   2048 × 1024 × 2048          34          24         16         18       20
+//   300 × 2048 × 2048           34          21         16         12       25
+//   128 × 6144 × 2048           34          21         16         12       28
+// Two workgroups of the largest tile share a CU, so that one's stores run under the other's products; below a tile per CU the smaller tiles
+// cover the chip.  Fewer than half as many tiles as CUs at 64 × 64: the few-row kernel's K split is as fast (128 × 2048 × 2048: 11 and 12 µs).
+template <typename E>
+static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
+    auto tiles = [&](int r, int c) { return (long)(g.rows.id ? g.rows.max_blocks * (g.rows.block / r) : cdiv(g.m, r)) * cdiv(g.n, c) * g.groups; };
+    if (tiles(128, 256) >= knobs().tiled_wide_min_tiles) return launch_big<E, 4, 8, 2, 2>(g, s);
+    if (tiles(128, 128) > knobs().tiled_half_max_tiles) return launch_big<E, 4, 4, 2, 2>(g, s);
+    return tiles(128, 64) > 160 ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 2, 2, 3, 3>(g, s);
 }
-static int launch_big(const TiledGemm<float>&, hipStream_t) { return 2; }      // (never taken: 16-bit only)
+template <> int launch_big<float>(const TiledGemm<float>&, hipStream_t) { return 2; }      // (never taken: 16-bit only)
 
 int tiled_gemm_slabs(int m, int n, int k) {
     if (m > 64) return 1;
@@ -432,8 +479,8 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
                    "tiled_gemm: sorted rows take plain sections");
         FH_REQUIRE(rows.block == 16 || rows.block == 32 || rows.block == 64 || ((rows.block == 128 || rows.block == 256) && sizeof(E) == 2), "tiled_gemm: blocks of %d rows", rows.block);
     }
-    const long tiles = (long)cdiv(g.m, 128) * cdiv(g.n, 128) * g.groups;
-    if (rows.id ? rows.block >= 128 : sizeof(E) == 2 && g.m > 64 && g.n >= 128 && g.slabs == 1 && tiles >= knobs().tiled_big_min_tiles) return launch_big(g, s);
+    const long tiles = (long)cdiv(g.m, 64) * cdiv(g.n, 64) * g.groups;
+    if (rows.id ? rows.block >= 128 : sizeof(E) == 2 && g.m > 64 && g.n >= 64 && g.slabs == 1 && tiles >= knobs().tiled_big_min_tiles) return launch_big(g, s);
     // rows per workgroup: as many as there are, fewer where narrow outputs would leave CUs idle
     int mt = rows.id ? rows.block / 16 : g.m <= 16 ? 1 : (g.m <= 32 ? 2 : 4);
     while (!rows.id && mt > 1 && (long)cdiv(g.m, 16 * mt) * (g.n / 16) * g.groups * g.slabs < knobs().tiled_min_tiles) mt /= 2;

@@ -102,6 +102,20 @@ def test_experts_of_long_prompts(pkg, tmp_path, forms, knobs, block, dtype):
     assert bool(h.get("tiled_gemm_grouped")) == (dtype == "float32" or block <= 64)
 
 
+@pytest.mark.parametrize("wide, half, block", [(1, 0, 128), (1, 0, 256), (10 ** 6, 0, 128), (10 ** 6, 0, 256), (10 ** 6, 10 ** 6, 128), (10 ** 6, 10 ** 6, 256)])
+def test_experts_in_every_tile_size(pkg, tmp_path, forms, knobs, wide, half, block):
+    """Sorted rows in tiles of 256, 128 and 64 columns: an odd and an even number of K steps, fewer of them than the ring holds, blocks that
+    several tiles share, columns past the last tile."""
+    knobs.set(MOE_ROWS_BLOCK=block, TILED_WIDE_MIN_TILES=wide, TILED_HALF_MAX_TILES=half)
+    for n, top, tokens, ff, width in ((4, 2, 400, 48, 160), (9, 3, 110, 70, 320), (6, 1, 75, 250, 96), (3, 2, 300, 33, 32)):
+        cfg = model([G.sink_attention(2, 8, 4, 8, 16, mlp=G.experts(n, top, ff))], width=width)
+        w = G.weights(cfg, 46)
+        silence(w, "mix.o", "side.norm")
+        agree(pkg, tmp_path / f"{n}{ff}", cfg, w, "bfloat16", n=tokens)
+    h = forms.hits()
+    assert h.get("tiled_gemm_grouped_big") and bool(h.get("tiled_gemm_256")) == (wide == 1)
+
+
 def test_experts_beside_the_mixer(pkg, cases, knobs):
     """Small batches run the experts on a stream of their own: the same ids as in one stream, eagerly and over many replays of the graph
     with eager work between them."""
