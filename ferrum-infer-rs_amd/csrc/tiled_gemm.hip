@@ -344,7 +344,7 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     float* lf = reinterpret_cast<float*>(smem) + wave * 32 * LD;
     const int cl = (lane % LANES) * 8, col = n0 + wn * 16 * NJ + cl;
     const GemmSection sec = gemm_section(p, min(col, p.n - 1));
-    const bool gated = gemm_gated_act(sec.act), vec = p.n_store % 8 == 0 && p.ldo % 8 == 0 && p.out_group % 8 == 0;
+    const bool gated = gemm_gated_act(sec.act), vec = p.n_store % 8 == 0 && p.ldo % 8 == 0 && p.out_group % 8 == 0 && ((uintptr_t)p.out & 15) == 0 && ((uintptr_t)p.out_f32 & 15) == 0;
     const bool active = gated ? col < p.n && !(col & 16) : col < p.n_store;
     const int oc = gated ? gemm_gated_col(sec, col) : col;
     float bias[8], bias_up[8];
@@ -504,5 +504,6 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
 }
 template int tiled_gemm<bf16>(const TiledGemm<bf16>&, hipStream_t);
 template int tiled_gemm<float>(const TiledGemm<float>&, hipStream_t);
+template int tiled_gemm<_Float16>(const TiledGemm<_Float16>&, hipStream_t);
 
 }  // namespace fh

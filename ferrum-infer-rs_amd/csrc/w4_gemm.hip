@@ -21,6 +21,7 @@
 #include "kernels.h"
 #include "knobs.h"
 #include "route_merge.h"
+#include "tiled_gemm.h"
 #include "w4_device.h"
 
 namespace fh {
@@ -3155,6 +3156,17 @@ static int f16t_gemm_impl(const __half* x, const __half* wt, OutT* out, int m, i
                           size_t workspace_bytes, hipStream_t stream) {
     if (m <= 0) return 0;
     FH_REQUIRE(k % 32 == 0, "f16t_gemm: K=%d must be a multiple of 32", k);
+    // The projections of the layered models (tiled_gemm.hip) read the same weight tiles: prompts in LDS tiles (2048 × 4096 × 1024: 115 → 24 µs), few
+    // rows with K split over the waves of a workgroup and no reduce launch (8 × 4096 × 1024: 12 → 7 µs).  A wide N at few rows (the lm_head) streams
+    // its weights once either way and stays here, as do N that are no multiple of 32.
+    if (n % 32 == 0 && (m > 64 || n < 32768) && ((uintptr_t)x & 15) == 0) {
+        TiledGemm<_Float16> g;
+        g.x = reinterpret_cast<const _Float16*>(x); g.ldx = k; g.w = reinterpret_cast<const _Float16*>(wt);
+        g.m = m; g.n = n; g.k = k; g.ldo = n;
+        if constexpr (sizeof(OutT) == 2) g.out = reinterpret_cast<_Float16*>(out);
+        else g.out_f32 = out;
+        return tiled_gemm(g, stream);
+    }
     int mt = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
     int row_blocks = cdiv(m, 16 * mt);
     int ntile2 = cdiv(n, 32);

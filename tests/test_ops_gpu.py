@@ -283,6 +283,26 @@ def test_dense_gemm(env, m, n, k, f32out):
     assert nmse(ref, host(out2)) < (1e-10 if f32out else NMSE_FP16_TOL)
 
 
+@pytest.mark.parametrize("f32out", [False, True])
+@pytest.mark.parametrize("m,n,k", [(1, 64, 32), (16, 4096, 1024), (17, 96, 1056), (64, 1024, 3072), (65, 8192, 32), (100, 6176, 96), (200, 2080, 64),
+                                   (129, 16416, 160), (300, 4128, 2080), (1100, 1056, 352), (2049, 4096, 128), (3000, 8224, 64)])
+def test_dense_gemm_tile_edges(env, m, n, k, f32out):
+    """Few rows and every tile size at rows and columns just past a tile, odd and even numbers of 32-column steps, fewer of them than a ring holds;
+    also into a result whose address only takes single elements."""
+    pkg, B, ctx, O, torch = env
+    gen = torch.Generator("cuda").manual_seed(m + n + k)
+    a, b = (torch.randn(r, k, generator=gen, device="cuda").half() for r in (m, n))
+    bt, want = B.dense_repack_f16t(ctx, b, n, k), a.double() @ b.double().T
+    # fp32 sums of exact products in any order, then one rounding to the output's type
+    bound = k * 2.0 ** -24 * (a.double().abs() @ b.double().abs().T) + (2.0 ** -24 if f32out else 2.0 ** -11) * want.abs() + 2.0 ** -24
+    for shift in (0, 1):
+        buf = torch.full((m * n + 64,), 7.0, dtype=torch.float32 if f32out else torch.float16, device="cuda")
+        B.gemm_f16t(ctx, a, bt, buf[shift:shift + m * n], m, n, k)
+        ctx.sync()
+        assert bool(((buf[shift:shift + m * n].view(m, n).double() - want).abs() <= bound).all())
+        assert bool((buf[:shift] == 7.0).all()) and bool((buf[shift + m * n:] == 7.0).all())
+
+
 # ── paged KV write / read ────────────────────────────────────────────────────
 def _rope(O, hd, max_seq, theta=1e6):
     return O.build_rope_cache(theta, hd, max_seq)
