@@ -485,14 +485,29 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     int mt = rows.id ? rows.block / 16 : g.m <= 16 ? 1 : (g.m <= 32 ? 2 : 4);
     while (!rows.id && mt > 1 && (long)cdiv(g.m, 16 * mt) * (g.n / 16) * g.groups * g.slabs < knobs().tiled_min_tiles) mt /= 2;
     const int rbs = rows.id ? rows.max_blocks : cdiv(g.m, 16 * mt), ksteps = g.k / 32, zs = rows.id ? 1 : g.groups * g.slabs;
-    // 32 columns per wave, 16 where 32 would leave CUs without a workgroup; K split over the waves until the launch has enough of them
-    int J = (long)rbs * (g.n / 32) * zs < (g.slabs > 1 ? 256 : g.n <= 96 && g.m > 64 ? 513 : 257) ? 1 : 2;       // (narrow outputs of prompts: two workgroups per CU)
+    // Columns and K parts of a wave, µs (bf16, weights from HBM; four waves a workgroup, K split over kw of them):
+    //                            32 columns      16 columns      before
+    //                            kw 4   kw 2     kw 4   kw 2
+    //   8 × 4096 × 1024           5.2             4.9    5.3     5.6 (16, eight waves, kw 8)
+    //   8 × 6144 × 1024           5.6                    5.6     8.6 (16, eight waves, kw 8)
+    //   8 × 8192 × 2048           8.8                    8.3     10.4 (16, eight waves, kw 8)
+    //   16 × 10240 × 2048        12.7   12.0            14.2     12.8 (32, eight waves, kw 8)
+    //   8 × 1024 × 3072           8.0             6.5            7.4 (16, eight waves, kw 8)
+    //   32 × 8192 × 2048         10.7                   12.4     13.9 (16, four waves, kw 4)
+    //   32 × 2048 × 2048          9.4             8.4            8.4
+    //   60 × 8192 × 2048         17.1                   20.1     20.8
+    // Fewer waves a workgroup wait for each other less.  Several row tiles, whose fragments a wave reads again for every column group: 32 columns
+    // sooner.  Slabs of a long K want every wave they can get (1 × 2048 × 8192 in four: eight waves 8.1, four 8.4).
+    const bool long_slabs = g.slabs > 1 && ksteps / g.slabs >= 64, narrow = sizeof(E) == 4 || long_slabs;
+    int J = narrow ? ((long)rbs * (g.n / 32) * zs < (g.slabs > 1 ? 256 : 257) ? 1 : 2)
+                   : (long)rbs * (g.n / 32) * g.groups < (g.n <= 96 && g.m > 64 ? 513 : mt == 1 ? 257 : 160) ? 1 : 2;
     if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : 2;
     if (gated) J = 2;
     const long cols = g.n / (16 * J);
-    int nw = mt == 1 ? 8 : 4, kw = 1;
+    int nw = mt == 1 && narrow ? 8 : 4, kw = 1;
     if (knobs().tiled_nw > 0) nw = std::min(8, knobs().tiled_nw);
-    while (kw < nw && (long)rbs * cols * zs * kw < (rows.id ? 8192 : 4096) && ksteps >= 8 * kw * g.slabs) kw *= 2;
+    const long enough = rows.id ? 8192 : narrow ? 4096 : J == 1 ? 768 : 4096;
+    while (kw < nw && (long)rbs * cols * zs * kw < enough && ksteps >= 8 * kw * g.slabs) kw *= 2;
     if (knobs().tiled_kw > 0) kw = std::min(nw, knobs().tiled_kw);
     const dim3 grid(cdiv(cols, nw / kw), rbs, zs);
     form_hit(rows.id ? FORM_TILED_GEMM_GROUPED : FORM_TILED_GEMM);
