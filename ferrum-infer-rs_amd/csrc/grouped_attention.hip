@@ -172,25 +172,30 @@ __global__ __launch_bounds__(256) void grouped_attn_plain_kernel(GroupedDims d, 
 constexpr int GROUPED_PARTIAL_PAD = 4;       // floats behind a partial row's outputs: maximum, sum
 typedef short shortx8 __attribute__((ext_vector_type(8)));
 // four elements of a row's result: columns [col, col + 4) of the concatenated heads
-__device__ __forceinline__ void grouped_store4(const GroupedBuffers<bf16>& p, long tok, int col, floatx4 x, float f) {
-    bf16x4 y;
+template <typename E>
+__device__ __forceinline__ void grouped_store4(const GroupedBuffers<E>& p, long tok, int col, floatx4 x, float f) {
+    typedef typename Frag<E>::v4 v4;
+    v4 y;
     if (p.value_gate) {
-        const bf16x4 g = *reinterpret_cast<const bf16x4*>(p.value_gate + tok * p.ld_value_gate + col);
+        const v4 g = *reinterpret_cast<const v4*>(p.value_gate + tok * p.ld_value_gate + col);
 #pragma unroll
-        for (int r = 0; r < 4; r++) y[r] = (bf16)(x[r] * f * (float)g[r]);
+        for (int r = 0; r < 4; r++) y[r] = (E)(x[r] * f * (float)g[r]);
     } else {
 #pragma unroll
-        for (int r = 0; r < 4; r++) y[r] = (bf16)(x[r] * f);
+        for (int r = 0; r < 4; r++) y[r] = (E)(x[r] * f);
     }
-    *reinterpret_cast<bf16x4*>(p.out + tok * p.ldo + col) = y;
+    *reinterpret_cast<v4*>(p.out + tok * p.ldo + col) = y;
 }
 
 // Few rows per sequence.  grid (16-row tiles × KV splits, kv_heads): the four waves take 32-key steps of the range in turn, straight from
-// the cache into registers (the next step is requested before this one is used), and merge through LDS.
+// the cache into registers (the next step is requested before this one is used), and merge through LDS.  32-bit models take it for prompts too: 16
+// (token, head) rows share a read of the cache that the plain form makes for each of them (16 heads of 128 dimensions on 4, a prompt of 1000 tokens
+// and 8 decoded: 3.61 -> 0.20 ms).  One set of operand registers there: keys are requested behind the scores, values behind their product.
 // FAR: scores fall with the logarithm of the distance.
-template <int DS, bool FAR>
-__global__ __launch_bounds__(256) void grouped_attn_keys_kernel(GroupedDims d, GroupedBuffers<bf16> p, BatchView v, int nsplit) {
-    constexpr int DT = 2 * DS, D = 32 * DS, LD = D + 4;
+template <typename E, int DS, bool FAR>
+__global__ __launch_bounds__(256) void grouped_attn_keys_kernel(GroupedDims d, GroupedBuffers<E> p, BatchView v, int nsplit) {
+    typedef typename Frag<E>::v8 v8;
+    constexpr int DT = 2 * DS, D = 32 * DS, LD = D + 4, NB = sizeof(E) == 2 ? 2 : 1;
     extern __shared__ __attribute__((aligned(16))) float lds_o[];              // [4][16][LD]
     __shared__ float lds_m[64], lds_l[64];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, a = lane >> 4, b = lane & 15;
@@ -206,65 +211,78 @@ __global__ __launch_bounds__(256) void grouped_attn_keys_kernel(GroupedDims d, G
     const int blk_lo = max(0, w.pos0 + t_first + 1 - d.window) / 16, blk_hi = (w.pos0 + t_last + 16) / 16, nstep = (blk_hi - blk_lo + 1) / 2;
     const int st_lo = nstep * split / nsplit, st_hi = nstep * (split + 1) / nsplit;
     const int32_t* bt = v.bt + (long)w.seq * v.max_blocks;
-    bf16x8 qf[DS], kf[2][2][DS], vf[2][2][DS];
+    v8 qf[DS], kf[NB][2][DS], vf[NB][2][DS];
     const long kd = (long)d.kv_heads * D * 16, off = (long)kvh * D * 16 + lane * 8;
-    auto load = [&](int buf, int st) {                                         // (past the end: a copy of the last block, masked below)
+    auto load = [&](v8 (&f)[2][DS], const E* pool, int st) {                    // (past the end: a copy of the last block, masked below)
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             const long blk = __builtin_amdgcn_readfirstlane(bt[min(blk_lo + 2 * st + i, blk_hi - 1)]);
 #pragma unroll
-            for (int s = 0; s < DS; s++) {
-                kf[buf][i][s] = *reinterpret_cast<const bf16x8*>(p.k_pool + blk * kd + off + s * 512);
-                vf[buf][i][s] = *reinterpret_cast<const bf16x8*>(p.v_pool + blk * kd + off + s * 512);
-            }
+            for (int s = 0; s < DS; s++) f[i][s] = *reinterpret_cast<const v8*>(pool + blk * kd + off + s * 512);
         }
     };
 #pragma unroll
-    for (int s = 0; s < DS; s++) qf[s] = *reinterpret_cast<const bf16x8*>(p.q + (tok * d.heads + head) * D + 32 * s + 8 * a);
+    for (int s = 0; s < DS; s++) qf[s] = *reinterpret_cast<const v8*>(p.q + (tok * d.heads + head) * D + 32 * s + 8 * a);
     float m_run = -INFINITY, l_run = 0.f;
     floatx4 o[DT];
 #pragma unroll
     for (int t = 0; t < DT; t++) o[t] = (floatx4){0.f, 0.f, 0.f, 0.f};
-    auto step = [&](int buf, int st) {
-        float sc[8], mx = -INFINITY;
+    auto scores = [&](const v8 (&kq)[2][DS], int st, float (&sc)[8]) {
 #pragma unroll
         for (int i = 0; i < 2; i++) {
             floatx4 s2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-            for (int s = 0; s < DS; s++) s2[s & 1] = Frag<bf16>::mma(kf[buf][i][s], qf[s], s2[s & 1]);
+            for (int s = 0; s < DS; s++) s2[s & 1] = Frag<E>::mma(kq[i][s], qf[s], s2[s & 1]);
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int key = (blk_lo + 2 * st + i) * 16 + 4 * a + r;
                 float z = (s2[0][r] + s2[1][r]) * d.scale;
-                if (FAR) z -= r1 * __logf(1.0f + r2 * (float)max(row_pos - key, 0));
+                if (FAR) z -= r1 * (sizeof(E) == 2 ? __logf(1.0f + r2 * (float)max(row_pos - key, 0)) : log1pf(r2 * (float)max(row_pos - key, 0)));
                 sc[4 * i + r] = ok && key <= row_pos && key >= win_lo ? z : -INFINITY;
-                mx = fmaxf(mx, sc[4 * i + r]);
             }
         }
-        const float m_new = fmaxf(m_run, rows_reduce_max(mx)), m_safe = m_new == -INFINITY ? 0.f : m_new, alpha = __expf(m_run - m_safe);
-        bf16x8 pf;
+    };
+    auto weigh = [&](const v8 (&vq)[2][DS], const float (&sc)[8]) {
+        float mx = sc[0];
+#pragma unroll
+        for (int j = 1; j < 8; j++) mx = fmaxf(mx, sc[j]);
+        const float m_new = fmaxf(m_run, rows_reduce_max(mx)), m_safe = m_new == -INFINITY ? 0.f : m_new, alpha = attn_exp<E>(m_run - m_safe);
+        v8 pf;
         float ps = 0.f;
 #pragma unroll
-        for (int j = 0; j < 8; j++) { const float e = __expf(sc[j] - m_safe); ps += e; pf[j] = (bf16)e; }
+        for (int j = 0; j < 8; j++) { const float e = attn_exp<E>(sc[j] - m_safe); ps += e; pf[j] = (E)e; }
         l_run = l_run * alpha + ps;                                            // (this lane's keys; the four lane groups meet at the end)
         m_run = m_new;
 #pragma unroll
         for (int t = 0; t < DT; t++) {
 #pragma unroll
             for (int r = 0; r < 4; r++) o[t][r] *= alpha;
-            o[t] = Frag<bf16>::mma(value_operand(vf[buf][0][t >> 1], vf[buf][1][t >> 1], t & 1), pf, o[t]);
+            o[t] = Frag<E>::mma(value_operand(vq[0][t >> 1], vq[1][t >> 1], t & 1), pf, o[t]);
         }
     };
     if (st_lo + wave < st_hi) {
         int st = st_lo + wave;
-        load(0, st);
+        float sc[8];
+        load(kf[0], p.k_pool, st);
+        load(vf[0], p.v_pool, st);
         while (true) {
-            load(1, st + 4);
-            step(0, st);
-            st += 4;
-            if (st >= st_hi) break;
-            load(0, st + 4);
-            step(1, st);
+            if constexpr (NB == 2) {
+                load(kf[1], p.k_pool, st + 4);
+                load(vf[1], p.v_pool, st + 4);
+                scores(kf[0], st, sc);
+                weigh(vf[0], sc);
+                st += 4;
+                if (st >= st_hi) break;
+                load(kf[0], p.k_pool, st + 4);
+                load(vf[0], p.v_pool, st + 4);
+                scores(kf[1], st, sc);
+                weigh(vf[1], sc);
+            } else {
+                scores(kf[0], st, sc);
+                load(kf[0], p.k_pool, st + 4);
+                weigh(vf[0], sc);
+                load(vf[0], p.v_pool, st + 4);
+            }
             st += 4;
             if (st >= st_hi) break;
         }
@@ -277,8 +295,8 @@ __global__ __launch_bounds__(256) void grouped_attn_keys_kernel(GroupedDims d, G
     for (int i = 0; i < 4; i++) M = fmaxf(M, lds_m[i * 16 + b]);
     const float M_safe = M == -INFINITY ? 0.f : M;
 #pragma unroll
-    for (int i = 0; i < 4; i++) L += lds_l[i * 16 + b] * __expf(lds_m[i * 16 + b] - M_safe);
-    const float f_own = __expf(m_run - M_safe);
+    for (int i = 0; i < 4; i++) L += lds_l[i * 16 + b] * attn_exp<E>(lds_m[i * 16 + b] - M_safe);
+    const float f_own = attn_exp<E>(m_run - M_safe);
 #pragma unroll
     for (int t = 0; t < DT; t++) {
         floatx4 x;
@@ -302,12 +320,13 @@ __global__ __launch_bounds__(256) void grouped_attn_keys_kernel(GroupedDims d, G
             continue;
         }
         const int rt = ro / G, rh = kvh * G + ro % G;
-        const float sink = p.sink ? __expf(p.sink[rh] - lds_m[row]) : 0.f;
+        const float sink = p.sink ? attn_exp<E>(p.sink[rh] - lds_m[row]) : 0.f;
         grouped_store4(p, w.tok0 + rt, rh * D + c, x, grouped_factor(p, lds_l[row] + sink, w.tok0 + rt, rh));
     }
 }
 // grid (tiles, kv_heads): one thread per (row, 4 dimensions)
-__global__ __launch_bounds__(256) void grouped_attn_reduce_kernel(GroupedDims d, GroupedBuffers<bf16> p, BatchView v, int nsplit) {
+template <typename E>
+__global__ __launch_bounds__(256) void grouped_attn_reduce_kernel(GroupedDims d, GroupedBuffers<E> p, BatchView v, int nsplit) {
     const int G = d.heads / d.kv_heads, kvh = blockIdx.y, quads = d.vp / 4;
     SeqTile w;
     if (!find_seq_tile(v, G, 16, blockIdx.x, &w)) return;
@@ -320,12 +339,12 @@ __global__ __launch_bounds__(256) void grouped_attn_reduce_kernel(GroupedDims d,
         for (int z = 0; z < nsplit; z++) M = fmaxf(M, src[z * 16 * ld + d.vp]);
         floatx4 acc = {0.f, 0.f, 0.f, 0.f};
         for (int z = 0; z < nsplit; z++) {
-            const float f = __expf(src[z * 16 * ld + d.vp] - M);
+            const float f = attn_exp<E>(src[z * 16 * ld + d.vp] - M);
             L += src[z * 16 * ld + d.vp + 1] * f;
             acc += *reinterpret_cast<const floatx4*>(src + z * 16 * ld + c) * f;
         }
         const int rt = ro / G, rh = kvh * G + ro % G;
-        if (p.sink) L += __expf(p.sink[rh] - M);
+        if (p.sink) L += attn_exp<E>(p.sink[rh] - M);
         grouped_store4(p, w.tok0 + rt, rh * d.vp + c, acc, grouped_factor(p, L, w.tok0 + rt, rh));
     }
 }
@@ -506,11 +525,11 @@ static int grouped_tile(const GroupedDims& d, const GroupedBuffers<bf16>& b, con
     FH_CHECK_LAUNCH();
     return 0;
 }
-template <int DS, bool FAR>
-static int grouped_keys(const GroupedDims& d, const GroupedBuffers<bf16>& b, const BatchView& v, hipStream_t s) {
+template <int DS, bool FAR, typename E>
+static int grouped_keys(const GroupedDims& d, const GroupedBuffers<E>& b, const BatchView& v, hipStream_t s) {
     constexpr size_t lds = (size_t)64 * (32 * DS + 4) * 4;
     static bool attr = false;
-    if (!attr) { FH_CHECK_HIP(hipFuncSetAttribute((const void*)grouped_attn_keys_kernel<DS, FAR>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); attr = true; }
+    if (!attr) { FH_CHECK_HIP(hipFuncSetAttribute((const void*)grouped_attn_keys_kernel<E, DS, FAR>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); attr = true; }
     const int G = d.heads / d.kv_heads, tiles = v.single ? v.num_seqs * cdiv(G, 16) : (int)((long)v.T * G / 16) + v.num_seqs;
     // split the keys while the launch has fewer workgroups than stay resident and a split keeps ≥ 128 keys
     const int keys = (int)std::min<long>(v.max_keys, (long)d.window + 16);
@@ -519,16 +538,27 @@ static int grouped_keys(const GroupedDims& d, const GroupedBuffers<bf16>& b, con
     if (knobs().grouped_splits > 0) ns = std::min(16, knobs().grouped_splits);
     while (ns > 1 && (size_t)tiles * d.kv_heads * ns * 16 * (d.vp + GROUPED_PARTIAL_PAD) * 4 > b.partial_bytes) ns /= 2;
     form_hit(ns > 1 ? FORM_GROUPED_ATTN_SPLIT : FORM_GROUPED_ATTN_KEYS);
-    hipLaunchKernelGGL((grouped_attn_keys_kernel<DS, FAR>), dim3(tiles * ns, d.kv_heads), dim3(256), lds, s, d, b, v, ns);
+    hipLaunchKernelGGL((grouped_attn_keys_kernel<E, DS, FAR>), dim3(tiles * ns, d.kv_heads), dim3(256), lds, s, d, b, v, ns);
     FH_CHECK_LAUNCH();
     if (ns > 1) {
-        hipLaunchKernelGGL(grouped_attn_reduce_kernel, dim3(tiles, d.kv_heads), dim3(256), 0, s, d, b, v, ns);
+        hipLaunchKernelGGL(grouped_attn_reduce_kernel<E>, dim3(tiles, d.kv_heads), dim3(256), 0, s, d, b, v, ns);
         FH_CHECK_LAUNCH();
     }
     return 0;
 }
 template <> int grouped_attention<float>(const GroupedDims& d, const GroupedBuffers<float>& b, const BatchView& v, hipStream_t s) {
-    return b.talk ? talking_attention(d, b, v, s) : grouped_plain(d, b, v, s);
+    if (b.talk) return talking_attention(d, b, v, s);
+    if (knobs().grouped_plain || d.dp != d.vp || d.dp > 256 || d.scale <= 0.f) return grouped_plain(d, b, v, s);
+#define GROUPED(DS) (b.r1 ? grouped_keys<DS, true>(d, b, v, s) : grouped_keys<DS, false>(d, b, v, s))
+    switch (d.dp / 32) {
+    case 1: return GROUPED(1);
+    case 2: return GROUPED(2);
+    case 3: return GROUPED(3);
+    case 4: return GROUPED(4);
+    case 6: return GROUPED(6);
+    default: return GROUPED(8);
+    }
+#undef GROUPED
 }
 template <> int grouped_attention<bf16>(const GroupedDims& d, const GroupedBuffers<bf16>& b, const BatchView& v, hipStream_t s) {
     if (b.talk) return talking_attention(d, b, v, s);

@@ -24,10 +24,11 @@
 namespace fh {
 
 // A row's statistics (maximum m, sum l of e^(score − m)) closed by its head's sink: factor of the row's Σ e^(score − m)·value
+template <typename E>
 __device__ __forceinline__ float softmax_factor(float m, float l, const float* __restrict__ sink, int h) {
     if (!sink) return l > 0.f ? 1.0f / l : 0.f;
-    const float z = sink[h], top = fmaxf(m, z), f = __expf(m - top);
-    return f / (l * f + __expf(z - top));
+    const float z = sink[h], top = fmaxf(m, z), f = attn_exp<E>(m - top);
+    return f / (l * f + attn_exp<E>(z - top));
 }
 
 // one wave per token: norm of the query latent, norm of the kv latent, rotation of the shared key part, cache write
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(256, MT == 1 ? 2 : 1) void latent_attn_kernel(Laten
                 if (KS >= 2 || wave < 2 * KS) *reinterpret_cast<floatx4*>(dst + (wave + 4 * t) * 16 + 4 * a) = o[mt][t];
             if (threadIdx.x < 16) { dst[32 * KS] = m_run[mt]; dst[32 * KS + 1] = L; }
         } else if (ok[mt]) {
-            const float inv = softmax_factor(m_run[mt], L, p.sink, head[mt]);
+            const float inv = softmax_factor<bf16>(m_run[mt], L, p.sink, head[mt]);
             bf16* dst = p.o_lat + qrow[mt] * (32 * KS);
 #pragma unroll
             for (int t = 0; t < DT; t++)
@@ -333,8 +334,8 @@ __global__ __launch_bounds__(256, MT == 1 ? 2 : 1) void latent_attn_kernel(Laten
     }
 }
 // grid (tiles, quads of output dimensions / 256): one thread per (row, 4 dimensions); every load is in flight at once
-template <int NS>
-__global__ __launch_bounds__(256) void latent_attn_reduce_kernel(LatentDims d, LatentBuffers<bf16> p, BatchView v, int rows) {
+template <typename E, int NS>
+__global__ __launch_bounds__(256) void latent_attn_reduce_kernel(LatentDims d, LatentBuffers<E> p, BatchView v, int rows) {
     SeqTile w;
     if (!find_seq_tile(v, d.heads, rows, blockIdx.x, &w)) return;
     const int quads = d.kp >> 2, id = blockIdx.y * 256 + threadIdx.x, row = id / quads, c = (id % quads) * 4, ro = w.tile * rows + row;
@@ -353,15 +354,172 @@ __global__ __launch_bounds__(256) void latent_attn_reduce_kernel(LatentDims d, L
     for (int z = 0; z < NS; z++) M = fmaxf(M, m[z]);
 #pragma unroll
     for (int z = 0; z < NS; z++) {
-        const float f = __expf(m[z] - M);
+        const float f = attn_exp<E>(m[z] - M);
         L += l[z] * f;
         acc += o[z] * f;
     }
-    const float inv = softmax_factor(M, L, p.sink, ro % d.heads);
-    bf16x4 y;
+    const float inv = softmax_factor<E>(M, L, p.sink, ro % d.heads);
+    typename Frag<E>::v4 y;
 #pragma unroll
-    for (int r = 0; r < 4; r++) y[r] = (bf16)(acc[r] * inv);
-    *reinterpret_cast<bf16x4*>(p.o_lat + ((long)w.tok0 * d.heads + ro) * d.kp + c) = y;
+    for (int r = 0; r < 4; r++) y[r] = (E)(acc[r] * inv);
+    *reinterpret_cast<typename Frag<E>::v4*>(p.o_lat + ((long)w.tok0 * d.heads + ro) * d.kp + c) = y;
+}
+
+
+// ── 32-bit models on the matrix cores ──
+// grid (tiles of 16 (token, head) rows × KV splits), 64 keys per step.  Scores: every wave takes a quarter of the dimensions for all keys, the four
+// partial sums meet in LDS.  Values: wave w takes 128 output dimensions (of latents of 256 and fewer also a part of the keys, summed at the end).
+// v_mfma_f32_16x16x4 takes four keys at a time; product j of eight works on dimensions 8b + j, so that the eight dimensions 8b … 8b + 7 of a key,
+// which lie together in the cache, are one lane's operands of the eight, and the keys 4a + r of a lane's scores are its weights as they are.
+// Bound by the fp32 matrix rate: 2·kv_rank + rot products a (row, key), and the cache is read once for 16 rows where the plain form reads it for
+// each.  kv_rank 512, 16 heads, a prompt of 1000 tokens and 8 decoded: plain 4.68 ms, this 0.60 ms; 20 sequences of 50
+// tokens and what they decode 1.64 -> 0.86 ms.  Keys dealt out to the waves were slower in decode: at few keys most waves have none.
+template <int KS, int RS>
+__global__ __launch_bounds__(256) void latent_attn_f32_kernel(LatentDims d, LatentBuffers<float> p, BatchView v, int nsplit) {
+    constexpr int KP = 32 * KS, kd = KP + 32 * RS, NG = (KP + 127) / 128, PARTS = NG > 2 ? 1 : 4 / NG, SW = (KS + RS + 3) / 4, LD = KP + 4;
+    __shared__ floatx4 lds_s[4][4][64];
+    __shared__ __attribute__((aligned(16))) float lds_o[PARTS > 1 ? 16 * LD : 4];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, a = lane >> 4, b = lane & 15;
+    const int split = blockIdx.x % nsplit, tile_id = blockIdx.x / nsplit, g = wave % NG, part = wave / NG;
+    SeqTile w;
+    if (!find_seq_tile(v, d.heads, 16, tile_id, &w)) return;
+    const int rows = w.q_len * d.heads, rho = w.tile * 16 + b;
+    const bool ok = rho < rows, weighs = part < PARTS;
+    const int tl = ok ? rho / d.heads : 0, head = ok ? rho - tl * d.heads : 0, row_pos = w.pos0 + tl, win_lo = max(0, row_pos + 1 - d.window);
+    const int t_first = w.tile * 16 / d.heads, t_last = min(w.q_len - 1, (w.tile * 16 + 15) / d.heads);
+    const int blk_lo = max(0, w.pos0 + t_first + 1 - d.window) / 16, blk_hi = (w.pos0 + t_last + 16) / 16, nstep = (blk_hi - blk_lo + 3) / 4;
+    const int st_lo = nstep * split / nsplit, st_hi = nstep * (split + 1) / nsplit;
+    const int32_t* bt = v.bt + (long)w.seq * v.max_blocks;
+    // 32-wide pieces wave, wave + 4, … of the query (past the last one: zeros)
+    floatx8 qf[SW];
+#pragma unroll
+    for (int i = 0; i < SW; i++) {
+        const int s = wave + 4 * i;
+        if (s < KS) {
+            qf[i] = *reinterpret_cast<const floatx8*>(p.q_lat + ((long)w.tok0 * d.heads + (ok ? rho : 0)) * KP + 32 * s + 8 * a);
+        } else if (s < KS + RS) {
+            const float* q = p.q + (w.tok0 + tl) * p.ldq + head * (d.dp + d.rp) + d.dp + 32 * (s - KS) + 8 * a;
+            qf[i] = rot_apply(*reinterpret_cast<const floatx8*>(q), rot_load(32 * (s - KS) + 8 * a, d.rot_dims, p.cos_t, p.sin_t, row_pos));
+        } else {
+            qf[i] = (floatx8){0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    float m_run = -INFINITY, l_run = 0.f;
+    floatx4 o[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) o[j] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    for (int st = st_lo; st < st_hi; st++) {
+        const float* blk[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {                                          // (past the end: a copy of the last block, masked)
+            blk[i] = p.pool + (long)__builtin_amdgcn_readfirstlane(bt[min(blk_lo + 4 * st + i, blk_hi - 1)]) * 16 * kd;
+        }
+        floatx4 s4[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) s4[i] = (floatx4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < SW; q++) {
+            const int s = min(wave + 4 * q, KS + RS - 1);
+            floatx8 k[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) k[i] = *reinterpret_cast<const floatx8*>(blk[i] + s * 512 + lane * 8);
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) s4[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][j], qf[q][j], s4[i], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) lds_s[wave][i][lane] = s4[i];
+        __syncthreads();
+        float sc[16], mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const floatx4 z = (lds_s[0][i][lane] + lds_s[1][i][lane]) + (lds_s[2][i][lane] + lds_s[3][i][lane]);
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int key = (blk_lo + 4 * st + i) * 16 + 4 * a + r;
+                sc[4 * i + r] = ok && key <= row_pos && key >= win_lo ? z[r] * d.scale : -INFINITY;
+                mx = fmaxf(mx, sc[4 * i + r]);
+            }
+        }
+        __syncthreads();                                                       // (the sums of the next step take their place)
+        const float m_new = fmaxf(m_run, rows_reduce_max(mx)), m_safe = m_new == -INFINITY ? 0.f : m_new, alpha = expf(m_run - m_safe);
+        float ps = 0.f;
+#pragma unroll
+        for (int j = 0; j < 16; j++) { sc[j] = expf(sc[j] - m_safe); ps += sc[j]; }
+        l_run = l_run * alpha + ps;                                            // (this lane's keys; the four lane groups meet at the end)
+        m_run = m_new;
+        if (!weighs) continue;
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) o[j][r] *= alpha;
+        const int chunk = min(16 * g + b, KP / 8 - 1);                         // (dimensions past the latent: not written)
+#pragma unroll
+        for (int q = 0; q < 4 / PARTS; q++) {
+            const float* block = blk[q];
+            float pr[4] = {sc[4 * q], sc[4 * q + 1], sc[4 * q + 2], sc[4 * q + 3]};
+            if (PARTS == 4) {
+#pragma unroll
+                for (int i = 1; i < 4; i++)
+                    if (part == i) {
+                        block = blk[i];
+#pragma unroll
+                        for (int r = 0; r < 4; r++) pr[r] = sc[4 * i + r];
+                    }
+            } else if (PARTS == 2 && part == 1) {
+                block = blk[2 + q];
+#pragma unroll
+                for (int r = 0; r < 4; r++) pr[r] = sc[8 + 4 * q + r];
+            }
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const floatx8 x = *reinterpret_cast<const floatx8*>(block + (chunk * 16 + 4 * a + r) * 8);
+#pragma unroll
+                for (int j = 0; j < 8; j++) o[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j], pr[r], o[j], 0, 0, 0);
+            }
+        }
+    }
+    const float l = rows_reduce_sum(l_run);
+    if (PARTS > 1) {
+        for (int turn = 1; turn < PARTS; turn++) {
+            if (part == turn) {
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (128 * g + 8 * (4 * a + r) < KP)
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            float* x = lds_o + b * LD + 128 * g + 8 * (4 * a + r) + j;
+                            *x = turn > 1 ? *x + o[j][r] : o[j][r];
+                        }
+            }
+            __syncthreads();
+        }
+        if (part == 0) {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                if (128 * g + 8 * (4 * a + r) < KP)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) o[j][r] += lds_o[b * LD + 128 * g + 8 * (4 * a + r) + j];
+        }
+    }
+    if (part > 0) return;
+    const float f = nsplit > 1 ? 1.f : softmax_factor<float>(m_run, l, p.sink, head);
+    float* dst = nsplit > 1 ? p.partial + ((long)blockIdx.x * 16 + b) * (KP + LATENT_PARTIAL_PAD) : p.o_lat + ((long)w.tok0 * d.heads + rho) * KP;
+    if (nsplit == 1 && !ok) return;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int c = 128 * g + 8 * (4 * a + r);
+        if (c >= KP) continue;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            floatx4 x;
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = o[4 * h + j][r] * f;
+            *reinterpret_cast<floatx4*>(dst + c + 4 * h) = x;
+        }
+    }
+    if (nsplit > 1 && g == 0 && a == 0) { dst[KP] = m_run; dst[KP + 1] = l; }
 }
 
 // ── portions over expanded keys and values ──
@@ -507,7 +665,7 @@ __global__ __launch_bounds__(256, 2) void latent_expanded_kernel(LatentDims d, L
         const float l = rows_reduce_sum(l_run[mt]);
         if (!ok[mt]) continue;
         const long tok = tok0 + tile0 + (wave * MT + mt) * 16 + b;
-        float f = softmax_factor(m_run[mt] * 0.6931471805599453f, l, p.sink, h);      // (the maximum is kept in base 2)
+        float f = softmax_factor<bf16>(m_run[mt] * 0.6931471805599453f, l, p.sink, h);      // (the maximum is kept in base 2)
         if (x.gate) f *= (float)x.gate[tok * x.ld_gate + h];
         bf16* dst = x.out + tok * x.ldo + h * d.vp + 4 * a;
 #pragma unroll
@@ -542,6 +700,16 @@ static int latent_plain(const LatentDims& d, const LatentBuffers<E>& b, const Ba
     const size_t lds = (size_t)(2 * d.kp + d.rp + 256 + 8) * 4;
     FH_REQUIRE(lds <= 64 * 1024, "latent attention: kv_rank %d + rotated %d do not fit LDS", d.kv_rank, d.rot_dim);
     hipLaunchKernelGGL(latent_attn_plain_kernel<E>, dim3(v.T, d.heads), dim3(256), lds, s, d, b, v);
+    FH_CHECK_LAUNCH();
+    return 0;
+}
+template <typename E>
+static int latent_reduce(const LatentDims& d, const LatentBuffers<E>& b, const BatchView& v, int tiles, int rows, int ns, hipStream_t s) {
+    const dim3 rg(tiles, cdiv(rows * (d.kp / 4), 256));
+    if (ns == 2) hipLaunchKernelGGL((latent_attn_reduce_kernel<E, 2>), rg, dim3(256), 0, s, d, b, v, rows);
+    else if (ns == 4) hipLaunchKernelGGL((latent_attn_reduce_kernel<E, 4>), rg, dim3(256), 0, s, d, b, v, rows);
+    else if (ns == 8) hipLaunchKernelGGL((latent_attn_reduce_kernel<E, 8>), rg, dim3(256), 0, s, d, b, v, rows);
+    else hipLaunchKernelGGL((latent_attn_reduce_kernel<E, 16>), rg, dim3(256), 0, s, d, b, v, rows);
     FH_CHECK_LAUNCH();
     return 0;
 }
@@ -583,18 +751,38 @@ static int latent_mfma(const LatentDims& d, const LatentBuffers<bf16>& b, const 
 #undef LATENT
 #undef LATENT2
     FH_CHECK_LAUNCH();
-    if (ns > 1) {
-        const dim3 rg(tiles, cdiv(rows * (d.kp / 4), 256));
-        if (ns == 2) hipLaunchKernelGGL(latent_attn_reduce_kernel<2>, rg, dim3(256), 0, s, d, b, v, rows);
-        else if (ns == 4) hipLaunchKernelGGL(latent_attn_reduce_kernel<4>, rg, dim3(256), 0, s, d, b, v, rows);
-        else if (ns == 8) hipLaunchKernelGGL(latent_attn_reduce_kernel<8>, rg, dim3(256), 0, s, d, b, v, rows);
-        else hipLaunchKernelGGL(latent_attn_reduce_kernel<16>, rg, dim3(256), 0, s, d, b, v, rows);
-        FH_CHECK_LAUNCH();
+    return ns > 1 ? latent_reduce(d, b, v, tiles, rows, ns, s) : 0;
+}
+static int latent_mfma(const LatentDims& d, const LatentBuffers<float>& b, const BatchView& v, hipStream_t s) {
+    const int tiles = v.single ? v.num_seqs * cdiv(d.heads, 16) : (int)(((long)v.T * d.heads) / 16) + v.num_seqs;
+    const int keys = (int)std::min<long>(v.max_keys, (long)d.window + 16);
+    // split the keys while there is less than a workgroup per CU and a split keeps ≥ 128 keys (two steps, 4 µs of products each)
+    int ns = 1;
+    while (ns < 16 && tiles * ns < 256 && keys >= 2 * ns * 128) ns *= 2;
+    if (knobs().latent_splits > 0)
+        for (ns = 1; ns < std::min(16, knobs().latent_splits); ns *= 2) {}
+    while (ns > 1 && (size_t)tiles * ns * 16 * (d.kp + LATENT_PARTIAL_PAD) * 4 > b.partial_bytes) ns /= 2;
+    form_hit(ns > 1 ? FORM_LATENT_ATTN_SPLIT : FORM_LATENT_ATTN);
+#define LATENT(KS)                                                                                                                       \
+    do {                                                                                                                                 \
+        if (d.rp == 32) hipLaunchKernelGGL((latent_attn_f32_kernel<KS, 1>), dim3(tiles * ns), dim3(256), 0, s, d, b, v, ns);             \
+        else hipLaunchKernelGGL((latent_attn_f32_kernel<KS, 2>), dim3(tiles * ns), dim3(256), 0, s, d, b, v, ns);                        \
+    } while (0)
+    switch (d.kp) {
+    case 32: LATENT(1); break;
+    case 64: LATENT(2); break;
+    case 128: LATENT(4); break;
+    case 256: LATENT(8); break;
+    case 384: LATENT(12); break;
+    default: LATENT(16); break;
     }
-    return 0;
+#undef LATENT
+    FH_CHECK_LAUNCH();
+    return ns > 1 ? latent_reduce(d, b, v, tiles, 16, ns, s) : 0;
 }
 template <> int latent_attention<float>(const LatentDims& d, const LatentBuffers<float>& b, const BatchView& v, hipStream_t s) {
-    return latent_plain(d, b, v, s);
+    if (knobs().latent_plain || d.kp > 512 || d.rp > 64) return latent_plain(d, b, v, s);
+    return latent_mfma(d, b, v, s);
 }
 template <> int latent_attention<bf16>(const LatentDims& d, const LatentBuffers<bf16>& b, const BatchView& v, hipStream_t s) {
     if (knobs().latent_plain || d.kp > 512 || d.rp > 64) return latent_plain(d, b, v, s);

@@ -5,6 +5,10 @@
 
 namespace fh {
 
+// Exponentials of the softmax: 16-bit models round the weights anyway, 32-bit models call the library functions.
+template <typename E> __device__ __forceinline__ float attn_exp(float x) { return sizeof(E) == 2 ? __expf(x) : expf(x); }
+template <typename E> __device__ __forceinline__ float attn_exp2(float x) { return sizeof(E) == 2 ? __builtin_amdgcn_exp2f(x) : exp2f(x); }
+
 // cosines and sines of the four pairs (2i, 2i + 1) starting at dimension d0, position `pos`; pairs past rot_dims pass unchanged
 struct Rot4 { float c[4], s[4]; };
 __device__ __forceinline__ Rot4 rot_load(int d0, int rot_dims, const float* __restrict__ cos_t, const float* __restrict__ sin_t, long pos) {

@@ -95,10 +95,11 @@ __global__ __launch_bounds__(256) void talk_attn_plain_kernel(GroupedDims d, Gro
 // to everyone through LDS, and weighs its heads' values with the weights of all 16·HB query heads.  32 keys per step, one barrier; keys and
 // values of the next step are on their way while this one is worked on.
 // Partial of a (token, split): [16·HB heads][kv_heads·D] outputs, then maximum and sum per head.
-template <int DS, int HB, int NW, int CW>
-__global__ __launch_bounds__(64 * NW) void talk_attn_keys_kernel(GroupedDims d, GroupedBuffers<bf16> p, BatchView v, int t0, int nsplit) {
+template <typename E, int DS, int HB, int NW, int CW>
+__global__ __launch_bounds__(64 * NW) void talk_attn_keys_kernel(GroupedDims d, GroupedBuffers<E> p, BatchView v, int t0, int nsplit) {
+    typedef typename Frag<E>::v8 v8;
     constexpr int DT = 2 * DS, D = 32 * DS, HP = 16 * HB;
-    __shared__ __attribute__((aligned(16))) bf16 lds_p[2][HP][4][8];
+    __shared__ __attribute__((aligned(16))) E lds_p[2][HP][4][8];
     __shared__ float lds_a[2][HP];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, a = lane >> 4, b = lane & 15;
     const int split = blockIdx.x % nsplit, unit = blockIdx.x / nsplit, tok = t0 + unit, G = d.heads / d.kv_heads;
@@ -109,10 +110,10 @@ __global__ __launch_bounds__(64 * NW) void talk_attn_keys_kernel(GroupedDims d, 
     const int32_t* bt = v.bt + (long)seq * v.max_blocks;
     const float sl2 = d.scale * LOG2E;
     const long kd = (long)d.kv_heads * D * 16;
-    for (int i = threadIdx.x; i < 2 * HP * 32; i += 64 * NW) (&lds_p[0][0][0][0])[i] = (bf16)0.f;
+    for (int i = threadIdx.x; i < 2 * HP * 32; i += 64 * NW) (&lds_p[0][0][0][0])[i] = (E)0.f;
     for (int i = threadIdx.x; i < 2 * HP; i += 64 * NW) (&lds_a[0][0])[i] = 1.f;
-    bf16x8 qf[CW][DS], kf[CW][2][DS], vf[CW][2][DS];
-    const bf16x8 zero = {};
+    v8 qf[CW][DS], kf[CW][2][DS], vf[CW][2][DS];
+    const v8 zero = {};
     bool live[CW];
     long off[CW];
 #pragma unroll
@@ -123,19 +124,19 @@ __global__ __launch_bounds__(64 * NW) void talk_attn_keys_kernel(GroupedDims d, 
         const int head = min(kvh * G + min(b, G - 1), d.heads - 1);
 #pragma unroll
         for (int s = 0; s < DS; s++) {
-            const bf16x8 q = *reinterpret_cast<const bf16x8*>(p.q + ((long)tok * d.heads + head) * D + 32 * s + 8 * a);
+            const v8 q = *reinterpret_cast<const v8*>(p.q + ((long)tok * d.heads + head) * D + 32 * s + 8 * a);
             qf[c][s] = live[c] && b < G ? q : zero;
         }
     }
     // (past the end: a copy of the last block, masked)
     auto block_of = [&](int st, int i) { return (long)__builtin_amdgcn_readfirstlane(bt[min(blk_lo + 2 * st + i, blk_hi - 1)]); };
-    auto load = [&](bf16x8 (&f)[CW][2][DS], const bf16* pool, const long (&blk)[2]) {
+    auto load = [&](v8 (&f)[CW][2][DS], const E* pool, const long (&blk)[2]) {
 #pragma unroll
         for (int c = 0; c < CW; c++)
 #pragma unroll
             for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int s = 0; s < DS; s++) f[c][i][s] = *reinterpret_cast<const bf16x8*>(pool + blk[i] * kd + off[c] + s * 512);
+                for (int s = 0; s < DS; s++) f[c][i][s] = *reinterpret_cast<const v8*>(pool + blk[i] * kd + off[c] + s * 512);
     };
     float m_run[CW], l_run[CW];
     floatx4 o[HB][CW][DT];
@@ -161,7 +162,7 @@ __global__ __launch_bounds__(64 * NW) void talk_attn_keys_kernel(GroupedDims d, 
             for (int i = 0; i < 2; i++) {
                 floatx4 s2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-                for (int s = 0; s < DS; s++) s2[s & 1] = Frag<bf16>::mma(kf[c][i][s], qf[c][s], s2[s & 1]);
+                for (int s = 0; s < DS; s++) s2[s & 1] = Frag<E>::mma(kf[c][i][s], qf[c][s], s2[s & 1]);
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const int key = (blk_lo + 2 * st + i) * 16 + 4 * a + r;
@@ -169,16 +170,16 @@ __global__ __launch_bounds__(64 * NW) void talk_attn_keys_kernel(GroupedDims d, 
                     mx = fmaxf(mx, sc[4 * i + r]);
                 }
             }
-            const float m_new = fmaxf(m_run[c], rows_reduce_max(mx)), m_safe = m_new == -INFINITY ? 0.f : m_new, alpha = __builtin_amdgcn_exp2f(m_run[c] - m_safe);
-            bf16x8 pf;
+            const float m_new = fmaxf(m_run[c], rows_reduce_max(mx)), m_safe = m_new == -INFINITY ? 0.f : m_new, alpha = attn_exp2<E>(m_run[c] - m_safe);
+            v8 pf;
             float ps = 0.f;
 #pragma unroll
-            for (int j = 0; j < 8; j++) { const float e = __builtin_amdgcn_exp2f(sc[j] - m_safe); ps += e; pf[j] = (bf16)e; }
+            for (int j = 0; j < 8; j++) { const float e = attn_exp2<E>(sc[j] - m_safe); ps += e; pf[j] = (E)e; }
             l_run[c] = l_run[c] * alpha + ps;                                  // (this lane's keys; the four lane groups meet at the end)
             m_run[c] = m_new;
             if (live[c] && b < G) {
                 const int h = (wave + NW * c) * G + b;
-                *reinterpret_cast<bf16x8*>(lds_p[buf][h][a]) = pf;
+                *reinterpret_cast<v8*>(lds_p[buf][h][a]) = pf;
                 if (a == 0) lds_a[buf][h] = alpha;
             }
         }
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(64 * NW) void talk_attn_keys_kernel(GroupedDims d, 
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");        // (weights of step st; the other buffer's readers are past it)
 #pragma unroll
         for (int h = 0; h < HB; h++) {
-            const bf16x8 pf = *reinterpret_cast<const bf16x8*>(lds_p[buf][h * 16 + b][a]);
+            const v8 pf = *reinterpret_cast<const v8*>(lds_p[buf][h * 16 + b][a]);
             const float alpha = lds_a[buf][h * 16 + b];
             const bool scaled = __ballot(alpha != 1.f) != 0;
 #pragma unroll
@@ -196,7 +197,7 @@ __global__ __launch_bounds__(64 * NW) void talk_attn_keys_kernel(GroupedDims d, 
                     if (scaled)
 #pragma unroll
                         for (int r = 0; r < 4; r++) o[h][c][t][r] *= alpha;
-                    o[h][c][t] = Frag<bf16>::mma(value_operand(vf[c][0][t >> 1], vf[c][1][t >> 1], t & 1), pf, o[h][c][t]);
+                    o[h][c][t] = Frag<E>::mma(value_operand(vf[c][0][t >> 1], vf[c][1][t >> 1], t & 1), pf, o[h][c][t]);
                 }
         }
         load(vf, p.v_pool, blk);
@@ -218,7 +219,9 @@ __global__ __launch_bounds__(64 * NW) void talk_attn_keys_kernel(GroupedDims d, 
     }
 }
 // grid (tokens, kv_heads): the splits of every head's sum over this head's values, then the mixture
-__global__ __launch_bounds__(256) void talk_attn_mix_kernel(GroupedDims d, GroupedBuffers<bf16> p, int t0, int nsplit, int hp) {
+template <typename E>
+__global__ __launch_bounds__(256) void talk_attn_mix_kernel(GroupedDims d, GroupedBuffers<E> p, int t0, int nsplit, int hp) {
+    typedef typename Frag<E>::v4 v4;
     extern __shared__ __attribute__((aligned(16))) float lds[];                // [heads][vp], factors [nsplit][heads], sums [nsplit][heads], rows of the mixture [G][heads]
     const int H = d.heads, G = H / d.kv_heads, kvh = blockIdx.y, D = d.vp, quads = D / 4;
     const long tok = t0 + blockIdx.x, kvd = (long)d.kv_heads * D, stride = hp * (kvd + 2);
@@ -235,11 +238,11 @@ __global__ __launch_bounds__(256) void talk_attn_mix_kernel(GroupedDims d, Group
         float M = -INFINITY, L = 0.f;
         for (int z = 0; z < nsplit; z++) M = fmaxf(M, f[z * H + h]);
         for (int z = 0; z < nsplit; z++) {
-            const float e = __builtin_amdgcn_exp2f(f[z * H + h] - M);
+            const float e = attn_exp2<E>(f[z * H + h] - M);
             f[z * H + h] = e;
             L += sum[z * H + h] * e;
         }
-        if (p.sink) L += __builtin_amdgcn_exp2f(p.sink[h] * LOG2E - M);
+        if (p.sink) L += attn_exp2<E>(p.sink[h] * LOG2E - M);
         const float inv = 1.0f / L;
         for (int z = 0; z < nsplit; z++) f[z * H + h] *= inv;
     }
@@ -261,8 +264,8 @@ __global__ __launch_bounds__(256) void talk_attn_mix_kernel(GroupedDims d, Group
     for (int i = threadIdx.x; i < G * quads; i += 256) {
         const int g0 = i / quads, h = kvh * G + g0, c = (i - g0 * quads) * 4, col = h * D + c;
         float f1 = p.gate ? (float)p.gate[tok * p.ld_gate + h] : 1.f;
-        bf16x4 y, gate = {(bf16)1.f, (bf16)1.f, (bf16)1.f, (bf16)1.f};
-        if (p.value_gate) gate = *reinterpret_cast<const bf16x4*>(p.value_gate + tok * p.ld_value_gate + col);
+        v4 y, gate = {(E)1.f, (E)1.f, (E)1.f, (E)1.f};
+        if (p.value_gate) gate = *reinterpret_cast<const v4*>(p.value_gate + tok * p.ld_value_gate + col);
         floatx4 x = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 4
         for (int g = 0; g < H; g++) {
@@ -272,8 +275,8 @@ __global__ __launch_bounds__(256) void talk_attn_mix_kernel(GroupedDims d, Group
             for (int r = 0; r < 4; r++) x[r] += w * v[r];
         }
 #pragma unroll
-        for (int r = 0; r < 4; r++) y[r] = (bf16)(x[r] * f1 * (float)gate[r]);
-        *reinterpret_cast<bf16x4*>(p.out + tok * p.ldo + col) = y;
+        for (int r = 0; r < 4; r++) y[r] = (E)(x[r] * f1 * (float)gate[r]);
+        *reinterpret_cast<v4*>(p.out + tok * p.ldo + col) = y;
     }
 }
 
@@ -628,6 +631,8 @@ bool talk_tile_supports(const GroupedDims& d) {
 bool talk_keys_supports(const GroupedDims& d) {
     return talk_tile_supports(d) && d.heads / d.kv_heads <= 16 && d.kv_heads <= (d.heads <= 16 && d.dp <= 128 ? 16 : 8);
 }
+// (32-bit operands: one key / value head per wave, eight waves up to 128 dimensions)
+bool talk_keys_supports_f32(const GroupedDims& d) { return talk_keys_supports(d) && d.kv_heads <= (d.dp <= 128 ? 8 : 4); }
 template <int DS, int HB, bool SHARED>
 int talk_tile(const GroupedDims& d, const GroupedBuffers<bf16>& b, const BatchView& v, int min_tokens, hipStream_t s) {
     constexpr size_t lds = ((size_t)32 * 16 * 4 * HB * 8 + (size_t)16 * HB * 16 * 32 + HB * HB * 512) * 2;
@@ -656,8 +661,8 @@ int talk_tile(const GroupedDims& d, const GroupedBuffers<bf16>& b, const BatchVi
     return 0;
 }
 // tokens [t0, t0 + n) of the batch
-template <int DS, int HB>
-int talk_keys(const GroupedDims& d, const GroupedBuffers<bf16>& b, const BatchView& v, int t0, int n, hipStream_t s) {
+template <int DS, int HB, typename E>
+int talk_keys(const GroupedDims& d, const GroupedBuffers<E>& b, const BatchView& v, int t0, int n, hipStream_t s) {
     const int keys = (int)std::min<long>(v.max_keys, (long)d.window + 16), room = (int)(b.partial_bytes / talk_partial(d)), hp = 16 * HB;
     FH_REQUIRE(room > 0, "attention with mixed heads: no scratch");
     form_hit(FORM_TALK_ATTN_KEYS);
@@ -669,13 +674,13 @@ int talk_keys(const GroupedDims& d, const GroupedBuffers<bf16>& b, const BatchVi
         if (knobs().grouped_splits > 0) ns = std::min(64, knobs().grouped_splits);
         while (ns > 1 && m * ns > room) ns /= 2;
         const dim3 grid(m * ns);
-#define KEYS(NW, CW) hipLaunchKernelGGL((talk_attn_keys_kernel<DS, HB, NW, CW>), grid, dim3(64 * NW), 0, s, d, b, v, t0 + done, ns)
+#define KEYS(NW, CW) hipLaunchKernelGGL((talk_attn_keys_kernel<E, DS, HB, NW, CW>), grid, dim3(64 * NW), 0, s, d, b, v, t0 + done, ns)
         if (d.kv_heads <= 4) KEYS(4, 1);
-        else if (d.kv_heads <= 8) KEYS(8, 1);
-        else if constexpr (HB == 1 && DS <= 4) KEYS(8, 2);
+        else if (d.kv_heads <= 8) { if constexpr (sizeof(E) == 2 || DS <= 4) KEYS(8, 1); }
+        else if constexpr (sizeof(E) == 2 && HB == 1 && DS <= 4) KEYS(8, 2);
 #undef KEYS
         FH_CHECK_LAUNCH();
-        hipLaunchKernelGGL(talk_attn_mix_kernel, dim3(m, d.kv_heads), dim3(256), (size_t)d.heads * (d.vp + 2 * ns + d.heads / d.kv_heads) * 4, s, d, b, t0 + done, ns, hp);
+        hipLaunchKernelGGL(talk_attn_mix_kernel<E>, dim3(m, d.kv_heads), dim3(256), (size_t)d.heads * (d.vp + 2 * ns + d.heads / d.kv_heads) * 4, s, d, b, t0 + done, ns, hp);
         FH_CHECK_LAUNCH();
         done += m;
     }
@@ -712,7 +717,28 @@ size_t talking_partial_bytes(const GroupedDims& d, int max_tokens) {
     return std::max(keys, talk_tile_supports(d) ? rows * d.heads * d.vp * 4 : 0);
 }
 
-template <> int talking_attention<float>(const GroupedDims& d, const GroupedBuffers<float>& b, const BatchView& v, hipStream_t s) { return talk_plain(d, b, v, s); }
+// 32-bit models take the keys form for portions too: fp32 products of every head with every key / value head's values cost kv_heads times the
+// values' share, but on the matrix cores and with the cache read once per token (16 heads of 128 dimensions on 4, a prompt of 1000 tokens and 8
+// decoded: plain 19.7 ms, keys 0.44 ms).
+template <> int talking_attention<float>(const GroupedDims& d, const GroupedBuffers<float>& b, const BatchView& v, hipStream_t s) {
+    if (knobs().grouped_plain || !talk_keys_supports_f32(d)) return talk_plain(d, b, v, s);
+    if (d.heads > 16) {
+        switch (d.dp / 32) {
+        case 1: return talk_keys<1, 2>(d, b, v, 0, v.T, s);
+        case 2: return talk_keys<2, 2>(d, b, v, 0, v.T, s);
+        case 3: return talk_keys<3, 2>(d, b, v, 0, v.T, s);
+        default: return talk_keys<4, 2>(d, b, v, 0, v.T, s);
+        }
+    }
+    switch (d.dp / 32) {
+    case 1: return talk_keys<1, 1>(d, b, v, 0, v.T, s);
+    case 2: return talk_keys<2, 1>(d, b, v, 0, v.T, s);
+    case 3: return talk_keys<3, 1>(d, b, v, 0, v.T, s);
+    case 4: return talk_keys<4, 1>(d, b, v, 0, v.T, s);
+    case 6: return talk_keys<6, 1>(d, b, v, 0, v.T, s);
+    default: return talk_keys<8, 1>(d, b, v, 0, v.T, s);
+    }
+}
 template <> int talking_attention<bf16>(const GroupedDims& d, const GroupedBuffers<bf16>& b, const BatchView& v, hipStream_t s) {
     if (knobs().grouped_plain || !talk_tile_supports(d)) return talk_plain(d, b, v, s);
     if (d.heads > 16) {

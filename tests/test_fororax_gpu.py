@@ -123,6 +123,25 @@ def test_far_attention_alone(pkg, tmp_path, knobs, forms, form, dtype, i):
     assert differs(cfg, wrong, t, taps)
 
 
+@pytest.mark.parametrize("form", ["keys", "split"])
+@pytest.mark.parametrize("i", range(len(FAR)))
+def test_far_attention_alone_in_32_bits(pkg, tmp_path, knobs, forms, form, i):
+    test_far_attention_alone(pkg, tmp_path, knobs, forms, form, "float32", i)
+
+
+@pytest.mark.parametrize("form", ["keys", "split"])
+@pytest.mark.parametrize("i", range(len(TALK)))
+def test_talking_attention_alone_in_32_bits(pkg, tmp_path, knobs, forms, form, i):
+    """On the matrix cores up to 32 heads, 16 of them on a key / value head, and as many key / value heads as waves; else the plain form."""
+    knobs.set(**FORMS[form])
+    cfg, m = model([TALK[i]]), TALK[i]["mixer"]
+    forms.reset()
+    agree(pkg, tmp_path, cfg, G.weights(cfg, 40 + i), "float32", tol=ALONE["float32"])
+    d, h = max(m["dim"], m["vdim"]), forms.hits()
+    keys = m["heads"] <= 32 and d <= (256 if m["heads"] <= 16 else 128) and m["heads"] // m["kv_heads"] <= 16 and m["kv_heads"] <= (8 if d <= 128 else 4)
+    assert h.get("talk_attn_keys" if keys else "talk_attn_plain") and not h.get("talk_attn_plain" if keys else "talk_attn_keys")
+
+
 @pytest.mark.parametrize("form,dtype", CASES)
 @pytest.mark.parametrize("i", range(len(TALK)))
 def test_talking_attention_alone(pkg, tmp_path, knobs, forms, form, dtype, i):

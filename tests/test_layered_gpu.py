@@ -451,6 +451,25 @@ def test_trace_replay(cases, tmp_path, name, dtype):
     assert p.wait(timeout=30) == 0
 
 
+@pytest.mark.parametrize("splits", [1, 4])
+@pytest.mark.parametrize("heads,dim,rot,vdim,rank,window", [(3, 20, 6, 36, 30, 700), (17, 16, 10, 8, 60, 33), (5, 24, 40, 12, 100, 64), (2, 8, 6, 8, 128, 1), (16, 32, 64, 16, 250, 90),
+                                                            (4, 16, 2, 16, 384, 700), (6, 8, 34, 10, 512, 130), (1, 8, 4, 8, 520, 50), (2, 8, 70, 8, 40, 20)])
+def test_latent_attention_in_32_bits(pkg, tmp_path, knobs, forms, heads, dim, rot, vdim, rank, window, splits):
+    """Every padded size of the latent, one head and more heads than a row tile, windows inside a step of keys and across several; whole prompts,
+    portions and single tokens, keys in one piece and split.  Latents of more than 512 and rotated parts of more than 64 take the plain form."""
+    knobs.set(LATENT_SPLITS=splits)
+    cfg = G.config(64, 80, [G.attention(heads, dim, rot, vdim, 40, rank, window)], buckets=13)
+    w, t = G.weights(cfg, rank), toks(cfg, 170, 9)
+    want = L.forward(cfg, w, t)
+    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), "float32")
+    forms.reset()
+    for seq, cuts in enumerate(([170], [100, 1, 1, 47, 20, 1], [1, 15, 16, 17, 121])):
+        assert rel(feed(m, seq, t, cuts), want) < TOL["float32"]
+        m.release(seq)
+    h, plain = forms.hits(), rank > 512 or rot > 64
+    assert bool(h.get("latent_attn_plain")) == plain and bool(h.get("latent_attn_split" if splits > 1 else "latent_attn")) != plain
+
+
 @pytest.mark.parametrize("name", ["wide", "shared", "sinks", "loop", "talks"])
 def test_few_row_and_tile_projections_agree(pkg, cases, knobs, forms, name):
     """The tile kernel in each of its sizes and the few-row kernel on the same portions."""
