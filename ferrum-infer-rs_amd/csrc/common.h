@@ -121,6 +121,16 @@ __device__ __forceinline__ void reduce_slabs8(const float* __restrict__ base, lo
     }
 }
 
+// act(gate) · up of a gated MLP: SiLU, or GELU in its tanh form (one definition: the fused and the separate launches give the same bits)
+template <bool GELU>
+__device__ __forceinline__ _Float16 gated_act(float g, float u) {
+    if (GELU) {
+        const float inner = 0.79788456f * (g + 0.044715f * g * g * g);
+        return (_Float16)(0.5f * g * (1.0f + tanhf(inner)) * u);
+    }
+    return (_Float16)(g / (1.0f + __expf(-g)) * u);
+}
+
 static inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 __host__ __device__ inline int cdiv_dev(int a, int b) { return (a + b - 1) / b; }

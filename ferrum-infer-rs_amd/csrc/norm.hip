@@ -457,16 +457,7 @@ __global__ void gated_act_kernel(const __half* __restrict__ gate_up, __half* __r
     half8 u = *reinterpret_cast<const half8*>(gate_up + t * 2 * im + im + i * 8);
     half8 o;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        float gf = (float)g[j], uf = (float)u[j], a;
-        if (GELU) {
-            float inner = 0.79788456f * (gf + 0.044715f * gf * gf * gf);
-            a = 0.5f * gf * (1.0f + tanhf(inner));
-        } else {
-            a = gf / (1.0f + __expf(-gf));
-        }
-        o[j] = (_Float16)(a * uf);
-    }
+    for (int j = 0; j < 8; j++) o[j] = gated_act<GELU>((float)g[j], (float)u[j]);
     *reinterpret_cast<half8*>(out + t * im + i * 8) = o;
 }
 
@@ -483,17 +474,7 @@ __global__ void gated_act_slabs_kernel(const float* __restrict__ slabs, int S, l
     reduce_slabs8(slabs + t * ld + im + i * 8, slab_stride, S, u);     // loop pays one memory round trip per slab)
     half8 o;
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const float gf = (float)(_Float16)g[j], uf = (float)(_Float16)u[j];
-        float a;
-        if (GELU) {
-            float inner = 0.79788456f * (gf + 0.044715f * gf * gf * gf);
-            a = 0.5f * gf * (1.0f + tanhf(inner));
-        } else {
-            a = gf / (1.0f + __expf(-gf));
-        }
-        o[j] = (_Float16)(a * uf);
-    }
+    for (int j = 0; j < 8; j++) o[j] = gated_act<GELU>((float)(_Float16)g[j], (float)(_Float16)u[j]);
     *reinterpret_cast<half8*>(out + t * im + i * 8) = o;
 }
 

@@ -1315,6 +1315,13 @@ int dense_linear(FerrumHipModel* m, const W4Device& w, const __half* x, __half* 
     return w4_gemm_dense(w, x, out, T, m->workspace, m->workspace_bytes, s);
 }
 
+// … of ≤ 32 rows as fp32 split-K slabs in the workspace, for a consumer that sums them
+int dense_slabs_gemm(FerrumHipModel* m, const W4Device& w, const __half* x, int T, int* S, int* rows_pad, int* n_pad, hipStream_t s) {
+    *S = 0;
+    if (w4_gemm_rows_splits(w, T, m->workspace_bytes)) return w4_gemm_rows(w, x, m->workspace, m->workspace_bytes, T, S, rows_pad, n_pad, s);
+    return w4_gemm_dense_slabs_lds(w, x, m->workspace, m->workspace_bytes, T, S, rows_pad, n_pad, s);
+}
+
 // Enqueue every kernel of one forward on m->stream.  Index tensors are already on the device.
 struct GreedyDeviceOpts {          // device pointers, already uploaded on m->stream
     const uint8_t* mask = nullptr; int mask_len = 0;
@@ -1463,18 +1470,21 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             form_hit(FORM_DENSE_CHAIN);
             const int I = c.intermediate;
             int S = 0, rows_pad = 0, n_pad = 0;
-            const bool slabs = m->dense_slabs && T > 16 && T <= 32;      // 17–32 rows: split-K slabs summed by their consumers
-            if (slabs) {
+            // ≤ 32 rows: split-K slabs summed by their consumers, gate_up of ≤ 16 with its activation in the launch
+            const bool slabs = m->dense_slabs && T <= 32 && (T > 16 || w4_gemm_rows_splits(L.down, T, m->workspace_bytes));
+            if (T > 16 && slabs) {
                 RUN(w4_gemm_dense_slabs_lds(L.gate_up, m->norm_out, m->workspace, m->workspace_bytes, T, &S, &rows_pad, &n_pad, s));
                 RUN(fused_gated_act_slabs_f16(m->workspace, S, (long)rows_pad * n_pad, n_pad, m->act_out, T, I, c.activation == 1, s));
                 S = 0;
-                RUN(w4_gemm_dense_slabs_lds(L.down, m->act_out, m->workspace, m->workspace_bytes, T, &S, &rows_pad, &n_pad, s));
+            } else if (w4_gemm_gated_supports(L.gate_up, T, I)) {
+                RUN(w4_gemm_gated(L.gate_up, m->norm_out, m->act_out, T, I, c.activation == 1, s));
             } else {
                 RUN(dense_linear(m, L.gate_up, m->norm_out, m->gate_up_out, T, s, true));
                 if (c.activation == 1) { RUN(fused_gelu_tanh_mul_split_f16(m->gate_up_out, m->act_out, T, I, s)); }
                 else { RUN(fused_silu_mul_split_f16(m->gate_up_out, m->act_out, T, I, s)); }
-                RUN(dense_linear(m, L.down, m->act_out, m->mlp_out, T, s));
             }
+            if (slabs) { RUN(dense_slabs_gemm(m, L.down, m->act_out, T, &S, &rows_pad, &n_pad, s)); }
+            else { RUN(dense_linear(m, L.down, m->act_out, m->mlp_out, T, s)); }
             if (li + 1 < c.num_layers && dense_chain_ok(li + 1)) {
                 pending_dense_tail = true;          // MLP output + residual + next input norm: the first role of the next layer's launch
                 tail_S = S; tail_rows_pad = rows_pad; tail_n_pad = n_pad;
@@ -1693,16 +1703,19 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             }
         } else {
             const int I = c.intermediate;
-            // 17–32 rows, one GPU: every projection of the MLP block writes fp32 split-K slabs (LDS-shared activations) and
-            // the consumer that exists anyway — add+norm, gated activation — sums them: no reduce launches.
+            // ≤ 32 rows, one GPU: the projections of the MLP block write fp32 split-K slabs (activations in LDS) and the consumer
+            // that exists anyway — add+norm, gated activation — sums them: no reduce launches (≤ 16 rows: gate_up applies its
+            // activation itself).
             // Tensor parallel (o / down row-parallel): the partial sums of the ranks meet in an all-reduce, so those two
             // projections produce fp16 partials (GEMM + reduce), all-reduce, then add + norm; the column-parallel gate_up keeps
             // its slabs → gated-activation form.  Everything stays stream-ordered device work, so the step is still one graph.
             const bool tp = c.tp_world > 1;
             // (act-order projections: every input of the chain arrives permuted from its producer — decode attention, the norms
             // below, gate_up's column order)
-            const bool slab_chain = m->dense_slabs && T > 16 && T <= 32 && (!L.o.perm || attn_perm) && (!L.down.perm || L.down.perm_folded) &&
-                                    L.o.qw && L.gate_up.qw && L.down.qw;   // INT4 slab kernels; unquantised projections take the op chain
+            const bool slab_chain = m->dense_slabs && T <= 32 && (!L.o.perm || attn_perm) && (!L.down.perm || L.down.perm_folded) &&
+                                    L.o.qw && L.gate_up.qw && L.down.qw &&   // INT4 slab kernels; unquantised projections take the op chain
+                                    (T > 16 || (!tp && w4_gemm_gated_supports(L.gate_up, T, I) && w4_gemm_rows_splits(L.o, T, m->workspace_bytes) &&
+                                                w4_gemm_rows_splits(L.down, T, m->workspace_bytes)));
             int S = 0, rows_pad = 0, n_pad = 0;
             if (slab_chain) {
                 form_hit(FORM_DENSE_SLAB_CHAIN);
@@ -1716,7 +1729,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
                     }
                 } else {
                 if (L.o.perm) form_hit(FORM_PERM_PRODUCER);
-                RUN(w4_gemm_dense_slabs_lds(L.o, m->attn_out, m->workspace, m->workspace_bytes, T, &S, &rows_pad, &n_pad, s));
+                RUN(dense_slabs_gemm(m, L.o, m->attn_out, T, &S, &rows_pad, &n_pad, s));
                 if (sandwich) {
                     RUN(sandwich_add_rms_norm_f32_slabs(m->workspace, S, (long)rows_pad * n_pad, n_pad, L.post_attn_ln, m->residual_f32,
                                                         L.post_ln, c.rms_eps, m->norm_out, T, H, s, gu_perm));
@@ -1727,10 +1740,13 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
                 }
                 if (gu_perm) form_hit(FORM_PERM_PRODUCER);
                 if (L.down.perm) form_hit(FORM_PERM_PRODUCER);
-                S = 0;
-                RUN(w4_gemm_dense_slabs_lds(L.gate_up, m->norm_out, m->workspace, m->workspace_bytes, T, &S, &rows_pad, &n_pad, s));
-                RUN(fused_gated_act_slabs_f16(m->workspace, S, (long)rows_pad * n_pad, n_pad, m->act_out, T, I, c.activation == 1, s));
-                S = 0;
+                if (T <= 16) {
+                    RUN(w4_gemm_gated(L.gate_up, m->norm_out, m->act_out, T, I, c.activation == 1, s));
+                } else {
+                    S = 0;
+                    RUN(w4_gemm_dense_slabs_lds(L.gate_up, m->norm_out, m->workspace, m->workspace_bytes, T, &S, &rows_pad, &n_pad, s));
+                    RUN(fused_gated_act_slabs_f16(m->workspace, S, (long)rows_pad * n_pad, n_pad, m->act_out, T, I, c.activation == 1, s));
+                }
                 if (tp) {
                     RUN(dense_linear(m, L.down, m->act_out, m->mlp_out, T, s));
                     if (sandwich) {
@@ -1743,7 +1759,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
                         RUN(add_inplace_f16(m->residual, m->mlp_out, (long)T * H, s));
                     }
                 } else {
-                RUN(w4_gemm_dense_slabs_lds(L.down, m->act_out, m->workspace, m->workspace_bytes, T, &S, &rows_pad, &n_pad, s));
+                RUN(dense_slabs_gemm(m, L.down, m->act_out, T, &S, &rows_pad, &n_pad, s));
                 if (sandwich) {
                     RUN(sandwich_add_rms_norm_f32_slabs(m->workspace, S, (long)rows_pad * n_pad, n_pad, L.post_ffn_ln, m->residual_f32,
                                                         next_ln, c.rms_eps, m->norm_out, T, H, s, next_qkv_perm));
@@ -1764,11 +1780,13 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             } else {
                 RUN(tp_all_reduce_add_rms_norm(m, m->o_out, m->residual, L.post_ln, c.rms_eps, m->norm_out, T, H, s, gu_perm));
             }
-            RUN(dense_linear(m, L.gate_up, m->norm_out, m->gate_up_out, T, s, true));
-            if (c.activation == 1) {
-                RUN(fused_gelu_tanh_mul_split_f16(m->gate_up_out, m->act_out, T, I, s));
+            if (w4_gemm_gated_supports(L.gate_up, T, I)) {
+                if (gu_perm) form_hit(FORM_PERM_PRODUCER);
+                RUN(w4_gemm_gated(L.gate_up, m->norm_out, m->act_out, T, I, c.activation == 1, s));
             } else {
-                RUN(fused_silu_mul_split_f16(m->gate_up_out, m->act_out, T, I, s));
+                RUN(dense_linear(m, L.gate_up, m->norm_out, m->gate_up_out, T, s, true));
+                if (c.activation == 1) { RUN(fused_gelu_tanh_mul_split_f16(m->gate_up_out, m->act_out, T, I, s)); }
+                else { RUN(fused_silu_mul_split_f16(m->gate_up_out, m->act_out, T, I, s)); }
             }
             RUN(dense_linear(m, L.down, m->act_out, m->mlp_out, T, s));
             if (sandwich) {

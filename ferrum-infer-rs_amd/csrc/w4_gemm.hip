@@ -180,6 +180,7 @@ struct W4Args {
     const __half* fa_ln;       // [K] norm weights
     float fa_eps;
     int fa_top_k;
+    int act_im, gelu;          // w4_gemm_wgsplit_kernel<…, GATED>: columns of the gate half, and which activation
 #ifdef FERRUM_HIP_EXPERIMENTS
     unsigned long long* tl;    // development: per-wave wall-clock stamps of the LDS-shared-activation kernel (tools/exp_timeline.py)
 #endif
@@ -1304,15 +1305,23 @@ __global__ void splitk_reduce_bias_kernel(const float* __restrict__ partial, __h
 // arithmetic of moe_combine_add_rmsnorm_kernel), x = rms_norm(residual')·ln — into LDS, after the first weight group has been
 // requested; workgroup 0 also stores residual'.  Every workgroup repeats the ≈ 36 KB per row of L2 reads: cheap at ≤ 4 rows,
 // prohibitive at 32, which is why only the small batches fuse.
-template <int MT, int NT, bool HAS_ZP, bool FUSE_A = false>
-__global__ __launch_bounds__(MT == 1 ? 1024 : (MT == 2 ? (NT == 1 ? 1024 : 512) : 256)) void w4_gemm_wgsplit_kernel(W4Args p) {
+// GATED (gate_up of a gated MLP): half of a workgroup's column tiles are gate columns, half the up columns that belong to them
+// (act_im columns on), so that act(gate)·up leaves the launch instead of both projections: no [rows, 2·im] round trip and one
+// dependent launch less.  Both are rounded to fp16 before, so the bits are those of the two launches.  4096→28672 at 5 / 12 rows
+// 13.1 / 14.5 µs against 12.6 / 14.0 + 5 for the activation, 5376→43008 22.9 / 26.0 against 22.3 / 25.8 + 5; within 128 registers
+// (1024 threads) 17.5 / 19.0, and with four tiles of each half, or the rows in LDS, 13.4 / 13.5 and 13.4 / 14.4 but 26 / 27.5 and too
+// much LDS for the wider one.
+template <int MT, int NT, bool HAS_ZP, bool FUSE_A = false, bool GATED = false>
+__global__ __launch_bounds__(MT == 1 ? (GATED ? 512 : 1024) : (MT == 2 ? (NT == 1 ? 1024 : 512) : 256)) void w4_gemm_wgsplit_kernel(W4Args p) {
     static_assert(!FUSE_A || MT == 1, "the fused prologue serves one 16-row tile");
+    static_assert(!GATED || (MT == 1 && NT > 1 && !FUSE_A), "gate and up tiles of one 16-row tile");
     extern __shared__ __attribute__((aligned(16))) float red[];
     const int W = blockDim.x >> 6;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
-    const int tile0 = blockIdx.x * NT;            // first 16-column tile of this workgroup
-    const int st = tile0 >> 2, nt0 = tile0 & 3;   // NT divides 4 → all tiles in one supertile
+    constexpr int NH = GATED ? NT / 2 : NT;       // neighbouring tiles (GATED: of each half)
+    const int tile0 = blockIdx.x * NH;            // first 16-column tile of this workgroup
+    const int st = tile0 >> 2, nt0 = tile0 & 3;   // NH divides 4 → all of them in one supertile
     const int rb = blockIdx.y;
     constexpr int V = MT * NT * 4;
 
@@ -1329,6 +1338,11 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : (MT == 2 ? (NT == 1 ? 1024 : 512) 
     const u32x4g* qw_lane = reinterpret_cast<const u32x4g*>(p.qw) + ((long)st * p.G * 4 + nt0) * 64 + lane;
     const uint2* sc_lane = reinterpret_cast<const uint2*>(p.sc) + ((long)st * p.G) * 16 + b;
     const uint2* zp_lane = HAS_ZP ? reinterpret_cast<const uint2*>(p.zp) + ((long)st * p.G) * 16 + b : nullptr;
+    // GATED: the up tiles, and the scales of both halves' tiles alone (act_im is a multiple of 16·NH, so they share a supertile too)
+    const int up0 = tile0 + (GATED ? p.act_im >> 4 : 0);
+    const u32x4g* qw_up = reinterpret_cast<const u32x4g*>(p.qw) + ((long)(up0 >> 2) * p.G * 4 + (up0 & 3)) * 64 + lane;
+    using Scales = std::conditional_t<NH == 2, uint32_t, uint16_t>;      // fp16 scales of NH tiles
+    const long s_gate = ((long)st * p.G * 16 + b) * 4 + nt0, s_up = ((long)(up0 >> 2) * p.G * 16 + b) * 4 + (up0 & 3);
 
     float4v acc[MT][NT];
 #pragma unroll
@@ -1338,9 +1352,20 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : (MT == 2 ? (NT == 1 ? 1024 : 512) 
 
     const int g0 = (int)((long)p.G * wave / W), g1 = (int)((long)p.G * (wave + 1) / W);
     u32x4g wq[2][NT];
-    uint2 scv[2], zpv[2];
+    uint2 scv[2], zpv[2];                         // (GATED: .x of the gate tiles, .y of the up tiles)
     half8 af[2][MT][4];
     auto issue_w = [&](int buf, int g) __attribute__((always_inline)) {
+        if constexpr (GATED) {
+#pragma unroll
+            for (int nt = 0; nt < NH; nt++) {
+                wq[buf][nt] = __builtin_nontemporal_load(qw_lane + ((long)g * 4 + nt) * 64);
+                wq[buf][NH + nt] = __builtin_nontemporal_load(qw_up + ((long)g * 4 + nt) * 64);
+            }
+            auto both = [&](const __half* t) { return uint2{*reinterpret_cast<const Scales*>(t + s_gate + (long)g * 64), *reinterpret_cast<const Scales*>(t + s_up + (long)g * 64)}; };
+            scv[buf] = both(p.sc);
+            if (HAS_ZP) zpv[buf] = both(p.zp);
+            return;
+        }
 #pragma unroll
         for (int nt = 0; nt < NT; nt++) wq[buf][nt] = __builtin_nontemporal_load(qw_lane + ((long)g * 4 + nt) * 64);
         scv[buf] = sc_lane[(long)g * 16];
@@ -1354,9 +1379,10 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : (MT == 2 ? (NT == 1 ? 1024 : 512) 
     };
     auto issue = [&](int buf, int g) __attribute__((always_inline)) { issue_w(buf, g); issue_a(buf, g); };
     auto consume = [&](int buf) {
-        const unsigned long long sb = ((unsigned long long)scv[buf].y << 32) | scv[buf].x;
-        const unsigned long long zb = HAS_ZP ? (((unsigned long long)zpv[buf].y << 32) | zpv[buf].x) : 0ull;
-        w4_consume_group<MT, NT, HAS_ZP, false>(wq[buf], sb, zb, nt0, af[buf], acc);
+        constexpr int UP = GATED ? 16 * NH : 32;
+        const unsigned long long sb = ((unsigned long long)scv[buf].y << UP) | scv[buf].x;
+        const unsigned long long zb = HAS_ZP ? (((unsigned long long)zpv[buf].y << UP) | zpv[buf].x) : 0ull;
+        w4_consume_group<MT, NT, HAS_ZP, false>(wq[buf], sb, zb, GATED ? 0 : nt0, af[buf], acc);
     };
 #define FH_PIN() __builtin_amdgcn_sched_barrier(0)
     if (FUSE_A) {
@@ -1447,6 +1473,23 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : (MT == 2 ? (NT == 1 ? 1024 : 512) 
 #pragma unroll
             for (int r = 0; r < 4; r++) red[((wave * V) + (mt * NT + nt) * 4 + r) * 64 + lane] = acc[mt][nt][r];
     __syncthreads();
+    if constexpr (GATED) {
+        for (int v = wave; v < V / 2; v += W) {
+            float g = 0.f, u = 0.f;
+            for (int w = 0; w < W; w++) {
+                g += red[(w * V + v) * 64 + lane];
+                u += red[(w * V + V / 2 + v) * 64 + lane];
+            }
+            const int row = 4 * a + (v & 3), col = (tile0 + (v >> 2)) * 16 + b;
+            if (row < p.M && col < p.act_im) {
+                if (p.bias) { g += __half2float(p.bias[col]); u += __half2float(p.bias[p.act_im + col]); }
+                g = (float)(_Float16)g;
+                u = (float)(_Float16)u;
+                reinterpret_cast<_Float16*>(p.out)[(long)row * p.ldo + col] = p.gelu ? gated_act<true>(g, u) : gated_act<false>(g, u);
+            }
+        }
+        return;
+    }
     for (int v = wave; v < V; v += W) {
         float sum = 0.f;
         for (int w = 0; w < W; w++) sum += red[(w * V + v) * 64 + lane];
@@ -1458,6 +1501,84 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : (MT == 2 ? (NT == 1 ? 1024 : 512) 
             p.out[(long)row * p.ldo + col] = __float2half(sum);
         }
     }
+}
+
+// ── dense GEMM for up to 16 rows into fp32 slabs: a workgroup's share of the activations RESIDENT in LDS ─────────────
+// The waves of w4_gemm_wgsplit_kernel read the activations of every column tile again: 4 KiB of 16-row fragments for each KiB of
+// weights where a workgroup has one tile, so that its time grows with the rows (14336→4096: 10.4 µs at 1 row, 14.5 at 12, 16.9 at 16)
+// while the weights stay the same.  Here a workgroup takes 128 columns and 1 / S of K: its rows of x come to LDS once (fragment-major,
+// one copy without registers), behind them the first weights, and after one barrier its eight waves — two tiles by half of its K
+// each — stream weights alone, two groups ahead; the halves meet in LDS and one slab of S leaves.  The consumer that exists anyway
+// (add + norm, the first role of the next layer's launch) sums the slabs in order.  S fills the chip with one round of workgroups.
+//   us, old → this with S slabs          1 row         5 rows        12 rows       16 rows
+//   14336→4096, S = 6                    10.4 →  8.4   10.8 →  8.8   14.5 →  9.4   16.9 →  9.7     (29 MB: 4.7 at 6.5 TB/s)
+//   21504→5376, S = 6                    24.3 → 12.5   26.2 → 13.1   37.5 → 14.1   44.7 → 14.7     (58 MB: 9.2)
+//    4096→5376, S = 6                     6.5 →  5.1    7.0 →  5.4    9.2 →  5.5   10.5 →  5.7
+// Four groups ahead instead of two, one tile a wave, or 64 columns a workgroup: 3 – 15 % slower.  A form with two row tiles for 17 – 32
+// rows lost to w4_gemm_ldsa_kernel (a step of 24 sequences 2.42 against 2.32 ms).
+constexpr int W4_ROWS_TILES = 8, W4_ROWS_LDS = 156 * 1024;
+template <bool HAS_ZP>
+__global__ __launch_bounds__(512) void w4_gemm_rows_kernel(W4Args p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    constexpr int NT = 2, TG = W4_ROWS_TILES / NT, KP = 8 / TG, DW = 2;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int a = lane >> 4, b = lane & 15;
+    const int z = blockIdx.y, G0 = (int)((long)p.G * z / p.S), Gs = (int)((long)p.G * (z + 1) / p.S) - G0;
+    const int tg = wave % TG, kp = wave / TG, tile0 = blockIdx.x * W4_ROWS_TILES + tg * NT, st = tile0 >> 2, nt0 = tile0 & 3;
+    const int g0 = G0 + Gs * kp / KP, g1 = G0 + Gs * (kp + 1) / KP, ng = g1 - g0;
+    // fragment f = group · 4 + k-step, 1 KiB each: lane (a, b) brings row b, k = 8a …
+    const __half* xr = p.x + (long)(b < p.M ? b : p.M - 1) * p.K + G0 * 128 + 8 * a;
+    for (int f = wave; f < Gs * 4; f += 8)
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xr + f * 32), (__attribute__((address_space(3))) void*)(lds + f * 1024), 16, 0, 0);
+    typedef uint32_t u32x4g __attribute__((ext_vector_type(4)));
+    // (a group past the wave's end, or a supertile past the last one, lies past the buffer's end: zeros, and no memory request)
+    const int end = st < p.n64 ? g1 : 0;
+    const __amdgpu_buffer_rsrc_t r_w = __builtin_amdgcn_make_buffer_rsrc((void*)(reinterpret_cast<const char*>(p.qw) + (long)st * p.G * 4096), 0, end * 4096, 0x00020000);
+    const __amdgpu_buffer_rsrc_t r_s = __builtin_amdgcn_make_buffer_rsrc((void*)(reinterpret_cast<const char*>(p.sc) + (long)st * p.G * 128), 0, end * 128, 0x00020000);
+    const __amdgpu_buffer_rsrc_t r_z = __builtin_amdgcn_make_buffer_rsrc((void*)(reinterpret_cast<const char*>(HAS_ZP ? p.zp : p.sc) + (long)st * p.G * 128), 0, end * 128, 0x00020000);
+    const int o_w = nt0 * 1024 + lane * 16, o_s = b * 8;
+    float4v acc[1][NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) acc[0][nt] = (float4v){0.f, 0.f, 0.f, 0.f};
+    u32x4g wq[DW][NT];
+    unsigned long long scv[DW], zpv[DW];
+    half8 af[1][4];
+    auto issue = [&](int slot, int g) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nt = 0; nt < NT; nt++) wq[slot][nt] = __builtin_bit_cast(u32x4g, __builtin_amdgcn_raw_buffer_load_b128(r_w, g * 4096 + o_w + nt * 1024, 0, 2));   // aux 2 = nontemporal
+        scv[slot] = __builtin_bit_cast(unsigned long long, __builtin_amdgcn_raw_buffer_load_b64(r_s, g * 128 + o_s, 0, 0));
+        zpv[slot] = HAS_ZP ? __builtin_bit_cast(unsigned long long, __builtin_amdgcn_raw_buffer_load_b64(r_z, g * 128 + o_s, 0, 0)) : 0ull;
+    };
+    auto consume = [&](int slot, int g) __attribute__((always_inline)) {
+        const half8* fr = reinterpret_cast<const half8*>(lds) + (size_t)(g - G0) * 4 * 64 + lane;
+#pragma unroll
+        for (int s = 0; s < 4; s++) af[0][s] = fr[s * 64];
+        w4_consume_group<1, NT, HAS_ZP, false>(wq[slot], scv[slot], zpv[slot], nt0, af, acc);
+    };
+#pragma unroll
+    for (int d = 0; d < DW; d++) issue(d, g0 + d);
+    __syncthreads();
+    int i = 0;
+    for (; i + DW <= ng; i += DW)
+#pragma unroll
+        for (int d = 0; d < DW; d++) {
+            consume(d, g0 + i + d);
+            issue(d, g0 + i + d + DW);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    if (i < ng) consume(0, g0 + i);
+    // the K halves meet in LDS: [half][tile][lane]
+    __syncthreads();
+    float4v* red = reinterpret_cast<float4v*>(lds);
+#pragma unroll
+    for (int nt = 0; nt < NT; nt++) red[(kp * W4_ROWS_TILES + tg * NT + nt) * 64 + lane] = acc[0][nt];
+    __syncthreads();
+    const int col = (blockIdx.x * W4_ROWS_TILES + wave) * 16 + b;      // eight tiles, eight waves
+    if (col >= p.n_pad) return;
+    const float4v v = red[wave * 64 + lane] + red[(W4_ROWS_TILES + wave) * 64 + lane];
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+        if (4 * a + r < p.M) p.partial[((long)z * p.rows_pad + 4 * a + r) * p.n_pad + col] = v[r];
 }
 
 // ── dense GEMM for 17–64 rows: activations staged ONCE per workgroup in LDS ───────────────────────
@@ -2579,6 +2700,10 @@ int w4_gemm_dense(const W4Device& w, const __half* x, __half* out, int m, float*
     // column tiles per workgroup: as wide as possible (A-fragment reuse) while ≥ ~384 workgroups exist
     int nt = 4;
     while (nt > 1 && (long)cdiv(n16, nt) * row_blocks < 384) nt >>= 1;
+    // … but one row tile takes two column tiles rather than one where those are more than a round of 256 workgroups: every tile reads
+    // the rows again (5376→8192 at 5 / 12 rows 8.9 → 7.0 / 11.6 → 8.3 µs, 4096→6144 7.0 → 5.6 / 9.2 → 6.6, 2048→5120 4.8 → 3.8 / 5.9
+    // → 4.4); 4096→4096 keeps one: 4.9 / 6.1 against 5.3 / 6.5
+    if (mt == 1 && nt == 1 && (long)n16 * row_blocks > 256) nt = 2;
     // with ≥ 2 row tiles the activation fragments dominate the load traffic: share each across two
     // column tiles as long as ≥ 128 workgroups remain (measured: qkv 2048→5120 at T=32 10.4 → 7.2 µs)
     if (mt >= 2 && nt == 1 && (long)cdiv(n16, 2) * row_blocks >= 128) nt = 2;
@@ -2838,6 +2963,69 @@ int w4_gemm_dense_slabs_tile(const W4Device& w, const __half* x, float* slabs, s
     *n_pad_out = a.n_pad;
     form_hit(FORM_W4_SLABS_TILE);
     return launch_tilep(a, w.zp != nullptr, dim3(cols, rts, S), stream);
+}
+
+// Splits of K with which w4_gemm_rows takes this projection, 0 where it does not: one round of workgroups over the chip, at least half
+// of it (with fewer columns w4_gemm_wgsplit_kernel has the more workgroups), a workgroup's share of the rows within LDS.  Six slabs at
+// most: eight make the launch of 14336→4096 shorter (9.4 → 8.9 µs at 12 rows), but what sums them longer: a decode step of 32 layers
+// took 1867 µs with eight, 1825 with six, 1841 with four (4 sequences: 1641, 1632, 1703).
+int w4_gemm_rows_splits(const W4Device& w, int m, size_t slab_bytes) {
+    if (m < 1 || m > 16 || !w.qw || w.bias) return 0;
+    const int cols = cdiv(w.n64, W4_ROWS_TILES / 4);
+    const int S = std::min({256 / cols, 6, w.G});
+    if (S < 1 || cols * S < 128 || cdiv(w.G, S) * 4096 > W4_ROWS_LDS) return 0;
+    return (size_t)S * 16 * w.n64 * 64 * sizeof(float) <= slab_bytes ? S : 0;
+}
+
+int w4_gemm_rows(const W4Device& w, const __half* x, float* slabs, size_t slab_bytes, int m, int* S_out, int* rows_pad_out, int* n_pad_out,
+                 hipStream_t stream) {
+    const int S = w4_gemm_rows_splits(w, m, slab_bytes);
+    FH_REQUIRE(S > 0, "w4_gemm_rows: m=%d K=%d N=%d is not one of its projections", m, w.k, w.n);
+    W4Args a{};
+    a.qw = w.qw; a.sc = w.sc; a.zp = w.zp;
+    a.x = x; a.M = m; a.K = w.k; a.N = w.n; a.G = w.G; a.n64 = w.n64; a.ldo = w.n; a.S = S;
+    *S_out = S;
+    *rows_pad_out = a.rows_pad = 16;
+    *n_pad_out = a.n_pad = w.n64 * 64;
+    a.partial = slabs;
+    form_hit(FORM_W4_ROWS);
+    const size_t lds = (size_t)1024 * std::max(cdiv(w.G, S) * 4, 2 * W4_ROWS_TILES);
+    const dim3 grid(cdiv(w.n64, W4_ROWS_TILES / 4), S);
+    auto go = [&](auto kernel) -> int {
+        FH_CHECK_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, W4_ROWS_LDS));
+        hipLaunchKernelGGL(kernel, grid, dim3(512), lds, stream, a);
+        FH_CHECK_LAUNCH();
+        return 0;
+    };
+    return w.zp ? go(w4_gemm_rows_kernel<true>) : go(w4_gemm_rows_kernel<false>);
+}
+
+// gate_up and its activation in one launch: up to 16 rows of an INT4 projection whose halves are whole column tiles
+bool w4_gemm_gated_supports(const W4Device& w, int m, int im) {
+    return m >= 1 && m <= 16 && w.qw && w.n == 2 * im && im % 32 == 0;
+}
+
+int w4_gemm_gated(const W4Device& w, const __half* x, __half* out, int m, int im, int gelu, hipStream_t stream) {
+    FH_REQUIRE(w4_gemm_gated_supports(w, m, im), "w4_gemm_gated: m=%d N=%d intermediate=%d", m, w.n, im);
+    W4Args a{};
+    a.qw = w.qw; a.sc = w.sc; a.zp = w.zp; a.bias = w.bias;
+    a.x = x; a.out = out; a.M = m; a.K = w.k; a.N = w.n; a.G = w.G; a.n64 = w.n64; a.ldo = im; a.S = 1;
+    a.act_im = im; a.gelu = gelu;
+    // tiles as for the plain projection (w4_gemm_dense), but at least a gate and an up tile, and four waves where those are enough
+    // (eight: 4096→28672 14.1 µs against 13.1; 2048→12288, a third of the workgroups, 5.3 against 5.8)
+    const int n16 = w.n / 16, nt = cdiv(n16, 4) >= 384 ? 4 : 2;
+    const long wgs = n16 / nt;
+    int W = 4;
+    while (wgs * W < 1024 && W * 2 <= std::min(8, w.G)) W <<= 1;
+    while (W > w.G && W > 1) W >>= 1;
+    form_hit(FORM_W4_GATED);
+    auto go = [&](auto kernel) -> int {
+        hipLaunchKernelGGL(kernel, dim3(wgs), dim3(W * 64), (size_t)W * nt * 4 * 64 * sizeof(float), stream, a);
+        FH_CHECK_LAUNCH();
+        return 0;
+    };
+    if (nt == 4) return w.zp ? go(w4_gemm_wgsplit_kernel<1, 4, true, false, true>) : go(w4_gemm_wgsplit_kernel<1, 4, false, false, true>);
+    return w.zp ? go(w4_gemm_wgsplit_kernel<1, 2, true, false, true>) : go(w4_gemm_wgsplit_kernel<1, 2, false, false, true>);
 }
 
 // Split count the LDS-shared-activation kernel wants for this shape (tools/exp_dense.py sweeps): enough workgroups to

@@ -84,6 +84,26 @@ def test_asymmetric_act_order_checkpoint_style(pkg, prompt_len, style, forms):
     forms.require("perm_producer", absent=("gather_columns",))                                                       # decode: none
 
 
+@pytest.mark.parametrize("kw,rows", [
+    (dict(hidden=2944, inter=1152, nq=8, nkv=2), True),                                            # the fewest columns of the resident form; 1 – 2 groups a slab
+    (dict(hidden=3072, inter=2176, nq=24, nkv=8, sandwich=True, activation=1, embed_scale=4.0), True),   # 17 groups in 6 slabs, GELU
+    (dict(hidden=3072, inter=768, nq=8, nkv=8, asym_act_order=True), True),                        # zero points, rows permuted by their producers
+    (dict(hidden=2816, inter=1152, nq=8, nkv=2), True),                                            # 22 column blocks: 132 workgroups
+    (dict(hidden=2560, inter=640, nq=8, nkv=2), False),                                            # 20: too few
+    (dict(hidden=1024, inter=12288, nq=8, nkv=2), False),                                          # two gate and two up tiles a workgroup
+    (dict(hidden=512, inter=12544, nq=4, nkv=2, asym_act_order=True, activation=1, sandwich=True, embed_scale=4.0), False),
+], ids=lambda kw: "-".join(f"{k}{v}" for k, v in kw.items()) if isinstance(kw, dict) else str(kw))
+@pytest.mark.parametrize("prompt_len", [1, 5, 16])
+def test_few_rows_resident_projections_and_gated_gate_up(pkg, prompt_len, kw, rows, forms):
+    """o_proj and down with their rows resident in LDS, and gate_up with its activation, at the edges of both and of the 16 rows."""
+    from tests import modelgen
+    forms.reset()
+    res = modelgen.run_parity_case(pkg, moe=False, layers=2, prompt_len=prompt_len, decode_steps=2, seed=400 + prompt_len, hd=128, **kw)
+    _assert_parity(res)
+    h = forms.require("w4_gated")
+    assert bool(h.get("w4_rows")) == rows, h
+
+
 @pytest.mark.parametrize("prompt_len", [9, 70])
 def test_act_order_attention_projections_in_a_moe_model(pkg, prompt_len, forms):
     """A MoE checkpoint whose ATTENTION projections are desc_act packs (the expert stacks are natural order here; act-order
