@@ -33,6 +33,12 @@ template <> struct Frag<_Float16> {
 template <> struct Frag<float> {
     typedef floatx8 v8;
     typedef floatx4 v4;
+    // 16 bytes of a lane: four of its eight k
+    static __device__ __forceinline__ floatx4 mma(v4 a, v4 b, floatx4 c) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
+        return c;
+    }
     static __device__ __forceinline__ floatx4 mma(v8 a, v8 b, floatx4 c) {
 #pragma unroll
         for (int j = 0; j < 8; j++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);

@@ -208,16 +208,17 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(TiledGemm<E> p, int kw)
     }
 }
 
-// Prompts, 16-bit: 2 × 2 waves hold MI × NJ tiles of 16 × 16 each.  Both operands go through LDS, copied there by the load unit itself:
-//  * weights in stages of 32 of K, a ring of 2G − 1; a fragment (16 columns × 32 of K) is one 1-KiB load in lane order;
-//  * rows in granules of 64 of K, a ring of G; a load takes 128 bytes (a cache line) of each of 8 rows, and the 16-byte pieces of row r lie in
-//    the order 0 … 7 xor r, so that the 16 lanes that read one piece of 16 rows touch every bank alike.
+// Prompts: 2 × 2 waves hold MI × NJ tiles of 16 × 16 each.  Both operands go through LDS, copied there by the load unit itself:
+//  * weights in stages of one k-step, a ring of 2G − 1: 16 bytes of every lane of a fragment.  In 16 bits that is 32 of K, one 1-KiB load in
+//    lane order; in 32 bits half of a fragment, 16 of K (the first or the last four of every lane's eight);
+//  * rows in granules of two steps, a ring of G; a load takes 128 bytes (a cache line) of each of 8 rows, and the 16-byte pieces of row r lie
+//    in the order 0 … 7 xor r, so that the 16 lanes that read one piece of 16 rows touch every bank alike.
 __device__ const uint16_t zero_fragment[512] = {};
 template <int MI, int NJ, int G>
 struct BigTile {
     static constexpr int RT = 2 * MI, CT = 2 * NJ, ROWS = 16 * RT, COLS = 16 * CT, STAGES = 2 * G - 1;
-    static constexpr int GRANULE = RT * 1024, STAGE = CT * 512;         // elements
-    static constexpr size_t LDS = ((size_t)G * GRANULE + STAGES * STAGE) * 2;
+    static constexpr int GRANULE = RT * 2048, STAGE = CT * 1024;        // bytes
+    static constexpr size_t LDS = (size_t)G * GRANULE + STAGES * STAGE;
     static_assert(MI % 2 == 0 && (NJ == 2 || NJ == 4 || NJ == 8), "every wave copies whole fragments");
     static_assert(LDS >= (size_t)4 * 32 * (16 * NJ + 4) * 4, "the epilogue's rows fit the stages");
 };
@@ -225,8 +226,11 @@ template <typename E, int MI, int NJ, int G, int PER_CU>
 __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E> p, int mtiles, int ntiles) {
     typedef BigTile<MI, NJ, G> T;
     typedef typename Frag<E>::v8 v8;
+    constexpr bool HALVES = sizeof(E) == 4;
+    constexpr int EP = 16 / sizeof(E), SK = 4 * EP;                     // elements of 16 bytes, K of a step
+    typedef std::conditional_t<HALVES, typename Frag<E>::v4, v8> operand;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    E *const rows_lds = reinterpret_cast<E*>(smem), *const w_lds = rows_lds + G * T::GRANULE;
+    unsigned char *const rows_lds = smem, *const w_lds = rows_lds + G * T::GRANULE;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
     // workgroups go round-robin over 8 XCDs: give each XCD a contiguous run of tiles, and walk 8 row tiles per column tile
@@ -237,7 +241,7 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     const int id = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + l / 8;
     const int band = id / (8 * ntiles), rows_in = min(8, mtiles - band * 8), in_band = id - band * 8 * ntiles;
     const int mt = band * 8 + in_band % rows_in, m0 = mt * T::ROWS, n0 = (in_band / rows_in) * T::COLS;
-    const int n = p.k >> 5, ntl = p.n >> 4, g = p.rows.id ? p.rows.group[m0 / p.rows.block] : blockIdx.z;
+    const int n = p.k / SK, ntl = p.n >> 4, g = p.rows.id ? p.rows.group[m0 / p.rows.block] : blockIdx.z;
     const int wm = wave >> 1, wn = wave & 1;
     // this wave's loads: MI of a granule (8 rows each), NJ / 2 of a weight stage
     const E *ap[MI], *bp[NJ / 2];
@@ -245,23 +249,23 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
 #pragma unroll
     for (int i = 0; i < MI; i++) {
         const int r = (MI * wave + i) * 8 + (lane >> 3);
-        ap[i] = gemm_row(p, (m0 + r) >> 4, g, piece, r & 15);
+        ap[i] = HALVES ? gemm_row(p, (m0 + r) >> 4, g, piece >> 1, r & 15) + 4 * (piece & 1) : gemm_row(p, (m0 + r) >> 4, g, piece, r & 15);
     }
 #pragma unroll
     for (int i = 0; i < NJ / 2; i++) {
         const int t = (n0 >> 4) + NJ / 2 * wave + i;
-        bp[i] = p.w + ((long)g * ntl + (t < ntl ? t : ntl - 1)) * n * 512 + lane * 8;
+        bp[i] = p.w + ((long)g * ntl + (t < ntl ? t : ntl - 1)) * (p.k >> 5) * 512 + lane * 8;
     }
-    const int xs = 2 * gemm_row_step(p);
-    const E* none = reinterpret_cast<const E*>(zero_fragment) + lane * 8;        // (past the end of K)
+    const int xs = (HALVES ? 1 : 2) * gemm_row_step(p);
+    const E* none = reinterpret_cast<const E*>(zero_fragment) + lane * EP;       // (past the end of K)
 #define BIG_COPY(src, dst) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src), (__attribute__((address_space(3))) void*)(dst), 16, 0, 0)
     auto issue_rows = [&](int i, int place, bool in) {
-        BIG_COPY(in ? ap[i] : none, rows_lds + place * T::GRANULE + (MI * wave + i) * 512);
+        BIG_COPY(in ? ap[i] : none, rows_lds + place * T::GRANULE + (MI * wave + i) * 1024);
         ap[i] += xs;
     };
-    auto issue_w = [&](int i, int place, bool in) {
-        BIG_COPY(in ? bp[i] : none, w_lds + place * T::STAGE + (NJ / 2 * wave + i) * 512);
-        bp[i] += 512;
+    auto issue_w = [&](int i, int place, bool in, bool second) {        // (second: of a fragment's halves)
+        BIG_COPY(in ? bp[i] : none, w_lds + place * T::STAGE + (NJ / 2 * wave + i) * 1024);
+        bp[i] += !HALVES ? 512 : second ? 508 : 4;
     };
 #undef BIG_COPY
     floatx4 acc[MI][NJ];
@@ -269,16 +273,18 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     for (int i = 0; i < MI; i++)
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = (floatx4){0.f, 0.f, 0.f, 0.f};
-    struct Operands { v8 x[MI], w[NJ]; };
+    // 32 bits: sums of 512 products, then sums of those (the few-row kernel's parts of K are as short; one chain over K = 6144 errs by 1.3 times)
+    floatx4 sum[HALVES ? MI : 1][HALVES ? NJ : 1] = {};
+    struct Operands { operand x[MI], w[NJ]; };
     constexpr int READS = MI + NJ;
-    const E* my_w = w_lds + wn * NJ * 512 + lane * 8;
-    const E* my_rows[2];
+    const unsigned char* my_w = w_lds + wn * NJ * 1024 + lane * 16;
+    const unsigned char* my_rows[2];
 #pragma unroll
-    for (int h = 0; h < 2; h++) my_rows[h] = rows_lds + wm * MI * 1024 + b * 64 + ((4 * h + a) ^ (b & 7)) * 8;
+    for (int h = 0; h < 2; h++) my_rows[h] = rows_lds + wm * MI * 2048 + b * 128 + ((HALVES ? 2 * a + h : 4 * h + a) ^ (b & 7)) * 16;
     // fragment f of a k-step: half h of the granule at `gran`, the weight stage at `stage`
     auto read = [&](Operands& o, int f, int h, int gran, int stage) {
-        if (f < NJ) o.w[f] = *reinterpret_cast<const v8*>(my_w + stage * T::STAGE + f * 512);
-        else o.x[f - NJ] = *reinterpret_cast<const v8*>(my_rows[h] + gran * T::GRANULE + (f - NJ) * 1024);
+        if (f < NJ) o.w[f] = *reinterpret_cast<const operand*>(my_w + stage * T::STAGE + f * 1024);
+        else o.x[f - NJ] = *reinterpret_cast<const operand*>(my_rows[h] + gran * T::GRANULE + (f - NJ) * 2048);
     };
     // every load but this wave's last `left` has arrived, for all waves
 #define BIG_WAIT(left)                                                          \
@@ -300,12 +306,12 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
         constexpr bool ODD = decltype(odd)::value;
         constexpr int LOADS = NJ / 2 + (ODD ? MI : 0), PER = MI * NJ / (READS + READS / 4);
         BIG_WAIT((T::STAGES - 2) * (NJ / 2) + (ODD ? G - 2 : G - 1) * MI);
-        const bool in = t + T::STAGES < n, rows_in_k = 32 * (t + T::STAGES) + 8 * piece < p.k;
+        const bool in = t + T::STAGES < n, rows_in_k = SK * (t + T::STAGES) + EP * piece < p.k;
         const int to = stage_after(stage), from = ODD ? granule_after(gran) : gran;
 #pragma unroll
         for (int q = 0; q <= READS; q++) {
             if (q < READS) read(then, q, ODD ? 0 : 1, from, to);
-            if (q < NJ / 2) issue_w(q, stage, in);
+            if (q < NJ / 2) issue_w(q, stage, in, !ODD);          // (2G − 1 steps on: the other half)
             else if (ODD && q < LOADS) issue_rows(q - NJ / 2, gran, rows_in_k);
 #pragma unroll
             for (int m = q * PER; m < (q < READS ? (q + 1) * PER : MI * NJ); m++) acc[m / NJ][m % NJ] = Frag<E>::mma(now.w[m % NJ], now.x[m / NJ], acc[m / NJ][m % NJ]);
@@ -316,10 +322,10 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
 #pragma unroll
     for (int i = 0; i < T::STAGES; i++) {
 #pragma unroll
-        for (int f = 0; f < NJ / 2; f++) issue_w(f, i, i < n);
+        for (int f = 0; f < NJ / 2; f++) issue_w(f, i, i < n, i % 2 == 1);
         if (i % 2 == 0) {
 #pragma unroll
-            for (int f = 0; f < MI; f++) issue_rows(f, i / 2, 32 * i + 8 * piece < p.k);
+            for (int f = 0; f < MI; f++) issue_rows(f, i / 2, SK * i + EP * piece < p.k);
         }
     }
     Operands even, odd;
@@ -333,6 +339,14 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
         step(odd, even, std::true_type{}, t + 1, stage, gran);
         stage = stage_after(stage);
         gran = granule_after(gran);
+        if (HALVES && ((t & 30) == 30 || t + 2 >= n))
+#pragma unroll
+            for (int i = 0; i < MI; i++)
+#pragma unroll
+                for (int j = 0; j < NJ; j++) {
+                    sum[i][j] += acc[i][j];
+                    acc[i][j] = t + 2 >= n ? sum[i][j] : (floatx4){0.f, 0.f, 0.f, 0.f};
+                }
     }
 #undef BIG_WAIT
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                    // (the requests past the end have landed: the epilogue reuses the ring)
@@ -434,11 +448,26 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
 template <typename E>
 static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
     auto tiles = [&](int r, int c) { return (long)(g.rows.id ? g.rows.max_blocks * (g.rows.block / r) : cdiv(g.m, r)) * cdiv(g.n, c) * g.groups; };
-    if (tiles(128, 256) >= knobs().tiled_wide_min_tiles) return launch_big<E, 4, 8, 2, 2>(g, s);
-    if (tiles(128, 128) > knobs().tiled_half_max_tiles) return launch_big<E, 4, 4, 2, 2>(g, s);
-    return tiles(128, 64) > 160 ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 2, 2, 3, 3>(g, s);
+    if constexpr (sizeof(E) == 4) {
+        // 32 bits: bound by the products alone, so the tile whose rounds over the CUs take least (µs of a round below, K = 2048; the few-row
+        // kernel, which reads both operands from L2 for every 64 × 32 outputs, is left at 75 TFLOP/s of the 154 of a large product):
+        //                        128 × 128   128 × 64   64 × 64   few-row kernel
+        //   2048 × 2048 × 2048      136         141                  222
+        //   1000 × 6144 × 2048      256         209                  330
+        //   1000 × 2048 × 2048      134          76                  115
+        //   500 × 2048 × 2048       133                    46         62
+        //   1000 × 1024 × 512        39                    15         19
+        //   128 × 8192 × 2048       133                    47         63
+        //   256 × 2048 × 2048       133                    44         39      (128 tiles: too few)
+        const long full = cdiv(tiles(128, 128), 256) * 133L, half = cdiv(tiles(128, 64), 256) * 72L, small = cdiv(tiles(64, 64), 256) * 42L;
+        if ((g.rows.id && g.rows.block < 128) || small < std::min(full, half)) return launch_big<E, 2, 2, 3, 3>(g, s);
+        return half < full ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 4, 4, 2, 2>(g, s);
+    } else {
+        if (tiles(128, 256) >= knobs().tiled_wide_min_tiles) return launch_big<E, 4, 8, 2, 2>(g, s);
+        if (tiles(128, 128) > knobs().tiled_half_max_tiles) return launch_big<E, 4, 4, 2, 2>(g, s);
+        return tiles(128, 64) > 160 ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 2, 2, 3, 3>(g, s);
+    }
 }
-template <> int launch_big<float>(const TiledGemm<float>&, hipStream_t) { return 2; }      // (never taken: 16-bit only)
 
 int tiled_gemm_slabs(int m, int n, int k) {
     if (m > 64) return 1;
@@ -479,8 +508,10 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
                    "tiled_gemm: sorted rows take plain sections");
         FH_REQUIRE(rows.block == 16 || rows.block == 32 || rows.block == 64 || ((rows.block == 128 || rows.block == 256) && sizeof(E) == 2), "tiled_gemm: blocks of %d rows", rows.block);
     }
-    const long tiles = (long)cdiv(g.m, 64) * cdiv(g.n, 64) * g.groups;
-    if (rows.id ? rows.block >= 128 : sizeof(E) == 2 && g.m > 64 && g.n >= 64 && g.slabs == 1 && tiles >= knobs().tiled_big_min_tiles) return launch_big(g, s);
+    constexpr bool F32 = sizeof(E) == 4;
+    const long tiles = (rows.id ? (long)rows.max_blocks * (rows.block / 64) : cdiv(g.m, 64)) * cdiv(g.n, 64) * g.groups;
+    const bool enough_tiles = tiles >= knobs().tiled_big_min_tiles * (F32 ? 5L : 4L) / 4;
+    if (rows.id ? (F32 ? rows.block >= 64 && g.n >= 64 && enough_tiles : rows.block >= 128) : g.m > 64 && g.n >= 64 && g.slabs == 1 && enough_tiles) return launch_big(g, s);
     // rows per workgroup: as many as there are, fewer where narrow outputs would leave CUs idle
     int mt = rows.id ? rows.block / 16 : g.m <= 16 ? 1 : (g.m <= 32 ? 2 : 4);
     while (!rows.id && mt > 1 && (long)cdiv(g.m, 16 * mt) * (g.n / 16) * g.groups * g.slabs < knobs().tiled_min_tiles) mt /= 2;

@@ -485,6 +485,30 @@ def test_few_row_and_tile_projections_agree(pkg, cases, knobs, forms, name):
         assert h.get(ran) and bool(h.get("tiled_gemm_big")) == (big == 1) and bool(h.get("tiled_gemm_256")) == (wide == 1)
 
 
+@pytest.mark.parametrize("name", ["wide", "shared", "sinks", "loop", "talks"])
+@pytest.mark.parametrize("big", [1, 10 ** 6])
+def test_32_bit_projections_of_prompts(pkg, cases, knobs, forms, name, big):
+    """64 × 64 tiles against the few-row kernel's oracle, whatever the projections' sizes."""
+    cfg, w, path = cases(name)
+    t = toks(cfg, 200, 12)
+    knobs.set(TILED_BIG_MIN_TILES=big)
+    m = load(pkg, path, "float32")
+    forms.reset()
+    assert rel(feed(m, 1, t, [200]), L.forward(cfg, w, t)) < TOL["float32"]
+    assert bool(forms.hits().get("tiled_gemm_big")) == (big == 1)
+
+
+@pytest.mark.parametrize("tokens,ff", [(700, 1024), (700, 1025), (2000, 1024), (1921, 1090)])
+def test_32_bit_tile_sizes(pkg, tmp_path, forms, tokens, ff):
+    """128 × 64 and 128 × 128 tiles, one k-step or two, rows and columns past the last tile."""
+    cfg = G.config(64, 80, [G.attention(2, 8, 6, 8, 20, 16, 40, ff=ff)], buckets=13)
+    w, t = G.weights(cfg, 31), toks(cfg, tokens, 9)
+    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), "float32", tokens=2048)
+    forms.reset()
+    assert rel(feed(m, 1, t, [tokens]), L.forward(cfg, w, t)) < TOL["float32"]
+    assert forms.hits().get("tiled_gemm_big")
+
+
 def test_missing_and_misshapen_weights_are_named(pkg, tmp_path):
     cfg = G.CONFIGS["tiny"]
     w = G.weights(cfg, 1)

@@ -116,6 +116,17 @@ def test_experts_in_every_tile_size(pkg, tmp_path, forms, knobs, wide, half, blo
     assert h.get("tiled_gemm_grouped_big") and bool(h.get("tiled_gemm_256")) == (wide == 1)
 
 
+@pytest.mark.parametrize("n,top,tokens,ff,width", [(4, 2, 400, 48, 160), (9, 3, 110, 70, 320), (6, 1, 200, 250, 96), (3, 2, 300, 33, 64)])
+def test_experts_in_32_bit_tiles(pkg, tmp_path, forms, knobs, n, top, tokens, ff, width):
+    """Sorted rows in tiles of 64 × 64: fewer k-steps than the ring holds, columns past the last tile, experts that receive few rows."""
+    knobs.set(MOE_ROWS_BLOCK=64, TILED_BIG_MIN_TILES=1)
+    cfg = model([G.sink_attention(2, 8, 4, 8, 16, mlp=G.experts(n, top, ff))], width=width)
+    w = G.weights(cfg, 46)
+    silence(w, "mix.o", "side.norm")
+    agree(pkg, tmp_path, cfg, w, "float32", n=tokens)
+    assert forms.hits().get("tiled_gemm_grouped_big")
+
+
 def test_experts_beside_the_mixer(pkg, cases, knobs):
     """Small batches run the experts on a stream of their own: the same ids as in one stream, eagerly and over many replays of the graph
     with eager work between them."""
