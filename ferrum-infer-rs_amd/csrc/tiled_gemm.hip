@@ -273,7 +273,8 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     for (int i = 0; i < MI; i++)
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = (floatx4){0.f, 0.f, 0.f, 0.f};
-    // 32 bits: sums of 512 products, then sums of those (the few-row kernel's parts of K are as short; one chain over K = 6144 errs by 1.3 times)
+    // 32 bits: sums of 128 products, then sums of those, as short as the few-row kernel's parts of K ever are.  Relative error against 64 bits
+    // at K = 512 / 2048 / 6144: 2.1 / 2.2 / 2.4e-7, with sums of 512 4.0 / 4.0 / 4.1e-7 and 2 % faster, the few-row kernel 2.1 / 4.0 / 7.0e-7.
     floatx4 sum[HALVES ? MI : 1][HALVES ? NJ : 1] = {};
     struct Operands { operand x[MI], w[NJ]; };
     constexpr int READS = MI + NJ;
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
         step(odd, even, std::true_type{}, t + 1, stage, gran);
         stage = stage_after(stage);
         gran = granule_after(gran);
-        if (HALVES && ((t & 30) == 30 || t + 2 >= n))
+        if (HALVES && ((t & 6) == 6 || t + 2 >= n))
 #pragma unroll
             for (int i = 0; i < MI; i++)
 #pragma unroll
@@ -452,13 +453,13 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
         // 32 bits: bound by the products alone, so the tile whose rounds over the CUs take least (µs of a round below, K = 2048; the few-row
         // kernel, which reads both operands from L2 for every 64 × 32 outputs, is left at 75 TFLOP/s of the 154 of a large product):
         //                        128 × 128   128 × 64   64 × 64   few-row kernel
-        //   2048 × 2048 × 2048      136         141                  222
-        //   1000 × 6144 × 2048      256         209                  330
-        //   1000 × 2048 × 2048      134          76                  115
-        //   500 × 2048 × 2048       133                    46         62
-        //   1000 × 1024 × 512        39                    15         19
-        //   128 × 8192 × 2048       133                    47         63
-        //   256 × 2048 × 2048       133                    44         39      (128 tiles: too few)
+        //   2048 × 2048 × 2048      142         147                  222
+        //   1000 × 6144 × 2048      266         215                  330
+        //   1000 × 2048 × 2048      140          83                  115
+        //   500 × 2048 × 2048       139                    50         62
+        //   1000 × 1024 × 512        41                    17         19
+        //   128 × 8192 × 2048       139                    50         63
+        //   256 × 2048 × 2048       138                    47         39      (128 tiles: too few)
         const long full = cdiv(tiles(128, 128), 256) * 133L, half = cdiv(tiles(128, 64), 256) * 72L, small = cdiv(tiles(64, 64), 256) * 42L;
         if ((g.rows.id && g.rows.block < 128) || small < std::min(full, half)) return launch_big<E, 2, 2, 3, 3>(g, s);
         return half < full ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 4, 4, 2, 2>(g, s);
