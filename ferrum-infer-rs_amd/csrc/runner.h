@@ -142,7 +142,7 @@ struct FerrumHipModel {
     uint8_t* idx_dev = nullptr;
 
     // decode-steps state
-    uint32_t* history = nullptr;   // [max_steps, max_seqs] device
+    uint32_t* history = nullptr;   // [steps, sequences] sampled ids, pinned: written by the steps, read by the host
     int history_cap = 0;
     int32_t* step_counter = nullptr;
     hipGraph_t graph = nullptr;

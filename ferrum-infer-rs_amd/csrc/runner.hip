@@ -119,10 +119,22 @@ __global__ void decode_advance_kernel(const uint32_t* __restrict__ sampled, uint
         tokens[i] = t;
         pos_offsets[i] += 1;
         kv_lens[i] += 1;
-        history[(long)step * n + i] = t;
+        __hip_atomic_store(&history[(long)step * n + i], t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     __syncthreads();
     if (i == 0) *step_counter = step + 1;
+}
+
+// What a decode call hands over: the used parts of the pinned index block, read from there, and the step index and ticket at zero.  One
+// launch in place of a copy of the whole block, whose places for prompt tokens a decode step does not use, and a fill; the sampled ids
+// are written where the host reads them.  A call of one step costs 16 – 29 µs more than a step of a long call; with the copies, and one
+// of the ids into pageable memory, 30 – 64 µs.
+struct IndexParts { int n = 0, word[10], words[10]; };
+__global__ __launch_bounds__(256) void decode_begin_kernel(const uint32_t* __restrict__ host, uint32_t* __restrict__ dev, IndexParts p, int32_t* __restrict__ step_counter) {
+    const int w0 = p.word[blockIdx.y], n = p.words[blockIdx.y];
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
+        dev[w0 + i] = __hip_atomic_load(host + w0 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 2) step_counter[threadIdx.x] = 0;
 }
 
 __global__ void f16_to_f32_kernel(const __half* __restrict__ src, float* __restrict__ dst, long n) {
@@ -438,12 +450,13 @@ int ferrum_hip_model_destroy(FerrumHipModel* m) {
                     (void*)m->sampled_hidden, (void*)m->moe_act, (void*)m->moe_down, (void*)m->moe_gather_x, (void*)m->moe_gather_h, (void*)m->router_logits,
                     (void*)m->expert_ids, (void*)m->sorted_ids, (void*)m->block_ids, (void*)m->total_post_pad,
                     (void*)m->expert_w, (void*)m->logits, (void*)m->out_tokens, (void*)m->workspace, (void*)m->taps,
-                    (void*)m->idx_dev, (void*)m->history, (void*)m->step_counter, (void*)m->residual2, (void*)m->chain_o_part, (void*)m->chain_attn_partial, (void*)m->chain_attn_tickets,
+                    (void*)m->idx_dev, (void*)m->step_counter, (void*)m->residual2, (void*)m->chain_o_part, (void*)m->chain_attn_partial, (void*)m->chain_attn_tickets,
                     (void*)m->route_cand, (void*)m->route_stats, (void*)m->route_arrive, (void*)m->cos_local,
                     (void*)m->sin_local, (void*)m->residual_f32, (void*)m->gather_scratch, (void*)m->greedy_opts_dev, (void*)m->tp_tmp,
                     (void*)m->expert_ids_local, (void*)m->ones, m->vp_pairs, m->vp_gathered})
         if (p) (void)hipFree(p);
     if (m->idx_host) (void)hipHostFree(m->idx_host);
+    if (m->history) (void)hipHostFree(m->history);
     if (m->inlaunch_timeouts) (void)hipHostFree(m->inlaunch_timeouts);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
@@ -2073,11 +2086,11 @@ int ferrum_hip_model_decode_steps(FerrumHipModel* m, const uint64_t* seq_ids, co
         // not be replayed (it would write the sampled ids into freed memory)
         drop_graph(m);
         FH_CHECK_HIP(hipStreamSynchronize(m->stream));
-        if (m->history) (void)hipFree(m->history);
+        if (m->history) (void)hipHostFree(m->history);
         m->history = nullptr;
         m->history_cap = 0;
         const int cap = std::max(steps * n, 4096);             // rarely regrown: 4096 ids cover 128 steps of 32 sequences
-        FH_CHECK_HIP(hipMalloc((void**)&m->history, (size_t)cap * 4));
+        FH_CHECK_HIP(hipHostMalloc((void**)&m->history, (size_t)cap * 4, hipHostMallocDefault));
         m->history_cap = cap;
     }
     uint32_t* h_tok = reinterpret_cast<uint32_t*>(m->idx_host + m->il.tokens);
@@ -2099,9 +2112,15 @@ int ferrum_hip_model_decode_steps(FerrumHipModel* m, const uint64_t* seq_ids, co
         for (int b = 0; b < m->max_blocks_per_seq; b++) row[b] = b < (int)st.blocks.size() ? (int32_t)st.blocks[b] : 0;
     }
     h_cu[n] = (uint32_t)n;
-    size_t used = m->il.block_tables + (size_t)n * m->max_blocks_per_seq * 4;
-    FH_CHECK_HIP(hipMemcpyAsync(m->idx_dev, m->idx_host, used, hipMemcpyHostToDevice, m->stream));
-    FH_CHECK_HIP(hipMemsetAsync(m->step_counter, 0, 8, m->stream));    // step index + the advance ticket
+    IndexParts parts;
+    auto hand_over = [&](size_t offset, size_t words) { parts.word[parts.n] = (int)(offset / 4); parts.words[parts.n++] = (int)words; };
+    for (size_t o : {m->il.tokens, m->il.pos_offsets, m->il.kv_lens, m->il.sampled_idx}) hand_over(o, n);
+    hand_over(m->il.cu_seqlens, n + 1);
+    if (m->layered) {
+        for (size_t o : {m->il.tok_seq, m->il.prev_tokens, m->il.state_slots}) hand_over(o, n);
+        hand_over(m->il.scan_units, 2 * (size_t)m->batch_units);
+    }
+    hand_over(m->il.block_tables, (size_t)n * m->max_blocks_per_seq);
 
     auto enqueue_step = [&]() -> int {
         // the step's bookkeeping (sampled id → next input, positions, history) rides in the last stage of the argmax
@@ -2156,18 +2175,19 @@ int ferrum_hip_model_decode_steps(FerrumHipModel* m, const uint64_t* seq_ids, co
             m->graph_max_kv = kv_bucket;
         }
     }
+    hipLaunchKernelGGL(decode_begin_kernel, dim3(4, parts.n), dim3(256), 0, m->stream, reinterpret_cast<const uint32_t*>(m->idx_host),
+                       reinterpret_cast<uint32_t*>(m->idx_dev), parts, m->step_counter);
+    FH_CHECK_LAUNCH();
     if (graph_ok) {
         for (int st = 0; st < steps; st++) { FH_CHECK_HIP(hipGraphLaunch(m->graph_exec, m->stream)); form_hit(FORM_GRAPH_REPLAY); }
     } else {
         for (int st = 0; st < steps; st++)
             if (int rc = enqueue_step()) return rc;
     }
-    if (out_tokens)
-        FH_CHECK_HIP(hipMemcpyAsync(out_tokens, m->history, (size_t)steps * n * 4, hipMemcpyDeviceToHost, m->stream));
-    // the last token each sequence was FED: the one sampled a step before the last
-    std::vector<uint32_t> fed(first_tokens, first_tokens + n);
-    if (steps > 1) FH_CHECK_HIP(hipMemcpyAsync(fed.data(), m->history + (size_t)(steps - 2) * n, (size_t)n * 4, hipMemcpyDeviceToHost, m->stream));
     FH_CHECK_HIP(hipStreamSynchronize(m->stream));
+    if (out_tokens) memcpy(out_tokens, m->history, (size_t)steps * n * 4);
+    // the last token each sequence was FED: the one sampled a step before the last
+    const uint32_t* fed = steps > 1 ? m->history + (size_t)(steps - 2) * n : first_tokens;
     for (int i = 0; i < n; i++) {
         m->seqs[seq_ids[i]].len += steps;
         m->seqs[seq_ids[i]].last_token = fed[i];

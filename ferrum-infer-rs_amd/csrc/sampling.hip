@@ -143,7 +143,7 @@ __global__ __launch_bounds__(64) void argmax_final_kernel(const float* __restric
             adv.tokens[row] = id;
             adv.pos_offsets[row] += 1;
             adv.kv_lens[row] += 1;
-            adv.history[(long)step * adv.n + row] = id;
+            __hip_atomic_store(&adv.history[(long)step * adv.n + row], id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             const unsigned t = __hip_atomic_fetch_add(adv.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (t == gridDim.x - 1) {
                 __hip_atomic_store(adv.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -246,7 +246,7 @@ __global__ void argmax_merge_ranks_kernel(const float2* __restrict__ gathered, u
             adv.tokens[r] = best_id;
             adv.pos_offsets[r] += 1;
             adv.kv_lens[r] += 1;
-            adv.history[(long)step * adv.n + r] = best_id;
+            __hip_atomic_store(&adv.history[(long)step * adv.n + r], best_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
     __syncthreads();                                   // one block (rows ≤ 1024): every row has read `step`

@@ -351,6 +351,30 @@ def near_greedy(cfg, w, prompt, out, slack):
     return float(gap.max() / np.sqrt(np.mean(lg ** 2))) <= slack
 
 
+@pytest.mark.parametrize("n,max_len", [(1, 48), (3, 1600), (20, 1600), (65, 272)])
+def test_what_a_decode_call_hands_over(pkg, cases, n, max_len):
+    """Calls of one step, in which positions, previous tokens and block tables (up to 2000 words) travel each time, against one long call, whose
+    later steps the device feeds itself; tables that get a block in between, a number of sequences that changes."""
+    cfg, _, path = cases("shared")
+    lens = [max_len - 40 - (7 * i) % 33 if i % 5 == 0 else 1 + (11 * i) % 30 for i in range(n)]
+    prompts = [toks(cfg, k if max_len > 48 else 5, 70 + i) for i, k in enumerate(lens)]
+    got = []
+    for calls in ([1] * 20, [20], [3, 1, 16]):
+        m = load(pkg, path, "float32", tokens=2048, seqs=n, max_len=max_len, blocks=n * ((max_len + 15) // 16) + 1)
+        nxt = np.concatenate([m.unified_forward([(i, p, 0, True)])[0] for i, p in enumerate(prompts)])
+        if n > 1:
+            m.decode_steps([n - 1], nxt[-1:], 1)
+            m.release(n - 1)
+            m.unified_forward([(n - 1, prompts[-1], 0, True)])
+        out = []
+        for steps in calls:
+            out.append(m.decode_steps(range(n), nxt, steps))
+            nxt = out[-1][-1]
+        got.append(np.concatenate(out))
+        assert [m.block_table(i)[1] for i in range(n)] == [len(p) + 20 for p in prompts]
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["odd", "wide", "sinks", "shared", "loop", "all", "far", "talks"])
 def test_long_decoding_through_the_graph(pkg, cases, forms, name, dtype):
