@@ -54,6 +54,8 @@ int w4_gemm_dense_slabs_tile(const W4Device& w, const __half* x, float* slabs, s
 int w4_gemm_rows_splits(const W4Device& w, int m, size_t slab_bytes);
 int w4_gemm_rows(const W4Device& w, const __half* x, float* slabs, size_t slab_bytes, int m, int* S_out, int* rows_pad_out, int* n_pad_out,
                  hipStream_t stream);
+bool f16t_gemm_gated_supports(const W4Device& w, int im);
+int f16t_gemm_gated(const W4Device& w, const __half* x, __half* out, int m, int im, int gelu, hipStream_t stream);
 bool w4_gemm_gated_supports(const W4Device& w, int m, int im);
 int w4_gemm_gated(const W4Device& w, const __half* x, __half* out, int m, int im, int gelu, hipStream_t stream);
 int w4_gemm_dense_lds_splits(const W4Device& w, int m);

@@ -159,6 +159,7 @@ enum Form : int {
     FORM_TALK_ATTN_TILE_SPLIT,  // … and several workgroups share the keys of a tile
     FORM_W4_ROWS,               // ≤ 16 rows: a workgroup's share of the rows resident in LDS, K split over the grid into slabs
     FORM_W4_GATED,              // ≤ 16 rows: gate_up with its activation in the launch
+    FORM_F16_GATED,             // unquantised gate_up with its activation in the launch
     FORM_COUNT
 };
 

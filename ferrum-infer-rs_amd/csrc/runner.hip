@@ -1796,6 +1796,8 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             if (w4_gemm_gated_supports(L.gate_up, T, I)) {
                 if (gu_perm) form_hit(FORM_PERM_PRODUCER);
                 RUN(w4_gemm_gated(L.gate_up, m->norm_out, m->act_out, T, I, c.activation == 1, s));
+            } else if (f16t_gemm_gated_supports(L.gate_up, I)) {
+                RUN(f16t_gemm_gated(L.gate_up, m->norm_out, m->act_out, T, I, c.activation == 1, s));
             } else {
                 RUN(dense_linear(m, L.gate_up, m->norm_out, m->gate_up_out, T, s, true));
                 if (c.activation == 1) { RUN(fused_gelu_tanh_mul_split_f16(m->gate_up_out, m->act_out, T, I, s)); }

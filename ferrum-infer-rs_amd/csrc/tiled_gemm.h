@@ -62,7 +62,8 @@ struct GemmSection {          // columns [begin, next section's begin) of a fuse
     float mul = 1.f;          // factor of the accumulator, ahead of bias and activation (a norm's gain that is a single number)
 };
 // A gated section pairs 16-column tiles (gate, up, gate, up, …) whose weights are packed that way; a wave holds both tiles of a pair, and
-// the result takes the first half of the section's columns.
+// the result takes the first half of the section's columns.  Weights that have all gate tiles ahead of all up tiles are read in that order
+// (TiledGemm::pair: the tiles of a half).
 
 // Rows sorted by weight group (an expert's tokens), in blocks of `block` rows of one group each; the kernels read the block count from
 // the device, so a launch is sized for the largest one.  Place p of the list stands for row id[p] of the output and row id[p] / div of x;
@@ -90,6 +91,7 @@ struct TiledGemm {
     GemmRows rows;                        // (bias, groups and the x / out group strides are not used with it)
     int nsec = 0;
     GemmSection sec[GEMM_MAX_SECTIONS] = {};
+    int pair = 0;                         // > 0, one gated section: column tile t is weight tile t / 2 + (t odd ? pair : 0)
 };
 template <typename E> int tiled_gemm(const TiledGemm<E>& g, hipStream_t s);
 // number of K parts worth making for a projection of m rows whose consumer sums slabs (≤ GEMM_MAX_SLABS)

@@ -90,7 +90,7 @@ __device__ __forceinline__ int gemm_row_step(const TiledGemm<E>& p) { return p.x
 template <typename E, int MT, int J, bool EXT>
 __global__ __launch_bounds__(512) void tiled_gemm_kernel(TiledGemm<E> p, int kw) {
     typedef typename Frag<E>::v8 v8;
-    if (!EXT) { p.rows.id = nullptr; p.col_scale = nullptr; }
+    if (!EXT) { p.rows.id = nullptr; p.col_scale = nullptr; p.pair = 0; }
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     floatx4* red = reinterpret_cast<floatx4*>(smem);            // [NW][MT·J][64]
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -110,7 +110,8 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(TiledGemm<E> p, int kw)
     const int xs = gemm_row_step(p);
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) xrow[mt] = gemm_row(p, rb * MT + mt, g, a, b);
-    const E* wt = p.w + ((long)g * (p.n >> 4) + (live ? n0 >> 4 : 0)) * ksteps * 512 + lane * 8;
+    const E* wt = p.w + ((long)g * (p.n >> 4) + (!live ? 0 : J == 2 && p.pair ? n0 >> 5 : n0 >> 4)) * ksteps * 512 + lane * 8;
+    const int next_tile = J == 2 && p.pair ? p.pair : 1;
     floatx4 acc[MT][J];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
@@ -123,7 +124,7 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(TiledGemm<E> p, int kw)
         for (int u = 0; u < U; u++) {
             const int ss = min(s + u, s1 - 1);
 #pragma unroll
-            for (int j = 0; j < J; j++) bq[u][j] = __builtin_nontemporal_load(reinterpret_cast<const v8*>(wt + ((long)j * ksteps + ss) * 512));
+            for (int j = 0; j < J; j++) bq[u][j] = __builtin_nontemporal_load(reinterpret_cast<const v8*>(wt + ((long)j * next_tile * ksteps + ss) * 512));
 #pragma unroll
             for (int mt = 0; mt < MT; mt++) aq[u][mt] = *reinterpret_cast<const v8*>(xrow[mt] + (long)ss * xs);
         }
@@ -253,8 +254,8 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     }
 #pragma unroll
     for (int i = 0; i < NJ / 2; i++) {
-        const int t = (n0 >> 4) + NJ / 2 * wave + i;
-        bp[i] = p.w + ((long)g * ntl + (t < ntl ? t : ntl - 1)) * (p.k >> 5) * 512 + lane * 8;
+        const int t = min((n0 >> 4) + NJ / 2 * wave + i, ntl - 1);
+        bp[i] = p.w + ((long)g * ntl + (p.pair ? (t >> 1) + (t & 1) * p.pair : t)) * (p.k >> 5) * 512 + lane * 8;
     }
     const int xs = (HALVES ? 1 : 2) * gemm_row_step(p);
     const E* none = reinterpret_cast<const E*>(zero_fragment) + lane * EP;       // (past the end of K)
@@ -355,9 +356,13 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     // complete in order), then a lane finishes 8 columns of a row: bias, activation and factors, and rows leave in 16-byte pieces.  In a
     // gated section the lanes of the up tiles have nothing to do, those of the gate tiles read both.
     __syncthreads();
-    constexpr int LD = 16 * NJ + 4, LANES = 2 * NJ, ROUND = 64 / LANES;          // lanes of a row, rows of a round
+    // Where the whole launch is one gated section, a row takes half as many lanes, none of them idle: an
+    // expert model's up-projections 286 → 272 µs a launch, 2048 rows of a 0.6B model's gate_up 48 → 41.
+    constexpr int LD = 16 * NJ + 4;
     float* lf = reinterpret_cast<float*>(smem) + wave * 32 * LD;
-    const int cl = (lane % LANES) * 8, col = n0 + wn * 16 * NJ + cl;
+    const bool pairs = p.nsec == 1 && p.sec[0].begin == 0 && gemm_gated_act(p.sec[0].act);
+    const int lanes = pairs ? NJ : 2 * NJ, place = lane & (lanes - 1), row_in = lane >> __builtin_ctz(lanes), rounds = lanes / 2;      // (rounds of 64 / lanes rows)
+    const int cl = pairs ? (place >> 1) * 32 + (place & 1) * 8 : place * 8, col = n0 + wn * 16 * NJ + cl;
     const GemmSection sec = gemm_section(p, min(col, p.n - 1));
     const bool gated = gemm_gated_act(sec.act), vec = p.n_store % 8 == 0 && p.ldo % 8 == 0 && p.out_group % 8 == 0 && ((uintptr_t)p.out & 15) == 0 && ((uintptr_t)p.out_f32 & 15) == 0;
     const bool active = gated ? col < p.n && !(col & 16) : col < p.n_store;
@@ -376,8 +381,8 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
             for (int j = 0; j < NJ; j++) *reinterpret_cast<floatx4*>(lf + (i * 16 + b) * LD + j * 16 + 4 * a) = acc[2 * ch + i][j];
         const int row0 = m0 + (wm * MI + 2 * ch) * 16;
 #pragma unroll 1
-        for (int q = 0; q < 32 / ROUND; q++) {
-            const int row = q * ROUND + lane / LANES, gr = gemm_out_row(p, row0 + row);
+        for (int q = 0; q < rounds; q++) {
+            const int row = q * (32 / rounds) + row_in, gr = gemm_out_row(p, row0 + row);
             if (gr < 0 || !active) continue;
             float v[8];
 #pragma unroll
@@ -503,6 +508,7 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     }
     FH_REQUIRE(!gated || (g.groups == 1 && !g.col_scale), "tiled_gemm: gated sections take one group and no column factors");
     FH_REQUIRE(!g.col_scale || (g.out && g.ld_col_scale % 8 == 0), "tiled_gemm: column factors with rows of %ld", g.ld_col_scale);
+    FH_REQUIRE(!g.pair || (gated && g.nsec == 1 && g.sec[0].begin == 0 && g.n == 32 * g.pair), "tiled_gemm: %d tiles of a half, n=%d", g.pair, g.n);
     const GemmRows& rows = g.rows;
     if (rows.id) {
         FH_REQUIRE(g.slabs == 1 && !g.bias && !g.x_blocks && !g.row_scale && rows.div > 0 && rows.max_blocks > 0 && rows.group && rows.total,

@@ -3382,6 +3382,21 @@ static int f16t_gemm_impl(const __half* x, const __half* wt, OutT* out, int m, i
     }
     return 0;
 }
+// gate_up and its activation in one launch, whatever the rows: two wrote and read [m, 2·im] between them, and a dependent launch costs 2 µs in
+// a captured step (a 0.6B model, 14 layers, 32 steps: 20.9 → 20.0 ms)
+bool f16t_gemm_gated_supports(const W4Device& w, int im) { return w.f16t && !w.bias && w.n == 2 * im && im % 16 == 0 && w.k % 32 == 0; }
+int f16t_gemm_gated(const W4Device& w, const __half* x, __half* out, int m, int im, int gelu, hipStream_t stream) {
+    FH_REQUIRE(f16t_gemm_gated_supports(w, im), "f16t_gemm_gated: N=%d K=%d intermediate=%d", w.n, w.k, im);
+    form_hit(FORM_F16_DENSE_LINEAR);
+    form_hit(FORM_F16_GATED);
+    TiledGemm<_Float16> g;
+    g.x = reinterpret_cast<const _Float16*>(x); g.ldx = w.k; g.w = reinterpret_cast<const _Float16*>(w.f16t);
+    g.m = m; g.n = w.n; g.k = w.k; g.out = reinterpret_cast<_Float16*>(out); g.ldo = im;
+    g.nsec = 1; g.sec[0].begin = 0; g.sec[0].act = gelu ? GEMM_ACT_GELU_GLU : GEMM_ACT_SILU_GLU;
+    g.pair = im / 16;
+    return tiled_gemm(g, stream);
+}
+
 int f16t_gemm(const __half* x, const __half* wt, __half* out, int m, int n, int k, float* workspace,
               size_t workspace_bytes, hipStream_t stream) {
     return f16t_gemm_impl<__half>(x, wt, out, m, n, k, workspace, workspace_bytes, stream);

@@ -161,6 +161,20 @@ def test_unquantised_dense_linear_model(pkg, prompt_len, forms):
     _assert_parity(res)
 
 
+@pytest.mark.parametrize("prompt_len,inter,wide,half", [(1, 128, 257, 255), (16, 896, 257, 255), (23, 128, 257, 255), (64, 384, 257, 255), (70, 896, 257, 255),
+                                                        (200, 896, 1, 0), (200, 384, 10 ** 6, 0), (200, 896, 10 ** 6, 10 ** 6), (200, 128, 10 ** 6, 10 ** 6)])
+@pytest.mark.parametrize("activation", [0, 1])
+def test_unquantised_gate_up_with_its_activation(pkg, prompt_len, inter, wide, half, activation, knobs, forms):
+    """One gate and one up tile of a wave, and pairs of tiles within every size of the tile kernel."""
+    from tests import modelgen
+    knobs.set(TILED_BIG_MIN_TILES=1 if prompt_len == 200 else 128, TILED_WIDE_MIN_TILES=wide, TILED_HALF_MAX_TILES=half)
+    res = modelgen.run_parity_case(pkg, moe=False, layers=2, prompt_len=prompt_len, decode_steps=2, seed=171 + prompt_len, dense_proj=True, tied=True,
+                                   inter=inter, activation=activation)
+    h = forms.require("f16_gated", "tiled_gemm")
+    assert bool(h.get("tiled_gemm_big")) == (prompt_len == 200) and bool(h.get("tiled_gemm_256")) == (wide == 1)
+    _assert_parity(res)
+
+
 def test_qwen3_06b_dims_unquantised_layer(pkg, forms):
     """BASELINE configs[0] (Qwen3-0.6B: H 1024, 16/8 heads × 128, I 3072, QK-norm, θ 1e6, tied lm_head, unquantised weights) —
     one layer at its real dimensions (vocabulary cut to 2048), 24 sequences: 40-token prompts in one forward, then three
