@@ -643,9 +643,9 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void paged_prefill_attn_ker
 // operand against Pᵀ: every lane's accumulator then holds Σ_keys P of its query row, rescaled by α like O), and steps whose 64
 // keys are visible to every row of a tile (all but the diagonal ones) run a mask-free body.  Same staging, tile layout and
 // per-row arithmetic otherwise (Sᵀ = K·Qᵀ, lane-local exp2, Oᵀ += Vᵀ·Pᵀ); l is the sum of the fp16 P the numerator uses.
-template <int HD>
+template <int HD, int MT>
 __global__ __launch_bounds__(256, 2) void paged_prefill_attn64_kernel(AttnArgs p) {
-    constexpr int NW = 4, MT = 2, DT = HD / 16, KS = HD / 32, TILE = 16 * HD;
+    constexpr int NW = 4, DT = HD / 16, KS = HD / 32, TILE = 16 * HD;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     __half* lds_kv = reinterpret_cast<__half*>(smem);          // [2 stages][2 pairs][K0, K1, V0, V1][TILE]; reused by the epilogue
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -1183,8 +1183,7 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
     const Knobs& kn = knobs();                                   // read once at library load (knobs.h), never per launch
     const bool flash_off = kn.attn_no_flash;
     const long flash_min_rows = kn.attn_flash_min_rows;          // tests lower it
-    // … and only when its workgroups (128 rows × one kv head each) cover the chip: a lone 256-token prompt has 64 of them and
-    // is faster KV-split over 512 workgroups (TTFT 6.7 vs 7.1 ms)
+    // … and only when its workgroups (64 or 128 rows × one kv head each) cover the chip, below which the KV-split form has more of them
     const long flash_min_wgs = kn.attn_flash_min_rows_set ? 1 : 256;
     // short prompts whose whole context fits one LDS image (kv ≤ 256 at head_dim 128): resident-K/V form, two workgroups per
     // (sequence, kv head).  max_kv_len bounds every sequence; needs ≥ 4 row tiles per sequence on average to pay off.
@@ -1201,10 +1200,19 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
         form_hit(FORM_ATTN_RESIDENT);
         return 0;
     }
-    if (!fq && cu_seqlens_q && !flash_off && (long)max_q_len * G >= flash_min_rows &&
-        (long)total_q_tokens * 2 >= (long)num_seqs * max_q_len &&
-        ((long)total_q_tokens * G / (head_dim == 256 ? 64 : 128)) * num_kv_heads >= flash_min_wgs) {
-        const int mt = head_dim == 256 ? 1 : 2, unit_tiles = 4 * mt;
+    // head_dim 128 has two sizes of workgroup.  128 rows read K/V from LDS half as often, 64 rows make twice the workgroups and half of a step's
+    // vector work in each: µs, row-split or KV-split form / 64 rows / 128 rows (workgroups of 128 rows × kv heads)
+    //   8B heads (32 on 8)    1 × 8100 (2024)      2372 / 919 / 779      1 × 2048 (512)        196 / 95 / 82     1 × 1024 (256)         62 / 33 / 37
+    //                         1 × 700 (175)          32 / 25 / 28        1 × 500 (125)          19 / 17 / 24     1 × 300 (75)           11 / 11 / 17
+    //   16 on 8               1500 and 548 (256)     82 / 46 / 63        293, 1389, 366 (256)   87 / 48 / 62     1 × 986 at 366 (123)   49 / 35 / 54
+    //                         6 × 100, 1400 (250)    80 / 39 / 53        1 × 500 (62)           14 / 16 / 24
+    // A batch qualifies where most of its sequences bring many rows, or they bring 256 on average.
+    const long rows_heads = (long)total_q_tokens * G * num_kv_heads;
+    const bool two_sizes = head_dim == 128 && !kn.attn_flash32, half_units = two_sizes && (kn.attn_flash_rows ? kn.attn_flash_rows == 64 : rows_heads < 512 * 128);
+    const bool flash_fits = (long)total_q_tokens * 2 >= (long)num_seqs * max_q_len || (two_sizes && (long)total_q_tokens * G >= (long)num_seqs * 256);
+    if (!fq && cu_seqlens_q && !flash_off && (long)max_q_len * G >= flash_min_rows && flash_fits &&
+        rows_heads / (half_units || head_dim == 256 ? 64 : 128) >= (half_units && !kn.attn_flash_min_rows_set ? 192 : flash_min_wgs)) {
+        const int mt = half_units || head_dim == 256 ? 1 : 2, unit_tiles = 4 * mt;
         const long tiles_bound = ((long)total_q_tokens * G) / 16 + num_seqs;
         const long units = cdiv(tiles_bound, (long)unit_tiles) + num_seqs;
         const dim3 grid((unsigned)units, num_kv_heads, 1);
@@ -1223,10 +1231,12 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
             const size_t lds64 = 2 * lds;
             static bool attr64 = false;
             if (!attr64) {
-                FH_CHECK_HIP(hipFuncSetAttribute((const void*)paged_prefill_attn64_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64));
+                FH_CHECK_HIP(hipFuncSetAttribute((const void*)paged_prefill_attn64_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64));
+                FH_CHECK_HIP(hipFuncSetAttribute((const void*)paged_prefill_attn64_kernel<128, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64));
                 attr64 = true;
             }
-            hipLaunchKernelGGL((paged_prefill_attn64_kernel<128>), grid, dim3(256), lds64, s, a);
+            if (mt == 1) hipLaunchKernelGGL((paged_prefill_attn64_kernel<128, 1>), grid, dim3(256), lds64, s, a);
+            else hipLaunchKernelGGL((paged_prefill_attn64_kernel<128, 2>), grid, dim3(256), lds64, s, a);
         } else if (head_dim == 128) FH_FLASH(128, 2) else if (head_dim == 64) FH_FLASH(64, 2) else FH_FLASH(256, 1)
 #undef FH_FLASH
         FH_CHECK_LAUNCH();

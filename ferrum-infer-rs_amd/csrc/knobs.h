@@ -24,6 +24,7 @@ struct Knobs {
     bool attn_narrow = false;
     bool attn_no_resident = false;    // never take the resident-K/V short-prompt prefill form
     long attn_resident_min_wgs = 128; // … and only from this many workgroups (tests lower it)
+    int attn_flash_rows = 0;          // 64 / 128: forced rows per workgroup of the 64-key form
     bool attn_flash32 = false;        // the flash form with 32-key steps (paged_prefill_attn_kernel) for head_dim 128 too
     // INT4 GEMMs (w4_gemm.hip)
     int moe_kw_pairs = 16;

@@ -729,6 +729,40 @@ def test_paged_prefill_attention_resident_kv(env, window, nq, nkv, knobs, forms)
         assert nmse(ref, got[cu[s_]:cu[s_ + 1]]) < 1e-5, s_
 
 
+@pytest.mark.parametrize("rows", [64, 128])
+@pytest.mark.parametrize("window,nq,nkv", [(0, 8, 2), (24, 14, 2), (0, 32, 4), (1, 6, 6), (40, 3, 1)])
+def test_paged_prefill_attention_in_both_unit_sizes(env, window, nq, nkv, rows, knobs, forms):
+    knobs.set(ATTN_FLASH_ROWS=rows)
+    test_paged_prefill_attention_lds_shared_kv(env, window, nq, nkv, 128, knobs, forms)
+
+
+@pytest.mark.parametrize("nq,nkv,q_lens,pos,flash", [
+    (16, 8, [1500, 548], [0, 0], True), (16, 8, [293, 1389, 366], [1133, 0, 0], True), (16, 8, [100] * 6 + [1400], [0] * 7, True),
+    (16, 8, [986], [366], True), (16, 8, [767], [0], False), (16, 8, [769], [0], True), (32, 8, [384], [0], True), (32, 8, [383], [1], False),
+    (4, 2, [1] * 40 + [2500], [600] * 41, False), (32, 8, [2049], [0], True)])
+def test_prompt_attention_takes_the_shared_form_by_size(env, nq, nkv, q_lens, pos, flash, forms, knobs):
+    """Ragged batches on either side of the rule, against the forms without shared K/V (fp16 results of two orders of summation)."""
+    pkg, B, ctx, O, torch = env
+    S, total, kv = len(q_lens), sum(q_lens), max(p + t for p, t in zip(pos, q_lens))
+    mb = (kv + 15) // 16
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    rand = lambda *n: torch.randn(*n, device="cuda", generator=gen).half()
+    k, v, q = rand(S * mb * nkv * 2048), rand(S * mb * nkv * 2048), rand(total, nq, 128)
+    tables = torch.randperm(S * mb, device="cuda", generator=gen).to(torch.int32).reshape(S, mb)
+    cu = torch.from_numpy(np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)).cuda()
+    po = torch.from_numpy(np.array(pos, np.int32)).cuda()
+    outs = []
+    for off in (None, 1):
+        knobs.set(ATTN_NO_FLASH=off)
+        forms.reset()
+        out = torch.zeros(total, nq, 128, dtype=torch.float16, device="cuda")
+        B.paged_varlen_attention(ctx, q, k, v, out, cu, po, tables, S, total, kv, nq, nkv, 128, 0, 16, mb, max(q_lens))
+        ctx.sync()
+        assert bool(forms.hits().get("attn_flash")) == (flash and not off)
+        outs.append(host(out))
+    assert nmse(outs[1], outs[0]) < 1e-5
+
+
 def test_paged_prefill_attention_lds_shared_kv_many_sequences(env, knobs, forms):
     """The flash form over 70 sequences (two passes of its in-kernel sequence lookup), two of them empty."""
     pkg, B, ctx, O, torch = env
