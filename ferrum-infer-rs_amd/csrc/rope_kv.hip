@@ -12,34 +12,42 @@
 
 namespace fh {
 
-// One quarter wave per (token, head): a 64-thread workgroup covers 4 consecutive heads of one token
-// (q heads, then k heads, then v heads).  Row maths in rope_rows.h.
+// One quarter wave per (token, head): a wave takes four consecutive tokens of a head (q heads, then k heads, then v heads), a workgroup
+// four heads.  Row maths in rope_rows.h.  Bound by bytes (read q|k|v once, write it once); with a workgroup of one wave per token and four
+// heads it was bound by the workgroups' starts, 0.8 ns each, and by V's stores of two bytes: a tile keeps four keys of a dimension
+// together, which is the four tokens of a wave where their positions are aligned, exchanged between its quarters (head_dim 128).
+//   8100 tokens × (32 + 2·8) heads: 80 → 41 µs (200 MB, what a copy takes); 2048 × (16 + 2·8): 16.5 → 10 µs
 template <int HD>
-__global__ __launch_bounds__(64) void split_qkv_norm_rope_paged_kernel(
+__global__ __launch_bounds__(256) void split_qkv_norm_rope_paged_kernel(
     const __half* __restrict__ qkv, const __half* __restrict__ q_norm_w, const __half* __restrict__ k_norm_w,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t, __half* __restrict__ q_out,
     __half* __restrict__ cache_k, __half* __restrict__ cache_v, const uint32_t* __restrict__ cu_seqlens_q,
-    const uint32_t* __restrict__ pos_offsets, const int32_t* __restrict__ block_tables, int num_seqs,
+    const uint32_t* __restrict__ pos_offsets, const int32_t* __restrict__ block_tables, int num_seqs, int m_total,
     int q_heads, int kv_heads, float eps, int qk_mode, int max_blocks_per_seq) {
     constexpr int PPL = HD / 32, HALF = HD / 2;
-    const int tok = blockIdx.x, lane = threadIdx.x, q16 = lane & 15;
-    const int heads = q_heads + 2 * kv_heads;
-    const int head_raw = blockIdx.y * 4 + (lane >> 4);
-    const bool act = head_raw < heads;
-    const int head = act ? head_raw : heads - 1;          // clamped: loads stay unconditional
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, q16 = lane & 15, quarter = lane >> 4;
+    const int head = blockIdx.y * 4 + wave;
+    if (head >= q_heads + 2 * kv_heads) return;
+    const int tok0 = blockIdx.x * 4, tok = min(tok0 + quarter, m_total - 1);         // clamped: loads stay unconditional
+    const bool act = tok0 + quarter < m_total;
     const int q_dim = q_heads * HD, kv_dim = kv_heads * HD;
     const __half* row = qkv + (long)tok * (q_dim + 2 * kv_dim);
 
-    // locate the sequence: the last s with cu_seqlens_q[s] ≤ tok (what the reference kernel's linear scan returns), found
+    // locate the sequences: the last s with cu_seqlens_q[s] ≤ tok (what the reference kernel's linear scan returns), found
     // 64 sequences per memory round trip — a serial scan costs the tokens of the 32nd prompt 31 dependent loads
-    int seq = 0;
+    int seq4[4] = {0, 0, 0, 0};
     for (int s0 = 0; s0 < num_seqs; s0 += 64) {
         const int s = s0 + lane;
-        const unsigned long long le = __ballot(s < num_seqs && cu_seqlens_q[s] <= (uint32_t)tok);
-        if (le == 0) break;
-        seq = s0 + 63 - __clzll((long long)le);
-        if (le != ~0ull) break;
+        const uint32_t first = s < num_seqs ? cu_seqlens_q[s] : 0xffffffffu;
+        unsigned long long le = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            le = __ballot(first <= (uint32_t)min(tok0 + j, m_total - 1));
+            if (le) seq4[j] = s0 + 63 - __clzll((long long)le);
+        }
+        if (le != ~0ull) break;                              // (the fourth token's is the largest set)
     }
+    const int seq = quarter == 0 ? seq4[0] : quarter == 1 ? seq4[1] : quarter == 2 ? seq4[2] : seq4[3];
     const int pos = (int)pos_offsets[seq] + (tok - (int)cu_seqlens_q[seq]);
 
     const bool is_q = head < q_heads;
@@ -49,9 +57,9 @@ __global__ __launch_bounds__(64) void split_qkv_norm_rope_paged_kernel(
     const int mode = (is_q || is_k) ? qk_mode : 0;
     const RopeRow<HD> rr = rope_row16<HD>(src, is_q ? q_norm_w : k_norm_w, cos_t + (long)pos * HALF, sin_t + (long)pos * HALF,
                                           mode, qk_mode == 1, qk_mode != 0, eps, q16);
-    if (!act) return;
     using hv = typename RopeRow<HD>::hv;
     if (is_q) {
+        if (!act) return;
         __half* dst = q_out + ((long)tok * q_heads + local_head) * HD;
         *reinterpret_cast<hv*>(dst + rr.off0) = rr.out0;
         *reinterpret_cast<hv*>(dst + rr.off1) = rr.out1;
@@ -61,15 +69,42 @@ __global__ __launch_bounds__(64) void split_qkv_norm_rope_paged_kernel(
     const long physical = block_tables[(long)seq * max_blocks_per_seq + logical];
     __half* tile = (is_k ? cache_k : cache_v) + (physical * kv_heads + local_head) * kv_tile_elems(HD);
     _Float16* t16 = reinterpret_cast<_Float16*>(tile);
+    if (is_k) {                                              // (PPL dimensions of a row lie within one chunk of eight)
+        if (!act) return;
+        *reinterpret_cast<hv*>(t16 + k_tile_off(slot, rr.off0)) = rr.out0;
+        *reinterpret_cast<hv*>(t16 + k_tile_off(slot, rr.off1)) = rr.out1;
+        return;
+    }
+    if constexpr (HD == 128) {
+        const int pos_first = __builtin_amdgcn_readfirstlane(pos);
+        if (tok0 + 3 < m_total && seq4[0] == seq4[3] && pos_first % 4 == 0) {
+            // quarter t holds token t's dimensions off0 … + 3 and off1 … + 3, as four pairs; quarter r leaves with pair r of all four tokens
+            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+            const u32x2 lo = __builtin_bit_cast(u32x2, rr.out0), hi = __builtin_bit_cast(u32x2, rr.out1);
+            uint32_t from[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int pair = (quarter + i) & 3;          // quarter t sends the pair of quarter t + i
+                const uint32_t mine = pair == 0 ? lo[0] : pair == 1 ? lo[1] : pair == 2 ? hi[0] : hi[1];
+                from[i] = i == 0 ? mine : (uint32_t)__shfl((int)mine, ((quarter - i) & 3) * 16 + q16, 64);
+            }
+            uint32_t key[4];                                 // from[i] is of token (quarter − i) mod 4
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                const int i = (quarter - t) & 3;
+                key[t] = i == 0 ? from[0] : i == 1 ? from[1] : i == 2 ? from[2] : from[3];
+            }
+            const int d = (quarter < 2 ? rr.off0 : rr.off1) + 2 * (quarter & 1);
+            *reinterpret_cast<u32x2*>(t16 + v_tile_off(slot & ~3, d)) = (u32x2){(key[0] & 0xffff) | key[1] << 16, (key[2] & 0xffff) | key[3] << 16};
+            *reinterpret_cast<u32x2*>(t16 + v_tile_off(slot & ~3, d + 1)) = (u32x2){key[0] >> 16 | (key[1] & 0xffff0000u), key[2] >> 16 | (key[3] & 0xffff0000u)};
+            return;
+        }
+    }
+    if (!act) return;
 #pragma unroll
     for (int k = 0; k < PPL; k++) {
-        if (is_k) {
-            t16[k_tile_off(slot, rr.off0 + k)] = rr.out0[k];
-            t16[k_tile_off(slot, rr.off1 + k)] = rr.out1[k];
-        } else {
-            t16[v_tile_off(slot, rr.off0 + k)] = rr.out0[k];
-            t16[v_tile_off(slot, rr.off1 + k)] = rr.out1[k];
-        }
+        t16[v_tile_off(slot, rr.off0 + k)] = rr.out0[k];
+        t16[v_tile_off(slot, rr.off1 + k)] = rr.out1[k];
     }
 }
 
@@ -82,10 +117,10 @@ int split_qkv_norm_rope_into_paged_cache_varlen_f16(
     FH_REQUIRE(block_size == KV_BLOCK, "paged KV: block_size=%d unsupported (native layout uses 16)", block_size);
     FH_REQUIRE(head_dim == 64 || head_dim == 128 || head_dim == 256, "paged KV: head_dim=%d must be 64, 128 or 256", head_dim);
     FH_REQUIRE(qk_mode >= 0 && qk_mode <= 3, "paged KV: qk_mode=%d out of range", qk_mode);
-    const dim3 grid(m_total, cdiv(q_heads + 2 * kv_heads, 4));
+    const dim3 grid(cdiv(m_total, 4), cdiv(q_heads + 2 * kv_heads, 4));
 #define FH_ROPE(HDV)                                                                                                   \
-    hipLaunchKernelGGL(split_qkv_norm_rope_paged_kernel<HDV>, grid, dim3(64), 0, s, qkv, q_norm_w, k_norm_w, cos_t, sin_t, \
-                       q_out, cache_k, cache_v, cu_seqlens_q, pos_offsets, block_tables, num_seqs, q_heads, kv_heads, eps, \
+    hipLaunchKernelGGL(split_qkv_norm_rope_paged_kernel<HDV>, grid, dim3(256), 0, s, qkv, q_norm_w, k_norm_w, cos_t, sin_t, \
+                       q_out, cache_k, cache_v, cu_seqlens_q, pos_offsets, block_tables, num_seqs, m_total, q_heads, kv_heads, eps, \
                        qk_mode, max_blocks_per_seq)
     if (head_dim == 64) FH_ROPE(64); else if (head_dim == 128) FH_ROPE(128); else FH_ROPE(256);
 #undef FH_ROPE

@@ -308,6 +308,35 @@ def _rope(O, hd, max_seq, theta=1e6):
     return O.build_rope_cache(theta, hd, max_seq)
 
 
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("q_lens,pos,nq,nkv", [([1], [0], 1, 1), ([4], [12], 3, 1), ([3, 5], [1, 4], 2, 2), ([16, 0, 8, 0], [0, 3, 4, 0], 5, 3), ([7, 9, 64, 33], [1, 0, 0, 7], 8, 2),
+                                               ([4] * 70, [4 * (i % 5) for i in range(70)], 2, 1), ([5] * 66 + [0] * 3, [i % 7 for i in range(69)], 3, 2)])
+def test_quads_of_tokens_in_the_paged_cache(env, q_lens, pos, nq, nkv, hd):
+    """Four tokens of a wave at aligned positions and not, across sequences and past the batch, empty sequences in between and at the end: copies."""
+    pkg, B, ctx, O, torch = env
+    rng = np.random.default_rng(len(q_lens) + hd)
+    S, T, mb = len(q_lens), sum(q_lens), (max(p + n for p, n in zip(pos, q_lens)) + 15) // 16
+    qkv = f16r(rng.standard_normal((T, (nq + 2 * nkv) * hd)))
+    tables = rng.permutation(S * mb).astype(np.int32).reshape(S, mb)
+    cu = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+    ck, cv = B.alloc_paged_pool(S * mb, nkv, hd), B.alloc_paged_pool(S * mb, nkv, hd)
+    one, cos, sin = torch.ones(hd, dtype=torch.float16, device="cuda"), torch.ones(512, hd // 2, device="cuda"), torch.zeros(512, hd // 2, device="cuda")
+    q_out = torch.full((T + 1, nq * hd), 7.0, dtype=torch.float16, device="cuda")
+    B.split_qkv_norm_rope_into_paged_cache_varlen(ctx, dev16(torch, qkv), one, one, cos, sin, q_out, ck, cv, torch.from_numpy(cu).cuda(),
+                                                  torch.from_numpy(np.array(pos, np.int32)).cuda(), torch.from_numpy(tables).cuda(), S, T, nq, nkv, hd, 1e-6, 0, 16, mb)
+    ctx.sync()
+    assert np.array_equal(host(q_out)[:T], qkv[:, :nq * hd]) and np.all(host(q_out)[T] == 7.0)
+    left = [ck.float().abs().sum().item(), cv.float().abs().sum().item()]
+    for s in range(S):
+        kk, vv = B.paged_kv_read(ctx, ck, cv, torch.from_numpy(tables[s]).cuda(), pos[s] + q_lens[s], nkv, hd)
+        ctx.sync()
+        for got, at in ((kk, nq), (vv, nq + nkv)):
+            got = host(got).reshape(-1, nkv * hd)
+            assert np.array_equal(got[pos[s]:], qkv[cu[s]:cu[s + 1], at * hd:(at + nkv) * hd]) and not got[:pos[s]].any()
+    want = [np.abs(qkv[:, at * hd:(at + nkv) * hd].astype(np.float64)).sum() for at in (nq, nq + nkv)]
+    assert np.allclose(left, want, rtol=1e-4)                              # nothing else was written
+
+
 @pytest.mark.parametrize("qk_mode,hd", [(1, 128), (2, 128), (3, 128), (0, 128), (1, 64), (2, 256)])
 def test_split_qkv_norm_rope_into_paged_cache_varlen(env, qk_mode, hd):
     pkg, B, ctx, O, torch = env
