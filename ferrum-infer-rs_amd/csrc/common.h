@@ -121,12 +121,13 @@ __device__ __forceinline__ void reduce_slabs8(const float* __restrict__ base, lo
     }
 }
 
-// act(gate) · up of a gated MLP: SiLU, or GELU in its tanh form (one definition: the fused and the separate launches give the same bits)
+// act(gate) · up of a gated MLP: SiLU, or GELU in its tanh form, ½·g·(1 + tanh z) = g / (1 + exp(−2z)) — without the cancellation of 1 + tanh
+// left of zero, and a third of tanhf's instructions (one definition: the fused and the separate launches give the same bits)
 template <bool GELU>
 __device__ __forceinline__ _Float16 gated_act(float g, float u) {
     if (GELU) {
         const float inner = 0.79788456f * (g + 0.044715f * g * g * g);
-        return (_Float16)(0.5f * g * (1.0f + tanhf(inner)) * u);
+        return (_Float16)(g / (1.0f + __expf(-2.0f * inner)) * u);
     }
     return (_Float16)(g / (1.0f + __expf(-g)) * u);
 }

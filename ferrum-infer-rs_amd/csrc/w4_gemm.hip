@@ -2187,18 +2187,21 @@ __global__ __launch_bounds__(256, 2) void w4_gemm_tilep_kernel(W4Args p) {
 // k-half's operands are expanded between the MFMAs of the current one; activations global → registers → LDS one group ahead,
 // weights two groups ahead.
 // MODE 0 dense; 1 / 2 the MoE grouped GEMM over MT·16-row align blocks (rows gathered through sorted_token_ids, the block's
-// expert from block_ids; 2 = gate_up with the silu·mul epilogue), tiles dealt to the XCDs like w4_gemm_tile_kernel's.
+// expert from block_ids; 2 = gate_up with the silu·mul epilogue), tiles dealt to the XCDs like w4_gemm_tile_kernel's; 3 / 4 dense gate_up
+// whose wave pairs two gate tiles with their up tiles and stores silu / gelu(gate)·up, rounded as the two launches
+// round: the projection's [rows, 2·im] is not written and read again (8100 × 28672 × 4096 and its activation, a layer: 1490 + 200 → 1553 µs).
 template <int MT, bool HAS_ZP, int MODE = 0>
 __global__ __launch_bounds__(256, MT <= 6 ? 2 : 1) void w4_gemm_big_kernel(W4Args p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     half8* lds_a = reinterpret_cast<half8*>(lds_raw);          // [2][MT][4 s][64] half8
     constexpr int FR = MT * 256, ROWS = MT * 16;
+    constexpr bool MOE = MODE == 1 || MODE == 2, PAIRS = MODE >= 3;
     typedef _Float16 half2v_ __attribute__((ext_vector_type(2)));
     typedef uint32_t u32x4g __attribute__((ext_vector_type(4)));
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
     int ct = blockIdx.x, rb = blockIdx.y;
-    if (MODE != 0) {        // each XCD walks a contiguous range of (column tile, row block), row block fastest: one expert's blocks meet its weights in one L2
+    if (MOE) {        // each XCD walks a contiguous range of (column tile, row block), row block fastest: one expert's blocks meet its weights in one L2
         const int nwg = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y;
         const int xcd = lin & 7, virt = xcd * (nwg >> 3) + min(xcd, nwg & 7) + (lin >> 3);
         ct = virt / (int)gridDim.y;
@@ -2211,8 +2214,8 @@ __global__ __launch_bounds__(256, MT <= 6 ? 2 : 1) void w4_gemm_big_kernel(W4Arg
     const __half* sc = p.sc;
     const __half* zp = p.zp;
     uint32_t aoff[MT];                                          // byte offset of this thread's staging rows: scalar base + 32-bit offset
-    int row_out_l[MODE != 0 ? MT : 1];                          // MoE: output row (pair id) of tile row mt·16 + b, −1 = padding
-    if (MODE != 0) {
+    int row_out_l[MOE ? MT : 1];                          // MoE: output row (pair id) of tile row mt·16 + b, −1 = padding
+    if (MOE) {
         // the three reads a tile starts with are independent and in bounds for every launched row block (padding blocks hold
         // sentinels): request them together, then decide — one memory round trip instead of three before the first A row
         const int total = *p.total_post_pad;
@@ -2240,7 +2243,7 @@ __global__ __launch_bounds__(256, MT <= 6 ? 2 : 1) void w4_gemm_big_kernel(W4Arg
     // MoE: the valid rows of an align block are a prefix; 16-row tiles that hold only padding are skipped (their MFMAs, not the
     // side work riding behind them): at ≈ 512 pairs per expert 96-row blocks carry ≈ 19 % padding rows, 16-row granularity ≈ 2 %
     int mt_valid = MT;
-    if (MODE != 0) {
+    if (MOE) {
         mt_valid = 0;
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) mt_valid += __ballot(row_out_l[mt] >= 0) != 0 ? 1 : 0;
@@ -2249,6 +2252,17 @@ __global__ __launch_bounds__(256, MT <= 6 ? 2 : 1) void w4_gemm_big_kernel(W4Arg
     const char* qw_wave = reinterpret_cast<const char*>(qw) + ((long)st * p.G * 4) * 64 * 16;
     const char* sc_wave = reinterpret_cast<const char*>(sc) + ((long)st * p.G) * 16 * 8;
     const char* zp_wave = HAS_ZP ? reinterpret_cast<const char*>(zp) + ((long)st * p.G) * 16 * 8 : nullptr;
+    // PAIRS: tiles 0, 1 of the wave are gate columns st·32 …, tiles 2, 3 the up columns act_im on, each pair half of a supertile
+    const int up0 = PAIRS ? (p.act_im >> 4) + 2 * st : 0;
+    long up_w = 0, up_s = 0;                                    // bytes from the gate pair to the up pair
+    if (PAIRS) {
+        qw_wave = reinterpret_cast<const char*>(qw) + ((long)(st >> 1) * p.G * 4 + (st & 1) * 2) * 1024;
+        up_w = ((long)(up0 >> 2) * p.G * 4 + (up0 & 3)) * 1024 - ((long)(st >> 1) * p.G * 4 + (st & 1) * 2) * 1024;
+        const long s_gate = (long)(st >> 1) * p.G * 128 + (st & 1) * 4;
+        sc_wave = reinterpret_cast<const char*>(sc) + s_gate;
+        if (HAS_ZP) zp_wave = reinterpret_cast<const char*>(zp) + s_gate;
+        up_s = (long)(up0 >> 2) * p.G * 128 + (up0 & 3) * 2 - s_gate;
+    }
     const char* x_base = reinterpret_cast<const char*>(p.x);
     const uint32_t lane16 = lane * 16, b8 = b * 8;
 
@@ -2268,7 +2282,13 @@ __global__ __launch_bounds__(256, MT <= 6 ? 2 : 1) void w4_gemm_big_kernel(W4Arg
     auto issue_w = [&](int sl, int g) __attribute__((always_inline)) {
 #pragma unroll
         for (int nt = 0; nt < 4; nt++)
-            wq[sl][nt] = *reinterpret_cast<const u32x4g*>(qw_wave + ((uint32_t)g * 4096u + lane16) + nt * 1024);
+            wq[sl][nt] = *reinterpret_cast<const u32x4g*>((PAIRS && nt > 1 ? qw_wave + up_w : qw_wave) + ((uint32_t)g * 4096u + lane16) + (PAIRS ? nt & 1 : nt) * 1024);
+        if (PAIRS) {
+            auto both = [&](const char* t) { return uint2{*reinterpret_cast<const uint32_t*>(t + ((uint32_t)g * 128u + b8)), *reinterpret_cast<const uint32_t*>(t + up_s + ((uint32_t)g * 128u + b8))}; };
+            scv[sl] = both(sc_wave);
+            if (HAS_ZP) zpv[sl] = both(zp_wave);
+            return;
+        }
         scv[sl] = *reinterpret_cast<const uint2*>(sc_wave + ((uint32_t)g * 128u + b8));
         if (HAS_ZP) zpv[sl] = *reinterpret_cast<const uint2*>(zp_wave + ((uint32_t)g * 128u + b8));
     };
@@ -2410,7 +2430,7 @@ __global__ __launch_bounds__(256, MT <= 6 ? 2 : 1) void w4_gemm_big_kernel(W4Arg
                      : "a"(acc[mt][nt][0]), "a"(acc[mt][nt][1]), "a"(acc[mt][nt][2]), "a"(acc[mt][nt][3]));
         return v;
     };
-    if (MODE != 0) {        // D row 4a + r of tile mt ↔ block row mt·16 + 4a + r, whose pair id lives in lane (·, b = 4a + r)
+    if (MOE) {        // D row 4a + r of tile mt ↔ block row mt·16 + 4a + r, whose pair id lives in lane (·, b = 4a + r)
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
             int orow[4];
@@ -2437,6 +2457,22 @@ __global__ __launch_bounds__(256, MT <= 6 ? 2 : 1) void w4_gemm_big_kernel(W4Arg
                 }
             }
         }
+        return;
+    }
+    if constexpr (PAIRS) {
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+            for (int jj = 0; jj < 2; jj++) {
+                const float4v gt = acc_get(mt, jj), up = acc_get(mt, 2 + jj);
+                const int col = st * 32 + jj * 16 + b;
+                const float b_gate = p.bias ? __half2float(p.bias[col]) : 0.f, b_up = p.bias ? __half2float(p.bias[p.act_im + col]) : 0.f;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int row = rb * ROWS + mt * 16 + 4 * a + r;
+                    if (row < p.M) reinterpret_cast<_Float16*>(p.out)[(long)row * p.ldo + col] = gated_act<MODE == 4>((float)(_Float16)(gt[r] + b_gate), (float)(_Float16)(up[r] + b_up));
+                }
+            }
         return;
     }
     if (p.partial) {
@@ -2573,6 +2609,23 @@ static int launch_w4_slabs(const W4Args& a, int mt, bool has_zp, dim3 grid, hipS
     return launch_w4<0>(a, mt, has_zp, grid, stream);
 }
 
+// ≥ 96 rows: 96- / 128- / 256-row tiles with the group scale folded into the fp16 B operand (w4_gemm_big_kernel) when they
+// fill the chip.  Deep K (≥ 24 groups): the tallest tile whose last round of 256 workgroups is ≥ 70 % full — 4096→28672 at
+// M = 8192: 64-row tiles 905, 96-row 1204, 128-row 1171, 256-row 1277 TFLOP/s (tools/exp_prefill_gemm.py, a throttled
+// back-to-back loop; one prefill of Llama-3.1-8B: 133 → 101 ms).  Shallow K: the 96-row form, two workgroups per CU, whose
+// prologues and epilogues overlap (2048→5120 at M = 8192: 852 / 924 TFLOP/s for 128 / 256 rows, 962 for 96).
+static int w4_big_tiles(const W4Device& w, int m) {
+    const Knobs& kn = knobs();
+    if (kn.w4_big < 0 || m < 96 || w.G % 2) return 0;
+    const int cols = cdiv(w.n64, 4);
+    const long wgs6 = (long)cols * cdiv(m, 96), wgs8 = (long)cols * cdiv(m, 128), wgs16 = (long)cols * cdiv(m, 256);
+    auto fill = [](long wgs) { return (double)wgs / (double)(cdiv(wgs, 256) * 256); };
+    if (kn.w4_big == 6 || kn.w4_big == 8 || kn.w4_big == 16) return m >= 16 * kn.w4_big ? kn.w4_big : 0;       // development: forced
+    if (w.G >= 24 && m >= 256 && wgs16 >= 192 && fill(wgs16) >= 0.7) return 16;
+    if (w.G >= 24 && m >= 128 && wgs8 >= 192 && fill(wgs8) >= 0.7) return 8;
+    return wgs6 >= 128 ? 6 : 0;
+}
+
 // Dense y[M,N] = x[M,K]·Wᵀ (+bias).  One launch: K is split across the waves of each workgroup.
 bool w4_gemm_dense_can_fuse_combine_norm(const W4Device& w, int m) {
     return m >= 1 && m <= 4 && w.qw != nullptr && w.f16t == nullptr && w.perm == nullptr && w.k % 8 == 0 && w.k <= 8192;
@@ -2606,27 +2659,12 @@ int w4_gemm_dense(const W4Device& w, const __half* x, __half* out, int m, float*
     // skinny kernels' four row tiles re-fetch every activation fragment per 16–64 columns (c=48 decode, Llama-3.1-8B 5.18 →
     // 4.02 ms per step, Gemma-3-27B 15.1 → 11.5; the 2048→5120 / 4096→2048 projections of Qwen3-30B-A3B are faster skinny)
     const Knobs& kn = knobs();
-    // ≥ 96 rows: 96- / 128- / 256-row tiles with the group scale folded into the fp16 B operand (w4_gemm_big_kernel) when they
-    // fill the chip.  Deep K (≥ 24 groups): the tallest tile whose last round of 256 workgroups is ≥ 70 % full — 4096→28672 at
-    // M = 8192: 64-row tiles 905, 96-row 1204, 128-row 1171, 256-row 1277 TFLOP/s (tools/exp_prefill_gemm.py, a throttled
-    // back-to-back loop; one prefill of Llama-3.1-8B: 133 → 101 ms).  Shallow K: the 96-row form, two workgroups per CU, whose
-    // prologues and epilogues overlap (2048→5120 at M = 8192: 852 / 924 TFLOP/s for 128 / 256 rows, 962 for 96).
-    if (kn.w4_big >= 0 && m >= 96 && w.G % 2 == 0) {
-        const int cols = cdiv(w.n64, 4);
-        const long wgs6 = (long)cols * cdiv(m, 96), wgs8 = (long)cols * cdiv(m, 128), wgs16 = (long)cols * cdiv(m, 256);
-        auto fill = [](long wgs) { return (double)wgs / (double)(cdiv(wgs, 256) * 256); };
-        int MTv = 0;
-        if (kn.w4_big == 6 || kn.w4_big == 8 || kn.w4_big == 16) MTv = m >= 16 * kn.w4_big ? kn.w4_big : 0;       // development: forced
-        else if (w.G >= 24 && m >= 256 && wgs16 >= 192 && fill(wgs16) >= 0.7) MTv = 16;
-        else if (w.G >= 24 && m >= 128 && wgs8 >= 192 && fill(wgs8) >= 0.7) MTv = 8;
-        else if (wgs6 >= 128) MTv = 6;
-        if (MTv) {
-            a.S = 1; a.partial = nullptr;
-            form_hit(FORM_W4_BIG);
-            const dim3 grid(cols, cdiv(m, 16 * MTv), 1);
-            if (MTv == 6) return launch_big<6>(a, w.zp != nullptr, grid, stream);
-            return MTv == 16 ? launch_big<16>(a, w.zp != nullptr, grid, stream) : launch_big<8>(a, w.zp != nullptr, grid, stream);
-        }
+    if (const int MTv = w4_big_tiles(w, m)) {
+        a.S = 1; a.partial = nullptr;
+        form_hit(FORM_W4_BIG);
+        const dim3 grid(cdiv(w.n64, 4), cdiv(m, 16 * MTv), 1);
+        if (MTv == 6) return launch_big<6>(a, w.zp != nullptr, grid, stream);
+        return MTv == 16 ? launch_big<16>(a, w.zp != nullptr, grid, stream) : launch_big<8>(a, w.zp != nullptr, grid, stream);
     }
 #ifdef FERRUM_HIP_EXPERIMENTS
     if (kn.w4_ldsk && mt >= 2 && w.perm == nullptr) {
@@ -3000,9 +3038,10 @@ int w4_gemm_rows(const W4Device& w, const __half* x, float* slabs, size_t slab_b
     return w.zp ? go(w4_gemm_rows_kernel<true>) : go(w4_gemm_rows_kernel<false>);
 }
 
-// gate_up and its activation in one launch: up to 16 rows of an INT4 projection whose halves are whole column tiles
+// gate_up and its activation in one launch: up to 16 rows, and the prompts that w4_gemm_big_kernel takes, of an INT4 projection whose
+// halves are whole pairs of column tiles
 bool w4_gemm_gated_supports(const W4Device& w, int m, int im) {
-    return m >= 1 && m <= 16 && w.qw && w.n == 2 * im && im % 32 == 0;
+    return w.qw && w.n == 2 * im && im % 32 == 0 && m >= 1 && (m <= 16 || w4_big_tiles(w, m));
 }
 
 int w4_gemm_gated(const W4Device& w, const __half* x, __half* out, int m, int im, int gelu, hipStream_t stream) {
@@ -3011,6 +3050,15 @@ int w4_gemm_gated(const W4Device& w, const __half* x, __half* out, int m, int im
     a.qw = w.qw; a.sc = w.sc; a.zp = w.zp; a.bias = w.bias;
     a.x = x; a.out = out; a.M = m; a.K = w.k; a.N = w.n; a.G = w.G; a.n64 = w.n64; a.ldo = im; a.S = 1;
     a.act_im = im; a.gelu = gelu;
+    form_hit(FORM_W4_GATED);
+    const bool zp = w.zp != nullptr;
+    if (const int MTv = m > 16 ? w4_big_tiles(w, m) : 0) {
+        form_hit(FORM_W4_BIG);
+        const dim3 grid(cdiv(w.n64, 4), cdiv(m, 16 * MTv), 1);
+        if (MTv == 6) return gelu ? launch_big<6, 4>(a, zp, grid, stream) : launch_big<6, 3>(a, zp, grid, stream);
+        if (MTv == 8) return gelu ? launch_big<8, 4>(a, zp, grid, stream) : launch_big<8, 3>(a, zp, grid, stream);
+        return gelu ? launch_big<16, 4>(a, zp, grid, stream) : launch_big<16, 3>(a, zp, grid, stream);
+    }
     // tiles as for the plain projection (w4_gemm_dense), but at least a gate and an up tile, and four waves where those are enough
     // (eight: 4096→28672 14.1 µs against 13.1; 2048→12288, a third of the workgroups, 5.3 against 5.8)
     const int n16 = w.n / 16, nt = cdiv(n16, 4) >= 384 ? 4 : 2;
@@ -3018,7 +3066,6 @@ int w4_gemm_gated(const W4Device& w, const __half* x, __half* out, int m, int im
     int W = 4;
     while (wgs * W < 1024 && W * 2 <= std::min(8, w.G)) W <<= 1;
     while (W > w.G && W > 1) W >>= 1;
-    form_hit(FORM_W4_GATED);
     auto go = [&](auto kernel) -> int {
         hipLaunchKernelGGL(kernel, dim3(wgs), dim3(W * 64), (size_t)W * nt * 4 * 64 * sizeof(float), stream, a);
         FH_CHECK_LAUNCH();

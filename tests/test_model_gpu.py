@@ -104,6 +104,20 @@ def test_few_rows_resident_projections_and_gated_gate_up(pkg, prompt_len, kw, ro
     assert bool(h.get("w4_rows")) == rows, h
 
 
+@pytest.mark.parametrize("big,prompt_len", [(6, 97), (8, 200), (16, 256), (16, 300)])
+@pytest.mark.parametrize("inter,activation,asym", [(384, 0, False), (640, 1, False), (128, 0, True), (1152, 1, True)])
+def test_prompt_gate_up_with_its_activation(pkg, big, prompt_len, inter, activation, asym, knobs, forms):
+    """A wave's two gate tiles and their up tiles in every row size of the large tiles: rows and columns past the last tile, zero points, act-order."""
+    from tests import modelgen
+    knobs.set(W4_BIG=big)
+    kw = dict(sandwich=True, embed_scale=4.0) if activation else {}
+    forms.reset()
+    res = modelgen.run_parity_case(pkg, moe=False, layers=2, prompt_len=prompt_len, decode_steps=0, seed=500 + prompt_len, hidden=256, inter=inter,
+                                   activation=activation, asym_act_order=asym, max_seq_len=320, **kw)
+    _assert_parity(res)
+    assert forms.require("w4_gated", "w4_big")["w4_gated"] == 2
+
+
 @pytest.mark.parametrize("prompt_len", [9, 70])
 def test_act_order_attention_projections_in_a_moe_model(pkg, prompt_len, forms):
     """A MoE checkpoint whose ATTENTION projections are desc_act packs (the expert stacks are natural order here; act-order
