@@ -104,6 +104,34 @@ def test_few_rows_resident_projections_and_gated_gate_up(pkg, prompt_len, kw, ro
     assert bool(h.get("w4_rows")) == rows, h
 
 
+@pytest.mark.parametrize("c", [1, 9, 16])
+def test_resident_down_projection_ahead_of_the_merged_attention_half(pkg, c, knobs, forms):
+    """down's slabs summed by the first role of the next layer's launch, and by the add + norm behind the last layer: against the launches one by one, at one
+    sequence against the oracle."""
+    from tests import modelgen
+    kw = dict(hidden=4096, nq=32, nkv=8, hd=128, inter=1152, vocab=1024, qk_norm=False)
+    if c == 1:
+        forms.reset()
+        _assert_parity(modelgen.run_parity_case(pkg, moe=False, layers=3, prompt_len=5, decode_steps=3, seed=77, **kw))
+        forms.require("dense_chain", "w4_rows", "w4_gated")
+        return
+    tm = modelgen.TinyModel(False, layers=3, seed=78, max_seq_len=64, **kw)
+    rng = np.random.default_rng(5)
+    prompts, toks = [rng.integers(0, 1024, 4).astype(np.uint32) for _ in range(c)], rng.integers(0, 1024, (3, c)).astype(np.uint32)
+    got = {}
+    for name, set_to in (("chain", dict(DENSE_CHAIN=None)), ("launches", dict(DENSE_CHAIN=0)), ("fp16", dict(DENSE_CHAIN=None, DENSE_SLABS=0))):
+        knobs.set(**set_to)
+        hm = tm.hip_model(pkg, kv_num_blocks=2 * c + 2, max_seqs=c, max_tokens=4 * c)
+        hm.unified_forward([(i, p, 0, True) for i, p in enumerate(prompts)], greedy=True)
+        forms.reset()
+        got[name] = [hm.unified_forward([(i, [int(t[i])], 4 + s, True) for i in range(c)], want_logits=True)[1].copy() for s, t in enumerate(toks)]
+        h = forms.hits()
+        assert h.get("w4_rows", 0) == {"chain": 9, "launches": 18, "fp16": 0}[name] and bool(h.get("dense_chain")) == (name != "launches"), h
+    for name in ("chain", "launches"):
+        for a, b in zip(got[name], got["fp16"]):
+            assert np.abs(a - b).max() < 0.02 * np.abs(b).max()
+
+
 @pytest.mark.parametrize("big,prompt_len", [(6, 97), (8, 200), (16, 256), (16, 300)])
 @pytest.mark.parametrize("inter,activation,asym", [(384, 0, False), (640, 1, False), (128, 0, True), (1152, 1, True)])
 def test_prompt_gate_up_with_its_activation(pkg, big, prompt_len, inter, activation, asym, knobs, forms):
