@@ -117,7 +117,9 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(TiledGemm<E> p, int kw)
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int j = 0; j < J; j++) acc[mt][j] = (floatx4){0.f, 0.f, 0.f, 0.f};
-    constexpr int U = sizeof(E) == 2 ? (MT * J == 1 ? 8 : 4) : 1;
+    // (four row tiles by two: two k-steps, 150 registers; four spilled, which cost 13 % — 60 × 8192 × 2048 16.9 → 14.7 µs, 100 × 6144 × 2048
+    // 25.6 → 21.4 — and made every stream's first launch allocate scratch memory, 10 ms)
+    constexpr int U = sizeof(E) == 2 ? (MT * J == 1 ? 8 : MT * J == 8 ? 2 : 4) : 1;
     v8 bw[2][U][J], ax[2][U][MT];
     auto load = [&](v8 (&bq)[U][J], v8 (&aq)[U][MT], int s) {
 #pragma unroll
@@ -533,7 +535,7 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     //   8 × 1024 × 3072           8.0             6.5            7.4 (16, eight waves, kw 8)
     //   32 × 8192 × 2048         10.7                   12.4     13.9 (16, four waves, kw 4)
     //   32 × 2048 × 2048          9.4             8.4            8.4
-    //   60 × 8192 × 2048         17.1                   20.1     20.8
+    //   60 × 8192 × 2048         14.7                   20.1     20.8
     // Fewer waves a workgroup wait for each other less.  Several row tiles, whose fragments a wave reads again for every column group: 32 columns
     // sooner.  Slabs of a long K want every wave they can get (1 × 2048 × 8192 in four: eight waves 8.1, four 8.4).
     const bool long_slabs = g.slabs > 1 && ksteps / g.slabs >= 64, narrow = sizeof(E) == 4 || long_slabs;

@@ -3029,13 +3029,16 @@ int w4_gemm_rows(const W4Device& w, const __half* x, float* slabs, size_t slab_b
     form_hit(FORM_W4_ROWS);
     const size_t lds = (size_t)1024 * std::max(cdiv(w.G, S) * 4, 2 * W4_ROWS_TILES);
     const dim3 grid(cdiv(w.n64, W4_ROWS_TILES / 4), S);
-    auto go = [&](auto kernel) -> int {
-        FH_CHECK_HIP(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, W4_ROWS_LDS));
-        hipLaunchKernelGGL(kernel, grid, dim3(512), lds, stream, a);
-        FH_CHECK_LAUNCH();
-        return 0;
-    };
-    return w.zp ? go(w4_gemm_rows_kernel<true>) : go(w4_gemm_rows_kernel<false>);
+    static bool attr = false;
+    if (!attr) {
+        FH_CHECK_HIP(hipFuncSetAttribute((const void*)w4_gemm_rows_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, W4_ROWS_LDS));
+        FH_CHECK_HIP(hipFuncSetAttribute((const void*)w4_gemm_rows_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, W4_ROWS_LDS));
+        attr = true;
+    }
+    if (w.zp) hipLaunchKernelGGL(w4_gemm_rows_kernel<true>, grid, dim3(512), lds, stream, a);
+    else hipLaunchKernelGGL(w4_gemm_rows_kernel<false>, grid, dim3(512), lds, stream, a);
+    FH_CHECK_LAUNCH();
+    return 0;
 }
 
 // gate_up and its activation in one launch: up to 16 rows, and the prompts that w4_gemm_big_kernel takes, of an INT4 projection whose
