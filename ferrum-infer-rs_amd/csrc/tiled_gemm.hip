@@ -117,8 +117,8 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(TiledGemm<E> p, int kw)
     for (int mt = 0; mt < MT; mt++)
 #pragma unroll
         for (int j = 0; j < J; j++) acc[mt][j] = (floatx4){0.f, 0.f, 0.f, 0.f};
-    // (four row tiles by two: two k-steps, 150 registers; four spilled, which cost 13 % — 60 × 8192 × 2048 16.9 → 14.7 µs, 100 × 6144 × 2048
-    // 25.6 → 21.4 — and made every stream's first launch allocate scratch memory, 10 ms)
+    // (four row tiles by two: two k-steps, 150 registers; four spilled, which cost 13 %: 60 × 8192 × 2048 16.9 → 14.7 µs, 100 × 6144 × 2048
+    // 25.6 → 21.4)
     constexpr int U = sizeof(E) == 2 ? (MT * J == 1 ? 8 : MT * J == 8 ? 2 : 4) : 1;
     v8 bw[2][U][J], ax[2][U][MT];
     auto load = [&](v8 (&bq)[U][J], v8 (&aq)[U][MT], int s) {
