@@ -2555,13 +2555,16 @@ static int launch_ldsa(const W4Args& a_in, bool has_zp, dim3 grid, hipStream_t s
 #include "experiments_w4_decode_launchers.inc"
 #endif
 
+// LDS of the fused combine + add + norm prologue (≤ 4 rows), and what it may take together with the waves' sums
+constexpr size_t WGSPLIT_FUSED_LDS = 64 * 1024;
+static size_t wgsplit_fused_lds(int m, int k) { return (size_t)m * (k + 8) * sizeof(__half) + 64 * sizeof(float); }
 template <int MT, int NT>
 static int launch_wgsplit(const W4Args& a, bool has_zp, dim3 grid, int W, hipStream_t stream) {
     size_t lds = (size_t)W * MT * NT * 4 * 64 * sizeof(float);
     if constexpr (MT == 1) {
         if (a.fa_down) {                                       // fused combine + add + norm prologue (≤ 4 rows)
-            lds += (size_t)a.M * (a.K + 8) * sizeof(__half) + 64 * sizeof(float);
-            FH_REQUIRE(lds <= 64 * 1024, "w4_gemm_dense: fused prologue needs %zu bytes of LDS", lds);
+            lds += wgsplit_fused_lds(a.M, a.K);
+            FH_REQUIRE(lds <= WGSPLIT_FUSED_LDS, "w4_gemm_dense: fused prologue needs %zu bytes of LDS", lds);
             form_hit(FORM_W4_FUSED_TAIL);
             if (has_zp) hipLaunchKernelGGL((w4_gemm_wgsplit_kernel<1, NT, true, true>), grid, dim3(W * 64), lds, stream, a);
             else hipLaunchKernelGGL((w4_gemm_wgsplit_kernel<1, NT, false, true>), grid, dim3(W * 64), lds, stream, a);
@@ -2626,9 +2629,42 @@ static int w4_big_tiles(const W4Device& w, int m) {
     return wgs6 >= 128 ? 6 : 0;
 }
 
+// Column tiles and waves (= K slices) of a workgroup of w4_gemm_wgsplit_kernel over `row_blocks` blocks of mt row tiles; fa_lds: bytes of LDS that
+// the fused combine + norm prologue takes beside the waves' sums (0: no prologue).
+struct WgSplit { int nt, W; };
+static WgSplit wgsplit_shape(const W4Device& w, int mt, int row_blocks, size_t fa_lds) {
+    const int n16 = w.n64 * 4;
+    auto waves = [&](int nt) {
+        // enough waves to cover the chip, ≥ 1 group each, LDS ≤ 128 KiB
+        const long wgs = (long)cdiv(n16, nt) * row_blocks;
+        const int w_cap = mt == 1 ? 16 : (mt == 2 ? (nt == 1 ? 16 : 8) : 4);    // matches the kernel's __launch_bounds__
+        int W = 4;
+        while (wgs * W < 2048 && W * 2 <= std::min(w_cap, w.G) && W * 2 * mt * nt * 4 <= 512) W <<= 1;
+        while (W > w.G && W > 1) W >>= 1;
+        return W;
+    };
+    auto fits = [&](int nt, int W) { return !fa_lds || fa_lds + (size_t)W * nt * 1024 <= WGSPLIT_FUSED_LDS; };
+    // column tiles per workgroup: as wide as possible (A-fragment reuse) while ≥ ~384 workgroups exist
+    int nt = 4;
+    while (nt > 1 && (long)cdiv(n16, nt) * row_blocks < 384) nt >>= 1;
+    // … but one row tile takes two column tiles rather than one where those are more than a round of 256 workgroups: every tile reads
+    // the rows again (5376→8192 at 5 / 12 rows 8.9 → 7.0 / 11.6 → 8.3 µs, 4096→6144 7.0 → 5.6 / 9.2 → 6.6, 2048→5120 4.8 → 3.8 / 5.9
+    // → 4.4); 4096→4096 keeps one: 4.9 / 6.1 against 5.3 / 6.5
+    if (mt == 1 && nt == 1 && (long)n16 * row_blocks > 256) nt = 2;
+    // with ≥ 2 row tiles the activation fragments dominate the load traffic: share each across two
+    // column tiles as long as ≥ 128 workgroups remain (measured: qkv 2048→5120 at T=32 10.4 → 7.2 µs)
+    if (mt >= 2 && nt == 1 && (long)cdiv(n16, 2) * row_blocks >= 128) nt = 2;
+    // (beside the prologue's rows: narrower, then fewer waves)
+    while (nt > 1 && !fits(nt, waves(nt))) nt >>= 1;
+    int W = waves(nt);
+    while (W > 1 && !fits(nt, W)) W >>= 1;
+    return {nt, W};
+}
+
 // Dense y[M,N] = x[M,K]·Wᵀ (+bias).  One launch: K is split across the waves of each workgroup.
 bool w4_gemm_dense_can_fuse_combine_norm(const W4Device& w, int m) {
-    return m >= 1 && m <= 4 && w.qw != nullptr && w.f16t == nullptr && w.perm == nullptr && w.k % 8 == 0 && w.k <= 8192;
+    return m >= 1 && m <= 4 && w.qw != nullptr && w.f16t == nullptr && w.perm == nullptr && w.k % 8 == 0 && w.k <= 8192 &&
+           wgsplit_fused_lds(m, w.k) + 4 * 1024 <= WGSPLIT_FUSED_LDS;            // (four waves of one column tile)
 }
 
 int w4_gemm_dense(const W4Device& w, const __half* x, __half* out, int m, float* workspace,
@@ -2735,22 +2771,7 @@ int w4_gemm_dense(const W4Device& w, const __half* x, __half* out, int m, float*
         return 0;
     }
     const int n16 = w.n64 * 4;
-    // column tiles per workgroup: as wide as possible (A-fragment reuse) while ≥ ~384 workgroups exist
-    int nt = 4;
-    while (nt > 1 && (long)cdiv(n16, nt) * row_blocks < 384) nt >>= 1;
-    // … but one row tile takes two column tiles rather than one where those are more than a round of 256 workgroups: every tile reads
-    // the rows again (5376→8192 at 5 / 12 rows 8.9 → 7.0 / 11.6 → 8.3 µs, 4096→6144 7.0 → 5.6 / 9.2 → 6.6, 2048→5120 4.8 → 3.8 / 5.9
-    // → 4.4); 4096→4096 keeps one: 4.9 / 6.1 against 5.3 / 6.5
-    if (mt == 1 && nt == 1 && (long)n16 * row_blocks > 256) nt = 2;
-    // with ≥ 2 row tiles the activation fragments dominate the load traffic: share each across two
-    // column tiles as long as ≥ 128 workgroups remain (measured: qkv 2048→5120 at T=32 10.4 → 7.2 µs)
-    if (mt >= 2 && nt == 1 && (long)cdiv(n16, 2) * row_blocks >= 128) nt = 2;
-    // waves per workgroup (= K slices): enough waves to cover the chip, ≥ 1 group each, LDS ≤ 128 KiB
-    const long wgs = (long)cdiv(n16, nt) * row_blocks;
-    const int w_cap = mt == 1 ? 16 : (mt == 2 ? (nt == 1 ? 16 : 8) : 4);    // matches the kernel's __launch_bounds__
-    int W = 4;
-    while (wgs * W < 2048 && W * 2 <= std::min(w_cap, w.G) && W * 2 * mt * nt * 4 <= 512) W <<= 1;
-    while (W > w.G && W > 1) W >>= 1;
+    auto [nt, W] = wgsplit_shape(w, mt, row_blocks, fa ? wgsplit_fused_lds(m, w.k) : 0);
     if (kn.w4_nt) nt = kn.w4_nt;        // tuning overrides (development)
     if (kn.w4_w) W = kn.w4_w;
     dim3 grid(cdiv(n16, nt), row_blocks, 1);

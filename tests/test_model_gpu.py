@@ -132,6 +132,22 @@ def test_resident_down_projection_ahead_of_the_merged_attention_half(pkg, c, kno
             assert np.abs(a - b).max() < 0.02 * np.abs(b).max()
 
 
+@pytest.mark.parametrize("hidden,nq,nkv,fused", [
+    (4096, 32, 8, True),         # 384 column tiles: two of a workgroup and sixteen waves would take 66 KB beside four rows of 4096
+    (4096, 64, 16, True),        # 768: two without the rule for one row tile
+    (7680, 8, 2, False),         # four rows leave no room for four waves
+    (7552, 8, 2, True)])
+def test_fused_layer_tail_of_four_rows(pkg, hidden, nq, nkv, fused, monkeypatch, forms):
+    """The combine + add + norm prologue of the next q|k|v at its largest number of rows, where its LDS bounds the shape of the workgroup."""
+    from tests import modelgen
+    monkeypatch.setenv("FERRUM_HIP_FUSE_TAIL_ROWS", "4")
+    forms.reset()
+    res = modelgen.run_parity_case(pkg, moe=True, layers=2, prompt_len=4, decode_steps=0, seed=600, hidden=hidden, nq=nq, nkv=nkv, hd=128, experts=32,
+                                   expert_inter=128, max_seq_len=64)
+    assert bool(forms.hits().get("w4_fused_tail")) == fused
+    _assert_parity(res)
+
+
 @pytest.mark.parametrize("big,prompt_len", [(6, 97), (8, 200), (16, 256), (16, 300)])
 @pytest.mark.parametrize("inter,activation,asym", [(384, 0, False), (640, 1, False), (128, 0, True), (1152, 1, True)])
 def test_prompt_gate_up_with_its_activation(pkg, big, prompt_len, inter, activation, asym, knobs, forms):
