@@ -129,12 +129,23 @@ __global__ void decode_advance_kernel(const uint32_t* __restrict__ sampled, uint
 // launch in place of a copy of the whole block, whose places for prompt tokens a decode step does not use, and a fill; the sampled ids
 // are written where the host reads them.  A call of one step costs 16 – 29 µs more than a step of a long call; with the copies, and one
 // of the ids into pageable memory, 30 – 64 µs.
+// Bound by the round trip to the host, so all of it is requested at once: a workgroup per 1024 words, four of a thread before its first store.
+// The block tables are n × the longest possible one, whatever is in use.  A call of one step, two small layers (µs): the copies / four workgroups a part,
+// a word a thread and round trip / this:
+//   64 sequences × 32 blocks      153 / 138 / 137          64 × 2048      196 / 321 / 173
+//   8 × 2048                      104 / 102 /  83          256 × 2048     328 / 903 / 313
 struct IndexParts { int n = 0, word[10], words[10]; };
+constexpr int BEGIN_LOADS = 4, BEGIN_WORDS = 256 * BEGIN_LOADS;
 __global__ __launch_bounds__(256) void decode_begin_kernel(const uint32_t* __restrict__ host, uint32_t* __restrict__ dev, IndexParts p, int32_t* __restrict__ step_counter) {
-    const int w0 = p.word[blockIdx.y], n = p.words[blockIdx.y];
-    for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256)
-        dev[w0 + i] = __hip_atomic_load(host + w0 + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    const int w0 = p.word[blockIdx.y], n = p.words[blockIdx.y], first = blockIdx.x * BEGIN_WORDS + threadIdx.x;
     if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 2) step_counter[threadIdx.x] = 0;
+    if (first >= n) return;
+    uint32_t v[BEGIN_LOADS];
+#pragma unroll
+    for (int j = 0; j < BEGIN_LOADS; j++) v[j] = __hip_atomic_load(host + w0 + min(first + 256 * j, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+#pragma unroll
+    for (int j = 0; j < BEGIN_LOADS; j++)
+        if (first + 256 * j < n) dev[w0 + first + 256 * j] = v[j];
 }
 
 __global__ void f16_to_f32_kernel(const __half* __restrict__ src, float* __restrict__ dst, long n) {
@@ -2177,7 +2188,8 @@ int ferrum_hip_model_decode_steps(FerrumHipModel* m, const uint64_t* seq_ids, co
             m->graph_max_kv = kv_bucket;
         }
     }
-    hipLaunchKernelGGL(decode_begin_kernel, dim3(4, parts.n), dim3(256), 0, m->stream, reinterpret_cast<const uint32_t*>(m->idx_host),
+    const int most = *std::max_element(parts.words, parts.words + parts.n);
+    hipLaunchKernelGGL(decode_begin_kernel, dim3(cdiv(most, BEGIN_WORDS), parts.n), dim3(256), 0, m->stream, reinterpret_cast<const uint32_t*>(m->idx_host),
                        reinterpret_cast<uint32_t*>(m->idx_dev), parts, m->step_counter);
     FH_CHECK_LAUNCH();
     if (graph_ok) {

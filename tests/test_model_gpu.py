@@ -148,6 +148,30 @@ def test_fused_layer_tail_of_four_rows(pkg, hidden, nq, nkv, fused, monkeypatch,
     _assert_parity(res)
 
 
+def test_long_block_tables_are_handed_over_at_once(pkg):
+    """A decode call of 64 sequences hands 64 whole rows of the block table over: the same ids from short tables and from rows of 2048 blocks, and the long ones
+    cost the call what moving and writing 512 KiB takes (a DMA copy 45 us more, one word a thread and round trip 185 us)."""
+    import time
+    ids, best = {}, {}
+    models = {}
+    for span in (512, 32768):
+        m = pkg.HipModel(group_size=128, num_layers=2, hidden=256, num_heads=4, num_kv_heads=2, head_dim=128, intermediate=256, vocab=512, has_qk_norm=1, activation=0,
+                         rms_eps=1e-6, rope_theta=1e6, max_seq_len=span, kv_num_blocks=64 * 20, max_seqs=64, max_tokens=64 * 64)
+        m.init_synthetic(3)
+        m.finalize()
+        rng = np.random.default_rng(4)
+        m.unified_forward([(i, rng.integers(0, 512, 17 + (i * 5) % 40).astype(np.uint32), 0, True) for i in range(64)], greedy=True)
+        ids[span], best[span], models[span] = [m.decode_steps(range(64), [i + 7 for i in range(64)], 3)], float("inf"), m
+    for _ in range(40):                                                                   # (in turn, so that a slow moment of the host meets both)
+        for span, m in models.items():
+            t = time.perf_counter()
+            out = m.decode_steps(range(64), [i + 7 for i in range(64)], 1)
+            best[span] = min(best[span], time.perf_counter() - t)
+            ids[span].append(out)
+    assert all(np.array_equal(a, b) for a, b in zip(ids[512], ids[32768]))
+    assert best[32768] - best[512] < 110e-6, best
+
+
 @pytest.mark.parametrize("big,prompt_len", [(6, 97), (8, 200), (16, 256), (16, 300)])
 @pytest.mark.parametrize("inter,activation,asym", [(384, 0, False), (640, 1, False), (128, 0, True), (1152, 1, True)])
 def test_prompt_gate_up_with_its_activation(pkg, big, prompt_len, inter, activation, asym, knobs, forms):
