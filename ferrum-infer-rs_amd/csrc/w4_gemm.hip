@@ -1507,7 +1507,7 @@ __global__ __launch_bounds__(MT == 1 ? (GATED ? 512 : 1024) : (MT == 2 ? (NT == 
 // The waves of w4_gemm_wgsplit_kernel read the activations of every column tile again: 4 KiB of 16-row fragments for each KiB of
 // weights where a workgroup has one tile, so that its time grows with the rows (14336→4096: 10.4 µs at 1 row, 14.5 at 12, 16.9 at 16)
 // while the weights stay the same.  Here a workgroup takes 128 columns and 1 / S of K: its rows of x come to LDS once (fragment-major,
-// one copy without registers), behind them the first weights, and after one barrier its eight waves — two tiles by half of its K
+// one copy without registers) together with the first weights, and after one barrier its eight waves — two tiles by half of its K
 // each — stream weights alone, two groups ahead; the halves meet in LDS and one slab of S leaves.  The consumer that exists anyway
 // (add + norm, the first role of the next layer's launch) sums the slabs in order.  S fills the chip with one round of workgroups.
 //   us, old → this with S slabs          1 row         5 rows        12 rows       16 rows
@@ -1557,6 +1557,7 @@ __global__ __launch_bounds__(512) void w4_gemm_rows_kernel(W4Args p) {
     };
 #pragma unroll
     for (int d = 0; d < DW; d++) issue(d, g0 + d);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                   // (every wave's rows have landed)
     __syncthreads();
     int i = 0;
     for (; i + DW <= ng; i += DW)
