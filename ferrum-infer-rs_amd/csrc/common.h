@@ -122,7 +122,8 @@ __device__ __forceinline__ void reduce_slabs8(const float* __restrict__ base, lo
 }
 
 // act(gate) · up of a gated MLP: SiLU, or GELU in its tanh form, ½·g·(1 + tanh z) = g / (1 + exp(−2z)) — without the cancellation of 1 + tanh
-// left of zero, and a third of tanhf's instructions (one definition: the fused and the separate launches give the same bits)
+// left of zero, and a third of tanhf's instructions.  INT4 projections take it in fused and separate launches alike, on gate and up rounded to
+// fp16: the same bits.  (Unquantised ones apply gemm_glu to their fp32 sums.)
 template <bool GELU>
 __device__ __forceinline__ _Float16 gated_act(float g, float u) {
     if (GELU) {

@@ -98,7 +98,7 @@ template <typename E> int tiled_gemm(const TiledGemm<E>& g, hipStream_t s);
 constexpr int GEMM_MAX_SLABS = 8;
 int tiled_gemm_slabs(int m, int n, int k);
 
-// Activations on fp32 accumulators.  Models in 16 bits round the result to 2⁻⁹, so their form uses the hardware exponential and
+// Activations on fp32 accumulators.  Models in 16 bits round the result to 2⁻⁹ or 2⁻¹², so their form uses the hardware exponential and
 // reciprocal (relative error ≈ 2⁻²²); 32-bit models call the library functions.
 template <typename E> struct ActMath;
 template <> struct ActMath<float> {
@@ -118,9 +118,13 @@ template <> struct ActMath<bf16> {
     }
 };
 template <> struct ActMath<_Float16> : ActMath<bf16> {};
+// ½·z·(1 + tanh t) = z·σ(2t): in 16 bits as the latter, whose relative error stays that of the exponential where 1 + tanh t cancels (left of −2
+// the former was off by more than fp16's rounding, left of −5 by as much as the result)
 template <typename E>
 __device__ __forceinline__ float gelu_tanh_f32(float z) {
-    return 0.5f * z * (1.0f + ActMath<E>::tanh(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+    const float t = 0.7978845608028654f * (z + 0.044715f * z * z * z);
+    if (sizeof(E) == 2) return z * ActMath<E>::sigmoid(2.0f * t);
+    return 0.5f * z * (1.0f + ActMath<E>::tanh(t));
 }
 // gate bounded from above, linear half on both sides
 template <typename E>

@@ -257,6 +257,44 @@ def test_unquantised_gate_up_with_its_activation(pkg, prompt_len, inter, wide, h
     _assert_parity(res)
 
 
+@pytest.mark.parametrize("tokens", [1, 100])
+@pytest.mark.parametrize("activation,lo,hi", [(1, -5.5, -2.0), (1, -2.0, 3.0), (0, -12.0, 12.0)])
+def test_unquantised_activation_errs_by_its_rounding(pkg, activation, lo, hi, tokens, knobs, forms):
+    """One layer whose every product is a single exact one: gate and up are given numbers, down copies, nothing else is added.  What is left is the activation in
+    fp32 (arguments of the exponential up to 21, so 2 x 21 x 2^-23 of their rounding and as much again for the rest) and one rounding to fp16."""
+    H, I = 256, 1024
+    rng = np.random.default_rng(7)
+    m = pkg.HipModel(group_size=128, num_layers=1, hidden=H, num_heads=2, num_kv_heads=1, head_dim=128, intermediate=I, vocab=256, has_qk_norm=0, activation=activation,
+                     rms_eps=1e-12, rope_theta=1e6, max_seq_len=128, kv_num_blocks=16, max_seqs=2, max_tokens=128)
+    one = lambda rows, cols, at: np.float32(np.arange(cols)[None] == at) * np.ones((rows, 1), np.float32)
+    embed = one(256, H, 0) * 4.0                                        # normed: sqrt(256) in column 0
+    gate = np.float16(rng.uniform(lo, hi, I) / 16).astype(np.float32)
+    up = np.float32(2.0) ** rng.integers(-3, 0, I) * (4094 * 2 if hi < 0 else 2.0)      # (left of zero: 65504 and less, so that the results are normal)
+    m.set_global("embed", embed)
+    m.set_global("lm_head", embed)
+    m.set_global("final_norm", np.ones(H, np.float32))
+    for name in ("input_ln", "post_ln"):
+        m.set_layer_dense(0, name, np.ones(H, np.float32))
+    m.set_dense(0, "qkv", np.zeros((512, H), np.float32), H, 512)
+    m.set_dense(0, "o", np.zeros((H, 256), np.float32), 256, H)
+    m.set_dense(0, "gate_up", np.concatenate([gate, up])[:, None] * one(2 * I, H, 0), H, 2 * I)
+    down = np.zeros((H, I), np.float32)
+    down[np.arange(1, 256), np.arange(1, 256)] = 1.0
+    m.set_dense(0, "down", down, I, H)
+    m.finalize()
+    m.enable_taps()
+    knobs.set(TILED_BIG_MIN_TILES=1 if tokens > 64 else 10 ** 6)
+    forms.reset()
+    m.unified_forward([(0, np.arange(tokens, dtype=np.uint32), 0, True)], greedy=True)
+    forms.require("f16_gated", "tiled_gemm_big" if tokens > 64 else "tiled_gemm")
+    got = m.read_taps(tokens)[0][:, 1:256].astype(np.float64)
+    g, u = 16.0 * gate[1:256].astype(np.float64), 16.0 * up[1:256].astype(np.float64)
+    t = 2 * 0.7978845608028654 * (g + 0.044715 * g ** 3) if activation else g
+    want = g / (1.0 + np.exp(-t)) * u
+    assert np.abs(want).min() > 2.0 ** -14                               # (normal in fp16)
+    assert (np.abs(got - want) <= (2.0 ** -11 + 4 * 21 * 2.0 ** -23) * np.abs(want)).all()
+
+
 def test_qwen3_06b_dims_unquantised_layer(pkg, forms):
     """BASELINE configs[0] (Qwen3-0.6B: H 1024, 16/8 heads × 128, I 3072, QK-norm, θ 1e6, tied lm_head, unquantised weights) —
     one layer at its real dimensions (vocabulary cut to 2048), 24 sequences: 40-token prompts in one forward, then three
