@@ -186,7 +186,7 @@ int ferrum_hip_alloc(void** dev_ptr, size_t bytes) {
     *dev_ptr = nullptr;
     if (bytes == 0) return 0;
     FH_CHECK_HIP(hipMalloc(dev_ptr, bytes));
-    FH_CHECK_HIP(hipMemset(*dev_ptr, 0, bytes));
+    FH_CHECK_HIP(device_zero(*dev_ptr, bytes));
     return 0;
 }
 int ferrum_hip_free(void* dev_ptr) { if (dev_ptr) FH_CHECK_HIP(hipFree(dev_ptr)); return 0; }
@@ -561,7 +561,7 @@ int ferrum_hip_moe_gemm_phase_expert_major_pair_f16(FerrumHipGptq* gate_up_stack
         g->pair_arrive = nullptr;
         const size_t words = (size_t)2 * num_experts * MOE_PAIR_COUNTER_STRIDE + 4;
         FH_CHECK_HIP(hipMalloc((void**)&g->pair_arrive, words * sizeof(unsigned)));
-        FH_CHECK_HIP(hipMemset(g->pair_arrive, 0, words * sizeof(unsigned)));
+        FH_CHECK_HIP(device_zero(g->pair_arrive, words * sizeof(unsigned)));
         g->pair_experts = num_experts;
     }
     // op level: the counters are zeroed by a memset node in front of every launch (a captured call replays with the same
@@ -600,7 +600,7 @@ int ferrum_hip_moe_gemm_phase_block_major_pair_f16(FerrumHipGptq* gate_up_stack,
         g->pair_arrive = nullptr;
         const size_t words = (size_t)2 * num_experts * MOE_PAIR_COUNTER_STRIDE + 4;
         FH_CHECK_HIP(hipMalloc((void**)&g->pair_arrive, words * sizeof(unsigned)));
-        FH_CHECK_HIP(hipMemset(g->pair_arrive, 0, words * sizeof(unsigned)));
+        FH_CHECK_HIP(device_zero(g->pair_arrive, words * sizeof(unsigned)));
         g->pair_experts = num_experts;
     }
     unsigned* arrive = g->pair_arrive;

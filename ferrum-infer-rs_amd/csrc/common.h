@@ -133,6 +133,13 @@ __device__ __forceinline__ _Float16 gated_act(float g, float u) {
     return (_Float16)(g / (1.0f + __expf(-g)) * u);
 }
 
+// Device memory to zero, done on return: a fill by hipMemset is only queued on the null stream by then (8 GiB: 1.4 ms later), and streams made with
+// hipStreamNonBlocking, which all of this library's are, do not wait for that one.
+static inline hipError_t device_zero(void* p, size_t bytes) {
+    const hipError_t e = hipMemset(p, 0, bytes);
+    return e == hipSuccess ? hipStreamSynchronize(nullptr) : e;
+}
+
 static inline hipStream_t as_stream(void* s) { return reinterpret_cast<hipStream_t>(s); }
 static inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 __host__ __device__ inline int cdiv_dev(int a, int b) { return (a + b - 1) / b; }

@@ -66,7 +66,7 @@ public:
         if (!n) return 0;
         FH_CHECK_HIP(hipMalloc((void**)p, n * sizeof(T)));
         mem_.push_back(*p);
-        FH_CHECK_HIP(hipMemset(*p, 0, n * sizeof(T)));
+        FH_CHECK_HIP(device_zero(*p, n * sizeof(T)));
         return 0;
     }
     template <typename T> int upload(T** p, const std::vector<T>& v) {

@@ -38,7 +38,7 @@ int dev_alloc(T** p, size_t count) {
     *p = nullptr;
     if (!count) return 0;
     FH_CHECK_HIP(hipMalloc((void**)p, count * sizeof(T)));
-    FH_CHECK_HIP(hipMemset(*p, 0, count * sizeof(T)));
+    FH_CHECK_HIP(device_zero(*p, count * sizeof(T)));
     return 0;
 }
 
@@ -782,7 +782,7 @@ static int finalize_batch_buffers(FerrumHipModel* m) {
     m->il.total = off;
     FH_CHECK_HIP(hipHostMalloc((void**)&m->idx_host, off, hipHostMallocDefault));
     FH_CHECK_HIP(hipMalloc((void**)&m->idx_dev, off));
-    FH_CHECK_HIP(hipMemset(m->idx_dev, 0, off));
+    FH_CHECK_HIP(device_zero(m->idx_dev, off));
     if (int r = dev_alloc(&m->step_counter, (size_t)4)) return r;
     return 0;
 }

@@ -460,11 +460,11 @@ int oneshot_alloc(FerrumHipComm* c, size_t max_bytes) {
         c->buf = nullptr;
         FH_CHECK_HIP(hipMalloc((void**)&c->buf, total));
     }
-    FH_CHECK_HIP(hipMemset(c->buf, 0, total));
+    FH_CHECK_HIP(device_zero(c->buf, total));
     FH_CHECK_HIP(hipHostMalloc((void**)&c->timeouts_host, 64, hipHostMallocDefault));
     *c->timeouts_host = 0u;
     FH_CHECK_HIP(hipMalloc((void**)&c->state, 64));
-    FH_CHECK_HIP(hipMemset(c->state, 0, 64));
+    FH_CHECK_HIP(device_zero(c->state, 64));
     FH_CHECK_HIP(hipMalloc((void**)&c->peers_dev, sizeof(void*) * 8));
     FH_CHECK_HIP(hipDeviceSynchronize());
     return 0;

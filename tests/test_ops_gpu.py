@@ -303,6 +303,24 @@ def test_dense_gemm_tile_edges(env, m, n, k, f32out):
         assert bool((buf[:shift] == 7.0).all()) and bool((buf[shift + m * n:] == 7.0).all())
 
 
+def test_allocated_memory_is_zero_on_return(env):
+    """What another stream writes into new memory stays: no fill is on its way any more (a gigabyte of it takes 0.2 ms, this write a tenth of that)."""
+    import ctypes as C
+    lib = env[0].load_library()
+    stream, p, size = C.c_void_p(), C.c_void_p(), 4 << 30
+    want, got = (C.c_uint8 * 64)(*[7] * 64), (C.c_uint8 * 64)()
+    assert lib.ferrum_hip_stream_create(C.byref(stream)) == 0
+    for _ in range(3):
+        assert lib.ferrum_hip_alloc(C.byref(p), C.c_size_t(size)) == 0
+        end = C.c_void_p(p.value + size - 128)
+        assert lib.ferrum_hip_memcpy_h2d(end, want, C.c_size_t(64), stream) == 0
+        assert lib.ferrum_hip_stream_synchronize(None) == 0
+        assert lib.ferrum_hip_memcpy_d2h(got, end, C.c_size_t(64), stream) == 0 and bytes(got) == bytes(want)
+        assert lib.ferrum_hip_memcpy_d2h(got, C.c_void_p(end.value + 64), C.c_size_t(64), stream) == 0 and not any(got)
+        assert lib.ferrum_hip_free(p) == 0
+    assert lib.ferrum_hip_stream_destroy(stream) == 0
+
+
 # ── paged KV write / read ────────────────────────────────────────────────────
 def _rope(O, hd, max_seq, theta=1e6):
     return O.build_rope_cache(theta, hd, max_seq)
