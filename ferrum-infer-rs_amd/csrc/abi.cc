@@ -208,9 +208,7 @@ int ferrum_hip_memcpy_d2d(void* dst, const void* src, size_t bytes, void* stream
     return 0;
 }
 int ferrum_hip_memset_zero(void* p, size_t bytes, void* stream) {
-    if (bytes == 0) return 0;
-    FH_CHECK_HIP(hipMemsetAsync(p, 0, bytes, ST(stream)));
-    return 0;
+    return zero_async(p, bytes, ST(stream));
 }
 
 int ferrum_hip_workspace_create(FerrumHipWorkspace** ws, size_t bytes) {
@@ -564,11 +562,11 @@ int ferrum_hip_moe_gemm_phase_expert_major_pair_f16(FerrumHipGptq* gate_up_stack
         FH_CHECK_HIP(device_zero(g->pair_arrive, words * sizeof(unsigned)));
         g->pair_experts = num_experts;
     }
-    // op level: the counters are zeroed by a memset node in front of every launch (a captured call replays with the same
+    // op level: the counters are zeroed by a launch in front of every other (a captured call replays with the same
     // pointers, so the runner's alternating halves do not apply); the give-up word is checked by ferrum_hip_moe_pair_status
     unsigned* arrive = g->pair_arrive;
     const size_t half = (size_t)g->pair_experts * MOE_PAIR_COUNTER_STRIDE;
-    FH_CHECK_HIP(hipMemsetAsync(arrive, 0, half * sizeof(unsigned), ST(stream)));
+    if (int rc = zero_async(arrive, half * sizeof(unsigned), ST(stream))) return rc;
     int took = 0;
     if (int rc = w4_gemm_moe_expert_major_pair(g->dev, down_stack->dev, x_in, H(act_out), H(output), expert_ids_per_pair, num_experts,
                                                prob_m, top_k, arrive, arrive + half, arrive + 2 * half, &took, ST(stream)))
@@ -605,7 +603,7 @@ int ferrum_hip_moe_gemm_phase_block_major_pair_f16(FerrumHipGptq* gate_up_stack,
     }
     unsigned* arrive = g->pair_arrive;
     const size_t half = (size_t)g->pair_experts * MOE_PAIR_COUNTER_STRIDE;
-    FH_CHECK_HIP(hipMemsetAsync(arrive, 0, half * sizeof(unsigned), ST(stream)));
+    if (int rc = zero_async(arrive, half * sizeof(unsigned), ST(stream))) return rc;
     int took = 0;
     if (int rc = w4_gemm_moe_block_major_pair(g->dev, down_stack->dev, x_in, H(act_out), H(output), expert_ids_per_pair, num_experts, prob_m,
                                               std::min(max_blocks, num_experts), top_k, arrive, arrive + half, arrive + 2 * half, &took,

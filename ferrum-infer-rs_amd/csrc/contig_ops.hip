@@ -6,11 +6,30 @@
 // (scaled_add_inplace); maths cpu.rs:1645-1783, 1993-2060, 2179-2259.
 // The paged lane (rope_kv.hip / attention.hip) is the fast path; these exist so that a backend built on this library
 // implements the WHOLE core trait, and they are simple, bandwidth-shaped kernels rather than tuned ones.
+#include <algorithm>
+
 #include "common.h"
 #include "kernels.h"
 #include "rope_rows.h"
 
 namespace fh {
+
+// Zeros by a launch of the stream: a memory fill recorded into a captured graph has gone wrong on replays after the first.
+// Thread i writes the i-th whole 16 bytes; the first 16 threads also the bytes ahead of them and behind.
+__global__ __launch_bounds__(256) void zero_kernel(uint8_t* __restrict__ p, size_t bytes, size_t head, size_t quads) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, tail = head + quads * 16;
+    if (i < quads) *reinterpret_cast<uint4*>(p + head + i * 16) = uint4{0, 0, 0, 0};
+    if (i < head) p[i] = 0;
+    if (i < bytes - tail) p[tail + i] = 0;
+}
+int zero_async(void* p, size_t bytes, hipStream_t s) {
+    if (bytes == 0) return 0;
+    const size_t head = std::min<size_t>(bytes, -(uintptr_t)p & 15), quads = (bytes - head) / 16;
+    FH_REQUIRE(quads >> 38 == 0, "zero: %zu bytes", bytes);
+    hipLaunchKernelGGL(zero_kernel, dim3((unsigned)std::max<size_t>(1, (quads + 255) / 256)), dim3(256), 0, s, (uint8_t*)p, bytes, head, quads);
+    FH_CHECK_LAUNCH();
+    return 0;
+}
 
 __global__ void split_qkv_kernel(const __half* __restrict__ qkv, __half* __restrict__ q, __half* __restrict__ k,
                                  __half* __restrict__ v, int q_dim, int kv_dim) {

@@ -43,6 +43,7 @@ struct FusedCombineNorm {
     const __half* down; const float* weights; const __half* residual_in; __half* residual_out; const __half* ln_w;
     float eps; int top_k;
 };
+int zero_async(void* p, size_t bytes, hipStream_t stream);
 bool w4_gemm_dense_can_fuse_combine_norm(const W4Device& w, int m);
 int w4_gemm_dense(const W4Device& w, const __half* x, __half* out, int m, float* workspace,
                   size_t workspace_bytes, hipStream_t stream, const FusedCombineNorm* fa = nullptr);

@@ -2286,7 +2286,7 @@ int ferrum_hip_model_time_kernel(FerrumHipModel* m, int which, int n_seqs, int m
     FH_REQUIRE(which < 6 || which == 8 || E == 0, "time_kernel: dense MLP kernel on a MoE model");
     if (which == 8) {
         FH_REQUIRE(em && knobs().moe_em2 && m->em2_arrive && !m->em2_failed, "time_kernel: the merged gate_up → down launch is not what this batch takes");
-        FH_CHECK_HIP(hipMemsetAsync(m->em2_arrive, 0, 2 * m->arrive_half_words * sizeof(unsigned), s));
+        if (int rc = zero_async(m->em2_arrive, 2 * m->arrive_half_words * sizeof(unsigned), s)) return rc;
     }
     const bool same_layer = knobs().time_same_layer;   // experiment: weights resident in the Infinity Cache
     // warm-up round (code objects, TLBs), then the timed rounds

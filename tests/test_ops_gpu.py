@@ -321,6 +321,33 @@ def test_allocated_memory_is_zero_on_return(env):
     assert lib.ferrum_hip_stream_destroy(stream) == 0
 
 
+def test_zeros_on_every_replay(env):
+    """Ranges that start and end anywhere, alone and on each of several replays of a captured graph with eager work and synchronizations in between."""
+    import ctypes as C
+    pkg, B, ctx, O, torch = env
+    size = 1 << 20
+    buf, ranges = torch.zeros(size, dtype=torch.uint8, device="cuda"), [(0, 0), (5, 1), (31, 2), (49, 15), (65, 16), (100, 29), (160, 4096), (5001, 4103), (20003, 900001)]
+    want = torch.full((size,), 7, dtype=torch.uint8, device="cuda")
+    for at, n in ranges:
+        want[at:at + n] = 0
+    with torch.cuda.stream(torch.cuda.Stream()):
+        c2 = B.new_context()                                       # capture needs a non-default stream
+
+        def zero():
+            for at, n in ranges:
+                assert c2.lib.ferrum_hip_memset_zero(C.c_void_p(buf.data_ptr() + at), C.c_size_t(n), c2.stream) == 0
+        B.begin_graph_capture(c2)
+        zero()
+        graph = B.end_graph_capture(c2)
+        for replay in [False] + [True] * 6:
+            buf.fill_(7)
+            torch.cuda.synchronize()
+            B.replay_graph(c2, graph) if replay else zero()
+            c2.sync()
+            assert torch.equal(buf, want)
+        B.reset_graph(c2, graph)
+
+
 # ── paged KV write / read ────────────────────────────────────────────────────
 def _rope(O, hd, max_seq, theta=1e6):
     return O.build_rope_cache(theta, hd, max_seq)
