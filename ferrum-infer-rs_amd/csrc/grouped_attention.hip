@@ -19,6 +19,16 @@
 
 namespace fh {
 
+// a token's values of all heads into its block, zeros into the `clear` slots behind it
+template <typename E>
+__device__ __forceinline__ void grouped_write_values(const GroupedDims& d, E* __restrict__ block, const E* __restrict__ values, int slot, int clear) {
+    for (int i = threadIdx.x; i < d.kv_heads * d.vp; i += 256) {
+        E* head = block + (long)(i / d.vp) * d.vp * 16;
+        head[value_offset(slot, i % d.vp)] = values[i];
+        for (int s = slot + 1; s <= slot + clear; s++) head[value_offset(s, i % d.vp)] = (E)0.f;
+    }
+}
+
 // one workgroup per token
 template <typename E>
 __global__ __launch_bounds__(256) void grouped_prepare_kernel(GroupedDims d, GroupedBuffers<E> p, BatchView v) {
@@ -26,7 +36,7 @@ __global__ __launch_bounds__(256) void grouped_prepare_kernel(GroupedDims d, Gro
     __shared__ float red[8];
     const int t = blockIdx.x, tid = threadIdx.x, seq = v.tok_seq[t];
     const long pos = (long)v.pos[seq] + t - v.cu[seq];
-    const int nq = d.heads * d.dp, nk = d.kv_heads * d.dp, nv = d.kv_heads * d.vp;
+    const int nq = d.heads * d.dp, nk = d.kv_heads * d.dp;
     const E *qr = p.q_in + t * p.ld, *kr = p.k_in + t * p.ld, *vr = p.v_in + t * p.ld;
     float sq = 0.f, sk = 0.f;
     for (int i = tid * 8; i < nq + nk; i += 2048) {
@@ -59,8 +69,7 @@ __global__ __launch_bounds__(256) void grouped_prepare_kernel(GroupedDims d, Gro
         E* dst = query ? p.q + (long)t * nq + c : p.k_pool + (block * d.kv_heads + c / d.dp) * d.dp * 16 + (dim0 * 2 + slot) * 8;
         *reinterpret_cast<v8*>(dst) = o;
     }
-    E* vt = p.v_pool + block * d.kv_heads * d.vp * 16;
-    for (int i = tid; i < nv; i += 256) vt[(long)(i / d.vp) * d.vp * 16 + value_offset(slot, i % d.vp)] = vr[i];
+    grouped_write_values(d, p.v_pool + block * d.kv_heads * d.vp * 16, vr, slot, slots_to_clear(v, seq, t, pos));
 }
 
 // the same with norms of one head each: a power of two of lanes (`sub`) per head, 8 dimensions a lane
@@ -99,8 +108,7 @@ __global__ __launch_bounds__(256) void grouped_prepare_heads_kernel(GroupedDims 
     }
     if (!p.k_in) return;
     const E* vr = p.v_in + t * p.ld;
-    E* vt = p.v_pool + block * d.kv_heads * d.vp * 16;
-    for (int i = tid; i < d.kv_heads * d.vp; i += 256) vt[(long)(i / d.vp) * d.vp * 16 + value_offset(slot, i % d.vp)] = vr[i];
+    grouped_write_values(d, p.v_pool + block * d.kv_heads * d.vp * 16, vr, slot, slots_to_clear(v, seq, t, pos));
 }
 
 // factor of a row's Σ e^(score − m)·value (l: with the sink)

@@ -72,6 +72,8 @@ __global__ __launch_bounds__(256) void latent_prepare_kernel(const E* __restrict
         }
         *reinterpret_cast<v8*>(tile + i * 16) = x;
     }
+    const int clear = slots_to_clear(v, seq, t, pos);
+    for (int i = lane; i < clear * (d.kp >> 3); i += 64) *reinterpret_cast<v8*>(tile + (i / clear) * 128 + (i % clear + 1) * 8) = v8{};
 }
 
 template <typename E>

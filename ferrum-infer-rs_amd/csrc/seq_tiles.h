@@ -9,6 +9,13 @@ namespace fh {
 template <typename E> __device__ __forceinline__ float attn_exp(float x) { return sizeof(E) == 2 ? __expf(x) : expf(x); }
 template <typename E> __device__ __forceinline__ float attn_exp2(float x) { return sizeof(E) == 2 ? __builtin_amdgcn_exp2f(x) : exp2f(x); }
 
+// Slots of a cache block behind token `t` that no token of its sequence has written yet and that hold what another one left: the matrix-core forms weigh
+// them with zero, which a number that is not finite survives, so the token that leaves a block begun in this forward unfinished clears them.
+__device__ __forceinline__ int slots_to_clear(const BatchView& v, int seq, int t, long pos) {
+    const int slot = pos % 16;
+    return t + 1 == (int)v.cu[seq + 1] && pos - slot >= (long)v.pos[seq] ? 15 - slot : 0;
+}
+
 // cosines and sines of the four pairs (2i, 2i + 1) starting at dimension d0, position `pos`; pairs past rot_dims pass unchanged
 struct Rot4 { float c[4], s[4]; };
 __device__ __forceinline__ Rot4 rot_load(int d0, int rot_dims, const float* __restrict__ cos_t, const float* __restrict__ sin_t, long pos) {

@@ -533,6 +533,26 @@ def test_32_bit_tile_sizes(pkg, tmp_path, forms, tokens, ff):
     assert forms.hits().get("tiled_gemm_big")
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("name", ["wide", "odd", "shared", "sinks", "loop", "uneven", "talks", "far"])
+def test_pages_that_held_no_numbers(pkg, tmp_path, name, dtype):
+    """A sequence whose embedding is infinite leaves its pages to the next one, whose blocks end anywhere: nothing of it is seen in a prompt, in portions or a token at a
+    time over the edge of a block."""
+    cfg = G.CONFIGS[name]
+    w = dict(G.weights(cfg, 5))
+    w["embed"] = w["embed"].copy()
+    w["embed"][3] = np.inf
+    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), dtype, tokens=64, seqs=2, blocks=4)
+    t = toks(cfg, 40, 9)
+    t[t == 3] = 4
+    for seq, cuts in enumerate(([21], [5, 1, 1], [15, 3, 1], [16, 16, 8])):
+        assert not np.isfinite(feed(m, 9, np.full(40, 3, np.uint32), [40])).any()
+        m.release(9)
+        got = feed(m, seq, t[:40 if cuts[-1] == 8 else 21], cuts)
+        assert np.isfinite(np.delete(got, 3, axis=1)).all()                     # (the column of that token, where the embedding serves as the head, is infinite)
+        m.release(seq)
+
+
 def test_missing_and_misshapen_weights_are_named(pkg, tmp_path):
     cfg = G.CONFIGS["tiny"]
     w = G.weights(cfg, 1)
