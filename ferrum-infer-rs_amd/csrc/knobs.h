@@ -60,6 +60,7 @@ struct Knobs {
     int tiled_wide_min_tiles = 257;   // … and in 16 bits its 128 × 256 form from this many tiles of that size
     int tiled_min_tiles = 128;        // few-row kernel: 16-row tiles until there are this many row × 16-column tiles
     int tiled_half_max_tiles = 255;   // … its 128 × 64 and 64 × 64 forms up to this many tiles of 128 × 128
+    int tiled_small_max_tiles = 160;  // … the latter up to this many tiles of 128 × 64
     int moe_rows_block = 0;           // > 0: forced rows per block of the sorted expert rows
     int tiled_nw = 0, tiled_kw = 0, tiled_j = 0;      // > 0: forced waves per workgroup, K parts, 16-column tiles per wave of the few-row kernel
     int layer_overlap_max_tokens = 64;   // parallel blocks: experts on a stream of their own beside the mixer up to this many tokens (0 = never)
@@ -133,7 +134,7 @@ enum Form : int {
     FORM_ROUTE_GEMM_TOPK,       // prefill router: logits (MFMA) + softmax + top-k in one launch (moe_route_gemm_topk_kernel)
     FORM_TILED_GEMM,            // layered models: projection with K split over the waves of a workgroup
     FORM_TILED_GEMM_BIG,        // … tiles of up to 128 × 256, operands copied to LDS
-    FORM_TILED_GEMM_256,        // … 128 × 256 tiles
+    FORM_TILED_GEMM_128X256, FORM_TILED_GEMM_128X128, FORM_TILED_GEMM_128X64, FORM_TILED_GEMM_64X64,      // … by the size of the tile, sorted rows too
     FORM_TILED_GEMM_GROUPED,    // … rows sorted by expert
     FORM_TILED_GEMM_GROUPED_BIG,
     FORM_MOE_ROUTE_SORT,        // … router's top-k and the sorted rows in one workgroup

@@ -435,7 +435,7 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
     }
     const int mtiles = g.rows.id ? g.rows.max_blocks * (g.rows.block / T::ROWS) : cdiv(g.m, T::ROWS), ntiles = cdiv(g.n, T::COLS);
     form_hit(g.rows.id ? FORM_TILED_GEMM_GROUPED_BIG : FORM_TILED_GEMM_BIG);
-    if (T::COLS == 256) form_hit(FORM_TILED_GEMM_256);
+    form_hit(T::ROWS == 64 ? FORM_TILED_GEMM_64X64 : T::COLS == 256 ? FORM_TILED_GEMM_128X256 : T::COLS == 128 ? FORM_TILED_GEMM_128X128 : FORM_TILED_GEMM_128X64);
     hipLaunchKernelGGL((tiled_gemm_big_kernel<E, MI, NJ, G, PER_CU>), dim3(mtiles * ntiles, 1, g.groups), dim3(256), T::LDS, s, g, mtiles, ntiles);
     FH_CHECK_LAUNCH();
     return 0;
@@ -473,7 +473,7 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
     } else {
         if (tiles(128, 256) >= knobs().tiled_wide_min_tiles) return launch_big<E, 4, 8, 2, 2>(g, s);
         if (tiles(128, 128) > knobs().tiled_half_max_tiles) return launch_big<E, 4, 4, 2, 2>(g, s);
-        return tiles(128, 64) > 160 ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 2, 2, 3, 3>(g, s);
+        return tiles(128, 64) > knobs().tiled_small_max_tiles ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 2, 2, 3, 3>(g, s);
     }
 }
 

@@ -4,7 +4,10 @@
 host logic and the C-ABI export check; `-m gpu` are the parity tests proper and
 call the HIP kernels through the C-ABI (they fail loudly without the .so).
 """
+import functools
+import glob
 import os
+import re
 import sys
 
 import pytest
@@ -43,12 +46,24 @@ def _knobs_follow_the_environment():
         lib.ferrum_hip_debug_reload_knobs()
 
 
+@functools.lru_cache(None)
+def knob_names():
+    """The switches that the library's sources read."""
+    names = set()
+    for path in glob.glob(os.path.join(ROOT, "ferrum-infer-rs_amd", "csrc", "*")):
+        with open(path, encoding="utf-8") as f:
+            names.update(re.findall(r'"FERRUM_HIP_(\w+)"', f.read()))
+    return names
+
+
 class _Knobs:
     def __init__(self, monkeypatch):
         self.mp = monkeypatch
 
     def set(self, **kw):
-        """knobs.set(ATTN_RS_MIN_WGS=1, NO_GRAPH=None): set / unset FERRUM_HIP_<NAME> and make the library re-read them."""
+        """knobs.set(ATTN_RS_MIN_WGS=1, NO_GRAPH=None): set / unset FERRUM_HIP_<NAME> and make the library re-read them.  A name that the
+        library does not read is a mistake of the test, which would steer nothing."""
+        assert knob_names().issuperset(kw), sorted(set(kw) - knob_names())
         for k, v in kw.items():
             name = "FERRUM_HIP_" + k
             if v is None:

@@ -11,6 +11,7 @@ import pytest
 
 from tests import layered_gen as G
 from tests import layered_oracle as L
+from tests.tile_sizes import FEW_ROWS, SIZES, sizes_that_ran
 
 pytestmark = pytest.mark.gpu
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -496,23 +497,26 @@ def test_latent_attention_in_32_bits(pkg, tmp_path, knobs, forms, heads, dim, ro
 
 @pytest.mark.parametrize("name", ["wide", "shared", "sinks", "loop", "talks"])
 def test_few_row_and_tile_projections_agree(pkg, cases, knobs, forms, name):
-    """The tile kernel in each of its sizes and the few-row kernel on the same portions."""
+    """The 16-bit tile kernel in each of its sizes and the few-row kernel on the same portions."""
     cfg, w, path = cases(name)
     t = toks(cfg, 200, 12)
     want = L.forward(cfg, w, t)
-    for big, wide, half, ran in ((1, 10 ** 6, 0, "tiled_gemm_big"), (1, 10 ** 6, 10 ** 6, "tiled_gemm_big"), (1, 1, 0, "tiled_gemm_256"), (10 ** 6, 192, 128, "tiled_gemm")):
-        knobs.set(TILED_BIG_MIN_TILES=big, TILED_WIDE_MIN_TILES=wide, TILED_WIDE_MIN_K=0, TILED_HALF_MAX_TILES=half)
+    for size, set_to in (*SIZES.items(), (None, FEW_ROWS)):
+        knobs.set(**set_to)
         m = load(pkg, path, "bfloat16")
         forms.reset()
         assert rel(feed(m, 1, t, [200]), want) < TOL["bfloat16"]
         h = forms.hits()
-        assert h.get(ran) and bool(h.get("tiled_gemm_big")) == (big == 1) and bool(h.get("tiled_gemm_256")) == (wide == 1)
+        if size:
+            assert h.get("tiled_gemm_big") and sizes_that_ran(h) == {size}
+        else:                                                              # (blocks of an expert's rows have a rule of their own)
+            assert h.get("tiled_gemm") and not h.get("tiled_gemm_big")
 
 
 @pytest.mark.parametrize("name", ["wide", "shared", "sinks", "loop", "talks"])
 @pytest.mark.parametrize("big", [1, 10 ** 6])
 def test_32_bit_projections_of_prompts(pkg, cases, knobs, forms, name, big):
-    """64 × 64 tiles against the few-row kernel's oracle, whatever the projections' sizes."""
+    """The tiles that so few rows take, mostly of 64 × 64, and the few-row kernel, whatever the projections' sizes."""
     cfg, w, path = cases(name)
     t = toks(cfg, 200, 12)
     knobs.set(TILED_BIG_MIN_TILES=big)
@@ -522,15 +526,17 @@ def test_32_bit_projections_of_prompts(pkg, cases, knobs, forms, name, big):
     assert bool(forms.hits().get("tiled_gemm_big")) == (big == 1)
 
 
-@pytest.mark.parametrize("tokens,ff", [(700, 1024), (700, 1025), (2000, 1024), (1921, 1090)])
-def test_32_bit_tile_sizes(pkg, tmp_path, forms, tokens, ff):
-    """128 × 64 and 128 × 128 tiles, one k-step or two, rows and columns past the last tile."""
-    cfg = G.config(64, 80, [G.attention(2, 8, 6, 8, 20, 16, 40, ff=ff)], buckets=13)
+@pytest.mark.parametrize("tokens,width,ff,size", [(700, 64, 1024, "64x64"), (700, 64, 1025, "64x64"), (700, 200, 1400, "128x64"), (641, 64, 1500, "128x64"),
+                                                  (656, 330, 1300, "128x64"), (2000, 64, 1500, "128x128"), (1921, 200, 1400, "128x128"), (2047, 130, 1601, "128x128")])
+def test_32_bit_tile_sizes(pkg, tmp_path, forms, tokens, width, ff, size):
+    """Every tile of a 32-bit prompt's up-projection: rows and columns past the last tile, K of 4, 10, 14 and 22 steps of 16 (fewer than the ring of rows holds, and
+    past the 128 products that are summed apart)."""
+    cfg = G.config(width, 80, [G.attention(2, 8, 6, 8, 20, 16, 40, ff=ff)], buckets=13)
     w, t = G.weights(cfg, 31), toks(cfg, tokens, 9)
     m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), "float32", tokens=2048)
     forms.reset()
     assert rel(feed(m, 1, t, [tokens]), L.forward(cfg, w, t)) < TOL["float32"]
-    assert forms.hits().get("tiled_gemm_big")
+    assert size in sizes_that_ran(forms.hits())
 
 
 @pytest.mark.parametrize("dtype", DTYPES)

@@ -243,17 +243,17 @@ def test_unquantised_dense_linear_model(pkg, prompt_len, forms):
     _assert_parity(res)
 
 
-@pytest.mark.parametrize("prompt_len,inter,wide,half", [(1, 128, 257, 255), (16, 896, 257, 255), (23, 128, 257, 255), (64, 384, 257, 255), (70, 896, 257, 255),
-                                                        (200, 896, 1, 0), (200, 384, 10 ** 6, 0), (200, 896, 10 ** 6, 10 ** 6), (200, 128, 10 ** 6, 10 ** 6)])
+@pytest.mark.parametrize("prompt_len,inter,size", [(1, 128, None), (16, 896, None), (23, 128, None), (64, 384, None), (70, 896, None), (200, 896, "128x256"),
+                                                   (200, 384, "128x128"), (200, 896, "128x64"), (200, 128, "128x64"), (200, 896, "64x64"), (200, 128, "64x64")])
 @pytest.mark.parametrize("activation", [0, 1])
-def test_unquantised_gate_up_with_its_activation(pkg, prompt_len, inter, wide, half, activation, knobs, forms):
+def test_unquantised_gate_up_with_its_activation(pkg, prompt_len, inter, size, activation, knobs, forms):
     """One gate and one up tile of a wave, and pairs of tiles within every size of the tile kernel."""
-    from tests import modelgen
-    knobs.set(TILED_BIG_MIN_TILES=1 if prompt_len == 200 else 128, TILED_WIDE_MIN_TILES=wide, TILED_HALF_MAX_TILES=half)
+    from tests import modelgen, tile_sizes
+    knobs.set(**tile_sizes.SIZES.get(size, {}))
     res = modelgen.run_parity_case(pkg, moe=False, layers=2, prompt_len=prompt_len, decode_steps=2, seed=171 + prompt_len, dense_proj=True, tied=True,
                                    inter=inter, activation=activation)
     h = forms.require("f16_gated", "tiled_gemm")
-    assert bool(h.get("tiled_gemm_big")) == (prompt_len == 200) and bool(h.get("tiled_gemm_256")) == (wide == 1)
+    assert tile_sizes.sizes_that_ran(h) == ({size} if size else set())
     _assert_parity(res)
 
 

@@ -9,6 +9,7 @@ import pytest
 from tests import layered_gen as G
 from tests import layered_oracle as L
 from tests.test_layered_gpu import DTYPES, TOL, cases, feed, load, pkg, rel, taps_of, toks  # noqa: F401  (two are fixtures)
+from tests.tile_sizes import SIZES, sizes_that_ran
 
 pytestmark = pytest.mark.gpu
 ALONE = {"float32": 1e-5, "bfloat16": 2e-2}
@@ -102,18 +103,19 @@ def test_experts_of_long_prompts(pkg, tmp_path, forms, knobs, block, dtype):
     assert bool(h.get("tiled_gemm_grouped")) == (dtype == "float32" or block <= 64)
 
 
-@pytest.mark.parametrize("wide, half, block", [(1, 0, 128), (1, 0, 256), (10 ** 6, 0, 128), (10 ** 6, 0, 256), (10 ** 6, 10 ** 6, 128), (10 ** 6, 10 ** 6, 256)])
-def test_experts_in_every_tile_size(pkg, tmp_path, forms, knobs, wide, half, block):
-    """Sorted rows in tiles of 256, 128 and 64 columns: an odd and an even number of K steps, fewer of them than the ring holds, blocks that
+@pytest.mark.parametrize("block", [128, 256])
+@pytest.mark.parametrize("size", SIZES)
+def test_experts_in_every_tile_size(pkg, tmp_path, forms, knobs, size, block):
+    """Sorted rows in every size of the tile kernel: an odd and an even number of K steps, fewer of them than the ring holds, blocks that
     several tiles share, columns past the last tile."""
-    knobs.set(MOE_ROWS_BLOCK=block, TILED_WIDE_MIN_TILES=wide, TILED_HALF_MAX_TILES=half)
+    knobs.set(MOE_ROWS_BLOCK=block, **SIZES[size])
     for n, top, tokens, ff, width in ((4, 2, 400, 48, 160), (9, 3, 110, 70, 320), (6, 1, 75, 250, 96), (3, 2, 300, 33, 32)):
         cfg = model([G.sink_attention(2, 8, 4, 8, 16, mlp=G.experts(n, top, ff))], width=width)
         w = G.weights(cfg, 46)
         silence(w, "mix.o", "side.norm")
         agree(pkg, tmp_path / f"{n}{ff}", cfg, w, "bfloat16", n=tokens)
     h = forms.hits()
-    assert h.get("tiled_gemm_grouped_big") and bool(h.get("tiled_gemm_256")) == (wide == 1)
+    assert h.get("tiled_gemm_grouped_big") and sizes_that_ran(h) == {size}
 
 
 @pytest.mark.parametrize("n,top,tokens,ff,width", [(4, 2, 400, 48, 160), (9, 3, 110, 70, 320), (6, 1, 200, 250, 96), (3, 2, 300, 33, 64)])
@@ -124,7 +126,7 @@ def test_experts_in_32_bit_tiles(pkg, tmp_path, forms, knobs, n, top, tokens, ff
     w = G.weights(cfg, 46)
     silence(w, "mix.o", "side.norm")
     agree(pkg, tmp_path, cfg, w, "float32", n=tokens)
-    assert forms.hits().get("tiled_gemm_grouped_big")
+    assert forms.hits().get("tiled_gemm_grouped_big") and sizes_that_ran(forms.hits()) == {"64x64"}
 
 
 def test_experts_beside_the_mixer(pkg, cases, knobs):
