@@ -52,8 +52,8 @@ void reload_knobs() {
     k.tiled_big_min_tiles = env_int("FERRUM_HIP_TILED_BIG_MIN_TILES", 128);
     k.tiled_wide_min_tiles = env_int("FERRUM_HIP_TILED_WIDE_MIN_TILES", 257);
     k.tiled_min_tiles = env_int("FERRUM_HIP_TILED_MIN_TILES", 128);
-    k.tiled_half_max_tiles = env_int("FERRUM_HIP_TILED_HALF_MAX_TILES", 255);
-    k.tiled_small_max_tiles = env_int("FERRUM_HIP_TILED_SMALL_MAX_TILES", 160);
+    k.tiled_half_max_tiles = env_int("FERRUM_HIP_TILED_HALF_MAX_TILES", 256);
+    k.tiled_small_max_tiles = env_int("FERRUM_HIP_TILED_SMALL_MAX_TILES", 256);
     k.moe_rows_block = env_int("FERRUM_HIP_MOE_ROWS_BLOCK", 0);
     k.tiled_nw = env_int("FERRUM_HIP_TILED_NW", 0);
     k.tiled_kw = env_int("FERRUM_HIP_TILED_KW", 0);

@@ -56,11 +56,11 @@ struct Knobs {
     int lds_min_wgs = 128;
     int lds_min_groups = 8;
     // layered models (tiled_gemm.hip, latent_attention.hip, grouped_attention.hip, linear_attention.hip, rglru.hip)
-    int tiled_big_min_tiles = 128;    // projections of > 64 rows take the tile kernel from this many tiles of 64 × 64 (32-bit: and a quarter)
+    int tiled_big_min_tiles = 128;    // projections of > 64 rows take the tile kernel from this many tiles of 64 × 64 (32-bit: and one)
     int tiled_wide_min_tiles = 257;   // … and in 16 bits its 128 × 256 form from this many tiles of that size
     int tiled_min_tiles = 128;        // few-row kernel: 16-row tiles until there are this many row × 16-column tiles
-    int tiled_half_max_tiles = 255;   // … its 128 × 64 and 64 × 64 forms up to this many tiles of 128 × 128
-    int tiled_small_max_tiles = 160;  // … the latter up to this many tiles of 128 × 64
+    int tiled_half_max_tiles = 256;   // … its 128 × 64 and 64 × 64 forms up to this many tiles of 128 × 128
+    int tiled_small_max_tiles = 256;  // … the latter up to this many of them
     int moe_rows_block = 0;           // > 0: forced rows per block of the sorted expert rows
     int tiled_nw = 0, tiled_kw = 0, tiled_j = 0;      // > 0: forced waves per workgroup, K parts, 16-column tiles per wave of the few-row kernel
     int layer_overlap_max_tokens = 64;   // parallel blocks: experts on a stream of their own beside the mixer up to this many tokens (0 = never)

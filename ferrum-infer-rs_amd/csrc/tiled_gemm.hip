@@ -452,7 +452,12 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
 //   300 × 2048 × 2048           34          21         16         12       25
 //   128 × 6144 × 2048           34          21         16         12       28
 // Two workgroups of the largest tile share a CU, so that one's stores run under the other's products; below a tile per CU the smaller tiles
-// cover the chip.  Fewer than half as many tiles as CUs at 64 × 64: the few-row kernel's K split is as fast (128 × 2048 × 2048: 11 and 12 µs).
+// cover the chip.  The lines between them, µs on both sides (tiles of the size whose round of 256 or 512 workgroups ends there):
+//   128 × 256 → 128 × 128     256 tiles: 456 × 16384 × 2048   39.5 → 39.0     260: 456 × 16640 × 2048   53.9 → 56.3
+//   128 × 64 → 128 × 128      256 of 128 × 128: 200 × 16384 × 6144   72 → 81, 968 × 4096 × 2048   26 → 29     264: 200 × 16896 × 6144   100 → 90
+//   64 × 64 → 128 × 64        256: 253 × 4096 × 2048   14.5 → 17.3, 125 × 8192 × 4096   26 → 31     288: 253 × 4608 × 2048   19.8 → 17.5
+//   few rows → 64 × 64        112: 253 × 1792 × 2048   13.9 → 14.2     128: 253 × 2048 × 2048   14.0 → 14.2, 125 × 4096 × 1024   9.9 → 9.6
+//                             144: 253 × 2304 × 2048   22.5 → 14.3
 template <typename E>
 static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
     auto tiles = [&](int r, int c) { return (long)(g.rows.id ? g.rows.max_blocks * (g.rows.block / r) : cdiv(g.m, r)) * cdiv(g.n, c) * g.groups; };
@@ -466,14 +471,14 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
         //   500 × 2048 × 2048       139                    50         62
         //   1000 × 1024 × 512        41                    17         19
         //   128 × 8192 × 2048       139                    50         63
-        //   256 × 2048 × 2048       138                    47         39      (128 tiles: too few)
+        //   256 × 2048 × 2048       138                    47         39      (128 tiles: too few; 253 × 2304 × 2048, 144 tiles: 46 and 60)
         const long full = cdiv(tiles(128, 128), 256) * 133L, half = cdiv(tiles(128, 64), 256) * 72L, small = cdiv(tiles(64, 64), 256) * 42L;
         if ((g.rows.id && g.rows.block < 128) || small < std::min(full, half)) return launch_big<E, 2, 2, 3, 3>(g, s);
         return half < full ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 4, 4, 2, 2>(g, s);
     } else {
         if (tiles(128, 256) >= knobs().tiled_wide_min_tiles) return launch_big<E, 4, 8, 2, 2>(g, s);
         if (tiles(128, 128) > knobs().tiled_half_max_tiles) return launch_big<E, 4, 4, 2, 2>(g, s);
-        return tiles(128, 64) > knobs().tiled_small_max_tiles ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 2, 2, 3, 3>(g, s);
+        return tiles(64, 64) > knobs().tiled_small_max_tiles ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 2, 2, 3, 3>(g, s);
     }
 }
 
@@ -519,7 +524,7 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     }
     constexpr bool F32 = sizeof(E) == 4;
     const long tiles = (rows.id ? (long)rows.max_blocks * (rows.block / 64) : cdiv(g.m, 64)) * cdiv(g.n, 64) * g.groups;
-    const bool enough_tiles = tiles >= knobs().tiled_big_min_tiles * (F32 ? 5L : 4L) / 4;
+    const bool enough_tiles = tiles >= knobs().tiled_big_min_tiles + F32;
     if (rows.id ? (F32 ? rows.block >= 64 && g.n >= 64 && enough_tiles : rows.block >= 128) : g.m > 64 && g.n >= 64 && g.slabs == 1 && enough_tiles) return launch_big(g, s);
     // rows per workgroup: as many as there are, fewer where narrow outputs would leave CUs idle
     int mt = rows.id ? rows.block / 16 : g.m <= 16 ? 1 : (g.m <= 32 ? 2 : 4);

@@ -348,6 +348,40 @@ def test_zeros_on_every_replay(env):
         B.reset_graph(c2, graph)
 
 
+@pytest.mark.parametrize("m,n,k", [(125, 9216, 4096), (456, 8192, 6144)])
+def test_projections_take_the_faster_side_of_a_line(env, m, n, k, knobs):
+    """Shapes at the lines between tile sizes where the wrong side costs 15 to 20 %: what is chosen is as fast as any choice, to a tenth."""
+    from tests.tile_sizes import SIZES
+    pkg, B, ctx, O, torch = env
+    gen = torch.Generator("cuda").manual_seed(1)
+    a, b = (torch.randn(r, k, generator=gen, device="cuda").half() for r in (m, n))
+    out, bt = torch.empty(m, n, dtype=torch.float16, device="cuda"), B.dense_repack_f16t(ctx, b, n, k)
+    ways = {"chosen": {}, **SIZES}
+    names = {name for w in ways.values() for name in w}
+    graphs, best = {}, {}
+    with torch.cuda.stream(torch.cuda.Stream()):
+        c2 = B.new_context()
+        for way, set_to in ways.items():
+            knobs.set(**{**dict.fromkeys(names), **set_to})
+            B.gemm_f16t(c2, a, bt, out, m, n, k)                            # (a kernel's first use sets its LDS size)
+            c2.sync()
+            B.begin_graph_capture(c2)
+            for _ in range(20):
+                B.gemm_f16t(c2, a, bt, out, m, n, k)
+            graphs[way], best[way] = B.end_graph_capture(c2), float("inf")
+        for _ in range(8):
+            for way, graph in graphs.items():
+                start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+                start.record()
+                B.replay_graph(c2, graph)
+                end.record()
+                end.synchronize()
+                best[way] = min(best[way], start.elapsed_time(end) / 20)
+        for graph in graphs.values():
+            B.reset_graph(c2, graph)
+    assert best["chosen"] < 1.1 * min(best.values()), best
+
+
 # ── paged KV write / read ────────────────────────────────────────────────────
 def _rope(O, hd, max_seq, theta=1e6):
     return O.build_rope_cache(theta, hd, max_seq)
