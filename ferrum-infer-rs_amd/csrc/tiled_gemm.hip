@@ -84,6 +84,9 @@ __device__ __forceinline__ const E* gemm_row(const TiledGemm<E>& p, int t, int g
 template <typename E>
 __device__ __forceinline__ int gemm_row_step(const TiledGemm<E>& p) { return p.x_blocks ? 512 : 32; }
 
+// models whose gate tiles all lie ahead of the up tiles (elsewhere the distance of a pair's tiles stays a constant: 5 % of a gated launch of few rows)
+template <typename E> constexpr bool PAIRED = std::is_same_v<E, _Float16>;
+
 // grid (column blocks, row blocks, groups or K slabs); NW waves = (NW / kw) column groups × kw parts of K.  Two register buffers of U
 // k-steps: the next one is requested before the current one is multiplied; loads past the part's end repeat its last k-step.
 // EXT: with sorted rows, column factors, gated sections or rare activations (each is a branch on the latency-bound path of the launches without).
@@ -110,8 +113,9 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(TiledGemm<E> p, int kw)
     const int xs = gemm_row_step(p);
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) xrow[mt] = gemm_row(p, rb * MT + mt, g, a, b);
-    const E* wt = p.w + ((long)g * (p.n >> 4) + (!live ? 0 : J == 2 && p.pair ? n0 >> 5 : n0 >> 4)) * ksteps * 512 + lane * 8;
-    const int next_tile = J == 2 && p.pair ? p.pair : 1;
+    const bool halves = PAIRED<E> && J == 2 && p.pair;
+    const E* wt = p.w + ((long)g * (p.n >> 4) + (!live ? 0 : halves ? n0 >> 5 : n0 >> 4)) * ksteps * 512 + lane * 8;
+    const int next_tile = halves ? p.pair : 1;
     floatx4 acc[MT][J];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++)
@@ -515,7 +519,7 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     }
     FH_REQUIRE(!gated || (g.groups == 1 && !g.col_scale), "tiled_gemm: gated sections take one group and no column factors");
     FH_REQUIRE(!g.col_scale || (g.out && g.ld_col_scale % 8 == 0), "tiled_gemm: column factors with rows of %ld", g.ld_col_scale);
-    FH_REQUIRE(!g.pair || (gated && g.nsec == 1 && g.sec[0].begin == 0 && g.n == 32 * g.pair), "tiled_gemm: %d tiles of a half, n=%d", g.pair, g.n);
+    FH_REQUIRE(!g.pair || (PAIRED<E> && gated && g.nsec == 1 && g.sec[0].begin == 0 && g.n == 32 * g.pair), "tiled_gemm: %d tiles of a half, n=%d", g.pair, g.n);
     const GemmRows& rows = g.rows;
     if (rows.id) {
         FH_REQUIRE(g.slabs == 1 && !g.bias && !g.x_blocks && !g.row_scale && rows.div > 0 && rows.max_blocks > 0 && rows.group && rows.total,
@@ -530,29 +534,56 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     int mt = rows.id ? rows.block / 16 : g.m <= 16 ? 1 : (g.m <= 32 ? 2 : 4);
     while (!rows.id && mt > 1 && (long)cdiv(g.m, 16 * mt) * (g.n / 16) * g.groups * g.slabs < knobs().tiled_min_tiles) mt /= 2;
     const int rbs = rows.id ? rows.max_blocks : cdiv(g.m, 16 * mt), ksteps = g.k / 32, zs = rows.id ? 1 : g.groups * g.slabs;
-    // Columns and K parts of a wave, µs (bf16, weights from HBM; four waves a workgroup, K split over kw of them):
+    // Columns and K parts of a wave.  Several row tiles, whose fragments a wave reads again for every column group: 16 columns as long as a
+    // round of 256 workgroups holds all of them with K in four parts, else 32, and as many parts as make rounds / parts least (a tie: fewer
+    // parts where they are long, so that less is summed through LDS).  µs, bf16, weights from HBM, K in 4 / 2 parts of a workgroup's four waves:
+    //                            workgroups     16 columns      32 columns
+    //   64 × 4096 × 2048          256 | 128    12.9 | 20.4     14.5 | 22.9
+    //   64 × 5120 × 2048          320 | 160    21.1 | 20.4     14.6 | 23.1
+    //   64 × 8256 × 2048          516 | 258    28.8 | 35.2     23.6 | 23.4
+    //   64 × 8256 × 6144          516 | 258    82.7 | 97.4     66.1 | 59.1
+    //   64 × 5120 × 256                                         6.5 |  8.5      (two k-steps a part; 16 columns in two parts 6.9)
+    //   32 × 2560 × 6144 in four slabs                         14.7 | 13.4      (16 columns in two parts 16.7)
+    // One row tile: four parts up to a round of workgroups, two up to the next; 32 columns where 16 would be more than a round in two parts (8 × 8192 ×
+    // 2048: 16 columns 8.2, 32 8.6; 8256 columns: 11.3 and 10.9).  µs (four waves a workgroup, K split over kw of them):
     //                            32 columns      16 columns      before
     //                            kw 4   kw 2     kw 4   kw 2
     //   8 × 4096 × 1024           5.2             4.9    5.3     5.6 (16, eight waves, kw 8)
     //   8 × 6144 × 1024           5.6                    5.6     8.6 (16, eight waves, kw 8)
+    //   8 × 5120 × 2048           7.0             8.1    7.3
     //   8 × 8192 × 2048           8.8                    8.3     10.4 (16, eight waves, kw 8)
     //   16 × 10240 × 2048        12.7   12.0            14.2     12.8 (32, eight waves, kw 8)
     //   8 × 1024 × 3072           8.0             6.5            7.4 (16, eight waves, kw 8)
-    //   32 × 8192 × 2048         10.7                   12.4     13.9 (16, four waves, kw 4)
-    //   32 × 2048 × 2048          9.4             8.4            8.4
-    //   60 × 8192 × 2048         14.7                   20.1     20.8
-    // Fewer waves a workgroup wait for each other less.  Several row tiles, whose fragments a wave reads again for every column group: 32 columns
-    // sooner.  Slabs of a long K want every wave they can get (1 × 2048 × 8192 in four: eight waves 8.1, four 8.4).
+    // Fewer waves a workgroup wait for each other less.  Slabs of a long K want every wave they can get (1 × 2048 × 8192 in four: eight waves 8.1,
+    // four 8.4), and so do wide outputs that stream a long K: 8 × 24576 × 4096 in four parts of four waves 39.7, in eight of eight 36.8; 8 × 65536 × 2048
+    // in two parts 50, in four 43, in eight 42.  Of a short one rounds decide again: 8 × 49152 × 1024 in two parts 19.3, in eight 21.2.
+    // Sorted rows: K is split below 8192 column groups (24 blocks of 16 rows, 4096 × 2048: four parts 68, one 75; 64 blocks: 161 and 137).
     const bool long_slabs = g.slabs > 1 && ksteps / g.slabs >= 64, narrow = sizeof(E) == 4 || long_slabs;
-    int J = narrow ? ((long)rbs * (g.n / 32) * zs < (g.slabs > 1 ? 256 : 257) ? 1 : 2)
-                   : (long)rbs * (g.n / 32) * g.groups < (g.n <= 96 && g.m > 64 ? 513 : mt == 1 ? 257 : 160) ? 1 : 2;
+    const long groups16 = (long)rbs * (g.n / 16) * zs;
+    const bool plain = !narrow && !rows.id, wide = plain && g.slabs == 1 && groups16 >= 896, several = plain && mt > 1 && !wide && !(g.n <= 96 && g.m > 64);
+    int J = several ? (groups16 <= 256 ? 1 : 2)
+            : narrow ? (groups16 / 2 < (g.slabs > 1 ? 256 : 257) ? 1 : 2)
+                     : (long)rbs * (g.n / 32) * g.groups < (g.n <= 96 && g.m > 64 ? 513 : mt == 1 ? 257 : 160) ? 1 : 2;       // (narrow outputs of prompts: two workgroups per CU)
     if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : 2;
     if (gated) J = 2;
     const long cols = g.n / (16 * J);
-    int nw = mt == 1 && narrow ? 8 : 4, kw = 1;
+    int nw = mt == 1 && (narrow || (wide && ksteps >= 128)) ? 8 : 4, kw = 1;
     if (knobs().tiled_nw > 0) nw = std::min(8, knobs().tiled_nw);
-    const long enough = rows.id ? 8192 : narrow ? 4096 : J == 1 ? 768 : 4096;
-    while (kw < nw && (long)rbs * cols * zs * kw < enough && ksteps >= 8 * kw * g.slabs) kw *= 2;
+    if (several || (wide && mt == 1 && ksteps < 64)) {
+        const int steps = ksteps / g.slabs;
+        long least = 0;
+        for (int k : {4, 2, 1}) {
+            if (k > 1 && steps < 2 * k) continue;
+            const long rounds = cdiv((long)rbs * cdiv(cols, 4 / k) * zs, 256);
+            const bool tie = least && rounds * kw == least * k;
+            if (!least || rounds * kw < least * k || (tie && (k > 1 || steps >= 128) && (steps >= 32 || steps < 4 * kw))) { kw = k; least = rounds; }
+        }
+    } else if (wide && mt == 1) {
+        kw = nw;
+    } else {
+        const long enough = rows.id ? 8192 : J == 1 && plain ? 513 : 4096;
+        while (kw < nw && (long)rbs * cols * zs * kw < enough && ksteps >= 8 * kw * g.slabs) kw *= 2;
+    }
     if (knobs().tiled_kw > 0) kw = std::min(nw, knobs().tiled_kw);
     const dim3 grid(cdiv(cols, nw / kw), rbs, zs);
     form_hit(rows.id ? FORM_TILED_GEMM_GROUPED : FORM_TILED_GEMM);

@@ -285,7 +285,8 @@ def test_dense_gemm(env, m, n, k, f32out):
 
 @pytest.mark.parametrize("f32out", [False, True])
 @pytest.mark.parametrize("m,n,k", [(1, 64, 32), (16, 4096, 1024), (17, 96, 1056), (64, 1024, 3072), (65, 8192, 32), (100, 6176, 96), (200, 2080, 64),
-                                   (129, 16416, 160), (300, 4128, 2080), (1100, 1056, 352), (2049, 4096, 128), (3000, 8224, 64)])
+                                   (129, 16416, 160), (300, 4128, 2080), (1100, 1056, 352), (2049, 4096, 128), (3000, 8224, 64), (9, 14400, 2080), (16, 16416, 4128),
+                                   (5, 20512, 96), (48, 5152, 256), (33, 8256, 544), (64, 8256, 2080), (64, 10272, 4128)])
 def test_dense_gemm_tile_edges(env, m, n, k, f32out):
     """Few rows and every tile size at rows and columns just past a tile, odd and even numbers of 32-column steps, fewer of them than a ring holds;
     also into a result whose address only takes single elements."""
@@ -348,15 +349,15 @@ def test_zeros_on_every_replay(env):
         B.reset_graph(c2, graph)
 
 
-@pytest.mark.parametrize("m,n,k", [(125, 9216, 4096), (456, 8192, 6144)])
+@pytest.mark.parametrize("m,n,k", [(125, 9216, 4096), (456, 8192, 6144), (64, 5120, 256), (64, 8256, 6144)])
 def test_projections_take_the_faster_side_of_a_line(env, m, n, k, knobs):
-    """Shapes at the lines between tile sizes where the wrong side costs 15 to 20 %: what is chosen is as fast as any choice, to a tenth."""
+    """Shapes at the lines between tile sizes and between parts of K where the wrong side costs 12 to 30 %: what is chosen is as fast as any choice, to a tenth."""
     from tests.tile_sizes import SIZES
     pkg, B, ctx, O, torch = env
     gen = torch.Generator("cuda").manual_seed(1)
     a, b = (torch.randn(r, k, generator=gen, device="cuda").half() for r in (m, n))
     out, bt = torch.empty(m, n, dtype=torch.float16, device="cuda"), B.dense_repack_f16t(ctx, b, n, k)
-    ways = {"chosen": {}, **SIZES}
+    ways = {"chosen": {}, **(SIZES if m > 64 else {f"{16 * j} columns, K in {w}": dict(TILED_J=j, TILED_KW=w) for j in (1, 2) for w in (1, 2, 4)})}
     names = {name for w in ways.values() for name in w}
     graphs, best = {}, {}
     with torch.cuda.stream(torch.cuda.Stream()):
