@@ -58,7 +58,7 @@ struct Knobs {
     // layered models (tiled_gemm.hip, latent_attention.hip, grouped_attention.hip, linear_attention.hip, rglru.hip)
     int tiled_big_min_tiles = 128;    // projections of > 64 rows take the tile kernel from this many tiles of 64 × 64 (32-bit: and one)
     int tiled_wide_min_tiles = 257;   // … and in 16 bits its 128 × 256 form from this many tiles of that size
-    int tiled_min_tiles = 128;        // few-row kernel: 16-row tiles until there are this many row × 16-column tiles
+    int tiled_min_tiles = 128;        // few-row kernel: rows of a workgroup are halved until there are this many row × 16-column tiles (16-bit: up to twice as many)
     int tiled_half_max_tiles = 256;   // … its 128 × 64 and 64 × 64 forms up to this many tiles of 128 × 128
     int tiled_small_max_tiles = 256;  // … the latter up to this many of them
     int moe_rows_block = 0;           // > 0: forced rows per block of the sorted expert rows

@@ -530,9 +530,12 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     const long tiles = (rows.id ? (long)rows.max_blocks * (rows.block / 64) : cdiv(g.m, 64)) * cdiv(g.n, 64) * g.groups;
     const bool enough_tiles = tiles >= knobs().tiled_big_min_tiles + F32;
     if (rows.id ? (F32 ? rows.block >= 64 && g.n >= 64 && enough_tiles : rows.block >= 128) : g.m > 64 && g.n >= 64 && g.slabs == 1 && enough_tiles) return launch_big(g, s);
-    // rows per workgroup: as many as there are, fewer where narrow outputs would leave CUs idle
+    // rows per workgroup: as many as there are, fewer where narrow outputs would leave CUs idle: in 16 bits as long as a round of 256 workgroups
+    // holds the launch (64 × 2048 × 4096, four row tiles | two: 20.6 | 12.8 µs; 65 × 1024 × 4096, two | one: 20.2 | 12.6; past the round, 24 × 3072 ×
+    // 2048, two | one: 7.7 | 8.4)
     int mt = rows.id ? rows.block / 16 : g.m <= 16 ? 1 : (g.m <= 32 ? 2 : 4);
-    while (!rows.id && mt > 1 && (long)cdiv(g.m, 16 * mt) * (g.n / 16) * g.groups * g.slabs < knobs().tiled_min_tiles) mt /= 2;
+    auto row_tiles = [&](int t) { return (long)cdiv(g.m, 16 * t) * (g.n / 16) * g.groups * g.slabs; };
+    while (!rows.id && mt > 1 && (F32 ? row_tiles(mt) < knobs().tiled_min_tiles : row_tiles(mt / 2) <= 2 * knobs().tiled_min_tiles)) mt /= 2;
     const int rbs = rows.id ? rows.max_blocks : cdiv(g.m, 16 * mt), ksteps = g.k / 32, zs = rows.id ? 1 : g.groups * g.slabs;
     // Columns and K parts of a wave.  Several row tiles, whose fragments a wave reads again for every column group: 16 columns as long as a
     // round of 256 workgroups holds all of them with K in four parts, else 32, and as many parts as make rounds / parts least (a tie: fewer

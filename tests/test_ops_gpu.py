@@ -349,26 +349,19 @@ def test_zeros_on_every_replay(env):
         B.reset_graph(c2, graph)
 
 
-@pytest.mark.parametrize("m,n,k", [(125, 9216, 4096), (456, 8192, 6144), (64, 5120, 256), (64, 8256, 6144)])
-def test_projections_take_the_faster_side_of_a_line(env, m, n, k, knobs):
-    """Shapes at the lines between tile sizes and between parts of K where the wrong side costs 12 to 30 %: what is chosen is as fast as any choice, to a tenth."""
-    from tests.tile_sizes import SIZES
+def _times(env, knobs, call, ways):
+    """Best time of a call under every setting of the switches, ms: captured, so that the host does not count, and in turn, so that a slow moment meets all."""
     pkg, B, ctx, O, torch = env
-    gen = torch.Generator("cuda").manual_seed(1)
-    a, b = (torch.randn(r, k, generator=gen, device="cuda").half() for r in (m, n))
-    out, bt = torch.empty(m, n, dtype=torch.float16, device="cuda"), B.dense_repack_f16t(ctx, b, n, k)
-    ways = {"chosen": {}, **(SIZES if m > 64 else {f"{16 * j} columns, K in {w}": dict(TILED_J=j, TILED_KW=w) for j in (1, 2) for w in (1, 2, 4)})}
-    names = {name for w in ways.values() for name in w}
-    graphs, best = {}, {}
+    names, graphs, best = {name for w in ways.values() for name in w}, {}, {}
     with torch.cuda.stream(torch.cuda.Stream()):
         c2 = B.new_context()
         for way, set_to in ways.items():
             knobs.set(**{**dict.fromkeys(names), **set_to})
-            B.gemm_f16t(c2, a, bt, out, m, n, k)                            # (a kernel's first use sets its LDS size)
+            call(c2)                                                       # (a kernel's first use sets its LDS size)
             c2.sync()
             B.begin_graph_capture(c2)
             for _ in range(20):
-                B.gemm_f16t(c2, a, bt, out, m, n, k)
+                call(c2)
             graphs[way], best[way] = B.end_graph_capture(c2), float("inf")
         for _ in range(8):
             for way, graph in graphs.items():
@@ -380,6 +373,20 @@ def test_projections_take_the_faster_side_of_a_line(env, m, n, k, knobs):
                 best[way] = min(best[way], start.elapsed_time(end) / 20)
         for graph in graphs.values():
             B.reset_graph(c2, graph)
+    return best
+
+
+@pytest.mark.parametrize("m,n,k", [(125, 9216, 4096), (456, 8192, 6144), (64, 5120, 256), (64, 8256, 6144), (65, 1024, 4096)])
+def test_projections_take_the_faster_side_of_a_line(env, m, n, k, knobs):
+    """Shapes at the lines between tile sizes, rows of a workgroup and parts of K where the wrong side costs 12 to 60 %: what is chosen is as fast as any choice, to a
+    tenth."""
+    from tests.tile_sizes import SIZES
+    pkg, B, ctx, O, torch = env
+    gen = torch.Generator("cuda").manual_seed(1)
+    a, b = (torch.randn(r, k, generator=gen, device="cuda").half() for r in (m, n))
+    out, bt = torch.empty(m, n, dtype=torch.float16, device="cuda"), B.dense_repack_f16t(ctx, b, n, k)
+    ways = SIZES if m > 65 else {f"{16 * j} columns, K in {w}, rows {t}": dict(TILED_J=j, TILED_KW=w, TILED_MIN_TILES=t) for j in (1, 2) for w in (1, 2, 4) for t in (64, 128)}
+    best = _times(env, knobs, lambda c: B.gemm_f16t(c, a, bt, out, m, n, k), {"chosen": {}, **ways})
     assert best["chosen"] < 1.1 * min(best.values()), best
 
 
