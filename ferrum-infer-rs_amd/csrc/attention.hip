@@ -1201,14 +1201,17 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
         return 0;
     }
     // head_dim 128 has two sizes of workgroup.  128 rows read K/V from LDS half as often, 64 rows make twice the workgroups and half of a step's
-    // vector work in each: µs, row-split or KV-split form / 64 rows / 128 rows (workgroups of 128 rows × kv heads)
+    // vector work in each; two workgroups of either share a CU.  The line lies where 128 rows, less of a round of 512 as they are, have the less
+    // work in all: at 360 of them, at 300 under a window, which leaves every workgroup as many keys.  Over 840 batches between 256 and 512 that
+    // choice is 2 % from the faster of the two, always 64 rows 4 %, always 128 5 %.
+    // µs, row-split or KV-split form / 64 rows / 128 rows (workgroups of 128 rows × kv heads)
     //   8B heads (32 on 8)    1 × 8100 (2024)      2372 / 919 / 779      1 × 2048 (512)        196 / 95 / 82     1 × 1024 (256)         62 / 33 / 37
     //                         1 × 700 (175)          32 / 25 / 28        1 × 500 (125)          19 / 17 / 24     1 × 300 (75)           11 / 11 / 17
     //   16 on 8               1500 and 548 (256)     82 / 46 / 63        293, 1389, 366 (256)   87 / 48 / 62     1 × 986 at 366 (123)   49 / 35 / 54
     //                         6 × 100, 1400 (250)    80 / 39 / 53        1 × 500 (62)           14 / 16 / 24
     // A batch qualifies where most of its sequences bring many rows, or they bring 256 on average.
     const long rows_heads = (long)total_q_tokens * G * num_kv_heads;
-    const bool two_sizes = head_dim == 128 && !kn.attn_flash32, half_units = two_sizes && (kn.attn_flash_rows ? kn.attn_flash_rows == 64 : rows_heads < 512 * 128);
+    const bool two_sizes = head_dim == 128 && !kn.attn_flash32, half_units = two_sizes && (kn.attn_flash_rows ? kn.attn_flash_rows == 64 : rows_heads < (sliding_window > 0 && max_kv_len > sliding_window ? 300 : 360) * 128);
     const bool flash_fits = (long)total_q_tokens * 2 >= (long)num_seqs * max_q_len || (two_sizes && (long)total_q_tokens * G >= (long)num_seqs * 256);
     if (!fq && cu_seqlens_q && !flash_off && (long)max_q_len * G >= flash_min_rows && flash_fits &&
         rows_heads / (half_units || head_dim == 256 ? 64 : 128) >= (half_units && !kn.attn_flash_min_rows_set ? 192 : flash_min_wgs)) {

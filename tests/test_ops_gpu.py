@@ -390,6 +390,20 @@ def test_projections_take_the_faster_side_of_a_line(env, m, n, k, knobs):
     assert best["chosen"] < 1.1 * min(best.values()), best
 
 
+@pytest.mark.parametrize("nq,nkv,tokens,pos,seqs,window", [(32, 4, 64, 700, 24, 0), (14, 2, 4096, 0, 1, 512), (32, 8, 700, 0, 1, 0)])
+def test_prompt_attention_takes_the_faster_unit(env, nq, nkv, tokens, pos, seqs, window, knobs):
+    """Batches on both sides of the line between units of 64 and 128 rows, where the wrong one costs 12 to 40 %."""
+    pkg, B, ctx, O, torch = env
+    gen = torch.Generator("cuda").manual_seed(1)
+    T, kv, mb = tokens * seqs, pos + tokens, (pos + tokens + 15) // 16
+    q, k, v = (torch.randn(n, generator=gen, device="cuda").half() for n in (T * nq * 128, seqs * mb * nkv * 2048, seqs * mb * nkv * 2048))
+    out, tables = torch.empty_like(q), torch.arange(seqs * mb, device="cuda", dtype=torch.int32).reshape(seqs, mb)
+    cu, po = torch.arange(seqs + 1, device="cuda", dtype=torch.int32) * tokens, torch.full((seqs,), pos, device="cuda", dtype=torch.int32)
+    best = _times(env, knobs, lambda c: B.paged_varlen_attention(c, q, k, v, out, cu, po, tables, seqs, T, kv, nq, nkv, 128, window, 16, mb, tokens),
+                  {"chosen": {}, "64": dict(ATTN_FLASH_ROWS=64), "128": dict(ATTN_FLASH_ROWS=128)})
+    assert best["chosen"] < 1.1 * min(best.values()), best
+
+
 # ── paged KV write / read ────────────────────────────────────────────────────
 def _rope(O, hd, max_seq, theta=1e6):
     return O.build_rope_cache(theta, hd, max_seq)
