@@ -36,6 +36,7 @@ void reload_knobs() {
     k.attn_no_rs = env_flag("FERRUM_HIP_ATTN_NO_RS");
     k.attn_narrow = env_flag("FERRUM_HIP_ATTN_NARROW");
     k.attn_flash_rows = env_int("FERRUM_HIP_ATTN_FLASH_ROWS", 0);
+    k.rope_quad_rows = env_int("FERRUM_HIP_ROPE_QUAD_ROWS", 8192);
     k.attn_flash32 = env_flag("FERRUM_HIP_ATTN_FLASH32");
     k.attn_no_resident = env_flag("FERRUM_HIP_ATTN_NO_RESIDENT");
     k.attn_resident_min_wgs = env_int("FERRUM_HIP_ATTN_RESIDENT_MIN_WGS", 128);

@@ -26,6 +26,7 @@ struct Knobs {
     long attn_resident_min_wgs = 128; // … and only from this many workgroups (tests lower it)
     int attn_flash_rows = 0;          // 64 / 128: forced rows per workgroup of the 64-key form
     bool attn_flash32 = false;        // the flash form with 32-key steps (paged_prefill_attn_kernel) for head_dim 128 too
+    int rope_quad_rows = 8192;        // split q|k|v, norm, rotation, cache write: four tokens of a head a wave from this many rows of a head
     // INT4 GEMMs (w4_gemm.hip)
     int moe_kw_pairs = 16;
     int decode_chain = 1;             // MoE decode at ≤ 32 rows: tail + q|k|v + attention + o_proj + route as ONE launch (0 = five launches)

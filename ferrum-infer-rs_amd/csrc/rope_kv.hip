@@ -7,6 +7,7 @@
 // K/V land in pool block block_tables[seq][pos/16], slot pos%16; Q goes out token-major.
 #include "common.h"
 #include "kernels.h"
+#include "knobs.h"
 #include "kv_layout.h"
 #include "rope_rows.h"
 
@@ -17,19 +18,24 @@ namespace fh {
 // heads it was bound by the workgroups' starts, 0.8 ns each, and by V's stores of two bytes: a tile keeps four keys of a dimension
 // together, which is the four tokens of a wave where their positions are aligned, exchanged between its quarters (head_dim 128).
 //   8100 tokens × (32 + 2·8) heads: 80 → 41 µs (200 MB, what a copy takes); 2048 × (16 + 2·8): 16.5 → 10 µs
-template <int HD>
-__global__ __launch_bounds__(256) void split_qkv_norm_rope_paged_kernel(
+// Few rows (QUADS false): a wave takes four consecutive heads of one token, a workgroup one wave.  µs by tokens, quads | heads:
+//   (32 + 2·8) × 128    8: 3.4 | 2.7    128: 3.9 | 3.7    192: 4.2 | 4.2    256: 4.4 | 4.9    1024:  8.4 | 10.7
+//   (32 + 2·8) × 256    8: 4.7 | 3.3    128: 5.6 | 4.8    192: 6.2 | 5.8    256: 6.6 | 7.0    1024: 15.7 | 17.5
+//   (8 + 2·2) × 128     8: 3.3 | 2.7    512: 3.8 | 3.8    768: 4.3 | 4.3   1024: 4.3 | 4.9
+template <int HD, bool QUADS>
+__global__ __launch_bounds__(QUADS ? 256 : 64) void split_qkv_norm_rope_paged_kernel(
     const __half* __restrict__ qkv, const __half* __restrict__ q_norm_w, const __half* __restrict__ k_norm_w,
     const float* __restrict__ cos_t, const float* __restrict__ sin_t, __half* __restrict__ q_out,
     __half* __restrict__ cache_k, __half* __restrict__ cache_v, const uint32_t* __restrict__ cu_seqlens_q,
     const uint32_t* __restrict__ pos_offsets, const int32_t* __restrict__ block_tables, int num_seqs, int m_total,
     int q_heads, int kv_heads, float eps, int qk_mode, int max_blocks_per_seq) {
     constexpr int PPL = HD / 32, HALF = HD / 2;
+    constexpr int TOKENS = QUADS ? 4 : 1;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, q16 = lane & 15, quarter = lane >> 4;
-    const int head = blockIdx.y * 4 + wave;
-    if (head >= q_heads + 2 * kv_heads) return;
-    const int tok0 = blockIdx.x * 4, tok = min(tok0 + quarter, m_total - 1);         // clamped: loads stay unconditional
-    const bool act = tok0 + quarter < m_total;
+    const int heads = q_heads + 2 * kv_heads, head_raw = blockIdx.y * 4 + (QUADS ? wave : quarter), head = min(head_raw, heads - 1);
+    if (QUADS && head_raw >= heads) return;
+    const int tok0 = blockIdx.x * TOKENS, tok = QUADS ? min(tok0 + quarter, m_total - 1) : tok0;         // clamped: loads stay unconditional
+    const bool act = QUADS ? tok0 + quarter < m_total : head_raw < heads;
     const int q_dim = q_heads * HD, kv_dim = kv_heads * HD;
     const __half* row = qkv + (long)tok * (q_dim + 2 * kv_dim);
 
@@ -41,13 +47,13 @@ __global__ __launch_bounds__(256) void split_qkv_norm_rope_paged_kernel(
         const uint32_t first = s < num_seqs ? cu_seqlens_q[s] : 0xffffffffu;
         unsigned long long le = 0;
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < TOKENS; j++) {
             le = __ballot(first <= (uint32_t)min(tok0 + j, m_total - 1));
             if (le) seq4[j] = s0 + 63 - __clzll((long long)le);
         }
-        if (le != ~0ull) break;                              // (the fourth token's is the largest set)
+        if (le != ~0ull) break;                              // (the last token's is the largest set)
     }
-    const int seq = quarter == 0 ? seq4[0] : quarter == 1 ? seq4[1] : quarter == 2 ? seq4[2] : seq4[3];
+    const int seq = !QUADS || quarter == 0 ? seq4[0] : quarter == 1 ? seq4[1] : quarter == 2 ? seq4[2] : seq4[3];
     const int pos = (int)pos_offsets[seq] + (tok - (int)cu_seqlens_q[seq]);
 
     const bool is_q = head < q_heads;
@@ -75,7 +81,7 @@ __global__ __launch_bounds__(256) void split_qkv_norm_rope_paged_kernel(
         *reinterpret_cast<hv*>(t16 + k_tile_off(slot, rr.off1)) = rr.out1;
         return;
     }
-    if constexpr (HD == 128) {
+    if constexpr (QUADS && HD == 128) {
         const int pos_first = __builtin_amdgcn_readfirstlane(pos);
         if (tok0 + 3 < m_total && seq4[0] == seq4[3] && pos_first % 4 == 0) {
             // quarter t holds token t's dimensions off0 … + 3 and off1 … + 3, as four pairs; quarter r leaves with pair r of all four tokens
@@ -117,12 +123,14 @@ int split_qkv_norm_rope_into_paged_cache_varlen_f16(
     FH_REQUIRE(block_size == KV_BLOCK, "paged KV: block_size=%d unsupported (native layout uses 16)", block_size);
     FH_REQUIRE(head_dim == 64 || head_dim == 128 || head_dim == 256, "paged KV: head_dim=%d must be 64, 128 or 256", head_dim);
     FH_REQUIRE(qk_mode >= 0 && qk_mode <= 3, "paged KV: qk_mode=%d out of range", qk_mode);
-    const dim3 grid(cdiv(m_total, 4), cdiv(q_heads + 2 * kv_heads, 4));
-#define FH_ROPE(HDV)                                                                                                   \
-    hipLaunchKernelGGL(split_qkv_norm_rope_paged_kernel<HDV>, grid, dim3(256), 0, s, qkv, q_norm_w, k_norm_w, cos_t, sin_t, \
-                       q_out, cache_k, cache_v, cu_seqlens_q, pos_offsets, block_tables, num_seqs, m_total, q_heads, kv_heads, eps, \
+    const bool quads = (long)m_total * (q_heads + 2 * kv_heads) >= knobs().rope_quad_rows;
+    const dim3 grid(quads ? cdiv(m_total, 4) : m_total, cdiv(q_heads + 2 * kv_heads, 4));
+#define FH_ROPE(HDV, QUADS)                                                                                            \
+    hipLaunchKernelGGL((split_qkv_norm_rope_paged_kernel<HDV, QUADS>), grid, dim3(QUADS ? 256 : 64), 0, s, qkv, q_norm_w, k_norm_w, cos_t, \
+                       sin_t, q_out, cache_k, cache_v, cu_seqlens_q, pos_offsets, block_tables, num_seqs, m_total, q_heads, kv_heads, eps, \
                        qk_mode, max_blocks_per_seq)
-    if (head_dim == 64) FH_ROPE(64); else if (head_dim == 128) FH_ROPE(128); else FH_ROPE(256);
+    if (quads) { if (head_dim == 64) FH_ROPE(64, true); else if (head_dim == 128) FH_ROPE(128, true); else FH_ROPE(256, true); }
+    else { if (head_dim == 64) FH_ROPE(64, false); else if (head_dim == 128) FH_ROPE(128, false); else FH_ROPE(256, false); }
 #undef FH_ROPE
     FH_CHECK_LAUNCH();
     return 0;

@@ -404,16 +404,32 @@ def test_prompt_attention_takes_the_faster_unit(env, nq, nkv, tokens, pos, seqs,
     assert best["chosen"] < 1.1 * min(best.values()), best
 
 
+@pytest.mark.parametrize("hd,tokens", [(256, 1), (256, 40), (128, 8), (128, 2048)])
+def test_cache_write_takes_the_faster_form(env, hd, tokens, knobs):
+    """A token of four heads a wave, or four tokens of a head."""
+    pkg, B, ctx, O, torch = env
+    nq, nkv, mb = 32, 8, (tokens + 15) // 16
+    qkv, one = torch.randn(tokens, (nq + 2 * nkv) * hd, device="cuda").half(), torch.ones(hd, device="cuda").half()
+    cos, q_out, (ck, cv) = torch.ones(tokens, hd // 2, device="cuda"), torch.empty(tokens, nq * hd, device="cuda").half(), (B.alloc_paged_pool(mb, nkv, hd) for _ in range(2))
+    tables, cu, po = torch.arange(mb, device="cuda", dtype=torch.int32)[None], torch.tensor([0, tokens], device="cuda", dtype=torch.int32), torch.zeros(1, device="cuda", dtype=torch.int32)
+    best = _times(env, knobs, lambda c: B.split_qkv_norm_rope_into_paged_cache_varlen(c, qkv, one, one, cos, cos, q_out, ck, cv, cu, po, tables, 1, tokens, nq, nkv, hd, 1e-6, 1, 16, mb),
+                  {"chosen": {}, "quads": dict(ROPE_QUAD_ROWS=0), "heads": dict(ROPE_QUAD_ROWS=10 ** 9)})
+    assert best["chosen"] < 1.1 * min(best.values()), best
+
+
 # ── paged KV write / read ────────────────────────────────────────────────────
 def _rope(O, hd, max_seq, theta=1e6):
     return O.build_rope_cache(theta, hd, max_seq)
 
 
+@pytest.mark.parametrize("quad_rows", [0, 10 ** 9])
 @pytest.mark.parametrize("hd", [64, 128, 256])
 @pytest.mark.parametrize("q_lens,pos,nq,nkv", [([1], [0], 1, 1), ([4], [12], 3, 1), ([3, 5], [1, 4], 2, 2), ([16, 0, 8, 0], [0, 3, 4, 0], 5, 3), ([7, 9, 64, 33], [1, 0, 0, 7], 8, 2),
                                                ([4] * 70, [4 * (i % 5) for i in range(70)], 2, 1), ([5] * 66 + [0] * 3, [i % 7 for i in range(69)], 3, 2)])
-def test_quads_of_tokens_in_the_paged_cache(env, q_lens, pos, nq, nkv, hd):
-    """Four tokens of a wave at aligned positions and not, across sequences and past the batch, empty sequences in between and at the end: copies."""
+def test_quads_of_tokens_in_the_paged_cache(env, q_lens, pos, nq, nkv, hd, quad_rows, knobs):
+    """Four tokens of a wave at aligned positions and not, across sequences and past the batch, empty sequences in between and at the end, and four heads of a token
+    a wave: copies."""
+    knobs.set(ROPE_QUAD_ROWS=quad_rows)
     pkg, B, ctx, O, torch = env
     rng = np.random.default_rng(len(q_lens) + hd)
     S, T, mb = len(q_lens), sum(q_lens), (max(p + n for p, n in zip(pos, q_lens)) + 15) // 16
