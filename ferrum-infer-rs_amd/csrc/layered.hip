@@ -61,16 +61,17 @@ struct HostTensor { std::vector<float> data; std::vector<int64_t> shape; };
 class Arena {
 public:
     ~Arena() { for (void* p : mem_) (void)hipFree(p); }
-    template <typename T> int alloc(T** p, size_t n) {
+    template <typename T> int alloc(T** p, size_t n, bool zero = true) {      // (zero false: the caller writes all of it)
         *p = nullptr;
         if (!n) return 0;
         FH_CHECK_HIP(hipMalloc((void**)p, n * sizeof(T)));
         mem_.push_back(*p);
-        FH_CHECK_HIP(device_zero(*p, n * sizeof(T)));
+        if (zero) FH_CHECK_HIP(device_zero(*p, n * sizeof(T)));
         return 0;
     }
     template <typename T> int upload(T** p, const std::vector<T>& v) {
-        if (int rc = alloc(p, v.size())) return rc;
+        if (int rc = alloc(p, v.size(), false)) return rc;
+        if (v.empty()) return 0;
         FH_CHECK_HIP(hipMemcpy(*p, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice));
         return 0;
     }
@@ -1152,7 +1153,7 @@ private:
         L->n = n; L->k = k; L->groups = groups;
         const size_t total = (size_t)groups * n * k;
         if (synth_) {
-            FH_TRY(arena_.alloc(&L->w, total));
+            FH_TRY(arena_.alloc(&L->w, total, false));
             hipLaunchKernelGGL(synth_kernel<E>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream_, L->w, total, mix(++seed_), 1.0f / sqrtf((float)k));
             FH_CHECK_LAUNCH();
             return 0;
@@ -1244,7 +1245,7 @@ private:
         FH_TRY(need(name, {rows, cols}));
         const size_t total = (size_t)rows * n_pad;
         if (synth_) {
-            FH_TRY(arena_.alloc(out, total));
+            FH_TRY(arena_.alloc(out, total, false));
             hipLaunchKernelGGL(synth_kernel<E>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream_, *out, total, mix(++seed_), 1.0f);
             FH_CHECK_LAUNCH();
             return 0;
