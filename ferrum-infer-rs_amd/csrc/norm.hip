@@ -448,6 +448,8 @@ int gather_rows_f16(const __half* in, const int32_t* row_idx, __half* out, int n
 }
 
 // ── gated activations: [T, 2I] (gate columns, then up columns) → [T, I] ──────
+// gate_up computes its activation itself where it has a form for that: INT4 at ≤ 16 rows and in prompt tiles, unquantised weights at any rows.
+// This kernel serves the rest (INT4 rows in between, an intermediate size that is no multiple of 32, an unquantised gate_up with a bias) and its entry point.
 template <bool GELU>
 __global__ void gated_act_kernel(const __half* __restrict__ gate_up, __half* __restrict__ out, int im) {
     const long t = blockIdx.y;

@@ -3427,6 +3427,8 @@ static int f16t_gemm_impl(const __half* x, const __half* wt, OutT* out, int m, i
         else g.out_f32 = out;
         return tiled_gemm(g, stream);
     }
+    // What reaches this: a vocabulary projection of up to 64 rows, an N that is no multiple of 32 (a router of few experts, a shard of odd width) and, through
+    // the entry point, an x without 16-byte alignment.  Of these only the last two and 32768 – 65535 columns leave the chip short of waves, so that K is split.
     int mt = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
     int row_blocks = cdiv(m, 16 * mt);
     int ntile2 = cdiv(n, 32);
