@@ -15,18 +15,18 @@
 namespace fh {
 
 // Zeros by a launch of the stream: a memory fill recorded into a captured graph has gone wrong on replays after the first.
-// Thread i writes the i-th whole 16 bytes; the first 16 threads also the bytes ahead of them and behind.
+// A thread writes whole 16 bytes, a grid apart from 16 GiB on (a launch has less than 2^32 threads); the first 16 also the bytes ahead of them and behind.
+constexpr size_t ZERO_MAX_WGS = 1 << 22;
 __global__ __launch_bounds__(256) void zero_kernel(uint8_t* __restrict__ p, size_t bytes, size_t head, size_t quads) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, tail = head + quads * 16;
-    if (i < quads) *reinterpret_cast<uint4*>(p + head + i * 16) = uint4{0, 0, 0, 0};
+    for (size_t q = i; q < quads; q += (size_t)gridDim.x * 256) *reinterpret_cast<uint4*>(p + head + q * 16) = uint4{0, 0, 0, 0};
     if (i < head) p[i] = 0;
     if (i < bytes - tail) p[tail + i] = 0;
 }
 int zero_async(void* p, size_t bytes, hipStream_t s) {
     if (bytes == 0) return 0;
-    const size_t head = std::min<size_t>(bytes, -(uintptr_t)p & 15), quads = (bytes - head) / 16;
-    FH_REQUIRE(quads >> 38 == 0, "zero: %zu bytes", bytes);
-    hipLaunchKernelGGL(zero_kernel, dim3((unsigned)std::max<size_t>(1, (quads + 255) / 256)), dim3(256), 0, s, (uint8_t*)p, bytes, head, quads);
+    const size_t head = std::min<size_t>(bytes, -(uintptr_t)p & 15), quads = (bytes - head) / 16, wgs = std::max<size_t>(1, (quads + 255) / 256);
+    hipLaunchKernelGGL(zero_kernel, dim3((unsigned)std::min(wgs, ZERO_MAX_WGS)), dim3(256), 0, s, (uint8_t*)p, bytes, head, quads);
     FH_CHECK_LAUNCH();
     return 0;
 }

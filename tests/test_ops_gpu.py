@@ -322,6 +322,21 @@ def test_allocated_memory_is_zero_on_return(env):
     assert lib.ferrum_hip_stream_destroy(stream) == 0
 
 
+def test_zeros_of_any_length(env):
+    """A range of more 16-byte pieces than a launch has threads, from an odd address to an odd end, its last bytes and those around it."""
+    import ctypes as C
+    lib, p, size, sevens, got = env[0].load_library(), C.c_void_p(), (1 << 36) + (1 << 20), (C.c_uint8 * 64)(*[7] * 64), (C.c_uint8 * 64)()
+    assert lib.ferrum_hip_alloc(C.byref(p), C.c_size_t(size)) == 0
+    places = [0, 1 << 34, (1 << 34) + (1 << 20), (1 << 36) - 32, size - 64]
+    for at in places:
+        assert lib.ferrum_hip_memcpy_h2d(C.c_void_p(p.value + at), sevens, C.c_size_t(64), None) == 0
+    assert lib.ferrum_hip_memset_zero(C.c_void_p(p.value + 5), C.c_size_t(size - 5 - 9), None) == 0
+    for at in places:
+        assert lib.ferrum_hip_memcpy_d2h(got, C.c_void_p(p.value + at), C.c_size_t(64), None) == 0
+        assert bytes(got) == bytes(7 if at + i < 5 or at + i >= size - 9 else 0 for i in range(64)), at
+    assert lib.ferrum_hip_free(p) == 0
+
+
 def test_zeros_on_every_replay(env):
     """Ranges that start and end anywhere, alone and on each of several replays of a captured graph with eager work and synchronizations in between."""
     import ctypes as C
