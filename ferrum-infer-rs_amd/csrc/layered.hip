@@ -1159,11 +1159,11 @@ private:
             return 0;
         }
         std::vector<E> v(total);
-        const int ks = k / 32;
+        constexpr int EP = 16 / sizeof(E), SK = 4 * EP;
         for (int g = 0; g < groups; g++)
             for (int r = 0; r < n; r++)
                 for (int c = 0; c < k; c++) {
-                    const size_t o = ((((size_t)g * (n / 16) + r / 16) * ks + c / 32) * 64 + ((c % 32) / 8) * 16 + r % 16) * 8 + c % 8;
+                    const size_t o = ((((size_t)g * (n / 16) + r / 16) * (k / SK) + c / SK) * 64 + ((c % SK) / EP) * 16 + r % 16) * EP + c % EP;
                     store(&v[o], at(g, r, c));
                 }
         return arena_.upload(&L->w, v);

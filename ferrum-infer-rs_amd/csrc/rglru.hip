@@ -31,27 +31,28 @@ __device__ __forceinline__ float one_minus_exp(float t) {
 // grid (tiles, row blocks, blocks of the block-diagonal projections); a wave owns one 16-channel tile (ra and ri)
 template <typename E, int MT, bool STEP>
 __global__ __launch_bounds__(256) void rglru_gates_kernel(RglruDims d, RglruBuffers<E> p, BatchView v) {
-    typedef typename Frag<E>::v8 v8;
+    constexpr int EP = 16 / sizeof(E), SK = 4 * EP;             // numbers of 16 bytes, K of a step
+    typedef E piece_t __attribute__((ext_vector_type(EP)));
     const int lane = threadIdx.x & 63, a = lane >> 4, b = lane & 15, rb = blockIdx.y, g = blockIdx.z;
     const int tile = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (tile * 16 >= d.bp) return;
-    const int ksteps = d.bp >> 5;
+    const int ksteps = d.bp / SK;
     const E* xrow[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) {
         const int r = (rb * MT + mt) * 16 + b;
-        xrow[mt] = p.u + (long)(r < v.T ? r : v.T - 1) * d.wp + g * d.bp + 8 * a;
+        xrow[mt] = p.u + (long)(r < v.T ? r : v.T - 1) * d.wp + g * d.bp + EP * a;
     }
-    const E* wr = p.gate_w + ((long)(g * (d.bp >> 4) + tile) * 2) * ksteps * 512 + lane * 8;
+    const E* wr = p.gate_w + ((long)(g * (d.bp >> 4) + tile) * 2) * ksteps * (64 * EP) + lane * EP;
     floatx4 acc[MT][2];
 #pragma unroll
     for (int mt = 0; mt < MT; mt++) { acc[mt][0] = (floatx4){0.f, 0.f, 0.f, 0.f}; acc[mt][1] = (floatx4){0.f, 0.f, 0.f, 0.f}; }
 #pragma unroll 2
     for (int s = 0; s < ksteps; s++) {
-        const v8 w0 = *reinterpret_cast<const v8*>(wr + (long)s * 512), w1 = *reinterpret_cast<const v8*>(wr + (long)(ksteps + s) * 512);
+        const piece_t w0 = *reinterpret_cast<const piece_t*>(wr + (long)s * (64 * EP)), w1 = *reinterpret_cast<const piece_t*>(wr + (long)(ksteps + s) * (64 * EP));
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
-            const v8 ax = *reinterpret_cast<const v8*>(xrow[mt] + s * 32);
+            const piece_t ax = *reinterpret_cast<const piece_t*>(xrow[mt] + s * SK);
             acc[mt][0] = Frag<E>::mma(ax, w0, acc[mt][0]);
             acc[mt][1] = Frag<E>::mma(ax, w1, acc[mt][1]);
         }

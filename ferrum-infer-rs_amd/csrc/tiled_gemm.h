@@ -1,8 +1,8 @@
 // Dense projections over weights stored as MFMA-fragment tiles, for 16-bit and 32-bit models.
 //
-// Tile layout (the one f16t uses): [groups][n / 16][k / 32][64 lanes][8]; lane (a, b) of a k-step holds W[16·tile + b][32·step + 8a .. +8],
-// so a wave load of a fragment is contiguous and IS the B operand.  The 32-bit form keeps the same 8 values per lane and feeds them
-// to eight v_mfma_f32_16x16x4_f32: both operands permute the contraction index the same way, so no re-layout is needed.
+// Tile layout (in 16 bits the one f16t uses): [groups][n / 16][k / 32][64 lanes][8]; lane (a, b) of a k-step holds W[16·tile + b][32·step + 8a .. +8],
+// so a wave load of a fragment is contiguous and IS an operand.  32 bits: [groups][n / 16][k / 16][64 lanes][4], W[16·tile + b][16·step + 4a .. +4],
+// fed to four v_mfma_f32_16x16x4_f32: both operands permute the contraction index the same way.
 // n and k are padded to multiples of 32 with zero rows / columns, activations have padded leading dimensions: no kernel masks K.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -33,7 +33,7 @@ template <> struct Frag<_Float16> {
 template <> struct Frag<float> {
     typedef floatx8 v8;
     typedef floatx4 v4;
-    // 16 bytes of a lane: four of its eight k
+    // (four k of a lane: projections; eight, in tiles like the 16-bit ones: attention)
     static __device__ __forceinline__ floatx4 mma(v4 a, v4 b, floatx4 c) {
 #pragma unroll
         for (int j = 0; j < 4; j++) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);

@@ -35,27 +35,11 @@ __device__ __forceinline__ void gemm_store(const TiledGemm<E>& p, int g, int row
     const long o = row * p.ldo + (p.rows.id ? 0 : g * p.out_group) + col;
     if (p.out_f32) p.out_f32[o] = v; else p.out[o] = (E)v;
 }
-template <typename E, bool RARE>
-__device__ __forceinline__ void gemm_epilogue(const TiledGemm<E>& p, const GemmSection& sec, int g, int place, int col, float v) {
-    const int row = gemm_out_row(p, place);
-    if (row < 0 || col >= p.n_store) return;
-    v *= sec.mul;
-    if (p.bias) v += p.bias[(long)g * p.n + col];
-    gemm_store(p, g, row, col, gemm_act<E, RARE>(sec, v));
-}
 template <typename E>
 __device__ __forceinline__ float gemm_glu(const GemmSection& sec, float gate, float up) {
     if (sec.act == GEMM_ACT_SILU_GLU) return gate * ActMath<E>::sigmoid(gate) * up;
     if (sec.act == GEMM_ACT_GELU_GLU) return gelu_tanh_f32<E>(gate) * up;
     return clamped_glu_f32<E>(gate, up, sec.p, sec.q);
-}
-// accumulators of a (gate, up) pair of tiles; col: the gate's column
-template <typename E>
-__device__ __forceinline__ float gemm_gated(const TiledGemm<E>& p, const GemmSection& sec, int col, float gate, float up) {
-    gate *= sec.mul;
-    up *= sec.mul;
-    if (p.bias) { gate += p.bias[col]; up += p.bias[col + 16]; }
-    return gemm_glu<E>(sec, gate, up);
 }
 __device__ __forceinline__ int gemm_gated_col(const GemmSection& sec, int col) { return sec.begin + ((col - sec.begin) >> 5) * 16 + (col & 15); }
 template <typename E>
@@ -67,157 +51,230 @@ __device__ __forceinline__ GemmSection gemm_section(const TiledGemm<E>& p, int c
     return s;
 }
 
-// address of lane (a, b)'s 8 values of row tile t at k-step 0, and the distance between k-steps
+// address of the 16-byte piece a of row b of row tile t, and the distance between the steps of four pieces
 template <typename E>
 __device__ __forceinline__ const E* gemm_row(const TiledGemm<E>& p, int t, int g, int a, int b) {
+    constexpr int EP = 16 / sizeof(E);
     if (p.x_blocks) {
         const int tiles = (p.m + 15) >> 4;
-        return p.x + (long)p.x_blocks[t < tiles ? t : tiles - 1] * p.x_block_elems + (a * 16 + b) * 8;
+        return p.x + (long)p.x_blocks[t < tiles ? t : tiles - 1] * p.x_block_elems + (a * 16 + b) * EP;
     }
     int r = t * 16 + b;
     if (p.rows.id) {
         r = p.rows.id[r];
-        return p.x + (long)((unsigned)(r < p.m ? r : p.m - 1) / (unsigned)p.rows.div) * p.ldx + 8 * a;
+        return p.x + (long)((unsigned)(r < p.m ? r : p.m - 1) / (unsigned)p.rows.div) * p.ldx + EP * a;
     }
-    return p.x + (long)(r < p.m ? r : p.m - 1) * p.ldx + g * p.x_group + 8 * a;
+    return p.x + (long)(r < p.m ? r : p.m - 1) * p.ldx + g * p.x_group + EP * a;
 }
 template <typename E>
-__device__ __forceinline__ int gemm_row_step(const TiledGemm<E>& p) { return p.x_blocks ? 512 : 32; }
-
+__device__ __forceinline__ int gemm_row_step(const TiledGemm<E>& p) { return (p.x_blocks ? 1024 : 64) / sizeof(E); }
 // models whose gate tiles all lie ahead of the up tiles (elsewhere the distance of a pair's tiles stays a constant: 5 % of a gated launch of few rows)
 template <typename E> constexpr bool PAIRED = std::is_same_v<E, _Float16>;
 
-// grid (column blocks, row blocks, groups or K slabs); NW waves = (NW / kw) column groups × kw parts of K.  Two register buffers of U
-// k-steps: the next one is requested before the current one is multiplied; loads past the part's end repeat its last k-step.
-// EXT: with sorted rows, column factors, gated sections or rare activations (each is a branch on the latency-bound path of the launches without).
+// Few rows.  grid (column blocks, row blocks, groups or K slabs); a workgroup's waves are cw column groups × kw parts of K, and a part is taken in
+// chunks of U loads (16 bytes a lane: 32 of K, in 32 bits 16), the next chunk requested before the current one is multiplied; loads past the
+// part's end repeat its last one.
+//  * Weights go to registers, a contiguous KiB a load.
+//  * Rows go to LDS, a region of its own per wave: a load of 16 bytes a lane takes 64 · U bytes of 16 / U rows, whole cache lines, and the pieces
+//    of row r lie in the order 0 … xor (r & 7), so that the 16 lanes that read one piece of 16 rows touch every bank alike.
+// Bound by the weights' bytes and, below 30 MB, by the launch and the way to the first of them.  Fragments of the rows read from global memory, 64
+// bytes of 16 rows at a time, kept the load units busy for longer than the weights did: 32 × 4608 × 2048 10.0 → 7.4 µs, 8 × 4096 × 1024 4.8 →
+// 3.8, 8 × 1024 × 3072 6.5 → 5.3, 64 × 4096 × 2048 12.8 → 8.0, 32 × 32768 × 2048 31 → 26, in 32 bits 4 × 10240 × 2048 27.7 → 17.1 (a fragment is one
+// KiB there too); a read of the same weights and nothing else: 4.8, 2.7, 2.5, 4.0, 20.7, 14.2.
+// EXT: with sorted rows, rows from a cache, column factors, gated sections or rare activations (each is a branch on the latency-bound path of the
+// launches without).
+constexpr int FEW_LOADS = 4;
+struct FewRows { int kw_log2, cw, rows, chunk; uint32_t ldx16; };       // (rows of x in a region; loads of a part; pieces between rows of x)
 template <typename E, int MT, int J, bool EXT>
-__global__ __launch_bounds__(512) void tiled_gemm_kernel(TiledGemm<E> p, int kw) {
-    typedef typename Frag<E>::v8 v8;
-    if (!EXT) { p.rows.id = nullptr; p.col_scale = nullptr; p.pair = 0; }
+__global__ __launch_bounds__(512) void tiled_gemm_kernel(FewRows f, TiledGemm<E> p) {
+    constexpr int U = FEW_LOADS, EP = 16 / sizeof(E), PIECES = 4 * U, RPL = 64 / PIECES;       // numbers of a piece (16 bytes), pieces and rows of a load
+    typedef E piece_t __attribute__((ext_vector_type(EP)));
+    if (!EXT) { p.rows.id = nullptr; p.x_blocks = nullptr; p.col_scale = nullptr; p.pair = 0; }
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    floatx4* red = reinterpret_cast<floatx4*>(smem);            // [NW][MT·J][64]
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int a = lane >> 4, b = lane & 15;
-    const int cw = (blockDim.x >> 6) / kw, part = wave % kw, cg = wave / kw;
-    const int n0 = (blockIdx.x * cw + cg) * 16 * J, rb = blockIdx.y;
+    const int a = lane >> 4, b = lane & 15, kw = 1 << f.kw_log2;
+    const int part = wave & (kw - 1), cg = wave >> f.kw_log2;
+    const int n0 = (blockIdx.x * f.cw + cg) * 16 * J, rb = blockIdx.y;
     const int z = p.slabs > 1 ? blockIdx.z : 0;
     int g = p.slabs > 1 ? 0 : blockIdx.z;
-    if (p.rows.id) {
-        if (rb * 16 * MT >= *p.rows.total) return;
-        g = p.rows.group[rb];
-    }
-    const int ksteps = p.k >> 5, parts = kw * p.slabs, mine = z * kw + part;
+    const int loads = (unsigned)p.k / (4 * EP);
     const bool live = n0 < p.n;
-    const int s0 = live ? ksteps * mine / parts : 0, s1 = live ? ksteps * (mine + 1) / parts : 0;
-    const E* xrow[MT];
-    const int xs = gemm_row_step(p);
+    const int s0 = min(((z << f.kw_log2) + part) * f.chunk, loads), s1 = live ? min(s0 + f.chunk, loads) : 0;
+    // the rows that this lane copies, in pieces from p.x; places without a row repeat the last one
+    typedef std::conditional_t<EXT, uint64_t, uint32_t> place_t;        // (a cache may be larger than 2^32 pieces)
+    place_t at[MT * U];
+    const int row_in = lane / PIECES;
+    int id = 0;
+    if (EXT && p.rows.id) {
+        const int first = rb * 16 * MT, total = *p.rows.total;
+        id = p.rows.id[first + (lane & (16 * MT - 1))];
+        g = p.rows.group[rb];
+        if (first >= total) return;
+        const int row = (int)((unsigned)min(id, p.m - 1) / (unsigned)p.rows.div);
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++) xrow[mt] = gemm_row(p, rb * MT + mt, g, a, b);
-    const bool halves = PAIRED<E> && J == 2 && p.pair;
-    const E* wt = p.w + ((long)g * (p.n >> 4) + (!live ? 0 : halves ? n0 >> 5 : n0 >> 4)) * ksteps * 512 + lane * 8;
-    const int next_tile = halves ? p.pair : 1;
-    floatx4 acc[MT][J];
+        for (int l = 0; l < MT * U; l++) at[l] = (place_t)__shfl(row, l * RPL + row_in) * f.ldx16;
+    } else if (EXT && p.x_blocks) {
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int j = 0; j < J; j++) acc[mt][j] = (floatx4){0.f, 0.f, 0.f, 0.f};
-    // (four row tiles by two: two k-steps, 150 registers; four spilled, which cost 13 %: 60 × 8192 × 2048 16.9 → 14.7 µs, 100 × 6144 × 2048
-    // 25.6 → 21.4)
-    constexpr int U = sizeof(E) == 2 ? (MT * J == 1 ? 8 : MT * J == 8 ? 2 : 4) : 1;
-    v8 bw[2][U][J], ax[2][U][MT];
-    auto load = [&](v8 (&bq)[U][J], v8 (&aq)[U][MT], int s) {
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int ss = min(s + u, s1 - 1);
-#pragma unroll
-            for (int j = 0; j < J; j++) bq[u][j] = __builtin_nontemporal_load(reinterpret_cast<const v8*>(wt + ((long)j * next_tile * ksteps + ss) * 512));
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) aq[u][mt] = *reinterpret_cast<const v8*>(xrow[mt] + (long)ss * xs);
+        for (int l = 0; l < MT * U; l++) {
+            const int r = min(rb * 16 * MT + l * RPL + row_in, p.m - 1);
+            at[l] = (place_t)(p.x_blocks[r >> 4] * (p.x_block_elems / EP) + (r & 15));
         }
-    };
-    auto mul = [&](v8 (&bq)[U][J], v8 (&aq)[U][MT], int s) {
+    } else {
+#pragma unroll
+        for (int l = 0; l < MT * U; l++) at[l] = (place_t)min(rb * 16 * MT + l * RPL + row_in, p.m - 1) * f.ldx16 + (place_t)g * (place_t)(p.x_group / EP);
+    }
+    const int spread = EXT && p.x_blocks ? 4 : 0;               // (log2 of the pieces between a row's pieces)
+    const bool halves = PAIRED<E> && J == 2 && EXT && p.pair;
+    const unsigned char* wt = reinterpret_cast<const unsigned char*>(p.w) + ((long)g * (p.n >> 4) + (!live ? 0 : halves ? n0 >> 5 : n0 >> 4)) * loads * 1024 + lane * 16;
+    const long next_tile = (long)(halves ? p.pair : 1) * loads * 1024;
+    const int buffer = f.rows * PIECES * 16, region = max(2 * buffer, MT * J * 1024);
+    unsigned char* const rows_buf = smem + wave * region;
+    piece_t bw[2][U][J];
+    auto load = [&](piece_t (&bq)[U][J], int buf, int s) {
+#pragma unroll
+        for (int l = 0; l < MT * U; l++)
+            if (l * RPL < f.rows) {
+                const int piece = min(4 * s + ((lane & (PIECES - 1)) ^ ((l * RPL + row_in) & 7)), 4 * s1 - 1);
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(p.x + (uint64_t)(at[l] + ((place_t)piece << spread)) * EP),
+                                                 (__attribute__((address_space(3))) void*)(rows_buf + buf * buffer + l * 1024), 16, 0, 0);
+            }
+        // (rows ahead of weights: the wait of mul counts the latter)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < U; u++)
-            if (s + u < s1) {
 #pragma unroll
-                for (int j = 0; j < J; j++)
-#pragma unroll
-                    for (int mt = 0; mt < MT; mt++) acc[mt][j] = Frag<E>::mma(aq[u][mt], bq[u][j], acc[mt][j]);
-            }
+            for (int j = 0; j < J; j++) bq[u][j] = __builtin_nontemporal_load(reinterpret_cast<const piece_t*>(wt + j * next_tile + (long)min(s + u, s1 - 1) * 1024));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
     };
-    // every buffer is requested in the block that multiplies the other one, so each wait counts exactly the loads it needs
-    if (s0 < s1) {
-        int s = s0;
-        load(bw[0], ax[0], s);
-        while (true) {
-            if (s + U >= s1) { mul(bw[0], ax[0], s); break; }
-            load(bw[1], ax[1], s + U);
-            mul(bw[0], ax[0], s);
-            s += U;
-            if (s + U >= s1) { mul(bw[1], ax[1], s); break; }
-            load(bw[0], ax[0], s + U);
-            mul(bw[1], ax[1], s);
-            s += U;
-        }
-    }
-    if (p.slabs > 1) p.out_f32 += z * p.slab_stride;
+    if (s0 < s1) load(bw[0], 0, s0);
     const GemmSection sec = gemm_section(p, n0);
-    const bool gated = EXT && J == 2 && gemm_gated_act(sec.act);
-    if (kw == 1) {
-        if (!live) return;
-        if constexpr (J == 2)
-            if (gated) {
+    floatx4 bias[J], acc[MT][J];
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++)
+    for (int j = 0; j < J; j++) {
+        bias[j] = (floatx4){0.f, 0.f, 0.f, 0.f};
+        if (p.bias && live) bias[j] = *reinterpret_cast<const floatx4*>(p.bias + (long)g * p.n + n0 + 16 * j + 4 * a);
 #pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const int row = gemm_out_row(p, (rb * MT + mt) * 16 + 4 * a + r);
-                        if (row >= 0) gemm_store(p, g, row, gemm_gated_col(sec, n0 + b), gemm_gated(p, sec, n0 + b, acc[mt][0][r], acc[mt][J - 1][r]));
-                    }
-                return;
-            }
+        for (int mt = 0; mt < MT; mt++) acc[mt][j] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    }
+    int my_row[MT];
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++)
+    for (int mt = 0; mt < MT; mt++) my_row[mt] = min(16 * mt + b, f.rows - 1);
+    // multiplies a chunk of `steps` loads (0: all U); its rows have landed when at most `later` loads, the weights of the chunk behind it, are under way
+    auto mul = [&](piece_t (&bq)[U][J], int buf, auto later, int steps) {
+        constexpr int vm = decltype(later)::value;
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt((vm & 15) | 0xF70 | (vm >> 4) << 14);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (vm == 0 && u >= steps) break;
+            piece_t x[MT];
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+                x[mt] = *reinterpret_cast<const piece_t*>(rows_buf + buf * buffer + (my_row[mt] * PIECES + ((4 * u + a) ^ (my_row[mt] & 7))) * 16);
 #pragma unroll
             for (int j = 0; j < J; j++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) gemm_epilogue<E, EXT>(p, sec, g, (rb * MT + mt) * 16 + 4 * a + r, n0 + 16 * j + b, acc[mt][j][r]);
-        return;
+                for (int mt = 0; mt < MT; mt++) acc[mt][j] = Frag<E>::mma(bq[u][j], x[mt], acc[mt][j]);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");              // (the buffer is read before it is written again)
+    };
+    typedef std::integral_constant<int, U * J> behind;
+    typedef std::integral_constant<int, 0> last;
+    // 32 bits: sums of 128 products, then sums of those (relative error at K = 2048 / 8736: 2.1 / 2.2e-7, parts summed whole 2.9 / 3.8e-7; no slower)
+    constexpr bool F32 = sizeof(E) == 4;
+    floatx4 sums[F32 ? MT : 1][F32 ? J : 1] = {};
+    if (s0 < s1) {
+        int s = s0;
+        for (; s + 2 * U < s1; s += 2 * U) {
+            load(bw[1], 1, s + U);
+            mul(bw[0], 0, behind{}, U);
+            load(bw[0], 0, s + 2 * U);
+            mul(bw[1], 1, behind{}, U);
+            if constexpr (F32)
+#pragma unroll
+                for (int t = 0; t < MT * J; t++) {
+                    sums[t / J][t % J] += acc[t / J][t % J];
+                    acc[t / J][t % J] = (floatx4){0.f, 0.f, 0.f, 0.f};
+                }
+        }
+        if (s + U < s1) {
+            load(bw[1], 1, s + U);
+            mul(bw[0], 0, behind{}, U);
+            mul(bw[1], 1, last{}, s1 - s - U);
+        } else {
+            mul(bw[0], 0, last{}, s1 - s);
+        }
+        if constexpr (F32)
+#pragma unroll
+            for (int t = 0; t < MT * J; t++) acc[t / J][t % J] += sums[t / J][t % J];
     }
+    // the parts' sums, in their order, through the waves' regions (their rows are used up); tile t of a column group is finished by part t mod kw.
+    // The weights are the first operand: a lane holds four neighbouring columns of one row.
+    floatx4* const red = reinterpret_cast<floatx4*>(rows_buf);
 #pragma unroll
-    for (int mt = 0; mt < MT; mt++)
-#pragma unroll
-        for (int j = 0; j < J; j++) red[(wave * MT * J + mt * J + j) * 64 + lane] = acc[mt][j];
-    __syncthreads();
+    for (int t = 0; t < MT * J; t++) red[t * 64 + lane] = acc[t / J][t % J];
+    if (kw > 1) __syncthreads();
     if (!live) return;
     auto summed = [&](int t) {
-        floatx4 v = red[(cg * kw * MT * J + t) * 64 + lane];
-        for (int q = 1; q < kw; q++) v += red[((cg * kw + q) * MT * J + t) * 64 + lane];
-        return v;
+        const unsigned char* v = smem + (size_t)cg * kw * region + (t * 64 + lane) * 16;
+        floatx4 sum = *reinterpret_cast<const floatx4*>(v);
+#pragma unroll 1
+        for (int q = 1; q < kw; q++) sum += *reinterpret_cast<const floatx4*>(v += region);
+        return sum;
     };
-    if (gated) {
-        for (int mt = part; mt < MT; mt += kw) {
-            const floatx4 gate = summed(mt * J), up = summed(mt * J + 1);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int row = gemm_out_row(p, (rb * MT + mt) * 16 + 4 * a + r);
-                if (row >= 0) gemm_store(p, g, row, gemm_gated_col(sec, n0 + b), gemm_gated(p, sec, n0 + b, gate[r], up[r]));
-            }
-        }
-        return;
-    }
-    // tile t of the column group is summed (in the order of the K parts) and finished by part t mod kw
-    for (int t = part; t < MT * J; t += kw) {
-        const floatx4 v = summed(t);
+    if (p.slabs > 1) p.out_f32 += z * p.slab_stride;
+    const bool gated = EXT && J == 2 && gemm_gated_act(sec.act);
+    const bool vec = p.n_store % 4 == 0 && p.ldo % 4 == 0 && p.out_group % 4 == 0 && p.ld_col_scale % 4 == 0 && ((uintptr_t)p.out & 7) == 0 && ((uintptr_t)p.out_f32 & 15) == 0;
+    const int tiles = gated ? J : 1;
+#pragma unroll 1
+    for (int t = part * tiles; t < MT * J; t += kw * tiles) {
         const int mt = t / J, j = t % J;
+        floatx4 v = summed(t) * sec.mul + (j ? bias[J - 1] : bias[0]);
+        int col = n0 + 16 * j + 4 * a, row = (rb * MT + mt) * 16 + b;
+        if (EXT && p.rows.id) row = __shfl(id, 16 * mt + b);
+        if (row >= p.m) row = -1;
+        if (gated) {
+            const floatx4 up = summed(t + J - 1) * sec.mul + bias[J - 1];
 #pragma unroll
-        for (int r = 0; r < 4; r++) gemm_epilogue<E, EXT>(p, sec, g, (rb * MT + mt) * 16 + 4 * a + r, n0 + 16 * j + b, v[r]);
+            for (int r = 0; r < 4; r++) v[r] = gemm_glu<E>(sec, v[r], up[r]);
+            col = gemm_gated_col(sec, col);
+        } else if (sec.act != GEMM_ACT_NONE) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = gemm_act<E, EXT>(sec, v[r]);
+        }
+        if (row < 0) continue;
+        if (!vec) {
+#pragma unroll 1
+            for (int r = 0; r < 4; r++)
+                if (gated || col + r < p.n_store) gemm_store(p, g, row, col + r, r == 0 ? v[0] : r == 1 ? v[1] : r == 2 ? v[2] : v[3]);
+            continue;
+        }
+        if (!gated && col >= p.n_store) continue;
+        if (p.row_scale) v *= (float)p.row_scale[row * p.ld_scale + g];
+        typedef typename Frag<E>::v4 v4;
+        if (p.col_scale) {
+            const v4 c = *reinterpret_cast<const v4*>(p.col_scale + p.col_scale_row[row] * p.ld_col_scale + col);
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] *= (float)c[r];
+        }
+        const long o = row * p.ldo + (p.rows.id ? 0 : g * p.out_group) + col;
+        if (p.out_f32) *reinterpret_cast<floatx4*>(p.out_f32 + o) = v;
+        else {
+            v4 y;
+#pragma unroll
+            for (int r = 0; r < 4; r++) y[r] = (E)v[r];
+            *reinterpret_cast<v4*>(p.out + o) = y;
+        }
     }
 }
 
 // Prompts: 2 × 2 waves hold MI × NJ tiles of 16 × 16 each.  Both operands go through LDS, copied there by the load unit itself:
-//  * weights in stages of one k-step, a ring of 2G − 1: 16 bytes of every lane of a fragment.  In 16 bits that is 32 of K, one 1-KiB load in
-//    lane order; in 32 bits half of a fragment, 16 of K (the first or the last four of every lane's eight);
+//  * weights in stages of one k-step, a ring of 2G − 1: one 1-KiB load per fragment, 32 of K, in 32 bits 16;
 //  * rows in granules of two steps, a ring of G; a load takes 128 bytes (a cache line) of each of 8 rows, and the 16-byte pieces of row r lie
 //    in the order 0 … 7 xor r, so that the 16 lanes that read one piece of 16 rows touch every bank alike.
 __device__ const uint16_t zero_fragment[512] = {};
@@ -233,9 +290,9 @@ template <typename E, int MI, int NJ, int G, int PER_CU>
 __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E> p, int mtiles, int ntiles) {
     typedef BigTile<MI, NJ, G> T;
     typedef typename Frag<E>::v8 v8;
-    constexpr bool HALVES = sizeof(E) == 4;
+    constexpr bool F32 = sizeof(E) == 4;
     constexpr int EP = 16 / sizeof(E), SK = 4 * EP;                     // elements of 16 bytes, K of a step
-    typedef std::conditional_t<HALVES, typename Frag<E>::v4, v8> operand;
+    typedef E operand __attribute__((ext_vector_type(EP)));
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char *const rows_lds = smem, *const w_lds = rows_lds + G * T::GRANULE;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -256,23 +313,23 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
 #pragma unroll
     for (int i = 0; i < MI; i++) {
         const int r = (MI * wave + i) * 8 + (lane >> 3);
-        ap[i] = HALVES ? gemm_row(p, (m0 + r) >> 4, g, piece >> 1, r & 15) + 4 * (piece & 1) : gemm_row(p, (m0 + r) >> 4, g, piece, r & 15);
+        ap[i] = gemm_row(p, (m0 + r) >> 4, g, piece, r & 15);
     }
 #pragma unroll
     for (int i = 0; i < NJ / 2; i++) {
         const int t = min((n0 >> 4) + NJ / 2 * wave + i, ntl - 1);
-        bp[i] = p.w + ((long)g * ntl + (p.pair ? (t >> 1) + (t & 1) * p.pair : t)) * (p.k >> 5) * 512 + lane * 8;
+        bp[i] = p.w + ((long)g * ntl + (p.pair ? (t >> 1) + (t & 1) * p.pair : t)) * n * (64 * EP) + lane * EP;
     }
-    const int xs = (HALVES ? 1 : 2) * gemm_row_step(p);
+    const int xs = 2 * gemm_row_step(p);
     const E* none = reinterpret_cast<const E*>(zero_fragment) + lane * EP;       // (past the end of K)
 #define BIG_COPY(src, dst) __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src), (__attribute__((address_space(3))) void*)(dst), 16, 0, 0)
     auto issue_rows = [&](int i, int place, bool in) {
         BIG_COPY(in ? ap[i] : none, rows_lds + place * T::GRANULE + (MI * wave + i) * 1024);
         ap[i] += xs;
     };
-    auto issue_w = [&](int i, int place, bool in, bool second) {        // (second: of a fragment's halves)
+    auto issue_w = [&](int i, int place, bool in) {
         BIG_COPY(in ? bp[i] : none, w_lds + place * T::STAGE + (NJ / 2 * wave + i) * 1024);
-        bp[i] += !HALVES ? 512 : second ? 508 : 4;
+        bp[i] += 64 * EP;
     };
 #undef BIG_COPY
     floatx4 acc[MI][NJ];
@@ -280,15 +337,15 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     for (int i = 0; i < MI; i++)
 #pragma unroll
         for (int j = 0; j < NJ; j++) acc[i][j] = (floatx4){0.f, 0.f, 0.f, 0.f};
-    // 32 bits: sums of 128 products, then sums of those, as short as the few-row kernel's parts of K ever are.  Relative error against 64 bits
-    // at K = 512 / 2048 / 6144: 2.1 / 2.2 / 2.4e-7, with sums of 512 4.0 / 4.0 / 4.1e-7 and 2 % faster, the few-row kernel 2.1 / 4.0 / 7.0e-7.
-    floatx4 sum[HALVES ? MI : 1][HALVES ? NJ : 1] = {};
+    // 32 bits: sums of 128 products, then sums of those, as in the few-row kernel.  Relative error against 64 bits at K = 512 / 2048 / 6144:
+    // 2.1 / 2.2 / 2.4e-7, with sums of 512 4.0 / 4.0 / 4.1e-7 and 2 % faster.
+    floatx4 sum[F32 ? MI : 1][F32 ? NJ : 1] = {};
     struct Operands { operand x[MI], w[NJ]; };
     constexpr int READS = MI + NJ;
     const unsigned char* my_w = w_lds + wn * NJ * 1024 + lane * 16;
     const unsigned char* my_rows[2];
 #pragma unroll
-    for (int h = 0; h < 2; h++) my_rows[h] = rows_lds + wm * MI * 2048 + b * 128 + ((HALVES ? 2 * a + h : 4 * h + a) ^ (b & 7)) * 16;
+    for (int h = 0; h < 2; h++) my_rows[h] = rows_lds + wm * MI * 2048 + b * 128 + ((4 * h + a) ^ (b & 7)) * 16;
     // fragment f of a k-step: half h of the granule at `gran`, the weight stage at `stage`
     auto read = [&](Operands& o, int f, int h, int gran, int stage) {
         if (f < NJ) o.w[f] = *reinterpret_cast<const operand*>(my_w + stage * T::STAGE + f * 1024);
@@ -319,7 +376,7 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
 #pragma unroll
         for (int q = 0; q <= READS; q++) {
             if (q < READS) read(then, q, ODD ? 0 : 1, from, to);
-            if (q < NJ / 2) issue_w(q, stage, in, !ODD);          // (2G − 1 steps on: the other half)
+            if (q < NJ / 2) issue_w(q, stage, in);
             else if (ODD && q < LOADS) issue_rows(q - NJ / 2, gran, rows_in_k);
 #pragma unroll
             for (int m = q * PER; m < (q < READS ? (q + 1) * PER : MI * NJ); m++) acc[m / NJ][m % NJ] = Frag<E>::mma(now.w[m % NJ], now.x[m / NJ], acc[m / NJ][m % NJ]);
@@ -330,7 +387,7 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
 #pragma unroll
     for (int i = 0; i < T::STAGES; i++) {
 #pragma unroll
-        for (int f = 0; f < NJ / 2; f++) issue_w(f, i, i < n, i % 2 == 1);
+        for (int f = 0; f < NJ / 2; f++) issue_w(f, i, i < n);
         if (i % 2 == 0) {
 #pragma unroll
             for (int f = 0; f < MI; f++) issue_rows(f, i / 2, SK * i + EP * piece < p.k);
@@ -347,7 +404,7 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
         step(odd, even, std::true_type{}, t + 1, stage, gran);
         stage = stage_after(stage);
         gran = granule_after(gran);
-        if (HALVES && ((t & 6) == 6 || t + 2 >= n))
+        if (F32 && ((t & 6) == 6 || t + 2 >= n))
 #pragma unroll
             for (int i = 0; i < MI; i++)
 #pragma unroll
@@ -460,22 +517,22 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
 //   128 × 256 → 128 × 128     256 tiles: 456 × 16384 × 2048   39.5 → 39.0     260: 456 × 16640 × 2048   53.9 → 56.3
 //   128 × 64 → 128 × 128      256 of 128 × 128: 200 × 16384 × 6144   72 → 81, 968 × 4096 × 2048   26 → 29     264: 200 × 16896 × 6144   100 → 90
 //   64 × 64 → 128 × 64        256: 253 × 4096 × 2048   14.5 → 17.3, 125 × 8192 × 4096   26 → 31     288: 253 × 4608 × 2048   19.8 → 17.5
-//   few rows → 64 × 64        112: 253 × 1792 × 2048   13.9 → 14.2     128: 253 × 2048 × 2048   14.0 → 14.2, 125 × 4096 × 1024   9.9 → 9.6
-//                             144: 253 × 2304 × 2048   22.5 → 14.3
+//   few rows → 64 × 64        128: 253 × 2048 × 2048   9.0 → 14.3     192: 128 × 6144 × 2048   14.5 → 15.1, 65 × 6144 × 4096   27.1 → 26.0
+//                             224: 400 × 2048 × 1024   8.9 → 8.8      256: 65 × 8192 × 4096   30.3 → 28.6      288: 192 × 6144 × 2048   24.1 → 17.2
 template <typename E>
 static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
     auto tiles = [&](int r, int c) { return (long)(g.rows.id ? g.rows.max_blocks * (g.rows.block / r) : cdiv(g.m, r)) * cdiv(g.n, c) * g.groups; };
     if constexpr (sizeof(E) == 4) {
-        // 32 bits: bound by the products alone, so the tile whose rounds over the CUs take least (µs of a round below, K = 2048; the few-row
-        // kernel, which reads both operands from L2 for every 64 × 32 outputs, is left at 75 TFLOP/s of the 154 of a large product):
+        // 32 bits: bound by the products alone, so the tile whose rounds over the CUs take least (µs of a round below, K = 2048):
         //                        128 × 128   128 × 64   64 × 64   few-row kernel
-        //   2048 × 2048 × 2048      142         147                  222
-        //   1000 × 6144 × 2048      266         215                  330
-        //   1000 × 2048 × 2048      140          83                  115
-        //   500 × 2048 × 2048       139                    50         62
-        //   1000 × 1024 × 512        41                    17         19
-        //   128 × 8192 × 2048       139                    50         63
-        //   256 × 2048 × 2048       138                    47         39      (128 tiles: too few; 253 × 2304 × 2048, 144 tiles: 46 and 60)
+        //   2048 × 2048 × 2048      142         147
+        //   1000 × 6144 × 2048      266         215
+        //   1000 × 2048 × 2048      140          83
+        //   500 × 2048 × 2048       139                    50
+        //   1000 × 1024 × 512        41                    17
+        //   128 × 8192 × 2048       139                    47         47
+        //   253 × 2048 × 2048       138                    46         25      (128 tiles of 64 × 64: too few)
+        //   128 × 6144 × 2048                              47         45      (192)
         const long full = cdiv(tiles(128, 128), 256) * 133L, half = cdiv(tiles(128, 64), 256) * 72L, small = cdiv(tiles(64, 64), 256) * 42L;
         if ((g.rows.id && g.rows.block < 128) || small < std::min(full, half)) return launch_big<E, 2, 2, 3, 3>(g, s);
         return half < full ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 4, 4, 2, 2>(g, s);
@@ -496,8 +553,21 @@ int tiled_gemm_slabs(int m, int n, int k) {
 
 template <typename E, int MT, int J, bool EXT>
 static int launch_small(const TiledGemm<E>& g, dim3 grid, int nw, int kw, hipStream_t s) {
-    const size_t lds = kw == 1 ? 0 : (size_t)nw * MT * J * 1024;
-    hipLaunchKernelGGL((tiled_gemm_kernel<E, MT, J, EXT>), grid, dim3(64 * nw), lds, s, g, kw);
+    FewRows f;
+    f.kw_log2 = kw >= 8 ? 3 : kw >= 4 ? 2 : kw >= 2 ? 1 : 0;
+    f.cw = nw >> f.kw_log2;
+    f.rows = g.rows.id ? 16 * MT : std::min(16 * MT, (g.m + 3) / 4 * 4);
+    f.chunk = cdiv(g.k / (64 / (int)sizeof(E)), g.slabs << f.kw_log2);
+    f.ldx16 = (uint32_t)(g.ldx * sizeof(E) / 16);
+    const size_t lds = (size_t)nw * std::max(2 * f.rows * 64 * FEW_LOADS, MT * J * 1024);
+    if (lds > 64 * 1024) {
+        static bool attr = false;
+        if (!attr) {
+            FH_CHECK_HIP(hipFuncSetAttribute((const void*)tiled_gemm_kernel<E, MT, J, EXT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            attr = true;
+        }
+    }
+    hipLaunchKernelGGL((tiled_gemm_kernel<E, MT, J, EXT>), grid, dim3(64 * nw), lds, s, f, g);
     FH_CHECK_LAUNCH();
     return 0;
 }
@@ -510,6 +580,7 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     FH_REQUIRE(g.n > 0 && g.k > 0 && g.n % 32 == 0 && g.k % 32 == 0, "tiled_gemm: n=%d k=%d must be multiples of 32", g.n, g.k);
     FH_REQUIRE(g.ldx % 8 == 0 && g.x_group % 8 == 0 && g.n_store <= g.n && g.groups >= 1, "tiled_gemm: ldx=%ld group stride=%ld", g.ldx, g.x_group);
     FH_REQUIRE((g.out != nullptr) != (g.out_f32 != nullptr), "tiled_gemm: exactly one output");
+    FH_REQUIRE(!g.x_blocks || sizeof(E) == 2, "tiled_gemm: rows from a cache are 16-bit");
     FH_REQUIRE(g.slabs == 1 || (g.groups == 1 && g.out_f32 && !g.bias && !g.nsec && !g.row_scale), "tiled_gemm: slabs are plain fp32 partial sums");
     bool gated = false, rare = false;
     for (int i = 0; i < g.nsec; i++) {
@@ -528,71 +599,57 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     }
     constexpr bool F32 = sizeof(E) == 4;
     const long tiles = (rows.id ? (long)rows.max_blocks * (rows.block / 64) : cdiv(g.m, 64)) * cdiv(g.n, 64) * g.groups;
-    const bool enough_tiles = tiles >= knobs().tiled_big_min_tiles + F32;
+    const bool enough_tiles = tiles >= (knobs().tiled_big_min_tiles > 0 ? knobs().tiled_big_min_tiles : F32 ? 129 : 193);
     if (rows.id ? (F32 ? rows.block >= 64 && g.n >= 64 && enough_tiles : rows.block >= 128) : g.m > 64 && g.n >= 64 && g.slabs == 1 && enough_tiles) return launch_big(g, s);
-    // rows per workgroup: as many as there are, fewer where narrow outputs would leave CUs idle: in 16 bits as long as a round of 256 workgroups
-    // holds the launch (64 × 2048 × 4096, four row tiles | two: 20.6 | 12.8 µs; 65 × 1024 × 4096, two | one: 20.2 | 12.6; past the round, 24 × 3072 ×
-    // 2048, two | one: 7.7 | 8.4)
+    // Rows of a workgroup: as many as there are, fewer where narrow outputs would leave CUs idle: in 16 bits as long as a round of 256 workgroups
+    // holds the launch.
     int mt = rows.id ? rows.block / 16 : g.m <= 16 ? 1 : (g.m <= 32 ? 2 : 4);
     auto row_tiles = [&](int t) { return (long)cdiv(g.m, 16 * t) * (g.n / 16) * g.groups * g.slabs; };
     while (!rows.id && mt > 1 && (F32 ? row_tiles(mt) < knobs().tiled_min_tiles : row_tiles(mt / 2) <= 2 * knobs().tiled_min_tiles)) mt /= 2;
-    const int rbs = rows.id ? rows.max_blocks : cdiv(g.m, 16 * mt), ksteps = g.k / 32, zs = rows.id ? 1 : g.groups * g.slabs;
-    // Columns and K parts of a wave.  Several row tiles, whose fragments a wave reads again for every column group: 16 columns as long as a
-    // round of 256 workgroups holds all of them with K in four parts, else 32, and as many parts as make rounds / parts least (a tie: fewer
-    // parts where they are long, so that less is summed through LDS).  µs, bf16, weights from HBM, K in 4 / 2 parts of a workgroup's four waves:
-    //                            workgroups     16 columns      32 columns
-    //   64 × 4096 × 2048          256 | 128    12.9 | 20.4     14.5 | 22.9
-    //   64 × 5120 × 2048          320 | 160    21.1 | 20.4     14.6 | 23.1
-    //   64 × 8256 × 2048          516 | 258    28.8 | 35.2     23.6 | 23.4
-    //   64 × 8256 × 6144          516 | 258    82.7 | 97.4     66.1 | 59.1
-    //   64 × 5120 × 256                                         6.5 |  8.5      (two k-steps a part; 16 columns in two parts 6.9)
-    //   32 × 2560 × 6144 in four slabs                         14.7 | 13.4      (16 columns in two parts 16.7)
-    // One row tile: four parts up to a round of workgroups, two up to the next; 32 columns where 16 would be more than a round in two parts (8 × 8192 ×
-    // 2048: 16 columns 8.2, 32 8.6; 8256 columns: 11.3 and 10.9).  µs (four waves a workgroup, K split over kw of them):
-    //                            32 columns      16 columns      before
-    //                            kw 4   kw 2     kw 4   kw 2
-    //   8 × 4096 × 1024           5.2             4.9    5.3     5.6 (16, eight waves, kw 8)
-    //   8 × 6144 × 1024           5.6                    5.6     8.6 (16, eight waves, kw 8)
-    //   8 × 5120 × 2048           7.0             8.1    7.3
-    //   8 × 8192 × 2048           8.8                    8.3     10.4 (16, eight waves, kw 8)
-    //   16 × 10240 × 2048        12.7   12.0            14.2     12.8 (32, eight waves, kw 8)
-    //   8 × 1024 × 3072           8.0             6.5            7.4 (16, eight waves, kw 8)
-    // Fewer waves a workgroup wait for each other less.  Slabs of a long K want every wave they can get (1 × 2048 × 8192 in four: eight waves 8.1,
-    // four 8.4), and so do wide outputs that stream a long K: 8 × 24576 × 4096 in four parts of four waves 39.7, in eight of eight 36.8; 8 × 65536 × 2048
-    // in two parts 50, in four 43, in eight 42.  Of a short one rounds decide again: 8 × 49152 × 1024 in two parts 19.3, in eight 21.2.
-    // Sorted rows: K is split below 8192 column groups (24 blocks of 16 rows, 4096 × 2048: four parts 68, one 75; 64 blocks: 161 and 137).
-    const bool long_slabs = g.slabs > 1 && ksteps / g.slabs >= 64, narrow = sizeof(E) == 4 || long_slabs;
-    const long groups16 = (long)rbs * (g.n / 16) * zs;
-    const bool plain = !narrow && !rows.id, wide = plain && g.slabs == 1 && groups16 >= 896, several = plain && mt > 1 && !wide && !(g.n <= 96 && g.m > 64);
-    int J = several ? (groups16 <= 256 ? 1 : 2)
-            : narrow ? (groups16 / 2 < (g.slabs > 1 ? 256 : 257) ? 1 : 2)
-                     : (long)rbs * (g.n / 32) * g.groups < (g.n <= 96 && g.m > 64 ? 513 : mt == 1 ? 257 : 160) ? 1 : 2;       // (narrow outputs of prompts: two workgroups per CU)
+    // Columns of a wave (16 · J), waves of a workgroup, K parts among them; µs, bf16, weights from HBM, inside a graph:
+    //                             16 columns of a wave,                     32 columns                a read of the weights
+    //                             K in 4     K in 2     8 waves, K in 8     K in 4     8, K in 8      and nothing else
+    //   8 × 4096 × 1024            3.84       4.3        4.25                4.6                       2.7
+    //   8 × 1024 × 3072            5.35                  5.28                6.7        6.9            2.5
+    //   3 × 128 × 8128             8.88                  7.53               12.0       11.9            2.0
+    //   8 × 6144 × 1024            4.83       4.58       4.90                4.79                      3.7
+    //   7 × 6528 × 6912           17.3       18.8                           16.4       16.9           14.8
+    //   8 × 2048 × 8192, 4 slabs   8.96       9.4        8.72                           7.93           6.5
+    //   8 × 12288 × 1024           6.35       6.70       6.65                                          5.3
+    //   1 × 10240 × 2048           9.34       9.39       8.93               10.3                       7.8
+    //   8 × 20032 × 2048          15.4                  14.97               16.3       15.7           13.6
+    //   32 × 4608 × 2048           9.0        8.6       10.6                 7.42       7.60           4.8
+    //   32 × 2048 × 2048, 4 slabs  4.87       4.50                           4.79       5.12           2.7
+    //   60 × 8192 × 2048                     12.5                           10.6                       6.5
+    //   43 × 9600 × 1920          18.0                                      16.5 (K in 2: 14.1)        7.3
+    // One row tile: 16 columns, since a wave then has half as much under way before its first sum; K in four up to a round of 256 workgroups
+    // and past two, in two between, where that saves a round, unless the parts of a long K get longer than the second round costs; eight waves
+    // where a wave of four would read 16 loads and more.  Several row tiles: their rows are read again for every column group, so 32 columns
+    // past one round.  Four row tiles leave room for one workgroup per CU, so the parts that make rounds / parts least.
+    const int rbs = rows.id ? rows.max_blocks : cdiv(g.m, 16 * mt), zs = rows.id ? 1 : g.groups * g.slabs;
+    const int loads = g.k / (F32 ? 16 : 32) / g.slabs;                  // (of a wave that has all of a slab's K)
+    const long tiles16 = (long)rbs * (g.n / 16) * zs;
+    const bool two_rounds = !rows.id && tiles16 > 256 && tiles16 <= 512, longer = loads > 64 || (loads == 64 && g.slabs > 1);
+    int J = rows.id ? 2 : mt == 1 ? (two_rounds && longer ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
     if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : 2;
     if (gated) J = 2;
-    const long cols = g.n / (16 * J);
-    int nw = mt == 1 && (narrow || (wide && ksteps >= 128)) ? 8 : 4, kw = 1;
-    if (knobs().tiled_nw > 0) nw = std::min(8, knobs().tiled_nw);
-    if (several || (wide && mt == 1 && ksteps < 64)) {
-        const int steps = ksteps / g.slabs;
-        long least = 0;
-        for (int k : {4, 2, 1}) {
-            if (k > 1 && steps < 2 * k) continue;
-            const long rounds = cdiv((long)rbs * cdiv(cols, 4 / k) * zs, 256);
-            const bool tie = least && rounds * kw == least * k;
-            if (!least || rounds * kw < least * k || (tie && (k > 1 || steps >= 128) && (steps >= 32 || steps < 4 * kw))) { kw = k; least = rounds; }
-        }
-    } else if (wide && mt == 1) {
-        kw = nw;
-    } else {
-        const long enough = rows.id ? 8192 : J == 1 && plain ? 513 : 4096;
-        while (kw < nw && (long)rbs * cols * zs * kw < enough && ksteps >= 8 * kw * g.slabs) kw *= 2;
-    }
-    if (knobs().tiled_kw > 0) kw = std::min(nw, knobs().tiled_kw);
+    const long cols = g.n / (16 * J), blocks = (long)rbs * cols * zs;
+    int nw = mt == 1 && !rows.id && ((blocks > 512 && loads >= 64) || (blocks <= 256 && J == 1 && loads >= 96)) ? 8 : 4, kw = nw;
+    if (J == 1 && two_rounds) kw = 2;
+    if (two_rounds && g.slabs > 1 && loads == 64 && mt < 4) nw = kw = 8;
+    if (mt == 4 && rows.id) kw = 2;                                     // (64 tokens, 24 experts, blocks of 64, 2048 × 2048: in four 55, in two 48)
+    else if (mt == 4)
+        for (int k : {2, 1})
+            if (cdiv((long)rbs * cdiv(cols, 4 / k) * zs, 256) * kw <= cdiv((long)rbs * cdiv(cols, 4 / kw) * zs, 256) * k) kw = k;
+    while (kw > 1 && loads < 2 * kw) kw /= 2;
+    auto power_of_two = [](int v) { return v >= 8 ? 8 : v >= 4 ? 4 : v >= 2 ? 2 : 1; };
+    if (knobs().tiled_nw > 0) nw = std::min(mt == 4 ? 4 : 8, power_of_two(knobs().tiled_nw));
+    if (knobs().tiled_kw > 0 || kw > nw) kw = std::min(nw, power_of_two(knobs().tiled_kw > 0 ? knobs().tiled_kw : kw));
     const dim3 grid(cdiv(cols, nw / kw), rbs, zs);
     form_hit(rows.id ? FORM_TILED_GEMM_GROUPED : FORM_TILED_GEMM);
 #define SMALL(J_, EXT_) \
     (mt == 1 ? launch_small<E, 1, J_, EXT_>(g, grid, nw, kw, s) : mt == 2 ? launch_small<E, 2, J_, EXT_>(g, grid, nw, kw, s) : launch_small<E, 4, J_, EXT_>(g, grid, nw, kw, s))
-    if (rows.id || g.col_scale || gated || rare) return J == 1 ? SMALL(1, true) : SMALL(2, true);
+    if (rows.id || g.x_blocks || g.col_scale || gated || rare) return J == 1 ? SMALL(1, true) : SMALL(2, true);
     return J == 1 ? SMALL(1, false) : SMALL(2, false);
 #undef SMALL
 }

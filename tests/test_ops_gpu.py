@@ -405,6 +405,28 @@ def test_projections_take_the_faster_side_of_a_line(env, m, n, k, knobs):
     assert best["chosen"] < 1.1 * min(best.values()), best
 
 
+@pytest.mark.parametrize("kw", [0, 1, 2, 4, 8])
+@pytest.mark.parametrize("j", [1, 2])
+@pytest.mark.parametrize("m,n,k", [(1, 32, 32), (3, 64, 64), (4, 96, 96), (5, 160, 128), (13, 288, 160), (16, 32, 1120), (17, 96, 288), (32, 160, 1024), (33, 64, 544), (49, 96, 4128),
+                                   (64, 32, 256), (79, 96, 96)])
+def test_few_rows_of_every_count(env, m, n, k, j, kw, knobs, forms):
+    """Rows that fill no load and no tile, parts of K of no, one and several chunks that end within one, column groups past the last tile.  Against 64 bits: an fp32 sum
+    of K exact products errs by K x 2^-24 of the sum of their magnitudes at most, and fp16 rounds by 2^-11."""
+    pkg, B, ctx, O, torch = env
+    knobs.set(TILED_J=j, TILED_NW=8 if kw == 8 else 4, TILED_KW=kw, TILED_BIG_MIN_TILES=10 ** 6)
+    gen = torch.Generator("cuda").manual_seed(m * n + k)
+    a, b = (torch.randn(r, k, generator=gen, device="cuda").half() for r in (m, n))
+    buf = torch.full(((m + 2) * n,), 7.0, dtype=torch.float16, device="cuda")
+    out = buf[n:n + m * n]
+    forms.reset()
+    B.gemm_f16t(ctx, a, B.dense_repack_f16t(ctx, b, n, k), out, m, n, k)
+    ctx.sync()
+    forms.require("tiled_gemm")
+    want, size = a.double() @ b.double().T, a.double().abs() @ b.double().abs().T
+    assert ((out.reshape(m, n).double() - want).abs() <= 2.0 ** -11 * want.abs() + k * 2.0 ** -24 * size + 2.0 ** -25).all()
+    assert (buf[:n] == 7.0).all() and (buf[n + m * n:] == 7.0).all()
+
+
 @pytest.mark.parametrize("nq,nkv,tokens,pos,seqs,window", [(32, 4, 64, 700, 24, 0), (14, 2, 4096, 0, 1, 512), (32, 8, 700, 0, 1, 0)])
 def test_prompt_attention_takes_the_faster_unit(env, nq, nkv, tokens, pos, seqs, window, knobs):
     """Batches on both sides of the line between units of 64 and 128 rows, where the wrong one costs 12 to 40 %."""
