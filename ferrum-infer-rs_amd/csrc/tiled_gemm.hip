@@ -234,7 +234,10 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(FewRows f, TiledGemm<E>
 #pragma unroll 1
     for (int t = part * tiles; t < MT * J; t += kw * tiles) {
         const int mt = t / J, j = t % J;
-        floatx4 v = summed(t) * sec.mul + (j ? bias[J - 1] : bias[0]);
+        floatx4 v = bias[0];
+#pragma unroll
+        for (int i = 1; i < J; i++) v = j == i ? bias[i] : v;
+        v += summed(t) * sec.mul;
         int col = n0 + 16 * j + 4 * a, row = (rb * MT + mt) * 16 + b;
         if (EXT && p.rows.id) row = __shfl(id, 16 * mt + b);
         if (row >= p.m) row = -1;
@@ -625,12 +628,22 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     // One row tile: 16 columns, since a wave then has half as much under way before its first sum; K in four up to a round of 256 workgroups
     // and past two, in two between, where that saves a round, unless the parts of a long K get longer than the second round costs; eight waves
     // where a wave of four would read 16 loads and more.  Several row tiles: their rows are read again for every column group, so 32 columns
-    // past one round.  Four row tiles leave room for one workgroup per CU, so the parts that make rounds / parts least.
+    // past one round.  Four row tiles leave room for one workgroup per CU, two with 64 columns for two: the parts that make rounds / parts least.
+    // A vocabulary, many rounds of workgroups: the rows' share grows with rows and K (µs; 64 columns: with two row tiles and K in one part)
+    //                             16 columns, 8 waves   32 columns, 8 waves   32 columns, 4 waves   64 columns
+    //   8 × 128256 × 4096             154                                         > 160
+    //   8 × 131072 × 5376             226                    205                   205
+    //   16 × 151936 × 2048            117                     95                    98
+    //   32 × 131072 × 5376                                                         275                  231
+    //   32 × 151936 × 2048                                                         108                  117
+    //   64 × 151936 × 1024, 32 columns, K in four parts 97, in one 79; 49 × 16992 × 1376: 20.8 and 19.5
     const int rbs = rows.id ? rows.max_blocks : cdiv(g.m, 16 * mt), zs = rows.id ? 1 : g.groups * g.slabs;
     const int loads = g.k / (F32 ? 16 : 32) / g.slabs;                  // (of a wave that has all of a slab's K)
     const long tiles16 = (long)rbs * (g.n / 16) * zs;
     const bool two_rounds = !rows.id && tiles16 > 256 && tiles16 <= 512, longer = loads > 64 || (loads == 64 && g.slabs > 1);
-    int J = rows.id ? 2 : mt == 1 ? (two_rounds && longer ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
+    const bool ext = rows.id || g.x_blocks || g.col_scale || gated || rare, wide = !rows.id && tiles16 > 2048;
+    int J = rows.id ? 2 : mt == 1 ? ((two_rounds && longer) || (wide && (g.m > 12 || loads > 128)) ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
+    if (mt == 2 && wide && loads >= 128 && !ext && g.n % 64 == 0) J = 4;
     if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : 2;
     if (gated) J = 2;
     const long cols = g.n / (16 * J), blocks = (long)rbs * cols * zs;
@@ -638,9 +651,12 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     if (J == 1 && two_rounds) kw = 2;
     if (two_rounds && g.slabs > 1 && loads == 64 && mt < 4) nw = kw = 8;
     if (mt == 4 && rows.id) kw = 2;                                     // (64 tokens, 24 experts, blocks of 64, 2048 × 2048: in four 55, in two 48)
-    else if (mt == 4)
-        for (int k : {2, 1})
-            if (cdiv((long)rbs * cdiv(cols, 4 / k) * zs, 256) * kw <= cdiv((long)rbs * cdiv(cols, 4 / kw) * zs, 256) * k) kw = k;
+    else if (mt == 4 && (long)rbs * cdiv(cols, 4) * zs > 128) kw = 1;
+    else if (mt == 4 || J == 4)
+        for (int k : {2, 1}) {
+            const int slots = mt == 4 ? 256 : 512;
+            if (cdiv((long)rbs * cdiv(cols, 4 / k) * zs, slots) * kw <= cdiv((long)rbs * cdiv(cols, 4 / kw) * zs, slots) * k) kw = k;
+        }
     while (kw > 1 && loads < 2 * kw) kw /= 2;
     auto power_of_two = [](int v) { return v >= 8 ? 8 : v >= 4 ? 4 : v >= 2 ? 2 : 1; };
     if (knobs().tiled_nw > 0) nw = std::min(mt == 4 ? 4 : 8, power_of_two(knobs().tiled_nw));
@@ -649,7 +665,8 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     form_hit(rows.id ? FORM_TILED_GEMM_GROUPED : FORM_TILED_GEMM);
 #define SMALL(J_, EXT_) \
     (mt == 1 ? launch_small<E, 1, J_, EXT_>(g, grid, nw, kw, s) : mt == 2 ? launch_small<E, 2, J_, EXT_>(g, grid, nw, kw, s) : launch_small<E, 4, J_, EXT_>(g, grid, nw, kw, s))
-    if (rows.id || g.x_blocks || g.col_scale || gated || rare) return J == 1 ? SMALL(1, true) : SMALL(2, true);
+    if (ext) return J == 1 ? SMALL(1, true) : SMALL(2, true);
+    if (J == 4) return launch_small<E, 2, 4, false>(g, grid, nw, kw, s);
     return J == 1 ? SMALL(1, false) : SMALL(2, false);
 #undef SMALL
 }

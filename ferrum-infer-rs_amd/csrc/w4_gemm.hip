@@ -3331,12 +3331,11 @@ int f16t_repack(const __half* w_rowmajor, __half* out_tiled, int n, int k, hipSt
 }
 size_t f16t_elems(int n, int k) { return (size_t)cdiv(n, 16) * 16 * k; }
 
-// J = 16-column tiles per wave: 2, or 4 for two row tiles against a wide N (the lm_head at 17–32 rows: with 2 the activation
-// fragments a wave re-reads from L2 are as many bytes as the weights it streams from HBM)
-template <int MT, typename OutT, int J = 2>
+template <int MT, typename OutT>
 __global__ __launch_bounds__(256) void f16t_gemm_kernel(const __half* __restrict__ x, const __half* __restrict__ wt,
                                                         OutT* __restrict__ out, float* __restrict__ partial, int M, int N,
                                                         int K, int S, int rows_pad, int n_pad) {
+    constexpr int J = 2;                            // 16-column tiles of a wave
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
     const int ntile2 = blockIdx.x * 4 + wave;       // group of J 16-column tiles
@@ -3417,9 +3416,9 @@ static int f16t_gemm_impl(const __half* x, const __half* wt, OutT* out, int m, i
     if (m <= 0) return 0;
     FH_REQUIRE(k % 32 == 0, "f16t_gemm: K=%d must be a multiple of 32", k);
     // The projections of the layered models (tiled_gemm.hip) read the same weight tiles: prompts in LDS tiles (2048 × 4096 × 1024: 115 → 24 µs), few
-    // rows with K split over the waves of a workgroup and no reduce launch (8 × 4096 × 1024: 12 → 7 µs).  A wide N at few rows (the lm_head) streams
-    // its weights once either way and stays here, as do N that are no multiple of 32.
-    if (n % 32 == 0 && (m > 64 || n < 32768) && ((uintptr_t)x & 15) == 0) {
+    // rows with theirs in LDS and K split over the waves of a workgroup (8 × 4096 × 1024: 12 → 3.8; 8 × 151936 × 1024 55 → 48, 1 × 128256 × 4096 170 → 152,
+    // 48 × 128256 × 4096 278 → 207).
+    if (n % 32 == 0 && ((uintptr_t)x & 15) == 0) {
         TiledGemm<_Float16> g;
         g.x = reinterpret_cast<const _Float16*>(x); g.ldx = k; g.w = reinterpret_cast<const _Float16*>(wt);
         g.m = m; g.n = n; g.k = k; g.ldo = n;
@@ -3427,8 +3426,8 @@ static int f16t_gemm_impl(const __half* x, const __half* wt, OutT* out, int m, i
         else g.out_f32 = out;
         return tiled_gemm(g, stream);
     }
-    // What reaches this: a vocabulary projection of up to 64 rows, an N that is no multiple of 32 (a router of few experts, a shard of odd width) and, through
-    // the entry point, an x without 16-byte alignment.  Of these only the last two and 32768 – 65535 columns leave the chip short of waves, so that K is split.
+    // What reaches this: an N that is no multiple of 32 (a router of few experts, a shard of odd width) and, through the entry point, an x without
+    // 16-byte alignment.
     int mt = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
     int row_blocks = cdiv(m, 16 * mt);
     int ntile2 = cdiv(n, 32);
@@ -3438,12 +3437,6 @@ static int f16t_gemm_impl(const __half* x, const __half* wt, OutT* out, int m, i
     while (tasks * S < 2048 && S * 2 <= ksteps / 8) S *= 2;
     int rows_pad = row_blocks * 16 * mt, n_pad = ntile2 * 32;
     if (S > 1 && (size_t)S * rows_pad * n_pad * sizeof(float) > workspace_bytes) S = 1;
-    if (mt == 2 && S == 1 && n >= 32768 && n % 64 == 0) {       // wide N at 17–32 rows (the lm_head): 64 columns per wave
-        hipLaunchKernelGGL((f16t_gemm_kernel<2, OutT, 4>), dim3(cdiv(cdiv(n, 64), 4), row_blocks, 1), dim3(256), 0, stream, x, wt, out, workspace, m,
-                           n, k, 1, rows_pad, n_pad);
-        FH_CHECK_LAUNCH();
-        return 0;
-    }
     dim3 grid(cdiv(ntile2, 4), row_blocks, S);
     if (mt == 1) hipLaunchKernelGGL((f16t_gemm_kernel<1, OutT>), grid, dim3(256), 0, stream, x, wt, out, workspace, m, n, k, S, rows_pad, n_pad);
     else if (mt == 2) hipLaunchKernelGGL((f16t_gemm_kernel<2, OutT>), grid, dim3(256), 0, stream, x, wt, out, workspace, m, n, k, S, rows_pad, n_pad);
