@@ -10,17 +10,25 @@
 
 namespace fh {
 
-template <typename E, bool RARE = false>
-__device__ __forceinline__ float gemm_act(const GemmSection& sec, float v) {
-    if (sec.act == GEMM_ACT_SIGMOID) return ActMath<E>::sigmoid(v);
-    if (sec.act == GEMM_ACT_GELU_TANH) return gelu_tanh_f32<E>(v);
-    if (sec.act == GEMM_ACT_XIELU) return xielu_f32<E>(v, sec.p, sec.q);
-    if (sec.act == GEMM_ACT_RELU2) { v = fmaxf(v, 0.f); return v * v; }
-    if (sec.act == GEMM_ACT_SILU) return v * ActMath<E>::sigmoid(v);
-    if (RARE && sec.act == GEMM_ACT_SOFTPLUS) return softplus_f32<E>(v);
-    if (RARE && sec.act == GEMM_ACT_LOG_SIGMOID) return sec.p * log_sigmoid_f32<E>(v);
-    if (RARE && sec.act == GEMM_ACT_SOFTCAP) return sec.p * ActMath<E>::tanh(v / sec.p);
-    return v;
+// N neighbouring columns of one section, whose kind of activation is a scalar: one chain of branches for all of them (one for each number made squared
+// ReLUs cost a launch of 4096 × 6144 × 2048 21 µs of 115, now 3)
+template <typename E, bool RARE, int N, typename V>
+__device__ __forceinline__ void gemm_act(const GemmSection& sec, int act, V& v) {
+#define EACH(...)                            \
+    do {                                     \
+        _Pragma("unroll") for (int e = 0; e < N; e++) { const float z = v[e]; v[e] = __VA_ARGS__; } \
+        return;                              \
+    } while (0)
+    if (act == GEMM_ACT_NONE) return;
+    if (act == GEMM_ACT_SIGMOID) EACH(ActMath<E>::sigmoid(z));
+    if (act == GEMM_ACT_GELU_TANH) EACH(gelu_tanh_f32<E>(z));
+    if (act == GEMM_ACT_XIELU) EACH(xielu_f32<E>(z, sec.p, sec.q));
+    if (act == GEMM_ACT_RELU2) EACH(fmaxf(z, 0.f) * fmaxf(z, 0.f));
+    if (act == GEMM_ACT_SILU) EACH(z * ActMath<E>::sigmoid(z));
+    if (RARE && act == GEMM_ACT_SOFTPLUS) EACH(softplus_f32<E>(z));
+    if (RARE && act == GEMM_ACT_LOG_SIGMOID) EACH(sec.p * log_sigmoid_f32<E>(z));
+    if (RARE && act == GEMM_ACT_SOFTCAP) EACH(sec.p * ActMath<E>::tanh(z / sec.p));
+#undef EACH
 }
 // output row of place r, −1: none
 template <typename E>
@@ -35,11 +43,18 @@ __device__ __forceinline__ void gemm_store(const TiledGemm<E>& p, int g, int row
     const long o = row * p.ldo + (p.rows.id ? 0 : g * p.out_group) + col;
     if (p.out_f32) p.out_f32[o] = v; else p.out[o] = (E)v;
 }
-template <typename E>
-__device__ __forceinline__ float gemm_glu(const GemmSection& sec, float gate, float up) {
-    if (sec.act == GEMM_ACT_SILU_GLU) return gate * ActMath<E>::sigmoid(gate) * up;
-    if (sec.act == GEMM_ACT_GELU_GLU) return gelu_tanh_f32<E>(gate) * up;
-    return clamped_glu_f32<E>(gate, up, sec.p, sec.q);
+template <typename E, int N, typename V>
+__device__ __forceinline__ void gemm_glu(const GemmSection& sec, int act, V& gate, const V& up) {
+    if (act == GEMM_ACT_SILU_GLU) {
+#pragma unroll
+        for (int e = 0; e < N; e++) gate[e] = gate[e] * ActMath<E>::sigmoid(gate[e]) * up[e];
+    } else if (act == GEMM_ACT_GELU_GLU) {
+#pragma unroll
+        for (int e = 0; e < N; e++) gate[e] = gelu_tanh_f32<E>(gate[e]) * up[e];
+    } else {
+#pragma unroll
+        for (int e = 0; e < N; e++) gate[e] = clamped_glu_f32<E>(gate[e], up[e], sec.p, sec.q);
+    }
 }
 __device__ __forceinline__ int gemm_gated_col(const GemmSection& sec, int col) { return sec.begin + ((col - sec.begin) >> 5) * 16 + (col & 15); }
 template <typename E>
@@ -243,13 +258,9 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(FewRows f, TiledGemm<E>
         if (row >= p.m) row = -1;
         if (gated) {
             const floatx4 up = summed(t + J - 1) * sec.mul + bias[J - 1];
-#pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = gemm_glu<E>(sec, v[r], up[r]);
+            gemm_glu<E, 4>(sec, sec.act, v, up);
             col = gemm_gated_col(sec, col);
-        } else if (sec.act != GEMM_ACT_NONE) {
-#pragma unroll
-            for (int r = 0; r < 4; r++) v[r] = gemm_act<E, EXT>(sec, v[r]);
-        }
+        } else gemm_act<E, EXT, 4>(sec, sec.act, v);
         if (row < 0) continue;
         if (!vec) {
 #pragma unroll 1
@@ -423,7 +434,7 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     // gated section the lanes of the up tiles have nothing to do, those of the gate tiles read both.
     __syncthreads();
     // Where the whole launch is one gated section, a row takes half as many lanes, none of them idle: an
-    // expert model's up-projections 286 → 272 µs a launch, 2048 rows of a 0.6B model's gate_up 48 → 41.
+    // expert model's up-projections 286 → 272 µs a launch.
     constexpr int LD = 16 * NJ + 4;
     float* lf = reinterpret_cast<float*>(smem) + wave * 32 * LD;
     const bool pairs = p.nsec == 1 && p.sec[0].begin == 0 && gemm_gated_act(p.sec[0].act);
@@ -433,59 +444,117 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     const bool gated = gemm_gated_act(sec.act), vec = p.n_store % 8 == 0 && p.ldo % 8 == 0 && p.out_group % 8 == 0 && ((uintptr_t)p.out & 15) == 0 && ((uintptr_t)p.out_f32 & 15) == 0;
     const bool active = gated ? col < p.n && !(col & 16) : col < p.n_store;
     const int oc = gated ? gemm_gated_col(sec, col) : col;
-    float bias[8], bias_up[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        bias[e] = p.bias && active ? p.bias[(long)g * p.n + col + e] : 0.f;
-        bias_up[e] = p.bias && active && gated ? p.bias[(long)g * p.n + col + 16 + e] : 0.f;
+    floatx8 bias = {}, bias_up = {};
+    if (p.bias && active) {
+        bias = *reinterpret_cast<const floatx8*>(p.bias + (long)g * p.n + col);
+        if (gated) bias_up = *reinterpret_cast<const floatx8*>(p.bias + (long)g * p.n + col + 16);
     }
-#pragma unroll
+    // (here and not at the first use in a loop: there the wait would be for the stores of the round before, too)
+    asm volatile("" : "+v"(bias), "+v"(bias_up));
+    // the output row of a wave's row (one a lane), −1: none; rows' ids in memory would be a wait for every round
+    const int own_row = gemm_out_row(p, m0 + wm * MI * 16 + (lane & (16 * MI - 1)));
+    // A wave's columns are of one kind unless a section begins within them: then the kind is a scalar, chosen ahead of the rounds, and a round is
+    // without branches.  With a chain of them for each of the 8 numbers, ids from memory and waits for stores a tile of 128 × 256 took 8 – 9 µs from its
+    // last product to its last store, as long as half of a K of 1024; now 4 – 5, of which 0.6 are the stores' (µs of a launch, plain | bias and sigmoid
+    // | SiLU-gated: 4096 × 6144 × 2048 96 | 121 | 99 → 93 | 95 | 91, 2048 × 6144 × 1024 38 | 53 | 42 → 35 | 37 | 34).  Stores from the registers, without LDS
+    // but 64 bytes of a row at a time: 8192 × 16384 × 2048 536 µs, and 474 this way.
+    const int act = __builtin_amdgcn_readfirstlane(sec.act);
+    const bool one_kind = vec && __all(sec.act == act) && !p.row_scale && !p.col_scale;
+    const long base = (p.rows.id ? 0 : g * p.out_group) + oc;
+    const uint32_t ldo = (uint32_t)p.ldo;
+    const int round_rows = 32 / rounds;
+    const float* from = lf + row_in * LD + cl;
+#pragma unroll 1
     for (int ch = 0; ch < MI / 2; ch++) {
 #pragma unroll
-        for (int i = 0; i < 2; i++)
+        for (int c = 0; c < MI / 2; c++)
+            if (c == ch)
 #pragma unroll
-            for (int j = 0; j < NJ; j++) *reinterpret_cast<floatx4*>(lf + (i * 16 + b) * LD + j * 16 + 4 * a) = acc[2 * ch + i][j];
-        const int row0 = m0 + (wm * MI + 2 * ch) * 16;
+                for (int i = 0; i < 2; i++)
+#pragma unroll
+                    for (int j = 0; j < NJ; j++) *reinterpret_cast<floatx4*>(lf + (i * 16 + b) * LD + j * 16 + 4 * a) = acc[2 * c + i][j];
+        auto round = [&](auto glu, auto f32, auto finish) {
+            constexpr bool GLU = decltype(glu)::value, F32_OUT = decltype(f32)::value;
+            floatx4 next[GLU ? 4 : 2];
+            int next_row;
+            auto fetch = [&](int q) {
+                const floatx4* at = reinterpret_cast<const floatx4*>(from + q * round_rows * LD);
+                next[0] = at[0]; next[1] = at[1];
+                if constexpr (GLU) { next[2] = at[4]; next[3] = at[5]; }
+                next_row = __shfl(own_row, 32 * ch + q * round_rows + row_in);
+            };
+            fetch(0);
 #pragma unroll 1
-        for (int q = 0; q < rounds; q++) {
-            const int row = q * (32 / rounds) + row_in, gr = gemm_out_row(p, row0 + row);
-            if (gr < 0 || !active) continue;
-            float v[8];
+            for (int q = 0; q < rounds; q++) {
+                const int row = next_row;
+                floatx8 v, up;
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[e] = lf[row * LD + cl + e] * sec.mul + bias[e];
-            if (gated) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = gemm_glu<E>(sec, v[e], lf[row * LD + cl + 16 + e] * sec.mul + bias_up[e]);
-            } else if (sec.act != GEMM_ACT_NONE) {
-#pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = gemm_act<E, true>(sec, v[e]);
+                for (int e = 0; e < 8; e++) {
+                    v[e] = next[e >> 2][e & 3] * sec.mul + bias[e];
+                    if constexpr (GLU) up[e] = next[2 + (e >> 2)][e & 3] * sec.mul + bias_up[e];
+                }
+                fetch(min(q + 1, rounds - 1));
+                finish(v, up);
+                if (row >= 0 && active) {
+                    const uint64_t o = (uint64_t)(uint32_t)row * ldo + base;
+                    if constexpr (F32_OUT) *reinterpret_cast<floatx8*>(p.out_f32 + o) = v;
+                    else *reinterpret_cast<v8*>(p.out + o) = __builtin_convertvector(v, v8);
+                }
             }
-            if (!vec) {
-                for (int e = 0; e < 8; e++)
-                    if (gated || col + e < p.n_store) gemm_store(p, g, gr, oc + e, v[e]);
-                continue;
-            }
-            if (p.row_scale) {
-                const float f = (float)p.row_scale[gr * p.ld_scale + g];
+        };
+        typedef std::true_type yes;
+        typedef std::false_type no;
+#define KIND(GLU, ACT) round(GLU{}, no{}, [&](floatx8& v, const floatx8& up) { if constexpr (GLU::value) gemm_glu<E, 8>(sec, ACT, v, up); else gemm_act<E, true, 8>(sec, ACT, v); })
+        if (one_kind && p.out_f32 && act == GEMM_ACT_NONE) round(no{}, yes{}, [](floatx8&, const floatx8&) {});
+        else if (one_kind && p.out && act == GEMM_ACT_NONE) KIND(no, GEMM_ACT_NONE);
+        else if (one_kind && p.out && act == GEMM_ACT_SILU_GLU) KIND(yes, GEMM_ACT_SILU_GLU);
+        else if (one_kind && p.out && act == GEMM_ACT_GELU_GLU) KIND(yes, GEMM_ACT_GELU_GLU);
+        else if (one_kind && p.out && act == GEMM_ACT_CLAMPED_GLU) KIND(yes, GEMM_ACT_CLAMPED_GLU);
+        else if (one_kind && p.out && act == GEMM_ACT_SIGMOID) KIND(no, GEMM_ACT_SIGMOID);
+        else if (one_kind && p.out && act == GEMM_ACT_GELU_TANH) KIND(no, GEMM_ACT_GELU_TANH);
+        else if (one_kind && p.out && act == GEMM_ACT_XIELU) KIND(no, GEMM_ACT_XIELU);
+        else if (one_kind && p.out && act == GEMM_ACT_RELU2) KIND(no, GEMM_ACT_RELU2);
+        else if (one_kind && p.out && act == GEMM_ACT_SILU) KIND(no, GEMM_ACT_SILU);
+        else {
+            // several kinds, one after the other, factors, and rows or columns that no 16-byte piece begins at
+#pragma unroll 1
+            for (int q = 0; q < rounds; q++) {
+                const int row = __shfl(own_row, 32 * ch + q * round_rows + row_in);
+                const floatx4* at = reinterpret_cast<const floatx4*>(from + q * round_rows * LD);
+                floatx8 v, up = {};
 #pragma unroll
-                for (int e = 0; e < 8; e++) v[e] *= f;
-            }
-            if (p.col_scale) {
-                const v8 f = *reinterpret_cast<const v8*>(p.col_scale + p.col_scale_row[gr] * p.ld_col_scale + oc);
+                for (int e = 0; e < 8; e++) v[e] = at[e >> 2][e & 3] * sec.mul + bias[e];
+                if (gated)
 #pragma unroll
-                for (int e = 0; e < 8; e++) v[e] *= (float)f[e];
-            }
-            const long o = gr * p.ldo + (p.rows.id ? 0 : g * p.out_group) + oc;
-            if (p.out_f32) {
-                *reinterpret_cast<floatx4*>(p.out_f32 + o) = (floatx4){v[0], v[1], v[2], v[3]};
-                *reinterpret_cast<floatx4*>(p.out_f32 + o + 4) = (floatx4){v[4], v[5], v[6], v[7]};
-            } else {
-                v8 y;
+                    for (int e = 0; e < 8; e++) up[e] = at[4 + (e >> 2)][e & 3] * sec.mul + bias_up[e];
+                for (uint64_t todo = __ballot(true); todo;) {
+                    const int kind = __builtin_amdgcn_readlane(sec.act, __builtin_ctzll(todo));
+                    const bool mine = sec.act == kind;
+                    if (mine) {
+                        if (gemm_gated_act(kind)) gemm_glu<E, 8>(sec, kind, v, up);
+                        else gemm_act<E, true, 8>(sec, kind, v);
+                    }
+                    todo &= ~__ballot(mine);
+                }
+                if (row < 0 || !active) continue;
+                if (!vec) {
 #pragma unroll
-                for (int e = 0; e < 8; e++) y[e] = (E)v[e];
-                *reinterpret_cast<v8*>(p.out + o) = y;
+                    for (int e = 0; e < 8; e++)
+                        if (gated || col + e < p.n_store) gemm_store(p, g, row, oc + e, v[e]);
+                    continue;
+                }
+                if (p.row_scale) v *= (float)p.row_scale[row * p.ld_scale + g];
+                if (p.col_scale) {
+                    const v8 f = *reinterpret_cast<const v8*>(p.col_scale + p.col_scale_row[row] * p.ld_col_scale + oc);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) v[e] *= (float)f[e];
+                }
+                const uint64_t o = (uint64_t)(uint32_t)row * ldo + base;
+                if (p.out_f32) *reinterpret_cast<floatx8*>(p.out_f32 + o) = v;
+                else *reinterpret_cast<v8*>(p.out + o) = __builtin_convertvector(v, v8);
             }
         }
+#undef KIND
     }
 }
 
