@@ -451,8 +451,6 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     }
     // (here and not at the first use in a loop: there the wait would be for the stores of the round before, too)
     asm volatile("" : "+v"(bias), "+v"(bias_up));
-    // the output row of a wave's row (one a lane), −1: none; rows' ids in memory would be a wait for every round
-    const int own_row = gemm_out_row(p, m0 + wm * MI * 16 + (lane & (16 * MI - 1)));
     // A wave's columns are of one kind unless a section begins within them: then the kind is a scalar, chosen ahead of the rounds, and a round is
     // without branches.  With a chain of them for each of the 8 numbers, ids from memory and waits for stores a tile of 128 × 256 took 8 – 9 µs from its
     // last product to its last store, as long as half of a K of 1024; now 4 – 5, of which 0.6 are the stores' (µs of a launch, plain | bias and sigmoid
@@ -466,6 +464,8 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     const float* from = lf + row_in * LD + cl;
 #pragma unroll 1
     for (int ch = 0; ch < MI / 2; ch++) {
+        // the output rows of these, one a lane, −1: none; ids in memory would be a wait for every round
+        const int own_row = gemm_out_row(p, m0 + (wm * MI + 2 * ch) * 16 + (lane & 31));
 #pragma unroll
         for (int c = 0; c < MI / 2; c++)
             if (c == ch)
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
                 const floatx4* at = reinterpret_cast<const floatx4*>(from + q * round_rows * LD);
                 next[0] = at[0]; next[1] = at[1];
                 if constexpr (GLU) { next[2] = at[4]; next[3] = at[5]; }
-                next_row = __shfl(own_row, 32 * ch + q * round_rows + row_in);
+                next_row = __shfl(own_row, q * round_rows + row_in);
             };
             fetch(0);
 #pragma unroll 1
@@ -519,7 +519,7 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
             // several kinds, one after the other, factors, and rows or columns that no 16-byte piece begins at
 #pragma unroll 1
             for (int q = 0; q < rounds; q++) {
-                const int row = __shfl(own_row, 32 * ch + q * round_rows + row_in);
+                const int row = __shfl(own_row, q * round_rows + row_in);
                 const floatx4* at = reinterpret_cast<const floatx4*>(from + q * round_rows * LD);
                 floatx8 v, up = {};
 #pragma unroll

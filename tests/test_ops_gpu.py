@@ -283,6 +283,29 @@ def test_dense_gemm(env, m, n, k, f32out):
     assert nmse(ref, host(out2)) < (1e-10 if f32out else NMSE_FP16_TOL)
 
 
+@pytest.mark.parametrize("shift", [0, 1, 4])
+@pytest.mark.parametrize("n", [328, 640])
+@pytest.mark.parametrize("mt", [6, 8, 16])
+def test_prefill_tiles_at_any_address(env, mt, n, shift, knobs, forms):
+    """Rows and results that begin at a 16-byte piece and not, columns that end within a wave's 64, a last tile of few rows: the same numbers, and nothing beside them."""
+    pkg, B, ctx, O, torch = env
+    k, m = 256, 16 * mt + 5
+    qw, sc, qz = O.make_synthetic_gptq(k, n, 128, 3, symmetric=False)
+    sc = f16r(sc / (0.28 * np.sqrt(k)))
+    lin = pkg.GptqLinear.from_raw(qw, sc, qz, None, None, 4, 128, k, n)
+    knobs.set(W4_BIG=mt)
+    x = f16r(np.random.default_rng(m).standard_normal((m, k)))
+    src, buf = (torch.full((rows * cols + 16,), 7.0, dtype=torch.float16, device="cuda") for rows, cols in ((m, k), (m, n)))
+    src[shift:shift + m * k] = dev16(torch, x).reshape(-1)
+    forms.reset()
+    lin.forward(ctx, src[shift:shift + m * k], buf[shift:shift + m * n], m)
+    ctx.sync()
+    forms.require("w4_big")
+    got = host(buf)
+    assert nmse(O.gemm(x, O.dequant_gptq(qw, sc, qz, 128, k, n), m, n, k), got[shift:shift + m * n].reshape(m, n)) < NMSE_FP16_TOL
+    assert np.all(got[:shift] == 7.0) and np.all(got[shift + m * n:] == 7.0)
+
+
 @pytest.mark.parametrize("f32out", [False, True])
 @pytest.mark.parametrize("m,n,k", [(1, 64, 32), (16, 4096, 1024), (17, 96, 1056), (64, 1024, 3072), (65, 8192, 32), (100, 6176, 96), (200, 2080, 64),
                                    (129, 16416, 160), (300, 4128, 2080), (1100, 1056, 352), (2049, 4096, 128), (3000, 8224, 64), (9, 14400, 2080), (16, 16416, 4128),
