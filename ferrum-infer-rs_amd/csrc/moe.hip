@@ -12,6 +12,32 @@
 
 namespace fh {
 
+// One expert a lane (64 at most), top_k of them by their place among all rather than one after the other: a maximum over the wave costs as much as
+// ten comparisons with a lane's value.  (A launch of 32 tokens, two a wave, on 24 experts in 8 groups of 3, top 8: 19 → 11 µs, of which
+// 7.4 the choice; two tokens on 30, one group: 7.7 → 6.1; bound by the instructions of 16 waves on one CU, with few tokens by their latency.)
+// place: how many of the first `n` lanes hold a larger v, the lower lane first on ties; −∞ and NaN are behind all and have no place (≥ 64)
+__device__ __forceinline__ int route_place(float v, int lane, int n) {
+    const bool in = v > -INFINITY;
+    if (!in) v = -INFINITY;
+    int place = 0;
+    for (int l0 = 0; l0 < n; l0 += 8)                   // (lanes past the n-th hold −∞)
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int l = l0 + j;
+            const float x = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), l));
+            place += x > v || (x == v && l < lane);
+        }
+    return in ? place : 64;
+}
+__device__ __forceinline__ bool route_by_place(int per_lane, int num_experts, int top_k) { return per_lane == 1 && num_experts <= 8 * top_k; }
+// lane k < top_k: what the lane of place k has, `none` where no lane has it
+template <typename T>
+__device__ __forceinline__ T route_at_place(T x, int place, int lane, int top_k, T none) {
+    static_assert(sizeof(T) == 4, "");
+    const int got = __builtin_amdgcn_ds_permute((place < top_k ? place : 63) << 2, __builtin_bit_cast(int, x));
+    const int places = __popcll(__ballot(place < top_k));
+    return lane < places ? __builtin_bit_cast(T, got) : none;
+}
 // Router of one token on one wave (E ≤ 64·PER, lane l looks at experts l, l + 64, …): f32 softmax, k argmax-mask passes, ties → lowest
 // index.  Lane k ends up with the k-th choice.
 template <int PER, typename T>
@@ -42,6 +68,12 @@ __device__ __forceinline__ void route_token(const T* __restrict__ row, int lane,
     float sel_sum = 0.f;
     weight = 0.f;
     id = 0;
+    if (route_by_place(PER, num_experts, top_k)) {
+        const int place = route_place(v[0], lane, num_experts);
+        id = route_at_place(lane, place, lane, top_k, 0);
+        weight = route_at_place(v[0], place, lane, top_k, -INFINITY);
+        for (int k = 0; k < top_k; k++) sel_sum += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), k));
+    } else
     for (int k = 0; k < top_k; k++) {
         float best = -INFINITY;
         int mine = 1 << 20;
@@ -114,6 +146,27 @@ __device__ __forceinline__ void route_drop_groups(float (&v)[PER], const int (&g
             if (place[i] >= rule.keep) v[i] = -INFINITY;
         return;
     }
+    if constexpr (PER == 1) {
+        // every lane its own group's two largest, from the group's lanes, and its place among the others'
+        const float x = v[0] > -INFINITY ? v[0] : -INFINITY;
+        float m1 = -INFINITY, m2 = -INFINITY;
+        for (int j = 0; j < per_group; j++) {
+            const float o = __shfl(x, grp[0] * per_group + j, 64);
+            m2 = fmaxf(m2, fminf(m1, o));
+            m1 = fmaxf(m1, o);
+        }
+        float sum = per_group > 1 ? m1 + m2 : m1;
+        if (!(sum > -INFINITY)) sum = -INFINITY;
+        int place = 0, real = 0;
+        for (int g = 0; g < rule.groups; g++) {
+            const float o = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sum), g * per_group));
+            place += o > sum || (o == sum && g < grp[0]);
+            real += o > -INFINITY;
+        }
+        // (groups without a value are not chosen; in place of those missing, the first)
+        if (!((sum > -INFINITY && place < rule.keep) || (real < rule.keep && grp[0] == 0))) v[0] = -INFINITY;
+        return;
+    }
     float mine = -INFINITY, top;                     // lane g: group g's
     for (int g = 0; g < rule.groups; g++) {
         float w[PER], second = 0.f;
@@ -173,6 +226,12 @@ __device__ __forceinline__ void route_token_corrected(const float* __restrict__ 
     float sum = 0.f;
     weight = 0.f;
     id = 0;
+    if (route_by_place(PER, num_experts, top_k)) {
+        const int place = route_place(v[0], lane, num_experts);
+        id = route_at_place(lane, place, lane, top_k, 0);
+        weight = route_at_place(s[0], place, lane, top_k, __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s[0]), 0)));
+        for (int k = 0; k < top_k; k++) sum += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), k));
+    } else
     for (int k = 0; k < top_k; k++) {
         const int e = max(route_best<PER>(v, top), 0);
         float score = 0.f;
@@ -252,14 +311,13 @@ __global__ __launch_bounds__(1024) void moe_route_sort_kernel(const float* __res
     if (CORRECTED) num_experts -= rule.unlisted;               // (the sorted list's)
     int e = tid < n_pairs ? lds_id[tid] : -1;
     if (e >= num_experts) e = -1;
-    int rank = 0, same = 0;
-    if (wave < nw)
-#pragma unroll
-        for (int l = 0; l < 64; l++) {
-            const int other = __builtin_amdgcn_readlane(e, l);
-            same += other == e;
-            rank += other == e && l < lane;
-        }
+    // the lanes with the same expert, bit by bit of its number
+    unsigned long long alike = ~0ull;
+    for (int bit = 0; (1 << bit) <= num_experts; bit++) {          // (as far as −1 differs from every number)
+        const unsigned long long set = __ballot(e >> bit & 1);
+        alike &= e >> bit & 1 ? set : ~set;
+    }
+    const int rank = __popcll(alike & ((1ull << lane) - 1)), same = __popcll(alike);
     if (e >= 0 && rank == 0) hist[wave][e] = (int16_t)same;
     __syncthreads();
     // counts of earlier waves per expert, and the padded start of every expert's rows

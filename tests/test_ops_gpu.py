@@ -1122,6 +1122,42 @@ def test_route_ties_lowest_index(env):
     assert np.all(np.abs(w.cpu().numpy() - 0.125) < 1e-7)
 
 
+@pytest.mark.parametrize("norm", [False, True])
+@pytest.mark.parametrize("ne,k", [(1, 1), (2, 1), (7, 7), (8, 2), (9, 1), (24, 8), (31, 4), (40, 5), (41, 5), (63, 8), (64, 8), (64, 64), (65, 8)])
+def test_route_by_place_and_by_maxima(env, ne, k, norm):
+    """Up to eight experts a choice are ranked at once, more by one maximum after the other: numbers, ties, -inf and NaN among the logits, against k passes of a maximum in
+    which a NaN takes no part, the first expert standing in where none is left."""
+    pkg, B, ctx, O, torch = env
+    rng = np.random.default_rng(ne * 64 + k)
+    logits = rng.standard_normal((8, ne)).astype(np.float32)
+    logits[1] = 0.25
+    logits[2, ::2] = 1.5
+    logits[3] = np.round(logits[3])
+    logits[4, ne // 2:] = -np.inf
+    logits[5, 1:] = -200.0
+    logits[6, ne - 1] = np.nan
+    logits[7] = -np.inf
+    ids, w = torch.empty(8, k, dtype=torch.int32, device="cuda"), torch.empty(8, k, dtype=torch.float32, device="cuda")
+    B.route_topk_softmax(ctx, torch.from_numpy(logits).cuda(), ids, w, 8, ne, k, norm)
+    ctx.sync()
+    with np.errstate(all="ignore"):
+        p = np.exp(logits - np.fmax.reduce(logits, axis=1, keepdims=True)).astype(np.float32)
+        p /= p.sum(1, keepdims=True)
+        for r in range(8):
+            v, want, ww = p[r].copy(), [], []
+            for _ in range(k):
+                ok = np.where(v > -np.inf, v, -np.inf)
+                e = int(np.argmax(ok)) if np.any(v > -np.inf) else 0
+                want.append(e)
+                ww.append(ok[e])
+                v[e] = -np.inf
+            total = np.float32(sum(ww))
+            ww = (np.array(ww) / total if total > 0 else np.full(k, 1.0 / k)) if norm else np.array(ww)
+            assert ids[r].tolist() == want, (r, ids[r].tolist(), want)
+            got = w[r].cpu().numpy()
+            assert np.all((np.abs(got - ww) < 1e-6) | (got == ww)), (r, got, ww)
+
+
 @pytest.mark.parametrize("tokens,ne,k", [(1, 128, 8), (32, 128, 8), (700, 128, 8), (5, 8, 2), (0, 16, 2)])
 def test_moe_align_block_size_bit_exact(env, tokens, ne, k):
     pkg, B, ctx, O, torch = env
