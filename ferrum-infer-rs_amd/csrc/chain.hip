@@ -147,6 +147,15 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t chain_rsrc(const void* base, l
 __device__ __forceinline__ half8 load16_sc1(__amdgpu_buffer_rsrc_t r, int byte_off) {
     return __builtin_bit_cast(half8, __builtin_amdgcn_raw_buffer_load_b128(r, byte_off, 0, 16));      // aux 16 = sc1
 }
+// at most N of the wave's loads and stores are still under way
+template <int N>
+__device__ __forceinline__ void chain_landed() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt((N & 15) | 0xF70 | (N >> 4) << 14);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
 __device__ __forceinline__ void store16_sc1(__amdgpu_buffer_rsrc_t r, int byte_off, half8 v) {
     __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, byte_off, 0, 16);
 }
@@ -158,9 +167,15 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
     const int H = p.H, nvec = H >> 3, top_k = p.top_k;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     constexpr int CH = 2;                        // H ≤ 8192 with 512 threads
-    half8 v[CH];
+    half8 v[CH], ln[CH];
     float ss = 0.f;
     const __amdgpu_buffer_rsrc_t r_res = chain_rsrc(p.res_a, (long)p.T * H * 2), r_n1 = chain_rsrc(p.norm1, (long)p.T * H * 2);
+    // (the norm's weights are on their way with the rows, and no store of the residual row lies ahead of a wait: loads and stores retire in order)
+#pragma unroll
+    for (int c = 0; c < CH; c++) {
+        const int i = threadIdx.x + c * 512;
+        ln[c] = *reinterpret_cast<const half8*>(p.ln_in + (i < nvec ? i : 0) * 8);
+    }
 #pragma unroll
     for (int c = 0; c < CH; c++) {
         const int i = threadIdx.x + c * 512;
@@ -170,7 +185,6 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
             half8 rv = *reinterpret_cast<const half8*>(p.res_in + (long)row * H + i * 8);
 #pragma unroll
             for (int j = 0; j < 8; j++) rv[j] = (_Float16)((float)rv[j] + (float)xv[j]);
-            store16_sc1(r_res, (int)(((long)row * H + i * 8) * 2), rv);
             v[c] = rv;
 #pragma unroll
             for (int j = 0; j < 8; j++) ss += (float)rv[j] * (float)rv[j];
@@ -182,7 +196,6 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
             half8 rv = *reinterpret_cast<const half8*>(p.res_in + (long)row * H + i * 8);
 #pragma unroll
             for (int j = 0; j < 8; j++) rv[j] = (_Float16)((float)rv[j] + (float)(_Float16)o[j]);
-            store16_sc1(r_res, (int)(((long)row * H + i * 8) * 2), rv);
             v[c] = rv;
 #pragma unroll
             for (int j = 0; j < 8; j++) ss += (float)rv[j] * (float)rv[j];
@@ -212,7 +225,6 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
             }
 #pragma unroll
             for (int j = 0; j < 8; j++) rv[j] = (_Float16)((float)rv[j] + acc[j]);
-            store16_sc1(r_res, (int)(((long)row * H + i * 8) * 2), rv);
             v[c] = rv;
 #pragma unroll
             for (int j = 0; j < 8; j++) ss += (float)rv[j] * (float)rv[j];
@@ -230,10 +242,10 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
     for (int c = 0; c < CH; c++) {
         const int i = threadIdx.x + c * 512;
         if (i < nvec) {
-            const half8 wv = *reinterpret_cast<const half8*>(p.ln_in + i * 8);
             half8 o;
 #pragma unroll
-            for (int j = 0; j < 8; j++) o[j] = (_Float16)((float)v[c][j] * inv * (float)wv[j]);
+            for (int j = 0; j < 8; j++) o[j] = (_Float16)((float)v[c][j] * inv * (float)ln[c][j]);
+            store16_sc1(r_res, (int)(((long)row * H + i * 8) * 2), v[c]);
             store16_sc1(r_n1, (int)(((long)row * H + i * 8) * 2), o);
         }
     }
@@ -243,10 +255,13 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
 }
 
 // ── GEMM roles (q|k|v and o_proj): one 16-row block × NST 64-column supertiles per workgroup, K split over its 8 waves ───
-// All GPW quant groups of a wave's K slice are requested before the wait; the activations follow the wait (sc1), two groups
-// in flight; the 8 partial sums meet in LDS (summed in wave order) and leave as 16-byte write-through stores.  A workgroup
-// reads rows × K activation bytes after its wait, at the ≈ 70 GB/s a workgroup gets for handed-off bytes — so the rows are
-// split over workgroups (16 each) rather than the columns made narrower (32 rows × 4096: 8.0 µs behind the wait).
+// All GPW quant groups of a wave's K slice are requested before the wait, and as many of them as registers hold become numbers there; the
+// rows follow the wait (sc1), all at once and in whole lines, into the wave's region of LDS; the 8 partial sums meet in LDS (summed in wave
+// order) and leave as 16-byte write-through stores.  A workgroup reads rows × K activation bytes after its wait, at the ≈ 70 GB/s a
+// workgroup gets for handed-off bytes — so the rows are split over workgroups (16 each) rather than the columns made narrower.
+// Behind the wait of 12 rows of 4096, 64 columns: 0.9 µs until the rows are there, 1.0 the products, 0.8 the slowest wave's and the meeting, 0.5
+// the result (64-byte pieces of 16 rows, two groups ahead, weights expanded behind the wait: 4.1 in all, now 3.2; 16 rows of 2048 in
+// 128 columns 4.2 → 3.3, o_proj's halves of K 2.7 → 2.0).
 struct ChainEdge { unsigned* base; int shards, reps; unsigned total; };      // base == nullptr: nothing to wait for
 
 // NTL = 16-column tiles of the 64-column supertile a workgroup takes (NST = 1): 4, or 2 — a 32-column block `cb` = supertile cb / 2,
@@ -260,8 +275,8 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
                                                 unsigned* timeout, unsigned char* smem, const ChainArgs& p, int g_base = 0, float* out32 = nullptr) {
     static_assert(NTL == 4 || (NTL == 2 && NST == 1), "half supertiles only for single-supertile blocks");
     constexpr int V = NST * NTL * 4, CPR = NST * NTL * 2;                       // accumulator floats per lane; 16-byte chunks per output row
-    float* red = reinterpret_cast<float*>(smem);                     // [8][V][64]
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    float* red = reinterpret_cast<float*>(smem);                     // [8 regions of a wave][V][64]
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
     CH_TL(0);
     const int g0 = g_base + wave * GPW;                               // G = 8·GPW (· 2 with F32OUT; checked by the launcher)
@@ -279,36 +294,82 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
             scv[i][s] = (reinterpret_cast<const uint2*>(w.sc) + (st * w.G) * 16 + b)[(long)(g0 + i) * 16];
             if (HAS_ZP) zpv[i][s] = (reinterpret_cast<const uint2*>(w.zp) + (st * w.G) * 16 + b)[(long)(g0 + i) * 16];
         }
+    // the first PRE groups' weights become numbers (q − 8) while the predecessor works: their expansion, and the products that take the
+    // offset of in-place nibbles back, are not behind the wait
+    constexpr int FIT = 8 / (NST * NTL), PRE = HAS_ZP ? 0 : (GPW < FIT ? GPW : FIT);       // (128 registers)
+    half8 wx[PRE ? PRE : 1][NST][NTL][4];
+    if constexpr (PRE > 0) {
+        const uint32_t magic = opaque_vgpr(0x64006400u), magic_hi = opaque_vgpr(0x54005400u);
+        const uint32_t m_lo = opaque_sgpr(0x000F000Fu), m_hi = opaque_sgpr(0x00F000F0u);
+#pragma unroll
+        for (int i = 0; i < PRE; i++)
+#pragma unroll
+            for (int s = 0; s < NST; s++)
+#pragma unroll
+                for (int nt = 0; nt < NTL; nt++)
+#pragma unroll
+                    for (int pr = 0; pr < 2; pr++) {
+                        const uint32_t d0 = wq[i][s][nt][2 * pr], d1 = wq[i][s][nt][2 * pr + 1], d0s = d0 >> 8, d1s = d1 >> 8;
+                        half8 lo = pack_half8(and_or(d0, m_lo, magic), and_or(d0s, m_lo, magic), and_or(d1, m_lo, magic), and_or(d1s, m_lo, magic));
+                        half8 hi = pack_half8(and_or(d0, m_hi, magic_hi), and_or(d0s, m_hi, magic_hi), and_or(d1, m_hi, magic_hi), and_or(d1s, m_hi, magic_hi));
+                        lo -= splat_half8(1032.0f);
+                        hi -= splat_half8(72.0f);
+                        asm volatile("" : "+v"(lo), "+v"(hi));            // (here, not at the use)
+                        wx[i][s][nt][2 * pr] = lo;
+                        wx[i][s][nt][2 * pr + 1] = hi;
+                    }
+    }
     __builtin_amdgcn_sched_barrier(0);
     if (wait.base) chain_wait(wait.base, wait.shards, wait.reps, wait.total, timeout);
     CH_TL(1);
     const __amdgpu_buffer_rsrc_t r_x = chain_rsrc(x_in, (long)T * w.K * 2);
-    const int r_in = rb * 16 + b;
-    const int xoff = ((r_in < T ? r_in : T - 1) * w.K + 8 * a) * 2;
-    half8 af[2][1][4];
-    auto issue_a = [&](int buf, int g) {
+    constexpr int REGION = GPW * 4096;                                // a wave's rows: [group][16 rows][16 pieces of 16 bytes, piece xor row]
+    static_assert(V * 256 <= REGION, "a wave's partial sums take its rows' place");
+    unsigned char* const mine = smem + wave * REGION;
+    chain_landed<0>();                                                // the weights: from here on only row copies are counted
 #pragma unroll
-        for (int s = 0; s < 4; s++) af[buf][0][s] = load16_sc1(r_x, xoff + (g * 128 + 32 * s) * 2);
-    };
+    for (int i = 0; i < GPW; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int r = 4 * q + a;                                  // (rows past the last lie outside of the buffer: zeros, and no traffic)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r_x, (__attribute__((address_space(3))) void*)(mine + (i * 4 + q) * 1024), 16,
+                                                     ((rb * 16 + r) * w.K + (b ^ r) * 8) * 2, (g0 + i) * 256, 0, 16);
+        }
     float4v acc[NST][1][NTL];
 #pragma unroll
     for (int s = 0; s < NST; s++)
 #pragma unroll
         for (int nt = 0; nt < NTL; nt++) acc[s][0][nt] = (float4v){0.f, 0.f, 0.f, 0.f};
-    issue_a(0, g0);
-    if (GPW > 1) issue_a(1, g0 + 1);
-    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < GPW; i++) {
+        if (i == GPW - 1) chain_landed<0>();
+        else if (i == GPW - 2) chain_landed<4>();
+        else if (i == GPW - 3) chain_landed<8>();
+        else chain_landed<12>();
+        half8 af[1][4];
+#pragma unroll
+        for (int s = 0; s < 4; s++) af[0][s] = *reinterpret_cast<const half8*>(mine + i * 4096 + b * 256 + ((4 * s + a) ^ b) * 16);
 #pragma unroll
         for (int s = 0; s < NST; s++) {
             const unsigned long long sb = ((unsigned long long)scv[i][s].y << 32) | scv[i][s].x;
             const unsigned long long zb = HAS_ZP ? (((unsigned long long)zpv[i][s].y << 32) | zpv[i][s].x) : 0ull;
-            w4_consume_group<1, NTL, HAS_ZP, false>(wq[i][s], sb, zb, nt0, af[i & 1], acc[s]);
+            if (i < PRE) {
+                float4v t[NTL];
+#pragma unroll
+                for (int nt = 0; nt < NTL; nt++) t[nt] = (float4v){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+#pragma unroll
+                    for (int nt = 0; nt < NTL; nt++) t[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[0][k], wx[i < PRE ? i : 0][s][nt][k], t[nt], 0, 0, 0);
+#pragma unroll
+                for (int nt = 0; nt < NTL; nt++) {
+                    const float s_f = (float)__builtin_bit_cast(_Float16, (uint16_t)(sb >> 16 * (nt0 + nt)));
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[s][0][nt][r] = __builtin_fmaf(s_f, t[nt][r], acc[s][0][nt][r]);
+                }
+            } else
+                w4_consume_group<1, NTL, HAS_ZP, false>(wq[i][s], sb, zb, nt0, af, acc[s]);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        if (i + 2 < GPW) issue_a(i & 1, g0 + i + 2);
-        __builtin_amdgcn_sched_barrier(0);
     }
     // cross-wave reduction through LDS: red[wave][v][lane], v = (supertile·4 + tile)·4 + r
 #pragma unroll
@@ -316,7 +377,7 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
 #pragma unroll
         for (int nt = 0; nt < NTL; nt++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) red[((wave * V) + (s * NTL + nt) * 4 + r) * 64 + lane] = acc[s][0][nt][r];
+            for (int r = 0; r < 4; r++) red[wave * (REGION / 4) + ((s * NTL + nt) * 4 + r) * 64 + lane] = acc[s][0][nt][r];
     __syncthreads();
     // thread → (row, 8 consecutive columns): one 16-byte write-through store
     if (threadIdx.x < 16 * CPR) {
@@ -328,8 +389,8 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
         float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ww = 0; ww < CH_W; ww++) {
-            const float4v lo = *reinterpret_cast<const float4v*>(&red[(ww * V + v) * 64 + ln]);
-            const float4v hi = *reinterpret_cast<const float4v*>(&red[(ww * V + v) * 64 + ln + 4]);
+            const float4v lo = *reinterpret_cast<const float4v*>(&red[ww * (REGION / 4) + v * 64 + ln]);
+            const float4v hi = *reinterpret_cast<const float4v*>(&red[ww * (REGION / 4) + v * 64 + ln + 4]);
 #pragma unroll
             for (int j = 0; j < 4; j++) { sum[j] += lo[j]; sum[4 + j] += hi[j]; }
         }
@@ -420,23 +481,24 @@ __device__ __forceinline__ void chain_role_attn(const ChainArgs& p, int wg, unsi
     Frags cur, nxt;
     if (first < my_hi) issue(first, cur);
     const int last_blk = pos0 / KV_BLOCK, slot_new = pos0 % KV_BLOCK;
-    // norm weights and the RoPE row of this position do not depend on the projection either
+    // norm weights, the RoPE row of this position and the new token's block do not depend on the projection either
+    constexpr int HALF = HD / 2;
+    const int r16 = threadIdx.x >> 4, q16 = threadIdx.x & 15;
+    const int rc = r16 < G + 2 ? r16 : G + 1, rope_mode = rc <= G ? p.qk_mode : 0;
+    const RopeCoef<HD> coef = rope_coef16<HD>(rc < G ? p.q_norm_w : p.k_norm_w, p.cos_t + (long)pos0 * HALF, p.sin_t + (long)pos0 * HALF,
+                                              rope_mode, p.qk_mode == 1, p.qk_mode != 0, q16);
+    const int phys_new = bt[last_blk];
     __builtin_amdgcn_sched_barrier(0);
     // the q|k|v columns of this kv head: G + 2 heads, each one workgroup per 16-row block of the projection role
     chain_wait(p.cnt + (CH_QKV_SLOT + kvh * CH_QKV_R) * CH_STRIDE, 1, CH_QKV_R, (unsigned)((G + 2) * (WIDE ? 1 : (p.qkv_half ? 4 : 2)) * ((p.T + 15) >> 4)), p.timeout);
     CH_TL(1);
     half8 qf[KS];
     {
-        constexpr int HALF = HD / 2;
         const int q_dim = p.nq * HD, kv_dim = p.nkv * HD;
         const __half* qrow = p.qkv_out + (long)seq * (q_dim + 2 * kv_dim);
-        const int r16 = threadIdx.x >> 4, q16 = threadIdx.x & 15;
-        const int rc = r16 < G + 2 ? r16 : G + 1;
         const __half* src = rc < G ? qrow + (kvh * G + rc) * HD
                                    : rc == G ? qrow + q_dim + kvh * HD : qrow + q_dim + kv_dim + kvh * HD;
-        const RopeRow<HD> rr = rope_row16<HD, true>(src, rc < G ? p.q_norm_w : p.k_norm_w, p.cos_t + (long)pos0 * HALF,
-                                                    p.sin_t + (long)pos0 * HALF, rc <= G ? p.qk_mode : 0, p.qk_mode == 1,
-                                                    p.qk_mode != 0, p.eps, q16);
+        const RopeRow<HD> rr = rope_row16<HD, true>(src, coef, rope_mode, p.eps, q16);
         using hv = typename RopeRow<HD>::hv;
         hv z0, z1;
 #pragma unroll
@@ -454,16 +516,17 @@ __device__ __forceinline__ void chain_role_attn(const ChainArgs& p, int wg, unsi
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < KS; s++) qf[s] = *reinterpret_cast<const half8*>(lds_q + b * HD + 32 * s + 8 * a);
-        // the new token's K (wave 0) and V (wave 1) go to the cache (read by later launches only)
+    }
+    // the new token's K (wave 0) and V (wave 1) go to the cache, read by later launches only: last of all
+    auto keep_new = [&]() {
         if (wave < 2 && split == NS - 1) {
-            const long phys = p.block_tables[(long)seq * p.max_blocks + last_blk];
-            const long toff = (phys * p.nkv + kvh) * kv_tile_elems(HD);
+            const long toff = ((long)phys_new * p.nkv + kvh) * kv_tile_elems(HD);
             for (int d = lane; d < HD; d += 64) {
                 if (wave == 0) p.k_pool[toff + k_tile_off(slot_new, d)] = lds_kv[d];
                 else p.v_pool[toff + v_tile_off(slot_new, d)] = lds_kv[HD + d];
             }
         }
-    }
+    };
     float m_run = -INFINITY, l_run = 0.f;
     float4v o_acc[DT];
 #pragma unroll
@@ -585,35 +648,40 @@ __device__ __forceinline__ void chain_role_attn(const ChainArgs& p, int wg, unsi
         int* s_tk = reinterpret_cast<int*>(lds_m);                     // (the merge above is done with lds_m)
         if (threadIdx.x == 0) *s_tk = (int)__hip_atomic_fetch_add(p.attn_tickets + unit, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
-        if (*s_tk != NS - 1) { CH_TL(2); CH_TL(3); return; }           // not the last: the merge (and the signal) is someone else's
+        if (*s_tk != NS - 1) { keep_new(); CH_TL(2); CH_TL(3); return; }           // not the last: the merge (and the signal) is someone else's
         if (threadIdx.x == 0) __hip_atomic_store(p.attn_tickets + unit, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (row < G) {
             const int base = (int)(((long)unit * NS * 16 * PST + row * PST) * 4);
-            float ms[CH_MAX_SPLITS], ls[CH_MAX_SPLITS];
-            Mm = -INFINITY;
+            // (no branch around a load: all of them are under way together)
+            auto merge = [&](auto most) {
+                constexpr int N = decltype(most)::value;
+                float4v ml[N], os[N];
 #pragma unroll
-            for (int sp = 0; sp < CH_MAX_SPLITS; sp++) {
-                if (sp < NS) {
-                    const float4v ml = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(pr_, base + sp * 16 * PST * 4 + HD * 4, 0, 16));
-                    ms[sp] = ml[0]; ls[sp] = ml[1];
-                    Mm = fmaxf(Mm, ms[sp]);
+                for (int sp = 0; sp < N; sp++) {
+                    const int at = base + min(sp, NS - 1) * 16 * PST * 4;
+                    ml[sp] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(pr_, at + HD * 4, 0, 16));
+                    os[sp] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(pr_, at + dl * 16, 0, 16));
                 }
-            }
-            const float Msafe = Mm == -INFINITY ? 0.f : Mm;
-            Lm = 0.f;
+                Mm = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < DPT; i++) ov[i] = 0.f;
+                for (int sp = 0; sp < N; sp++) Mm = fmaxf(Mm, ml[sp][0]);          // (repeats of the last range change no maximum)
+                const float Msafe = Mm == -INFINITY ? 0.f : Mm;
+                Lm = 0.f;
 #pragma unroll
-            for (int sp = 0; sp < CH_MAX_SPLITS; sp++) {
-                if (sp < NS) {
-                    const float4v os = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(pr_, base + sp * 16 * PST * 4 + dl * 16, 0, 16));
-                    const float f = __expf(ms[sp] - Msafe);
-                    Lm += ls[sp] * f;
+                for (int i = 0; i < DPT; i++) ov[i] = 0.f;
 #pragma unroll
-                    for (int i = 0; i < DPT; i++) ov[i] += os[i] * f;
+                for (int sp = 0; sp < N; sp++) {
+                    const float f = sp < NS ? __expf(ml[sp][0] - Msafe) : 0.f;
+                    if (sp < NS) {
+                        Lm += ml[sp][1] * f;
+#pragma unroll
+                        for (int i = 0; i < DPT; i++) ov[i] += os[sp][i] * f;
+                    }
                 }
-            }
+            };
+            if (NS <= 8) merge(std::integral_constant<int, 8>{});
+            else merge(std::integral_constant<int, CH_MAX_SPLITS>{});
         }
     }
     if (row < G) {
@@ -626,6 +694,7 @@ __device__ __forceinline__ void chain_role_attn(const ChainArgs& p, int wg, unsi
     }
     CH_TL(2);
     chain_signal(p.cnt + CH_ATTN_SLOT * CH_STRIDE, unit % CH_ATTN_SH, CH_ATTN_R);
+    keep_new();
     CH_TL(3);
 }
 
@@ -722,6 +791,7 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
     if (num_experts <= 0) { CH_TL(2); CH_TL(3); return; }           // dense model: add + norm only (norm2 / res_b_out written above)
     __syncthreads();
     const int a = lane >> 4, b = lane & 15;
+    // (all sixteen rows of a product are the token's: a row of zeros would need a branch at every read)
     for (int u = wave; u < tiles_q * ksplit; u += 8) {
         const int tl = u / ksplit, ks = u % ksplit;
         const int tile = q * tiles_q + tl;
@@ -732,8 +802,7 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
         if (u == wave && pre) {
 #pragma unroll
             for (int kk = 0; kk < U; kk++) {
-                half8 av = {0, 0, 0, 0, 0, 0, 0, 0};
-                if (b == 0) av = *reinterpret_cast<const half8*>(xs + (s + kk) * 32 + 8 * a);
+                const half8 av = *reinterpret_cast<const half8*>(xs + (s + kk) * 32 + 8 * a);
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bw_pre[kk], acc, 0, 0, 0);
             }
             s += U;
@@ -744,15 +813,13 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
             for (int k = 0; k < U; k++) bw[k] = *reinterpret_cast<const half8*>(wrow + (long)(s + k) * 512);
 #pragma unroll
             for (int k = 0; k < U; k++) {
-                half8 av = {0, 0, 0, 0, 0, 0, 0, 0};
-                if (b == 0) av = *reinterpret_cast<const half8*>(xs + (s + k) * 32 + 8 * a);
+                const half8 av = *reinterpret_cast<const half8*>(xs + (s + k) * 32 + 8 * a);
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bw[k], acc, 0, 0, 0);
             }
         }
         for (; s < s1; s++) {
             const half8 bwv = *reinterpret_cast<const half8*>(wrow + (long)s * 512);
-            half8 av = {0, 0, 0, 0, 0, 0, 0, 0};
-            if (b == 0) av = *reinterpret_cast<const half8*>(xs + s * 32 + 8 * a);
+            const half8 av = *reinterpret_cast<const half8*>(xs + s * 32 + 8 * a);
             acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bwv, acc, 0, 0, 0);
         }
         if (a == 0) part[ks * tiles_q * 16 + tl * 16 + b] = acc[0];
@@ -765,28 +832,44 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
     float l = -INFINITY;
     if (t < EQ && e_glob < num_experts) {
         l = 0.f;
-        for (int ks = 0; ks < ksplit; ks++) l += part[ks * EQ + t];
+        float lp[8];
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) lp[ks] = part[(ks < ksplit ? ks : 0) * EQ + t];
+#pragma unroll
+        for (int ks = 0; ks < 8; ks++) if (ks < ksplit) l += lp[ks];
     }
-    if (t < EQ) lgs[t] = l;
-    float mx = wave_reduce_max(l);
-    if (lane == 0) red[wave] = mx;
-    __syncthreads();
-    mx = fmaxf(red[0], red[1]);
-    __syncthreads();
-    const float ex = (t < EQ && e_glob < num_experts) ? expf(l - mx) : 0.f;
-    const float sm = wave_reduce_sum(ex);
-    if (lane == 0) red[wave] = sm;
     const int keep = top_k < EQ ? top_k : EQ;
-    if (t < EQ) {
-        int rank = 0;
-        for (int j = 0; j < EQ; j++) {
-            const float lj = lgs[j];
-            rank += (lj > l || (lj == l && j < t)) ? 1 : 0;
+    float mx = wave_reduce_max(l), sm;
+    int rank = 0;
+    if (EQ <= 64) {
+        // one wave has them all
+        if (wave != 0) return;
+        sm = wave_reduce_sum((t < EQ && e_glob < num_experts) ? expf(l - mx) : 0.f);
+        rank = route_rank(route_key(l, t), EQ);
+        if (t < EQ && rank < keep) cand_s[rank] = ((unsigned long long)(unsigned)e_glob << 32) | __float_as_uint(l);
+        if (t >= keep && t < 8) cand_s[t] = (0x7fffffffull << 32) | __float_as_uint(-INFINITY);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+    } else {
+        if (t < EQ) lgs[t] = l;
+        if (lane == 0) red[wave] = mx;
+        __syncthreads();
+        mx = fmaxf(red[0], red[1]);
+        __syncthreads();
+        const float ex = (t < EQ && e_glob < num_experts) ? expf(l - mx) : 0.f;
+        sm = wave_reduce_sum(ex);
+        if (lane == 0) red[wave] = sm;
+        if (t < EQ) {
+            for (int j = 0; j < EQ; j++) {
+                const float lj = lgs[j];
+                rank += (lj > l || (lj == l && j < t)) ? 1 : 0;
+            }
+            if (rank < keep) cand_s[rank] = ((unsigned long long)(unsigned)e_glob << 32) | __float_as_uint(l);
         }
-        if (rank < keep) cand_s[rank] = ((unsigned long long)(unsigned)e_glob << 32) | __float_as_uint(l);
+        if (t >= keep && t < 8) cand_s[t] = (0x7fffffffull << 32) | __float_as_uint(-INFINITY);
+        __syncthreads();
+        sm = red[0] + red[1];
     }
-    if (t >= keep && t < 8) cand_s[t] = (0x7fffffffull << 32) | __float_as_uint(-INFINITY);
-    __syncthreads();
     CH_TL(2);
     if (wave != 0) return;
     if (p.defer_merge) {
@@ -795,7 +878,7 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
         unsigned long long* cand_g = reinterpret_cast<unsigned long long*>(p.cand) + (row * Q + q) * 8;
         if (lane < 8) cand_g[lane] = cand_s[lane];
         if (lane == 8) reinterpret_cast<unsigned long long*>(p.stats)[row * Q + q] =
-            ((unsigned long long)__float_as_uint(red[0] + red[1]) << 32) | __float_as_uint(mx);
+            ((unsigned long long)__float_as_uint(sm) << 32) | __float_as_uint(mx);
         CH_TL(3);
         return;
     }
@@ -810,7 +893,7 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
         unsigned long long g = 0;
         if (lane < 8) g = (1ull << 48) | ((cand_s[lane] >> 32 & 0xffffull) << 32) | (cand_s[lane] & 0xffffffffull);
         else if (lane == 8) g = (1ull << 32) | __float_as_uint(mx);
-        else if (lane == 9) g = (1ull << 32) | __float_as_uint(red[0] + red[1]);
+        else if (lane == 9) g = (1ull << 32) | __float_as_uint(sm);
         if (lane < CH_GRAN) __hip_atomic_store(gran + q * CH_GRAN + lane, g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
@@ -838,7 +921,7 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
         }
         if (lane < 8) gr[lane] = (1ull << 48) | ((cand_s[lane] >> 32 & 0xffffull) << 32) | (cand_s[lane] & 0xffffffffull);
         else if (lane == 8) gr[8] = (1ull << 32) | __float_as_uint(mx);
-        else if (lane == 9) gr[9] = (1ull << 32) | __float_as_uint(red[0] + red[1]);
+        else if (lane == 9) gr[9] = (1ull << 32) | __float_as_uint(sm);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");       // one wave: its own LDS writes, in order
         __builtin_amdgcn_wave_barrier();
     }
@@ -855,10 +938,10 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
         psum = __uint_as_float((unsigned)gr[lane * CH_GRAN + 9]);
     }
     float ww = 0.f;
-    const int rank = route_merge_token(c, ncand, pmx, psum, Q, top_k, p.norm_topk, true, &ww);
-    if (rank < top_k) {
-        p.ids[row * top_k + rank] = (int)(c >> 32);
-        p.weights[row * top_k + rank] = ww;
+    const int place = route_merge_token(c, ncand, pmx, psum, Q, top_k, p.norm_topk, true, &ww);
+    if (place < top_k) {
+        p.ids[row * top_k + place] = (int)(c >> 32);
+        p.weights[row * top_k + place] = ww;
     }
     CH_TL(3);
 }
@@ -868,7 +951,7 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
 // instructions on the critical path)
 template <int GPW_QKV, int GPW_O, bool HAS_ZP, bool KVS = false, bool WIDE = false>
 __global__ __launch_bounds__(512, 2) void decode_chain_kernel(ChainArgs p) {
-    __shared__ __attribute__((aligned(16))) unsigned char smem[CH_SMEM];
+    __shared__ __attribute__((aligned(16))) unsigned char smem[CH_SMEM > CH_W * GPW_QKV * 4096 ? CH_SMEM : CH_W * GPW_QKV * 4096];
     const int RH = (p.T + 15) >> 4;                                   // 16-row blocks
     const int QB = WIDE ? 128 : (p.qkv_half ? 32 : 64);             // q|k|v block width
     const int n_a = p.has_a ? p.T : 0, n_qkv = p.qkv.N / QB * RH, n_attn = p.T * p.nkv * (KVS ? p.attn_splits : 1), n_o = p.o.N / (p.o_half ? 32 : 64 * CH_O_NST) * RH * CH_O_KS;
@@ -976,7 +1059,9 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
 #endif
     const int rh = (d.T + 15) / 16;
     a.attn_splits = std::max(1, d.attn_splits); a.attn_partial = d.attn_partial; a.attn_tickets = d.attn_tickets;
-    a.qkv_half = (knobs().chain_qkv_half && d.T <= 16) ? 1 : 0;
+    // 32-column q|k|v blocks for up to 16 rows, as long as they and the attention role are resident together: beyond, the role's last
+    // workgroups enter behind the projection
+    a.qkv_half = (knobs().chain_qkv_half && d.T <= 16 && d.qkv->n / 32 + d.T * d.nkv * a.attn_splits <= knobs().chain_slots) ? 1 : 0;
     // (narrow o_proj only: 2048 columns → 64 blocks; Llama-3.1-8B's 4096 columns are 64 blocks of 64 already: c=8 1.908 → 1.930 ms with 32)
     a.o_half = (knobs().chain_o_half && d.T <= 16 && d.o->n <= 2048) ? 1 : 0;
     // 128-column q|k|v blocks (hidden 2048 only: the two-group weight ring): where the 64-column blocks + the attention role do not fit

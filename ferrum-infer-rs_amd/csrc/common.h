@@ -94,12 +94,14 @@ __device__ __forceinline__ float wave_reduce_max(float v) {
     return rows_reduce_max(v);
 }
 
-// Sum S ≤ 8 fp32 split-K slabs of one 8-element span in slab order.  All 16 loads are issued up front (index
-// clamped, not branched: a load under a runtime condition costs one L2 round trip per slab) and masked in the add.
-__device__ __forceinline__ void reduce_slabs8(const float* __restrict__ base, long slab_stride, int S, float (&o)[8]) {
-    float4v sv[8][2];
+// Sum fp32 split-K slabs of one 8-element span in slab order.  The loads of up to eight are issued up front (a load under a condition of
+// its own costs one L2 round trip per slab), no more than two of them repeats of the last slab: one workgroup that sums a row takes its
+// slabs at what a CU gets (6 slabs of 4096 columns: 128 → 96 KB).
+template <int N>
+__device__ __forceinline__ void reduce_slabs_upto(const float* __restrict__ base, long slab_stride, int S, float (&o)[8]) {
+    float4v sv[N][2];
 #pragma unroll
-    for (int z = 0; z < 8; z++) {
+    for (int z = 0; z < N; z++) {
         const float4v* sp = reinterpret_cast<const float4v*>(base + (long)(z < S ? z : S - 1) * slab_stride);
         sv[z][0] = sp[0];
         sv[z][1] = sp[1];
@@ -107,12 +109,17 @@ __device__ __forceinline__ void reduce_slabs8(const float* __restrict__ base, lo
 #pragma unroll
     for (int j = 0; j < 8; j++) o[j] = 0.f;
 #pragma unroll
-    for (int z = 0; z < 8; z++) {
+    for (int z = 0; z < N; z++) {
         if (z < S) {
 #pragma unroll
             for (int j = 0; j < 4; j++) { o[j] += sv[z][0][j]; o[4 + j] += sv[z][1][j]; }
         }
     }
+}
+__device__ __forceinline__ void reduce_slabs8(const float* __restrict__ base, long slab_stride, int S, float (&o)[8]) {
+    if (S <= 4) return reduce_slabs_upto<4>(base, slab_stride, S, o);
+    if (S <= 6) return reduce_slabs_upto<6>(base, slab_stride, S, o);
+    reduce_slabs_upto<8>(base, slab_stride, S, o);
     for (int z = 8; z < S; z++) {          // S > 8: rare, serial
         const float4v* sp = reinterpret_cast<const float4v*>(base + (long)z * slab_stride);
         float4v s0 = sp[0], s1 = sp[1];

@@ -21,19 +21,45 @@ struct RopeRow {
     int off0, off1;
 };
 
+// What rotates and scales a row besides the row itself.
+template <int HD>
+struct RopeCoef {
+    typename RopeRow<HD>::hv w0, w1;
+    typename RopeRow<HD>::fv cv, sv;
+};
+template <int HD>
+__device__ __forceinline__ int rope_off0(int mode, int q16) { return mode == 3 ? q16 * (HD / 16) : q16 * (HD / 32); }
+template <int HD>
+__device__ __forceinline__ int rope_off1(int mode, int q16) { return mode == 3 ? q16 * (HD / 16) + HD / 32 : q16 * (HD / 32) + HD / 2; }
+template <int HD>
+__device__ __forceinline__ RopeCoef<HD> rope_coef16(const __half* nw, const float* cs, const float* sn, int mode, bool have_nw, bool have_rope,
+                                                    int q16) {
+    using R = RopeRow<HD>;
+    RopeCoef<HD> c;
+#pragma unroll
+    for (int k = 0; k < R::PPL; k++) { c.w0[k] = (_Float16)1.f; c.w1[k] = (_Float16)1.f; c.cv[k] = 1.f; c.sv[k] = 0.f; }
+    if (have_nw) {
+        c.w0 = *reinterpret_cast<const typename R::hv*>(nw + rope_off0<HD>(mode, q16));
+        c.w1 = *reinterpret_cast<const typename R::hv*>(nw + rope_off1<HD>(mode, q16));
+    }
+    if (have_rope) {
+        c.cv = *reinterpret_cast<const typename R::fv*>(cs + q16 * R::PPL);
+        c.sv = *reinterpret_cast<const typename R::fv*>(sn + q16 * R::PPL);
+    }
+    return c;
+}
+
 // SC1: the source row was written by another workgroup of THIS launch (write-through stores behind a counter): it is read with
 // L1-bypassing loads (relaxed agent-scope 8-byte loads; head_dim 128 only).
 template <int HD, bool SC1 = false>
-__device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const __half* nw, const float* cs, const float* sn,
-                                                  int mode, bool have_nw, bool have_rope, float eps, int q16) {
+__device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const RopeCoef<HD>& coef, int mode, float eps, int q16) {
 #pragma clang fp contract(off)
     using R = RopeRow<HD>;
-    constexpr int PPL = R::PPL, HALF = HD / 2;
-    const int base = q16 * PPL;
+    constexpr int PPL = R::PPL;
     const bool m3 = mode == 3;
     R r;
-    r.off0 = m3 ? 2 * base : base;
-    r.off1 = m3 ? 2 * base + PPL : base + HALF;
+    r.off0 = rope_off0<HD>(mode, q16);
+    r.off1 = rope_off1<HD>(mode, q16);
     typename R::hv c0, c1;
     if constexpr (SC1) {
         static_assert(!SC1 || PPL == 4, "the in-launch hand-off form reads 8-byte pieces");
@@ -45,18 +71,8 @@ __device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const __hal
         c0 = *reinterpret_cast<const typename R::hv*>(src + r.off0);
         c1 = *reinterpret_cast<const typename R::hv*>(src + r.off1);
     }
-    typename R::hv w0, w1;
-    typename R::fv cv, sv;
-#pragma unroll
-    for (int k = 0; k < PPL; k++) { w0[k] = (_Float16)1.f; w1[k] = (_Float16)1.f; cv[k] = 1.f; sv[k] = 0.f; }
-    if (have_nw) {
-        w0 = *reinterpret_cast<const typename R::hv*>(nw + r.off0);
-        w1 = *reinterpret_cast<const typename R::hv*>(nw + r.off1);
-    }
-    if (have_rope) {
-        cv = *reinterpret_cast<const typename R::fv*>(cs + base);
-        sv = *reinterpret_cast<const typename R::fv*>(sn + base);
-    }
+    const typename R::hv w0 = coef.w0, w1 = coef.w1;
+    const typename R::fv cv = coef.cv, sv = coef.sv;
     float c[2 * PPL], w[2 * PPL];
 #pragma unroll
     for (int k = 0; k < PPL; k++) {
@@ -100,6 +116,11 @@ __device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const __hal
 #pragma unroll
     for (int k = 0; k < PPL; k++) { r.out0[k] = (_Float16)o[k]; r.out1[k] = (_Float16)o[PPL + k]; }
     return r;
+}
+template <int HD, bool SC1 = false>
+__device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const __half* nw, const float* cs, const float* sn,
+                                                  int mode, bool have_nw, bool have_rope, float eps, int q16) {
+    return rope_row16<HD, SC1>(src, rope_coef16<HD>(nw, cs, sn, mode, have_nw, have_rope, q16), mode, eps, q16);
 }
 
 }  // namespace fh

@@ -1431,12 +1431,14 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
         d.cand = m->route_cand; d.stats = m->route_stats; d.route_arrive = m->route_arrive; d.ids = m->expert_ids; d.weights = m->expert_w;
         d.timeout = m->inlaunch_timeouts;
         // KV ranges per (sequence, kv head) in the attention role: ≈ chain_split_keys (256) keys each while the role stays within
-        // W workgroups — W = 32 … 256 growing with the (sequence, kv head) count: the chain holds one workgroup per CU, and ranges
+        // W workgroups — W = 128 … 256 growing with the (sequence, kv head) count: the chain holds one workgroup per CU, and ranges
         // beyond that push the o_proj / router roles (which prefetch their weights while they wait) out of residence — but never
-        // more than ≈ 1024 keys per range while 256 workgroups allow (profiles/r03_chain_kv_splits.txt: c × context × ranges)
+        // more than ≈ 1024 keys per range while 256 workgroups allow.  (µs of a step with half of / as many / twice as many ranges as this
+        // rule's: 32 layers of 8 kv heads, one sequence of 4000 keys 1677 / 1642 / –, two of 2000 1758 / 1667 / 1703, four of 1000
+        // 1754 / 1683 / 1730, eight of 2000 2016 / 2011 / 2200; 8 expert layers of 4 kv heads, one of 8000 448 / 412 / –, four of 2000 511 / 486 / 517)
         const long keys = d.sliding_window > 0 ? std::min<long>(sh.max_kv_len, d.sliding_window) : sh.max_kv_len;
         const long units = (long)T * nkv, sk = std::max(1, knobs().chain_split_keys);
-        const long cap_w = std::min<long>(256, std::max<long>(4 * units, std::min<long>(8 * units, 64)));
+        const long cap_w = std::min<long>(256, std::max<long>(4 * units, 128));
         long ns_l = std::min<long>({16, std::max<long>(1, cap_w / units), (keys + sk - 1) / sk});
         ns_l = std::max<long>(ns_l, std::min<long>({16, std::max<long>(1, 256 / units), (keys + 4 * sk - 1) / (4 * sk)}));
         int ns = keys <= 2 * sk ? 1 : (int)std::max<long>(1, ns_l);        // (≤ 512 keys: one range — c=4 at 256+: 2.31 vs 2.36 ms split in two)

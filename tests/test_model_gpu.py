@@ -939,6 +939,38 @@ def test_decode_chain_attention_kv_splits(pkg, forms, knobs, window):
                 assert srt[r, -1] - srt[r, -2] <= 2 * err[r] + 1e-6, (other, s, int(r))
 
 
+@pytest.mark.parametrize("c", [1, 4, 8, 9, 16, 17])
+def test_decode_chain_of_wide_layers(pkg, c, forms):
+    """Hidden 4096: four quant groups a wave in the q|k|v role (two for hidden 2048), its blocks 32 columns wide up to the rows at which they and
+    the attention role still fit the chip together (8 here), 64 beyond.  Rows against the oracle as in the other tests of the launch."""
+    from tests import modelgen
+    from oracle import oracle as O
+    if "wide" not in _CHAIN_TM:
+        _CHAIN_TM["wide"] = modelgen.TinyModel(False, layers=2, hidden=4096, nq=32, nkv=8, hd=128, inter=2048, vocab=2048, seed=59, max_seq_len=64,
+                                               qk_norm=False, rope_theta=500000.0)
+    tm = _CHAIN_TM["wide"]
+    plen, steps, followed = 5, 2, sorted({0, c - 1})
+    O.set_threads(ORACLE_THREADS)
+    om = tm.oracle_model()
+    rng = np.random.default_rng(61)
+    prompts = [rng.integers(0, 2048, size=plen).astype(np.uint32) for _ in range(c)]
+    par = modelgen.Parity(f"wide-chain-c{c}", cos_min=0.999, rel_max=5e-2)
+    hm = tm.hip_model(pkg, kv_num_blocks=c * 2 + 4, max_seqs=c, max_tokens=max(c * plen, 64))
+    toks, lg = hm.unified_forward([(i, p, 0, True) for i, p in enumerate(prompts)], greedy=True, want_logits=True)
+    cur = np.array(toks, np.uint32)
+    for oc, i in enumerate(followed):
+        cur[i] = par.check(f"prefill/{i}", om.forward(oc, prompts[i], 0), lg[i], toks[i], float("inf"))
+    forms.reset()
+    for s in range(steps):
+        toks, lg = hm.unified_forward([(i, [int(cur[i])], plen + s, True) for i in range(c)], greedy=True, want_logits=True)
+        fed, cur = cur, np.array(toks, np.uint32)
+        for oc, i in enumerate(followed):
+            cur[i] = par.check(f"step{s}/{i}", om.forward(oc, np.array([fed[i]], np.uint32), plen + s), lg[i], toks[i], float("inf"))
+    assert forms.hits().get("decode_chain", 0) == 2 * steps, forms.hits()
+    O.set_threads(1)
+    par.finish(max_mismatches=1, max_route_ties=0)
+
+
 # ── the same launch for the attention half of a DENSE layer (Llama-style: no q/k norm, no router) ─────────────────────────────
 # Three layers, so that the tail of a layer — the MLP's down projection as split-K slabs + residual + next input norm — runs as the
 # first role of the next layer's launch: oracle-followed rows, the five-launch layer on the same tokens, graph ≡ eager.
