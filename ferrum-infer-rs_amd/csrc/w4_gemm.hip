@@ -1506,30 +1506,39 @@ __global__ __launch_bounds__(MT == 1 ? (GATED ? 512 : 1024) : (MT == 2 ? (NT == 
 // ── dense GEMM for up to 16 rows into fp32 slabs: a workgroup's share of the activations RESIDENT in LDS ─────────────
 // The waves of w4_gemm_wgsplit_kernel read the activations of every column tile again: 4 KiB of 16-row fragments for each KiB of
 // weights where a workgroup has one tile, so that its time grows with the rows (14336→4096: 10.4 µs at 1 row, 14.5 at 12, 16.9 at 16)
-// while the weights stay the same.  Here a workgroup takes 128 columns and 1 / S of K: its rows of x come to LDS once (fragment-major,
-// one copy without registers) together with the first weights, and after one barrier its eight waves — two tiles by half of its K
-// each — stream weights alone, two groups ahead; the halves meet in LDS and one slab of S leaves.  The consumer that exists anyway
+// while the weights stay the same.  Here a workgroup takes 128 columns and 1 / S of K: its rows of x come to LDS once (whole lines, a copy
+// without registers) ahead of the first weights, and after one barrier, which the rows alone are waited for, its eight waves — two tiles by
+// half of its K each — stream weights, two groups ahead; the halves meet in LDS and one slab of S leaves.  The consumer that exists anyway
 // (add + norm, the first role of the next layer's launch) sums the slabs in order.  S fills the chip with one round of workgroups.
+// As a launch of decode, µs, rows as 64-byte pieces of 16 and six slabs → this: 14336→4096 1 row 8.6 → 8.2, 12 rows 9.7 → 8.8;
+// 21504→5376 5 rows 13.2 → 12.2.  Measured alone, with pieces and six slabs:
 //   us, old → this with S slabs          1 row         5 rows        12 rows       16 rows
 //   14336→4096, S = 6                    10.4 →  8.4   10.8 →  8.8   14.5 →  9.4   16.9 →  9.7     (29 MB: 4.7 at 6.5 TB/s)
 //   21504→5376, S = 6                    24.3 → 12.5   26.2 → 13.1   37.5 → 14.1   44.7 → 14.7     (58 MB: 9.2)
 //    4096→5376, S = 6                     6.5 →  5.1    7.0 →  5.4    9.2 →  5.5   10.5 →  5.7
-// Four groups ahead instead of two, one tile a wave, or 64 columns a workgroup: 3 – 15 % slower.  A form with two row tiles for 17 – 32
+// Three or four groups ahead instead of two: within 1 %.  One tile a wave, or 64 columns a workgroup: 3 – 15 % slower.  A form with two row tiles for 17 – 32
 // rows lost to w4_gemm_ldsa_kernel (a step of 24 sequences 2.42 against 2.32 ms).
-constexpr int W4_ROWS_TILES = 8, W4_ROWS_LDS = 156 * 1024;
+constexpr int W4_ROWS_TILES = 8, W4_ROWS_LDS = 156 * 1024, W4_ROWS_AHEAD = 2;
 template <bool HAS_ZP>
 __global__ __launch_bounds__(512) void w4_gemm_rows_kernel(W4Args p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    constexpr int NT = 2, TG = W4_ROWS_TILES / NT, KP = 8 / TG, DW = 2;
+    constexpr int NT = 2, TG = W4_ROWS_TILES / NT, KP = 8 / TG, DW = W4_ROWS_AHEAD;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
     const int z = blockIdx.y, G0 = (int)((long)p.G * z / p.S), Gs = (int)((long)p.G * (z + 1) / p.S) - G0;
     const int tg = wave % TG, kp = wave / TG, tile0 = blockIdx.x * W4_ROWS_TILES + tg * NT, st = tile0 >> 2, nt0 = tile0 & 3;
     const int g0 = G0 + Gs * kp / KP, g1 = G0 + Gs * (kp + 1) / KP, ng = g1 - g0;
-    // fragment f = group · 4 + k-step, 1 KiB each: lane (a, b) brings row b, k = 8a …
-    const __half* xr = p.x + (long)(b < p.M ? b : p.M - 1) * p.K + G0 * 128 + 8 * a;
-    for (int f = wave; f < Gs * 4; f += 8)
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xr + f * 32), (__attribute__((address_space(3))) void*)(lds + f * 1024), 16, 0, 0);
+    // rows by whole lines: [group][16 rows][16 pieces of 16 bytes, piece xor row], a quarter of a group's rows a load (rows past the last lie
+    // past the buffer's end: no memory request)
+    const int quad = wave & 3, row_in = 4 * quad + a;
+    if (4 * quad < p.M) {
+        const __amdgpu_buffer_rsrc_t r_x = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, p.M * p.K * 2, 0x00020000);
+        const int o_x = (row_in * p.K + (b ^ row_in) * 8) * 2;
+        for (int g = wave >> 2; g < Gs; g += 2)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r_x, (__attribute__((address_space(3))) void*)(lds + (g * 4 + quad) * 1024), 16, o_x, (G0 + g) * 256, 0, 0);
+    }
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
     typedef uint32_t u32x4g __attribute__((ext_vector_type(4)));
     // (a group past the wave's end, or a supertile past the last one, lies past the buffer's end: zeros, and no memory request)
     const int end = st < p.n64 ? g1 : 0;
@@ -1550,15 +1559,21 @@ __global__ __launch_bounds__(512) void w4_gemm_rows_kernel(W4Args p) {
         zpv[slot] = HAS_ZP ? __builtin_bit_cast(unsigned long long, __builtin_amdgcn_raw_buffer_load_b64(r_z, g * 128 + o_s, 0, 0)) : 0ull;
     };
     auto consume = [&](int slot, int g) __attribute__((always_inline)) {
-        const half8* fr = reinterpret_cast<const half8*>(lds) + (size_t)(g - G0) * 4 * 64 + lane;
+        const unsigned char* fr = lds + (g - G0) * 4096 + b * 256;
 #pragma unroll
-        for (int s = 0; s < 4; s++) af[0][s] = fr[s * 64];
+        for (int s = 0; s < 4; s++) af[0][s] = *reinterpret_cast<const half8*>(fr + ((4 * s + a) ^ b) * 16);
         w4_consume_group<1, NT, HAS_ZP, false>(wq[slot], scv[slot], zpv[slot], nt0, af, acc);
     };
 #pragma unroll
     for (int d = 0; d < DW; d++) issue(d, g0 + d);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                   // (every wave's rows have landed)
-    __syncthreads();
+    constexpr int later = DW * (HAS_ZP ? NT + 2 : NT + 1);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt((later & 15) | 0xF70 | (later >> 4) << 14);             // (the wave's rows have landed, its weights are under way)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
     int i = 0;
     for (; i + DW <= ng; i += DW)
 #pragma unroll
@@ -1567,7 +1582,9 @@ __global__ __launch_bounds__(512) void w4_gemm_rows_kernel(W4Args p) {
             issue(d, g0 + i + d + DW);
             __builtin_amdgcn_sched_barrier(0);
         }
-    if (i < ng) consume(0, g0 + i);
+#pragma unroll
+    for (int d = 0; d + 1 < DW; d++)
+        if (i + d < ng) consume(d, g0 + i + d);
     // the K halves meet in LDS: [half][tile][lane]
     __syncthreads();
     float4v* red = reinterpret_cast<float4v*>(lds);
@@ -3043,15 +3060,15 @@ int w4_gemm_dense_slabs_tile(const W4Device& w, const __half* x, float* slabs, s
 }
 
 // Splits of K with which w4_gemm_rows takes this projection, 0 where it does not: one round of workgroups over the chip, at least half
-// of it (with fewer columns w4_gemm_wgsplit_kernel has the more workgroups), a workgroup's share of the rows within LDS.  Six slabs at
-// most: eight make the launch of 14336→4096 shorter (9.4 → 8.9 µs at 12 rows), but what sums them longer: a decode step of 32 layers
-// took 1867 µs with eight, 1825 with six, 1841 with four (4 sequences: 1641, 1632, 1703).
+// of it (with fewer columns w4_gemm_wgsplit_kernel has the more workgroups), a workgroup's share of the rows within LDS, the slabs within
+// what there is for them.  Seven at most: µs of a step of 32 layers (14336→4096) with four / six / seven / eight at 1 row 1718 / 1681 /
+// 1670 / 1676, at 12 rows 1708 / 1666 / 1655 / 1654: what sums them takes longer with each.
 int w4_gemm_rows_splits(const W4Device& w, int m, size_t slab_bytes) {
     if (m < 1 || m > 16 || !w.qw || w.bias) return 0;
     const int cols = cdiv(w.n64, W4_ROWS_TILES / 4);
-    const int S = std::min({256 / cols, 6, w.G});
+    const int S = std::min({256 / cols, 7, w.G, (int)std::min<size_t>(slab_bytes / ((size_t)16 * w.n64 * 64 * sizeof(float)), 7)});
     if (S < 1 || cols * S < 128 || cdiv(w.G, S) * 4096 > W4_ROWS_LDS) return 0;
-    return (size_t)S * 16 * w.n64 * 64 * sizeof(float) <= slab_bytes ? S : 0;
+    return S;
 }
 
 int w4_gemm_rows(const W4Device& w, const __half* x, float* slabs, size_t slab_bytes, int m, int* S_out, int* rows_pad_out, int* n_pad_out,
