@@ -609,7 +609,7 @@ __device__ __forceinline__ void chain_role_attn(const ChainArgs& p, int wg, unsi
     }
 #pragma unroll
     for (int dt = 0; dt < DT; dt++)
-        *reinterpret_cast<float4v*>(&lds_o[(wave * 16 + b) * OSTRIDE + dt * 16 + 4 * a]) = o_acc[dt];
+        if (row_ok) *reinterpret_cast<float4v*>(&lds_o[(wave * 16 + b) * OSTRIDE + dt * 16 + 4 * a]) = o_acc[dt];       // (rows past the group are not read)
     __syncthreads();
     constexpr int TPR = NW * 4;                                       // threads per row: 32 → 4 dims each
     const int row = threadIdx.x / TPR, dl = threadIdx.x % TPR;

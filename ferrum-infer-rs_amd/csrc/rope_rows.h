@@ -49,10 +49,31 @@ __device__ __forceinline__ RopeCoef<HD> rope_coef16(const __half* nw, const floa
     return c;
 }
 
+// The lane's pieces of the row itself.
+template <int HD>
+struct RopeSource { typename RopeRow<HD>::hv c0, c1; };
+template <int HD>
+__device__ __forceinline__ RopeSource<HD> rope_source16(const __half* src, int mode, int q16) {
+    using hv = typename RopeRow<HD>::hv;
+    return {*reinterpret_cast<const hv*>(src + rope_off0<HD>(mode, q16)), *reinterpret_cast<const hv*>(src + rope_off1<HD>(mode, q16))};
+}
+
 // SC1: the source row was written by another workgroup of THIS launch (write-through stores behind a counter): it is read with
 // L1-bypassing loads (relaxed agent-scope 8-byte loads; head_dim 128 only).
 template <int HD, bool SC1 = false>
-__device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const RopeCoef<HD>& coef, int mode, float eps, int q16) {
+__device__ __forceinline__ RopeSource<HD> rope_source16_sc1(const __half* src, int mode, int q16) {
+    using R = RopeRow<HD>;
+    static_assert(!SC1 || R::PPL == 4, "the in-launch hand-off form reads 8-byte pieces");
+    if constexpr (!SC1) return rope_source16<HD>(src, mode, q16);
+    const unsigned long long u0 = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(src + rope_off0<HD>(mode, q16)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long u1 = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(src + rope_off1<HD>(mode, q16)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    RopeSource<HD> r;
+    __builtin_memcpy(&r.c0, &u0, sizeof r.c0);
+    __builtin_memcpy(&r.c1, &u1, sizeof r.c1);
+    return r;
+}
+template <int HD>
+__device__ __forceinline__ RopeRow<HD> rope_row16(const RopeSource<HD>& source, const RopeCoef<HD>& coef, int mode, float eps, int q16) {
 #pragma clang fp contract(off)
     using R = RopeRow<HD>;
     constexpr int PPL = R::PPL;
@@ -60,17 +81,7 @@ __device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const RopeC
     R r;
     r.off0 = rope_off0<HD>(mode, q16);
     r.off1 = rope_off1<HD>(mode, q16);
-    typename R::hv c0, c1;
-    if constexpr (SC1) {
-        static_assert(!SC1 || PPL == 4, "the in-launch hand-off form reads 8-byte pieces");
-        const unsigned long long u0 = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(src + r.off0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned long long u1 = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(src + r.off1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        c0 = __builtin_bit_cast(typename R::hv, u0);
-        c1 = __builtin_bit_cast(typename R::hv, u1);
-    } else {
-        c0 = *reinterpret_cast<const typename R::hv*>(src + r.off0);
-        c1 = *reinterpret_cast<const typename R::hv*>(src + r.off1);
-    }
+    const typename R::hv c0 = source.c0, c1 = source.c1;
     const typename R::hv w0 = coef.w0, w1 = coef.w1;
     const typename R::fv cv = coef.cv, sv = coef.sv;
     float c[2 * PPL], w[2 * PPL];
@@ -117,10 +128,14 @@ __device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const RopeC
     for (int k = 0; k < PPL; k++) { r.out0[k] = (_Float16)o[k]; r.out1[k] = (_Float16)o[PPL + k]; }
     return r;
 }
-template <int HD, bool SC1 = false>
+template <int HD, bool SC1>
+__device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const RopeCoef<HD>& coef, int mode, float eps, int q16) {
+    return rope_row16<HD>(rope_source16_sc1<HD, SC1>(src, mode, q16), coef, mode, eps, q16);
+}
+template <int HD>
 __device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const __half* nw, const float* cs, const float* sn,
                                                   int mode, bool have_nw, bool have_rope, float eps, int q16) {
-    return rope_row16<HD, SC1>(src, rope_coef16<HD>(nw, cs, sn, mode, have_nw, have_rope, q16), mode, eps, q16);
+    return rope_row16<HD>(rope_source16<HD>(src, mode, q16), rope_coef16<HD>(nw, cs, sn, mode, have_nw, have_rope, q16), mode, eps, q16);
 }
 
 }  // namespace fh
