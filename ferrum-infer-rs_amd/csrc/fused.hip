@@ -62,6 +62,7 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_route_kernel(
     const int i = threadIdx.x;
     half8 v;
     float ss = 0.f;
+    const half8 wv = *reinterpret_cast<const half8*>(w + (i < nvec ? i : 0) * 8);
     if (i < nvec) {
         float o[8];
         if (SLABS) {     // o_proj arrives as S fp32 split-K slabs: reduce in slab order, round like the fp16 op output
@@ -76,7 +77,6 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_route_kernel(
         half8 rv = *reinterpret_cast<const half8*>(residual + row * H + i * 8);
 #pragma unroll
         for (int j = 0; j < 8; j++) rv[j] = (_Float16)((float)rv[j] + o[j]);
-        *reinterpret_cast<half8*>(residual + row * H + i * 8) = rv;
         v = rv;
 #pragma unroll
         for (int j = 0; j < 8; j++) ss += (float)rv[j] * (float)rv[j];
@@ -84,12 +84,12 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_route_kernel(
     const float total = block_sum_1024(ss, red);
     const float inv = 1.0f / sqrtf(total / (float)H + eps);
     if (i < nvec) {
-        half8 wv = *reinterpret_cast<const half8*>(w + i * 8);
         half8 o;
 #pragma unroll
         for (int j = 0; j < 8; j++) o[j] = (_Float16)((float)v[j] * inv * (float)wv[j]);
         if (!out_perm) *reinterpret_cast<half8*>(norm_out + row * H + i * 8) = o;
         *reinterpret_cast<half8*>(xs + i * 8) = o;
+        *reinterpret_cast<half8*>(residual + row * H + i * 8) = v;
     }
     __syncthreads();
     // act-order consumer: the row leaves in the packed-row order of its weights (the router below reads the natural row)

@@ -31,7 +31,9 @@ __device__ __forceinline__ void store_row_gathered_256(__half* out_row, const _F
     for (int i = threadIdx.x; i < nvec; i += 256) *reinterpret_cast<half8*>(out_row + i * 8) = lds_gather8(stage, perm, i * 8);
 }
 
-// One 256-thread workgroup per row; each thread keeps up to CHUNKS 16-byte chunks in registers.
+// One 256-thread workgroup per row; each thread keeps up to CHUNKS 16-byte chunks in registers.  A few rows are latency alone: the weights are
+// requested with the row, and the new residual is stored behind the result (loads and stores retire in order, so a load behind a store
+// waits for it too).
 template <bool FUSED_ADD, int CHUNKS>
 __global__ __launch_bounds__(256) void rms_norm_kernel(const __half* __restrict__ x, __half* __restrict__ residual,
                                                        const __half* __restrict__ w, float eps,
@@ -41,7 +43,12 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const __half* __restrict_
     extern __shared__ _Float16 stage[];            // dim halves when out_perm
     const long row = blockIdx.x;
     const int nvec = dim >> 3;
-    half8 v[CHUNKS];
+    half8 v[CHUNKS], wv[CHUNKS];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; c++) {
+        const int i = threadIdx.x + c * 256;
+        wv[c] = *reinterpret_cast<const half8*>(w + (i < nvec ? i : 0) * 8);
+    }
     float ss = 0.f;
 #pragma unroll
     for (int c = 0; c < CHUNKS; c++) {
@@ -55,7 +62,6 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const __half* __restrict_
                 // the updated residual is stored as fp16 and the variance is taken from the
                 // rounded values (same rounding point as the reference's fp16 lane,
                 // kernels/fused_add_rms_norm.cu:88-101)
-                *reinterpret_cast<half8*>(residual + row * dim + i * 8) = rv;
                 xv = rv;
             }
             v[c] = xv;
@@ -69,12 +75,12 @@ __global__ __launch_bounds__(256) void rms_norm_kernel(const __half* __restrict_
     for (int c = 0; c < CHUNKS; c++) {
         int i = threadIdx.x + c * 256;
         if (i < nvec) {
-            half8 wv = *reinterpret_cast<const half8*>(w + i * 8);
             half8 o;
 #pragma unroll
-            for (int j = 0; j < 8; j++) o[j] = (_Float16)((float)v[c][j] * inv * (float)wv[j]);
+            for (int j = 0; j < 8; j++) o[j] = (_Float16)((float)v[c][j] * inv * (float)wv[c][j]);
             if (out_perm) *reinterpret_cast<half8*>(stage + i * 8) = o;
             else *reinterpret_cast<half8*>(out + row * dim + i * 8) = o;
+            if (FUSED_ADD) *reinterpret_cast<half8*>(residual + row * dim + i * 8) = v[c];
         }
     }
     if (out_perm) store_row_gathered_256(out + row * dim, stage, out_perm, nvec);
@@ -122,7 +128,12 @@ __global__ __launch_bounds__(256) void gather_rms_norm_kernel(const __half* __re
     if (blockIdx.x == 0 && zero_words)
         for (int i = threadIdx.x; i < n_zero; i += 256) zero_words[i] = 0u;
     const int nvec = dim >> 3;
-    half8 v[CHUNKS];
+    half8 v[CHUNKS], wv[CHUNKS];
+#pragma unroll
+    for (int c = 0; c < CHUNKS; c++) {
+        const int i = threadIdx.x + c * 256;
+        wv[c] = *reinterpret_cast<const half8*>(w + (i < nvec ? i : 0) * 8);
+    }
     float ss = 0.f;
 #pragma unroll
     for (int c = 0; c < CHUNKS; c++) {
@@ -132,15 +143,6 @@ __global__ __launch_bounds__(256) void gather_rms_norm_kernel(const __half* __re
             if (scale != 0.0f) {
 #pragma unroll
                 for (int j = 0; j < 8; j++) xv[j] = (_Float16)((float)xv[j] * scale);
-            }
-            if (copy_f16) *reinterpret_cast<half8*>(copy_f16 + row * dim + i * 8) = xv;
-            if (copy_f32) {
-                float4v lo, hi;
-#pragma unroll
-                for (int j = 0; j < 4; j++) { lo[j] = (float)xv[j]; hi[j] = (float)xv[4 + j]; }
-                float4v* d = reinterpret_cast<float4v*>(copy_f32 + row * dim + i * 8);
-                d[0] = lo;
-                d[1] = hi;
             }
             v[c] = xv;
 #pragma unroll
@@ -153,12 +155,20 @@ __global__ __launch_bounds__(256) void gather_rms_norm_kernel(const __half* __re
     for (int c = 0; c < CHUNKS; c++) {
         const int i = threadIdx.x + c * 256;
         if (i < nvec) {
-            const half8 wv = *reinterpret_cast<const half8*>(w + i * 8);
             half8 o;
 #pragma unroll
-            for (int j = 0; j < 8; j++) o[j] = (_Float16)((float)v[c][j] * inv * (float)wv[j]);
+            for (int j = 0; j < 8; j++) o[j] = (_Float16)((float)v[c][j] * inv * (float)wv[c][j]);
             if (out_perm) *reinterpret_cast<half8*>(stage + i * 8) = o;
             else *reinterpret_cast<half8*>(out + row * dim + i * 8) = o;
+            if (copy_f16) *reinterpret_cast<half8*>(copy_f16 + row * dim + i * 8) = v[c];
+            if (copy_f32) {
+                float4v lo, hi;
+#pragma unroll
+                for (int j = 0; j < 4; j++) { lo[j] = (float)v[c][j]; hi[j] = (float)v[c][4 + j]; }
+                float4v* d = reinterpret_cast<float4v*>(copy_f32 + row * dim + i * 8);
+                d[0] = lo;
+                d[1] = hi;
+            }
         }
     }
     if (out_perm) store_row_gathered_256(out + row * dim, stage, out_perm, nvec);
@@ -343,12 +353,13 @@ __global__ __launch_bounds__(1024) void sandwich_add_norm_f32_wide_kernel(const 
         r[j] = (j < 4 ? r0[j] : r1[j - 4]) + x[j] * inv1 * (float)wb[j];
         if (on) ss2 += r[j] * r[j];
     }
+    const float sum2 = w_next ? block_sum(ss2) : 0.f;
     if (on) {
         rp[0] = (float4v){r[0], r[1], r[2], r[3]};
         rp[1] = (float4v){r[4], r[5], r[6], r[7]};
     }
     if (w_next == nullptr) return;
-    const float inv2 = 1.0f / sqrtf(block_sum(ss2) / (float)H + eps);
+    const float inv2 = 1.0f / sqrtf(sum2 / (float)H + eps);
     half8 o;
 #pragma unroll
     for (int j = 0; j < 8; j++) o[j] = (_Float16)(r[j] * inv2 * (float)wn[j]);

@@ -58,9 +58,25 @@ __device__ __forceinline__ float block_sum(float q, float* red) {
     q = wave_reduce_sum(q);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = q;
     __syncthreads();
-    float t = 0.f;
-    for (int i = 0; i < (int)(blockDim.x >> 6); i++) t += red[i];
+    float r[16], t = 0.f;                                              // (red holds 16, all read at once)
+#pragma unroll
+    for (int i = 0; i < 16; i++) r[i] = red[i];
+#pragma unroll
+    for (int i = 0; i < 16; i++) t += i < (int)(blockDim.x >> 6) ? r[i] : 0.f;
     return t;
+}
+// Σ over the slabs of a branch, in their order; up to four are under way together (one after the other each cost a round trip, 0.7 µs)
+__device__ __forceinline__ floatx4 sum_slabs(const float* p, int slabs, long stride) {
+    if (slabs == 1) return *reinterpret_cast<const floatx4*>(p);
+    floatx4 t[4];
+#pragma unroll
+    for (int z = 0; z < 4; z++) t[z] = *reinterpret_cast<const floatx4*>(p + (z < slabs ? z : slabs - 1) * stride);
+    floatx4 v = t[0];
+#pragma unroll
+    for (int z = 1; z < 4; z++)
+        if (z < slabs) v += t[z];
+    for (int z = 4; z < slabs; z++) v += *reinterpret_cast<const floatx4*>(p + z * stride);
+    return v;
 }
 
 // x += Σ slabs of `sub` + Σ_j weights[row][j] · pairs[row·top + j]; elementwise, grid (rows, quads of columns / 256)
@@ -75,9 +91,8 @@ __global__ __launch_bounds__(256) void branch_add_kernel(const float* __restrict
     const E* pr = pairs + row * top * ld_pair + i;
     if (VEC) {
         typedef E e4 __attribute__((ext_vector_type(4)));
-        floatx4 v = *reinterpret_cast<const floatx4*>(sr);
         const floatx4 xv = *reinterpret_cast<const floatx4*>(x + row * dim + i);
-        for (int z = 1; z < slabs; z++) v += *reinterpret_cast<const floatx4*>(sr + z * slab_stride);
+        floatx4 v = sum_slabs(sr, slabs, slab_stride);
 #pragma unroll 4
         for (int j = 0; j < top; j++) {
             const e4 e = *reinterpret_cast<const e4*>(pr + j * ld_pair);
@@ -113,9 +128,9 @@ int branch_add(const float* sub, long ld_sub, int slabs, long slab_stride, const
     return 0;
 }
 
-// One workgroup per row; a thread holds up to 4 quads of the row in registers, so the branch is read once.  NEXT: the copy is the row
+// One workgroup per row; a thread holds VEC quads of the row in registers (0: any length, from memory), so the branch is read once.  NEXT: the copy is the row
 // divided by its root mean square, the input of a block that norms ahead of its sublayers.
-template <typename E, bool VEC, bool GATE, bool NEXT>
+template <typename E, int VEC, bool GATE, bool NEXT>
 __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __restrict__ sub, long ld_sub, int slabs, long slab_stride, const E* __restrict__ gate,
                                                              long ld_gate, const float* __restrict__ w, float mult, float eps,
                                                              float* __restrict__ x, E* __restrict__ xb, int dim, int ldb) {
@@ -126,26 +141,25 @@ __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __rest
     float* xr = x + row * dim;
     E* br = xb + row * ldb;
     float q = 0.f, n = 0.f;
-    if (VEC) {
+    if constexpr (VEC > 0) {
         typedef E e4 __attribute__((ext_vector_type(4)));
-        floatx4 v[4], xv[4], wv[4];
+        floatx4 v[VEC ? VEC : 1], xv[VEC ? VEC : 1], wv[VEC ? VEC : 1];
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
+        for (int c = 0; c < VEC; c++) {
             const int i = (c * blockDim.x + threadIdx.x) * 4;
             if (i < dim) {
-                v[c] = *reinterpret_cast<const floatx4*>(sr + i);
-                for (int z = 1; z < slabs; z++) v[c] += *reinterpret_cast<const floatx4*>(sr + z * slab_stride + i);
-                e4 gv = {};
-                if (GATE) gv = *reinterpret_cast<const e4*>(gr + i);
                 xv[c] = *reinterpret_cast<const floatx4*>(xr + i);
                 wv[c] = *reinterpret_cast<const floatx4*>(w + i);
+                e4 gv = {};
+                if (GATE) gv = *reinterpret_cast<const e4*>(gr + i);
+                v[c] = sum_slabs(sr + i, slabs, slab_stride);
 #pragma unroll
                 for (int j = 0; j < 4; j++) { if (GATE) v[c][j] *= (float)gv[j]; q += v[c][j] * v[c][j]; }
             }
         }
         const float inv = mult / sqrtf(block_sum(q, red) / (float)dim + eps);
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
+        for (int c = 0; c < VEC; c++) {
             const int i = (c * blockDim.x + threadIdx.x) * 4;
             if (i < dim) {
 #pragma unroll
@@ -155,7 +169,7 @@ __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __rest
         }
         const float unit = NEXT ? 1.0f / sqrtf(block_sum(n, red + 16) / (float)dim + eps) : 1.0f;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
+        for (int c = 0; c < VEC; c++) {
             const int i = (c * blockDim.x + threadIdx.x) * 4;
             if (i < dim) {
                 e4 o;
@@ -190,10 +204,15 @@ int post_norm_add(const float* sub, long ld_sub, int slabs, long slab_stride, co
                   float* x, E* xb, int rows, int dim, int ldb, hipStream_t s) {
     const int threads = rows <= 512 && dim >= 2048 ? 1024 : 256;
     const bool vec = dim % 4 == 0 && dim <= threads * 16 && ld_sub % 4 == 0 && ld_gate % 4 == 0 && ldb % 4 == 0 && slab_stride % 4 == 0;
-#define POST(V, G, N) hipLaunchKernelGGL((post_norm_add_kernel<E, V, G, N>), dim3(rows), dim3(threads), 0, s, sub, ld_sub, slabs, slab_stride, gate, ld_gate, w, mult, eps, x, xb, dim, ldb)
-    if (gate) { if (next_norm) { if (vec) POST(true, true, true); else POST(false, true, true); } else { if (vec) POST(true, true, false); else POST(false, true, false); } }
-    else { if (next_norm) { if (vec) POST(true, false, true); else POST(false, false, true); } else { if (vec) POST(true, false, false); else POST(false, false, false); } }
-#undef POST
+    auto go = [&](auto v, auto g, auto n) {
+        hipLaunchKernelGGL((post_norm_add_kernel<E, decltype(v)::value, decltype(g)::value, decltype(n)::value>), dim3(rows), dim3(threads), 0, s, sub, ld_sub, slabs,
+                           slab_stride, gate, ld_gate, w, mult, eps, x, xb, dim, ldb);
+    };
+    auto with_next = [&](auto v, auto g) { next_norm ? go(v, g, std::true_type{}) : go(v, g, std::false_type{}); };
+    auto with_gate = [&](auto v) { gate ? with_next(v, std::true_type{}) : with_next(v, std::false_type{}); };
+    if (!vec) with_gate(std::integral_constant<int, 0>{});
+    else if (dim <= threads * 4) with_gate(std::integral_constant<int, 1>{});
+    else with_gate(std::integral_constant<int, 4>{});
     FH_CHECK_LAUNCH();
     return 0;
 }
@@ -212,9 +231,28 @@ int copy_rows(const E* x, long ldx, E* out, long ldo, int rows, int cols, hipStr
 template <typename E>
 __global__ __launch_bounds__(256) void rms_norm_rows_kernel(const float* __restrict__ x, const int32_t* __restrict__ row_idx,
                                                             const float* __restrict__ w, float eps, E* __restrict__ out, int dim, int ldo) {
-    __shared__ float red[4];
+    __shared__ float red[16];
     const float* xr = x + (row_idx ? (long)row_idx[blockIdx.x] : (long)blockIdx.x) * dim;
     float q = 0.f;
+    if (dim <= 8 * 256) {
+        // the row and its weights requested together, and read once
+        float xv[8], wv[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const int i = threadIdx.x + c * 256, at = i < dim ? i : 0;
+            wv[c] = w ? w[at] : 1.f;
+            xv[c] = xr[at];
+        }
+#pragma unroll
+        for (int c = 0; c < 8; c++) q += (int)threadIdx.x + c * 256 < dim ? xv[c] * xv[c] : 0.f;
+        const float inv = 1.0f / sqrtf(block_sum(q, red) / (float)dim + eps);
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const int i = threadIdx.x + c * 256;
+            if (i < dim) out[(long)blockIdx.x * ldo + i] = (E)(xv[c] * inv * wv[c]);
+        }
+        return;
+    }
     for (int i = threadIdx.x; i < dim; i += 256) q += xr[i] * xr[i];
     const float inv = 1.0f / sqrtf(block_sum(q, red) / (float)dim + eps);
     for (int i = threadIdx.x; i < dim; i += 256) out[(long)blockIdx.x * ldo + i] = (E)(w ? xr[i] * inv * w[i] : xr[i] * inv);
@@ -226,8 +264,8 @@ int rms_norm_rows(const float* x, const int32_t* row_idx, const float* w, float 
     return 0;
 }
 
-// One workgroup per row; a thread holds up to 4 quads of the row in registers.  POST: the sum itself is normed.
-template <typename E, bool VEC, bool POST>
+// One workgroup per row; a thread holds VEC quads of the row in registers (0: any length, from memory).  POST: the sum itself is normed.
+template <typename E, int VEC, bool POST>
 __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) {
     __shared__ float red[64];
     const long row = blockIdx.x;
@@ -246,26 +284,53 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
                 if (u.pair_ids[row * u.top + j] >= u.pair_limit) keep += u.weights[row * u.top + j];
     }
     auto listed = [&](int j) { return !POST || !u.pair_ids || u.pair_ids[row * u.top + j] < u.pair_limit; };
-    if (VEC) {
+    if constexpr (VEC > 0) {
         typedef E e4 __attribute__((ext_vector_type(4)));
-        floatx4 v[4], r[4], xv[4];
+        floatx4 v[VEC ? VEC : 1], r[VEC ? VEC : 1], xv[VEC ? VEC : 1], w1[VEC ? VEC : 1], w2[VEC ? VEC : 1], wn[VEC ? VEC : 1];
+        // (weights are requested ahead of the sums that they are for)
+#pragma unroll
+        for (int c = 0; c < VEC; c++) {
+            const int at = (c * nt + threadIdx.x) * 4, i = at < dim ? at : 0;
+            if (POST) w1[c] = *reinterpret_cast<const floatx4*>(u.post_w + i);
+            if (POST && u.gate) w2[c] = *reinterpret_cast<const floatx4*>(u.gate_w + i);
+            if (joined) { w1[c] = *reinterpret_cast<const floatx4*>(u.w + i); w2[c] = *reinterpret_cast<const floatx4*>(u.w2 + i); }
+            wn[c] = (floatx4){1.f, 1.f, 1.f, 1.f};
+            if (u.out && u.next_w) wn[c] = *reinterpret_cast<const floatx4*>(u.next_w + i);
+        }
         float q1 = 0.f, q2 = 0.f, n = 0.f;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
+        for (int c = 0; c < VEC; c++) {
             const int i = (c * nt + threadIdx.x) * 4;
             if (i < dim) {
+                xv[c] = (floatx4){0.f, 0.f, 0.f, 0.f};
+                if (!u.replace) xv[c] = *reinterpret_cast<const floatx4*>(xr + i);
+                if (joined) r[c] = sum_slabs(s2 + i, u.slabs2, u.slab_stride2);
                 v[c] = (floatx4){0.f, 0.f, 0.f, 0.f};
-                if (u.sub) v[c] = *reinterpret_cast<const floatx4*>(s1 + i);
-                for (int z = 1; z < u.slabs; z++) v[c] += *reinterpret_cast<const floatx4*>(s1 + z * u.slab_stride + i);
+                if (u.sub) v[c] = sum_slabs(s1 + i, u.slabs, u.slab_stride);
                 if (POST)
 #pragma unroll
                     for (int k = 0; k < 4; k++) v[c][k] *= factor;
-                xv[c] = (floatx4){0.f, 0.f, 0.f, 0.f};
-                if (!u.replace) xv[c] = *reinterpret_cast<const floatx4*>(xr + i);
                 if (POST)
 #pragma unroll
                     for (int k = 0; k < 4; k++) xv[c][k] *= keep;
                 if (u.add) xv[c] += *reinterpret_cast<const floatx4*>(u.add + i);
+                if (!POST)
+                    for (int j0 = 0; j0 < u.top; j0 += 8) {             // (eight at once)
+                        e4 e[8];
+                        float w[8];
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            const int at = min(j0 + j, u.top - 1);
+                            e[j] = *reinterpret_cast<const e4*>(pr + at * u.ld_pair + i);
+                            w[j] = u.weights[row * u.top + at];
+                        }
+#pragma unroll
+                        for (int j = 0; j < 8; j++)
+                            if (j0 + j < u.top)
+#pragma unroll
+                                for (int k = 0; k < 4; k++) v[c][k] += w[j] * (float)e[j][k];
+                    }
+                else
 #pragma unroll 4
                 for (int j = 0; j < u.top; j++) {
                     if (!listed(j)) continue;
@@ -275,8 +340,6 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
                     for (int k = 0; k < 4; k++) v[c][k] += w * (float)e[k];
                 }
                 if (joined) {
-                    r[c] = *reinterpret_cast<const floatx4*>(s2 + i);
-                    for (int z = 1; z < u.slabs2; z++) r[c] += *reinterpret_cast<const floatx4*>(s2 + z * u.slab_stride2 + i);
 #pragma unroll
                     for (int k = 0; k < 4; k++) { q1 += v[c][k] * v[c][k]; q2 += r[c][k] * r[c][k]; }
                 }
@@ -288,13 +351,12 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
             i2 = 0.5f / sqrtf(block_sum(q2, red + 16) / (float)dim + u.eps);
         }
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
+        for (int c = 0; c < VEC; c++) {
             const int i = (c * nt + threadIdx.x) * 4;
             if (i < dim) {
                 if (joined) {
-                    const floatx4 w1 = *reinterpret_cast<const floatx4*>(u.w + i), w2 = *reinterpret_cast<const floatx4*>(u.w2 + i);
 #pragma unroll
-                    for (int k = 0; k < 4; k++) v[c][k] = v[c][k] * i1 * w1[k] + r[c][k] * i2 * w2[k];
+                    for (int k = 0; k < 4; k++) v[c][k] = v[c][k] * i1 * w1[c][k] + r[c][k] * i2 * w2[c][k];
                 }
                 xv[c] += v[c];
 #pragma unroll
@@ -307,14 +369,13 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
             float z = 0.f;
             n = 0.f;
 #pragma unroll
-            for (int c = 0; c < 4; c++) {
+            for (int c = 0; c < VEC; c++) {
                 const int i = (c * nt + threadIdx.x) * 4;
                 if (i < dim) {
-                    const floatx4 w = *reinterpret_cast<const floatx4*>(u.post_w + i);
                     floatx4 g = {0.f, 0.f, 0.f, 0.f};
-                    if (u.gate) g = *reinterpret_cast<const floatx4*>(u.gate_w + i);
+                    if (u.gate) g = w2[c];
 #pragma unroll
-                    for (int k = 0; k < 4; k++) { xv[c][k] *= inv * w[k]; n += xv[c][k] * xv[c][k]; z += xv[c][k] * g[k]; }
+                    for (int k = 0; k < 4; k++) { xv[c][k] *= inv * w1[c][k]; n += xv[c][k] * xv[c][k]; z += xv[c][k] * g[k]; }
                     *reinterpret_cast<floatx4*>(xr + i) = xv[c];
                 }
             }
@@ -326,14 +387,12 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
         if (!u.out) return;
         const float unit = u.next_w ? 1.0f / sqrtf(block_sum(n, red + 32) / (float)dim + u.eps) : 1.0f;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
+        for (int c = 0; c < VEC; c++) {
             const int i = (c * nt + threadIdx.x) * 4;
             if (i < dim) {
-                floatx4 w = {1.f, 1.f, 1.f, 1.f};
-                if (u.next_w) w = *reinterpret_cast<const floatx4*>(u.next_w + i);
                 e4 o;
 #pragma unroll
-                for (int k = 0; k < 4; k++) o[k] = (E)(xv[c][k] * unit * w[k]);
+                for (int k = 0; k < 4; k++) o[k] = (E)(xv[c][k] * unit * wn[c][k]);
                 *reinterpret_cast<e4*>(out + i) = o;
             }
         }
@@ -392,9 +451,10 @@ int stream_update(const StreamUpdate<E>& u, hipStream_t s) {
     FH_REQUIRE(u.post_w ? !u.sub2 : u.keep == 1.f && !u.pair_ids && !u.sub_scale && !u.gate, "stream update: factors and the stream's own pairs belong to a normed sum of one branch");
     const int threads = u.rows <= 512 && u.dim >= 2048 ? 1024 : 256;
     const bool vec = u.dim % 4 == 0 && u.dim <= threads * 16 && u.ld_sub % 4 == 0 && u.ld_pair % 4 == 0 && u.ldo % 4 == 0 && u.slab_stride % 4 == 0 && u.slab_stride2 % 4 == 0;
+    const int quads = !vec ? 0 : u.dim <= threads * 4 ? 1 : u.dim <= threads * 8 ? 2 : 4;
 #define UPDATE(V, P) hipLaunchKernelGGL((stream_update_kernel<E, V, P>), dim3(u.rows), dim3(threads), 0, s, u)
-    if (u.post_w) { if (vec) UPDATE(true, true); else UPDATE(false, true); }
-    else { if (vec) UPDATE(true, false); else UPDATE(false, false); }
+    if (u.post_w) { if (quads == 1) UPDATE(1, true); else if (quads == 2) UPDATE(2, true); else if (quads) UPDATE(4, true); else UPDATE(0, true); }
+    else { if (quads == 1) UPDATE(1, false); else if (quads == 2) UPDATE(2, false); else if (quads) UPDATE(4, false); else UPDATE(0, false); }
 #undef UPDATE
     FH_CHECK_LAUNCH();
     return 0;
