@@ -780,6 +780,10 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn64_kernel(AttnArgs p
     };
 
     const float sl2 = p.scale * 1.4426950408889634f;
+    // A row's reference m_run stays until its maximum is more than SLACK (log2 units) above: probabilities reach 2^SLACK instead of 1, which
+    // costs none of their bits, and the accumulators are multiplied in a row's first steps instead of in most of them (8100 tokens of
+    // 32 heads on 8: 724 → 705 µs, 2048: 79 → 76)
+    constexpr float SLACK = 8.f;
     float m_run[MT];
     float4v o_acc[MT][DT], l_acc[MT];
 #pragma unroll
@@ -835,10 +839,9 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn64_kernel(AttnArgs p
 #pragma unroll
             for (int q = 1; q < 4; q++) mx = fmaxf(mx, fmaxf(fmaxf(sv[mt][q][0], sv[mt][q][1]), fmaxf(sv[mt][q][2], sv[mt][q][3])));
             mx = rows_reduce_max(mx * sl2);                       // sl2 > 0: the maximum commutes with the scaling
-            const float m_new = fmaxf(m_run[mt], mx);
-            const float m_safe = m_new == -INFINITY ? 0.f : m_new;
-            if (__ballot(m_new != m_run[mt]) != 0) {              // wave-uniform: some row's maximum moved
-                const float alpha = __builtin_amdgcn_exp2f(m_run[mt] - m_safe);
+            if (__ballot(mx > m_run[mt] + SLACK) != 0) {          // wave-uniform: some row's maximum has left the range of its reference
+                const float m_new = fmaxf(m_run[mt], mx);
+                const float alpha = __builtin_amdgcn_exp2f(m_run[mt] - (m_new == -INFINITY ? 0.f : m_new));
 #pragma unroll
                 for (int dt = 0; dt < DT; dt++)
 #pragma unroll
@@ -847,6 +850,7 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn64_kernel(AttnArgs p
                 for (int r = 0; r < 4; r++) l_acc[mt][r] *= alpha;
                 m_run[mt] = m_new;
             }
+            const float m_safe = m_run[mt] == -INFINITY ? 0.f : m_run[mt];
 #pragma unroll
             for (int j = 0; j < 2; j++)
 #pragma unroll

@@ -969,6 +969,35 @@ def test_prompt_attention_takes_the_shared_form_by_size(env, nq, nkv, q_lens, po
     assert nmse(outs[1], outs[0]) < 1e-5
 
 
+@pytest.mark.parametrize("rows", [64, 128])
+@pytest.mark.parametrize("rise", [0.05, 0.12, 0.6, -0.05])
+def test_prompt_attention_of_rising_scores(env, rise, rows, forms, knobs):
+    """Maxima that stay within the range of a row's reference for some steps, leave it now and then or in every step, or fall; four keys of 700
+    are hidden behind -inf."""
+    pkg, B, ctx, O, torch = env
+    knobs.set(ATTN_FLASH_ROWS=rows, ATTN_FLASH_MIN_ROWS=1)
+    T, nq, nkv = 700, 4, 2
+    mb = (T + 15) // 16
+    gen = torch.Generator("cuda").manual_seed(5)
+    q, k, v = (torch.randn(n, T, 128, generator=gen, device="cuda").half() for n in (nq, nkv, nkv))
+    q[:, :, 0], k[:, :, 0] = 16.0, torch.arange(T, device="cuda") * (rise * 128 ** 0.5 / 16)          # a score of rise x position (nepers)
+    k[:, 100:104, 0] = -float("inf")
+    ck, cv = _fill_pool(env, [host(k.transpose(0, 1))], [host(v.transpose(0, 1))], np.arange(mb, dtype=np.int32)[None], [T], nkv, 128, mb)
+    out = torch.empty(T, nq, 128, dtype=torch.float16, device="cuda")
+    B.paged_varlen_attention(ctx, q.transpose(0, 1).contiguous(), ck, cv, out, torch.tensor([0, T], dtype=torch.int32, device="cuda"),
+                             torch.zeros(1, dtype=torch.int32, device="cuda"), torch.arange(mb, dtype=torch.int32, device="cuda")[None], 1, T, T, nq, nkv, 128, 0, 16, mb, T)
+    ctx.sync()
+    forms.require("attn_flash")
+    for h in range(nq):
+        s = q[h].double() @ k[h // 2].double().T * 128 ** -0.5
+        p = s.masked_fill(torch.ones_like(s, dtype=torch.bool).triu(1), -float("inf")).softmax(-1)
+        want, size = p @ v[h // 2].double(), p @ v[h // 2].double().abs()
+        # 16-bit probabilities in numerator and denominator (2^-11 each), scores of up to 420 in 32 bits (128 roundings of 2^-24 of their terms'
+        # size), probabilities below 2^-14 (2^-25 each), the result
+        bound = (2.0 ** -10 + 2 ** -24 * 128 * s.abs().nan_to_num(posinf=0).amax() / 4) * size + T * 2.0 ** -25 * 5 + 2.0 ** -11 * want.abs()
+        assert ((out[:, h].double() - want).abs() <= bound).all()
+
+
 def test_paged_prefill_attention_lds_shared_kv_many_sequences(env, knobs, forms):
     """The flash form over 70 sequences (two passes of its in-kernel sequence lookup), two of them empty."""
     pkg, B, ctx, O, torch = env
