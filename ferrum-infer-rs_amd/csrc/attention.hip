@@ -40,7 +40,7 @@ struct AttnArgs {
     const uint32_t* kv_lens;        // decode form: [num_seqs] kv length incl. the new token (pos = len-1)
     const int32_t* block_tables;    // [num_seqs, max_blocks]
     float* partial;         // [tiles][nsplit][16][hd+2] when nsplit > 1
-    int num_seqs, nq, nkv, tiles_per_seq, max_blocks, sliding_window, nsplit;
+    int num_seqs, nq, nkv, tiles_per_seq, max_blocks, sliding_window, nsplit, units;
     int compact;            // grid.x enumerates real work units of a ragged batch (see the kernel), not num_seqs × tiles_per_seq
     float scale;
     // fused decode form (FUSED_QKV): q / new K / new V come straight from the qkv projection output
@@ -671,11 +671,26 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn64_kernel(AttnArgs p
     __half* lds_kv = reinterpret_cast<__half*>(smem);          // [2 stages][2 pairs][K0, K1, V0, V1][TILE]; reused by the epilogue
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
-    const int kvh = blockIdx.y;
+    // workgroup → (kv head, unit): workgroups go to the XCDs in turn, and a head's units are taken on one XCD (on 8 / nkv of them with fewer
+    // heads), whose L2 holds the keys of 8000 tokens.  Dealt over all XCDs every L2 saw every head, and a step waited for the last-level
+    // cache (8100 tokens of 32 heads on 8 705 → 590 µs, 2048 76 → 62; 1500 and 548 of 16 on 8 47.6 → 42.5).
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    int kvh, from_last;
+    if ((p.nkv & 7) == 0) {
+        kvh = xcd + 8 * (slot / p.units);
+        from_last = slot % p.units;
+    } else if ((8 % p.nkv) == 0) {
+        kvh = xcd % p.nkv;
+        from_last = slot * (8 / p.nkv) + xcd / p.nkv;
+    } else {
+        kvh = blockIdx.x / p.units;
+        from_last = blockIdx.x % p.units;
+    }
+    if (from_last >= p.units) return;
     const int G = p.nq / p.nkv;
     int seq = -1, unit = 0;
     {
-        const int w = gridDim.x - 1 - blockIdx.x;       // launch order reversed: the longest key ranges (last units of a causal prompt) start first
+        const int w = p.units - 1 - from_last;       // launch order reversed: the longest key ranges (last units of a causal prompt) start first
         int base = 0;
         for (int s0 = 0; s0 < p.num_seqs; s0 += 64) {
             const int s = s0 + lane;
@@ -1226,17 +1241,19 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
         return 0;
     }
     // head_dim 128 has two sizes of workgroup.  128 rows read K/V from LDS half as often, 64 rows make twice the workgroups and half of a step's
-    // vector work in each; two workgroups of either share a CU.  The line lies where 128 rows, less of a round of 512 as they are, have the less
-    // work in all: at 360 of them, at 300 under a window, which leaves every workgroup as many keys.  Over 840 batches between 256 and 512 that
-    // choice is 2 % from the faster of the two, always 64 rows 4 %, always 128 5 %.
+    // vector work in each; two workgroups of either share a CU.  The longest keys of a prompt are a workgroup's alone, and 64 rows pass them
+    // in 0.65 of the time, until there are rounds enough to hide that: 64 rows below 620 workgroups of 128.  Where a window or a context of
+    // more than 1.5 times the new tokens leaves every workgroup about as many keys, below 360.  Over 230 batches between 256 and 2300 that
+    // choice is 1.2 % from the faster of the two (128 rows take up to 1.6 times as long below 500, 64 rows 1.3 times from 1000 on).
     // µs, row-split or KV-split form / 64 rows / 128 rows (workgroups of 128 rows × kv heads)
-    //   8B heads (32 on 8)    1 × 8100 (2024)      2372 / 919 / 779      1 × 2048 (512)        196 / 95 / 82     1 × 1024 (256)         62 / 33 / 37
-    //                         1 × 700 (175)          32 / 25 / 28        1 × 500 (125)          19 / 17 / 24     1 × 300 (75)           11 / 11 / 17
-    //   16 on 8               1500 and 548 (256)     82 / 46 / 63        293, 1389, 366 (256)   87 / 48 / 62     1 × 986 at 366 (123)   49 / 35 / 54
-    //                         6 × 100, 1400 (250)    80 / 39 / 53        1 × 500 (62)           14 / 16 / 24
+    //   8B heads (32 on 8)    1 × 8100 (2024)      2372 / 750 / 587      1 × 2048 (512)        196 / 69 / 64     1 × 1024 (256)         62 / 27 / 32
+    //                         1 × 2180 (545)            - / 75 / 90      1 × 700 (175)          32 / 22 / 31     1 × 500 (125)          19 / 16 / 20
+    //   16 on 8               1500 and 548 (256)     82 / 43 / 62        293, 1389, 366 (256)   87 / 40 / 56     1 × 986 at 366 (123)   49 / 36 / 50
+    //                         6 × 100, 1400 (250)    80 / 38 / 84        1 × 500 (62)           14 / 14 / 15     1 × 4360 on 32 (1090)   - / 244 / 190
     // A batch qualifies where most of its sequences bring many rows, or they bring 256 on average.
     const long rows_heads = (long)total_q_tokens * G * num_kv_heads;
-    const bool two_sizes = head_dim == 128 && !kn.attn_flash32, half_units = two_sizes && (kn.attn_flash_rows ? kn.attn_flash_rows == 64 : rows_heads < (sliding_window > 0 && max_kv_len > sliding_window ? 300 : 360) * 128);
+    const bool two_sizes = head_dim == 128 && !kn.attn_flash32, even = (sliding_window > 0 && max_kv_len > sliding_window) || (long)max_kv_len * 2 >= (long)max_q_len * 5;
+    const bool half_units = two_sizes && (kn.attn_flash_rows ? kn.attn_flash_rows == 64 : rows_heads < (even ? 360 : 620) * 128);
     const bool flash_fits = (long)total_q_tokens * 2 >= (long)num_seqs * max_q_len || (two_sizes && (long)total_q_tokens * G >= (long)num_seqs * 256);
     if (!fq && cu_seqlens_q && !flash_off && (long)max_q_len * G >= flash_min_rows && flash_fits &&
         rows_heads / (half_units || head_dim == 256 ? 64 : 128) >= (half_units && !kn.attn_flash_min_rows_set ? 192 : flash_min_wgs)) {
@@ -1263,8 +1280,10 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
                 FH_CHECK_HIP(hipFuncSetAttribute((const void*)paged_prefill_attn64_kernel<128, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64));
                 attr64 = true;
             }
-            if (mt == 1) hipLaunchKernelGGL((paged_prefill_attn64_kernel<128, 1>), grid, dim3(256), lds64, s, a);
-            else hipLaunchKernelGGL((paged_prefill_attn64_kernel<128, 2>), grid, dim3(256), lds64, s, a);
+            a.units = (int)units;
+            const dim3 flat((unsigned)(num_kv_heads < 8 && 8 % num_kv_heads == 0 ? 8 * cdiv(units, 8 / num_kv_heads) : units * num_kv_heads));
+            if (mt == 1) hipLaunchKernelGGL((paged_prefill_attn64_kernel<128, 1>), flat, dim3(256), lds64, s, a);
+            else hipLaunchKernelGGL((paged_prefill_attn64_kernel<128, 2>), flat, dim3(256), lds64, s, a);
         } else if (head_dim == 128) FH_FLASH(128, 2) else if (head_dim == 64) FH_FLASH(64, 2) else FH_FLASH(256, 1)
 #undef FH_FLASH
         FH_CHECK_LAUNCH();
