@@ -2205,7 +2205,7 @@ __global__ __launch_bounds__(256, 2) void w4_gemm_tilep_kernel(W4Args p) {
 // k-half's operands are expanded between the MFMAs of the current one; activations global → registers → LDS one group ahead,
 // weights two groups ahead.
 // MODE 0 dense; 1 / 2 the MoE grouped GEMM over MT·16-row align blocks (rows gathered through sorted_token_ids, the block's
-// expert from block_ids; 2 = gate_up with the silu·mul epilogue), tiles dealt to the XCDs like w4_gemm_tile_kernel's; 3 / 4 dense gate_up
+// expert from block_ids; 2 = gate_up with the silu·mul epilogue); 3 / 4 dense gate_up
 // whose wave pairs two gate tiles with their up tiles and stores silu / gelu(gate)·up, rounded as the two launches
 // round: the projection's [rows, 2·im] is not written and read again (8100 × 28672 × 4096 and its activation, a layer: 1490 + 200 → 1553 µs).
 template <int MT, bool HAS_ZP, int MODE = 0>
@@ -2218,13 +2218,16 @@ __global__ __launch_bounds__(256, MT <= 6 ? 2 : 1) void w4_gemm_big_kernel(W4Arg
     typedef uint32_t u32x4g __attribute__((ext_vector_type(4)));
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
-    int ct = blockIdx.x, rb = blockIdx.y;
-    if (MOE) {        // each XCD walks a contiguous range of (column tile, row block), row block fastest: one expert's blocks meet its weights in one L2
-        const int nwg = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y;
-        const int xcd = lin & 7, virt = xcd * (nwg >> 3) + min(xcd, nwg & 7) + (lin >> 3);
-        ct = virt / (int)gridDim.y;
-        rb = virt % (int)gridDim.y;
-    }
+    // Each XCD walks a contiguous range of tiles, row block fastest.  MoE: over all row blocks, so that one expert's meet its weights in one L2.
+    // Dense: over bands of up to BAND row blocks; what an XCD's CUs read in a step is then a few row blocks (64 KiB each) and a few column tiles
+    // (16), not, as with 16 column tiles in launch order, two of these and all row blocks there are: 8100 rows 4096 → 4096 252 → 241 µs,
+    // 14336 → 4096 795 → 763, 4096 → 6144 370 → 359, 4096 → 28672 1472 → 1464; 4096 rows 4096 → 2048 80 → 74 (bands of 2 the same, of 8 1 – 2 % slower).
+    constexpr int BAND = 4;
+    const int nwg = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y;
+    const int xcd = lin & 7, virt = xcd * (nwg >> 3) + min(xcd, nwg & 7) + (lin >> 3);
+    const int rows_n = gridDim.y, band = MOE ? rows_n : cdiv_dev(rows_n, cdiv_dev(rows_n, BAND));
+    const int band0 = virt / (band * (int)gridDim.x) * band, band_h = min(band, rows_n - band0);
+    const int in_band = virt - band0 * (int)gridDim.x, ct = in_band / band_h, rb = band0 + in_band % band_h;
     const int st_raw = ct * 4 + wave;
     const bool st_ok = st_raw < p.n64;
     const int st = st_ok ? st_raw : p.n64 - 1;

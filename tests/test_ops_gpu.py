@@ -306,6 +306,28 @@ def test_prefill_tiles_at_any_address(env, mt, n, shift, knobs, forms):
     assert np.all(got[:shift] == 7.0) and np.all(got[shift + m * n:] == 7.0)
 
 
+@pytest.mark.parametrize("blocks,n", [(1, 200), (4, 64), (5, 1480), (6, 520), (9, 264), (13, 712)])
+def test_w4_big_tiles_in_bands(env, blocks, n, knobs, forms):
+    """Bands of row blocks that divide their number and not, one column tile and several, fewer tiles than XCDs and no multiple of them: each
+    tile is taken once."""
+    pkg, B, ctx, O, torch = env
+    k, m = 256, max(128, 128 * blocks - 3)
+    qw, sc, qz = O.make_synthetic_gptq(k, n, 128, 3, symmetric=True)
+    sc = f16r(sc / (0.28 * np.sqrt(k)))
+    lin = pkg.GptqLinear.from_raw(qw, sc, qz, None, None, 4, 128, k, n)
+    knobs.set(W4_BIG=8)
+    x = f16r(np.random.default_rng(m).standard_normal((m, k)))
+    out = torch.full((m + 1, n), 7.0, dtype=torch.float16, device="cuda")
+    forms.reset()
+    lin.forward(ctx, dev16(torch, x), out, m)
+    ctx.sync()
+    forms.require("w4_big")
+    ref, got = O.gemm(x, O.dequant_gptq(qw, sc, qz, 128, k, n), m, n, k), host(out)
+    for r in range(0, m, 128):
+        assert nmse(ref[r:r + 128], got[r:min(r + 128, m)]) < NMSE_FP16_TOL, r
+    assert np.all(got[m] == 7.0)
+
+
 @pytest.mark.parametrize("f32out", [False, True])
 @pytest.mark.parametrize("m,n,k", [(1, 64, 32), (16, 4096, 1024), (17, 96, 1056), (64, 1024, 3072), (65, 8192, 32), (100, 6176, 96), (200, 2080, 64),
                                    (129, 16416, 160), (300, 4128, 2080), (1100, 1056, 352), (2049, 4096, 128), (3000, 8224, 64), (9, 14400, 2080), (16, 16416, 4128),
