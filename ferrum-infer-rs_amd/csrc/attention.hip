@@ -795,10 +795,9 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn64_kernel(AttnArgs p
     };
 
     const float sl2 = p.scale * 1.4426950408889634f;
-    // A row's reference m_run stays until its maximum is more than SLACK (log2 units) above: probabilities reach 2^SLACK instead of 1, which
-    // costs none of their bits, and the accumulators are multiplied in a row's first steps instead of in most of them (8100 tokens of
-    // 32 heads on 8: 724 → 705 µs, 2048: 79 → 76)
-    constexpr float SLACK = 8.f;
+    // A row's reference m_run is its largest score so far, whose probability then is exactly 1.  (Left up to 2^8 behind, which saves most
+    // multiplications of the accumulators and 0 – 3 % of a launch (8100 tokens of 32 heads on 8: 578 µs for 591, 2048: 66 both), it makes the
+    // largest probabilities round like any other: 1.16 and 1.20 times the error of P·V for 1536 keys with scores of deviation 2 and 4.)
     float m_run[MT];
     float4v o_acc[MT][DT], l_acc[MT];
 #pragma unroll
@@ -854,9 +853,10 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn64_kernel(AttnArgs p
 #pragma unroll
             for (int q = 1; q < 4; q++) mx = fmaxf(mx, fmaxf(fmaxf(sv[mt][q][0], sv[mt][q][1]), fmaxf(sv[mt][q][2], sv[mt][q][3])));
             mx = rows_reduce_max(mx * sl2);                       // sl2 > 0: the maximum commutes with the scaling
-            if (__ballot(mx > m_run[mt] + SLACK) != 0) {          // wave-uniform: some row's maximum has left the range of its reference
-                const float m_new = fmaxf(m_run[mt], mx);
-                const float alpha = __builtin_amdgcn_exp2f(m_run[mt] - (m_new == -INFINITY ? 0.f : m_new));
+            const float m_new = fmaxf(m_run[mt], mx);
+            const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+            if (__ballot(m_new != m_run[mt]) != 0) {              // wave-uniform: some row's maximum moved
+                const float alpha = __builtin_amdgcn_exp2f(m_run[mt] - m_safe);
 #pragma unroll
                 for (int dt = 0; dt < DT; dt++)
 #pragma unroll
@@ -865,7 +865,6 @@ __global__ __launch_bounds__(256, 2) void paged_prefill_attn64_kernel(AttnArgs p
                 for (int r = 0; r < 4; r++) l_acc[mt][r] *= alpha;
                 m_run[mt] = m_new;
             }
-            const float m_safe = m_run[mt] == -INFINITY ? 0.f : m_run[mt];
 #pragma unroll
             for (int j = 0; j < 2; j++)
 #pragma unroll

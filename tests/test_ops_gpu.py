@@ -994,8 +994,7 @@ def test_prompt_attention_takes_the_shared_form_by_size(env, nq, nkv, q_lens, po
 @pytest.mark.parametrize("rows", [64, 128])
 @pytest.mark.parametrize("rise", [0.05, 0.12, 0.6, -0.05])
 def test_prompt_attention_of_rising_scores(env, rise, rows, forms, knobs):
-    """Maxima that stay within the range of a row's reference for some steps, leave it now and then or in every step, or fall; four keys of 700
-    are hidden behind -inf."""
+    """Maxima that move a little or far in every step, or never; four keys of 700 are hidden behind -inf."""
     pkg, B, ctx, O, torch = env
     knobs.set(ATTN_FLASH_ROWS=rows, ATTN_FLASH_MIN_ROWS=1)
     T, nq, nkv = 700, 4, 2
@@ -1018,6 +1017,44 @@ def test_prompt_attention_of_rising_scores(env, rise, rows, forms, knobs):
         # size), probabilities below 2^-14 (2^-25 each), the result
         bound = (2.0 ** -10 + 2 ** -24 * 128 * s.abs().nan_to_num(posinf=0).amax() / 4) * size + T * 2.0 ** -25 * 5 + 2.0 ** -11 * want.abs()
         assert ((out[:, h].double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("rows", [64, 128])
+@pytest.mark.parametrize("spread", [1.0, 2.0, 4.0])
+def test_prompt_attention_errs_as_its_rounded_probabilities(env, spread, rows, forms, knobs):
+    """Keys in pairs whose values all but cancel, so that what is left of a result shows the rounding of its probabilities: no more of it than with each probability
+    divided by the row's largest so far, which then is exactly 1.  The arithmetic beside that rounding is 32-bit (scores err by about 1e-6 of themselves, against 2.8e-4
+    for a rounding), so the two errors agree to a few percent; with a reference 2^8 behind the maximum the first is 1.16 and 1.20 times the second at deviations of 2 and 4."""
+    pkg, B, ctx, O, torch = env
+    knobs.set(ATTN_FLASH_ROWS=rows, ATTN_FLASH_MIN_ROWS=1)
+    T, nq, nkv = 1536, 4, 2
+    mb = T // 16
+    gen = torch.Generator("cuda").manual_seed(11)
+    q, k, v = (torch.randn(n, T, 128, generator=gen, device="cuda") for n in (nq, nkv, nkv))
+    q, k = (q * spread ** 0.5).half(), (k * spread ** 0.5).half()
+    q[:, :, 0] = 16.0
+    k[:, 1::2] = k[:, ::2]
+    k[:, ::2, 0], k[:, 1::2, 0] = 0.0, 0.1 + 0.6 * torch.rand(nkv, T // 2, generator=gen, device="cuda").half()
+    v[:, 1::2] = -v[:, ::2] * torch.exp(k[:, 1::2, :1].float() * -16 * 128 ** -0.5)
+    v = v.half()
+    ck, cv = _fill_pool(env, [host(k.transpose(0, 1))], [host(v.transpose(0, 1))], np.arange(mb, dtype=np.int32)[None], [T], nkv, 128, mb)
+    out = torch.empty(T, nq, 128, dtype=torch.float16, device="cuda")
+    B.paged_varlen_attention(ctx, q.transpose(0, 1).contiguous(), ck, cv, out, torch.tensor([0, T], dtype=torch.int32, device="cuda"),
+                             torch.zeros(1, dtype=torch.int32, device="cuda"), torch.arange(mb, dtype=torch.int32, device="cuda")[None], 1, T, T, nq, nkv, 128, 0, 16, mb, T)
+    ctx.sync()
+    forms.require("attn_flash")
+    got = allowed = 0.0
+    for h in range(nq):
+        s = q[h].double() @ k[h // 2].double().T * 128 ** -0.5
+        s = s.masked_fill(torch.ones_like(s, dtype=torch.bool).triu(1), -float("inf"))
+        value = v[h // 2].double()
+        largest = s.reshape(T, -1, 64).amax(-1).cummax(-1).values.repeat_interleave(64, -1)          # (a step takes 64 keys)
+        p = (s - largest).exp().half().double() * (largest - largest[:, -1:]).exp()
+        want = s.softmax(-1) @ value
+        whole = slice(1, None, 2)                                   # (rows that see both keys of their last pair)
+        got += ((out[:, h].double() - want)[whole] ** 2).sum().item()
+        allowed += ((p @ value / p.sum(-1, keepdim=True) - want)[whole] ** 2).sum().item()
+    assert got <= 1.05 ** 2 * allowed, (got / allowed) ** 0.5
 
 
 def test_paged_prefill_attention_lds_shared_kv_many_sequences(env, knobs, forms):
