@@ -839,19 +839,20 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
         for (int ks = 0; ks < 8; ks++) if (ks < ksplit) l += lp[ks];
     }
     const int keep = top_k < EQ ? top_k : EQ;
+    const float lc = route_logit(l);
     float mx = wave_reduce_max(l), sm;
     int rank = 0;
     if (EQ <= 64) {
         // one wave has them all
         if (wave != 0) return;
         sm = wave_reduce_sum((t < EQ && e_glob < num_experts) ? expf(l - mx) : 0.f);
-        rank = route_rank(route_key(l, t), EQ);
-        if (t < EQ && rank < keep) cand_s[rank] = ((unsigned long long)(unsigned)e_glob << 32) | __float_as_uint(l);
+        rank = route_rank(route_key(lc, t), EQ);
+        if (t < EQ && rank < keep) cand_s[rank] = ((unsigned long long)(unsigned)e_glob << 32) | __float_as_uint(lc);
         if (t >= keep && t < 8) cand_s[t] = (0x7fffffffull << 32) | __float_as_uint(-INFINITY);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __builtin_amdgcn_wave_barrier();
     } else {
-        if (t < EQ) lgs[t] = l;
+        if (t < EQ) lgs[t] = lc;
         if (lane == 0) red[wave] = mx;
         __syncthreads();
         mx = fmaxf(red[0], red[1]);
@@ -862,9 +863,9 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
         if (t < EQ) {
             for (int j = 0; j < EQ; j++) {
                 const float lj = lgs[j];
-                rank += (lj > l || (lj == l && j < t)) ? 1 : 0;
+                rank += (lj > lc || (lj == lc && j < t)) ? 1 : 0;
             }
-            if (rank < keep) cand_s[rank] = ((unsigned long long)(unsigned)e_glob << 32) | __float_as_uint(l);
+            if (rank < keep) cand_s[rank] = ((unsigned long long)(unsigned)e_glob << 32) | __float_as_uint(lc);
         }
         if (t >= keep && t < 8) cand_s[t] = (0x7fffffffull << 32) | __float_as_uint(-INFINITY);
         __syncthreads();

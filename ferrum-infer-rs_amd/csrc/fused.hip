@@ -11,6 +11,7 @@
 // argmax-mask passes with lowest-index ties).
 #include "common.h"
 #include "kernels.h"
+#include "route_merge.h"
 
 namespace fh {
 
@@ -155,14 +156,14 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_route_kernel(
     __syncthreads();
     // sequential-ish order (wave partials 0..7) — fp32, within the 1e-6 weight tolerance of router.rs:219-222
     sm = ((red[0] + red[1]) + (red[2] + red[3])) + ((red[4] + red[5]) + (red[6] + red[7]));
-    const float p_mine = ex * (1.0f / sm);
-    if (t < tiles * 16) prob[t] = t < num_experts ? p_mine : -INFINITY;
+    const float p_mine = ex * (1.0f / sm), p_order = route_logit(p_mine);
+    if (t < tiles * 16) prob[t] = t < num_experts ? p_order : -INFINITY;
     __syncthreads();
     if (t < num_experts) {
         int rank = 0;
         for (int j = 0; j < num_experts; j++) {
             float pj = prob[j];
-            rank += (pj > p_mine || (pj == p_mine && j < t)) ? 1 : 0;
+            rank += (pj > p_order || (pj == p_order && j < t)) ? 1 : 0;
         }
         if (rank < top_k) { sel_w[rank] = p_mine; sel_id[rank] = t; }
     }
@@ -366,7 +367,8 @@ __global__ __launch_bounds__(512) void add_rmsnorm_route_part_kernel(
         for (int ks = 0; ks < ksplit; ks++) l += part[ks * EQ + t];
         if (logits_out) logits_out[row * num_experts + e_glob] = l;
     }
-    if (t < EQ) lgs[t] = l;
+    const float lc = route_logit(l);
+    if (t < EQ) lgs[t] = lc;
     // part statistics (EQ ≤ 128 → waves 0,1)
     float mx = wave_reduce_max(l);
     if (lane == 0) red[wave] = mx;
@@ -381,9 +383,9 @@ __global__ __launch_bounds__(512) void add_rmsnorm_route_part_kernel(
         int rank = 0;
         for (int j = 0; j < EQ; j++) {
             float lj = lgs[j];
-            rank += (lj > l || (lj == l && j < t)) ? 1 : 0;
+            rank += (lj > lc || (lj == lc && j < t)) ? 1 : 0;
         }
-        if (rank < keep) cand_s[rank] = ((unsigned long long)(unsigned)e_glob << 32) | __float_as_uint(l);
+        if (rank < keep) cand_s[rank] = ((unsigned long long)(unsigned)e_glob << 32) | __float_as_uint(lc);
     }
     if (t >= keep && t < 8) cand_s[t] = (0x7fffffffull << 32) | __float_as_uint(-INFINITY);   // unused slots of a short list
     __syncthreads();

@@ -8,6 +8,9 @@
 
 namespace fh {
 
+// A logit as the selection takes it: a NaN counts as −∞, behind every number, so that each expert has a place of its own in its part's list and none is
+// left to a slot that nothing was written to, or to an unused one, whose id no expert has.  (The softmax's sums take the NaN itself.)
+__device__ __forceinline__ float route_logit(float l) { return l > -INFINITY ? l : -INFINITY; }
 // The order of the selection as one number, the larger first: logits as unsigned numbers of the same order (−0 as 0), then the lower id
 __device__ __forceinline__ unsigned long long route_key(float logit, int id) {
     const unsigned u = __float_as_uint(logit + 0.0f);

@@ -939,6 +939,33 @@ def test_decode_chain_attention_kv_splits(pkg, forms, knobs, window):
                 assert srt[r, -1] - srt[r, -2] <= 2 * err[r] + 1e-6, (other, s, int(r))
 
 
+@pytest.mark.parametrize("bits", [0x7e00, 0xfe00])
+@pytest.mark.parametrize("c", [1, 2, 9])
+def test_decode_chain_of_a_router_with_nan(pkg, c, bits, forms, knobs):
+    """A router row of NaN, of either sign: the merged launch chooses as the launches of their own do, among the other experts (the sum of all
+    weights being NaN, those of the chosen are equal), in the launch and in the next one's prologue."""
+    tm = _chain_model()
+    kept = [L["dense"]["router"] for L in tm.layers]
+    try:
+        for i, L in enumerate(tm.layers):
+            L["dense"]["router"] = kept[i].copy()
+            L["dense"]["router"][[5, 77]] = np.array([bits], np.uint16).view(np.float16).astype(np.float32)
+        out = {}
+        for chain in (1, 0):
+            knobs.set(DECODE_CHAIN=chain, MOE_EM2=chain)
+            hm = tm.hip_model(pkg, kv_num_blocks=c * 2 + 4, max_seqs=c, max_tokens=64)
+            hm.unified_forward([(i, [7 + i, 300, 21], 0, True) for i in range(c)], greedy=True)
+            forms.reset()
+            out[chain] = hm.unified_forward([(i, [50 + i], 3, True) for i in range(c)], greedy=True, want_logits=True)[1]
+            assert forms.hits().get("decode_chain", 0) == (3 if chain else 0), forms.hits()
+            del hm
+    finally:
+        for L, router in zip(tm.layers, kept):
+            L["dense"]["router"] = router
+    assert np.isfinite(out[0]).all()
+    assert np.abs(out[1] - out[0]).max() < 0.02 * np.abs(out[0]).max()
+
+
 @pytest.mark.parametrize("c", [1, 4, 8, 9, 16, 17])
 def test_decode_chain_of_wide_layers(pkg, c, forms):
     """Hidden 4096: four quant groups a wave in the q|k|v role (two for hidden 2048), its blocks 32 columns wide up to the rows at which they and

@@ -1597,6 +1597,33 @@ def test_route_split_in_launch_merge_equals_route_topk(env, tokens, H, E, K, Q, 
         assert np.max(np.abs(wts.cpu().numpy() - rwt_ref)) < 1e-6
 
 
+@pytest.mark.parametrize("sign", ["+", "-"])
+@pytest.mark.parametrize("bad", ["one", "some", "all"])
+@pytest.mark.parametrize("tokens,H,E,K,Q", [(3, 1024, 128, 8, 4), (9, 512, 64, 4, 2), (2, 512, 16, 2, 1), (5, 512, 128, 8, 1)])
+def test_router_logits_that_are_nan_come_last(env, tokens, H, E, K, Q, bad, sign):
+    """Every place of a choice is an expert's, each expert once: with NaN among the logits, of either sign, those are behind all numbers in the split router, and make
+    all probabilities of the single kernel NaN, which then takes the first experts."""
+    pkg, B, ctx, O, torch = env
+    gen = torch.Generator("cuda").manual_seed(E + K)
+    rnd = lambda *s: torch.randn(*s, generator=gen, device="cuda").half()
+    r, x, w, rw = rnd(tokens, H), rnd(tokens, H), rnd(H), rnd(E, H) * 0.05
+    which = {"one": [E // 2], "some": list(range(0, E, 3)), "all": slice(None)}[bad]
+    rw.view(torch.int16)[which] = 0x7e00 if sign == "+" else 0x7e00 - 0x8000
+    rwt = B.dense_repack_f16t(ctx, rw, E, H)
+    cand, stats = torch.zeros(tokens * Q * 16, dtype=torch.int32, device="cuda"), torch.zeros(tokens * Q * 2, device="cuda")
+    nd, lg, arrive = torch.empty_like(x), torch.empty(tokens, E, device="cuda"), torch.zeros(tokens, dtype=torch.int32, device="cuda")
+    ids, wts = (torch.full((2, tokens, K), -1, dtype=t, device="cuda") for t in (torch.int32, torch.float32))
+    B.fused_add_rms_norm_route_split(ctx, r, torch.empty_like(r), x, None, 0, 0, H, w, 1e-6, nd, rwt, E, K, 1, Q, cand, stats, arrive, ids[0], wts[0], lg, tokens, H)
+    B.fused_add_rms_norm_route(ctx, r.clone(), x, w, 1e-6, nd, rwt, E, K, True, ids[1], wts[1], None, tokens, H)
+    ctx.sync()
+    assert lg.isnan().sum() == rw.isnan().any(1).sum() * tokens
+    order = torch.where(lg.isnan(), -float("inf"), lg).sort(dim=1, descending=True, stable=True).indices[:, :K]
+    assert torch.equal(ids[0].long(), order)
+    assert torch.equal(ids[1].long(), torch.arange(K, device="cuda").expand(tokens, K))
+    lists = cand.reshape(tokens, Q, 8, 2)[:, :, :min(K, E // Q), 1].flatten(1)
+    assert all(len(set(row)) == len(row) and max(row) < E for row in lists.tolist())
+
+
 @pytest.mark.parametrize("tokens,H,K,with_norm", [(1, 2048, 8, True), (32, 2048, 8, True), (7, 1024, 2, False)])
 def test_moe_combine_add_rms_norm_equals_op_chain(env, tokens, H, K, with_norm):
     pkg, B, ctx, O, torch = env
