@@ -163,7 +163,13 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(FewRows f, TiledGemm<E>
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
-    if (s0 < s1) load(bw[0], 0, s0);
+    // The part's loads are taken from a chunk of its own on, in a circle.  Where K is a multiple of a high power of two all waves' weights begin at the same
+    // address modulo that power, and waves that go on in step ask the same few channels of the memory (µs from the first chunk on → so:
+    // 8 × 4096 × 8192 16.1 → 12.9, 8 × 8192 × 4096 16.4 → 14.2, 1 × 2048 × 16384 in four slabs 16.1 → 14.3; K that are no such multiple ± 1 %).
+    const int len = s1 - s0, chunks = len > 0 && len % U == 0 ? len / U : 1;
+    const int turn = ((blockIdx.x * f.cw + cg + part + z) & ((chunks & -chunks) - 1)) * U;
+    auto place = [&](int i) { i += turn; return s0 + (i < len ? i : i - len); };
+    if (len > 0) load(bw[0], 0, place(0));
     const GemmSection sec = gemm_section(p, n0);
     floatx4 bias[J], acc[MT][J];
 #pragma unroll
@@ -203,12 +209,12 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(FewRows f, TiledGemm<E>
     // 32 bits: sums of 128 products, then sums of those (relative error at K = 2048 / 8736: 2.1 / 2.2e-7, parts summed whole 2.9 / 3.8e-7; no slower)
     constexpr bool F32 = sizeof(E) == 4;
     floatx4 sums[F32 ? MT : 1][F32 ? J : 1] = {};
-    if (s0 < s1) {
-        int s = s0;
-        for (; s + 2 * U < s1; s += 2 * U) {
-            load(bw[1], 1, s + U);
+    if (len > 0) {
+        int i = 0;
+        for (; i + 2 * U < len; i += 2 * U) {
+            load(bw[1], 1, place(i + U));
             mul(bw[0], 0, behind{}, U);
-            load(bw[0], 0, s + 2 * U);
+            load(bw[0], 0, place(i + 2 * U));
             mul(bw[1], 1, behind{}, U);
             if constexpr (F32)
 #pragma unroll
@@ -217,12 +223,12 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(FewRows f, TiledGemm<E>
                     acc[t / J][t % J] = (floatx4){0.f, 0.f, 0.f, 0.f};
                 }
         }
-        if (s + U < s1) {
-            load(bw[1], 1, s + U);
+        if (i + U < len) {
+            load(bw[1], 1, place(i + U));
             mul(bw[0], 0, behind{}, U);
-            mul(bw[1], 1, last{}, s1 - s - U);
+            mul(bw[1], 1, last{}, len - i - U);
         } else {
-            mul(bw[0], 0, last{}, s1 - s);
+            mul(bw[0], 0, last{}, len - i);
         }
         if constexpr (F32)
 #pragma unroll
@@ -686,7 +692,13 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     //   3 × 128 × 8128             8.88                  7.53               12.0       11.9            2.0
     //   8 × 6144 × 1024            4.83       4.58       4.90                4.79                      3.7
     //   7 × 6528 × 6912           17.3       18.8                           16.4       16.9           14.8
-    //   8 × 2048 × 8192, 4 slabs   8.96       9.4        8.72                           7.93           6.5
+    //   8 × 2048 × 7680, 4 slabs   7.74       7.68       7.94                7.86       8.03
+    //   8 × 2048 × 8192, 4 slabs   7.74       8.12       8.04                7.98       8.20           6.5
+    //   8 × 2048 × 9216, 4 slabs   8.54       8.49       9.57                8.70       9.43
+    //   16 × 5120 × 1536           6.81       6.55       7.38                5.96       6.60
+    //   16 × 5120 × 2048           7.88       7.56       8.09                7.03       7.15
+    //   8 × 8192 × 2048            7.83       7.84       8.29                8.21       8.27
+    //   16 × 8192 × 3072          11.46      11.64      11.76               11.18      11.49
     //   8 × 12288 × 1024           6.35       6.70       6.65                                          5.3
     //   1 × 10240 × 2048           9.34       9.39       8.93               10.3                       7.8
     //   8 × 20032 × 2048          15.4                  14.97               16.3       15.7           13.6
@@ -695,8 +707,8 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     //   60 × 8192 × 2048                     12.5                           10.6                       6.5
     //   43 × 9600 × 1920          18.0                                      16.5 (K in 2: 14.1)        7.3
     // One row tile: 16 columns, since a wave then has half as much under way before its first sum; K in four up to a round of 256 workgroups
-    // and past two, in two between, where that saves a round, unless the parts of a long K get longer than the second round costs; eight waves
-    // where a wave of four would read 16 loads and more.  Several row tiles: their rows are read again for every column group, so 32 columns
+    // and past two, in two between, where that saves a round, up to the 64 loads (of a slab's K) from which on parts of a half get too long and 32 columns
+    // in four parts save it; eight waves where a wave of four would read 16 loads and more.  Several row tiles: their rows are read again for every column group, so 32 columns
     // past one round.  Four row tiles leave room for one workgroup per CU, two with 64 columns for two: the parts that make rounds / parts least.
     // A vocabulary, many rounds of workgroups: the rows' share grows with rows and K (µs; 64 columns: with two row tiles and K in one part)
     //                             16 columns, 8 waves   32 columns, 8 waves   32 columns, 4 waves   64 columns
@@ -709,16 +721,15 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     const int rbs = rows.id ? rows.max_blocks : cdiv(g.m, 16 * mt), zs = rows.id ? 1 : g.groups * g.slabs;
     const int loads = g.k / (F32 ? 16 : 32) / g.slabs;                  // (of a wave that has all of a slab's K)
     const long tiles16 = (long)rbs * (g.n / 16) * zs;
-    const bool two_rounds = !rows.id && tiles16 > 256 && tiles16 <= 512, longer = loads > 64 || (loads == 64 && g.slabs > 1);
+    const bool two_rounds = !rows.id && tiles16 > 256 && tiles16 <= 512;
     const bool ext = rows.id || g.x_blocks || g.col_scale || gated || rare, wide = !rows.id && tiles16 > 2048;
-    int J = rows.id ? 2 : mt == 1 ? ((two_rounds && longer) || (wide && (g.m > 12 || loads > 128)) ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
+    int J = rows.id ? 2 : mt == 1 ? ((two_rounds && loads >= 64) || (wide && (g.m > 12 || loads > 128)) ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
     if (mt == 2 && wide && loads >= 128 && !ext && g.n % 64 == 0) J = 4;
     if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : 2;
     if (gated) J = 2;
     const long cols = g.n / (16 * J), blocks = (long)rbs * cols * zs;
     int nw = mt == 1 && !rows.id && ((blocks > 512 && loads >= 64) || (blocks <= 256 && J == 1 && loads >= 96)) ? 8 : 4, kw = nw;
     if (J == 1 && two_rounds) kw = 2;
-    if (two_rounds && g.slabs > 1 && loads == 64 && mt < 4) nw = kw = 8;
     if (mt == 4 && rows.id) kw = 2;                                     // (64 tokens, 24 experts, blocks of 64, 2048 × 2048: in four 55, in two 48)
     else if (mt == 4 && (long)rbs * cdiv(cols, 4) * zs > 128) kw = 1;
     else if (mt == 4 || J == 4)

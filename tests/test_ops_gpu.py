@@ -472,6 +472,24 @@ def test_few_rows_of_every_count(env, m, n, k, j, kw, knobs, forms):
     assert (buf[:n] == 7.0).all() and (buf[n + m * n:] == 7.0).all()
 
 
+@pytest.mark.parametrize("n,k", [(4096, 8192), (8192, 8192), (8192, 4096)])
+def test_few_rows_of_a_power_of_two(env, n, k, knobs):
+    """A K whose rows of weights all begin at the same place among the memory's channels takes about as long as one that is a little longer; weights from memory, not from
+    the caches."""
+    pkg, B, ctx, O, torch = env
+    took = []
+    for kk in (k, k + 160):
+        a, out = torch.randn(8, kk, device="cuda").half(), torch.empty(8, n, dtype=torch.float16, device="cuda")
+        copies = torch.randn((700 << 20) // (2 * n * kk), n, kk, dtype=torch.float16, device="cuda")          # (tiles of some weights)
+
+        def call(c):
+            for w in copies:
+                B.gemm_f16t(c, a, w, out, 8, n, kk)
+        took.append(_times(env, knobs, call, {"chosen": {}})["chosen"] / len(copies))
+        del copies
+    assert took[0] < 1.15 * took[1], took
+
+
 @pytest.mark.parametrize("nq,nkv,tokens,pos,seqs,window", [(32, 4, 64, 700, 24, 0), (14, 2, 4096, 0, 1, 512), (32, 8, 700, 0, 1, 0)])
 def test_prompt_attention_takes_the_faster_unit(env, nq, nkv, tokens, pos, seqs, window, knobs):
     """Batches on both sides of the line between units of 64 and 128 rows, where the wrong one costs 12 to 40 %."""
