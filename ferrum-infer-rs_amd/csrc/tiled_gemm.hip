@@ -725,7 +725,7 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     const bool ext = rows.id || g.x_blocks || g.col_scale || gated || rare, wide = !rows.id && tiles16 > 2048;
     int J = rows.id ? 2 : mt == 1 ? ((two_rounds && loads >= 64) || (wide && (g.m > 12 || loads > 128)) ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
     if (mt == 2 && wide && loads >= 128 && !ext && g.n % 64 == 0) J = 4;
-    if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : 2;
+    if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : knobs().tiled_j == 4 && mt == 2 && !ext && g.n % 64 == 0 ? 4 : 2;
     if (gated) J = 2;
     const long cols = g.n / (16 * J), blocks = (long)rbs * cols * zs;
     int nw = mt == 1 && !rows.id && ((blocks > 512 && loads >= 64) || (blocks <= 256 && J == 1 && loads >= 96)) ? 8 : 4, kw = nw;
@@ -746,7 +746,10 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
 #define SMALL(J_, EXT_) \
     (mt == 1 ? launch_small<E, 1, J_, EXT_>(g, grid, nw, kw, s) : mt == 2 ? launch_small<E, 2, J_, EXT_>(g, grid, nw, kw, s) : launch_small<E, 4, J_, EXT_>(g, grid, nw, kw, s))
     if (ext) return J == 1 ? SMALL(1, true) : SMALL(2, true);
-    if (J == 4) return launch_small<E, 2, 4, false>(g, grid, nw, kw, s);
+    if (J == 4) {
+        form_hit(FORM_TILED_GEMM_COLS64);
+        return launch_small<E, 2, 4, false>(g, grid, nw, kw, s);
+    }
     return J == 1 ? SMALL(1, false) : SMALL(2, false);
 #undef SMALL
 }

@@ -457,16 +457,35 @@ def test_projections_take_the_faster_side_of_a_line(env, m, n, k, knobs):
 def test_few_rows_of_every_count(env, m, n, k, j, kw, knobs, forms):
     """Rows that fill no load and no tile, parts of K of no, one and several chunks that end within one, column groups past the last tile.  Against 64 bits: an fp32 sum
     of K exact products errs by K x 2^-24 of the sum of their magnitudes at most, and fp16 rounds by 2^-11."""
-    pkg, B, ctx, O, torch = env
     knobs.set(TILED_J=j, TILED_NW=8 if kw == 8 else 4, TILED_KW=kw, TILED_BIG_MIN_TILES=10 ** 6)
+    _few_rows(env, m, n, k)
+    forms.require("tiled_gemm")
+
+
+@pytest.mark.parametrize("kw", [1, 2, 4, 8])
+@pytest.mark.parametrize("j", [1, 2, 4])
+@pytest.mark.parametrize("m,n,k", [(17, 64, 32), (18, 320, 96), (23, 192, 768), (28, 64, 1120), (29, 576, 1024), (32, 128, 4128), (33, 64, 544), (50, 320, 768), (64, 192, 1056)])
+def test_few_rows_of_several_row_tiles(env, m, n, k, j, kw, knobs, forms):
+    """The same with two and four row tiles a workgroup, which sizes as small as these would not take, and up to 64 columns a wave; parts of several chunks that are taken in a
+    circle and that are not."""
+    knobs.set(TILED_J=j, TILED_NW=8 if kw == 8 else 4, TILED_KW=kw, TILED_BIG_MIN_TILES=10 ** 6, TILED_MIN_TILES=-1)
+    _few_rows(env, m, n, k)
+    forms.require("tiled_gemm", *(["tiled_gemm_cols64"] if j == 4 and m <= 32 else []))
+
+
+def test_wide_outputs_take_64_columns_a_wave(env, forms):
+    _few_rows(env, 17, 32832, 4128)
+    forms.require("tiled_gemm_cols64")
+
+
+def _few_rows(env, m, n, k):
+    pkg, B, ctx, O, torch = env
     gen = torch.Generator("cuda").manual_seed(m * n + k)
     a, b = (torch.randn(r, k, generator=gen, device="cuda").half() for r in (m, n))
     buf = torch.full(((m + 2) * n,), 7.0, dtype=torch.float16, device="cuda")
     out = buf[n:n + m * n]
-    forms.reset()
     B.gemm_f16t(ctx, a, B.dense_repack_f16t(ctx, b, n, k), out, m, n, k)
     ctx.sync()
-    forms.require("tiled_gemm")
     want, size = a.double() @ b.double().T, a.double().abs() @ b.double().abs().T
     assert ((out.reshape(m, n).double() - want).abs() <= 2.0 ** -11 * want.abs() + k * 2.0 ** -24 * size + 2.0 ** -25).all()
     assert (buf[:n] == 7.0).all() and (buf[n + m * n:] == 7.0).all()
