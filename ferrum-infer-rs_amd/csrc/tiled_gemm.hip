@@ -710,25 +710,33 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     // and past two, in two between, where that saves a round, up to the 64 loads (of a slab's K) from which on parts of a half get too long and 32 columns
     // in four parts save it; eight waves where a wave of four would read 16 loads and more.  Several row tiles: their rows are read again for every column group, so 32 columns
     // past one round.  Four row tiles leave room for one workgroup per CU, two with 64 columns for two: the parts that make rounds / parts least.
-    // A vocabulary, many rounds of workgroups: the rows' share grows with rows and K (µs; 64 columns: with two row tiles and K in one part)
-    //                             16 columns, 8 waves   32 columns, 8 waves   32 columns, 4 waves   64 columns
-    //   8 × 128256 × 4096             154                                         > 160
-    //   8 × 131072 × 5376             226                    205                   205
-    //   16 × 151936 × 2048            117                     95                    98
-    //   32 × 131072 × 5376                                                         275                  231
-    //   32 × 151936 × 2048                                                         108                  117
+    // A vocabulary, many rounds of workgroups (those of 17 – 32 rows on more than 139000 columns do not come here: f16t_gemm): the rows' share grows with rows
+    // and K, so wider blocks; eight waves, each with whole chunks, else four.  µs:
+    //                             16 columns, 8 waves   32 columns, 8 waves   32 columns, 4 waves   64 columns, K in parts by the rule
+    //   8 × 128256 × 4096             154                    156                   167
+    //   12 × 128256 × 4096            167                    159                   173
+    //   12 × 151936 × 2048            105                     95                    93
+    //   12 × 262208 × 5376            498                    437                   431
+    //   16 × 262208 × 5376            554                    463                   448
+    //   32 × 49152 × 8192                                    143                   138                   159
+    //   24 × 65536 × 2048                                     54                    45                    48
+    //   32 × 65536 × 2048                                     56                    47                    48
+    //   17 × 98304 × 3072                                    103                    94                    95
+    //   32 × 98304 × 3072                                    121                   110                   101
+    //   32 × 131072 × 1536                                   104                    84                    74
+    //   32 × 131072 × 5376                                   295                   273                   232
     //   64 × 151936 × 1024, 32 columns, K in four parts 97, in one 79; 49 × 16992 × 1376: 20.8 and 19.5
     const int rbs = rows.id ? rows.max_blocks : cdiv(g.m, 16 * mt), zs = rows.id ? 1 : g.groups * g.slabs;
     const int loads = g.k / (F32 ? 16 : 32) / g.slabs;                  // (of a wave that has all of a slab's K)
     const long tiles16 = (long)rbs * (g.n / 16) * zs;
     const bool two_rounds = !rows.id && tiles16 > 256 && tiles16 <= 512;
     const bool ext = rows.id || g.x_blocks || g.col_scale || gated || rare, wide = !rows.id && tiles16 > 2048;
-    int J = rows.id ? 2 : mt == 1 ? ((two_rounds && loads >= 64) || (wide && (g.m > 12 || loads > 128)) ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
-    if (mt == 2 && wide && loads >= 128 && !ext && g.n % 64 == 0) J = 4;
+    int J = rows.id ? 2 : mt == 1 ? ((two_rounds && loads >= 64) || (wide && (g.m > 12 || (g.m > 8 && loads >= 48) || loads > 128)) ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
+    if (mt == 2 && !ext && tiles16 >= 4096 && loads >= (g.m > 24 ? 48 : 96) && g.n % 64 == 0) J = 4;
     if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : knobs().tiled_j == 4 && mt == 2 && !ext && g.n % 64 == 0 ? 4 : 2;
     if (gated) J = 2;
     const long cols = g.n / (16 * J), blocks = (long)rbs * cols * zs;
-    int nw = mt == 1 && !rows.id && ((blocks > 512 && loads >= 64) || (blocks <= 256 && J == 1 && loads >= 96)) ? 8 : 4, kw = nw;
+    int nw = mt == 1 && !rows.id && ((blocks > 512 && loads >= 64 && (!wide || loads % 32 == 0)) || (blocks <= 256 && J == 1 && loads >= 96)) ? 8 : 4, kw = nw;
     if (J == 1 && two_rounds) kw = 2;
     if (mt == 4 && rows.id) kw = 2;                                     // (64 tokens, 24 experts, blocks of 64, 2048 × 2048: in four 55, in two 48)
     else if (mt == 4 && (long)rbs * cdiv(cols, 4) * zs > 128) kw = 1;

@@ -3368,11 +3368,12 @@ int f16t_repack(const __half* w_rowmajor, __half* out_tiled, int n, int k, hipSt
 }
 size_t f16t_elems(int n, int k) { return (size_t)cdiv(n, 16) * 16 * k; }
 
-template <int MT, typename OutT>
+// J = 16-column tiles of a wave: 2, or 4 for two row tiles against a vocabulary (with 2 the fragments of the rows, which a wave reads for every column group, are
+// as many bytes as the weights)
+template <int MT, typename OutT, int J = 2>
 __global__ __launch_bounds__(256) void f16t_gemm_kernel(const __half* __restrict__ x, const __half* __restrict__ wt,
                                                         OutT* __restrict__ out, float* __restrict__ partial, int M, int N,
                                                         int K, int S, int rows_pad, int n_pad) {
-    constexpr int J = 2;                            // 16-column tiles of a wave
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
     const int ntile2 = blockIdx.x * 4 + wave;       // group of J 16-column tiles
@@ -3455,7 +3456,19 @@ static int f16t_gemm_impl(const __half* x, const __half* wt, OutT* out, int m, i
     // The projections of the layered models (tiled_gemm.hip) read the same weight tiles: prompts in LDS tiles (2048 × 4096 × 1024: 115 → 24 µs), few
     // rows with theirs in LDS and K split over the waves of a workgroup (8 × 4096 × 1024: 12 → 3.8; 8 × 151936 × 1024 55 → 48, 1 × 128256 × 4096 170 → 152,
     // 48 × 128256 × 4096 278 → 207).
-    if (n % 32 == 0 && ((uintptr_t)x & 15) == 0) {
+    // What stays here of them, f16t_gemm_kernel against the best form there (µs; without LDS a workgroup has more of its loads' issue, and reads all of K):
+    //  * 17 – 32 rows on many workgroups of 4 × 64 columns:
+    //                          17 rows        24             32                                  17 rows        24             32
+    //      135168 × 3072      146 | 139      148 | 143      150 | 145        262208 × 2048    160 | 167      161 | 175      163 | 177
+    //      143360 × 4096      183 | 193      184 | 197      190 | 204        262208 × 4096    338 | 352      340 | 362      340 | 373
+    //      151936 × 2048       94 |  95       96 | 101      100 | 104        262208 × 5376    410 | 446      422 | 463      489 | 484
+    //      151936 × 4096      192 | 204      196 | 217      203 | 226        151936 × 1024     60 |  51       61 |  53       62 |  55
+    //    so it takes them from 544 workgroups and K beyond 1024 on; 200064 – 229376 × 2048 would be 4 – 14 % faster there.
+    //  * 9 – 16 rows where its workgroups of 4 × 32 columns all but fill a round of four per CU, and K is long: 128256 × 5376, 12 rows 198 | 208, 16 rows
+    //    201 | 215 (114688 × 5376 180 | 180, 132096 255 | 211; 128256 × 4096 161 | 163, × 8192 315 | 322).
+    const bool rows32 = m > 16 && m <= 32 && n % 64 == 0 && k > 1024 && cdiv(n, 256) >= 544;
+    const bool rows16 = m > 8 && m <= 16 && k > 4096 && cdiv(n, 128) > 944 && cdiv(n, 128) <= 1024;
+    if (n % 32 == 0 && ((uintptr_t)x & 15) == 0 && !rows32 && !rows16) {
         TiledGemm<_Float16> g;
         g.x = reinterpret_cast<const _Float16*>(x); g.ldx = k; g.w = reinterpret_cast<const _Float16*>(wt);
         g.m = m; g.n = n; g.k = k; g.ldo = n;
@@ -3463,7 +3476,7 @@ static int f16t_gemm_impl(const __half* x, const __half* wt, OutT* out, int m, i
         else g.out_f32 = out;
         return tiled_gemm(g, stream);
     }
-    // What reaches this: an N that is no multiple of 32 (a router of few experts, a shard of odd width) and, through the entry point, an x without
+    // Besides: an N that is no multiple of 32 (a router of few experts, a shard of odd width) and, through the entry point, an x without
     // 16-byte alignment.
     int mt = m <= 16 ? 1 : (m <= 32 ? 2 : 4);
     int row_blocks = cdiv(m, 16 * mt);
@@ -3474,6 +3487,11 @@ static int f16t_gemm_impl(const __half* x, const __half* wt, OutT* out, int m, i
     while (tasks * S < 2048 && S * 2 <= ksteps / 8) S *= 2;
     int rows_pad = row_blocks * 16 * mt, n_pad = ntile2 * 32;
     if (S > 1 && (size_t)S * rows_pad * n_pad * sizeof(float) > workspace_bytes) S = 1;
+    if (mt == 2 && S == 1 && n >= 32768 && n % 64 == 0) {
+        hipLaunchKernelGGL((f16t_gemm_kernel<2, OutT, 4>), dim3(cdiv(n, 256), row_blocks), dim3(256), 0, stream, x, wt, out, workspace, m, n, k, 1, rows_pad, n_pad);
+        FH_CHECK_LAUNCH();
+        return 0;
+    }
     dim3 grid(cdiv(ntile2, 4), row_blocks, S);
     if (mt == 1) hipLaunchKernelGGL((f16t_gemm_kernel<1, OutT>), grid, dim3(256), 0, stream, x, wt, out, workspace, m, n, k, S, rows_pad, n_pad);
     else if (mt == 2) hipLaunchKernelGGL((f16t_gemm_kernel<2, OutT>), grid, dim3(256), 0, stream, x, wt, out, workspace, m, n, k, S, rows_pad, n_pad);

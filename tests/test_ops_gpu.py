@@ -473,9 +473,12 @@ def test_few_rows_of_several_row_tiles(env, m, n, k, j, kw, knobs, forms):
     forms.require("tiled_gemm", *(["tiled_gemm_cols64"] if j == 4 and m <= 32 else []))
 
 
-def test_wide_outputs_take_64_columns_a_wave(env, forms):
-    _few_rows(env, 17, 32832, 4128)
-    forms.require("tiled_gemm_cols64")
+@pytest.mark.parametrize("m,n,k,form", [(30, 65600, 1568, "tiled_gemm_cols64"), (17, 65600, 3104, "tiled_gemm_cols64"), (20, 139328, 1056, None), (32, 139264, 1056, None), (12, 120960, 4128, None),
+                                        (12, 120832, 4128, "tiled_gemm"), (32, 139008, 1056, "tiled_gemm"), (10, 65568, 2080, "tiled_gemm"), (15, 32800, 96, "tiled_gemm")])
+def test_vocabularies_on_both_sides_of_a_line(env, m, n, k, form, knobs, forms):
+    """What is chosen for a wide output: 64 columns a wave, or the kernel that holds no rows in LDS where that is the faster one."""
+    _few_rows(env, m, n, k)
+    assert form in forms.hits() if form else "tiled_gemm" not in forms.hits(), forms.hits()
 
 
 def _few_rows(env, m, n, k):
