@@ -738,7 +738,17 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     const long cols = g.n / (16 * J), blocks = (long)rbs * cols * zs;
     int nw = mt == 1 && !rows.id && ((blocks > 512 && loads >= 64 && (!wide || loads % 32 == 0)) || (blocks <= 256 && J == 1 && loads >= 96)) ? 8 : 4, kw = nw;
     if (J == 1 && two_rounds) kw = 2;
-    if (mt == 4 && rows.id) kw = 2;                                     // (64 tokens, 24 experts, blocks of 64, 2048 × 2048: in four 55, in two 48)
+    // Sorted rows, 32 columns: K in as many parts as there are waves, until workgroups are so many that the parts' sums and their waits only add.  µs in
+    // 4 | 2 | 1 part, tokens of 8 experts each × columns × K (blocks of 32 columns):
+    //   16 rows a block    8 of 8: 4 of 64 × 4096 × 1536 (4096)   54 |  53 |  56       160 of 128 × 4096 × 1536 (26624)  257 | 248 | 249
+    //                      in 8:   16 of 24 × 8192 × 4096 (8192) 258 | 246 | 244, 240   48 of 64 × 4096 × 4096 (11264)   341 | 333 | 326, 323
+    //   32 rows            16 of 8 × 2048 × 512 (768)            6.8 | 7.0 | 8.6        100 of 64 × 2048 × 512 (5696)   38.5 | 29.3 | 27.0
+    //                      200 of 128 × 2048 × 512 (11392)        72 |  56 |  52        200 of 128 × 4096 × 1536 (22784) 273 | 250 | 251
+    //                      200 of 64 × 1536 × 2048 (5472)         73 |  88 |  84
+    //   64 rows            32 of 8 × 1024 × 2048 (384)          11.1 | 15.1 | 24.3      64 of 24 × 2048 × 2048 (2048)      55 | 48 | 49
+    //                      600 of 128 × 4096 × 1536 (25984)      466 | 402 | 373
+    if (rows.id && mt == 1 && loads >= 96) nw = kw = 8;
+    else if (rows.id) kw = mt == 1 ? (blocks < 20000 ? 4 : 1) : mt == 2 ? (blocks < 4096 ? 4 : 1) : blocks < 512 ? 4 : blocks < 3000 ? 2 : 1;
     else if (mt == 4 && (long)rbs * cdiv(cols, 4) * zs > 128) kw = 1;
     else if (mt == 4 || J == 4)
         for (int k : {2, 1}) {

@@ -103,6 +103,19 @@ def test_experts_of_long_prompts(pkg, tmp_path, forms, knobs, block, dtype):
     assert bool(h.get("tiled_gemm_grouped")) == (dtype == "float32" or block <= 64)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("block,nw,kw", [(16, 8, 8), (16, 8, 2), (16, 4, 4), (16, 4, 1), (32, 4, 4), (32, 4, 1), (64, 4, 4), (64, 4, 2), (64, 4, 1)])
+def test_experts_in_every_split(pkg, tmp_path, forms, knobs, block, nw, kw, dtype):
+    """Few sorted rows: every number of waves and of parts of K, with parts of several chunks, of a fraction of one and of nothing."""
+    knobs.set(MOE_ROWS_BLOCK=block, TILED_NW=nw, TILED_KW=kw, TILED_BIG_MIN_TILES=10 ** 6)
+    for n, top, tokens, ff, width in ((6, 3, 70, 48, 1056), (9, 2, 40, 250, 96)):
+        cfg = model([G.sink_attention(2, 8, 4, 8, 16, mlp=G.experts(n, top, ff))], width=width)
+        w = G.weights(cfg, 47)
+        silence(w, "mix.o", "side.norm")
+        agree(pkg, tmp_path / str(n), cfg, w, dtype, n=tokens)
+    assert forms.hits().get("tiled_gemm_grouped") and not forms.hits().get("tiled_gemm_grouped_big")
+
+
 @pytest.mark.parametrize("block", [128, 256])
 @pytest.mark.parametrize("size", SIZES)
 def test_experts_in_every_tile_size(pkg, tmp_path, forms, knobs, size, block):
