@@ -13,7 +13,7 @@
 namespace fh {
 
 // One expert a lane (64 at most), top_k of them by their place among all rather than one after the other: a maximum over the wave costs as much as
-// ten comparisons with a lane's value.  (A launch of 32 tokens, two a wave, on 24 experts in 8 groups of 3, top 8: 19 → 11 µs, of which
+// six comparisons with a lane's value.  (A launch of 32 tokens, two a wave, on 24 experts in 8 groups of 3, top 8: 19 → 11 µs, of which
 // 7.4 the choice; two tokens on 30, one group: 7.7 → 6.1; bound by the instructions of 16 waves on one CU, with few tokens by their latency.)
 // place: how many of the first `n` lanes hold a larger v, the lower lane first on ties; −∞ and NaN are behind all and have no place (≥ 64)
 __device__ __forceinline__ int route_place(float v, int lane, int n) {
@@ -29,7 +29,9 @@ __device__ __forceinline__ int route_place(float v, int lane, int n) {
         }
     return in ? place : 64;
 }
-__device__ __forceinline__ bool route_by_place(int per_lane, int num_experts, int top_k) { return per_lane == 1 && num_experts <= 8 * top_k; }
+// Comparisons come in eights.  µs of a launch of 32 tokens, maxima | places: 32 experts, 8 of them 3.43 | 3.01, 6 3.19 | 3.08, 4 2.85 | 3.04; 48, 8 3.42 | 3.37,
+// 6 3.18 | 3.42; 24, 4 2.86 | 2.86, 3 2.77 | 2.93; 64, 8 3.45 | 3.76.
+__device__ __forceinline__ bool route_by_place(int per_lane, int num_experts, int top_k) { return per_lane == 1 && (num_experts + 7) / 8 * 8 <= 6 * top_k; }
 // lane k < top_k: what the lane of place k has, `none` where no lane has it
 template <typename T>
 __device__ __forceinline__ T route_at_place(T x, int place, int lane, int top_k, T none) {

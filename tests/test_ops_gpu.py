@@ -1251,9 +1251,9 @@ def test_route_ties_lowest_index(env):
 
 
 @pytest.mark.parametrize("norm", [False, True])
-@pytest.mark.parametrize("ne,k", [(1, 1), (2, 1), (7, 7), (8, 2), (9, 1), (24, 8), (31, 4), (40, 5), (41, 5), (63, 8), (64, 8), (64, 64), (65, 8)])
+@pytest.mark.parametrize("ne,k", [(1, 1), (2, 1), (7, 7), (8, 2), (9, 1), (24, 4), (24, 8), (25, 4), (31, 4), (40, 5), (41, 5), (48, 8), (49, 8), (63, 8), (64, 8), (64, 64), (65, 8)])
 def test_route_by_place_and_by_maxima(env, ne, k, norm):
-    """Up to eight experts a choice are ranked at once, more by one maximum after the other: numbers, ties, -inf and NaN among the logits, against k passes of a maximum in
+    """Up to six experts a choice, counted in eights, are ranked at once, more by one maximum after the other: numbers, ties, -inf and NaN among the logits, against k passes of a maximum in
     which a NaN takes no part, the first expert standing in where none is left."""
     pkg, B, ctx, O, torch = env
     rng = np.random.default_rng(ne * 64 + k)
