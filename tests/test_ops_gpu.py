@@ -65,7 +65,7 @@ def test_layer_norm_and_gelu_core_ops(env, tokens, dim):
     assert nmse(O.gelu(x), host(out)) < NMSE_FP16_TOL
 
 
-@pytest.mark.parametrize("tokens,dim", [(1, 1024), (5, 2048), (32, 4096), (3, 5376), (2, 8192), (7, 128)])
+@pytest.mark.parametrize("tokens,dim", [(1, 1024), (5, 2048), (32, 4096), (3, 5376), (2, 8192), (7, 128), (256, 2056), (257, 2056), (300, 8192), (260, 16384), (513, 136)])
 def test_rms_norm_and_fused_add(env, tokens, dim):
     pkg, B, ctx, O, torch = env
     rng = np.random.default_rng(dim + tokens)
