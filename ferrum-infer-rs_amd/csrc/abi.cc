@@ -50,7 +50,7 @@ void reload_knobs() {
     k.chain_split_keys = env_int("FERRUM_HIP_CHAIN_SPLIT_KEYS", 256);
     k.chain_attn_splits = env_int("FERRUM_HIP_CHAIN_ATTN_SPLITS", 0);
     k.route_gemm_topk = env_int("FERRUM_HIP_ROUTE_GEMM_TOPK", 1);
-    k.tiled_big_min_tiles = env_int("FERRUM_HIP_TILED_BIG_MIN_TILES", 0);
+    k.tiled_big_min_tiles = env_int("FERRUM_HIP_TILED_BIG_MIN_TILES", -1);
     k.tiled_wide_min_tiles = env_int("FERRUM_HIP_TILED_WIDE_MIN_TILES", 257);
     k.tiled_min_tiles = env_int("FERRUM_HIP_TILED_MIN_TILES", 128);
     k.tiled_half_max_tiles = env_int("FERRUM_HIP_TILED_HALF_MAX_TILES", 256);

@@ -57,7 +57,7 @@ struct Knobs {
     int lds_min_wgs = 128;
     int lds_min_groups = 8;
     // layered models (tiled_gemm.hip, latent_attention.hip, grouped_attention.hip, linear_attention.hip, rglru.hip)
-    int tiled_big_min_tiles = 0;      // > 0: projections of > 64 rows take the tile kernel from this many tiles of 64 × 64 (0: from 193, in 32 bits 129)
+    int tiled_big_min_tiles = -1;     // ≥ 0: projections of > 64 rows take the tile kernel from this many tiles of 64 × 64 (32-bit: and one); −1: from 193, in 32 bits 129
     int tiled_wide_min_tiles = 257;   // … and in 16 bits its 128 × 256 form from this many tiles of that size
     int tiled_min_tiles = 128;        // few-row kernel: rows of a workgroup are halved until there are this many row × 16-column tiles (16-bit: up to twice as many)
     int tiled_half_max_tiles = 256;   // … its 128 × 64 and 64 × 64 forms up to this many tiles of 128 × 128

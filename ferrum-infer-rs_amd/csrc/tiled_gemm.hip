@@ -677,7 +677,7 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     }
     constexpr bool F32 = sizeof(E) == 4;
     const long tiles = (rows.id ? (long)rows.max_blocks * (rows.block / 64) : cdiv(g.m, 64)) * cdiv(g.n, 64) * g.groups;
-    const bool enough_tiles = tiles >= (knobs().tiled_big_min_tiles > 0 ? knobs().tiled_big_min_tiles : F32 ? 129 : 193);
+    const bool enough_tiles = tiles >= (knobs().tiled_big_min_tiles >= 0 ? knobs().tiled_big_min_tiles + F32 : F32 ? 129 : 193);
     if (rows.id ? (F32 ? rows.block >= 64 && g.n >= 64 && enough_tiles : rows.block >= 128) : g.m > 64 && g.n >= 64 && g.slabs == 1 && enough_tiles) return launch_big(g, s);
     // Rows of a workgroup: as many as there are, fewer where narrow outputs would leave CUs idle: in 16 bits as long as a round of 256 workgroups
     // holds the launch.

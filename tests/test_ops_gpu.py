@@ -481,6 +481,14 @@ def test_vocabularies_on_both_sides_of_a_line(env, m, n, k, form, knobs, forms):
     assert form in forms.hits() if form else "tiled_gemm" not in forms.hits(), forms.hits()
 
 
+@pytest.mark.parametrize("tiles,form", [(0, "tiled_gemm_big"), (2, "tiled_gemm_big"), (3, "tiled_gemm"), (None, "tiled_gemm")])
+def test_tile_kernel_from_a_given_number_of_tiles(env, tiles, form, knobs, forms):
+    """Two tiles of 64 x 64: a number asked for, 0 among them, or the rule."""
+    knobs.set(TILED_BIG_MIN_TILES=tiles)
+    _few_rows(env, 65, 64, 64)
+    assert set(forms.hits()) & {"tiled_gemm", "tiled_gemm_big"} == {form}
+
+
 def _few_rows(env, m, n, k):
     pkg, B, ctx, O, torch = env
     gen = torch.Generator("cuda").manual_seed(m * n + k)
