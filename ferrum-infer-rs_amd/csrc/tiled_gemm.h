@@ -95,7 +95,7 @@ struct TiledGemm {
 };
 template <typename E> int tiled_gemm(const TiledGemm<E>& g, hipStream_t s);
 // number of K parts worth making for a projection of m rows whose consumer sums slabs (≤ GEMM_MAX_SLABS)
-constexpr int GEMM_MAX_SLABS = 8;
+constexpr int GEMM_MAX_SLABS = 4;
 int tiled_gemm_slabs(int m, int n, int k);
 
 // Activations on fp32 accumulators.  Models in 16 bits round the result to 2⁻⁹ or 2⁻¹², so their form uses the hardware exponential and

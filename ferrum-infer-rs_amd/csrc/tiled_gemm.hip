@@ -623,9 +623,13 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
 
 int tiled_gemm_slabs(int m, int n, int k) {
     if (m > 64) return 1;
-    // narrow outputs: enough (column group, K part) workgroups to cover the chip, two k-steps or more per wave
+    // Narrow outputs: slabs until 32 columns of one of them for each CU, 1024 of K in two.  µs of the launch and the norm that sums its slabs, bf16, one slab | two |
+    // four | eight:
+    //   1 × 1024 × 4096    7.7 |  6.9 |  6.3 |  7.3      8 × 1536 × 4096    9.3 |  8.3 |  8.1 | 10.4      64 × 1024 × 2048    7.4 |  7.3 |  7.7 |  9.4
+    //   8 × 2048 × 8192   12.9 | 10.9 | 10.9 | 12.2     16 × 2048 × 12288  20.5 | 14.6 | 14.1 | 16.4      64 × 2048 × 8192   18.4 | 16.9 | 14.9 | 17.2
+    //   1 × 2048 × 1024    5.9 |  6.0 |  6.0 |  7.1      8 × 3072 × 4096   10.1 | 10.3 | 10.0 | 11.5      32 × 4096 × 4096   14.0 | 13.3 | 13.9 | 17.4
     int S = 1;
-    while (S < GEMM_MAX_SLABS && (n / 32) * S < 256 && k / 32 >= 2 * 8 * 2 * S) S *= 2;
+    while (S < GEMM_MAX_SLABS && (n / 32) * S < 256 && k >= 1024 * S) S *= 2;
     return S;
 }
 
