@@ -699,10 +699,15 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     //   8 × 2048 × 7680, 4 slabs   7.74       7.68       7.94                7.86       8.03
     //   8 × 2048 × 8192, 4 slabs   7.74       8.12       8.04                7.98       8.20           6.5
     //   8 × 2048 × 9216, 4 slabs   8.54       8.49       9.57                8.70       9.43
-    //   16 × 5120 × 1536           6.81       6.55       7.38                5.96       6.60
-    //   16 × 5120 × 2048           7.88       7.56       8.09                7.03       7.15
+    //   8 × 4096 × 3072, 2 slabs   6.59       6.52       7.15                6.84       7.13
+    //   8 × 4096 × 4096, 2 slabs   7.72       9.40       8.16                8.10       8.35
+    //   8 × 5120 × 1024            4.74       4.88       5.21                4.61       4.83
+    //   8 × 5120 × 1536            5.99       5.67       6.43                5.56       6.02
+    //   16 × 6144 × 2048           7.96       7.95       8.31                7.50       7.62
     //   8 × 8192 × 2048            7.83       7.84       8.29                8.21       8.27
+    //   8 × 8192 × 3072           10.29      10.32      10.58               10.75      10.77
     //   16 × 8192 × 3072          11.46      11.64      11.76               11.18      11.49
+    //   8 × 8192 × 5120           15.34      15.79      15.75               15.90      16.12
     //   8 × 12288 × 1024           6.35       6.70       6.65                                          5.3
     //   1 × 10240 × 2048           9.34       9.39       8.93               10.3                       7.8
     //   8 × 20032 × 2048          15.4                  14.97               16.3       15.7           13.6
@@ -711,8 +716,9 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     //   60 × 8192 × 2048                     12.5                           10.6                       6.5
     //   43 × 9600 × 1920          18.0                                      16.5 (K in 2: 14.1)        7.3
     // One row tile: 16 columns, since a wave then has half as much under way before its first sum; K in four up to a round of 256 workgroups
-    // and past two, in two between, where that saves a round, up to the 64 loads (of a slab's K) from which on parts of a half get too long and 32 columns
-    // in four parts save it; eight waves where a wave of four would read 16 loads and more.  Several row tiles: their rows are read again for every column group, so 32 columns
+    // and past two, in two between, where that saves a round, until parts of a half get too long: 32 columns in four parts save the round too, and take
+    // over at 48 loads of a wave with all of K where the second round is less than three quarters full, at 80 where it is fuller, at 64 of a
+    // slab's; eight waves where a wave of four would read 16 loads and more.  Several row tiles: their rows are read again for every column group, so 32 columns
     // past one round.  Four row tiles leave room for one workgroup per CU, two with 64 columns for two: the parts that make rounds / parts least.
     // A vocabulary, many rounds of workgroups (those of 17 – 32 rows on more than 139000 columns do not come here: f16t_gemm): the rows' share grows with rows
     // and K, so wider blocks; eight waves, each with whole chunks, else four.  µs:
@@ -735,7 +741,7 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     const long tiles16 = (long)rbs * (g.n / 16) * zs;
     const bool two_rounds = !rows.id && tiles16 > 256 && tiles16 <= 512;
     const bool ext = rows.id || g.x_blocks || g.col_scale || gated || rare, wide = !rows.id && tiles16 > 2048;
-    int J = rows.id ? 2 : mt == 1 ? ((two_rounds && loads >= 64) || (wide && (g.m > 12 || (g.m > 8 && loads >= 48) || loads > 128)) ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
+    int J = rows.id ? 2 : mt == 1 ? ((two_rounds && loads >= (tiles16 < 448 ? 48 : g.slabs > 1 ? 64 : 80)) || (wide && (g.m > 12 || (g.m > 8 && loads >= 48) || loads > 128)) ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
     if (mt == 2 && !ext && tiles16 >= 4096 && loads >= (g.m > 24 ? 48 : 96) && g.n % 64 == 0) J = 4;
     if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : knobs().tiled_j == 4 && mt == 2 && !ext && g.n % 64 == 0 ? 4 : 2;
     if (gated) J = 2;
