@@ -54,10 +54,17 @@ int embed_tokens(const Embedding<E>& e, const BatchView& v, float* x, E* xb, int
     return 0;
 }
 
+// AT_ONCE: the waves' sums read together, for launches whose time is latency; of many rows the loop is no slower and leaves 16 registers (2048 × 2048 9.1, not 10.4 µs)
+template <bool AT_ONCE = true>
 __device__ __forceinline__ float block_sum(float q, float* red) {
     q = wave_reduce_sum(q);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = q;
     __syncthreads();
+    if (!AT_ONCE) {
+        float t = 0.f;
+        for (int i = 0; i < (int)(blockDim.x >> 6); i++) t += red[i];
+        return t;
+    }
     float r[16], t = 0.f;                                              // (red holds 16, all read at once)
 #pragma unroll
     for (int i = 0; i < 16; i++) r[i] = red[i];
@@ -65,9 +72,18 @@ __device__ __forceinline__ float block_sum(float q, float* red) {
     for (int i = 0; i < 16; i++) t += i < (int)(blockDim.x >> 6) ? r[i] : 0.f;
     return t;
 }
-// Σ over the slabs of a branch, in their order; up to four are under way together (one after the other each cost a round trip, 0.7 µs)
+// Σ over the slabs of a branch, in their order; TOGETHER: two, or up to four, are under way at once (one after the other each cost a round trip, 0.7 µs)
+template <bool TOGETHER = true>
 __device__ __forceinline__ floatx4 sum_slabs(const float* p, int slabs, long stride) {
-    if (slabs == 1) return *reinterpret_cast<const floatx4*>(p);
+    if (!TOGETHER || slabs == 1) {
+        floatx4 v = *reinterpret_cast<const floatx4*>(p);
+        for (int z = 1; z < slabs; z++) v += *reinterpret_cast<const floatx4*>(p + z * stride);
+        return v;
+    }
+    if (slabs == 2) {
+        const floatx4 a = *reinterpret_cast<const floatx4*>(p), b = *reinterpret_cast<const floatx4*>(p + stride);
+        return a + b;
+    }
     floatx4 t[4];
 #pragma unroll
     for (int z = 0; z < 4; z++) t[z] = *reinterpret_cast<const floatx4*>(p + (z < slabs ? z : slabs - 1) * stride);
@@ -130,6 +146,9 @@ int branch_add(const float* sub, long ld_sub, int slabs, long slab_stride, const
 
 // One workgroup per row; a thread holds VEC quads of the row in registers (0: any length, from memory), so the branch is read once.  NEXT: the copy is the row
 // divided by its root mean square, the input of a block that norms ahead of its sublayers.
+// One quad a thread (decode, and narrow rows): latency alone, so everything is requested at once, what the first sum does not need ahead of it.  Of
+// several quads the row's own are requested first, and what is not needed yet does not take registers (all at once: rows of 6144 in two slabs
+// 3.6 → 4.2 µs, 512 of them 7.7 → 9.1; the update below 1024 × 4096 8.5 → 15.5, 8192 × 2880 43 → 100).
 template <typename E, int VEC, bool GATE, bool NEXT>
 __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __restrict__ sub, long ld_sub, int slabs, long slab_stride, const E* __restrict__ gate,
                                                              long ld_gate, const float* __restrict__ w, float mult, float eps,
@@ -148,16 +167,21 @@ __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __rest
         for (int c = 0; c < VEC; c++) {
             const int i = (c * blockDim.x + threadIdx.x) * 4;
             if (i < dim) {
-                xv[c] = *reinterpret_cast<const floatx4*>(xr + i);
-                wv[c] = *reinterpret_cast<const floatx4*>(w + i);
+                auto rest = [&] {
+                    xv[c] = *reinterpret_cast<const floatx4*>(xr + i);
+                    wv[c] = *reinterpret_cast<const floatx4*>(w + i);
+                };
+                if (VEC == 1) rest();
                 e4 gv = {};
-                if (GATE) gv = *reinterpret_cast<const e4*>(gr + i);
-                v[c] = sum_slabs(sr + i, slabs, slab_stride);
+                if (GATE && VEC == 1) gv = *reinterpret_cast<const e4*>(gr + i);
+                v[c] = sum_slabs<VEC == 1>(sr + i, slabs, slab_stride);
+                if (GATE && VEC != 1) gv = *reinterpret_cast<const e4*>(gr + i);
+                if (VEC != 1) rest();
 #pragma unroll
                 for (int j = 0; j < 4; j++) { if (GATE) v[c][j] *= (float)gv[j]; q += v[c][j] * v[c][j]; }
             }
         }
-        const float inv = mult / sqrtf(block_sum(q, red) / (float)dim + eps);
+        const float inv = mult / sqrtf(block_sum<VEC == 1>(q, red) / (float)dim + eps);
 #pragma unroll
         for (int c = 0; c < VEC; c++) {
             const int i = (c * blockDim.x + threadIdx.x) * 4;
@@ -167,7 +191,7 @@ __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __rest
                 *reinterpret_cast<floatx4*>(xr + i) = xv[c];
             }
         }
-        const float unit = NEXT ? 1.0f / sqrtf(block_sum(n, red + 16) / (float)dim + eps) : 1.0f;
+        const float unit = NEXT ? 1.0f / sqrtf(block_sum<VEC == 1>(n, red + 16) / (float)dim + eps) : 1.0f;
 #pragma unroll
         for (int c = 0; c < VEC; c++) {
             const int i = (c * blockDim.x + threadIdx.x) * 4;
@@ -186,7 +210,7 @@ __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __rest
         return GATE ? t * (float)gr[i] : t;
     };
     for (int i = threadIdx.x; i < dim; i += blockDim.x) { const float t = branch(i); q += t * t; }
-    const float inv = mult / sqrtf(block_sum(q, red) / (float)dim + eps);
+    const float inv = mult / sqrtf(block_sum<VEC == 1>(q, red) / (float)dim + eps);
     for (int i = threadIdx.x; i < dim; i += blockDim.x) {
         const float t = xr[i] + branch(i) * inv * w[i];
         xr[i] = t;
@@ -194,7 +218,7 @@ __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __rest
         if (!NEXT) br[i] = (E)t;
     }
     if (NEXT) {
-        const float unit = 1.0f / sqrtf(block_sum(n, red + 16) / (float)dim + eps);
+        const float unit = 1.0f / sqrtf(block_sum<VEC == 1>(n, red + 16) / (float)dim + eps);
         for (int i = threadIdx.x; i < dim; i += blockDim.x) br[i] = (E)(xr[i] * unit);
     }
 }
@@ -234,25 +258,27 @@ __global__ __launch_bounds__(256) void rms_norm_rows_kernel(const float* __restr
     __shared__ float red[16];
     const float* xr = x + (row_idx ? (long)row_idx[blockIdx.x] : (long)blockIdx.x) * dim;
     float q = 0.f;
-    if (dim <= 8 * 256) {
-        // the row and its weights requested together, and read once
-        float xv[8], wv[8];
+    // the row and its weights requested together, and read once
+    auto held = [&](auto numbers) {
+        constexpr int N = decltype(numbers)::value;
+        float xv[N], wv[N];
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
+        for (int c = 0; c < N; c++) {
             const int i = threadIdx.x + c * 256, at = i < dim ? i : 0;
             wv[c] = w ? w[at] : 1.f;
             xv[c] = xr[at];
         }
 #pragma unroll
-        for (int c = 0; c < 8; c++) q += (int)threadIdx.x + c * 256 < dim ? xv[c] * xv[c] : 0.f;
+        for (int c = 0; c < N; c++) q += (int)threadIdx.x + c * 256 < dim ? xv[c] * xv[c] : 0.f;
         const float inv = 1.0f / sqrtf(block_sum(q, red) / (float)dim + eps);
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
+        for (int c = 0; c < N; c++) {
             const int i = threadIdx.x + c * 256;
             if (i < dim) out[(long)blockIdx.x * ldo + i] = (E)(xv[c] * inv * wv[c]);
         }
-        return;
-    }
+    };
+    if (dim <= 2 * 256) return held(std::integral_constant<int, 2>{});
+    if (dim <= 8 * 256) return held(std::integral_constant<int, 8>{});
     for (int i = threadIdx.x; i < dim; i += 256) q += xr[i] * xr[i];
     const float inv = 1.0f / sqrtf(block_sum(q, red) / (float)dim + eps);
     for (int i = threadIdx.x; i < dim; i += 256) out[(long)blockIdx.x * ldo + i] = (E)(w ? xr[i] * inv * w[i] : xr[i] * inv);
@@ -287,15 +313,21 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
     if constexpr (VEC > 0) {
         typedef E e4 __attribute__((ext_vector_type(4)));
         floatx4 v[VEC ? VEC : 1], r[VEC ? VEC : 1], xv[VEC ? VEC : 1], w1[VEC ? VEC : 1], w2[VEC ? VEC : 1], wn[VEC ? VEC : 1];
-        // (weights are requested ahead of the sums that they are for)
-#pragma unroll
-        for (int c = 0; c < VEC; c++) {
-            const int at = (c * nt + threadIdx.x) * 4, i = at < dim ? at : 0;
+        constexpr bool EARLY = VEC == 1;
+        // weights, of one quad ahead of the sums that they are for (see above)
+        auto branch_weights = [&](int c, int i) {
             if (POST) w1[c] = *reinterpret_cast<const floatx4*>(u.post_w + i);
             if (POST && u.gate) w2[c] = *reinterpret_cast<const floatx4*>(u.gate_w + i);
             if (joined) { w1[c] = *reinterpret_cast<const floatx4*>(u.w + i); w2[c] = *reinterpret_cast<const floatx4*>(u.w2 + i); }
+        };
+        auto next_weights = [&](int c, int i) {
             wn[c] = (floatx4){1.f, 1.f, 1.f, 1.f};
             if (u.out && u.next_w) wn[c] = *reinterpret_cast<const floatx4*>(u.next_w + i);
+        };
+        if (EARLY) {
+            const int at = threadIdx.x * 4, i = at < dim ? at : 0;
+            branch_weights(0, i);
+            next_weights(0, i);
         }
         float q1 = 0.f, q2 = 0.f, n = 0.f;
 #pragma unroll
@@ -303,10 +335,11 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
             const int i = (c * nt + threadIdx.x) * 4;
             if (i < dim) {
                 xv[c] = (floatx4){0.f, 0.f, 0.f, 0.f};
-                if (!u.replace) xv[c] = *reinterpret_cast<const floatx4*>(xr + i);
-                if (joined) r[c] = sum_slabs(s2 + i, u.slabs2, u.slab_stride2);
+                if (EARLY && !u.replace) xv[c] = *reinterpret_cast<const floatx4*>(xr + i);
+                if (EARLY && joined) r[c] = sum_slabs(s2 + i, u.slabs2, u.slab_stride2);
                 v[c] = (floatx4){0.f, 0.f, 0.f, 0.f};
-                if (u.sub) v[c] = sum_slabs(s1 + i, u.slabs, u.slab_stride);
+                if (u.sub) v[c] = sum_slabs<EARLY>(s1 + i, u.slabs, u.slab_stride);
+                if (!EARLY && !u.replace) xv[c] = *reinterpret_cast<const floatx4*>(xr + i);
                 if (POST)
 #pragma unroll
                     for (int k = 0; k < 4; k++) v[c][k] *= factor;
@@ -314,7 +347,7 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
 #pragma unroll
                     for (int k = 0; k < 4; k++) xv[c][k] *= keep;
                 if (u.add) xv[c] += *reinterpret_cast<const floatx4*>(u.add + i);
-                if (!POST)
+                if (!POST && EARLY)
                     for (int j0 = 0; j0 < u.top; j0 += 8) {             // (eight at once)
                         e4 e[8];
                         float w[8];
@@ -340,6 +373,7 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
                     for (int k = 0; k < 4; k++) v[c][k] += w * (float)e[k];
                 }
                 if (joined) {
+                    if (!EARLY) r[c] = sum_slabs<false>(s2 + i, u.slabs2, u.slab_stride2);
 #pragma unroll
                     for (int k = 0; k < 4; k++) { q1 += v[c][k] * v[c][k]; q2 += r[c][k] * r[c][k]; }
                 }
@@ -347,14 +381,15 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
         }
         float i1 = 0.f, i2 = 0.f;
         if (joined) {
-            i1 = 0.5f / sqrtf(block_sum(q1, red) / (float)dim + u.eps);
-            i2 = 0.5f / sqrtf(block_sum(q2, red + 16) / (float)dim + u.eps);
+            i1 = 0.5f / sqrtf(block_sum<VEC == 1>(q1, red) / (float)dim + u.eps);
+            i2 = 0.5f / sqrtf(block_sum<VEC == 1>(q2, red + 16) / (float)dim + u.eps);
         }
 #pragma unroll
         for (int c = 0; c < VEC; c++) {
             const int i = (c * nt + threadIdx.x) * 4;
             if (i < dim) {
                 if (joined) {
+                    if (!EARLY) branch_weights(c, i);
 #pragma unroll
                     for (int k = 0; k < 4; k++) v[c][k] = v[c][k] * i1 * w1[c][k] + r[c][k] * i2 * w2[c][k];
                 }
@@ -365,13 +400,14 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
             }
         }
         if (POST) {
-            const float inv = 1.0f / sqrtf(block_sum(n, red) / (float)dim + u.eps);
+            const float inv = 1.0f / sqrtf(block_sum<VEC == 1>(n, red) / (float)dim + u.eps);
             float z = 0.f;
             n = 0.f;
 #pragma unroll
             for (int c = 0; c < VEC; c++) {
                 const int i = (c * nt + threadIdx.x) * 4;
                 if (i < dim) {
+                    if (!EARLY) branch_weights(c, i);
                     floatx4 g = {0.f, 0.f, 0.f, 0.f};
                     if (u.gate) g = w2[c];
 #pragma unroll
@@ -380,16 +416,17 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
                 }
             }
             if (u.gate) {
-                z = block_sum(z, red + 16);
+                z = block_sum<VEC == 1>(z, red + 16);
                 if (threadIdx.x == 0) u.gate[row] = 1.0f / (1.0f + expf(-z));
             }
         }
         if (!u.out) return;
-        const float unit = u.next_w ? 1.0f / sqrtf(block_sum(n, red + 32) / (float)dim + u.eps) : 1.0f;
+        const float unit = u.next_w ? 1.0f / sqrtf(block_sum<VEC == 1>(n, red + 32) / (float)dim + u.eps) : 1.0f;
 #pragma unroll
         for (int c = 0; c < VEC; c++) {
             const int i = (c * nt + threadIdx.x) * 4;
             if (i < dim) {
+                if (!EARLY) next_weights(c, i);
                 e4 o;
 #pragma unroll
                 for (int k = 0; k < 4; k++) o[k] = (E)(xv[c][k] * unit * wn[c][k]);
@@ -415,8 +452,8 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
     if (joined) {
         float q1 = 0.f, q2 = 0.f;
         for (int i = threadIdx.x; i < dim; i += nt) { const float a = first(i), b = second(i); q1 += a * a; q2 += b * b; }
-        i1 = 0.5f / sqrtf(block_sum(q1, red) / (float)dim + u.eps);
-        i2 = 0.5f / sqrtf(block_sum(q2, red + 16) / (float)dim + u.eps);
+        i1 = 0.5f / sqrtf(block_sum<VEC == 1>(q1, red) / (float)dim + u.eps);
+        i2 = 0.5f / sqrtf(block_sum<VEC == 1>(q2, red + 16) / (float)dim + u.eps);
     }
     for (int i = threadIdx.x; i < dim; i += nt) {
         float t = joined ? first(i) * i1 * u.w[i] + second(i) * i2 * u.w2[i] : first(i);
@@ -426,7 +463,7 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
         n += t * t;
     }
     if (POST) {
-        const float inv = 1.0f / sqrtf(block_sum(n, red) / (float)dim + u.eps);
+        const float inv = 1.0f / sqrtf(block_sum<VEC == 1>(n, red) / (float)dim + u.eps);
         float z = 0.f;
         n = 0.f;
         for (int i = threadIdx.x; i < dim; i += nt) {            // (a thread's own elements)
@@ -436,12 +473,12 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
             if (u.gate) z += t * u.gate_w[i];
         }
         if (u.gate) {
-            z = block_sum(z, red + 16);
+            z = block_sum<VEC == 1>(z, red + 16);
             if (threadIdx.x == 0) u.gate[row] = 1.0f / (1.0f + expf(-z));
         }
     }
     if (!u.out) return;
-    const float unit = u.next_w ? 1.0f / sqrtf(block_sum(n, red + 32) / (float)dim + u.eps) : 1.0f;
+    const float unit = u.next_w ? 1.0f / sqrtf(block_sum<VEC == 1>(n, red + 32) / (float)dim + u.eps) : 1.0f;
     for (int i = threadIdx.x; i < dim; i += nt) out[i] = (E)(u.next_w ? xr[i] * unit * u.next_w[i] : xr[i]);
 }
 template <typename E>

@@ -43,6 +43,15 @@ def differs(cfg, w, t, taps, bound=1e-3):
     return rel(other, taps) > bound
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,n", [(1030, 9), (1056, 40), (2044, 17), (2052, 520), (4100, 5)])
+def test_rows_of_several_quads_a_thread(pkg, tmp_path, dtype, width, n):
+    """The sum itself normed, with the experts' rows and the gate, in rows that a thread holds two or four pieces of, or none.  One layer: the worst of 520 rows is off
+    by 0.018 in 16 bits, and a second attention over such rows trebles what it is told."""
+    cfg = model([G.far_attention(2, 1, 8, 8, mlp=G.identity_experts(4, 2, 2, 12, 20))], width=width)
+    agree(pkg, tmp_path, cfg, G.weights(cfg, 19), dtype, n=n, tol=2 * ALONE[dtype])
+
+
 # ── embedding, norm of the sum, capped logits ─────────────────────────────────────────────────────────────────────────────
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("width,factor", [(72, 2.5), (45, 0.3), (33, 1.0)])

@@ -77,7 +77,7 @@ def one_layer(layer, width=72, vocab=50, mult=1.0, **kw):
 
 
 def taps_of(pkg, tmp_path, cfg, w, dtype, tokens):
-    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), dtype)
+    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), dtype, tokens=max(512, len(tokens)))
     m.enable_taps()
     m.forward_rows([(1, tokens, 0)], [len(tokens) - 1])
     return m.read_taps(len(tokens))
@@ -101,6 +101,17 @@ def test_pair_embedding_across_portions(pkg, tmp_path, dtype):
             assert np.abs(m.read_taps(n)[0] - want[at:at + n]).max() < 1e-6
             at += n
         m.release(seq)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,n", [(1030, 9), (1056, 40), (2044, 17), (2052, 520), (4100, 5)])
+def test_rows_of_several_quads_a_thread(pkg, tmp_path, dtype, width, n):
+    """Gated branches, normed and added, in rows that a thread holds two or four pieces of, or none."""
+    cfg = G.config(width, 50, [G.attention(2, 8, 4, 8, 16, 24, 7, ff=20), G.recurrent(24, 2, 2, ff=33)])
+    t, taps = toks(cfg, n, 6), []
+    w = G.weights(cfg, 19)
+    L.forward(cfg, w, t, taps)
+    assert rel(taps_of(pkg, tmp_path, cfg, w, dtype, t), taps) < TOL[dtype]
 
 
 ATTN = [G.attention(3, 20, 6, 36, 44, 52, 9, base=300.0), G.attention(16, 32, 16, 32, 32, 64, 40), G.attention(5, 64, 34, 17, 33, 130, 25, scale=0.3),

@@ -43,6 +43,14 @@ def silence(w, *what):
             w[k][:] = 0.0
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,n", [(1030, 9), (1056, 40), (2044, 17), (2052, 520), (4100, 5)])
+def test_rows_of_several_quads_a_thread(pkg, tmp_path, dtype, width, n):
+    """Experts' rows added and the token's side normed, in rows that a thread holds two or four pieces of, or none."""
+    cfg = model([G.sink_attention(2, 8, 4, 8, 16, mlp=G.experts(4, 2, 12)), G.sink_attention(1, 8, 4, 8, 16, mlp=G.glu(20, 0.7))], width=width)
+    agree(pkg, tmp_path, cfg, G.weights(cfg, 19), dtype, n=n, tol=2 * ALONE[dtype])
+
+
 # ── each mechanism alone ──────────────────────────────────────────────────────────────────────────────────────────────────
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("side,width", [(12, 72), (1, 33), (64, 96), (45, 130)])

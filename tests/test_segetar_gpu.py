@@ -64,6 +64,14 @@ def portions_agree(pkg, tmp_path, cfg, w, dtype, n, cuts, seed=6):
     return t, want
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,n", [(1030, 9), (1056, 40), (2044, 17), (2052, 520), (4100, 5)])
+def test_rows_of_several_quads_a_thread(pkg, tmp_path, dtype, width, n):
+    """Both branches of a layer normed and joined, experts' rows added, in rows that a thread holds two or four pieces of, or none."""
+    cfg = model([G.gated_pair(2, 1, 8, 8, 9, 1, 8, 8), G.scan(24, 3, 5, 2, mlp=G.grouped_experts(4, 2, 12))], width=width)
+    agree(pkg, tmp_path, cfg, G.weights(cfg, 19), dtype, n=n, tol=2 * ALONE[dtype])
+
+
 # ── grouped attention ─────────────────────────────────────────────────────────────────────────────────────────────────────
 ATTN = [(6, 2, 20, 28, 9, 6), (4, 4, 32, 32, 40, 32), (24, 1, 64, 64, 25, 40), (1, 1, 5, 3, 1, 2), (8, 4, 96, 70, 64, 0), (35, 7, 128, 128, 33, 128), (3, 3, 200, 190, 50, 100),
         (2, 1, 256, 256, 30, 256), (2, 2, 300, 40, 20, 300)]
