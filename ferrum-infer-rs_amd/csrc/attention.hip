@@ -1242,13 +1242,13 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
     // head_dim 128 has two sizes of workgroup.  128 rows read K/V from LDS half as often, 64 rows make twice the workgroups and half of a step's
     // vector work in each; two workgroups of either share a CU.  The longest keys of a prompt are a workgroup's alone, and 64 rows pass them
     // in 0.65 of the time, until there are rounds enough to hide that: 64 rows below 620 workgroups of 128.  Where a window or a context of
-    // more than 1.5 times the new tokens leaves every workgroup about as many keys, below 360.  Over 230 batches between 256 and 2300 that
-    // choice is 1.2 % from the faster of the two (128 rows take up to 1.6 times as long below 500, 64 rows 1.3 times from 1000 on).
+    // more than 1.5 times the new tokens leaves every workgroup about as many keys, below 360.  Over 229 batches between 256 and 2300 that
+    // choice is 0.6 % from the faster of the two, always 128 rows 7, always 64 rows 11 (128 rows take up to 1.7 times as long below 360, 64 rows 1.4 times from 1000 on).
     // µs, row-split or KV-split form / 64 rows / 128 rows (workgroups of 128 rows × kv heads)
-    //   8B heads (32 on 8)    1 × 8100 (2024)      2372 / 750 / 587      1 × 2048 (512)        196 / 69 / 64     1 × 1024 (256)         62 / 27 / 32
-    //                         1 × 2180 (545)            - / 75 / 90      1 × 700 (175)          32 / 22 / 31     1 × 500 (125)          19 / 16 / 20
-    //   16 on 8               1500 and 548 (256)     82 / 43 / 62        293, 1389, 366 (256)   87 / 40 / 56     1 × 986 at 366 (123)   49 / 36 / 50
-    //                         6 × 100, 1400 (250)    80 / 38 / 84        1 × 500 (62)           14 / 14 / 15     1 × 4360 on 32 (1090)   - / 244 / 190
+    //   8B heads (32 on 8)    1 × 8100 (2024)      2372 / 789 / 606      1 × 2048 (512)        196 / 66 / 65     1 × 1024 (256)         62 / 27 / 34
+    //                         1 × 2180 (545)            - / 75 / 92      1 × 700 (175)          32 / 21 / 31     1 × 500 (125)          19 / 16 / 19
+    //   16 on 8               1500 and 548 (256)     82 / 43 / 61        293, 1389, 366 (256)   87 / 40 / 56     1 × 986 at 366 (123)   49 / 36 / 51
+    //                         6 × 100, 1400 (250)    80 / 37 / 82        1 × 500 (62)           14 / 14 / 15     32 on 8, 1 × 4360 (1090)  - / 246 / 199
     // A batch qualifies where most of its sequences bring many rows, or they bring 256 on average.
     const long rows_heads = (long)total_q_tokens * G * num_kv_heads;
     const bool two_sizes = head_dim == 128 && !kn.attn_flash32, even = (sliding_window > 0 && max_kv_len > sliding_window) || (long)max_kv_len * 2 >= (long)max_q_len * 5;
