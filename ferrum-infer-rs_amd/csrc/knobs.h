@@ -13,6 +13,7 @@
 
 namespace fh {
 
+constexpr int TILED_WIDE_MIN_TILES = 257;
 struct Knobs {
     // paged attention (attention.hip)
     bool attn_no_flash = false;
@@ -58,7 +59,8 @@ struct Knobs {
     int lds_min_groups = 8;
     // layered models (tiled_gemm.hip, latent_attention.hip, grouped_attention.hip, linear_attention.hip, rglru.hip)
     int tiled_big_min_tiles = -1;     // ≥ 0: projections of > 64 rows take the tile kernel from this many tiles of 64 × 64 (32-bit: and one); −1: from 193, in 32 bits 129
-    int tiled_wide_min_tiles = 257;   // … and in 16 bits its 128 × 256 form from this many tiles of that size
+    int tiled_wide_min_tiles = TILED_WIDE_MIN_TILES;   // … and in 16 bits its 128 × 256 form from this many tiles of that size
+    int tiled_256 = 0;                // … 256 × 256: 1 wherever they can, 0 where they take less, −1 never
     int tiled_min_tiles = 128;        // few-row kernel: rows of a workgroup are halved until there are this many row × 16-column tiles (16-bit: up to twice as many)
     int tiled_half_max_tiles = 256;   // … its 128 × 64 and 64 × 64 forms up to this many tiles of 128 × 128
     int tiled_small_max_tiles = 256;  // … the latter up to this many of them
@@ -164,6 +166,7 @@ enum Form : int {
     FORM_W4_GATED,              // ≤ 16 rows: gate_up with its activation in the launch
     FORM_F16_GATED,             // unquantised gate_up with its activation in the launch
     FORM_TILED_GEMM_COLS64,     // few-row projection with 64 columns a wave
+    FORM_TILED_GEMM_256X256,    // prompts: tiles of 256 × 256, a workgroup's one after the other (tiled_gemm_wide.hip)
     FORM_COUNT
 };
 

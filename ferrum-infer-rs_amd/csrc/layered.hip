@@ -584,7 +584,7 @@ private:
         z.n_store = routed; z.nsec = 1; z.sec[0] = {0, GEMM_ACT_NONE, 0, 0, L.g2};
         RUN(tiled_gemm(z, s));
         GemmRows rows;
-        rows.block = moe_block(pairs, E_);
+        rows.block = moe_block(pairs, E_, L.up.k % 128 == 0 && L.down.k % 128 == 0);
         rows.max_blocks = std::min(pairs, pairs / rows.block + std::min(E_, pairs));
         rows.id = sorted_; rows.group = sorted_expert_; rows.total = sorted_total_;
         const bool corrected = L.s.ff != FERRUM_HIP_FF_MOE_RELU2;
@@ -608,10 +608,12 @@ private:
         return 0;
     }
     // rows per block of the sorted list: a large block shares an expert's weights between more rows, a small one pads less
-    static int moe_block(int pairs, int experts) {
+    // (256: for the tiles of that many rows, which save 6 % of a long launch, where the half of a block more that an expert leaves empty is a small part of its rows:
+    // 32 × 256 tokens, 8 of 24 experts, 2731 rows each: prompt 9.87 → 9.46 ms; 4002 tokens, 1067 each: 2.13 → 2.16)
+    static int moe_block(int pairs, int experts, bool tiles256) {
         const int mean = pairs / experts, forced = knobs().moe_rows_block;
         if (forced > 0 && (sizeof(E) == 2 || forced <= 64)) return forced;
-        if (sizeof(E) == 2 && mean >= 48) return 128;
+        if (sizeof(E) == 2 && mean >= 48) return tiles256 && mean >= 2048 ? 256 : 128;
         return mean >= 32 ? 64 : mean >= 12 ? 32 : 16;
     }
 

@@ -141,6 +141,10 @@ __device__ __forceinline__ float log_sigmoid_f32(float z) { return fminf(z, 0.f)
 // quadratic right of zero, exponential left of it, slope 1/2 at zero; sp / sq: softplus of the two trained numbers
 template <typename E>
 __device__ __forceinline__ float xielu_f32(float z, float sp, float sq) {
+    if (sizeof(E) == 2) {                                   // (both sides: an exponential costs less than a branch)
+        const float right = sp * z * z, left = (0.5f + sq) * ActMath<E>::expm1_minus(z);
+        return (z > 0.f ? right : left) + 0.5f * z;
+    }
     return (z > 0.f ? sp * z * z : (0.5f + sq) * ActMath<E>::expm1_minus(z)) + 0.5f * z;
 }
 

@@ -7,35 +7,10 @@
 #include "common.h"
 #include "knobs.h"
 #include "tiled_gemm.h"
+#include "tiled_gemm_device.h"
 
 namespace fh {
 
-// N neighbouring columns of one section, whose kind of activation is a scalar: one chain of branches for all of them (one for each number made squared
-// ReLUs cost a launch of 4096 × 6144 × 2048 21 µs of 115, now 3)
-template <typename E, bool RARE, int N, typename V>
-__device__ __forceinline__ void gemm_act(const GemmSection& sec, int act, V& v) {
-#define EACH(...)                            \
-    do {                                     \
-        _Pragma("unroll") for (int e = 0; e < N; e++) { const float z = v[e]; v[e] = __VA_ARGS__; } \
-        return;                              \
-    } while (0)
-    if (act == GEMM_ACT_NONE) return;
-    if (act == GEMM_ACT_SIGMOID) EACH(ActMath<E>::sigmoid(z));
-    if (act == GEMM_ACT_GELU_TANH) EACH(gelu_tanh_f32<E>(z));
-    if (act == GEMM_ACT_XIELU) EACH(xielu_f32<E>(z, sec.p, sec.q));
-    if (act == GEMM_ACT_RELU2) EACH(fmaxf(z, 0.f) * fmaxf(z, 0.f));
-    if (act == GEMM_ACT_SILU) EACH(z * ActMath<E>::sigmoid(z));
-    if (RARE && act == GEMM_ACT_SOFTPLUS) EACH(softplus_f32<E>(z));
-    if (RARE && act == GEMM_ACT_LOG_SIGMOID) EACH(sec.p * log_sigmoid_f32<E>(z));
-    if (RARE && act == GEMM_ACT_SOFTCAP) EACH(sec.p * ActMath<E>::tanh(z / sec.p));
-#undef EACH
-}
-// output row of place r, −1: none
-template <typename E>
-__device__ __forceinline__ int gemm_out_row(const TiledGemm<E>& p, int r) {
-    if (p.rows.id) r = p.rows.id[r];
-    return r < p.m ? r : -1;
-}
 template <typename E>
 __device__ __forceinline__ void gemm_store(const TiledGemm<E>& p, int g, int row, int col, float v) {
     if (p.row_scale) v *= (float)p.row_scale[row * p.ld_scale + g];
@@ -43,29 +18,6 @@ __device__ __forceinline__ void gemm_store(const TiledGemm<E>& p, int g, int row
     const long o = row * p.ldo + (p.rows.id ? 0 : g * p.out_group) + col;
     if (p.out_f32) p.out_f32[o] = v; else p.out[o] = (E)v;
 }
-template <typename E, int N, typename V>
-__device__ __forceinline__ void gemm_glu(const GemmSection& sec, int act, V& gate, const V& up) {
-    if (act == GEMM_ACT_SILU_GLU) {
-#pragma unroll
-        for (int e = 0; e < N; e++) gate[e] = gate[e] * ActMath<E>::sigmoid(gate[e]) * up[e];
-    } else if (act == GEMM_ACT_GELU_GLU) {
-#pragma unroll
-        for (int e = 0; e < N; e++) gate[e] = gelu_tanh_f32<E>(gate[e]) * up[e];
-    } else {
-#pragma unroll
-        for (int e = 0; e < N; e++) gate[e] = clamped_glu_f32<E>(gate[e], up[e], sec.p, sec.q);
-    }
-}
-__device__ __forceinline__ int gemm_gated_col(const GemmSection& sec, int col) { return sec.begin + ((col - sec.begin) >> 5) * 16 + (col & 15); }
-template <typename E>
-__device__ __forceinline__ GemmSection gemm_section(const TiledGemm<E>& p, int col) {
-    GemmSection s = {0, GEMM_ACT_NONE, 0.f, 0.f, 1.f};
-#pragma unroll
-    for (int i = 0; i < GEMM_MAX_SECTIONS; i++)
-        if (i < p.nsec && col >= p.sec[i].begin) s = p.sec[i];
-    return s;
-}
-
 // address of the 16-byte piece a of row b of row tile t, and the distance between the steps of four pieces
 template <typename E>
 __device__ __forceinline__ const E* gemm_row(const TiledGemm<E>& p, int t, int g, int a, int b) {
@@ -597,6 +549,12 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
 //   64 × 64 → 128 × 64        256: 253 × 4096 × 2048   14.5 → 17.3, 125 × 8192 × 4096   26 → 31     288: 253 × 4608 × 2048   19.8 → 17.5
 //   few rows → 64 × 64        128: 253 × 2048 × 2048   9.0 → 14.3     192: 128 × 6144 × 2048   14.5 → 15.1, 65 × 6144 × 4096   27.1 → 26.0
 //                             224: 400 × 2048 × 1024   8.9 → 8.8      256: 65 × 8192 × 4096   30.3 → 28.6      288: 192 × 6144 × 2048   24.1 → 17.2
+// 256 × 256 (tiled_gemm_wide.hip): a round of 256 tiles, one per CU, takes 11.6 µs + K · 0.0201, a round of 256 of 128 × 256, of which two share a CU, 5.5 + K · 0.01185.
+// 150 shapes, 500 – 8192 rows × 1024 – 16384 × 512 – 4096, µs of the latter (rounds) | of the former (rounds):
+//   2001 × 8192 × 1024  35.6 (2) | 34.3 (1)     3500 × 8192 × 2048    110 (4) | 100 (2)      8192 × 10240 × 4096  539 (10) | 463 (5)
+//   4096 × 4096 × 4096   112 (2) | 98.8 (1)     4096 × 10240 × 2048   148 (5) | 146 (3)      7000 × 8192 × 1024   109 (7) | 111 (4)
+//   3000 × 8192 × 4096   164 (3) | 173 (2)      4096 × 6144 × 1024    57 (3) | 67 (2)        5000 × 3072 × 512    22.9 (2) | 23.4 (1)
+// so wherever its rounds are half as many as the other's, but for short K.
 template <typename E>
 static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
     auto tiles = [&](int r, int c) { return (long)(g.rows.id ? g.rows.max_blocks * (g.rows.block / r) : cdiv(g.m, r)) * cdiv(g.n, c) * g.groups; };
@@ -615,6 +573,11 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
         if ((g.rows.id && g.rows.block < 128) || small < std::min(full, half)) return launch_big<E, 2, 2, 3, 3>(g, s);
         return half < full ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 4, 4, 2, 2>(g, s);
     } else {
+        // (a forced size of the tiles above stays what it is)
+        const long halves = cdiv(tiles(128, 256), 256), rounds = cdiv(tiles(256, 256), 256);
+        const bool fits = knobs().tiled_wide_min_tiles == TILED_WIDE_MIN_TILES && halves > 1 && (!g.rows.id || g.rows.block % 256 == 0)
+                          && rounds * (11.6f + 0.0201f * g.k) < (g.k > 512 ? 0.97f : 0.93f) * halves * (5.5f + 0.01185f * g.k);
+        if ((knobs().tiled_256 > 0 || (knobs().tiled_256 == 0 && fits)) && tiled_gemm_wide_supports(g)) return tiled_gemm_wide(g, s);
         if (tiles(128, 256) >= knobs().tiled_wide_min_tiles) return launch_big<E, 4, 8, 2, 2>(g, s);
         if (tiles(128, 128) > knobs().tiled_half_max_tiles) return launch_big<E, 4, 4, 2, 2>(g, s);
         return tiles(64, 64) > knobs().tiled_small_max_tiles ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 2, 2, 3, 3>(g, s);

@@ -524,6 +524,27 @@ def test_few_row_and_tile_projections_agree(pkg, cases, knobs, forms, name):
             assert h.get("tiled_gemm") and not h.get("tiled_gemm_big")
 
 
+EVEN = {"nerenex": lambda: G.config(256, 260, [G.recurrent(256, 2, 3, ff=384), G.attention(20, 64, 32, 48, 128, 256, 130, ff=640), G.recurrent(640, 5, 2, ff=128)], mult=0.6),
+        "safolorn": lambda: G.safolorn(128, 260, 40, [G.sink_attention(8, 64, 32, 64, 256, 1e5, G.LONG, mlp=G.glu(384, 1.5)), G.sink_attention(4, 64, 32, 32, 256, 1e5, G.LONG, mlp=G.experts(5, 2, 256))]),
+        "segetar": lambda: G.segetar(256, 260, [G.scan(256, 16, 128, 4, mlp=G.dense(384)), G.gated_pair(8, 2, 64, 64, 130, 4, 64, 64, mlp=G.grouped_experts(6, 2, 128, 2, 1))]),
+        "fororax": lambda: G.fororax(128, 260, [G.talk_attention(8, 2, 64, 32, mlp=G.identity_experts(6, 2, 2, 128, 160)), G.far_attention(4, 2, 64, 96, mlp=G.identity_experts(3, 1, 1, 384, 96))])}
+
+
+@pytest.mark.parametrize("name", EVEN)
+def test_projections_in_tiles_of_256_x_256(pkg, tmp_path, knobs, forms, name):
+    """K of whole rounds of four steps: sections that begin within a wave's columns and between two, gated and rare activations among them, biases, experts' blocks of
+    256 rows with experts that receive few."""
+    cfg = EVEN[name]()
+    w, t = G.weights(cfg, 31), toks(cfg, 420, 12)
+    path, want = G.write_checkpoint(tmp_path, cfg, w), L.forward(cfg, w, t)
+    knobs.set(TILED_256=1, TILED_BIG_MIN_TILES=1, MOE_ROWS_BLOCK=256)
+    m = load(pkg, path, "bfloat16")
+    forms.reset()
+    assert rel(feed(m, 1, t, [420]), want) < TOL["bfloat16"]
+    h = forms.hits()
+    assert h.get("tiled_gemm_256x256") and bool(h.get("tiled_gemm_grouped_big")) == (name != "nerenex")
+
+
 @pytest.mark.parametrize("name", ["wide", "shared", "sinks", "loop", "talks"])
 @pytest.mark.parametrize("big", [1, 10 ** 6])
 def test_32_bit_projections_of_prompts(pkg, cases, knobs, forms, name, big):

@@ -481,6 +481,15 @@ def test_vocabularies_on_both_sides_of_a_line(env, m, n, k, form, knobs, forms):
     assert form in forms.hits() if form else "tiled_gemm" not in forms.hits(), forms.hits()
 
 
+@pytest.mark.parametrize("f32", [False, True])
+@pytest.mark.parametrize("m,n,k", [(65, 64, 128), (255, 288, 256), (257, 320, 384), (511, 1056, 128), (300, 8256, 512), (2310, 8224, 128), (5000, 4160, 256), (700, 512, 4096)])
+def test_tiles_of_256_x_256(env, m, n, k, f32, knobs, forms):
+    """Rows and columns on both sides of a tile's end, one round of four steps and several, less than one tile for each workgroup and up to four one after the other."""
+    knobs.set(TILED_256=1, TILED_BIG_MIN_TILES=1)
+    _few_rows(env, m, n, k, f32)
+    forms.require("tiled_gemm_256x256")
+
+
 @pytest.mark.parametrize("tiles,form", [(0, "tiled_gemm_big"), (2, "tiled_gemm_big"), (3, "tiled_gemm"), (None, "tiled_gemm")])
 def test_tile_kernel_from_a_given_number_of_tiles(env, tiles, form, knobs, forms):
     """Two tiles of 64 x 64: a number asked for, 0 among them, or the rule."""
@@ -489,16 +498,16 @@ def test_tile_kernel_from_a_given_number_of_tiles(env, tiles, form, knobs, forms
     assert set(forms.hits()) & {"tiled_gemm", "tiled_gemm_big"} == {form}
 
 
-def _few_rows(env, m, n, k):
+def _few_rows(env, m, n, k, f32=False):
     pkg, B, ctx, O, torch = env
     gen = torch.Generator("cuda").manual_seed(m * n + k)
     a, b = (torch.randn(r, k, generator=gen, device="cuda").half() for r in (m, n))
-    buf = torch.full(((m + 2) * n,), 7.0, dtype=torch.float16, device="cuda")
+    buf = torch.full(((m + 2) * n,), 7.0, dtype=torch.float32 if f32 else torch.float16, device="cuda")
     out = buf[n:n + m * n]
     B.gemm_f16t(ctx, a, B.dense_repack_f16t(ctx, b, n, k), out, m, n, k)
     ctx.sync()
     want, size = a.double() @ b.double().T, a.double().abs() @ b.double().abs().T
-    assert ((out.reshape(m, n).double() - want).abs() <= 2.0 ** -11 * want.abs() + k * 2.0 ** -24 * size + 2.0 ** -25).all()
+    assert ((out.reshape(m, n).double() - want).abs() <= (0 if f32 else 2.0 ** -11 * want.abs() + 2.0 ** -25) + k * 2.0 ** -24 * size).all()
     assert (buf[:n] == 7.0).all() and (buf[n + m * n:] == 7.0).all()
 
 
