@@ -6,21 +6,23 @@
 // round trips and its drain (≈ 4–5 µs each even when trivial) on top of the kernel boundary, while HBM idles.  Here the five
 // links are ROLES of one grid, laid out in dependency order (blocks of role A first, …): every workgroup requests what does
 // not depend on its predecessor — its INT4 weights (all of them: a wave's K slice is 2–4 quant groups), its block table and
-// first K/V tiles, its norm and router weights — and only then waits for the predecessor's counter.  What is left on the
+// first K/V tiles, its norm and router weights — and only then waits for the predecessor's rows.  What is left on the
 // critical path of a link is: activations in, arithmetic, result out.  One 512-thread workgroup per CU is resident (the
 // attention role holds two K/V fragment sets, 232 registers): at 32 rows the tail (32 workgroups), the q|k|v projection (80)
 // and attention (128) are all there from the start, the o projection's workgroups move in as the tail's and q|k|v's leave
 // (long before attention is done) and the router's as attention's leave — each early enough to have its weights on the way.
 //
-// Hand-offs (MI355X_MICROARCH.md § visibility, valid forms; cdna_hip_programming.md Guideline 16): every byte that crosses
-// workgroups inside the launch is stored write-through (sc1, 8- or 16-byte stores), every storing wave drains its stores
-// (s_waitcnt vmcnt(0)), the workgroup meets at a barrier and ONE lane adds to the consumer's counter; a consumer polls its
-// counter with relaxed agent-scope loads from one lane (s_sleep between polls), releases its other waves through a workgroup
-// barrier, and reads the handed-off bytes with sc1 loads only.  No role waits before all its predecessors' workgroups have been
-// dispatched (dependency order = dispatch order, and nothing that waits comes before something it waits for); every wait
-// is bounded (≈ 20 ms) and a give-up is counted in a host-visible word, so a missing producer costs a wrong result that the
-// runner reports, never a hang.  Counters live on 256-byte lines of their own, are zero on entry and the launch zeroes the
-// OTHER half of a double buffer for the next launch (no memset node per layer).
+// Hand-offs: the rows are their own flags.  A row that crosses workgroups inside the launch is all ones on entry (NOT_YET); its producer
+// stores it write-through (sc1, 8- or 16-byte stores) and is done; a consumer's wave asks for just what it needs (sc1 loads, the GEMM roles
+// straight into LDS) until no 32-bit word of it is NOT_YET any more, whatever the order in which pieces arrive.  What a producer stores is
+// never NOT_YET: the NaN that would read so loses its sign.  Nothing lies between a producer's stores and its consumers' loads: no drain, no
+// counter, no second round trip for the data behind the one that found the flag set (a counter for each link instead: 1.3 – 2 µs from the end of
+// a role's work to its consumer's first product, now 0.6 – 1.0; a launch of one row of 2048 columns 17.0 → 15.05 µs, 8 rows 19.7 → 18.05; a step
+// of one sequence through 8 expert layers, 32 steps and the prompt: 13.34 → 12.59 ms, of 12 through 32 layers of 4096 75.6 → 72.3).  No role
+// waits before all its predecessors' workgroups have been dispatched (dependency order = dispatch order, and nothing that waits comes before
+// something it waits for); every wait is bounded (≈ 20 ms) and a give-up is counted in a host-visible word, so a missing producer costs a wrong
+// result that the runner reports, never a hang.  The rows are double-buffered: the q|k|v workgroups, behind their own result, make the OTHER
+// half all ones for the next launch, which nobody reads any more (no fill node per layer; the forward's head kernel does it for its first launch).
 //
 // Arithmetic: each role is the arithmetic of the stand-alone kernel it replaces, operation for operation —
 // moe_combine_add_rmsnorm_kernel, w4_gemm_wgsplit_kernel<MT, 2> (K split over the 8 waves, LDS reduction in wave order),
@@ -39,21 +41,12 @@ namespace fh {
 namespace {
 
 constexpr int CH_W = 8;                 // waves per workgroup
-constexpr int CH_STRIDE = 64;           // words between counters (one 256-byte line each)
-// Counter groups (slots of CH_STRIDE words).  A group is `shards` × `reps` counters: producer i adds to EVERY replica of shard
-// i mod shards (one wave instruction, `reps` lanes), a waiting workgroup polls ONE replica of every shard (one wave instruction,
-// `shards` lanes).  Shards cut the serialised arrivals per line (≈ 12 ns each), replicas the pollers per line — with one
-// counter per edge the hand-offs took 2–4 µs each (128 pollers + 64 arrivals on one line: 4.2 µs).
-constexpr int CH_NORM_SLOT = 0, CH_NORM_SH = 1, CH_NORM_R = 8;          // tail → q|k|v: T arrivals, ≤ 80 pollers
-constexpr int CH_O_SLOT = 8, CH_O_SH = 4, CH_O_R = 4;                   // o_proj → route: 64 arrivals, 128 pollers
-constexpr int CH_ATTN_SLOT = 24, CH_ATTN_SH = 8, CH_ATTN_R = 4;         // attention → o_proj: T·nkv arrivals, 64 pollers
-constexpr int CH_QKV_SLOT = 56, CH_QKV_R = 4;                           // q|k|v → attention, one group per kv head: (G + 2)·row blocks arrivals, T pollers
 constexpr int CH_MAX_KVH = 16;
-constexpr int CH_SLOTS = CH_QKV_SLOT + CH_QKV_R * CH_MAX_KVH;
+constexpr uint32_t NOT_YET = ~0u;        // a word of a handed-off row that has not been written
 constexpr int CH_GRAN = 10;              // granules per (token, router part): 8 candidates + max + Σexp
 constexpr int CH_O_KS = 2;                // o_proj: K parts per block, each a workgroup of its own (fp32 partial rows, role B adds them)
 constexpr int CH_MAX_SPLITS = 16;          // KV ranges per (sequence, kv head) in the attention role
-constexpr int CH_MAX_T = 128;
+constexpr int CH_MAX_T = CHAIN_MAX_ROWS;
 constexpr int CH_GRAN_WORDS = CH_MAX_T * 4 * CH_GRAN * 2;      // T ≤ 64 tokens × Q ≤ 4 parts, 8-byte granules
 constexpr int CH_SMEM = 8 * 16 * (128 + 4) * 4 + 2 * 8 * 16 * 4 + 16 * 128 * 2 + 2 * 128 * 2;     // the attention role's arena: 73,216 B
 
@@ -88,12 +81,12 @@ struct ChainArgs {
     float scale;
     __half* attn_out;             // [T, nq·128]
     ChainGemm o;
-    __half* o_out;                // [T, H]
     // role B
     __half* res_b_out; const __half* post_ln; __half* norm2; const __half* router_w;
     int E, r_top_k, Q, norm_topk, defer_merge;
     RouteCand* cand; float* stats; unsigned* route_arrive; int32_t* ids; float* weights;
     unsigned* cnt; unsigned* cnt_next; unsigned* timeout;
+    uint32_t* rows_next; int rows_next_pieces;      // the other half of the handed-off rows: NOT_YET again behind this launch
 #ifdef FERRUM_HIP_EXPERIMENTS
     unsigned long long* tl;       // development: per-workgroup wall-clock stamps (tools/exp_timeline_chain.py)
 #endif
@@ -111,35 +104,21 @@ unsigned long long* g_chain_timeline = nullptr;
 #define CH_TL(i) do {} while (0)
 #endif
 
-// `shards` lanes of wave 0 poll (one replica of every shard), the workgroup barrier releases the other waves (the polling
-// wave's own loads follow its match).  `total` producers, producer i ↔ shard i mod shards.
-__device__ __forceinline__ void chain_wait(unsigned* base, int shards, int reps, unsigned total, unsigned* timeout) {
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x;
-        const unsigned need = lane < shards ? (total + (unsigned)(shards - 1 - lane)) / (unsigned)shards : 0u;
-        unsigned* slot = base + ((lane < shards ? lane : 0) * reps + (int)(blockIdx.x % (unsigned)reps)) * CH_STRIDE;
-        const unsigned long long t0 = wall_clock64();
-        unsigned spins = 0;
-        for (;;) {
-            const unsigned c = lane < shards ? __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
-            if (__ballot(c < need) == 0ull) break;
-            __builtin_amdgcn_s_sleep(4);
-            if ((++spins & 255u) == 0u && wall_clock64() - t0 > 2000000ull) {
-                if (lane == 0) __hip_atomic_fetch_add(timeout, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                break;
-            }
+// A wave goes on when `ready` (the same for all its lanes) says so.
+template <typename F>
+__device__ __forceinline__ void chain_until(const F& ready, unsigned* timeout) {
+    const unsigned long long t0 = wall_clock64();
+    unsigned spins = 0;
+    while (!ready()) {
+        __builtin_amdgcn_s_sleep(1);
+        if ((++spins & 255u) == 0u && wall_clock64() - t0 > 2000000ull) {
+            if ((threadIdx.x & 63) == 0) __hip_atomic_fetch_add(timeout, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            break;
         }
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");      // no instruction: keeps later loads behind the poll
-    __syncthreads();
+    asm volatile("" ::: "memory");
 }
-
-// Every wave drains its (write-through) stores, the workgroup meets, `reps` lanes signal (every replica of the shard).
-__device__ __forceinline__ void chain_signal(unsigned* base, int shard, int reps) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if ((int)threadIdx.x < reps) __hip_atomic_fetch_add(base + (shard * reps + (int)threadIdx.x) * CH_STRIDE, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
+__device__ __forceinline__ uint32_t most4(u32x4 v) { return max(max(v[0], v[1]), max(v[2], v[3])); }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t chain_rsrc(const void* base, long bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
@@ -156,8 +135,22 @@ __device__ __forceinline__ void chain_landed() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 }
+// Numbers that are handed off: the one fp16, and fp32, NaN that reads as NOT_YET loses its sign.
+__device__ __forceinline__ uint32_t written2(uint32_t w) {
+    if ((w & 0xFFFFu) == 0xFFFFu) w ^= 0x8000u;
+    return w >= 0xFFFF0000u ? w ^ 0x80000000u : w;
+}
 __device__ __forceinline__ void store16_sc1(__amdgpu_buffer_rsrc_t r, int byte_off, half8 v) {
-    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, byte_off, 0, 16);
+    u32x4 w = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = written2(w[i]);
+    __builtin_amdgcn_raw_buffer_store_b128(w, r, byte_off, 0, 16);
+}
+__device__ __forceinline__ void store16_sc1(__amdgpu_buffer_rsrc_t r, int byte_off, float4v v) {
+    u32x4 w = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = w[i] == NOT_YET ? w[i] ^ 0x80000000u : w[i];
+    __builtin_amdgcn_raw_buffer_store_b128(w, r, byte_off, 0, 16);
 }
 
 // ── role A: MoE combine + residual add + the next input norm (fused.hip kernel A), one workgroup per token ─────────────
@@ -249,21 +242,18 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
             store16_sc1(r_n1, (int)(((long)row * H + i * 8) * 2), o);
         }
     }
-    CH_TL(2);
-    chain_signal(p.cnt + CH_NORM_SLOT * CH_STRIDE, 0, CH_NORM_R);
-    CH_TL(3);
+    CH_TL(2); CH_TL(3);
 }
 
 // ── GEMM roles (q|k|v and o_proj): one 16-row block × NST 64-column supertiles per workgroup, K split over its 8 waves ───
 // All GPW quant groups of a wave's K slice are requested before the wait, and as many of them as registers hold become numbers there; the
-// rows follow the wait (sc1), all at once and in whole lines, into the wave's region of LDS; the 8 partial sums meet in LDS (summed in wave
+// rows (sc1) come all at once and in whole lines into the wave's region of LDS, over again until all of them have been written (from 5 rows on
+// one word of each is watched first: whole rows asked for in vain hold up their producers); the 8 partial sums meet in LDS (summed in wave
 // order) and leave as 16-byte write-through stores.  A workgroup reads rows × K activation bytes after its wait, at the ≈ 70 GB/s a
 // workgroup gets for handed-off bytes — so the rows are split over workgroups (16 each) rather than the columns made narrower.
 // Behind the wait of 12 rows of 4096, 64 columns: 0.9 µs until the rows are there, 1.0 the products, 0.8 the slowest wave's and the meeting, 0.5
 // the result (64-byte pieces of 16 rows, two groups ahead, weights expanded behind the wait: 4.1 in all, now 3.2; 16 rows of 2048 in
 // 128 columns 4.2 → 3.3, o_proj's halves of K 2.7 → 2.0).
-struct ChainEdge { unsigned* base; int shards, reps; unsigned total; };      // base == nullptr: nothing to wait for
-
 // NTL = 16-column tiles of the 64-column supertile a workgroup takes (NST = 1): 4, or 2 — a 32-column block `cb` = supertile cb / 2,
 // half cb % 2: half the weight bytes per workgroup, twice the workgroups (the stage is as long as its slowest workgroup's fetch).
 // F32OUT: the workgroup covers only the quant groups from g_base on (8·GPW of them) and leaves its fp32 partial sums in `out32`
@@ -271,8 +261,7 @@ struct ChainEdge { unsigned* base; int shards, reps; unsigned total; };      // 
 // are what its stage takes, and role B adds the two parts
 template <int NST, int GPW, bool HAS_ZP, int NTL = 4, bool F32OUT = false>
 __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int rb, const __half* x_in, __half* out, int T,
-                                                const ChainEdge& wait, unsigned* sig_base, int sig_shard, int sig_reps,
-                                                unsigned* timeout, unsigned char* smem, const ChainArgs& p, int g_base = 0, float* out32 = nullptr) {
+                                                bool handed_off, unsigned char* smem, const ChainArgs& p, int g_base = 0, float* out32 = nullptr) {
     static_assert(NTL == 4 || (NTL == 2 && NST == 1), "half supertiles only for single-supertile blocks");
     constexpr int V = NST * NTL * 4, CPR = NST * NTL * 2;                       // accumulator floats per lane; 16-byte chunks per output row
     float* red = reinterpret_cast<float*>(smem);                     // [8 regions of a wave][V][64]
@@ -320,21 +309,40 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
                     }
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (wait.base) chain_wait(wait.base, wait.shards, wait.reps, wait.total, timeout);
-    CH_TL(1);
     const __amdgpu_buffer_rsrc_t r_x = chain_rsrc(x_in, (long)T * w.K * 2);
     constexpr int REGION = GPW * 4096;                                // a wave's rows: [group][16 rows][16 pieces of 16 bytes, piece xor row]
     static_assert(V * 256 <= REGION, "a wave's partial sums take its rows' place");
     unsigned char* const mine = smem + wave * REGION;
     chain_landed<0>();                                                // the weights: from here on only row copies are counted
+    auto request = [&] {
 #pragma unroll
-    for (int i = 0; i < GPW; i++)
+        for (int i = 0; i < GPW; i++)
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int r = 4 * q + a;                                  // (rows past the last lie outside of the buffer: zeros, and no traffic)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r_x, (__attribute__((address_space(3))) void*)(mine + (i * 4 + q) * 1024), 16,
-                                                     ((rb * 16 + r) * w.K + (b ^ r) * 8) * 2, (g0 + i) * 256, 0, 16);
+            for (int q = 0; q < 4; q++) {
+                const int r = 4 * q + a;                              // (rows past the last lie outside of the buffer: zeros, and no traffic)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(r_x, (__attribute__((address_space(3))) void*)(mine + (i * 4 + q) * 1024), 16,
+                                                         ((rb * 16 + r) * w.K + (b ^ r) * 8) * 2, (g0 + i) * 256, 0, 16);
+            }
+    };
+    if (handed_off) {
+        // several rows: first a word of each, until one of them is there, so that whole rows are not asked for over and over
+        if (T > 4) {
+            const int at = a == 0 && rb * 16 + b < T ? ((rb * 16 + b) * w.K + g0 * 128 + (int)(blockIdx.x % (2 * GPW)) * 64) * 2 : -1;       // (a line of the wave's, by workgroup)
+            chain_until([&] { return __ballot(at >= 0 && __builtin_amdgcn_raw_buffer_load_b32(r_x, at, 0, 16) != NOT_YET) != 0ull; }, p.timeout);
         }
+        chain_until([&] {
+            request();
+            chain_landed<0>();
+            uint32_t most = 0;
+#pragma unroll
+            for (int i = 0; i < GPW * 4; i++) most = max(most, most4(*reinterpret_cast<const u32x4*>(mine + i * 1024 + lane * 16)));
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(most) :: "memory");
+            return __ballot(most == NOT_YET) == 0ull;
+        }, p.timeout);
+    } else {
+        request();
+    }
+    CH_TL(1);
     float4v acc[NST][1][NTL];
 #pragma unroll
     for (int s = 0; s < NST; s++)
@@ -342,7 +350,7 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
         for (int nt = 0; nt < NTL; nt++) acc[s][0][nt] = (float4v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < GPW; i++) {
-        if (i == GPW - 1) chain_landed<0>();
+        if (i == GPW - 1) chain_landed<0>();                          // (handed-off rows are there)
         else if (i == GPW - 2) chain_landed<4>();
         else if (i == GPW - 3) chain_landed<8>();
         else chain_landed<12>();
@@ -399,8 +407,8 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
             if (r_out < T) {
                 const __amdgpu_buffer_rsrc_t r_o = chain_rsrc(out32, (long)T * w.N * 4);
                 const int off = (r_out * w.N + cb * 16 * NTL * NST + c8) * 4;
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, (float4v){sum[0], sum[1], sum[2], sum[3]}), r_o, off, 0, 16);
-                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, (float4v){sum[4], sum[5], sum[6], sum[7]}), r_o, off + 16, 0, 16);
+                store16_sc1(r_o, off, (float4v){sum[0], sum[1], sum[2], sum[3]});
+                store16_sc1(r_o, off + 16, (float4v){sum[4], sum[5], sum[6], sum[7]});
             }
         } else {
             half8 o;
@@ -412,9 +420,7 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
             }
         }
     }
-    CH_TL(2);
-    chain_signal(sig_base, sig_shard, sig_reps);
-    CH_TL(3);
+    CH_TL(2); CH_TL(3);
 }
 
 // ── attention role: paged_attn_kernel<128, true, 8> (decode, one new token per sequence) ────────────────────────────────
@@ -489,16 +495,20 @@ __device__ __forceinline__ void chain_role_attn(const ChainArgs& p, int wg, unsi
                                               rope_mode, p.qk_mode == 1, p.qk_mode != 0, q16);
     const int phys_new = bt[last_blk];
     __builtin_amdgcn_sched_barrier(0);
-    // the q|k|v columns of this kv head: G + 2 heads, each one workgroup per 16-row block of the projection role
-    chain_wait(p.cnt + (CH_QKV_SLOT + kvh * CH_QKV_R) * CH_STRIDE, 1, CH_QKV_R, (unsigned)((G + 2) * (WIDE ? 1 : (p.qkv_half ? 4 : 2)) * ((p.T + 15) >> 4)), p.timeout);
-    CH_TL(1);
     half8 qf[KS];
     {
         const int q_dim = p.nq * HD, kv_dim = p.nkv * HD;
         const __half* qrow = p.qkv_out + (long)seq * (q_dim + 2 * kv_dim);
         const __half* src = rc < G ? qrow + (kvh * G + rc) * HD
                                    : rc == G ? qrow + q_dim + kvh * HD : qrow + q_dim + kv_dim + kvh * HD;
-        const RopeRow<HD> rr = rope_row16<HD, true>(src, coef, rope_mode, p.eps, q16);
+        RopeSource<HD> source;
+        chain_until([&] {
+            source = rope_source16_sc1<HD, true>(src, rope_mode, q16);
+            const uint2 c0 = __builtin_bit_cast(uint2, source.c0), c1 = __builtin_bit_cast(uint2, source.c1);
+            return __ballot(max(max(c0.x, c0.y), max(c1.x, c1.y)) == NOT_YET) == 0ull;
+        }, p.timeout);
+        CH_TL(1);
+        const RopeRow<HD> rr = rope_row16<HD>(source, coef, rope_mode, p.eps, q16);
         using hv = typename RopeRow<HD>::hv;
         hv z0, z1;
 #pragma unroll
@@ -690,17 +700,17 @@ __device__ __forceinline__ void chain_role_attn(const ChainArgs& p, int wg, unsi
 #pragma unroll
         for (int i = 0; i < DPT; i++) o.h[i] = (_Float16)(ov[i] * inv);
         __half* dst = p.attn_out + ((long)seq * p.nq + kvh * G + row) * HD + dl * DPT;
+        o.u = (unsigned long long)written2((uint32_t)(o.u >> 32)) << 32 | written2((uint32_t)o.u);
         __hip_atomic_store(reinterpret_cast<unsigned long long*>(dst), o.u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);     // 8-byte sc1 store
     }
     CH_TL(2);
-    chain_signal(p.cnt + CH_ATTN_SLOT * CH_STRIDE, unit % CH_ATTN_SH, CH_ATTN_R);
     keep_new();
     CH_TL(3);
 }
 
 // ── role B: residual += o; post-attention norm; router logits of this part's experts; candidates; in-launch merge ─────────
 // (add_rmsnorm_route_part_kernel<false> with arrive: grid (token, part) → wg = token·Q + part)
-__device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigned n_o_wgs, unsigned char* smem) {
+__device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigned char* smem) {
     const int H = p.H, Q = p.Q, num_experts = p.E, top_k = p.r_top_k;
     const long row = wg / Q;
     const int q = wg % Q;
@@ -735,32 +745,57 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
         }
     }
     __builtin_amdgcn_sched_barrier(0);
-    chain_wait(p.cnt + CH_O_SLOT * CH_STRIDE, CH_O_SH, CH_O_R, n_o_wgs, p.timeout);
-    CH_TL(1);
     float* red = part + tiles_q * 16 * (ksplit + 1);                  // [8] behind the logits
     unsigned long long* cand_s = reinterpret_cast<unsigned long long*>(red + 8);     // [8]
     const __amdgpu_buffer_rsrc_t r_x = chain_rsrc(p.o_part, (long)CH_O_KS * p.T * H * 4), r_res = chain_rsrc(p.res_a, (long)p.T * H * 2);
     half8 v[CH];
     float ss = 0.f;
+    // o_proj's row: its K parts (fp32) added in part order, rounded to the fp16 the projection's output is.  First one word of it, until it is there.
+    u32x4 parts[CH][CH_O_KS][2], res[CH];
+    if (wave * 64 < nvec) {
+        const int at = (int)((row * H + wave * 512) * 4);
+        chain_until([&] { return (uint32_t)__builtin_amdgcn_readfirstlane(__builtin_amdgcn_raw_buffer_load_b32(r_x, at, 0, 16)) != NOT_YET; }, p.timeout);
+    }
+    chain_until([&] {
+        uint32_t most = 0;
+#pragma unroll
+        for (int c = 0; c < CH; c++) {
+            const int i = threadIdx.x + c * 512;
+            if (i < nvec) {
+#pragma unroll
+                for (int ks = 0; ks < CH_O_KS; ks++) {
+                    const int o32 = (int)((((long)ks * p.T + row) * H + i * 8) * 4);
+                    parts[c][ks][0] = __builtin_amdgcn_raw_buffer_load_b128(r_x, o32, 0, 16);
+                    parts[c][ks][1] = __builtin_amdgcn_raw_buffer_load_b128(r_x, o32 + 16, 0, 16);
+                }
+                res[c] = __builtin_amdgcn_raw_buffer_load_b128(r_res, (int)((row * H + i * 8) * 2), 0, 16);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < CH; c++)
+            if ((int)threadIdx.x + c * 512 < nvec) {
+#pragma unroll
+                for (int ks = 0; ks < CH_O_KS; ks++) most = max(most, max(most4(parts[c][ks][0]), most4(parts[c][ks][1])));
+                if (p.has_a) most = max(most, most4(res[c]));         // (else it is an earlier launch's)
+            }
+        return __ballot(most == NOT_YET) == 0ull;
+    }, p.timeout);
+    CH_TL(1);
 #pragma unroll
     for (int c = 0; c < CH; c++) {
         const int i = threadIdx.x + c * 512;
         if (i < nvec) {
-            const int off = (int)((row * H + i * 8) * 2);
-            // o_proj's row: its K parts (fp32) added in part order, rounded to the fp16 the projection's output is
             float xs32[8];
 #pragma unroll
             for (int ks = 0; ks < CH_O_KS; ks++) {
-                const int o32 = (int)((((long)ks * p.T + row) * H + i * 8) * 4);
-                const float4v lo = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(r_x, o32, 0, 16));
-                const float4v hi = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(r_x, o32 + 16, 0, 16));
+                const float4v lo = __builtin_bit_cast(float4v, parts[c][ks][0]), hi = __builtin_bit_cast(float4v, parts[c][ks][1]);
 #pragma unroll
                 for (int j = 0; j < 4; j++) { xs32[j] = ks ? xs32[j] + lo[j] : lo[j]; xs32[4 + j] = ks ? xs32[4 + j] + hi[j] : hi[j]; }
             }
             half8 xv;
 #pragma unroll
             for (int j = 0; j < 8; j++) xv[j] = (_Float16)xs32[j];
-            half8 rv = load16_sc1(r_res, off);
+            half8 rv = __builtin_bit_cast(half8, res[c]);
 #pragma unroll
             for (int j = 0; j < 8; j++) rv[j] = (_Float16)((float)rv[j] + (float)xv[j]);
             v[c] = rv;
@@ -889,7 +924,7 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
     // next (the granules live in the double-buffered counter block: zero on entry).  One store → load latency instead of
     // store → drain → returning ticket → loads: 3.4–3.8 µs → ≈ 1.5 µs on the layer's critical path.
     //   candidate granule: [tag 1 : 16][expert id : 16][logit bits : 32]      statistic granule: [tag 1 : 32][value bits : 32]
-    unsigned long long* gran = reinterpret_cast<unsigned long long*>(p.cnt + CH_SLOTS * CH_STRIDE) + (row * Q) * CH_GRAN;
+    unsigned long long* gran = reinterpret_cast<unsigned long long*>(p.cnt) + (row * Q) * CH_GRAN;
     if (q != 0) {
         unsigned long long g = 0;
         if (lane < 8) g = (1ull << 48) | ((cand_s[lane] >> 32 & 0xffffull) << 32) | (cand_s[lane] & 0xffffffffull);
@@ -957,49 +992,43 @@ __global__ __launch_bounds__(512, 2) void decode_chain_kernel(ChainArgs p) {
     const int QB = WIDE ? 128 : (p.qkv_half ? 32 : 64);             // q|k|v block width
     const int n_a = p.has_a ? p.T : 0, n_qkv = p.qkv.N / QB * RH, n_attn = p.T * p.nkv * (KVS ? p.attn_splits : 1), n_o = p.o.N / (p.o_half ? 32 : 64 * CH_O_NST) * RH * CH_O_KS;
     int wg = blockIdx.x;
-    if (wg == 0) {                                                    // re-arm the other half: counters and route granules
-        if (threadIdx.x < CH_QKV_SLOT + CH_QKV_R * p.nkv) p.cnt_next[threadIdx.x * CH_STRIDE] = 0u;
-        for (int i = threadIdx.x; i < p.T * p.Q * CH_GRAN * 2; i += 512) p.cnt_next[CH_SLOTS * CH_STRIDE + i] = 0u;
+    if (wg == 0) {                                                    // re-arm the other half of the route granules
+        for (int i = threadIdx.x; i < p.T * p.Q * CH_GRAN * 2; i += 512) p.cnt_next[i] = 0u;
     }
     if (wg < n_a) { chain_role_a(p, wg, smem); return; }
     wg -= n_a;
     if (wg < n_qkv) {
-        // a column block is one head: its arrival counts for that head's kv head
-        const int cb = wg / RH, head = cb * QB / 128, G = p.nq / p.nkv;           // (a head is 128 columns)
-        const int kvh = head < p.nq ? head / G : (head < p.nq + p.nkv ? head - p.nq : head - p.nq - p.nkv);
-        const ChainEdge e{p.has_a ? p.cnt + CH_NORM_SLOT * CH_STRIDE : nullptr, CH_NORM_SH, CH_NORM_R, (unsigned)p.T};
+        const int cb = wg / RH;
         if constexpr (WIDE) {
             // one head (128 columns) per workgroup: half as many workgroups of twice the bytes — taken where the narrow blocks and the
             // attention role together exceed the workgroups the chip holds at once (decode_chain_f16)
-            chain_role_gemm<2, GPW_QKV, HAS_ZP>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, e,
-                                                p.cnt + (CH_QKV_SLOT + kvh * CH_QKV_R) * CH_STRIDE, 0, CH_QKV_R, p.timeout, smem, p);
+            chain_role_gemm<2, GPW_QKV, HAS_ZP>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, p.has_a != 0, smem, p);
         } else if (p.qkv_half)
-            chain_role_gemm<1, GPW_QKV, HAS_ZP, 2>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, e,
-                                                   p.cnt + (CH_QKV_SLOT + kvh * CH_QKV_R) * CH_STRIDE, 0, CH_QKV_R, p.timeout, smem, p);
+            chain_role_gemm<1, GPW_QKV, HAS_ZP, 2>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, p.has_a != 0, smem, p);
         else
-            chain_role_gemm<CH_QKV_NST, GPW_QKV, HAS_ZP>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, e,
-                                                         p.cnt + (CH_QKV_SLOT + kvh * CH_QKV_R) * CH_STRIDE, 0, CH_QKV_R, p.timeout, smem, p);
+            chain_role_gemm<CH_QKV_NST, GPW_QKV, HAS_ZP>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, p.has_a != 0, smem, p);
+        // (behind its own result; read by the launch after this one)
+        const __amdgpu_buffer_rsrc_t r_n = chain_rsrc(p.rows_next, (long)p.rows_next_pieces * 16);
+        for (int i = wg * 512 + threadIdx.x; i < p.rows_next_pieces; i += n_qkv * 512)
+            __builtin_amdgcn_raw_buffer_store_b128((u32x4){NOT_YET, NOT_YET, NOT_YET, NOT_YET}, r_n, i * 16, 0, 16);
         return;
     }
     wg -= n_qkv;
     if (wg < n_attn) { chain_role_attn<KVS, WIDE>(p, wg, smem); return; }
     wg -= n_attn;
     if (wg < n_o) {
-        const ChainEdge e{p.cnt + CH_ATTN_SLOT * CH_STRIDE, CH_ATTN_SH, CH_ATTN_R, (unsigned)(p.T * p.nkv)};      // (one arrival per (sequence, kv head): its last split's)
         // (K part fastest: the two workgroups of a block are neighbours)
         static_assert(GPW_O % CH_O_KS == 0, "o_proj's quant groups per wave divide over its K parts");
         const int ks = wg % CH_O_KS, blk = wg / CH_O_KS;
         float* part = p.o_part + (long)ks * p.T * p.o.N;
         if (p.o_half)
-            chain_role_gemm<1, GPW_O / CH_O_KS, HAS_ZP, 2, true>(p.o, blk / RH, blk % RH, p.attn_out, nullptr, p.T, e, p.cnt + CH_O_SLOT * CH_STRIDE,
-                                                                 wg % CH_O_SH, CH_O_R, p.timeout, smem, p, ks * (p.o.G / CH_O_KS), part);
+            chain_role_gemm<1, GPW_O / CH_O_KS, HAS_ZP, 2, true>(p.o, blk / RH, blk % RH, p.attn_out, nullptr, p.T, true, smem, p, ks * (p.o.G / CH_O_KS), part);
         else
-            chain_role_gemm<CH_O_NST, GPW_O / CH_O_KS, HAS_ZP, 4, true>(p.o, blk / RH, blk % RH, p.attn_out, nullptr, p.T, e, p.cnt + CH_O_SLOT * CH_STRIDE,
-                                                                        wg % CH_O_SH, CH_O_R, p.timeout, smem, p, ks * (p.o.G / CH_O_KS), part);
+            chain_role_gemm<CH_O_NST, GPW_O / CH_O_KS, HAS_ZP, 4, true>(p.o, blk / RH, blk % RH, p.attn_out, nullptr, p.T, true, smem, p, ks * (p.o.G / CH_O_KS), part);
         return;
     }
     wg -= n_o;
-    chain_role_b(p, wg, (unsigned)n_o, smem);
+    chain_role_b(p, wg, smem);
 }
 
 }  // namespace
@@ -1008,7 +1037,9 @@ __global__ __launch_bounds__(512, 2) void decode_chain_kernel(ChainArgs p) {
 extern "C" __attribute__((visibility("default"))) void ferrum_hip_debug_set_chain_timeline(void* p) { g_chain_timeline = (unsigned long long*)p; }
 #endif
 
-int decode_chain_counter_words() { return CH_SLOTS * CH_STRIDE + CH_GRAN_WORDS; }
+int decode_chain_counter_words() { return CH_GRAN_WORDS; }
+// handed-off rows of a token: role A's two, q|k|v's, attention's, o_proj's K parts
+size_t decode_chain_row_bytes(int H, int nq, int nkv) { return (size_t)4 * H + ((size_t)nq + 2 * nkv) * 256 + (size_t)nq * 256 + (size_t)CH_O_KS * 4 * H; }
 
 bool decode_chain_supports(const DecodeChainDesc& d) {
     const auto gemm_ok = [](const W4Device& w) {
@@ -1017,7 +1048,7 @@ bool decode_chain_supports(const DecodeChainDesc& d) {
     };
     if (!d.qkv || !d.o || !gemm_ok(*d.qkv) || !gemm_ok(*d.o)) return false;
     if (d.o->G / 8 != 4) return false;              // (the instantiated forms: o_proj's K slice per wave is four groups)
-    if (!d.o_part) return false;
+    if (!d.rows || !d.rows_next || CH_MAX_T * decode_chain_row_bytes(d.H, d.nq, d.nkv) >= (1UL << 31)) return false;
     if (d.attn_splits > CH_MAX_SPLITS || (d.attn_splits > 1 && (!d.attn_partial || !d.attn_tickets))) return false;
     if (d.T < 1 || d.T > CH_MAX_T || d.head_dim != 128 || d.nkv < 1 || d.nq % d.nkv != 0 || d.nq / d.nkv > 14 || d.nkv > CH_MAX_KVH) return false;
     if (d.H % 32 != 0 || d.H > 8192 || d.qkv->k != d.H || d.qkv->n != (d.nq + 2 * d.nkv) * 128 || d.o->k != d.nq * 128 || d.o->n != d.H) return false;
@@ -1041,16 +1072,22 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
     a.has_a = d.has_a ? (d.E > 0 ? 1 : (d.a_x ? 3 : 2)) : 0; a.top_k = d.top_k;
     a.a_x = d.a_x;
     a.a_slabs = d.a_slabs; a.a_S = d.a_S; a.a_slab_stride = d.a_slab_stride; a.a_ld = d.a_ld; a.down = d.down; a.comb_w = d.comb_w; a.res_in = d.res_in; a.ln_in = d.ln_in;
-    a.eps = d.eps; a.res_a = d.res_a; a.norm1 = d.norm1;
+    a.eps = d.eps;
+    unsigned char* rows = d.rows;
+    auto take = [&](size_t bytes) { unsigned char* at = rows; rows += bytes * d.T; return at; };
+    a.norm1 = reinterpret_cast<__half*>(take((size_t)2 * d.H));
+    a.res_a = reinterpret_cast<__half*>(take((size_t)2 * d.H));
+    if (!d.has_a) { a.norm1 = d.norm1; a.res_a = d.res_a; }
+    a.qkv_out = reinterpret_cast<__half*>(take(((size_t)d.nq + 2 * d.nkv) * 256));
+    a.attn_out = reinterpret_cast<__half*>(take((size_t)d.nq * 256));
+    a.o_part = reinterpret_cast<float*>(take((size_t)CH_O_KS * 4 * d.H));
+    a.rows_next = reinterpret_cast<uint32_t*>(d.rows_next); a.rows_next_pieces = (int)((rows - d.rows) / 16);
     a.qkv = ChainGemm{d.qkv->qw, d.qkv->sc, d.qkv->zp, d.qkv->G, d.qkv->n, d.qkv->k};
-    a.qkv_out = d.qkv_out;
     a.k_pool = d.k_pool; a.v_pool = d.v_pool; a.block_tables = d.block_tables; a.kv_lens = d.kv_lens;
     a.q_norm_w = d.q_norm_w; a.k_norm_w = d.k_norm_w; a.cos_t = d.cos_t; a.sin_t = d.sin_t;
     a.qk_mode = d.qk_mode; a.max_blocks = d.max_blocks; a.sliding_window = d.sliding_window;
     a.scale = 1.0f / sqrtf((float)d.head_dim);
-    a.attn_out = d.attn_out;
     a.o = ChainGemm{d.o->qw, d.o->sc, d.o->zp, d.o->G, d.o->n, d.o->k};
-    a.o_out = d.o_out;
     a.res_b_out = d.res_b_out; a.post_ln = d.post_ln; a.norm2 = d.norm2; a.router_w = d.router_w;
     a.E = d.E; a.r_top_k = d.r_top_k; a.Q = d.Q; a.norm_topk = d.norm_topk; a.defer_merge = d.defer_merge ? 1 : 0;
     a.cand = d.cand; a.stats = d.stats; a.route_arrive = d.route_arrive; a.ids = d.ids; a.weights = d.weights;
@@ -1068,7 +1105,6 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
     // 128-column q|k|v blocks (hidden 2048 only: the two-group weight ring): where the 64-column blocks + the attention role do not fit
     // the chip's resident workgroups, the role's last workgroups enter behind the projection (≈ 2.7 µs of K/V round trips on the
     // critical path, profiles/r03_decode_chain_timeline.txt) — c=32 4.025 → 3.995 ms per step, c=64 4.83 → 4.69; c=20–24 (where they fit) 3 % slower
-    a.o_part = d.o_part;
     a.qkv_wide = 0;
     if (!a.qkv_half && d.qkv->G / 8 == 2 && a.attn_splits == 1) {
         const int wide = knobs().chain_qkv_wide;

@@ -116,8 +116,8 @@ int f16t_gemm_f32out(const __half* x, const __half* wt, float* out, int m, int n
 // ── norms / elementwise (norm.hip) ───────────────────────────────────────────
 int rms_norm_f16(const __half* x, const __half* w, float eps, __half* out, int tokens, int dim, hipStream_t s);
 int embed_rms_norm_f16(const __half* table, const uint32_t* token_ids, float embed_scale, __half* residual, float* residual_f32,
-                       const __half* w, float eps, __half* norm_out, int tokens, int dim, unsigned* zero_words, int n_zero, hipStream_t s,
-                       const int32_t* out_perm = nullptr);   // out_perm: norm_out[row][j] = y[out_perm[j]] (act-order consumer)
+                       const __half* w, float eps, __half* norm_out, int tokens, int dim, unsigned* zero_words, int n_zero, unsigned* ones, int n_ones,
+                       hipStream_t s, const int32_t* out_perm = nullptr);   // out_perm: norm_out[row][j] = y[out_perm[j]] (act-order consumer)
 int gather_rms_norm_f16(const __half* x, const int32_t* row_idx, const __half* w, float eps, __half* out, int rows, int dim, hipStream_t s);
 int fused_add_rms_norm_f16(__half* residual, const __half* x, const __half* w, float eps, __half* out,
                            int tokens, int dim, hipStream_t s, const int32_t* out_perm = nullptr);
@@ -253,6 +253,7 @@ int fused_add_rms_norm_route_parts_f16(const __half* residual_in, __half* residu
 // [combine + add + norm of the previous layer's tail] → q|k|v → QK-norm / RoPE / KV write / attention → o_proj →
 // add + norm + router + top-k, as roles of one grid with in-launch hand-offs.  Buffers as the stand-alone kernels use them.
 constexpr int CHAIN_MAX_ATTN_WGS = 1024;      // (sequence, kv head, KV split) workgroups whose states the split buffer holds
+constexpr int CHAIN_MAX_ROWS = 128;
 struct DecodeChainDesc {
     int T = 0, H = 0, nq = 0, nkv = 0, head_dim = 0;
     bool has_a = false;          // the previous layer's tail runs as the first role (else norm1 / res_a come from an earlier launch)
@@ -262,27 +263,28 @@ struct DecodeChainDesc {
     const float* a_slabs = nullptr; int a_S = 0; long a_slab_stride = 0; int a_ld = 0;
     const __half* a_x = nullptr;  // … or, without slabs, the MLP output as fp16 rows [T, H]
     float eps = 0.f;
-    __half* res_a = nullptr;     // residual after the tail (role A's output, role B's input)
-    __half* norm1 = nullptr;     // [T, H] input rows of the q|k|v projection
-    const W4Device* qkv = nullptr; __half* qkv_out = nullptr;
+    // without a tail: the residual, and the input rows of the q|k|v projection, [T, H] each
+    __half* res_a = nullptr; __half* norm1 = nullptr;
+    const W4Device* qkv = nullptr;
     __half* k_pool = nullptr; __half* v_pool = nullptr; const int32_t* block_tables = nullptr; const uint32_t* kv_lens = nullptr;
     const __half* q_norm_w = nullptr; const __half* k_norm_w = nullptr; const float* cos_t = nullptr; const float* sin_t = nullptr;
     int qk_mode = 0, max_blocks = 0, sliding_window = 0;
-    __half* attn_out = nullptr;
-    const W4Device* o = nullptr; __half* o_out = nullptr;
+    const W4Device* o = nullptr;
     __half* res_b_out = nullptr; const __half* post_ln = nullptr; __half* norm2 = nullptr; const __half* router_w = nullptr;
     int E = 0, r_top_k = 0, Q = 0, norm_topk = 0;
     bool defer_merge = false;    // role B stops at the per-part candidate lists (cand / stats); the grouped GEMM that follows merges them
     RouteCand* cand = nullptr; float* stats = nullptr; unsigned* route_arrive = nullptr; int32_t* ids = nullptr; float* weights = nullptr;
-    float* o_part = nullptr;       // [2][T][H] fp32: o_proj's two K parts (one workgroup each per block; role B adds them)
+    // rows handed off inside the launch, decode_chain_row_bytes for each token: all ones on entry, and the launch leaves all ones in the other half
+    unsigned char *rows = nullptr, *rows_next = nullptr;
     int attn_splits = 1;           // KV ranges per (sequence, kv head) in the attention role (≤ 16); > 1 needs the two buffers below
     float* attn_partial = nullptr; // [T·nkv·attn_splits][16][head_dim + 4] fp32
     unsigned* attn_tickets = nullptr;   // [T·nkv] zeroed words (self-resetting)
-    unsigned* cnt = nullptr;       // decode_chain_counter_words() words, zero on entry
+    unsigned* cnt = nullptr;       // the router's granules: decode_chain_counter_words() words, zero on entry
     unsigned* cnt_next = nullptr;  // the other half of the double buffer: zeroed by this launch
     unsigned* timeout = nullptr;   // host-visible word, bumped by a bounded wait that gave up
 };
 int decode_chain_counter_words();
+size_t decode_chain_row_bytes(int H, int nq, int nkv);
 bool decode_chain_supports(const DecodeChainDesc& d);
 int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream);
 

@@ -122,20 +122,18 @@ int fused_add_rms_norm_f16(__half* residual, const __half* x, const __half* w, f
 // Head / tail of a forward in ONE launch each (a dependent launch costs ≈ 4 µs even when trivial; a decode step had nine of
 // them outside the layers): gather a row (embedding row by token id, or residual row by sampled index) → optional scale
 // (fp16 rounding, like scale_inplace) → optional copies of the gathered row (fp16 residual, fp32 residual stream) →
-// rms_norm·w → out.  Same per-element arithmetic as embedding_lookup → scale_inplace → rms_norm.  Block 0 also zeroes
-// `zero_words` (the split router's arrival counters, re-armed per forward).
+// rms_norm·w → out.  Same per-element arithmetic as embedding_lookup → scale_inplace → rms_norm.  The blocks also zero
+// `zero_words` (counters, re-armed per forward) and set `ones` to all ones (the rows that the first chain launch hands off), in 16-byte pieces.
 template <typename IdxT, int CHUNKS>
 __global__ __launch_bounds__(256) void gather_rms_norm_kernel(const __half* __restrict__ table, const IdxT* __restrict__ ids, float scale,
                                                               __half* __restrict__ copy_f16, float* __restrict__ copy_f32,
                                                               const __half* __restrict__ w, float eps, __half* __restrict__ out, int dim,
-                                                              unsigned* __restrict__ zero_words, int n_zero,
+                                                              unsigned* __restrict__ zero_words, int n_zero, unsigned* __restrict__ ones, int n_ones,
                                                               const int32_t* __restrict__ out_perm) {
     __shared__ float smem[4];
     extern __shared__ _Float16 stage[];            // dim halves when out_perm
     const long row = blockIdx.x;
     const long src = (long)ids[row];
-    if (blockIdx.x == 0 && zero_words)
-        for (int i = threadIdx.x; i < n_zero; i += 256) zero_words[i] = 0u;
     const int nvec = dim >> 3;
     half8 v[CHUNKS], wv[CHUNKS];
 #pragma unroll
@@ -181,17 +179,22 @@ __global__ __launch_bounds__(256) void gather_rms_norm_kernel(const __half* __re
         }
     }
     if (out_perm) store_row_gathered_256(out + row * dim, stage, out_perm, nvec);
+    if (zero_words)
+        for (int i = (int)row * 256 + threadIdx.x; i < n_zero / 4; i += gridDim.x * 256) reinterpret_cast<uint4*>(zero_words)[i] = uint4{0u, 0u, 0u, 0u};
+    if (ones)
+        for (int i = (int)row * 256 + threadIdx.x; i < n_ones / 4; i += gridDim.x * 256) reinterpret_cast<uint4*>(ones)[i] = uint4{~0u, ~0u, ~0u, ~0u};
 }
 
 template <typename IdxT>
 static int launch_gather_rms(const __half* table, const IdxT* ids, float scale, __half* copy_f16, float* copy_f32, const __half* w, float eps,
-                             __half* out, int rows, int dim, unsigned* zero_words, int n_zero, const int32_t* out_perm, hipStream_t s) {
+                             __half* out, int rows, int dim, unsigned* zero_words, int n_zero, unsigned* ones, int n_ones, const int32_t* out_perm, hipStream_t s) {
     if (rows <= 0) return 0;
+    FH_REQUIRE(n_zero % 4 == 0 && n_ones % 4 == 0, "gather_rms_norm: %d / %d words", n_zero, n_ones);
     FH_REQUIRE(dim % 8 == 0 && dim <= 8 * 256 * 8, "gather_rms_norm: dim=%d must be a multiple of 8 and <= 16384", dim);
     const int chunks = cdiv(dim / 8, 256);
     dim3 grid(rows), block(256);
     const size_t lds = out_perm ? (size_t)dim * 2 : 0;
-#define FH_GRN(C) hipLaunchKernelGGL((gather_rms_norm_kernel<IdxT, C>), grid, block, lds, s, table, ids, scale, copy_f16, copy_f32, w, eps, out, dim, zero_words, n_zero, out_perm)
+#define FH_GRN(C) hipLaunchKernelGGL((gather_rms_norm_kernel<IdxT, C>), grid, block, lds, s, table, ids, scale, copy_f16, copy_f32, w, eps, out, dim, zero_words, n_zero, ones, n_ones, out_perm)
     if (chunks <= 1) FH_GRN(1); else if (chunks <= 2) FH_GRN(2); else if (chunks <= 4) FH_GRN(4); else FH_GRN(8);
 #undef FH_GRN
     FH_CHECK_LAUNCH();
@@ -200,13 +203,13 @@ static int launch_gather_rms(const __half* table, const IdxT* ids, float scale, 
 // embedding_lookup (+ scale_inplace) + rms_norm of layer 0, the residual stream written on the way (fp16, and fp32 for
 // sandwich-norm models)
 int embed_rms_norm_f16(const __half* table, const uint32_t* token_ids, float embed_scale, __half* residual, float* residual_f32,
-                       const __half* w, float eps, __half* norm_out, int tokens, int dim, unsigned* zero_words, int n_zero, hipStream_t s,
-                       const int32_t* out_perm) {
-    return launch_gather_rms<uint32_t>(table, token_ids, embed_scale, residual, residual_f32, w, eps, norm_out, tokens, dim, zero_words, n_zero, out_perm, s);
+                       const __half* w, float eps, __half* norm_out, int tokens, int dim, unsigned* zero_words, int n_zero, unsigned* ones, int n_ones,
+                       hipStream_t s, const int32_t* out_perm) {
+    return launch_gather_rms<uint32_t>(table, token_ids, embed_scale, residual, residual_f32, w, eps, norm_out, tokens, dim, zero_words, n_zero, ones, n_ones, out_perm, s);
 }
 // gather_rows + rms_norm on the sampled rows (final norm)
 int gather_rms_norm_f16(const __half* x, const int32_t* row_idx, const __half* w, float eps, __half* out, int rows, int dim, hipStream_t s) {
-    return launch_gather_rms<int32_t>(x, row_idx, 0.0f, nullptr, nullptr, w, eps, out, rows, dim, nullptr, 0, nullptr, s);
+    return launch_gather_rms<int32_t>(x, row_idx, 0.0f, nullptr, nullptr, w, eps, out, rows, dim, nullptr, 0, nullptr, 0, nullptr, s);
 }
 
 // ── row gathers ──────────────────────────────────────────────────────────────

@@ -58,7 +58,7 @@ __device__ __forceinline__ RopeSource<HD> rope_source16(const __half* src, int m
     return {*reinterpret_cast<const hv*>(src + rope_off0<HD>(mode, q16)), *reinterpret_cast<const hv*>(src + rope_off1<HD>(mode, q16))};
 }
 
-// SC1: the source row was written by another workgroup of THIS launch (write-through stores behind a counter): it is read with
+// SC1: the source row was written by another workgroup of THIS launch (write-through stores): it is read with
 // L1-bypassing loads (relaxed agent-scope 8-byte loads; head_dim 128 only).
 template <int HD, bool SC1 = false>
 __device__ __forceinline__ RopeSource<HD> rope_source16_sc1(const __half* src, int mode, int q16) {
@@ -127,10 +127,6 @@ __device__ __forceinline__ RopeRow<HD> rope_row16(const RopeSource<HD>& source, 
 #pragma unroll
     for (int k = 0; k < PPL; k++) { r.out0[k] = (_Float16)o[k]; r.out1[k] = (_Float16)o[PPL + k]; }
     return r;
-}
-template <int HD, bool SC1>
-__device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const RopeCoef<HD>& coef, int mode, float eps, int q16) {
-    return rope_row16<HD>(rope_source16_sc1<HD, SC1>(src, mode, q16), coef, mode, eps, q16);
 }
 template <int HD>
 __device__ __forceinline__ RopeRow<HD> rope_row16(const __half* src, const __half* nw, const float* cs, const float* sn,

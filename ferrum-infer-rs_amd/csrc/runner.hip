@@ -463,7 +463,7 @@ int ferrum_hip_model_destroy(FerrumHipModel* m) {
                     (void*)m->sampled_hidden, (void*)m->moe_act, (void*)m->moe_down, (void*)m->moe_gather_x, (void*)m->moe_gather_h, (void*)m->router_logits,
                     (void*)m->expert_ids, (void*)m->sorted_ids, (void*)m->block_ids, (void*)m->total_post_pad,
                     (void*)m->expert_w, (void*)m->logits, (void*)m->out_tokens, (void*)m->workspace, (void*)m->taps,
-                    (void*)m->idx_dev, (void*)m->step_counter, (void*)m->residual2, (void*)m->chain_o_part, (void*)m->chain_attn_partial, (void*)m->chain_attn_tickets,
+                    (void*)m->idx_dev, (void*)m->step_counter, (void*)m->residual2, (void*)m->chain_rows, (void*)m->chain_attn_partial, (void*)m->chain_attn_tickets,
                     (void*)m->route_cand, (void*)m->route_stats, (void*)m->route_arrive, (void*)m->cos_local,
                     (void*)m->sin_local, (void*)m->residual_f32, (void*)m->gather_scratch, (void*)m->greedy_opts_dev, (void*)m->tp_tmp,
                     (void*)m->expert_ids_local, (void*)m->ones, m->vp_pairs, m->vp_gathered})
@@ -929,7 +929,10 @@ int ferrum_hip_model_finalize(FerrumHipModel* m) {
             *m->inlaunch_timeouts = 0u;
         }
     }
-    if (!rc && m->em2_arrive) rc |= dev_alloc(&m->chain_o_part, (size_t)4 * 128 * H);
+    if (!rc && m->em2_arrive) {
+        m->chain_rows_half = CHAIN_MAX_ROWS * decode_chain_row_bytes((int)H, c.num_heads, c.num_kv_heads);
+        rc |= dev_alloc(&m->chain_rows, 2 * m->chain_rows_half);
+    }
     if (!rc && m->em2_arrive && c.head_dim == 128) {
         rc |= dev_alloc(&m->chain_attn_partial, (size_t)CHAIN_MAX_ATTN_WGS * 16 * (c.head_dim + 4));
         rc |= dev_alloc(&m->chain_attn_tickets, (size_t)4096);
@@ -1396,9 +1399,11 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
     // act-order (desc_act) projections read x'[j] = x[perm[j]]: the kernel that PRODUCES the row writes it permuted wherever one
     // workgroup owns the row (every norm of the dense layer) or the rows are few (decode attention scatters); the gated
     // activation is permuted by gate_up's column order (pack_gate_up).  Only the prefill o_proj keeps a gather launch.
+    const bool chain_rows = m->chain_rows && sh.all_single_token && T <= std::min(CHAIN_MAX_ROWS, knobs().chain_max_rows);
     RUN(embed_rms_norm_f16(m->embed, tokens, c.embed_scale, m->residual, sandwich ? m->residual_f32 : nullptr, m->layers[0].input_ln,
-                           c.rms_eps, m->norm_out, T, H, m->route_arrive, m->route_arrive ? 64 + (int)m->arrive_half_words : 0, s, m->layers[0].qkv.perm));
-    m->em2_parity = 0;          // the head kernel zeroed half 0 of the merged launches' counters; every such launch zeroes the other half
+                           c.rms_eps, m->norm_out, T, H, m->route_arrive, m->route_arrive ? 64 + (int)m->arrive_half_words : 0,
+                           chain_rows ? reinterpret_cast<unsigned*>(m->chain_rows) : nullptr, chain_rows ? (int)(T * decode_chain_row_bytes(H, nq, nkv) / 4) : 0, s, m->layers[0].qkv.perm));
+    m->em2_parity = 0;          // the head kernel made half 0 of the merged launches' counters and rows ready; every such launch does that to the other half
     m->chain_parity = 0;
     bool qkv_in_perm = m->layers[0].qkv.perm != nullptr;      // norm_out holds the row in L.qkv's packed order
     // decode at ≤ 4 rows (MoE models): the tail of layer l — combine + residual add + next input norm — runs as the prologue of
@@ -1412,7 +1417,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
         d.T = T; d.H = H; d.nq = nq; d.nkv = nkv; d.head_dim = hd;
         d.top_k = c.top_k; d.down = m->moe_down; d.comb_w = m->expert_w; d.res_in = m->residual2; d.ln_in = L.input_ln; d.eps = c.rms_eps;
         d.res_a = m->residual; d.norm1 = m->norm_out;
-        d.qkv = &L.qkv; d.qkv_out = m->qkv_out;
+        d.qkv = &L.qkv;
         d.k_pool = L.k_pool; d.v_pool = L.v_pool; d.block_tables = bt; d.kv_lens = kvl;
         d.q_norm_w = L.q_norm ? L.q_norm : L.input_ln; d.k_norm_w = L.k_norm ? L.k_norm : L.input_ln;
         const int pattern = c.sliding_window_pattern;
@@ -1421,7 +1426,8 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
         d.cos_t = (!is_global && m->cos_local) ? m->cos_local : m->cos_t;
         d.sin_t = (!is_global && m->sin_local) ? m->sin_local : m->sin_t;
         d.qk_mode = qk_mode; d.max_blocks = m->max_blocks_per_seq;
-        d.attn_out = m->attn_out; d.o = &L.o; d.o_out = m->o_out; d.o_part = m->chain_o_part;
+        d.o = &L.o;
+        if (m->chain_rows) { d.rows = m->chain_rows + m->chain_parity * m->chain_rows_half; d.rows_next = m->chain_rows + (m->chain_parity ^ 1) * m->chain_rows_half; }
         d.res_b_out = m->residual2; d.post_ln = L.post_ln; d.norm2 = m->norm_out; d.router_w = L.router;
         d.E = c.num_experts; d.r_top_k = c.top_k; d.norm_topk = c.norm_topk_prob;
         int Q = m->route_parts;

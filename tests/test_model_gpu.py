@@ -966,6 +966,49 @@ def test_decode_chain_of_a_router_with_nan(pkg, c, bits, forms, knobs):
     assert np.abs(out[1] - out[0]).max() < 0.02 * np.abs(out[0]).max()
 
 
+@pytest.mark.parametrize("bits", [0xffff, 0x7fff, 0x7c00])
+@pytest.mark.parametrize("c", [1, 5, 17])
+def test_decode_chain_hands_off_every_number(pkg, c, bits, forms, knobs):
+    """Rows handed off inside the launch are their own flags, all ones while unwritten: numbers of that pattern (a norm's weights of NaN, in both halves
+    of a word, in one and across two) arrive as NaN too, and infinities as they are; no wait gives up (the call would fail)."""
+    tm = _chain_model()
+    L = tm.layers[1]["dense"]
+    kept = L["input_ln"]
+    try:
+        L["input_ln"] = kept.copy()
+        L["input_ln"][[6, 7, 12, 19, 20]] = np.array([bits], np.uint16).view(np.float16).astype(np.float32)
+        out = {}
+        for chain in (1, 0):
+            knobs.set(DECODE_CHAIN=chain, MOE_EM2=chain)
+            hm = tm.hip_model(pkg, kv_num_blocks=c * 2 + 4, max_seqs=c, max_tokens=64)
+            hm.unified_forward([(i, [7 + i, 300, 21], 0, True) for i in range(c)], greedy=True)
+            forms.reset()
+            out[chain] = hm.unified_forward([(i, [50 + i], 3, True) for i in range(c)], greedy=True, want_logits=True)[1]
+            assert forms.hits().get("decode_chain", 0) == (3 if chain else 0), forms.hits()
+            del hm
+    finally:
+        L["input_ln"] = kept
+    assert np.isnan(out[0]).all() and np.isnan(out[1]).all()
+
+
+def test_decode_chain_of_batches_that_change(pkg, knobs):
+    """The handed-off rows of a step lie by its batch: sequences join and leave between steps, and every step is what launches of their own make of it."""
+    tm = _chain_model()
+    out = {}
+    for chain in (1, 0):
+        knobs.set(DECODE_CHAIN=chain, MOE_EM2=chain)
+        hm = tm.hip_model(pkg, kv_num_blocks=33 * 2 + 4, max_seqs=33, max_tokens=128)
+        hm.unified_forward([(i, [7 + i, 300, 21], 0, True) for i in range(33)], greedy=True)
+        at, out[chain] = [3] * 33, []
+        for step, c in enumerate((33, 1, 16, 4, 5, 17, 2, 33)):
+            seqs = [(i * 7 + step) % 33 for i in range(c)]
+            out[chain].append(hm.unified_forward([(i, [50 + i + step], at[i], True) for i in seqs], greedy=True, want_logits=True)[1])
+            for i in seqs: at[i] += 1
+        del hm
+    for mine, other in zip(out[1], out[0]):
+        assert np.abs(mine - other).max() < 0.02 * np.abs(other).max()
+
+
 @pytest.mark.parametrize("c", [1, 4, 8, 9, 16, 17])
 def test_decode_chain_of_wide_layers(pkg, c, forms):
     """Hidden 4096: four quant groups a wave in the q|k|v role (two for hidden 2048), its blocks 32 columns wide up to the rows at which they and
