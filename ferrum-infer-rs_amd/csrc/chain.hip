@@ -1,4 +1,4 @@
-// The attention half of a MoE decode layer as ONE launch (gfx950).
+// The attention half of a decode layer as ONE launch (gfx950).
 //
 // A decode step of ≤ 32 rows is a chain of small dependent ops (qwen3_moe_forward_unified_layer.rs:46-455 issues them one
 // launch at a time): [tail of the previous layer: combine + add + norm] → q|k|v GEMM → QK-norm + RoPE + paged-KV write +
@@ -55,7 +55,7 @@ constexpr int CH_QKV_NST = 1, CH_O_NST = 1;     // 64-column supertiles per work
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct ChainGemm {
-    const uint32_t* qw; const __half* sc; const __half* zp;
+    const void* qw; const __half* sc;           // INT4 pack and its scales, or f16t tiles
     int G, N, K;
 };
 
@@ -254,12 +254,14 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
 // Behind the wait of 12 rows of 4096, 64 columns: 0.9 µs until the rows are there, 1.0 the products, 0.8 the slowest wave's and the meeting, 0.5
 // the result (64-byte pieces of 16 rows, two groups ahead, weights expanded behind the wait: 4.1 in all, now 3.2; 16 rows of 2048 in
 // 128 columns 4.2 → 3.3, o_proj's halves of K 2.7 → 2.0).
+// F16W: unquantised weights, fp16 fragments of a tile row after row of K, all of a wave's (32 – 128 registers) requested before the wait and
+// nothing left to expand; the products go straight into the sums.
 // NTL = 16-column tiles of the 64-column supertile a workgroup takes (NST = 1): 4, or 2 — a 32-column block `cb` = supertile cb / 2,
 // half cb % 2: half the weight bytes per workgroup, twice the workgroups (the stage is as long as its slowest workgroup's fetch).
 // F32OUT: the workgroup covers only the quant groups from g_base on (8·GPW of them) and leaves its fp32 partial sums in `out32`
 // ([K part][T][N]) — o_proj split over two workgroups per block: the rows a workgroup reads behind its wait (T·K·2 B through one CU)
 // are what its stage takes, and role B adds the two parts
-template <int NST, int GPW, bool HAS_ZP, int NTL = 4, bool F32OUT = false>
+template <int NST, int GPW, bool F16W, int NTL = 4, bool F32OUT = false>
 __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int rb, const __half* x_in, __half* out, int T,
                                                 bool handed_off, unsigned char* smem, const ChainArgs& p, int g_base = 0, float* out32 = nullptr) {
     static_assert(NTL == 4 || (NTL == 2 && NST == 1), "half supertiles only for single-supertile blocks");
@@ -270,24 +272,37 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
     CH_TL(0);
     const int g0 = g_base + wave * GPW;                               // G = 8·GPW (· 2 with F32OUT; checked by the launcher)
     const int nt0 = NTL == 2 ? (cb & 1) * 2 : 0;                      // first tile of the block inside its supertile
-    u32x4 wq[GPW][NST][NTL];
-    uint2 scv[GPW][NST], zpv[GPW][NST];
+    constexpr int FIT = 8 / (NST * NTL), PRE = F16W || GPW < FIT ? GPW : FIT;       // (128 registers)
+    static_assert(!F16W || GPW <= FIT, "16-bit weights: all of a wave's in registers");
+    u32x4 wq[F16W ? 1 : GPW][NST][NTL];
+    uint2 scv[F16W ? 1 : GPW][NST];
+    half8 wx[PRE][NST][NTL][4];
+    if constexpr (F16W) {
+        const half8* w_lane = reinterpret_cast<const half8*>(w.qw) + lane;          // f16t: [N / 16][K / 32][64 lanes]
 #pragma unroll
-    for (int i = 0; i < GPW; i++)
+        for (int i = 0; i < GPW; i++)
 #pragma unroll
-        for (int s = 0; s < NST; s++) {
-            const long st = NTL == 2 ? (long)(cb >> 1) : (long)cb * NST + s;
-            const u32x4* qw_lane = reinterpret_cast<const u32x4*>(w.qw) + (st * w.G * 4) * 64 + lane;
+            for (int s = 0; s < NST; s++)
 #pragma unroll
-            for (int nt = 0; nt < NTL; nt++) wq[i][s][nt] = __builtin_nontemporal_load(qw_lane + ((long)(g0 + i) * 4 + nt0 + nt) * 64);
-            scv[i][s] = (reinterpret_cast<const uint2*>(w.sc) + (st * w.G) * 16 + b)[(long)(g0 + i) * 16];
-            if (HAS_ZP) zpv[i][s] = (reinterpret_cast<const uint2*>(w.zp) + (st * w.G) * 16 + b)[(long)(g0 + i) * 16];
-        }
-    // the first PRE groups' weights become numbers (q − 8) while the predecessor works: their expansion, and the products that take the
+                for (int nt = 0; nt < NTL; nt++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        wx[i][s][nt][k] = __builtin_nontemporal_load(w_lane + (((long)(cb * NST + s) * NTL + nt) * (w.K / 32) + (g0 + i) * 4 + k) * 64);
+    } else {
+#pragma unroll
+        for (int i = 0; i < GPW; i++)
+#pragma unroll
+            for (int s = 0; s < NST; s++) {
+                const long st = NTL == 2 ? (long)(cb >> 1) : (long)cb * NST + s;
+                const u32x4* qw_lane = reinterpret_cast<const u32x4*>(w.qw) + (st * w.G * 4) * 64 + lane;
+#pragma unroll
+                for (int nt = 0; nt < NTL; nt++) wq[i][s][nt] = __builtin_nontemporal_load(qw_lane + ((long)(g0 + i) * 4 + nt0 + nt) * 64);
+                scv[i][s] = (reinterpret_cast<const uint2*>(w.sc) + (st * w.G) * 16 + b)[(long)(g0 + i) * 16];
+            }
+    }
+    // the first PRE groups' INT4 weights become numbers (q − 8) while the predecessor works: their expansion, and the products that take the
     // offset of in-place nibbles back, are not behind the wait
-    constexpr int FIT = 8 / (NST * NTL), PRE = HAS_ZP ? 0 : (GPW < FIT ? GPW : FIT);       // (128 registers)
-    half8 wx[PRE ? PRE : 1][NST][NTL][4];
-    if constexpr (PRE > 0) {
+    if constexpr (!F16W) {
         const uint32_t magic = opaque_vgpr(0x64006400u), magic_hi = opaque_vgpr(0x54005400u);
         const uint32_t m_lo = opaque_sgpr(0x000F000Fu), m_hi = opaque_sgpr(0x00F000F0u);
 #pragma unroll
@@ -359,8 +374,14 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
         for (int s = 0; s < 4; s++) af[0][s] = *reinterpret_cast<const half8*>(mine + i * 4096 + b * 256 + ((4 * s + a) ^ b) * 16);
 #pragma unroll
         for (int s = 0; s < NST; s++) {
-            const unsigned long long sb = ((unsigned long long)scv[i][s].y << 32) | scv[i][s].x;
-            const unsigned long long zb = HAS_ZP ? (((unsigned long long)zpv[i][s].y << 32) | zpv[i][s].x) : 0ull;
+            if constexpr (F16W) {
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+#pragma unroll
+                    for (int nt = 0; nt < NTL; nt++) acc[s][0][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[0][k], wx[i][s][nt][k], acc[s][0][nt], 0, 0, 0);
+                continue;
+            }
+            const unsigned long long sb = ((unsigned long long)scv[F16W ? 0 : i][s].y << 32) | scv[F16W ? 0 : i][s].x;
             if (i < PRE) {
                 float4v t[NTL];
 #pragma unroll
@@ -376,7 +397,7 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
                     for (int r = 0; r < 4; r++) acc[s][0][nt][r] = __builtin_fmaf(s_f, t[nt][r], acc[s][0][nt][r]);
                 }
             } else
-                w4_consume_group<1, NTL, HAS_ZP, false>(wq[i][s], sb, zb, nt0, af, acc[s]);
+                w4_consume_group<1, NTL, false, false>(wq[F16W ? 0 : i][s], sb, 0ull, nt0, af, acc[s]);
         }
     }
     // cross-wave reduction through LDS: red[wave][v][lane], v = (supertile·4 + tile)·4 + r
@@ -985,7 +1006,7 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
 // KVS / WIDE are kernels of their own, not branches: the one-range, 64-column kernel keeps the instruction layout it was tuned
 // with (with either compiled in as a runtime branch it lost ≈ 1 % at every batch size — roles entering late have their first
 // instructions on the critical path)
-template <int GPW_QKV, int GPW_O, bool HAS_ZP, bool KVS = false, bool WIDE = false>
+template <int GPW_QKV, int GPW_O, bool F16W, bool KVS = false, bool WIDE = false>
 __global__ __launch_bounds__(512, 2) void decode_chain_kernel(ChainArgs p) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[CH_SMEM > CH_W * GPW_QKV * 4096 ? CH_SMEM : CH_W * GPW_QKV * 4096];
     const int RH = (p.T + 15) >> 4;                                   // 16-row blocks
@@ -1002,11 +1023,11 @@ __global__ __launch_bounds__(512, 2) void decode_chain_kernel(ChainArgs p) {
         if constexpr (WIDE) {
             // one head (128 columns) per workgroup: half as many workgroups of twice the bytes — taken where the narrow blocks and the
             // attention role together exceed the workgroups the chip holds at once (decode_chain_f16)
-            chain_role_gemm<2, GPW_QKV, HAS_ZP>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, p.has_a != 0, smem, p);
+            chain_role_gemm<2, GPW_QKV, F16W>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, p.has_a != 0, smem, p);
         } else if (p.qkv_half)
-            chain_role_gemm<1, GPW_QKV, HAS_ZP, 2>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, p.has_a != 0, smem, p);
+            chain_role_gemm<1, GPW_QKV, F16W, 2>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, p.has_a != 0, smem, p);
         else
-            chain_role_gemm<CH_QKV_NST, GPW_QKV, HAS_ZP>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, p.has_a != 0, smem, p);
+            chain_role_gemm<CH_QKV_NST, GPW_QKV, F16W>(p.qkv, cb, wg % RH, p.norm1, p.qkv_out, p.T, p.has_a != 0, smem, p);
         // (behind its own result; read by the launch after this one)
         const __amdgpu_buffer_rsrc_t r_n = chain_rsrc(p.rows_next, (long)p.rows_next_pieces * 16);
         for (int i = wg * 512 + threadIdx.x; i < p.rows_next_pieces; i += n_qkv * 512)
@@ -1022,9 +1043,9 @@ __global__ __launch_bounds__(512, 2) void decode_chain_kernel(ChainArgs p) {
         const int ks = wg % CH_O_KS, blk = wg / CH_O_KS;
         float* part = p.o_part + (long)ks * p.T * p.o.N;
         if (p.o_half)
-            chain_role_gemm<1, GPW_O / CH_O_KS, HAS_ZP, 2, true>(p.o, blk / RH, blk % RH, p.attn_out, nullptr, p.T, true, smem, p, ks * (p.o.G / CH_O_KS), part);
+            chain_role_gemm<1, GPW_O / CH_O_KS, F16W, 2, true>(p.o, blk / RH, blk % RH, p.attn_out, nullptr, p.T, true, smem, p, ks * (p.o.G / CH_O_KS), part);
         else
-            chain_role_gemm<CH_O_NST, GPW_O / CH_O_KS, HAS_ZP, 4, true>(p.o, blk / RH, blk % RH, p.attn_out, nullptr, p.T, true, smem, p, ks * (p.o.G / CH_O_KS), part);
+            chain_role_gemm<CH_O_NST, GPW_O / CH_O_KS, F16W, 4, true>(p.o, blk / RH, blk % RH, p.attn_out, nullptr, p.T, true, smem, p, ks * (p.o.G / CH_O_KS), part);
         return;
     }
     wg -= n_o;
@@ -1042,12 +1063,16 @@ int decode_chain_counter_words() { return CH_GRAN_WORDS; }
 size_t decode_chain_row_bytes(int H, int nq, int nkv) { return (size_t)4 * H + ((size_t)nq + 2 * nkv) * 256 + (size_t)nq * 256 + (size_t)CH_O_KS * 4 * H; }
 
 bool decode_chain_supports(const DecodeChainDesc& d) {
-    const auto gemm_ok = [](const W4Device& w) {
-        return w.qw && !w.zp && !w.perm && !w.bias && !w.f16t && w.G % 8 == 0 && (w.G / 8 == 2 || w.G / 8 == 4) && w.n % 128 == 0 &&
+    if (!d.qkv || !d.o) return false;
+    const bool f16w = d.qkv->f16t != nullptr;
+    const auto gemm_ok = [&](const W4Device& w) {
+        return (f16w ? w.f16t && w.k == w.G * 128 : w.qw && !w.f16t) && !w.zp && !w.perm && !w.bias && w.G % 8 == 0 && w.n % 128 == 0 &&
                (long)CH_MAX_T * std::max(w.n, w.k) * 2 < (1L << 31);
     };
-    if (!d.qkv || !d.o || !gemm_ok(*d.qkv) || !gemm_ok(*d.o)) return false;
-    if (d.o->G / 8 != 4) return false;              // (the instantiated forms: o_proj's K slice per wave is four groups)
+    if (!gemm_ok(*d.qkv) || !gemm_ok(*d.o)) return false;
+    // the instantiated forms: a wave's K slices
+    const int gq = d.qkv->G / 8, go = d.o->G / 8;
+    if (f16w ? d.E > 0 || !((gq == 1 && go == 2) || (gq == 2 && (go == 2 || go == 4))) : !((gq == 2 || gq == 4) && go == 4)) return false;
     if (!d.rows || !d.rows_next || CH_MAX_T * decode_chain_row_bytes(d.H, d.nq, d.nkv) >= (1UL << 31)) return false;
     if (d.attn_splits > CH_MAX_SPLITS || (d.attn_splits > 1 && (!d.attn_partial || !d.attn_tickets))) return false;
     if (d.T < 1 || d.T > CH_MAX_T || d.head_dim != 128 || d.nkv < 1 || d.nq % d.nkv != 0 || d.nq / d.nkv > 14 || d.nkv > CH_MAX_KVH) return false;
@@ -1082,12 +1107,14 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
     a.attn_out = reinterpret_cast<__half*>(take((size_t)d.nq * 256));
     a.o_part = reinterpret_cast<float*>(take((size_t)CH_O_KS * 4 * d.H));
     a.rows_next = reinterpret_cast<uint32_t*>(d.rows_next); a.rows_next_pieces = (int)((rows - d.rows) / 16);
-    a.qkv = ChainGemm{d.qkv->qw, d.qkv->sc, d.qkv->zp, d.qkv->G, d.qkv->n, d.qkv->k};
+    const bool f16w = d.qkv->f16t != nullptr;
+    const auto gemm = [&](const W4Device& w) { return ChainGemm{f16w ? (const void*)w.f16t : w.qw, w.sc, w.G, w.n, w.k}; };
+    a.qkv = gemm(*d.qkv);
     a.k_pool = d.k_pool; a.v_pool = d.v_pool; a.block_tables = d.block_tables; a.kv_lens = d.kv_lens;
     a.q_norm_w = d.q_norm_w; a.k_norm_w = d.k_norm_w; a.cos_t = d.cos_t; a.sin_t = d.sin_t;
     a.qk_mode = d.qk_mode; a.max_blocks = d.max_blocks; a.sliding_window = d.sliding_window;
     a.scale = 1.0f / sqrtf((float)d.head_dim);
-    a.o = ChainGemm{d.o->qw, d.o->sc, d.o->zp, d.o->G, d.o->n, d.o->k};
+    a.o = gemm(*d.o);
     a.res_b_out = d.res_b_out; a.post_ln = d.post_ln; a.norm2 = d.norm2; a.router_w = d.router_w;
     a.E = d.E; a.r_top_k = d.r_top_k; a.Q = d.Q; a.norm_topk = d.norm_topk; a.defer_merge = d.defer_merge ? 1 : 0;
     a.cand = d.cand; a.stats = d.stats; a.route_arrive = d.route_arrive; a.ids = d.ids; a.weights = d.weights;
@@ -1101,12 +1128,13 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
     // workgroups enter behind the projection
     a.qkv_half = (knobs().chain_qkv_half && d.T <= 16 && d.qkv->n / 32 + d.T * d.nkv * a.attn_splits <= knobs().chain_slots) ? 1 : 0;
     // (narrow o_proj only: 2048 columns → 64 blocks; Llama-3.1-8B's 4096 columns are 64 blocks of 64 already: c=8 1.908 → 1.930 ms with 32)
-    a.o_half = (knobs().chain_o_half && d.T <= 16 && d.o->n <= 2048) ? 1 : 0;
+    // (and of 1024 columns up to 32 rows: a step of 32 through 14 unquantised layers 540 → 527 µs)
+    a.o_half = (knobs().chain_o_half && rh * d.o->n <= 2048) ? 1 : 0;
     // 128-column q|k|v blocks (hidden 2048 only: the two-group weight ring): where the 64-column blocks + the attention role do not fit
     // the chip's resident workgroups, the role's last workgroups enter behind the projection (≈ 2.7 µs of K/V round trips on the
     // critical path, profiles/r03_decode_chain_timeline.txt) — c=32 4.025 → 3.995 ms per step, c=64 4.83 → 4.69; c=20–24 (where they fit) 3 % slower
     a.qkv_wide = 0;
-    if (!a.qkv_half && d.qkv->G / 8 == 2 && a.attn_splits == 1) {
+    if (!f16w && !a.qkv_half && d.qkv->G / 8 == 2 && a.attn_splits == 1) {
         const int wide = knobs().chain_qkv_wide;
         const int n64 = d.qkv->n / 64 * rh, n_at = d.T * d.nkv * a.attn_splits;
         a.qkv_wide = wide >= 0 ? (wide > 0) : (n64 + n_at > knobs().chain_slots);
@@ -1115,7 +1143,21 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
     form_hit(FORM_DECODE_CHAIN);
     if (a.attn_splits > 1) form_hit(FORM_CHAIN_ATTN_KV_SPLITS);
     if (a.qkv_wide) form_hit(FORM_CHAIN_QKV_WIDE);
-    if (a.attn_splits > 1) {
+    // Unquantised layers (dense ones of 1024 – 2048 columns, up to 64 rows; a wave's weights of 4096 columns do not fit its registers, and such
+    // layers are streaming, not waiting).  A step of 14 layers of 1024 columns, the launches of their own | this one, µs: 1 row of 60 keys
+    // 470 | 380, 8 rows 505 | 424, 16 542 | 450, 17 538 | 491, 32 583 | 527, 33 655 | 572, 48 696 | 643, 64 735 | 723; 1 of 1500 keys 592 | 419, 8 of 900
+    // 622 | 538, 32 of 500 732 | 643, 64 of 300 857 | 826.
+    if (f16w) {
+        const int gq = d.qkv->G / 8, go = d.o->G / 8;
+        const bool kvs = a.attn_splits > 1;
+#define FH_CHAIN_F16(GQ, GO)                                                                                                                    \
+        do {                                                                                                                                    \
+            if (kvs) hipLaunchKernelGGL((decode_chain_kernel<GQ, GO, true, true>), dim3(blocks), dim3(512), 0, stream, a);                      \
+            else hipLaunchKernelGGL((decode_chain_kernel<GQ, GO, true>), dim3(blocks), dim3(512), 0, stream, a);                                \
+        } while (0)
+        if (gq == 1) FH_CHAIN_F16(1, 2); else if (go == 2) FH_CHAIN_F16(2, 2); else FH_CHAIN_F16(2, 4);
+#undef FH_CHAIN_F16
+    } else if (a.attn_splits > 1) {
         if (d.qkv->G / 8 == 2) hipLaunchKernelGGL((decode_chain_kernel<2, 4, false, true>), dim3(blocks), dim3(512), 0, stream, a);
         else hipLaunchKernelGGL((decode_chain_kernel<4, 4, false, true>), dim3(blocks), dim3(512), 0, stream, a);
     } else if (a.qkv_wide) hipLaunchKernelGGL((decode_chain_kernel<2, 4, false, false, true>), dim3(blocks), dim3(512), 0, stream, a);

@@ -1479,7 +1479,8 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
         const LayerWeights& L = m->layers[li];
         if (c.num_experts > 0 || !knobs().decode_chain || !knobs().dense_chain || m->em2_failed || !m->em2_arrive || !m->inlaunch_timeouts || !m->residual2) return false;
         if (!sh.all_single_token || !m->fuse_rope_attn || T > std::min(64, knobs().chain_max_rows) || m->taps_enabled || sandwich || c.tp_world > 1) return false;      // (beyond 64 rows the 64-row GEMM tiles win: Llama-3.1-8B c=96 5.56 vs 5.61 ms)
-        if (!L.o.qw || !L.gate_up.qw || !L.down.qw || L.gate_up.perm || L.down.perm || L.qkv.perm || L.o.perm) return false;
+        if (L.gate_up.perm || L.down.perm || L.qkv.perm || L.o.perm) return false;
+        if (L.o.f16t ? !L.down.f16t || !f16t_gemm_gated_supports(L.gate_up, c.intermediate) : !L.o.qw || !L.gate_up.qw || !L.down.qw) return false;
         if (L.qkv.bias || L.o.bias || !chain_kv_ok(li)) return false;
         DecodeChainDesc d = chain_desc(li);
         d.has_a = false;
@@ -1507,13 +1508,15 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             const int I = c.intermediate;
             int S = 0, rows_pad = 0, n_pad = 0;
             // ≤ 32 rows: split-K slabs summed by their consumers, gate_up of ≤ 16 with its activation in the launch
-            const bool slabs = m->dense_slabs && T <= 32 && (T > 16 || w4_gemm_rows_splits(L.down, T, m->workspace_bytes));
+            const bool slabs = L.down.qw && m->dense_slabs && T <= 32 && (T > 16 || w4_gemm_rows_splits(L.down, T, m->workspace_bytes));
             if (T > 16 && slabs) {
                 RUN(w4_gemm_dense_slabs_lds(L.gate_up, m->norm_out, m->workspace, m->workspace_bytes, T, &S, &rows_pad, &n_pad, s));
                 RUN(fused_gated_act_slabs_f16(m->workspace, S, (long)rows_pad * n_pad, n_pad, m->act_out, T, I, c.activation == 1, s));
                 S = 0;
             } else if (w4_gemm_gated_supports(L.gate_up, T, I)) {
                 RUN(w4_gemm_gated(L.gate_up, m->norm_out, m->act_out, T, I, c.activation == 1, s));
+            } else if (L.gate_up.f16t) {
+                RUN(f16t_gemm_gated(L.gate_up, m->norm_out, m->act_out, T, I, c.activation == 1, s));
             } else {
                 RUN(dense_linear(m, L.gate_up, m->norm_out, m->gate_up_out, T, s, true));
                 if (c.activation == 1) { RUN(fused_gelu_tanh_mul_split_f16(m->gate_up_out, m->act_out, T, I, s)); }

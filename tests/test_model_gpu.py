@@ -1041,6 +1041,62 @@ def test_decode_chain_of_wide_layers(pkg, c, forms):
     par.finish(max_mismatches=1, max_route_ties=0)
 
 
+@pytest.mark.parametrize("hidden,nq,nkv", [(1024, 16, 8), (2048, 16, 8), (2048, 32, 4)])
+@pytest.mark.parametrize("c,splits", [(1, 1), (9, 1), (16, 5), (17, 1), (33, 1), (64, 1)])
+def test_decode_chain_of_unquantised_layers(pkg, hidden, nq, nkv, c, splits, forms, knobs):
+    """fp16 projections in the launch: one or two 128-column slices of K a wave in q|k|v, two or four in o_proj's two parts, blocks of 32 and of 64
+    columns, one and several KV ranges; rows against the oracle, layers of several (the first role adds the MLP's fp16 rows), then the hipGraph loop."""
+    from tests import modelgen
+    from oracle import oracle as O
+    key = ("f16", hidden, nq)
+    if key not in _CHAIN_TM:
+        _CHAIN_TM[key] = modelgen.TinyModel(False, layers=2, hidden=hidden, nq=nq, nkv=nkv, hd=128, inter=1024, vocab=2048, seed=67, max_seq_len=64,
+                                            dense_proj=True, tied=True)
+    tm = _CHAIN_TM[key]
+    plen, steps, followed = 5, 2, sorted({0, c - 1})
+    O.set_threads(ORACLE_THREADS)
+    om = tm.oracle_model()
+    rng = np.random.default_rng(71)
+    prompts = [rng.integers(0, 2048, size=plen).astype(np.uint32) for _ in range(c)]
+    par = modelgen.Parity(f"f16-chain-{hidden}-{nq}-c{c}", cos_min=0.999, rel_max=2e-2)
+    knobs.set(CHAIN_ATTN_SPLITS=splits if splits > 1 else None)
+
+    def start():
+        hm = tm.hip_model(pkg, kv_num_blocks=c * 2 + 4, max_seqs=c, max_tokens=max(c * plen, 64))
+        toks, lg = hm.unified_forward([(i, p, 0, True) for i, p in enumerate(prompts)], greedy=True, want_logits=True)
+        return hm, np.array(toks, np.uint32), lg
+
+    hm, cur, lg = start()
+    for oc, i in enumerate(followed):
+        cur[i] = par.check(f"prefill/{i}", om.forward(oc, prompts[i], 0), lg[i], cur[i])
+    first = cur.copy()
+    forms.reset()
+    for s in range(steps):
+        fed = cur.copy()
+        toks, lg = hm.unified_forward([(i, [int(fed[i])], plen + s, True) for i in range(c)], greedy=True, want_logits=True)
+        cur = np.array(toks, np.uint32)
+        for oc, i in enumerate(followed):
+            cur[i] = par.check(f"step{s}/{i}", om.forward(oc, np.array([fed[i]], np.uint32), plen + s), lg[i], toks[i])
+    h = forms.hits()
+    assert h.get("decode_chain", 0) == 2 * steps and h.get("dense_chain", 0) == 2 * steps, h
+    assert h.get("chain_attn_kv_splits", 0) == (2 * steps if splits > 1 else 0), h
+    O.set_threads(1)
+    par.finish(max_mismatches=0, max_route_ties=0)
+    del hm
+    ids = []
+    for graph in (1, 0):
+        hm, _, _ = start()
+        if graph: ids.append(hm.decode_steps(list(range(c)), first, 4))
+        else:
+            fed, out = first, []
+            for s in range(4):
+                fed = np.array(hm.unified_forward([(i, [int(fed[i])], plen + s, True) for i in range(c)], greedy=True)[0], np.uint32)
+                out.append(fed)
+            ids.append(np.array(out))
+        del hm
+    assert np.array_equal(np.array(ids[0]), ids[1])
+
+
 # ── the same launch for the attention half of a DENSE layer (Llama-style: no q/k norm, no router) ─────────────────────────────
 # Three layers, so that the tail of a layer — the MLP's down projection as split-K slabs + residual + next input norm — runs as the
 # first role of the next layer's launch: oracle-followed rows, the five-launch layer on the same tokens, graph ≡ eager.
