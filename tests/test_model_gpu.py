@@ -991,6 +991,30 @@ def test_decode_chain_hands_off_every_number(pkg, c, bits, forms, knobs):
     assert np.isnan(out[0]).all() and np.isnan(out[1]).all()
 
 
+@pytest.mark.parametrize("window", [0, 300])
+def test_decode_chain_attention_of_several_rounds(pkg, window, forms, knobs):
+    """One KV range of 1 to 35 pairs of blocks over the eight waves: none, one, two (both under way before the rows are there), three and more to a wave,
+    the new token first, last and in the middle of its block and in either block of a pair; against the launches of their own."""
+    from tests import modelgen
+    kw = dict(BENCH_DIMS["qwen3-30b-a3b"])
+    tm = modelgen.TinyModel(kw.pop("moe"), layers=2, vocab=2048, seed=83, max_seq_len=1136, sliding_window=window, **kw)
+    lens = [1, 15, 16, 23, 31, 254, 255, 256, 257, 300, 510, 511, 512, 513, 767, 768, 784, 1100]
+    rng = np.random.default_rng(89)
+    prompts = [rng.integers(0, 2048, size=n).astype(np.uint32) for n in lens]
+    out = {}
+    for chain in (1, 0):
+        knobs.set(DECODE_CHAIN=chain, MOE_EM2=chain, CHAIN_SPLIT_KEYS=0, CHAIN_MAX_KEYS=1 << 20)
+        hm = tm.hip_model(pkg, kv_num_blocks=sum(n // 16 + 2 for n in lens), max_seqs=len(lens), max_tokens=1136)
+        for i, p in enumerate(prompts):
+            hm.unified_forward([(i, p, 0, True)], greedy=True)
+        forms.reset()
+        out[chain] = [hm.unified_forward([(i, [50 + i + s], n + s, True) for i, n in enumerate(lens)], greedy=True, want_logits=True)[1] for s in range(2)]
+        assert forms.hits().get("decode_chain", 0) == (4 if chain else 0), forms.hits()
+        del hm
+    for mine, other in zip(out[1], out[0]):
+        assert np.abs(mine - other).max() < 0.02 * np.abs(other).max()
+
+
 def test_decode_chain_of_batches_that_change(pkg, knobs):
     """The handed-off rows of a step lie by its batch: sequences join and leave between steps, and every step is what launches of their own make of it."""
     tm = _chain_model()
