@@ -24,6 +24,13 @@
 // result that the runner reports, never a hang.  The rows are double-buffered: the q|k|v workgroups, behind their own result, make the OTHER
 // half all ones for the next launch, which nobody reads any more (no fill node per layer; the forward's head kernel does it for its first launch).
 //
+// Dense layers of few rows go on behind role B (decode_chain_mlp_supports): gate_up and its activation (G), then down in K parts (D), as roles in
+// the same order and by the same rows.  gate_up's weights (59 MB of a layer of 4096 × 14336) are on their way from when q|k|v's workgroups leave,
+// which two launches began with; one G workgroup a CU holds 128 columns of them, all but the last group, so that there is one round of them
+// (64 columns and two rounds: the second's loads exposed, 39 µs a launch of one row, now 32 against 16 + 15.7 + 9 and two gaps before).  One row: B done
+// after 15 µs, G's rows seen 16.5 – 18.5, done 22 – 25, D's act seen 24 – 29, done 31.  (G workgroups that load D's weights through the XCD's cache under
+// their products: those took 2 µs longer, and D began no earlier.)
+//
 // Arithmetic: each role is the arithmetic of the stand-alone kernel it replaces, operation for operation —
 // moe_combine_add_rmsnorm_kernel, w4_gemm_wgsplit_kernel<MT, 2> (K split over the 8 waves, LDS reduction in wave order),
 // paged_attn_kernel<128, true, 8> (fused QK-norm / RoPE / KV write, 8 KV-splitting waves merged in wave order),
@@ -35,6 +42,7 @@
 #include "rope_rows.h"
 #include "w4_device.h"
 #include "route_merge.h"
+#include "tiled_gemm.h"
 
 namespace fh {
 
@@ -52,6 +60,7 @@ constexpr int CH_SMEM = 8 * 16 * (128 + 4) * 4 + 2 * 8 * 16 * 4 + 16 * 128 * 2 +
 
 constexpr int CH_QKV_NST = 1, CH_O_NST = 1;     // 64-column supertiles per workgroup: one head (128 columns) for q|k|v, 64 columns for o_proj; 16 rows each
 
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct ChainGemm {
@@ -96,6 +105,11 @@ struct ChainArgs {
     int attn_splits;              // KV ranges per (sequence, kv head): > 1 → partial states meet by ticket, the last arriver merges them
     float* attn_partial;          // [T·nkv][splits][16 rows][HD + 4] fp32 (m, l in the pad)
     unsigned* attn_tickets;       // [T·nkv] self-resetting
+    // the MLP (dense models): norm2 and act are handed-off rows then, and down's K parts fp32 slabs for the next launch
+    ChainGemm gu, dn;             // [2·inter, H] gate columns first, [H, inter]
+    __half* act;                  // [T, inter]
+    float* slabs;                 // [parts][T][H]
+    int gelu;
 };
 #ifdef FERRUM_HIP_EXPERIMENTS
 unsigned long long* g_chain_timeline = nullptr;
@@ -261,10 +275,13 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
 // F32OUT: the workgroup covers only the quant groups from g_base on (8·GPW of them) and leaves its fp32 partial sums in `out32`
 // ([K part][T][N]) — o_proj split over two workgroups per block: the rows a workgroup reads behind its wait (T·K·2 B through one CU)
 // are what its stage takes, and role B adds the two parts
-template <int NST, int GPW, bool F16W, int NTL = 4, bool F32OUT = false>
+// GLU: the gated MLP's first projection; half of a workgroup's columns are gate's and half the same of up's, and act(gate)·up leaves it: a
+// supertile of each (NST = 2, INT4: 4 groups of 128 columns, 128 registers, none expanded before the wait), or two tiles of each (NST = 1, fp16)
+template <int NST, int GPW, bool F16W, int NTL = 4, bool F32OUT = false, bool GLU = false>
 __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int rb, const __half* x_in, __half* out, int T,
                                                 bool handed_off, unsigned char* smem, const ChainArgs& p, int g_base = 0, float* out32 = nullptr) {
     static_assert(NTL == 4 || (NTL == 2 && NST == 1), "half supertiles only for single-supertile blocks");
+    static_assert(!GLU || (NTL == 4 && NST == (F16W ? 1 : 2) && !F32OUT), "tiles of both halves");
     constexpr int V = NST * NTL * 4, CPR = NST * NTL * 2;                       // accumulator floats per lane; 16-byte chunks per output row
     float* red = reinterpret_cast<float*>(smem);                     // [8 regions of a wave][V][64]
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -272,11 +289,12 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
     CH_TL(0);
     const int g0 = g_base + wave * GPW;                               // G = 8·GPW (· 2 with F32OUT; checked by the launcher)
     const int nt0 = NTL == 2 ? (cb & 1) * 2 : 0;                      // first tile of the block inside its supertile
-    constexpr int FIT = 8 / (NST * NTL), PRE = F16W || GPW < FIT ? GPW : FIT;       // (128 registers)
-    static_assert(!F16W || GPW <= FIT, "16-bit weights: all of a wave's in registers");
+    const int up = w.N / 32 - 2;                                      // GLU, fp16: tiles 2 and 3 of the block are this many on (N / 2 is whole supertiles)
+    constexpr int FIT = 8 / (NST * NTL), PRE = GLU && !F16W ? 0 : F16W || GPW < FIT ? GPW : FIT;       // (128 registers)
+    static_assert(!F16W || GPW <= 8 / (NST * NTL), "16-bit weights: all of a wave's in registers");
     u32x4 wq[F16W ? 1 : GPW][NST][NTL];
     uint2 scv[F16W ? 1 : GPW][NST];
-    half8 wx[PRE][NST][NTL][4];
+    half8 wx[PRE ? PRE : 1][NST][NTL][4];
     if constexpr (F16W) {
         const half8* w_lane = reinterpret_cast<const half8*>(w.qw) + lane;          // f16t: [N / 16][K / 32][64 lanes]
 #pragma unroll
@@ -287,22 +305,30 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
                 for (int nt = 0; nt < NTL; nt++)
 #pragma unroll
                     for (int k = 0; k < 4; k++)
-                        wx[i][s][nt][k] = __builtin_nontemporal_load(w_lane + (((long)(cb * NST + s) * NTL + nt) * (w.K / 32) + (g0 + i) * 4 + k) * 64);
-    } else {
-#pragma unroll
-        for (int i = 0; i < GPW; i++)
-#pragma unroll
-            for (int s = 0; s < NST; s++) {
-                const long st = NTL == 2 ? (long)(cb >> 1) : (long)cb * NST + s;
-                const u32x4* qw_lane = reinterpret_cast<const u32x4*>(w.qw) + (st * w.G * 4) * 64 + lane;
-#pragma unroll
-                for (int nt = 0; nt < NTL; nt++) wq[i][s][nt] = __builtin_nontemporal_load(qw_lane + ((long)(g0 + i) * 4 + nt0 + nt) * 64);
-                scv[i][s] = (reinterpret_cast<const uint2*>(w.sc) + (st * w.G) * 16 + b)[(long)(g0 + i) * 16];
-            }
+                        wx[i][s][nt][k] = __builtin_nontemporal_load(w_lane + ((GLU ? (long)cb * 2 + nt + (nt & 2 ? up : 0) : (long)(cb * NST + s) * NTL + nt) * (w.K / 32) +
+                                                                              (g0 + i) * 4 + k) * 64);
     }
+    // (GLU, four groups: the last is asked for behind the rows.  Its workgroups fill the chip when the ones before them leave, memory is still busy
+    // with their weights when the rows are there, and loads come back in order: the products of three start a quarter of them earlier)
+    constexpr int LATE = GLU && !F16W ? GPW / 4 : 0;
+    auto ask = [&](auto from, auto to) {
+        if constexpr (!F16W) {
+#pragma unroll
+            for (int i = decltype(from)::value; i < decltype(to)::value; i++)
+#pragma unroll
+                for (int s = 0; s < NST; s++) {
+                    const long st = GLU ? (long)cb + s * (w.N / 128) : NTL == 2 ? (long)(cb >> 1) : (long)cb * NST + s;
+                    const u32x4* qw_lane = reinterpret_cast<const u32x4*>(w.qw) + (st * w.G * 4) * 64 + lane;
+#pragma unroll
+                    for (int nt = 0; nt < NTL; nt++) wq[i][s][nt] = __builtin_nontemporal_load(qw_lane + ((long)(g0 + i) * 4 + nt0 + nt) * 64);
+                    scv[i][s] = (reinterpret_cast<const uint2*>(w.sc) + (st * w.G) * 16 + b)[(long)(g0 + i) * 16];
+                }
+        }
+    };
+    ask(std::integral_constant<int, 0>{}, std::integral_constant<int, GPW - LATE>{});
     // the first PRE groups' INT4 weights become numbers (q − 8) while the predecessor works: their expansion, and the products that take the
     // offset of in-place nibbles back, are not behind the wait
-    if constexpr (!F16W) {
+    if constexpr (!F16W && PRE > 0) {
         const uint32_t magic = opaque_vgpr(0x64006400u), magic_hi = opaque_vgpr(0x54005400u);
         const uint32_t m_lo = opaque_sgpr(0x000F000Fu), m_hi = opaque_sgpr(0x00F000F0u);
 #pragma unroll
@@ -358,6 +384,10 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
         request();
     }
     CH_TL(1);
+    if constexpr (LATE > 0) {
+        ask(std::integral_constant<int, GPW - LATE>{}, std::integral_constant<int, GPW>{});
+        __builtin_amdgcn_sched_barrier(0);
+    }
     float4v acc[NST][1][NTL];
 #pragma unroll
     for (int s = 0; s < NST; s++)
@@ -365,7 +395,8 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
         for (int nt = 0; nt < NTL; nt++) acc[s][0][nt] = (float4v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < GPW; i++) {
-        if (i == GPW - 1) chain_landed<0>();                          // (handed-off rows are there)
+        if constexpr (GLU) {                                          // (handed-off rows are there)
+        } else if (i == GPW - 1) chain_landed<0>();
         else if (i == GPW - 2) chain_landed<4>();
         else if (i == GPW - 3) chain_landed<8>();
         else chain_landed<12>();
@@ -408,6 +439,36 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
 #pragma unroll
             for (int r = 0; r < 4; r++) red[wave * (REGION / 4) + ((s * NTL + nt) * 4 + r) * 64 + lane] = acc[s][0][nt][r];
     __syncthreads();
+    if constexpr (GLU) {
+        // thread → (row, 4 columns of gate and of up): one 8-byte write-through store
+        constexpr int COLS = NST * NTL * 8;
+        if (threadIdx.x < 16 * (COLS / 4)) {
+            const int row = threadIdx.x / (COLS / 4), c4 = (threadIdx.x % (COLS / 4)) * 4;
+            const int v = (c4 >> 4) * 4 + (row & 3), ln = (row >> 2) * 16 + (c4 & 15);
+            float4v sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int ww = 0; ww < CH_W; ww++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) sum[h] += *reinterpret_cast<const float4v*>(&red[ww * (REGION / 4) + (v + V / 2 * h) * 64 + ln]);
+            union { _Float16 h[4]; uint32_t u[2]; } o;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                float g = sum[0][j], u = sum[1][j];
+                if constexpr (F16W) {                                 // as gemm_glu
+                    o.h[j] = (_Float16)((p.gelu ? gelu_tanh_f32<_Float16>(g) : g * ActMath<_Float16>::sigmoid(g)) * u);
+                } else {
+                    g = (float)(_Float16)g;
+                    u = (float)(_Float16)u;
+                    o.h[j] = p.gelu ? gated_act<true>(g, u) : gated_act<false>(g, u);
+                }
+            }
+            const int r_out = rb * 16 + row, n = w.N / 2;
+            if (r_out < T)
+                __builtin_amdgcn_raw_buffer_store_b64((u32x2){written2(o.u[0]), written2(o.u[1])}, chain_rsrc(out, (long)T * n * 2), (r_out * n + cb * COLS + c4) * 2, 0, 16);
+        }
+        CH_TL(2); CH_TL(3);
+        return;
+    }
     // thread → (row, 8 consecutive columns): one 16-byte write-through store
     if (threadIdx.x < 16 * CPR) {
         const int row = threadIdx.x / CPR, c8 = (threadIdx.x % CPR) * 8;
@@ -741,6 +802,7 @@ __device__ __forceinline__ void chain_role_attn(const ChainArgs& p, int wg, unsi
 
 // ── role B: residual += o; post-attention norm; router logits of this part's experts; candidates; in-launch merge ─────────
 // (add_rmsnorm_route_part_kernel<false> with arrive: grid (token, part) → wg = token·Q + part)
+template <bool MLP>
 __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigned char* smem) {
     const int H = p.H, Q = p.Q, num_experts = p.E, top_k = p.r_top_k;
     const long row = wg / Q;
@@ -847,14 +909,17 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
             half8 o;
 #pragma unroll
             for (int j = 0; j < 8; j++) o[j] = (_Float16)((float)v[c][j] * inv * (float)wv[j]);
+            if constexpr (MLP) store16_sc1(chain_rsrc(p.norm2, (long)p.T * H * 2), (int)((row * H + i * 8) * 2), o);
             *reinterpret_cast<half8*>(xs + i * 8) = o;
-            if (q == 0) {
+            if (MLP) {
+                *reinterpret_cast<half8*>(p.res_b_out + row * H + i * 8) = v[c];
+            } else if (q == 0) {
                 *reinterpret_cast<half8*>(p.norm2 + row * H + i * 8) = o;
                 *reinterpret_cast<half8*>(p.res_b_out + row * H + i * 8) = v[c];
             }
         }
     }
-    if (num_experts <= 0) { CH_TL(2); CH_TL(3); return; }           // dense model: add + norm only (norm2 / res_b_out written above)
+    if (MLP || num_experts <= 0) { CH_TL(2); CH_TL(3); return; }           // dense model: add + norm only (norm2 / res_b_out written above)
     __syncthreads();
     const int a = lane >> 4, b = lane & 15;
     // (all sixteen rows of a product are the token's: a row of zeros would need a branch at every read)
@@ -1016,9 +1081,11 @@ __device__ __forceinline__ void chain_role_b(const ChainArgs& p, int wg, unsigne
 // KVS / WIDE are kernels of their own, not branches: the one-range, 64-column kernel keeps the instruction layout it was tuned
 // with (with either compiled in as a runtime branch it lost ≈ 1 % at every batch size — roles entering late have their first
 // instructions on the critical path)
-template <int GPW_QKV, int GPW_O, bool F16W, bool KVS = false, bool WIDE = false>
+// GPW_D: quant groups of a wave in the MLP's second projection (dense models); 0: the launch ends with role B
+template <int GPW_QKV, int GPW_O, bool F16W, bool KVS = false, bool WIDE = false, int GPW_D = 0>
 __global__ __launch_bounds__(512, 2) void decode_chain_kernel(ChainArgs p) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[CH_SMEM > CH_W * GPW_QKV * 4096 ? CH_SMEM : CH_W * GPW_QKV * 4096];
+    static_assert(CH_W * GPW_D * 4096 <= (int)sizeof(smem) && CH_W * GPW_O / CH_O_KS * 4096 <= (int)sizeof(smem), "every role's rows");
     const int RH = (p.T + 15) >> 4;                                   // 16-row blocks
     const int QB = WIDE ? 128 : (p.qkv_half ? 32 : 64);             // q|k|v block width
     const int n_a = p.has_a ? p.T : 0, n_qkv = p.qkv.N / QB * RH, n_attn = p.T * p.nkv * (KVS ? p.attn_splits : 1), n_o = p.o.N / (p.o_half ? 32 : 64 * CH_O_NST) * RH * CH_O_KS;
@@ -1059,7 +1126,22 @@ __global__ __launch_bounds__(512, 2) void decode_chain_kernel(ChainArgs p) {
         return;
     }
     wg -= n_o;
-    chain_role_b(p, wg, smem);
+    if constexpr (GPW_D == 0) {
+        chain_role_b<false>(p, wg, smem);
+    } else {
+        if (wg < p.T) { chain_role_b<true>(p, wg, smem); return; }
+        wg -= p.T;
+        constexpr int GU = F16W ? 1 : 2;
+        const int n_gu = p.gu.N / (64 * GU) * RH;
+        if (wg < n_gu) { chain_role_gemm<GU, GPW_QKV, F16W, 4, false, true>(p.gu, wg / RH, wg % RH, p.norm2, p.act, p.T, true, smem, p); return; }
+        wg -= n_gu;
+        const int parts = p.dn.G / (8 * GPW_D), ks = wg % parts, blk = wg / parts;
+        float* slab = p.slabs + (long)ks * p.T * p.dn.N;
+        if constexpr (F16W)
+            chain_role_gemm<1, GPW_D, true, 2, true>(p.dn, blk / RH, blk % RH, p.act, nullptr, p.T, true, smem, p, ks * 8 * GPW_D, slab);
+        else
+            chain_role_gemm<2, GPW_D, false, 4, true>(p.dn, blk / RH, blk % RH, p.act, nullptr, p.T, true, smem, p, ks * 8 * GPW_D, slab);
+    }
 }
 
 }  // namespace
@@ -1069,8 +1151,27 @@ extern "C" __attribute__((visibility("default"))) void ferrum_hip_debug_set_chai
 #endif
 
 int decode_chain_counter_words() { return CH_GRAN_WORDS; }
-// handed-off rows of a token: role A's two, q|k|v's, attention's, o_proj's K parts
-size_t decode_chain_row_bytes(int H, int nq, int nkv) { return (size_t)4 * H + ((size_t)nq + 2 * nkv) * 256 + (size_t)nq * 256 + (size_t)CH_O_KS * 4 * H; }
+// handed-off rows of a token: role A's two, q|k|v's, attention's, o_proj's K parts; with an MLP in the launch (inter > 0) its input's and act's
+size_t decode_chain_row_bytes(int H, int nq, int nkv, int inter) {
+    return (size_t)4 * H + ((size_t)nq + 2 * nkv) * 256 + (size_t)nq * 256 + (size_t)CH_O_KS * 4 * H + (inter > 0 ? (size_t)2 * (H + inter) : 0);
+}
+static int chain_mlp_groups(bool f16w) { return f16w ? 1 : 2; }       // GPW_D
+bool decode_chain_mlp_supports(const W4Device& qkv, const W4Device& gu, const W4Device& dn, int inter, int rows, size_t slab_bytes) {
+    const bool f16w = qkv.f16t != nullptr;
+    for (const W4Device* w : {&gu, &dn})
+        if ((f16w ? !w->f16t || w->k != w->G * 128 : !w->qw || w->f16t) || w->zp || w->perm || w->bias || w->n % 128 != 0 ||
+            (long)CH_MAX_T * std::max(w->n, w->k) * 4 >= (1L << 31)) return false;
+    const int per = 8 * chain_mlp_groups(f16w);
+    return inter % 128 == 0 && gu.k == qkv.k && gu.n == 2 * inter && dn.k == inter && dn.n == qkv.k && dn.G % per == 0 && dn.G / per <= 8 &&
+           (size_t)(dn.G / per) * rows * dn.n * 4 <= slab_bytes;
+}
+// Rows up to which the launch takes the MLP: one block of them, and two of the smallest layers (µs of a step, the MLP's two launches behind the chain
+// | in it.  32 INT4 layers of 4096, inter 14336: 1 row 1393 | 1273, 4 rows 1430 | 1315, 12 of 120 keys 1568 | 1470, 16 1623 | 1513, 17 2096 | 2333, 1 of 8000
+// keys 1591 | 1437.  8 of 4096, 12288, GELU: 1 376 | 344, 8 393 | 368, 16 436 | 404, 17 550 | 557.  8 of 2048, 8192: 1 260 | 230, 8 287 | 246, 16 338 | 271, 17
+// 407 | 404, 32 428 | 428.  14 fp16 layers of 1024, 3072: 1 371 | 302, 8 418 | 330, 16 441 | 350, 17 488 | 439, 32 523 | 475, 64 707 | 751.  8 of 2048,
+// 6144: 1 310 | 268, 8 339 | 304, 16 368 | 321, 17 420 | 457, 32 450 | 492.)
+int decode_chain_mlp_max_rows(const W4Device& qkv) { return qkv.f16t && qkv.G == 8 ? 32 : 16; }
+int decode_chain_mlp_parts(const W4Device& dn) { return dn.G / (8 * chain_mlp_groups(dn.f16t != nullptr)); }
 
 bool decode_chain_supports(const DecodeChainDesc& d) {
     if (!d.qkv || !d.o) return false;
@@ -1083,7 +1184,9 @@ bool decode_chain_supports(const DecodeChainDesc& d) {
     // the instantiated forms: a wave's K slices
     const int gq = d.qkv->G / 8, go = d.o->G / 8;
     if (f16w ? d.E > 0 || !((gq == 1 && go == 2) || (gq == 2 && (go == 2 || go == 4))) : !((gq == 2 || gq == 4) && go == 4)) return false;
-    if (!d.rows || !d.rows_next || CH_MAX_T * decode_chain_row_bytes(d.H, d.nq, d.nkv) >= (1UL << 31)) return false;
+    if (!d.rows || !d.rows_next || CH_MAX_T * decode_chain_row_bytes(d.H, d.nq, d.nkv, d.rows_inter) >= (1UL << 31)) return false;
+    if (d.gate_up && (d.E > 0 || !d.down_proj || !d.slabs || d.rows_inter != d.down_proj->k ||
+                      !decode_chain_mlp_supports(*d.qkv, *d.gate_up, *d.down_proj, d.rows_inter, d.T, ~(size_t)0))) return false;
     if (d.attn_splits > CH_MAX_SPLITS || (d.attn_splits > 1 && (!d.attn_partial || !d.attn_tickets))) return false;
     if (d.T < 1 || d.T > CH_MAX_T || d.head_dim != 128 || d.nkv < 1 || d.nq % d.nkv != 0 || d.nq / d.nkv > 14 || d.nkv > CH_MAX_KVH) return false;
     if (d.H % 32 != 0 || d.H > 8192 || d.qkv->k != d.H || d.qkv->n != (d.nq + 2 * d.nkv) * 128 || d.o->k != d.nq * 128 || d.o->n != d.H) return false;
@@ -1116,7 +1219,12 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
     a.qkv_out = reinterpret_cast<__half*>(take(((size_t)d.nq + 2 * d.nkv) * 256));
     a.attn_out = reinterpret_cast<__half*>(take((size_t)d.nq * 256));
     a.o_part = reinterpret_cast<float*>(take((size_t)CH_O_KS * 4 * d.H));
+    if (d.rows_inter > 0) {
+        a.norm2 = reinterpret_cast<__half*>(take((size_t)2 * d.H));
+        a.act = reinterpret_cast<__half*>(take((size_t)2 * d.rows_inter));
+    }
     a.rows_next = reinterpret_cast<uint32_t*>(d.rows_next); a.rows_next_pieces = (int)((rows - d.rows) / 16);
+    const bool mlp = d.gate_up != nullptr;
     const bool f16w = d.qkv->f16t != nullptr;
     const auto gemm = [&](const W4Device& w) { return ChainGemm{f16w ? (const void*)w.f16t : w.qw, w.sc, w.G, w.n, w.k}; };
     a.qkv = gemm(*d.qkv);
@@ -1125,7 +1233,9 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
     a.qk_mode = d.qk_mode; a.max_blocks = d.max_blocks; a.sliding_window = d.sliding_window;
     a.scale = 1.0f / sqrtf((float)d.head_dim);
     a.o = gemm(*d.o);
-    a.res_b_out = d.res_b_out; a.post_ln = d.post_ln; a.norm2 = d.norm2; a.router_w = d.router_w;
+    if (mlp) { a.gu = gemm(*d.gate_up); a.dn = gemm(*d.down_proj); a.slabs = d.slabs; a.gelu = d.gelu; }
+    else a.norm2 = d.norm2;
+    a.res_b_out = d.res_b_out; a.post_ln = d.post_ln; a.router_w = d.router_w;
     a.E = d.E; a.r_top_k = d.r_top_k; a.Q = d.Q; a.norm_topk = d.norm_topk; a.defer_merge = d.defer_merge ? 1 : 0;
     a.cand = d.cand; a.stats = d.stats; a.route_arrive = d.route_arrive; a.ids = d.ids; a.weights = d.weights;
     a.cnt = d.cnt; a.cnt_next = d.cnt_next; a.timeout = d.timeout;
@@ -1144,15 +1254,17 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
     // the chip's resident workgroups, the role's last workgroups enter behind the projection (≈ 2.7 µs of K/V round trips on the
     // critical path, profiles/r03_decode_chain_timeline.txt) — c=32 4.025 → 3.995 ms per step, c=64 4.83 → 4.69; c=20–24 (where they fit) 3 % slower
     a.qkv_wide = 0;
-    if (!f16w && !a.qkv_half && d.qkv->G / 8 == 2 && a.attn_splits == 1) {
+    if (!f16w && !mlp && !a.qkv_half && d.qkv->G / 8 == 2 && a.attn_splits == 1) {
         const int wide = knobs().chain_qkv_wide;
         const int n64 = d.qkv->n / 64 * rh, n_at = d.T * d.nkv * a.attn_splits;
         a.qkv_wide = wide >= 0 ? (wide > 0) : (n64 + n_at > knobs().chain_slots);
     }
-    const int blocks = (d.has_a ? d.T : 0) + d.qkv->n / (a.qkv_half ? 32 : (a.qkv_wide ? 128 : 64)) * rh + d.T * d.nkv * a.attn_splits + d.o->n / (a.o_half ? 32 : 64 * CH_O_NST) * rh * CH_O_KS + d.T * d.Q;
+    const int blocks = (d.has_a ? d.T : 0) + d.qkv->n / (a.qkv_half ? 32 : (a.qkv_wide ? 128 : 64)) * rh + d.T * d.nkv * a.attn_splits + d.o->n / (a.o_half ? 32 : 64 * CH_O_NST) * rh * CH_O_KS + d.T * d.Q +
+                       (mlp ? d.gate_up->n / (f16w ? 64 : 128) * rh + d.H / (f16w ? 32 : 128) * rh * decode_chain_mlp_parts(*d.down_proj) : 0);
     form_hit(FORM_DECODE_CHAIN);
     if (a.attn_splits > 1) form_hit(FORM_CHAIN_ATTN_KV_SPLITS);
     if (a.qkv_wide) form_hit(FORM_CHAIN_QKV_WIDE);
+    if (mlp) form_hit(FORM_CHAIN_MLP);
     // Unquantised layers (dense ones of 1024 – 2048 columns, up to 64 rows; a wave's weights of 4096 columns do not fit its registers, and such
     // layers are streaming, not waiting).  A step of 14 layers of 1024 columns, the launches of their own | this one, µs: 1 row of 60 keys
     // 470 | 380, 8 rows 505 | 424, 16 542 | 450, 17 538 | 491, 32 583 | 527, 33 655 | 572, 48 696 | 643, 64 735 | 723; 1 of 1500 keys 592 | 419, 8 of 900
@@ -1162,11 +1274,21 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
         const bool kvs = a.attn_splits > 1;
 #define FH_CHAIN_F16(GQ, GO)                                                                                                                    \
         do {                                                                                                                                    \
-            if (kvs) hipLaunchKernelGGL((decode_chain_kernel<GQ, GO, true, true>), dim3(blocks), dim3(512), 0, stream, a);                      \
+            if (mlp && kvs) hipLaunchKernelGGL((decode_chain_kernel<GQ, GO, true, true, false, 1>), dim3(blocks), dim3(512), 0, stream, a);     \
+            else if (mlp) hipLaunchKernelGGL((decode_chain_kernel<GQ, GO, true, false, false, 1>), dim3(blocks), dim3(512), 0, stream, a);      \
+            else if (kvs) hipLaunchKernelGGL((decode_chain_kernel<GQ, GO, true, true>), dim3(blocks), dim3(512), 0, stream, a);                 \
             else hipLaunchKernelGGL((decode_chain_kernel<GQ, GO, true>), dim3(blocks), dim3(512), 0, stream, a);                                \
         } while (0)
         if (gq == 1) FH_CHAIN_F16(1, 2); else if (go == 2) FH_CHAIN_F16(2, 2); else FH_CHAIN_F16(2, 4);
 #undef FH_CHAIN_F16
+    } else if (mlp) {
+#define FH_CHAIN_MLP(GQ)                                                                                                                        \
+        do {                                                                                                                                    \
+            if (a.attn_splits > 1) hipLaunchKernelGGL((decode_chain_kernel<GQ, 4, false, true, false, 2>), dim3(blocks), dim3(512), 0, stream, a); \
+            else hipLaunchKernelGGL((decode_chain_kernel<GQ, 4, false, false, false, 2>), dim3(blocks), dim3(512), 0, stream, a);               \
+        } while (0)
+        if (d.qkv->G / 8 == 2) FH_CHAIN_MLP(2); else FH_CHAIN_MLP(4);
+#undef FH_CHAIN_MLP
     } else if (a.attn_splits > 1) {
         if (d.qkv->G / 8 == 2) hipLaunchKernelGGL((decode_chain_kernel<2, 4, false, true>), dim3(blocks), dim3(512), 0, stream, a);
         else hipLaunchKernelGGL((decode_chain_kernel<4, 4, false, true>), dim3(blocks), dim3(512), 0, stream, a);

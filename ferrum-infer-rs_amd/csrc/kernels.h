@@ -276,6 +276,9 @@ struct DecodeChainDesc {
     RouteCand* cand = nullptr; float* stats = nullptr; unsigned* route_arrive = nullptr; int32_t* ids = nullptr; float* weights = nullptr;
     // rows handed off inside the launch, decode_chain_row_bytes for each token: all ones on entry, and the launch leaves all ones in the other half
     unsigned char *rows = nullptr, *rows_next = nullptr;
+    int rows_inter = 0;            // > 0: … with the MLP's rows, in every launch of the forward whether it has the MLP or not
+    // dense models: the MLP as the last roles (null: the launch ends with norm2); down's decode_chain_mlp_parts K parts in slabs, [part][T][H]
+    const W4Device* gate_up = nullptr; const W4Device* down_proj = nullptr; float* slabs = nullptr; int gelu = 0;
     int attn_splits = 1;           // KV ranges per (sequence, kv head) in the attention role (≤ 16); > 1 needs the two buffers below
     float* attn_partial = nullptr; // [T·nkv·attn_splits][16][head_dim + 4] fp32
     unsigned* attn_tickets = nullptr;   // [T·nkv] zeroed words (self-resetting)
@@ -284,7 +287,10 @@ struct DecodeChainDesc {
     unsigned* timeout = nullptr;   // host-visible word, bumped by a bounded wait that gave up
 };
 int decode_chain_counter_words();
-size_t decode_chain_row_bytes(int H, int nq, int nkv);
+size_t decode_chain_row_bytes(int H, int nq, int nkv, int inter = 0);
+bool decode_chain_mlp_supports(const W4Device& qkv, const W4Device& gu, const W4Device& dn, int inter, int rows, size_t slab_bytes);
+int decode_chain_mlp_max_rows(const W4Device& qkv);
+int decode_chain_mlp_parts(const W4Device& dn);
 bool decode_chain_supports(const DecodeChainDesc& d);
 int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream);
 

@@ -42,6 +42,7 @@ struct Knobs {
     int chain_attn_splits = 0;        // > 0: that many KV ranges whatever the context (experiments)
     int chain_max_keys = 4096;        // decode chain only up to this many keys per attention workgroup (× T·nkv / 128)
     int dense_chain = 1;              // dense models at 17–32 rows: the attention half of the layer as the chain launch too (0 = five launches)
+    int chain_mlp_rows = 32;          // … and its MLP in that launch, up to this many rows (0 = its own two launches)
     int moe_em2 = 1;                  // decode: gate_up → down as one expert-major launch (0 = two launches)
     int moe_bm2 = 0;                  // decode at ≤ 64 pairs: gate_up → down as one block-major launch — measured slower than the two launches (profiles/r03_moe_bm2_timeline.txt): off
     int moe_deferred_merge = 1;       // decode chain: the grouped GEMM's prologue merges the router's candidate lists (0 = role B does)
@@ -167,6 +168,7 @@ enum Form : int {
     FORM_F16_GATED,             // unquantised gate_up with its activation in the launch
     FORM_TILED_GEMM_COLS64,     // few-row projection with 64 columns a wave
     FORM_TILED_GEMM_256X256,    // prompts: tiles of 256 × 256, a workgroup's one after the other (tiled_gemm_wide.hip)
+    FORM_CHAIN_MLP,             // decode chain: the MLP of a dense layer in the launch too
     FORM_COUNT
 };
 

@@ -930,7 +930,7 @@ int ferrum_hip_model_finalize(FerrumHipModel* m) {
         }
     }
     if (!rc && m->em2_arrive) {
-        m->chain_rows_half = CHAIN_MAX_ROWS * decode_chain_row_bytes((int)H, c.num_heads, c.num_kv_heads);
+        m->chain_rows_half = CHAIN_MAX_ROWS * decode_chain_row_bytes((int)H, c.num_heads, c.num_kv_heads, c.num_experts > 0 ? 0 : c.intermediate);
         rc |= dev_alloc(&m->chain_rows, 2 * m->chain_rows_half);
     }
     if (!rc && m->em2_arrive && c.head_dim == 128) {
@@ -1400,9 +1400,10 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
     // workgroup owns the row (every norm of the dense layer) or the rows are few (decode attention scatters); the gated
     // activation is permuted by gate_up's column order (pack_gate_up).  Only the prefill o_proj keeps a gather launch.
     const bool chain_rows = m->chain_rows && sh.all_single_token && T <= std::min(CHAIN_MAX_ROWS, knobs().chain_max_rows);
+    const int chain_inter = c.num_experts == 0 && T <= std::min(decode_chain_mlp_max_rows(m->layers[0].qkv), knobs().chain_mlp_rows) ? c.intermediate : 0;      // the MLP in the chain launch
     RUN(embed_rms_norm_f16(m->embed, tokens, c.embed_scale, m->residual, sandwich ? m->residual_f32 : nullptr, m->layers[0].input_ln,
                            c.rms_eps, m->norm_out, T, H, m->route_arrive, m->route_arrive ? 64 + (int)m->arrive_half_words : 0,
-                           chain_rows ? reinterpret_cast<unsigned*>(m->chain_rows) : nullptr, chain_rows ? (int)(T * decode_chain_row_bytes(H, nq, nkv) / 4) : 0, s, m->layers[0].qkv.perm));
+                           chain_rows ? reinterpret_cast<unsigned*>(m->chain_rows) : nullptr, chain_rows ? (int)(T * decode_chain_row_bytes(H, nq, nkv, chain_inter) / 4) : 0, s, m->layers[0].qkv.perm));
     m->em2_parity = 0;          // the head kernel made half 0 of the merged launches' counters and rows ready; every such launch does that to the other half
     m->chain_parity = 0;
     bool qkv_in_perm = m->layers[0].qkv.perm != nullptr;      // norm_out holds the row in L.qkv's packed order
@@ -1427,6 +1428,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
         d.sin_t = (!is_global && m->sin_local) ? m->sin_local : m->sin_t;
         d.qk_mode = qk_mode; d.max_blocks = m->max_blocks_per_seq;
         d.o = &L.o;
+        d.rows_inter = chain_inter;
         if (m->chain_rows) { d.rows = m->chain_rows + m->chain_parity * m->chain_rows_half; d.rows_next = m->chain_rows + (m->chain_parity ^ 1) * m->chain_rows_half; }
         d.res_b_out = m->residual2; d.post_ln = L.post_ln; d.norm2 = m->norm_out; d.router_w = L.router;
         d.E = c.num_experts; d.r_top_k = c.top_k; d.norm_topk = c.norm_topk_prob;
@@ -1473,7 +1475,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
     };
     // dense models at 17–32 rows: the same launch for the attention half (tail of the previous layer's MLP — its down slabs +
     // residual + norm — q|k|v, attention, o_proj, add + norm), then gate_up slabs → gated activation → down slabs
-    bool pending_dense_tail = false;
+    bool pending_dense_tail = false, tail_mlp = false;      // (tail_mlp: the slabs are the launch's own)
     int tail_S = 0, tail_rows_pad = 0, tail_n_pad = 0;
     auto dense_chain_ok = [&](int li) {
         const LayerWeights& L = m->layers[li];
@@ -1501,15 +1503,20 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             d.a_x = tail_S == 0 ? m->mlp_out : nullptr;
             d.cnt = m->em2_arrive + (size_t)m->chain_parity * m->arrive_half_words;
             d.cnt_next = m->em2_arrive + (size_t)(m->chain_parity ^ 1) * m->arrive_half_words;
+            const int I = c.intermediate;
+            // (several blocks of rows: a block's slabs are written when its rows are through the launch, so those that its tail reads must lie as these do)
+            const bool mlp = chain_inter > 0 && (T <= 16 || !pending_dense_tail || tail_mlp) && decode_chain_mlp_supports(L.qkv, L.gate_up, L.down, I, T, m->workspace_bytes);
+            if (mlp) { d.gate_up = &L.gate_up; d.down_proj = &L.down; d.slabs = m->workspace; d.gelu = c.activation == 1; }
             RUN(decode_chain_f16(d, s));
             m->chain_parity ^= 1;
             pending_dense_tail = false;
             form_hit(FORM_DENSE_CHAIN);
-            const int I = c.intermediate;
             int S = 0, rows_pad = 0, n_pad = 0;
             // ≤ 32 rows: split-K slabs summed by their consumers, gate_up of ≤ 16 with its activation in the launch
-            const bool slabs = L.down.qw && m->dense_slabs && T <= 32 && (T > 16 || w4_gemm_rows_splits(L.down, T, m->workspace_bytes));
-            if (T > 16 && slabs) {
+            const bool slabs = mlp || (L.down.qw && m->dense_slabs && T <= 32 && (T > 16 || w4_gemm_rows_splits(L.down, T, m->workspace_bytes)));
+            if (mlp) {
+                S = decode_chain_mlp_parts(L.down); rows_pad = T; n_pad = H;
+            } else if (T > 16 && slabs) {
                 RUN(w4_gemm_dense_slabs_lds(L.gate_up, m->norm_out, m->workspace, m->workspace_bytes, T, &S, &rows_pad, &n_pad, s));
                 RUN(fused_gated_act_slabs_f16(m->workspace, S, (long)rows_pad * n_pad, n_pad, m->act_out, T, I, c.activation == 1, s));
                 S = 0;
@@ -1522,11 +1529,12 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
                 if (c.activation == 1) { RUN(fused_gelu_tanh_mul_split_f16(m->gate_up_out, m->act_out, T, I, s)); }
                 else { RUN(fused_silu_mul_split_f16(m->gate_up_out, m->act_out, T, I, s)); }
             }
-            if (slabs) { RUN(dense_slabs_gemm(m, L.down, m->act_out, T, &S, &rows_pad, &n_pad, s)); }
+            if (mlp) {
+            } else if (slabs) { RUN(dense_slabs_gemm(m, L.down, m->act_out, T, &S, &rows_pad, &n_pad, s)); }
             else { RUN(dense_linear(m, L.down, m->act_out, m->mlp_out, T, s)); }
             if (li + 1 < c.num_layers && dense_chain_ok(li + 1)) {
                 pending_dense_tail = true;          // MLP output + residual + next input norm: the first role of the next layer's launch
-                tail_S = S; tail_rows_pad = rows_pad; tail_n_pad = n_pad;
+                tail_S = S; tail_rows_pad = rows_pad; tail_n_pad = n_pad; tail_mlp = mlp;
             } else if (!slabs) {
                 if (next_ln) { RUN(fused_add_rms_norm_f16(m->residual2, m->mlp_out, next_ln, c.rms_eps, m->norm_out, T, H, s, next_qkv_perm)); }
                 else { RUN(add_inplace_f16(m->residual2, m->mlp_out, (long)T * H, s)); }

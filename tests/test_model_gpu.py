@@ -1121,6 +1121,45 @@ def test_decode_chain_of_unquantised_layers(pkg, hidden, nq, nkv, c, splits, for
     assert np.array_equal(np.array(ids[0]), ids[1])
 
 
+@pytest.mark.parametrize("f16,hidden,inter,activation,c", [
+    (0, 4096, 2048, 0, 1), (0, 4096, 2048, 1, 16), (0, 2048, 8192, 0, 5), (0, 2048, 4096, 1, 4), (0, 2048, 4096, 0, 17),
+    (1, 1024, 1024, 0, 1), (1, 1024, 3072, 1, 16), (1, 1024, 3072, 0, 17), (1, 1024, 1024, 0, 32), (1, 1024, 1024, 0, 33), (1, 2048, 3072, 1, 9),
+    (0, 2048, 1152, 0, 3), (1, 1024, 1152, 0, 3)])
+def test_decode_chain_with_the_mlp(pkg, f16, hidden, inter, activation, c, forms, knobs):
+    """gate_up, its activation and down's K parts (1 to 4) as the launch's last roles, one block of rows and two, against the launches of their own; where
+    the rows or the groups of down do not fit it, they run.  Then a norm of all-ones NaN ahead of gate_up: the rows arrive all the same."""
+    from tests import modelgen
+    key = ("mlp", f16, hidden, inter, activation)
+    if key not in _CHAIN_TM:
+        kw = dict(dense_proj=True, tied=True) if f16 else {}
+        _CHAIN_TM[key] = modelgen.TinyModel(False, layers=2, hidden=hidden, nq=32 if not f16 else 16, nkv=8, hd=128, inter=inter, vocab=1024, seed=97,
+                                            max_seq_len=64, qk_norm=False, activation=activation, **kw)
+    tm = _CHAIN_TM[key]
+    taken = inter != 1152 and c <= (32 if f16 and hidden == 1024 else 16)
+    kept = tm.layers[1]["dense"]["post_ln"]
+    try:
+        for bits in (None, 0xffff):
+            if bits:
+                tm.layers[1]["dense"]["post_ln"] = np.full_like(kept, np.array([bits], np.uint16).view(np.float16).astype(np.float32)[0])
+            out = {}
+            for rows in (32, 0):
+                knobs.set(CHAIN_MLP_ROWS=rows)
+                hm = tm.hip_model(pkg, kv_num_blocks=c * 2 + 4, max_seqs=c, max_tokens=max(3 * c, 64))
+                hm.unified_forward([(i, [7 + i, 300, 21], 0, True) for i in range(c)], greedy=True)
+                forms.reset()
+                out[rows] = [hm.unified_forward([(i, [50 + i + s], 3 + s, True) for i in range(c)], greedy=True, want_logits=True)[1] for s in range(2)]
+                assert forms.hits().get("chain_mlp", 0) == (4 if rows and taken else 0), forms.hits()
+                assert forms.hits().get("dense_chain", 0) == 4, forms.hits()
+                del hm
+            for mine, other in zip(out[32], out[0]):
+                if bits:
+                    assert np.isnan(mine).all() and np.isnan(other).all()
+                else:
+                    assert np.abs(mine - other).max() < 0.02 * np.abs(other).max()
+    finally:
+        tm.layers[1]["dense"]["post_ln"] = kept
+
+
 # ── the same launch for the attention half of a DENSE layer (Llama-style: no q/k norm, no router) ─────────────────────────────
 # Three layers, so that the tail of a layer — the MLP's down projection as split-K slabs + residual + next input norm — runs as the
 # first role of the next layer's launch: oracle-followed rows, the five-launch layer on the same tokens, graph ≡ eager.
