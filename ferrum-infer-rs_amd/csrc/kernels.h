@@ -293,6 +293,8 @@ int decode_chain_mlp_max_rows(const W4Device& qkv);
 int decode_chain_mlp_parts(const W4Device& dn);
 bool decode_chain_supports(const DecodeChainDesc& d);
 int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream);
+// behind the last layer: the tail (has_a of a launch that will not follow) and the final norm of the sampled rows, out [n, H]
+int decode_tail_norm_f16(const DecodeChainDesc& d, const int32_t* rows, const __half* w, __half* out, int n, hipStream_t stream);
 
 // ── sampling (sampling.hip) ──────────────────────────────────────────────────
 int argmax_rows_f16_ws(const __half* logits, uint32_t* out_ids, const uint8_t* valid_mask, int mask_len, int m, int n,

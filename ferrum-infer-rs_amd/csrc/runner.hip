@@ -1406,6 +1406,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
                            chain_rows ? reinterpret_cast<unsigned*>(m->chain_rows) : nullptr, chain_rows ? (int)(T * decode_chain_row_bytes(H, nq, nkv, chain_inter) / 4) : 0, s, m->layers[0].qkv.perm));
     m->em2_parity = 0;          // the head kernel made half 0 of the merged launches' counters and rows ready; every such launch does that to the other half
     m->chain_parity = 0;
+    m->head_tail.has_a = false;
     bool qkv_in_perm = m->layers[0].qkv.perm != nullptr;      // norm_out holds the row in L.qkv's packed order
     // decode at ≤ 4 rows (MoE models): the tail of layer l — combine + residual add + next input norm — runs as the prologue of
     // layer l+1's q|k|v GEMM instead of as a launch of its own (every dependent launch costs ≈ 4 µs there)
@@ -1477,6 +1478,10 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
     // residual + norm — q|k|v, attention, o_proj, add + norm), then gate_up slabs → gated activation → down slabs
     bool pending_dense_tail = false, tail_mlp = false;      // (tail_mlp: the slabs are the launch's own)
     int tail_S = 0, tail_rows_pad = 0, tail_n_pad = 0;
+    auto dense_tail = [&](DecodeChainDesc& d) {
+        d.a_slabs = m->workspace; d.a_S = tail_S; d.a_slab_stride = (long)tail_rows_pad * tail_n_pad; d.a_ld = tail_n_pad;
+        d.a_x = tail_S == 0 ? m->mlp_out : nullptr;
+    };
     auto dense_chain_ok = [&](int li) {
         const LayerWeights& L = m->layers[li];
         if (c.num_experts > 0 || !knobs().decode_chain || !knobs().dense_chain || m->em2_failed || !m->em2_arrive || !m->inlaunch_timeouts || !m->residual2) return false;
@@ -1499,8 +1504,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
         if (dense_chain_ok(li)) {
             DecodeChainDesc d = chain_desc(li);
             d.has_a = pending_dense_tail;
-            d.a_slabs = m->workspace; d.a_S = tail_S; d.a_slab_stride = (long)tail_rows_pad * tail_n_pad; d.a_ld = tail_n_pad;
-            d.a_x = tail_S == 0 ? m->mlp_out : nullptr;
+            dense_tail(d);
             d.cnt = m->em2_arrive + (size_t)m->chain_parity * m->arrive_half_words;
             d.cnt_next = m->em2_arrive + (size_t)(m->chain_parity ^ 1) * m->arrive_half_words;
             const int I = c.intermediate;
@@ -1532,19 +1536,21 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             if (mlp) {
             } else if (slabs) { RUN(dense_slabs_gemm(m, L.down, m->act_out, T, &S, &rows_pad, &n_pad, s)); }
             else { RUN(dense_linear(m, L.down, m->act_out, m->mlp_out, T, s)); }
-            if (li + 1 < c.num_layers && dense_chain_ok(li + 1)) {
+            tail_S = S; tail_rows_pad = rows_pad; tail_n_pad = n_pad; tail_mlp = mlp;
+            if (li + 1 == c.num_layers && sh.num_sampled > 0) {
+                m->head_tail = d;                   // the final norm's (once: its slabs lie where the head works)
+                m->head_tail.has_a = true;
+                dense_tail(m->head_tail);
+            } else if (li + 1 < c.num_layers && dense_chain_ok(li + 1)) {
                 pending_dense_tail = true;          // MLP output + residual + next input norm: the first role of the next layer's launch
-                tail_S = S; tail_rows_pad = rows_pad; tail_n_pad = n_pad; tail_mlp = mlp;
-            } else if (!slabs) {
-                if (next_ln) { RUN(fused_add_rms_norm_f16(m->residual2, m->mlp_out, next_ln, c.rms_eps, m->norm_out, T, H, s, next_qkv_perm)); }
-                else { RUN(add_inplace_f16(m->residual2, m->mlp_out, (long)T * H, s)); }
-                FH_CHECK_HIP(hipMemcpyAsync(m->residual, m->residual2, (size_t)T * H * sizeof(__half), hipMemcpyDeviceToDevice, s));
-                qkv_in_perm = next_ln && next_qkv_perm != nullptr;
             } else {
                 // (the residual of this layer sits in the ping-pong buffer: the stand-alone tail works on it in place, then it moves back)
-                RUN(fused_add_rms_norm_route_slabs_f16(m->residual2, nullptr, m->workspace, S, (long)rows_pad * n_pad, n_pad,
-                                                       next_ln ? next_ln : L.input_ln, c.rms_eps, m->norm_out, nullptr, 0, 0, 0, nullptr, nullptr,
-                                                       nullptr, T, H, s, next_qkv_perm));
+                const __half* ln = next_ln ? next_ln : L.input_ln;
+                if (!slabs) { RUN(fused_add_rms_norm_f16(m->residual2, m->mlp_out, ln, c.rms_eps, m->norm_out, T, H, s, next_qkv_perm)); }
+                else {
+                    RUN(fused_add_rms_norm_route_slabs_f16(m->residual2, nullptr, m->workspace, S, (long)rows_pad * n_pad, n_pad, ln, c.rms_eps,
+                                                           m->norm_out, nullptr, 0, 0, 0, nullptr, nullptr, nullptr, T, H, s, next_qkv_perm));
+                }
                 FH_CHECK_HIP(hipMemcpyAsync(m->residual, m->residual2, (size_t)T * H * sizeof(__half), hipMemcpyDeviceToDevice, s));
                 qkv_in_perm = next_ln && next_qkv_perm != nullptr;
             }
@@ -1569,7 +1575,10 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             form_hit(d.Q > 1 ? FORM_ROUTE_SPLIT : FORM_ROUTE_FUSED);
             if (c.expert_parallel) RUN(moe_remap_expert_ids(m->expert_ids, m->expert_ids_local, P, m->ep_e0, m->ep_E, s));
             RUN(moe_decode_gemms(m, L, P, max_blocks, s, d.defer_merge ? &lists : nullptr));
-            if (!c.expert_parallel && li + 1 < c.num_layers && chain_ok(li + 1)) {
+            if (!c.expert_parallel && li + 1 == c.num_layers && sh.num_sampled > 0) {
+                m->head_tail = d;                   // the final norm's
+                m->head_tail.has_a = true;
+            } else if (!c.expert_parallel && li + 1 < c.num_layers && chain_ok(li + 1)) {
                 pending_chain_tail = true;          // combine + add + next input norm: the first role of the next layer's launch
             } else if (!c.expert_parallel) {
                 RUN(moe_combine_add_rms_norm_f16(m->moe_down, m->expert_w, m->residual2, m->residual, next_ln, c.rms_eps, m->norm_out, T, K, H, s,
@@ -1875,7 +1884,9 @@ int enqueue_head(FerrumHipModel* m, int rows) {
     if (c.sandwich_norms) {
         if (int rc = rms_norm_f32_to_f16(m->residual_f32, sampled_idx, m->final_norm, c.rms_eps, m->sampled_hidden, rows, c.hidden, s)) return rc;
     } else {
-        if (int rc = gather_rms_norm_f16(m->residual, sampled_idx, m->final_norm, c.rms_eps, m->sampled_hidden, rows, c.hidden, s)) return rc;
+        if (m->head_tail.has_a) {
+            if (int rc = decode_tail_norm_f16(m->head_tail, sampled_idx, m->final_norm, m->sampled_hidden, rows, s)) return rc;
+        } else if (int rc = gather_rms_norm_f16(m->residual, sampled_idx, m->final_norm, c.rms_eps, m->sampled_hidden, rows, c.hidden, s)) return rc;
     }
     // this rank's vocabulary rows (all of them unless vocabulary parallel)
     return f16t_gemm_f32out(m->sampled_hidden, m->lm_head_t, m->logits, rows, m->vp_n, c.hidden, m->workspace, m->workspace_bytes, s);

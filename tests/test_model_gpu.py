@@ -1160,6 +1160,37 @@ def test_decode_chain_with_the_mlp(pkg, f16, hidden, inter, activation, c, forms
         tm.layers[1]["dense"]["post_ln"] = kept
 
 
+@pytest.mark.parametrize("kind,c", [("moe", 5), ("int4", 5), ("int4", 40), ("f16", 3), ("f16", 40)])
+def test_decode_chain_samples_some_rows(pkg, kind, c, forms, knobs):
+    """Behind the last layer the tail and the final norm run for the sampled rows alone: all of them, some, one; a step that samples none leaves the
+    caches as it should, and listed rows find the residual.  (40 dense rows: the tail adds fp16 rows; fewer: slabs; experts: their combination.  Queries and keys are normed: without
+    that, attention of random weights is a step function, and a row at its edge was 18 % from the oracle in the launches of their own, 23 in this.)"""
+    from tests import modelgen
+    if kind == "moe":
+        tm = _chain_model()
+    else:
+        key = ("some", kind)
+        if key not in _CHAIN_TM:
+            kw = dict(dense_proj=True, tied=True) if kind == "f16" else {}
+            _CHAIN_TM[key] = modelgen.TinyModel(False, layers=2, hidden=1024 if kind == "f16" else 2048, nq=16 if kind == "f16" else 32, nkv=4, hd=128, inter=2048,
+                                                vocab=2048, seed=101, max_seq_len=64, qk_norm=True, **kw)
+        tm = _CHAIN_TM[key]
+    picks = [lambda i: True, lambda i: i % 2 == 1, lambda i: False, lambda i: i == c - 1, lambda i: True]
+    out = {}
+    for chain in (1, 0):
+        knobs.set(DECODE_CHAIN=chain, MOE_EM2=chain)
+        hm = tm.hip_model(pkg, kv_num_blocks=c * 2 + 4, max_seqs=c, max_tokens=max(3 * c, 64))
+        hm.unified_forward([(i, [7 + i, 300, 21], 0, True) for i in range(c)], greedy=True)
+        forms.reset()
+        out[chain] = [hm.unified_forward([(i, [50 + i + s], 3 + s, pick(i)) for i in range(c)], greedy=True, want_logits=True)[1] for s, pick in enumerate(picks)]
+        assert (forms.hits().get("decode_chain", 0) > 0) == bool(chain), forms.hits()
+        del hm
+    for s, (mine, other, pick) in enumerate(zip(out[1], out[0], picks)):
+        n = sum(bool(pick(i)) for i in range(c))
+        if n:
+            assert mine[:n].shape == other[:n].shape and np.abs(mine[:n] - other[:n]).max() < 0.02 * np.abs(other[:n]).max(), s
+
+
 # ── the same launch for the attention half of a DENSE layer (Llama-style: no q/k norm, no router) ─────────────────────────────
 # Three layers, so that the tail of a layer — the MLP's down projection as split-K slabs + residual + next input norm — runs as the
 # first role of the next layer's launch: oracle-followed rows, the five-launch layer on the same tokens, graph ≡ eager.
