@@ -200,8 +200,9 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
             // dense model: the MLP's down projection arrives as S fp32 split-K slabs — summed in slab order and rounded like the
             // fp16 op output (add_rmsnorm_route_kernel<true>, fused.hip), then the residual add
             float o[8];
-            reduce_slabs8(p.a_slabs + (long)row * p.a_ld + i * 8, p.a_slab_stride, p.a_S, o);
             half8 rv = *reinterpret_cast<const half8*>(p.res_in + (long)row * H + i * 8);
+            asm volatile("" ::: "memory");                            // (ahead of the slabs: behind them it is a round trip of its own)
+            reduce_slabs8(p.a_slabs + (long)row * p.a_ld + i * 8, p.a_slab_stride, p.a_S, o);
 #pragma unroll
             for (int j = 0; j < 8; j++) rv[j] = (_Float16)((float)rv[j] + (float)(_Float16)o[j]);
             v[c] = rv;
