@@ -929,7 +929,7 @@ int ferrum_hip_model_finalize(FerrumHipModel* m) {
             *m->inlaunch_timeouts = 0u;
         }
     }
-    if (!rc && m->em2_arrive) {
+    if (!rc && m->em2_arrive && c.head_dim == 128 && !c.sandwich_norms) {
         m->chain_rows_half = CHAIN_MAX_ROWS * decode_chain_row_bytes((int)H, c.num_heads, c.num_kv_heads, c.num_experts > 0 ? 0 : c.intermediate);
         rc |= dev_alloc(&m->chain_rows, 2 * m->chain_rows_half);
     }
@@ -1886,6 +1886,7 @@ int enqueue_head(FerrumHipModel* m, int rows) {
     } else {
         if (m->head_tail.has_a) {
             if (int rc = decode_tail_norm_f16(m->head_tail, sampled_idx, m->final_norm, m->sampled_hidden, rows, s)) return rc;
+            m->head_tail.has_a = false;
         } else if (int rc = gather_rms_norm_f16(m->residual, sampled_idx, m->final_norm, c.rms_eps, m->sampled_hidden, rows, c.hidden, s)) return rc;
     }
     // this rank's vocabulary rows (all of them unless vocabulary parallel)
