@@ -315,8 +315,10 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
                                                                               (g0 + i) * 4 + k) * 64);
     }
     // (GLU, four groups: the last is asked for behind the rows.  Its workgroups fill the chip when the ones before them leave, memory is still busy
-    // with their weights when the rows are there, and loads come back in order: the products of three start a quarter of them earlier)
+    // with their weights when the rows are there, and loads come back in order: the products of three start a quarter of them earlier.  From 5 rows on, whose rows take longer, two of them: a step of 32
+    // layers of 4096, one group | two, µs: 1 row 1259 | 1277, 4 1322 | 1340, 5 1318 | 1293, 8 1376 | 1340, 9 1411 | 1378, 12 of 120 keys 1460 | 1423, 16 1518 | 1488)
     constexpr int LATE = GLU && !F16W ? GPW / 4 : 0;
+    const bool two_late = LATE > 0 && T > 4;
     auto ask = [&](auto from, auto to) {
         if constexpr (!F16W) {
 #pragma unroll
@@ -331,7 +333,10 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
                 }
         }
     };
-    ask(std::integral_constant<int, 0>{}, std::integral_constant<int, GPW - LATE>{});
+    ask(std::integral_constant<int, 0>{}, std::integral_constant<int, GPW - 2 * LATE>{});
+    if constexpr (LATE > 0) {
+        if (!two_late) ask(std::integral_constant<int, GPW - 2 * LATE>{}, std::integral_constant<int, GPW - LATE>{});
+    }
     // the first PRE groups' INT4 weights become numbers (q − 8) while the predecessor works: their expansion, and the products that take the
     // offset of in-place nibbles back, are not behind the wait
     if constexpr (!F16W && PRE > 0) {
@@ -391,6 +396,7 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
     }
     CH_TL(1);
     if constexpr (LATE > 0) {
+        if (two_late) ask(std::integral_constant<int, GPW - 2 * LATE>{}, std::integral_constant<int, GPW - LATE>{});
         ask(std::integral_constant<int, GPW - LATE>{}, std::integral_constant<int, GPW>{});
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -1198,8 +1204,8 @@ bool decode_chain_mlp_supports(const W4Device& qkv, const W4Device& gu, const W4
            (size_t)(dn.G / per) * rows * dn.n * 4 <= slab_bytes;
 }
 // Rows up to which the launch takes the MLP: one block of them, and two of the smallest layers (µs of a step, the MLP's two launches behind the chain
-// | in it.  32 INT4 layers of 4096, inter 14336: 1 row 1393 | 1273, 4 rows 1430 | 1315, 12 of 120 keys 1568 | 1470, 16 1623 | 1513, 17 2096 | 2333, 1 of 8000
-// keys 1591 | 1437.  8 of 4096, 12288, GELU: 1 376 | 344, 8 393 | 368, 16 436 | 404, 17 550 | 557.  8 of 2048, 8192: 1 260 | 230, 8 287 | 246, 16 338 | 271, 17
+// | in it.  32 INT4 layers of 4096, inter 14336: 1 row 1393 | 1273, 4 rows 1430 | 1315, 12 of 120 keys 1568 | 1430, 16 1623 | 1483, 17 2096 | 2333, 1 of 8000
+// keys 1591 | 1437.  8 of 4096, 12288, GELU: 1 376 | 344, 8 393 | 362, 16 436 | 402, 17 550 | 557.  8 of 2048, 8192: 1 260 | 230, 8 287 | 246, 16 338 | 271, 17
 // 407 | 404, 32 428 | 428.  14 fp16 layers of 1024, 3072: 1 371 | 302, 8 418 | 330, 16 441 | 350, 17 488 | 439, 32 523 | 475, 64 707 | 751.  8 of 2048,
 // 6144: 1 310 | 268, 8 339 | 304, 16 368 | 321, 17 420 | 457, 32 450 | 492.)
 int decode_chain_mlp_max_rows(const W4Device& qkv) { return qkv.f16t && qkv.G == 8 ? 32 : 16; }
