@@ -1209,6 +1209,11 @@ bool decode_chain_mlp_supports(const W4Device& qkv, const W4Device& gu, const W4
 // 407 | 404, 32 428 | 428.  14 fp16 layers of 1024, 3072: 1 371 | 302, 8 418 | 330, 16 441 | 350, 17 488 | 439, 32 523 | 475, 64 707 | 751.  8 of 2048,
 // 6144: 1 310 | 268, 8 339 | 304, 16 368 | 321, 17 420 | 457, 32 450 | 492.)
 int decode_chain_mlp_max_rows(const W4Device& qkv) { return qkv.f16t && qkv.G == 8 ? 32 : 16; }
+// Rows up to which a dense layer takes the launch: beyond 64 the 64-row GEMM tiles win (INT4 of 4096 × 14336, 96 rows: 5.56 ms a step against 5.61), and through
+// fp16 layers of 2048 columns the fourth block of rows costs more than the launches of their own (µs of a step of 6 layers, those | this one: 32 heads on 8, 48 rows
+// 460 | 461, 52 464 | 517, 64 515 | 569; 32 on 4, 48 rows 412 | 410, 52 418 | 459, 64 445 | 495; 16 on 8, 48 rows 432 | 409, 52 438 | 449, 64 486 | 496; of 1024 columns,
+// 16 on 8: 52 rows 319 | 303, 64 365 | 341).
+int decode_chain_dense_max_rows(const W4Device& qkv) { return qkv.f16t && qkv.G > 8 ? 48 : 64; }
 int decode_chain_mlp_parts(const W4Device& dn) { return dn.G / (8 * chain_mlp_groups(dn.f16t != nullptr)); }
 
 bool decode_chain_supports(const DecodeChainDesc& d) {
@@ -1300,7 +1305,7 @@ int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
     if (a.attn_splits > 1) form_hit(FORM_CHAIN_ATTN_KV_SPLITS);
     if (a.qkv_wide) form_hit(FORM_CHAIN_QKV_WIDE);
     if (mlp) form_hit(FORM_CHAIN_MLP);
-    // Unquantised layers (dense ones of 1024 – 2048 columns, up to 64 rows; a wave's weights of 4096 columns do not fit its registers, and such
+    // Unquantised layers (dense ones of 1024 – 2048 columns; a wave's weights of 4096 columns do not fit its registers, and such
     // layers are streaming, not waiting).  A step of 14 layers of 1024 columns, the launches of their own | this one, µs: 1 row of 60 keys
     // 470 | 380, 8 rows 505 | 424, 16 542 | 450, 17 538 | 491, 32 583 | 527, 33 655 | 572, 48 696 | 643, 64 735 | 723; 1 of 1500 keys 592 | 419, 8 of 900
     // 622 | 538, 32 of 500 732 | 643, 64 of 300 857 | 826.

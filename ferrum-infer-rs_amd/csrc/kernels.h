@@ -291,6 +291,7 @@ size_t decode_chain_row_bytes(int H, int nq, int nkv, int inter = 0);
 bool decode_chain_mlp_supports(const W4Device& qkv, const W4Device& gu, const W4Device& dn, int inter, int rows, size_t slab_bytes);
 int decode_chain_mlp_max_rows(const W4Device& qkv);
 int decode_chain_mlp_parts(const W4Device& dn);
+int decode_chain_dense_max_rows(const W4Device& qkv);
 bool decode_chain_supports(const DecodeChainDesc& d);
 int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream);
 // behind the last layer: the tail (has_a of a launch that will not follow) and the final norm of the sampled rows, out [n, H]

@@ -1485,7 +1485,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
     auto dense_chain_ok = [&](int li) {
         const LayerWeights& L = m->layers[li];
         if (c.num_experts > 0 || !knobs().decode_chain || !knobs().dense_chain || m->em2_failed || !m->em2_arrive || !m->inlaunch_timeouts || !m->residual2) return false;
-        if (!sh.all_single_token || !m->fuse_rope_attn || T > std::min(64, knobs().chain_max_rows) || m->taps_enabled || sandwich || c.tp_world > 1) return false;      // (beyond 64 rows the 64-row GEMM tiles win: Llama-3.1-8B c=96 5.56 vs 5.61 ms)
+        if (!sh.all_single_token || !m->fuse_rope_attn || T > std::min(decode_chain_dense_max_rows(L.qkv), knobs().chain_max_rows) || m->taps_enabled || sandwich || c.tp_world > 1) return false;
         if (L.gate_up.perm || L.down.perm || L.qkv.perm || L.o.perm) return false;
         if (L.o.f16t ? !L.down.f16t || !f16t_gemm_gated_supports(L.gate_up, c.intermediate) : !L.o.qw || !L.gate_up.qw || !L.down.qw) return false;
         if (L.qkv.bias || L.o.bias || !chain_kv_ok(li)) return false;

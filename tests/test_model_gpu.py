@@ -1066,10 +1066,11 @@ def test_decode_chain_of_wide_layers(pkg, c, forms):
 
 
 @pytest.mark.parametrize("hidden,nq,nkv", [(1024, 16, 8), (2048, 16, 8), (2048, 32, 4)])
-@pytest.mark.parametrize("c,splits", [(1, 1), (9, 1), (16, 5), (17, 1), (33, 1), (64, 1)])
+@pytest.mark.parametrize("c,splits", [(1, 1), (9, 1), (16, 5), (17, 1), (33, 1), (48, 1), (49, 1), (64, 1)])
 def test_decode_chain_of_unquantised_layers(pkg, hidden, nq, nkv, c, splits, forms, knobs):
     """fp16 projections in the launch: one or two 128-column slices of K a wave in q|k|v, two or four in o_proj's two parts, blocks of 32 and of 64
-    columns, one and several KV ranges; rows against the oracle, layers of several (the first role adds the MLP's fp16 rows), then the hipGraph loop."""
+    columns, one and several KV ranges; rows against the oracle, layers of several (the first role adds the MLP's fp16 rows), then the hipGraph loop.  Layers of 2048
+    columns take it up to 48 rows."""
     from tests import modelgen
     from oracle import oracle as O
     key = ("f16", hidden, nq)
@@ -1102,7 +1103,8 @@ def test_decode_chain_of_unquantised_layers(pkg, hidden, nq, nkv, c, splits, for
         for oc, i in enumerate(followed):
             cur[i] = par.check(f"step{s}/{i}", om.forward(oc, np.array([fed[i]], np.uint32), plen + s), lg[i], toks[i])
     h = forms.hits()
-    assert h.get("decode_chain", 0) == 2 * steps and h.get("dense_chain", 0) == 2 * steps, h
+    launches = 2 * steps if hidden == 1024 or c <= 48 else 0
+    assert h.get("decode_chain", 0) == launches and h.get("dense_chain", 0) == launches, h
     assert h.get("chain_attn_kv_splits", 0) == (2 * steps if splits > 1 else 0), h
     O.set_threads(1)
     par.finish(max_mismatches=0, max_route_ties=0)
