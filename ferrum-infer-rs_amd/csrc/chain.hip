@@ -1103,7 +1103,7 @@ __global__ __launch_bounds__(512, 2) void decode_chain_kernel(ChainArgs p) {
     const int n_a = p.has_a ? p.T : 0, n_qkv = p.qkv.N / QB * RH, n_attn = p.T * p.nkv * (KVS ? p.attn_splits : 1), n_o = p.o.N / (p.o_half ? 32 : 64 * CH_O_NST) * RH * CH_O_KS;
     int wg = blockIdx.x;
     if (wg == 0) {                                                    // re-arm the other half of the route granules
-        for (int i = threadIdx.x; i < p.T * p.Q * CH_GRAN * 2; i += 512) p.cnt_next[i] = 0u;
+        for (int i = threadIdx.x; i < (p.E > 0 ? p.T * p.Q * CH_GRAN * 2 : 0); i += 512) p.cnt_next[i] = 0u;
     }
     if (wg < n_a) { chain_role_a(p, wg, smem); return; }
     wg -= n_a;
@@ -1227,7 +1227,7 @@ bool decode_chain_supports(const DecodeChainDesc& d) {
     // the instantiated forms: a wave's K slices
     const int gq = d.qkv->G / 8, go = d.o->G / 8;
     if (f16w ? d.E > 0 || !((gq == 1 && go == 2) || (gq == 2 && (go == 2 || go == 4))) : !((gq == 2 || gq == 4) && go == 4)) return false;
-    if (!d.rows || !d.rows_next || CH_MAX_T * decode_chain_row_bytes(d.H, d.nq, d.nkv, d.rows_inter) >= (1UL << 31)) return false;
+    if (CH_MAX_T * decode_chain_row_bytes(d.H, d.nq, d.nkv, d.rows_inter) >= (1UL << 31)) return false;
     if (d.gate_up && (d.E > 0 || !d.down_proj || !d.slabs || d.rows_inter != d.down_proj->k ||
                       !decode_chain_mlp_supports(*d.qkv, *d.gate_up, *d.down_proj, d.rows_inter, d.T, ~(size_t)0))) return false;
     if (d.attn_splits > CH_MAX_SPLITS || (d.attn_splits > 1 && (!d.attn_partial || !d.attn_tickets))) return false;
@@ -1247,7 +1247,7 @@ bool decode_chain_supports(const DecodeChainDesc& d) {
 }
 
 int decode_chain_f16(const DecodeChainDesc& d, hipStream_t stream) {
-    FH_REQUIRE(decode_chain_supports(d), "decode_chain: shapes not taken by the merged form");
+    FH_REQUIRE(d.rows && d.rows_next && decode_chain_supports(d), "decode_chain: shapes not taken by the merged form");
     ChainArgs a{};
     chain_tail_args(d, a);
     a.nq = d.nq; a.nkv = d.nkv;

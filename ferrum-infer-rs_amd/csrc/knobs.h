@@ -169,6 +169,7 @@ enum Form : int {
     FORM_TILED_GEMM_COLS64,     // few-row projection with 64 columns a wave
     FORM_TILED_GEMM_256X256,    // prompts: tiles of 256 × 256, a workgroup's one after the other (tiled_gemm_wide.hip)
     FORM_CHAIN_MLP,             // decode chain: the MLP of a dense layer in the launch too
+    FORM_CHAIN_ROWS,            // decode chain: a forward's head made its rows ready
     FORM_COUNT
 };
 

@@ -320,6 +320,28 @@ static int check_inlaunch_waits(FerrumHipModel* m) {
     return 3;
 }
 
+// What does not change from step to step of whether a layer takes the chain launch (chain.hip): the model's kind, the weights' forms and shapes.
+static DecodeChainDesc chain_shape(const FerrumHipModel* m, const LayerWeights& L) {
+    const FerrumHipModelConfig& c = m->cfg;
+    DecodeChainDesc d;
+    d.T = 1; d.H = c.hidden; d.nq = c.num_heads; d.nkv = c.num_kv_heads; d.head_dim = c.head_dim;
+    d.qkv = &L.qkv; d.o = &L.o;
+    d.E = c.num_experts; d.top_k = d.r_top_k = c.top_k; d.norm_topk = c.norm_topk_prob;
+    int Q = m->route_parts;
+    const int tiles = (c.num_experts + 15) / 16;
+    while (Q > 1 && (tiles % Q != 0 || Q > 8)) Q >>= 1;
+    d.Q = c.num_experts > 0 ? Q : 1;
+    return d;
+}
+static bool chain_takes_layer(const FerrumHipModel* m, const LayerWeights& L) {
+    const FerrumHipModelConfig& c = m->cfg;
+    if (c.sandwich_norms || (c.tp_world > 1 && (c.num_experts <= 0 || c.expert_parallel != 2))) return false;      // (tensor-parallel attention: an all-reduce sits behind o_proj)
+    if (c.num_experts > 0) return c.top_k <= 8 && decode_chain_supports(chain_shape(m, L));
+    if (L.gate_up.perm || L.down.perm || L.qkv.perm || L.o.perm || L.qkv.bias || L.o.bias) return false;
+    if (L.o.f16t ? !L.down.f16t || !f16t_gemm_gated_supports(L.gate_up, c.intermediate) : !L.o.qw || !L.gate_up.qw || !L.down.qw) return false;
+    return decode_chain_supports(chain_shape(m, L));
+}
+
 static int q_dim(const FerrumHipModelConfig& c) { return c.num_heads * c.head_dim; }
 static int kv_dim(const FerrumHipModelConfig& c) { return c.num_kv_heads * c.head_dim; }
 static int qkv_dim(const FerrumHipModelConfig& c) { return q_dim(c) + 2 * kv_dim(c); }
@@ -929,8 +951,15 @@ int ferrum_hip_model_finalize(FerrumHipModel* m) {
             *m->inlaunch_timeouts = 0u;
         }
     }
-    if (!rc && m->em2_arrive && c.head_dim == 128 && !c.sandwich_norms) {
-        m->chain_rows_half = CHAIN_MAX_ROWS * decode_chain_row_bytes((int)H, c.num_heads, c.num_kv_heads, c.num_experts > 0 ? 0 : c.intermediate);
+    // rows handed off inside the chain launch: for models with a layer that can take it
+    bool chain = false, chain_mlp = false;
+    for (const LayerWeights& L : m->layers) {
+        if (!chain_takes_layer(m, L)) continue;
+        chain = true;
+        chain_mlp |= c.num_experts == 0 && decode_chain_mlp_supports(L.qkv, L.gate_up, L.down, c.intermediate, 1, ~(size_t)0);
+    }
+    if (!rc && m->em2_arrive && chain) {
+        m->chain_rows_half = CHAIN_MAX_ROWS * decode_chain_row_bytes((int)H, c.num_heads, c.num_kv_heads, chain_mlp ? c.intermediate : 0);
         rc |= dev_alloc(&m->chain_rows, 2 * m->chain_rows_half);
     }
     if (!rc && m->em2_arrive && c.head_dim == 128) {
@@ -1390,23 +1419,11 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
         if ((rc = (x))) return rc;                                                   \
         if (trace) FH_CHECK_HIP(hipStreamSynchronize(s));                            \
     } while (0)
-    // arrival counters of the split route kernel: re-armed by the kernel itself, but zeroed per forward as well (by the head
-    // kernel below) so that an aborted launch can never poison the next one
     const bool sandwich = c.sandwich_norms != 0;
-    // head, one launch: embedding_lookup (+ the Gemma embedding scale, llama_family.rs:3656) → residual stream (fp16; for
-    // sandwich-norm models also the fp32 shadow, llama_family.rs:3664-3674) → layer 0's input norm.  Later layers get their
-    // input norm fused into the previous layer's tail.
-    // act-order (desc_act) projections read x'[j] = x[perm[j]]: the kernel that PRODUCES the row writes it permuted wherever one
-    // workgroup owns the row (every norm of the dense layer) or the rows are few (decode attention scatters); the gated
-    // activation is permuted by gate_up's column order (pack_gate_up).  Only the prefill o_proj keeps a gather launch.
-    const bool chain_rows = m->chain_rows && sh.all_single_token && T <= std::min(CHAIN_MAX_ROWS, knobs().chain_max_rows);
-    const int chain_inter = c.num_experts == 0 && T <= std::min(decode_chain_mlp_max_rows(m->layers[0].qkv), knobs().chain_mlp_rows) ? c.intermediate : 0;      // the MLP in the chain launch
-    RUN(embed_rms_norm_f16(m->embed, tokens, c.embed_scale, m->residual, sandwich ? m->residual_f32 : nullptr, m->layers[0].input_ln,
-                           c.rms_eps, m->norm_out, T, H, m->route_arrive, m->route_arrive ? 64 + (int)m->arrive_half_words : 0,
-                           chain_rows ? reinterpret_cast<unsigned*>(m->chain_rows) : nullptr, chain_rows ? (int)(T * decode_chain_row_bytes(H, nq, nkv, chain_inter) / 4) : 0, s, m->layers[0].qkv.perm));
-    m->em2_parity = 0;          // the head kernel made half 0 of the merged launches' counters and rows ready; every such launch does that to the other half
+    m->em2_parity = 0;          // the head kernel makes half 0 of the merged launches' counters and rows ready; every such launch does that to the other half
     m->chain_parity = 0;
     m->head_tail.has_a = false;
+    int chain_inter = c.num_experts == 0 && T <= std::min(decode_chain_mlp_max_rows(m->layers[0].qkv), knobs().chain_mlp_rows) ? c.intermediate : 0;      // the MLP in the chain launch
     bool qkv_in_perm = m->layers[0].qkv.perm != nullptr;      // norm_out holds the row in L.qkv's packed order
     // decode at ≤ 4 rows (MoE models): the tail of layer l — combine + residual add + next input norm — runs as the prologue of
     // layer l+1's q|k|v GEMM instead of as a launch of its own (every dependent launch costs ≈ 4 µs there)
@@ -1415,11 +1432,10 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
     bool pending_chain_tail = false;
     auto chain_desc = [&](int li) {
         LayerWeights& L = m->layers[li];
-        DecodeChainDesc d;
-        d.T = T; d.H = H; d.nq = nq; d.nkv = nkv; d.head_dim = hd;
-        d.top_k = c.top_k; d.down = m->moe_down; d.comb_w = m->expert_w; d.res_in = m->residual2; d.ln_in = L.input_ln; d.eps = c.rms_eps;
+        DecodeChainDesc d = chain_shape(m, L);
+        d.T = T;
+        d.down = m->moe_down; d.comb_w = m->expert_w; d.res_in = m->residual2; d.ln_in = L.input_ln; d.eps = c.rms_eps;
         d.res_a = m->residual; d.norm1 = m->norm_out;
-        d.qkv = &L.qkv;
         d.k_pool = L.k_pool; d.v_pool = L.v_pool; d.block_tables = bt; d.kv_lens = kvl;
         d.q_norm_w = L.q_norm ? L.q_norm : L.input_ln; d.k_norm_w = L.k_norm ? L.k_norm : L.input_ln;
         const int pattern = c.sliding_window_pattern;
@@ -1428,15 +1444,9 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
         d.cos_t = (!is_global && m->cos_local) ? m->cos_local : m->cos_t;
         d.sin_t = (!is_global && m->sin_local) ? m->sin_local : m->sin_t;
         d.qk_mode = qk_mode; d.max_blocks = m->max_blocks_per_seq;
-        d.o = &L.o;
         d.rows_inter = chain_inter;
-        if (m->chain_rows) { d.rows = m->chain_rows + m->chain_parity * m->chain_rows_half; d.rows_next = m->chain_rows + (m->chain_parity ^ 1) * m->chain_rows_half; }
+        d.rows = m->chain_rows + m->chain_parity * m->chain_rows_half; d.rows_next = m->chain_rows + (m->chain_parity ^ 1) * m->chain_rows_half;
         d.res_b_out = m->residual2; d.post_ln = L.post_ln; d.norm2 = m->norm_out; d.router_w = L.router;
-        d.E = c.num_experts; d.r_top_k = c.top_k; d.norm_topk = c.norm_topk_prob;
-        int Q = m->route_parts;
-        const int tiles = (c.num_experts + 15) / 16;
-        while (Q > 1 && (tiles % Q != 0 || Q > 8)) Q >>= 1;
-        d.Q = c.num_experts > 0 ? Q : 1;
         d.cand = m->route_cand; d.stats = m->route_stats; d.route_arrive = m->route_arrive; d.ids = m->expert_ids; d.weights = m->expert_w;
         d.timeout = m->inlaunch_timeouts;
         // KV ranges per (sequence, kv head) in the attention role: ≈ chain_split_keys (256) keys each while the role stays within
@@ -1467,13 +1477,41 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
         const long keys = window > 0 ? std::min<long>(sh.max_kv_len, window) : sh.max_kv_len;
         return keys <= (long)knobs().chain_max_keys * chain_desc(li).attn_splits * std::max<long>(1, (long)T * nkv / 128);
     };
-    auto chain_ok = [&](int li) {
-        if (c.num_experts <= 0 || !knobs().decode_chain || m->em2_failed || !m->em2_arrive || !m->inlaunch_timeouts) return false;
-        if (!sh.all_single_token || !m->fuse_rope_attn || T > knobs().chain_max_rows || m->taps_enabled || sandwich) return false;
-        if (c.tp_world > 1 && c.expert_parallel != 2) return false;             // (tensor-parallel attention: an all-reduce sits behind o_proj)
-        if (T * c.top_k > 1024 || c.top_k > 8 || T > 128 || !chain_kv_ok(li)) return false;
+    // the chain launch, from a step's side: single tokens, few rows, merged forms still on
+    const bool chain_step = m->chain_rows && m->em2_arrive && m->inlaunch_timeouts && !m->em2_failed && knobs().decode_chain && sh.all_single_token && m->fuse_rope_attn &&
+                            !m->taps_enabled && T <= std::min(CHAIN_MAX_ROWS, knobs().chain_max_rows) && (c.num_experts > 0 ? T * c.top_k <= 1024 : knobs().dense_chain && m->residual2);
+    auto layer_chains = [&](int li) {
+        const LayerWeights& L = m->layers[li];
+        if (!chain_step || !chain_takes_layer(m, L) || (c.num_experts == 0 && T > decode_chain_dense_max_rows(L.qkv)) || !chain_kv_ok(li)) return false;
         return decode_chain_supports(chain_desc(li));
     };
+    auto layer_chains_mlp = [&](int li) {
+        const LayerWeights& L = m->layers[li];
+        return chain_inter > 0 && decode_chain_mlp_supports(L.qkv, L.gate_up, L.down, c.intermediate, T, m->workspace_bytes);
+    };
+    auto chain_ok = [&](int li) { return c.num_experts > 0 && layer_chains(li); };
+    auto dense_chain_ok = [&](int li) { return c.num_experts == 0 && layer_chains(li); };
+    // … and only if some layer takes it are there rows to make ready, with the MLP's only if one takes its MLP too
+    bool chain_rows = false, chain_mlp = false;
+    for (int li = 0; chain_step && li < c.num_layers && !(chain_rows && (chain_mlp || chain_inter == 0)); li++)
+        if (layer_chains(li)) {
+            chain_rows = true;
+            chain_mlp |= layer_chains_mlp(li);
+        }
+    if (!chain_mlp) chain_inter = 0;
+    if (chain_rows) form_hit(FORM_CHAIN_ROWS);
+    // head, one launch: embedding_lookup (+ the Gemma embedding scale, llama_family.rs:3656) → residual stream (fp16; for
+    // sandwich-norm models also the fp32 shadow, llama_family.rs:3664-3674) → layer 0's input norm.  Later layers get their
+    // input norm fused into the previous layer's tail.
+    // act-order (desc_act) projections read x'[j] = x[perm[j]]: the kernel that PRODUCES the row writes it permuted wherever one
+    // workgroup owns the row (every norm of the dense layer) or the rows are few (decode attention scatters); the gated
+    // activation is permuted by gate_up's column order (pack_gate_up).  Only the prefill o_proj keeps a gather launch.
+    // arrival counters of the split route kernel: re-armed by the kernel itself, but zeroed per forward as well (by the head
+    // kernel below) so that an aborted launch can never poison the next one
+    const bool counters = c.num_experts > 0 && m->route_arrive;
+    RUN(embed_rms_norm_f16(m->embed, tokens, c.embed_scale, m->residual, sandwich ? m->residual_f32 : nullptr, m->layers[0].input_ln,
+                           c.rms_eps, m->norm_out, T, H, counters ? m->route_arrive : nullptr, counters ? 64 + (int)m->arrive_half_words : 0,
+                           chain_rows ? reinterpret_cast<unsigned*>(m->chain_rows) : nullptr, chain_rows ? (int)(T * decode_chain_row_bytes(H, nq, nkv, chain_inter) / 4) : 0, s, m->layers[0].qkv.perm));
     // dense models at 17–32 rows: the same launch for the attention half (tail of the previous layer's MLP — its down slabs +
     // residual + norm — q|k|v, attention, o_proj, add + norm), then gate_up slabs → gated activation → down slabs
     bool pending_dense_tail = false, tail_mlp = false;      // (tail_mlp: the slabs are the launch's own)
@@ -1481,17 +1519,6 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
     auto dense_tail = [&](DecodeChainDesc& d) {
         d.a_slabs = m->workspace; d.a_S = tail_S; d.a_slab_stride = (long)tail_rows_pad * tail_n_pad; d.a_ld = tail_n_pad;
         d.a_x = tail_S == 0 ? m->mlp_out : nullptr;
-    };
-    auto dense_chain_ok = [&](int li) {
-        const LayerWeights& L = m->layers[li];
-        if (c.num_experts > 0 || !knobs().decode_chain || !knobs().dense_chain || m->em2_failed || !m->em2_arrive || !m->inlaunch_timeouts || !m->residual2) return false;
-        if (!sh.all_single_token || !m->fuse_rope_attn || T > std::min(decode_chain_dense_max_rows(L.qkv), knobs().chain_max_rows) || m->taps_enabled || sandwich || c.tp_world > 1) return false;
-        if (L.gate_up.perm || L.down.perm || L.qkv.perm || L.o.perm) return false;
-        if (L.o.f16t ? !L.down.f16t || !f16t_gemm_gated_supports(L.gate_up, c.intermediate) : !L.o.qw || !L.gate_up.qw || !L.down.qw) return false;
-        if (L.qkv.bias || L.o.bias || !chain_kv_ok(li)) return false;
-        DecodeChainDesc d = chain_desc(li);
-        d.has_a = false;
-        return decode_chain_supports(d);
     };
     for (int li = 0; li < c.num_layers; li++) {
         LayerWeights& L = m->layers[li];
@@ -1509,7 +1536,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             d.cnt_next = m->em2_arrive + (size_t)(m->chain_parity ^ 1) * m->arrive_half_words;
             const int I = c.intermediate;
             // (several blocks of rows: a block's slabs are written when its rows are through the launch, so those that its tail reads must lie as these do)
-            const bool mlp = chain_inter > 0 && (T <= 16 || !pending_dense_tail || tail_mlp) && decode_chain_mlp_supports(L.qkv, L.gate_up, L.down, I, T, m->workspace_bytes);
+            const bool mlp = (T <= 16 || !pending_dense_tail || tail_mlp) && layer_chains_mlp(li);
             if (mlp) { d.gate_up = &L.gate_up; d.down_proj = &L.down; d.slabs = m->workspace; d.gelu = c.activation == 1; }
             RUN(decode_chain_f16(d, s));
             m->chain_parity ^= 1;

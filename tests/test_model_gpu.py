@@ -1065,6 +1065,31 @@ def test_decode_chain_of_wide_layers(pkg, c, forms):
     par.finish(max_mismatches=1, max_route_ties=0)
 
 
+@pytest.mark.parametrize("kind,c,chain,rows", [
+    ("moe", 1, 1, 1), ("moe", 1, 0, 0), ("int4", 1, 1, 1), ("int4", 64, 1, 1), ("int4", 65, 1, 0), ("int4", 1, 0, 0),
+    ("narrow", 1, 1, 0), ("f16", 64, 1, 1), ("f16", 65, 1, 0)])
+def test_decode_chain_rows_are_readied_where_it_runs(pkg, kind, c, chain, rows, forms, knobs):
+    """The head of a forward makes the chain's rows ready if a layer of it takes the chain, and only then: not past its rows, for layers of another width, with the
+    form switched off, or for prompts."""
+    from tests import modelgen
+    if kind == "moe":
+        tm = _chain_model()
+    else:
+        key = ("rows", kind)
+        if key not in _CHAIN_TM:
+            kw = dict(dense_proj=True, tied=True) if kind == "f16" else {}
+            _CHAIN_TM[key] = modelgen.TinyModel(False, layers=2, hidden=2048 if kind == "int4" else 1024, nq=32 if kind == "int4" else 16, nkv=4, hd=128, inter=1024,
+                                                vocab=512, seed=103, max_seq_len=64, **kw)
+        tm = _CHAIN_TM[key]
+    knobs.set(DECODE_CHAIN=chain)
+    hm = tm.hip_model(pkg, kv_num_blocks=c * 2 + 4, max_seqs=c, max_tokens=max(3 * c, 64))
+    forms.reset()
+    hm.unified_forward([(i, [7 + i, 300, 21], 0, True) for i in range(c)], greedy=True)
+    assert not forms.hits().get("chain_rows"), forms.hits()
+    hm.unified_forward([(i, [50 + i], 3, True) for i in range(c)], greedy=True)
+    assert forms.hits().get("chain_rows", 0) == rows and bool(forms.hits().get("decode_chain")) == bool(rows), forms.hits()
+
+
 @pytest.mark.parametrize("hidden,nq,nkv", [(1024, 16, 8), (2048, 16, 8), (2048, 32, 4)])
 @pytest.mark.parametrize("c,splits", [(1, 1), (9, 1), (16, 5), (17, 1), (33, 1), (48, 1), (49, 1), (64, 1)])
 def test_decode_chain_of_unquantised_layers(pkg, hidden, nq, nkv, c, splits, forms, knobs):
