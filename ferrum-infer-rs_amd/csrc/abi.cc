@@ -46,6 +46,7 @@ void reload_knobs() {
     k.moe_deferred_merge = env_int("FERRUM_HIP_MOE_DEFERRED_MERGE", 1);
     k.moe_bm2 = env_int("FERRUM_HIP_MOE_BM2", 0);
     k.dense_chain = env_int("FERRUM_HIP_DENSE_CHAIN", 1);
+    k.inlaunch_give_up = env_int("FERRUM_HIP_INLAUNCH_GIVE_UP", 0);
     k.chain_mlp_rows = env_int("FERRUM_HIP_CHAIN_MLP_ROWS", 32);
     k.chain_max_keys = env_int("FERRUM_HIP_CHAIN_MAX_KEYS", 4096);
     k.chain_split_keys = env_int("FERRUM_HIP_CHAIN_SPLIT_KEYS", 256);
@@ -111,7 +112,7 @@ static const char* const g_form_names[FORM_COUNT] = {
     "perm_producer", "moe_expert_major_pair", "decode_chain", "moe_deferred_merge", "dense_chain", "tp_allreduce_norm_fused", "moe_block_major_pair", "chain_attn_kv_splits", "chain_qkv_wide", "route_gemm_topk",
     "tiled_gemm", "tiled_gemm_big", "tiled_gemm_128x256", "tiled_gemm_128x128", "tiled_gemm_128x64", "tiled_gemm_64x64", "tiled_gemm_grouped", "tiled_gemm_grouped_big", "moe_route_sort", "latent_attn_plain", "latent_attn", "latent_attn_pair", "latent_attn_split", "latent_attn_expanded", "rglru_step", "rglru_scan",
     "grouped_attn_plain", "grouped_attn_keys", "grouped_attn_split", "grouped_attn_tile", "linear_step", "linear_chunk", "scan_step", "scan_chunk", "route_grouped",
-    "route_softmax", "talk_attn_plain", "talk_attn_keys", "talk_attn_tile", "talk_attn_tile_split", "w4_rows", "w4_gated", "f16_gated", "tiled_gemm_cols64", "tiled_gemm_256x256", "chain_mlp", "chain_rows"};
+    "route_softmax", "talk_attn_plain", "talk_attn_keys", "talk_attn_tile", "talk_attn_tile_split", "w4_rows", "w4_gated", "f16_gated", "tiled_gemm_cols64", "tiled_gemm_256x256", "chain_mlp", "chain_rows", "done_again"};
 const char* form_name(int f) { return f >= 0 && f < FORM_COUNT ? g_form_names[f] : nullptr; }
 }  // namespace fh
 

@@ -31,6 +31,7 @@ struct Knobs {
     // INT4 GEMMs (w4_gemm.hip)
     int moe_kw_pairs = 16;
     int decode_chain = 1;             // MoE decode at ≤ 32 rows: tail + q|k|v + attention + o_proj + route as ONE launch (0 = five launches)
+    int inlaunch_give_up = 0;         // tests: 1 = a forward with chain launches counts as one whose waits gave up, with NaN where it wrote K and V
     int chain_max_rows = 128;         // decode chain up to this many rows (≤ 128)
     int sandwich_wide = 1;            // sandwich add + norms of ≤ 64 rows: 1024 threads per row, loads ahead of the reductions (0 = 256 threads)
     int chain_qkv_half = 1;           // decode chain at ≤ 16 rows: q|k|v in 32-column blocks (0 = 64)
@@ -170,6 +171,7 @@ enum Form : int {
     FORM_TILED_GEMM_256X256,    // prompts: tiles of 256 × 256, a workgroup's one after the other (tiled_gemm_wide.hip)
     FORM_CHAIN_MLP,             // decode chain: the MLP of a dense layer in the launch too
     FORM_CHAIN_ROWS,            // decode chain: a forward's head made its rows ready
+    FORM_DONE_AGAIN,            // a call whose in-launch waits gave up was done again in separate launches
     FORM_COUNT
 };
 

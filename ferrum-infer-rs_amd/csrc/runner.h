@@ -87,6 +87,7 @@ struct FerrumHipModel {
     __half* residual2 = nullptr;          // ping-pong partner of `residual` for the Q-part route kernel
     unsigned char* chain_rows = nullptr;  // decode chain: the rows handed off inside a launch, two halves that its launches take in turn
     size_t chain_rows_half = 0;           // bytes
+    bool chain_ran = false;               // the forward queued last has chain launches
     fh::DecodeChainDesc head_tail;            // has_a: what the body just queued leaves its last layer's tail to the head
     float* chain_attn_partial = nullptr;  // decode chain, attention role with KV splits: [≤ 1024 (unit, split)][16][head_dim + 4] states
     unsigned* chain_attn_tickets = nullptr;   // [4096] one self-resetting ticket per (sequence, kv head)

@@ -297,27 +297,75 @@ static void drop_graph(FerrumHipModel* m) {
     if (m->graph) { (void)hipGraphDestroy(m->graph); m->graph = nullptr; }
 }
 
-// Merged launches hand data over between workgroups and bound every wait; a wait that gave up has produced garbage.  Called
-// after every host synchronisation of a forward: the call fails, the captured graph is dropped and the merged forms stay off.
-static int check_inlaunch_waits(FerrumHipModel* m) {
-    // tensor / expert / vocabulary parallel: a one-shot all-reduce or all-gather whose wait for a peer gave up left the rank's
-    // un-reduced partial in the output — ids sampled from it must not be handed back as a success
+// Tensor / expert / vocabulary parallel: a one-shot all-reduce or all-gather whose wait for a peer gave up left the rank's un-reduced partial in
+// the output — ids sampled from it must not be handed back as a success.  Called after every host synchronisation of a forward.
+static int check_peer_waits(FerrumHipModel* m) {
     if (const unsigned n = comm_take_timeouts(m->comm)) {
         drop_graph(m);
         fh::set_error("%u one-shot collective call(s) gave up waiting for a peer: the results of this call are invalid; the one-shot "
                       "transport is off from now on (RCCL, where the communicator has a rank)", n);
         return 3;
     }
+    return 0;
+}
+
+// K and V of the positions [begin, begin + n) of a sequence, which a call writes
+struct Written { uint64_t seq; int begin, n; };
+static __global__ void fill_slots_kernel(__half* __restrict__ k, __half* __restrict__ v, const int2* __restrict__ at, int nkv, int hd, uint16_t bits) {
+    const int2 p = at[blockIdx.x];
+    const long tile = ((long)p.x * nkv + blockIdx.y) * kv_tile_elems(hd);
+    for (int d = threadIdx.x; d < hd; d += 64) {
+        reinterpret_cast<uint16_t*>(k)[tile + k_tile_off(p.y, d)] = bits;
+        reinterpret_cast<uint16_t*>(v)[tile + v_tile_off(p.y, d)] = bits;
+    }
+}
+static int fill_written(FerrumHipModel* m, const std::vector<Written>& written, uint16_t bits) {
+    std::vector<int2> at;
+    for (const Written& w : written)
+        for (int p = w.begin; p < w.begin + w.n; p++) at.push_back(int2{(int)m->seqs[w.seq].blocks[p / KV_BLOCK], p % KV_BLOCK});
+    int2* dev = nullptr;
+    FH_CHECK_HIP(hipMalloc((void**)&dev, at.size() * sizeof(int2)));
+    hipError_t e = hipMemcpy(dev, at.data(), at.size() * sizeof(int2), hipMemcpyHostToDevice);
+    for (LayerWeights& L : m->layers)
+        if (e == hipSuccess) {
+            hipLaunchKernelGGL(fill_slots_kernel, dim3((unsigned)at.size(), m->cfg.num_kv_heads), dim3(64), 0, m->stream, L.k_pool, L.v_pool, dev, m->cfg.num_kv_heads, m->cfg.head_dim, bits);
+            e = hipGetLastError();
+        }
+    if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
+    (void)hipFree(dev);
+    FH_CHECK_HIP(e);
+    return 0;
+}
+
+// Merged launches (the decode chain, gate_up → down of experts) hand data over between workgroups and bound every wait.  One launch cannot starve itself: nothing
+// waits for a workgroup behind it.  Two of them can, on two streams or in two processes: the waiting workgroups of each may hold the places, on one XCD, that
+// the other's producers need; and a process that the system takes off the card for long waits too.  A wait that gave up has produced garbage: the
+// merged forms stay off, the captured graph is dropped, and the call's work is done again in separate launches.  (Its inputs are untouched; the K and V that it
+// wrote are cleared first: rows that nobody wrote are NaN, and attention's zero weight of a key behind a sequence's end keeps a NaN of its V.)  With other ranks in the
+// step the call fails instead, `*refused`.
+template <typename W, typename F>
+static int attempt(FerrumHipModel* m, int* refused, const W& written, const F& work) {
+    *refused = 0;
+    if (int rc = work()) return rc;
     if (!m->inlaunch_timeouts) return 0;
-    const unsigned now = *reinterpret_cast<volatile unsigned*>(m->inlaunch_timeouts);
-    if (now == m->inlaunch_timeouts_seen) return 0;
-    const unsigned n = now - m->inlaunch_timeouts_seen;
+    const bool forced = knobs().inlaunch_give_up && m->chain_ran;
+    const unsigned now = *reinterpret_cast<volatile unsigned*>(m->inlaunch_timeouts), n = now - m->inlaunch_timeouts_seen + forced;
+    if (!n) return 0;
     m->inlaunch_timeouts_seen = now;
     m->em2_failed = true;
     drop_graph(m);
-    fh::set_error("%u in-launch wait(s) of a merged kernel gave up (gate_up → down hand-off): the results of this call are invalid; "
-                  "the two-launch form is used from now on", n);
-    return 3;
+    if (forced)
+        if (int rc = fill_written(m, written(), 0xFFFF)) return rc;
+    if (int rc = fill_written(m, written(), 0)) return rc;
+    if (m->cfg.tp_world > 1) {
+        fh::set_error("%u wait(s) inside a merged launch (decode chain, or gate_up → down) gave up: the results of this call are invalid; separate launches "
+                      "are used from now on", n);
+        *refused = 3;
+        return 0;
+    }
+    fprintf(stderr, "[ferrum_hip] %u wait(s) inside a merged launch gave up: this call is done again in separate launches, which are used from now on\n", n);
+    form_hit(FORM_DONE_AGAIN);
+    return work();
 }
 
 // What does not change from step to step of whether a layer takes the chain launch (chain.hip): the model's kind, the weights' forms and shapes.
@@ -1499,6 +1547,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             chain_mlp |= layer_chains_mlp(li);
         }
     if (!chain_mlp) chain_inter = 0;
+    m->chain_ran = chain_rows;
     if (chain_rows) form_hit(FORM_CHAIN_ROWS);
     // head, one launch: embedding_lookup (+ the Gemma embedding scale, llama_family.rs:3656) → residual stream (fp16; for
     // sandwich-norm models also the fp32 shadow, llama_family.rs:3664-3674) → layer 0's input norm.  Later layers get their
@@ -2095,29 +2144,39 @@ static int forward_batch(FerrumHipModel* m, const FerrumHipBatchItem* items, int
             g.penalties = reinterpret_cast<const float*>(base + off_pen);
         }
     }
-    if (int rc = enqueue_forward(m, sh, greedy != 0, &g)) return rc;
-    // listed places: as many rows per head launch as the logits buffer holds
-    for (int r0 = 0; rows && r0 < num_rows; r0 += c.max_seqs) {
-        const int n = std::min(c.max_seqs, num_rows - r0);
-        if (r0) FH_CHECK_HIP(hipStreamSynchronize(m->stream));          // (the staging half of the index block is in use until then)
-        memcpy(h_samp, rows + r0, (size_t)n * 4);
-        FH_CHECK_HIP(hipMemcpyAsync(m->idx_dev + m->il.sampled_idx, h_samp, (size_t)n * 4, hipMemcpyHostToDevice, m->stream));
-        if (int rc = enqueue_head(m, n)) return rc;
-        FH_CHECK_HIP(hipMemcpyAsync(logits_out + (size_t)r0 * m->vp_n, m->logits, (size_t)n * m->vp_n * 4, hipMemcpyDeviceToHost, m->stream));
-    }
-    if (sh.num_sampled > 0) {
-        if (greedy && out_tokens)
-            FH_CHECK_HIP(hipMemcpyAsync(out_tokens, m->out_tokens, (size_t)sh.num_sampled * 4, hipMemcpyDeviceToHost, m->stream));
-        if (logits_out)
-            FH_CHECK_HIP(hipMemcpyAsync(logits_out, m->logits, (size_t)sh.num_sampled * m->vp_n * 4, hipMemcpyDeviceToHost, m->stream));
-    }
-    FH_CHECK_HIP(hipStreamSynchronize(m->stream));
+    auto written = [&] {
+        std::vector<Written> w;
+        for (int i = 0; i < num_items; i++) w.push_back({items[i].seq_id, items[i].pos_offset, items[i].num_q_tokens});
+        return w;
+    };
+    int refused = 0;
+    if (int rc = attempt(m, &refused, written, [&]() -> int {
+        if (int rc = enqueue_forward(m, sh, greedy != 0, &g)) return rc;
+        // listed places: as many rows per head launch as the logits buffer holds
+        for (int r0 = 0; rows && r0 < num_rows; r0 += c.max_seqs) {
+            const int n = std::min(c.max_seqs, num_rows - r0);
+            if (r0) FH_CHECK_HIP(hipStreamSynchronize(m->stream));          // (the staging half of the index block is in use until then)
+            memcpy(h_samp, rows + r0, (size_t)n * 4);
+            FH_CHECK_HIP(hipMemcpyAsync(m->idx_dev + m->il.sampled_idx, h_samp, (size_t)n * 4, hipMemcpyHostToDevice, m->stream));
+            if (int rc = enqueue_head(m, n)) return rc;
+            FH_CHECK_HIP(hipMemcpyAsync(logits_out + (size_t)r0 * m->vp_n, m->logits, (size_t)n * m->vp_n * 4, hipMemcpyDeviceToHost, m->stream));
+        }
+        if (sh.num_sampled > 0) {
+            if (greedy && out_tokens)
+                FH_CHECK_HIP(hipMemcpyAsync(out_tokens, m->out_tokens, (size_t)sh.num_sampled * 4, hipMemcpyDeviceToHost, m->stream));
+            if (logits_out)
+                FH_CHECK_HIP(hipMemcpyAsync(logits_out, m->logits, (size_t)sh.num_sampled * m->vp_n * 4, hipMemcpyDeviceToHost, m->stream));
+        }
+        FH_CHECK_HIP(hipStreamSynchronize(m->stream));
+        return 0;
+    })) return rc;
     for (int i = 0; i < num_items; i++) {
         SeqState& st = m->seqs[items[i].seq_id];
         st.len += items[i].num_q_tokens;
         st.last_token = items[i].q_tokens[items[i].num_q_tokens - 1];
     }
-    return check_inlaunch_waits(m);
+    const int rc = check_peer_waits(m);
+    return rc ? rc : refused;
 }
 
 int ferrum_hip_model_unified_forward_ex(FerrumHipModel* m, const FerrumHipBatchItem* items, int num_items, int greedy,
@@ -2222,45 +2281,54 @@ int ferrum_hip_model_decode_steps(FerrumHipModel* m, const uint64_t* seq_ids, co
     const bool use_graph = !(c.tp_world > 1 && m->tp_loopback) && !m->taps_enabled && !knobs().no_graph;
     int kv_bucket = cdiv(sh.max_kv_len, 256) * 256;
     sh.max_kv_len = kv_bucket;
-    bool graph_ok = use_graph && !m->graph_refused;
-    if (graph_ok && (!m->graph_exec || m->graph_n != n || m->graph_max_kv != kv_bucket)) {
-        drop_graph(m);
-        FH_CHECK_HIP(hipStreamSynchronize(m->stream));
-        form_hit(FORM_GRAPH_CAPTURE);
-        // (relaxed mode under tensor parallelism: the collective library may touch the allocator inside the capture window)
-        FH_CHECK_HIP(hipStreamBeginCapture(m->stream, c.tp_world > 1 ? hipStreamCaptureModeRelaxed : hipStreamCaptureModeThreadLocal));
-        int rc = enqueue_step();
-        hipError_t e = hipStreamEndCapture(m->stream, &m->graph);
-        if (!rc && e == hipSuccess) e = hipGraphInstantiate(&m->graph_exec, m->graph, nullptr, nullptr, 0);
-        if (rc || e != hipSuccess) {
-            // A step with a collective inside that the runtime will not capture (tensor parallel only): run it eagerly from now
-            // on rather than fail — the capture attempt enqueued nothing, so the device state is untouched.
-            (void)hipGetLastError();
+    auto written = [&] {
+        std::vector<Written> w;
+        for (int i = 0; i < n; i++) w.push_back({seq_ids[i], m->seqs[seq_ids[i]].len, steps});
+        return w;
+    };
+    int refused = 0;
+    if (int rc = attempt(m, &refused, written, [&]() -> int {
+        bool graph_ok = use_graph && !m->graph_refused;
+        if (graph_ok && (!m->graph_exec || m->graph_n != n || m->graph_max_kv != kv_bucket)) {
             drop_graph(m);
-            if (c.tp_world <= 1) {
-                if (rc) return rc;
-                FH_CHECK_HIP(e);
+            FH_CHECK_HIP(hipStreamSynchronize(m->stream));
+            form_hit(FORM_GRAPH_CAPTURE);
+            // (relaxed mode under tensor parallelism: the collective library may touch the allocator inside the capture window)
+            FH_CHECK_HIP(hipStreamBeginCapture(m->stream, c.tp_world > 1 ? hipStreamCaptureModeRelaxed : hipStreamCaptureModeThreadLocal));
+            int rc = enqueue_step();
+            hipError_t e = hipStreamEndCapture(m->stream, &m->graph);
+            if (!rc && e == hipSuccess) e = hipGraphInstantiate(&m->graph_exec, m->graph, nullptr, nullptr, 0);
+            if (rc || e != hipSuccess) {
+                // A step with a collective inside that the runtime will not capture (tensor parallel only): run it eagerly from now
+                // on rather than fail — the capture attempt enqueued nothing, so the device state is untouched.
+                (void)hipGetLastError();
+                drop_graph(m);
+                if (c.tp_world <= 1) {
+                    if (rc) return rc;
+                    FH_CHECK_HIP(e);
+                }
+                fprintf(stderr, "[ferrum_hip] decode step could not be captured under tensor parallelism (%s): eager launches from here on\n",
+                        rc ? fh::last_error() : hipGetErrorString(e));
+                m->graph_refused = true;
+                graph_ok = false;
+            } else {
+                m->graph_n = n;
+                m->graph_max_kv = kv_bucket;
             }
-            fprintf(stderr, "[ferrum_hip] decode step could not be captured under tensor parallelism (%s): eager launches from here on\n",
-                    rc ? fh::last_error() : hipGetErrorString(e));
-            m->graph_refused = true;
-            graph_ok = false;
-        } else {
-            m->graph_n = n;
-            m->graph_max_kv = kv_bucket;
         }
-    }
-    const int most = *std::max_element(parts.words, parts.words + parts.n);
-    hipLaunchKernelGGL(decode_begin_kernel, dim3(cdiv(most, BEGIN_WORDS), parts.n), dim3(256), 0, m->stream, reinterpret_cast<const uint32_t*>(m->idx_host),
-                       reinterpret_cast<uint32_t*>(m->idx_dev), parts, m->step_counter);
-    FH_CHECK_LAUNCH();
-    if (graph_ok) {
-        for (int st = 0; st < steps; st++) { FH_CHECK_HIP(hipGraphLaunch(m->graph_exec, m->stream)); form_hit(FORM_GRAPH_REPLAY); }
-    } else {
-        for (int st = 0; st < steps; st++)
-            if (int rc = enqueue_step()) return rc;
-    }
-    FH_CHECK_HIP(hipStreamSynchronize(m->stream));
+        const int most = *std::max_element(parts.words, parts.words + parts.n);
+        hipLaunchKernelGGL(decode_begin_kernel, dim3(cdiv(most, BEGIN_WORDS), parts.n), dim3(256), 0, m->stream, reinterpret_cast<const uint32_t*>(m->idx_host),
+                           reinterpret_cast<uint32_t*>(m->idx_dev), parts, m->step_counter);
+        FH_CHECK_LAUNCH();
+        if (graph_ok) {
+            for (int st = 0; st < steps; st++) { FH_CHECK_HIP(hipGraphLaunch(m->graph_exec, m->stream)); form_hit(FORM_GRAPH_REPLAY); }
+        } else {
+            for (int st = 0; st < steps; st++)
+                if (int rc = enqueue_step()) return rc;
+        }
+        FH_CHECK_HIP(hipStreamSynchronize(m->stream));
+        return 0;
+    })) return rc;
     if (out_tokens) memcpy(out_tokens, m->history, (size_t)steps * n * 4);
     // the last token each sequence was FED: the one sampled a step before the last
     const uint32_t* fed = steps > 1 ? m->history + (size_t)(steps - 2) * n : first_tokens;
@@ -2268,7 +2336,8 @@ int ferrum_hip_model_decode_steps(FerrumHipModel* m, const uint64_t* seq_ids, co
         m->seqs[seq_ids[i]].len += steps;
         m->seqs[seq_ids[i]].last_token = fed[i];
     }
-    return check_inlaunch_waits(m);
+    const int rc = check_peer_waits(m);
+    return rc ? rc : refused;
 }
 
 // Bench instrumentation: average device time of ONE launch of a hot kernel, measured with HIP events

@@ -1065,6 +1065,49 @@ def test_decode_chain_of_wide_layers(pkg, c, forms):
     par.finish(max_mismatches=1, max_route_ties=0)
 
 
+@pytest.mark.parametrize("first", ["forward", "steps"])
+@pytest.mark.parametrize("kind,c", [("moe", 1), ("moe", 5), ("moe", 33), ("int4", 3), ("int4", 17), ("f16", 8), ("f16", 33)])
+def test_calls_whose_waits_give_up_are_done_again(pkg, kind, c, first, forms, knobs):
+    """A call whose waits inside the chain count as given up (from the host: none of them really does) is done again in separate launches and returns what those
+    return, bit for bit, and so do the calls after it, of these sequences and of others on their blocks (what the first attempt left in the caches is NaN)."""
+    from tests import modelgen
+    if kind == "moe":
+        tm = _chain_model()
+    else:
+        key = ("again", kind)
+        if key not in _CHAIN_TM:
+            kw = dict(dense_proj=True, tied=True) if kind == "f16" else {}
+            _CHAIN_TM[key] = modelgen.TinyModel(False, layers=3, hidden=2048 if kind == "int4" else 1024, nq=32 if kind == "int4" else 16, nkv=4, hd=128, inter=2048,
+                                                vocab=2048, seed=107, max_seq_len=64, qk_norm=True, **kw)
+        tm = _CHAIN_TM[key]
+
+    def drive():
+        hm = tm.hip_model(pkg, kv_num_blocks=c + 1, max_seqs=c, max_tokens=max(3 * c, 64))
+        out, at = [], 3
+        start = lambda: hm.unified_forward([(i, [7 + i, 300, 21], 0, True) for i in range(c)], greedy=True, want_logits=True)[1]
+        step = lambda at: hm.unified_forward([(i, [50 + i + at], at, True) for i in range(c)], greedy=True, want_logits=True)[1]
+        out.append(start())
+        if first == "forward":
+            out.append(step(at))
+            at += 1
+        out.append(np.array(hm.decode_steps(list(range(c)), [60 + i for i in range(c)], 4)))
+        out.append(step(at + 4))
+        for i in range(c): hm.release(i)
+        out.append(start())
+        out.append(step(3))
+        return out
+
+    knobs.set(DECODE_CHAIN=0, MOE_EM2=0)
+    want = drive()
+    assert all(np.isfinite(w).all() for w in want)
+    knobs.set(DECODE_CHAIN=1, MOE_EM2=1, INLAUNCH_GIVE_UP=1)
+    forms.reset()
+    got = drive()
+    h = forms.hits()
+    assert h.get("done_again") == 1 and h.get("decode_chain") == 3, h
+    for a, b in zip(got, want): assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("kind,c,chain,rows", [
     ("moe", 1, 1, 1), ("moe", 1, 0, 0), ("int4", 1, 1, 1), ("int4", 64, 1, 1), ("int4", 65, 1, 0), ("int4", 1, 0, 0),
     ("narrow", 1, 1, 0), ("f16", 64, 1, 1), ("f16", 65, 1, 0)])
