@@ -53,7 +53,7 @@ void reload_knobs() {
     k.chain_attn_splits = env_int("FERRUM_HIP_CHAIN_ATTN_SPLITS", 0);
     k.route_gemm_topk = env_int("FERRUM_HIP_ROUTE_GEMM_TOPK", 1);
     k.tiled_big_min_tiles = env_int("FERRUM_HIP_TILED_BIG_MIN_TILES", -1);
-    k.tiled_wide_min_tiles = env_int("FERRUM_HIP_TILED_WIDE_MIN_TILES", TILED_WIDE_MIN_TILES);
+    k.tiled_wide_min_tiles = env_int("FERRUM_HIP_TILED_WIDE_MIN_TILES", -1);
     k.tiled_256 = env_int("FERRUM_HIP_TILED_256", 0);
     k.tiled_min_tiles = env_int("FERRUM_HIP_TILED_MIN_TILES", 128);
     k.tiled_half_max_tiles = env_int("FERRUM_HIP_TILED_HALF_MAX_TILES", 256);
@@ -112,7 +112,7 @@ static const char* const g_form_names[FORM_COUNT] = {
     "perm_producer", "moe_expert_major_pair", "decode_chain", "moe_deferred_merge", "dense_chain", "tp_allreduce_norm_fused", "moe_block_major_pair", "chain_attn_kv_splits", "chain_qkv_wide", "route_gemm_topk",
     "tiled_gemm", "tiled_gemm_big", "tiled_gemm_128x256", "tiled_gemm_128x128", "tiled_gemm_128x64", "tiled_gemm_64x64", "tiled_gemm_grouped", "tiled_gemm_grouped_big", "moe_route_sort", "latent_attn_plain", "latent_attn", "latent_attn_pair", "latent_attn_split", "latent_attn_expanded", "rglru_step", "rglru_scan",
     "grouped_attn_plain", "grouped_attn_keys", "grouped_attn_split", "grouped_attn_tile", "linear_step", "linear_chunk", "scan_step", "scan_chunk", "route_grouped",
-    "route_softmax", "talk_attn_plain", "talk_attn_keys", "talk_attn_tile", "talk_attn_tile_split", "w4_rows", "w4_gated", "f16_gated", "tiled_gemm_cols64", "tiled_gemm_256x256", "chain_mlp", "chain_rows", "done_again"};
+    "route_softmax", "talk_attn_plain", "talk_attn_keys", "talk_attn_tile", "talk_attn_tile_split", "w4_rows", "w4_gated", "f16_gated", "tiled_gemm_cols64", "tiled_gemm_256x256", "chain_mlp", "chain_rows", "moe_rows_256", "done_again"};
 const char* form_name(int f) { return f >= 0 && f < FORM_COUNT ? g_form_names[f] : nullptr; }
 }  // namespace fh
 

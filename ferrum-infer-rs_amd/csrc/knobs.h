@@ -13,7 +13,6 @@
 
 namespace fh {
 
-constexpr int TILED_WIDE_MIN_TILES = 257;
 struct Knobs {
     // paged attention (attention.hip)
     bool attn_no_flash = false;
@@ -61,7 +60,7 @@ struct Knobs {
     int lds_min_groups = 8;
     // layered models (tiled_gemm.hip, latent_attention.hip, grouped_attention.hip, linear_attention.hip, rglru.hip)
     int tiled_big_min_tiles = -1;     // ≥ 0: projections of > 64 rows take the tile kernel from this many tiles of 64 × 64 (32-bit: and one); −1: from 193, in 32 bits 129
-    int tiled_wide_min_tiles = TILED_WIDE_MIN_TILES;   // … and in 16 bits its 128 × 256 form from this many tiles of that size
+    int tiled_wide_min_tiles = -1;    // ≥ 0: … and in 16 bits its 128 × 256 form from this many tiles of that size, and no larger one; −1: from 257
     int tiled_256 = 0;                // … 256 × 256: 1 wherever they can, 0 where they take less, −1 never
     int tiled_min_tiles = 128;        // few-row kernel: rows of a workgroup are halved until there are this many row × 16-column tiles (16-bit: up to twice as many)
     int tiled_half_max_tiles = 256;   // … its 128 × 64 and 64 × 64 forms up to this many tiles of 128 × 128
@@ -171,6 +170,7 @@ enum Form : int {
     FORM_TILED_GEMM_256X256,    // prompts: tiles of 256 × 256, a workgroup's one after the other (tiled_gemm_wide.hip)
     FORM_CHAIN_MLP,             // decode chain: the MLP of a dense layer in the launch too
     FORM_CHAIN_ROWS,            // decode chain: a forward's head made its rows ready
+    FORM_MOE_ROWS_256,          // layered experts: sorted rows in blocks of 256
     FORM_DONE_AGAIN,            // a call whose in-launch waits gave up was done again in separate launches
     FORM_COUNT
 };

@@ -583,10 +583,22 @@ private:
         TiledGemm<E> z = linear_f32(L.router, xb_, Dp_, T, router_logits_, routed);
         z.n_store = routed; z.nsec = 1; z.sec[0] = {0, GEMM_ACT_NONE, 0, 0, L.g2};
         RUN(tiled_gemm(z, s));
-        GemmRows rows;
-        rows.block = moe_block(pairs, E_, L.up.k % 128 == 0 && L.down.k % 128 == 0);
-        rows.max_blocks = std::min(pairs, pairs / rows.block + std::min(E_, pairs));
-        rows.id = sorted_; rows.group = sorted_expert_; rows.total = sorted_total_;
+        auto sorted_rows = [&](int block, int div) {
+            GemmRows r;
+            r.block = block;
+            r.max_blocks = std::min(pairs, pairs / block + std::min(E_, pairs));
+            r.id = sorted_; r.group = sorted_expert_; r.total = sorted_total_;
+            r.div = div;
+            return r;
+        };
+        TiledGemm<E> u = linear(L.up, xb_, Dp_, pairs, expert_h_, L.down.k), y = linear(L.down, expert_h_, L.down.k, pairs, expert_y_, Dp_);
+        u.groups = y.groups = 1;
+        u.nsec = 1; u.sec[0] = L.ff_sec[0];
+        u.rows = sorted_rows(256, L.s.top); y.rows = sorted_rows(256, 1);
+        const GemmRows rows = sorted_rows(moe_block(pairs, E_, tiled_gemm_takes_256(u) || tiled_gemm_takes_256(y)), 1);
+        u.rows = y.rows = rows;
+        u.rows.div = L.s.top;
+        if (rows.block == 256) form_hit(FORM_MOE_ROWS_256);
         const bool corrected = L.s.ff != FERRUM_HIP_FF_MOE_RELU2;
         const MoeCorrectedRule rule = route_rule(L.s, L.correction);
         if (moe_route_sort_supports(T, routed, L.s.top)) {
@@ -598,18 +610,16 @@ private:
             RUN(moe_route_topk_softmax_f32(router_logits_, expert_ids_, expert_weights_, T, E_, L.s.top, 1, s));
             RUN(moe_align_block_size(expert_ids_, sorted_, sorted_expert_, sorted_total_, pairs, E_, rows.block, rows.max_blocks * rows.block, s));
         }
-        TiledGemm<E> u = linear(L.up, xb_, Dp_, pairs, expert_h_, L.down.k);
-        u.groups = 1; u.rows = rows; u.rows.div = L.s.top;
-        u.nsec = 1; u.sec[0] = L.ff_sec[0];
         RUN(tiled_gemm(u, s));
-        TiledGemm<E> y = linear(L.down, expert_h_, L.down.k, pairs, expert_y_, Dp_);
-        y.groups = 1; y.rows = rows;
         RUN(tiled_gemm(y, s));
         return 0;
     }
     // rows per block of the sorted list: a large block shares an expert's weights between more rows, a small one pads less
-    // (256: for the tiles of that many rows, which save 6 % of a long launch, where the half of a block more that an expert leaves empty is a small part of its rows:
-    // 32 × 256 tokens, 8 of 24 experts, 2731 rows each: prompt 9.87 → 9.46 ms; 4002 tokens, 1067 each: 2.13 → 2.16)
+    // (256: where one of the two projections takes tiles of that many rows, from 2048 rows a mean expert, where the half of a block more that an expert leaves empty is a
+    // small part of them. Whole prompts of 1.3 – 17 ms, time against blocks of 128 by the mean expert's rows:
+    //   24 experts, 8 chosen, widths of 1024: 1100 1.06 | 0.99, 1400 0.96 | 1.00, 1700 0.99 | 0.98, 1900 1.01 | 1.00, 2200 0.97 | 1.01, 2700 0.96 | 0.99, 4000 0.98 | 1.00
+    //   (two families); of 2048: 1100 1.00, 1900 0.96, 2700 0.97, 4000 0.95; 8 experts, 2 chosen, of 3072: 1100 1.04, 1900 0.99, 2200 0.98, 4000 0.98; 64, 8 of 1024:
+    //   1100 1.01, 1900 0.99, 2400 0.97; of 256 and 512, where neither takes them: 0.99 – 1.01)
     static int moe_block(int pairs, int experts, bool tiles256) {
         const int mean = pairs / experts, forced = knobs().moe_rows_block;
         if (forced > 0 && (sizeof(E) == 2 || forced <= 64)) return forced;

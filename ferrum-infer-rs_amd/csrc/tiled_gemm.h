@@ -94,6 +94,8 @@ struct TiledGemm {
     int pair = 0;                         // > 0, one gated section: column tile t is weight tile t / 2 + (t odd ? pair : 0)
 };
 template <typename E> int tiled_gemm(const TiledGemm<E>& g, hipStream_t s);
+// whether a launch of many rows runs in tiles of 256 × 256, which want blocks of 256 sorted rows
+template <typename E> bool tiled_gemm_takes_256(const TiledGemm<E>& g);
 // number of K parts worth making for a projection of m rows whose consumer sums slabs (≤ GEMM_MAX_SLABS)
 constexpr int GEMM_MAX_SLABS = 4;
 int tiled_gemm_slabs(int m, int n, int k);

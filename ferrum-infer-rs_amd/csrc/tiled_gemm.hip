@@ -555,9 +555,24 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
 //   4096 × 4096 × 4096   112 (2) | 98.8 (1)     4096 × 10240 × 2048   148 (5) | 146 (3)      7000 × 8192 × 1024   109 (7) | 111 (4)
 //   3000 × 8192 × 4096   164 (3) | 173 (2)      4096 × 6144 × 1024    57 (3) | 67 (2)        5000 × 3072 × 512    22.9 (2) | 23.4 (1)
 // so wherever its rounds are half as many as the other's, but for short K.
+static long big_tiles(const GemmRows& rows, int m, int n, int groups, int r, int c) { return (long)(rows.id ? rows.max_blocks * (rows.block / r) : cdiv(m, r)) * cdiv(n, c) * groups; }
+template <typename E>
+bool tiled_gemm_takes_256(const TiledGemm<E>& g) {
+    if constexpr (sizeof(E) == 4) {
+        return false;
+    } else {
+        if (knobs().tiled_256 < 0 || (g.rows.id && g.rows.block % 256)) return false;
+        if (knobs().tiled_256 == 0) {
+            if (knobs().tiled_wide_min_tiles >= 0) return false;        // (a forced size of the tiles below stays what it is)
+            const long halves = cdiv(big_tiles(g.rows, g.m, g.n, g.groups, 128, 256), 256), rounds = cdiv(big_tiles(g.rows, g.m, g.n, g.groups, 256, 256), 256);
+            if (halves <= 1 || rounds * (11.6f + 0.0201f * g.k) >= (g.k > 512 ? 0.97f : 0.93f) * halves * (5.5f + 0.01185f * g.k)) return false;
+        }
+        return tiled_gemm_wide_supports(g);
+    }
+}
 template <typename E>
 static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
-    auto tiles = [&](int r, int c) { return (long)(g.rows.id ? g.rows.max_blocks * (g.rows.block / r) : cdiv(g.m, r)) * cdiv(g.n, c) * g.groups; };
+    auto tiles = [&](int r, int c) { return big_tiles(g.rows, g.m, g.n, g.groups, r, c); };
     if constexpr (sizeof(E) == 4) {
         // 32 bits: bound by the products alone, so the tile whose rounds over the CUs take least (µs of a round below, K = 2048):
         //                        128 × 128   128 × 64   64 × 64   few-row kernel
@@ -573,12 +588,8 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
         if ((g.rows.id && g.rows.block < 128) || small < std::min(full, half)) return launch_big<E, 2, 2, 3, 3>(g, s);
         return half < full ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 4, 4, 2, 2>(g, s);
     } else {
-        // (a forced size of the tiles above stays what it is)
-        const long halves = cdiv(tiles(128, 256), 256), rounds = cdiv(tiles(256, 256), 256);
-        const bool fits = knobs().tiled_wide_min_tiles == TILED_WIDE_MIN_TILES && halves > 1 && (!g.rows.id || g.rows.block % 256 == 0)
-                          && rounds * (11.6f + 0.0201f * g.k) < (g.k > 512 ? 0.97f : 0.93f) * halves * (5.5f + 0.01185f * g.k);
-        if ((knobs().tiled_256 > 0 || (knobs().tiled_256 == 0 && fits)) && tiled_gemm_wide_supports(g)) return tiled_gemm_wide(g, s);
-        if (tiles(128, 256) >= knobs().tiled_wide_min_tiles) return launch_big<E, 4, 8, 2, 2>(g, s);
+        if (tiled_gemm_takes_256(g)) return tiled_gemm_wide(g, s);
+        if (tiles(128, 256) >= (knobs().tiled_wide_min_tiles >= 0 ? knobs().tiled_wide_min_tiles : 257)) return launch_big<E, 4, 8, 2, 2>(g, s);
         if (tiles(128, 128) > knobs().tiled_half_max_tiles) return launch_big<E, 4, 4, 2, 2>(g, s);
         return tiles(64, 64) > knobs().tiled_small_max_tiles ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 2, 2, 3, 3>(g, s);
     }
@@ -744,6 +755,8 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     return J == 1 ? SMALL(1, false) : SMALL(2, false);
 #undef SMALL
 }
+template bool tiled_gemm_takes_256<bf16>(const TiledGemm<bf16>&);
+template bool tiled_gemm_takes_256<float>(const TiledGemm<float>&);
 template int tiled_gemm<bf16>(const TiledGemm<bf16>&, hipStream_t);
 template int tiled_gemm<float>(const TiledGemm<float>&, hipStream_t);
 template int tiled_gemm<_Float16>(const TiledGemm<_Float16>&, hipStream_t);

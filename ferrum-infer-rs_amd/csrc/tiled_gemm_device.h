@@ -53,7 +53,7 @@ __device__ __forceinline__ GemmSection gemm_section(const TiledGemm<E>& p, int c
     return s;
 }
 
-// tiles of 256 × 256 (tiled_gemm_wide.hip): whether a launch has the form, and the launch
+// tiles of 256 × 256 (tiled_gemm_wide.hip): whether a launch can have the form (tiled_gemm.h: whether it takes it), and the launch
 template <typename E> bool tiled_gemm_wide_supports(const TiledGemm<E>& g);
 template <typename E> int tiled_gemm_wide(const TiledGemm<E>& g, hipStream_t s);
 

@@ -545,6 +545,26 @@ def test_projections_in_tiles_of_256_x_256(pkg, tmp_path, knobs, forms, name):
     assert h.get("tiled_gemm_256x256") and bool(h.get("tiled_gemm_grouped_big")) == (name != "nerenex")
 
 
+@pytest.mark.parametrize("ff,n,forced,taken", [(2048, 32, None, 1), (2048, 31, None, 0), (256, 32, None, 0), (2048, 32, 257, 0)])
+def test_blocks_of_256_sorted_rows(pkg, tmp_path, knobs, forms, ff, n, forced, taken):
+    """Two experts of which each token takes one: blocks of 256 rows from a mean of 2048 (128 tokens a sequence, and one more), where one of the two projections runs in
+    tiles of as many rows (2048 columns of K 1024), not where neither does (256 columns, K of 256) or another size is asked for; against blocks of 128."""
+    cfg = G.safolorn(1024, 260, 40, [G.sink_attention(4, 64, 32, 32, 256, 1e5, G.LONG, mlp=G.experts(2, 1, ff))])
+    path = G.write_checkpoint(tmp_path, cfg, G.weights(cfg, 33))
+    items = [(i, toks(cfg, 129, i), 0) for i in range(n)]
+    at = [129 * i + j for i in range(n) for j in (0, 64, 128)]
+    out = {}
+    for block in (None, 128):
+        knobs.set(TILED_WIDE_MIN_TILES=forced, MOE_ROWS_BLOCK=block)
+        m = load(pkg, path, "bfloat16", tokens=129 * n, seqs=n, blocks=9 * n + 2, max_len=256)
+        forms.reset()
+        out[block] = m.forward_rows(items, at)
+        if block is None:
+            assert forms.hits().get("moe_rows_256", 0) == taken, forms.hits()
+        del m
+    assert rel(out[None], out[128]) < 4e-3        # (both sum K in steps of 32 in fp32: equal but for the order, 16-bit results of one layer)
+
+
 @pytest.mark.parametrize("name", ["wide", "shared", "sinks", "loop", "talks"])
 @pytest.mark.parametrize("big", [1, 10 ** 6])
 def test_32_bit_projections_of_prompts(pkg, cases, knobs, forms, name, big):

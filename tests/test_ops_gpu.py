@@ -490,6 +490,16 @@ def test_tiles_of_256_x_256(env, m, n, k, f32, knobs, forms):
     forms.require("tiled_gemm_256x256")
 
 
+@pytest.mark.parametrize("n,forced,taken", [(8192, None, True), (8224, None, False), (8192, 257, False), (8192, 256, False), (8192, -1, True)])
+def test_rule_of_tiles_of_256_x_256(env, n, forced, taken, knobs, forms):
+    """2001 rows, K of 1024: one round of them where two of 128 x 256 fill the card, two where three do; a number of the latter asked for, their own line's among
+    them, is what runs."""
+    knobs.set(TILED_WIDE_MIN_TILES=forced)
+    _few_rows(env, 2001, n, 1024)
+    hits = forms.hits()
+    assert bool(hits.get("tiled_gemm_256x256")) == taken and bool(hits.get("tiled_gemm_128x256")) != taken, hits
+
+
 @pytest.mark.parametrize("tiles,form", [(0, "tiled_gemm_big"), (2, "tiled_gemm_big"), (3, "tiled_gemm"), (None, "tiled_gemm")])
 def test_tile_kernel_from_a_given_number_of_tiles(env, tiles, form, knobs, forms):
     """Two tiles of 64 x 64: a number asked for, 0 among them, or the rule."""
