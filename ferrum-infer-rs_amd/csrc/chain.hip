@@ -36,6 +36,7 @@
 // paged_attn_kernel<128, true, 8> (fused QK-norm / RoPE / KV write, 8 KV-splitting waves merged in wave order),
 // add_rmsnorm_route_part_kernel (Q expert parts per token, in-launch ticket merge) — so the results are the same bits.
 #include "common.h"
+#include "handed_off.h"
 #include "kernels.h"
 #include "knobs.h"
 #include "kv_layout.h"
@@ -50,7 +51,6 @@ namespace {
 
 constexpr int CH_W = 8;                 // waves per workgroup
 constexpr int CH_MAX_KVH = 16;
-constexpr uint32_t NOT_YET = ~0u;        // a word of a handed-off row that has not been written
 constexpr int CH_GRAN = 10;              // granules per (token, router part): 8 candidates + max + Σexp
 constexpr int CH_O_KS = 2;                // o_proj: K parts per block, each a workgroup of its own (fp32 partial rows, role B adds them)
 constexpr int CH_MAX_SPLITS = 16;          // KV ranges per (sequence, kv head) in the attention role
@@ -149,11 +149,6 @@ __device__ __forceinline__ void chain_landed() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_sched_barrier(0);
 }
-// Numbers that are handed off: the one fp16, and fp32, NaN that reads as NOT_YET loses its sign.
-__device__ __forceinline__ uint32_t written2(uint32_t w) {
-    if ((w & 0xFFFFu) == 0xFFFFu) w ^= 0x8000u;
-    return w >= 0xFFFF0000u ? w ^ 0x80000000u : w;
-}
 __device__ __forceinline__ void store16_sc1(__amdgpu_buffer_rsrc_t r, int byte_off, half8 v) {
     u32x4 w = __builtin_bit_cast(u32x4, v);
 #pragma unroll
@@ -163,7 +158,7 @@ __device__ __forceinline__ void store16_sc1(__amdgpu_buffer_rsrc_t r, int byte_o
 __device__ __forceinline__ void store16_sc1(__amdgpu_buffer_rsrc_t r, int byte_off, float4v v) {
     u32x4 w = __builtin_bit_cast(u32x4, v);
 #pragma unroll
-    for (int i = 0; i < 4; i++) w[i] = w[i] == NOT_YET ? w[i] ^ 0x80000000u : w[i];
+    for (int i = 0; i < 4; i++) w[i] = written1(w[i]);
     __builtin_amdgcn_raw_buffer_store_b128(w, r, byte_off, 0, 16);
 }
 

@@ -30,7 +30,7 @@ struct Knobs {
     // INT4 GEMMs (w4_gemm.hip)
     int moe_kw_pairs = 16;
     int decode_chain = 1;             // MoE decode at ≤ 32 rows: tail + q|k|v + attention + o_proj + route as ONE launch (0 = five launches)
-    int inlaunch_give_up = 0;         // tests: 1 = a forward with chain launches counts as one whose waits gave up, with NaN where it wrote K and V
+    int inlaunch_give_up = 0;         // tests: 1 = a forward with chain launches counts as one whose waits gave up, with NaN where it wrote K and V; −1 = a call whose waits give up fails
     int chain_max_rows = 128;         // decode chain up to this many rows (≤ 128)
     int sandwich_wide = 1;            // sandwich add + norms of ≤ 64 rows: 1024 threads per row, loads ahead of the reductions (0 = 256 threads)
     int chain_qkv_half = 1;           // decode chain at ≤ 16 rows: q|k|v in 32-column blocks (0 = 64)

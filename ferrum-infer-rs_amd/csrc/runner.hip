@@ -348,7 +348,7 @@ static int attempt(FerrumHipModel* m, int* refused, const W& written, const F& w
     *refused = 0;
     if (int rc = work()) return rc;
     if (!m->inlaunch_timeouts) return 0;
-    const bool forced = knobs().inlaunch_give_up && m->chain_ran;
+    const bool forced = knobs().inlaunch_give_up > 0 && m->chain_ran;
     const unsigned now = *reinterpret_cast<volatile unsigned*>(m->inlaunch_timeouts), n = now - m->inlaunch_timeouts_seen + forced;
     if (!n) return 0;
     m->inlaunch_timeouts_seen = now;
@@ -357,7 +357,7 @@ static int attempt(FerrumHipModel* m, int* refused, const W& written, const F& w
     if (forced)
         if (int rc = fill_written(m, written(), 0xFFFF)) return rc;
     if (int rc = fill_written(m, written(), 0)) return rc;
-    if (m->cfg.tp_world > 1) {
+    if (m->cfg.tp_world > 1 || knobs().inlaunch_give_up < 0) {
         fh::set_error("%u wait(s) inside a merged launch (decode chain, or gate_up → down) gave up: the results of this call are invalid; separate launches "
                       "are used from now on", n);
         *refused = 3;

@@ -969,8 +969,9 @@ def test_decode_chain_of_a_router_with_nan(pkg, c, bits, forms, knobs):
 @pytest.mark.parametrize("bits", [0xffff, 0x7fff, 0x7c00])
 @pytest.mark.parametrize("c", [1, 5, 17])
 def test_decode_chain_hands_off_every_number(pkg, c, bits, forms, knobs):
-    """Rows handed off inside the launch are their own flags, all ones while unwritten: numbers of that pattern (a norm's weights of NaN, in both halves
-    of a word, in one and across two) arrive as NaN too, and infinities as they are; no wait gives up (the call would fail)."""
+    """Rows handed off inside the launch are their own flags, all ones while unwritten: with numbers of that pattern in every norm1 row (a norm's weights of NaN, in both
+    halves of a word, in one and across two), other NaN and infinities no wait gives up (the call would fail), and nothing but NaN comes out, as of the separate
+    launches.  (What becomes of single words: test_kernel_sources.py.)"""
     tm = _chain_model()
     L = tm.layers[1]["dense"]
     kept = L["input_ln"]
@@ -989,6 +990,44 @@ def test_decode_chain_hands_off_every_number(pkg, c, bits, forms, knobs):
     finally:
         L["input_ln"] = kept
     assert np.isnan(out[0]).all() and np.isnan(out[1]).all()
+
+
+@pytest.mark.parametrize("bits", [0xffff, 0x7fff, 0x7c00, 0xfc00])
+@pytest.mark.parametrize("kind,c", [("moe", 5), ("moe", 17), ("int4", 6), ("f16", 6), ("f16", 17)])
+def test_decode_chain_keeps_special_numbers_to_their_rows(pkg, kind, c, bits, forms, knobs):
+    """Two sequences of a batch are fed a token whose embedding holds NaN, all ones among them, or infinities: their logits are no numbers where the separate launches'
+    are none, and the rows beside them, in the same blocks of 16, are what those make of them."""
+    from tests import modelgen
+    if kind == "moe":
+        tm = _chain_model()
+    else:
+        key = ("again", kind)
+        if key not in _CHAIN_TM:
+            kw = dict(dense_proj=True, tied=True) if kind == "f16" else {}
+            _CHAIN_TM[key] = modelgen.TinyModel(False, layers=3, hidden=2048 if kind == "int4" else 1024, nq=32 if kind == "int4" else 16, nkv=4, hd=128, inter=2048,
+                                                vocab=2048, seed=107, max_seq_len=64, qk_norm=True, **kw)
+        tm = _CHAIN_TM[key]
+    kept, bad = tm.glob, [1, c - 1]
+    try:
+        tm.glob = {k: v.copy() for k, v in kept.items()}
+        if "lm_head" not in tm.glob: tm.glob["lm_head"] = kept["embed"]                # (a tied head would meet the token's row in every sequence)
+        tm.glob["embed"][40, [6, 7, 12, 19, 20]] = np.array([bits], np.uint16).view(np.float16).astype(np.float32)
+        out = {}
+        for chain in (1, 0):
+            knobs.set(DECODE_CHAIN=chain, MOE_EM2=chain)
+            hm = tm.hip_model(pkg, kv_num_blocks=c * 2 + 4, max_seqs=c, max_tokens=64)
+            hm.unified_forward([(i, [7 + i, 300, 21], 0, True) for i in range(c)], greedy=True)
+            forms.reset()
+            out[chain] = [hm.unified_forward([(i, [40 if i in bad and s == 0 else 50 + i + s], 3 + s, True) for i in range(c)], greedy=True, want_logits=True)[1]
+                          for s in range(2)]
+            assert forms.hits().get("decode_chain", 0) == (6 if chain else 0), forms.hits()
+            del hm
+    finally:
+        tm.glob = kept
+    good = [i for i in range(c) if i not in bad]
+    for mine, other in zip(out[1], out[0]):
+        assert np.array_equal(np.isnan(mine), np.isnan(other)) and np.isnan(mine[bad]).all() and np.isfinite(mine[good]).all()
+        assert np.abs(mine[good] - other[good]).max() < 0.02 * np.abs(other[good]).max()
 
 
 @pytest.mark.parametrize("window", [0, 300])
@@ -1230,10 +1269,43 @@ def test_decode_chain_with_the_mlp(pkg, f16, hidden, inter, activation, c, forms
         tm.layers[1]["dense"]["post_ln"] = kept
 
 
+@pytest.mark.parametrize("f16,hidden,nkv,c,splits,mlp_rows", [
+    (0, 2048, 4, 1, 5, 32), (0, 2048, 4, 9, 3, 32), (0, 4096, 8, 1, 16, 32), (0, 4096, 8, 9, 2, 32), (0, 2048, 4, 3, 5, 0), (0, 4096, 8, 17, 3, 32),
+    (1, 1024, 8, 2, 5, 32), (1, 1024, 8, 17, 3, 32), (1, 1024, 8, 17, 3, 0), (1, 2048, 4, 9, 5, 32), (1, 2048, 4, 20, 3, 32),
+    (0, 2048, 4, 1, 0, 32), (0, 4096, 8, 9, 0, 32), (1, 1024, 8, 9, 0, 32)])
+def test_dense_decode_chain_with_kv_ranges(pkg, f16, hidden, nkv, c, splits, mlp_rows, forms, knobs):
+    """Dense layers whose attention role takes several KV ranges, with the MLP's roles behind it and without: forced ranges over short contexts, some of them empty, and the
+    ranges that contexts of more than 512 keys take by themselves; against the launches of their own."""
+    from tests import modelgen
+    keys = 600 if splits == 0 else 40
+    key = ("ranges", f16, hidden)
+    if key not in _CHAIN_TM:
+        kw = dict(dense_proj=True, tied=True) if f16 else {}
+        _CHAIN_TM[key] = modelgen.TinyModel(False, layers=2, hidden=hidden, nq=16 if f16 and hidden == 1024 else 32, nkv=nkv, hd=128, inter=2048, vocab=1024, seed=109,
+                                            max_seq_len=640, qk_norm=True, **kw)
+    tm = _CHAIN_TM[key]
+    lens = [keys - (i * 7) % 31 for i in range(c)]
+    rng = np.random.default_rng(113)
+    prompts = [rng.integers(0, 1024, size=n).astype(np.uint32) for n in lens]
+    mlp = mlp_rows > 0 and c <= (32 if f16 and hidden == 1024 else 16)
+    out = {}
+    for chain in (1, 0):
+        knobs.set(DECODE_CHAIN=chain, CHAIN_ATTN_SPLITS=splits or None, CHAIN_MLP_ROWS=mlp_rows)
+        hm = tm.hip_model(pkg, kv_num_blocks=sum(n // 16 + 2 for n in lens), max_seqs=c, max_tokens=640)
+        for i, p in enumerate(prompts): hm.unified_forward([(i, p, 0, True)], greedy=True)
+        forms.reset()
+        out[chain] = [hm.unified_forward([(i, [50 + i + s], n + s, True) for i, n in enumerate(lens)], greedy=True, want_logits=True)[1] for s in range(2)]
+        h, launches = forms.hits(), 4 if chain else 0
+        assert h.get("dense_chain", 0) == launches and h.get("chain_attn_kv_splits", 0) == launches and h.get("chain_mlp", 0) == (launches if mlp else 0), h
+        del hm
+    for mine, other in zip(out[1], out[0]):
+        assert np.abs(mine - other).max() < 0.02 * np.abs(other).max()
+
+
 @pytest.mark.parametrize("kind,c", [("moe", 5), ("int4", 5), ("int4", 40), ("f16", 3), ("f16", 40)])
 def test_decode_chain_samples_some_rows(pkg, kind, c, forms, knobs):
     """Behind the last layer the tail and the final norm run for the sampled rows alone: all of them, some, one; a step that samples none leaves the
-    caches as it should, and listed rows find the residual.  (40 dense rows: the tail adds fp16 rows; fewer: slabs; experts: their combination.  Queries and keys are normed: without
+    caches as it should, and rows that a call lists, more than a head takes at once, find the residual.  (40 dense rows: the tail adds fp16 rows; fewer: slabs; experts: their combination.  Queries and keys are normed: without
     that, attention of random weights is a step function, and a row at its edge was 18 % from the oracle in the launches of their own, 23 in this.)"""
     from tests import modelgen
     if kind == "moe":
@@ -1253,8 +1325,13 @@ def test_decode_chain_samples_some_rows(pkg, kind, c, forms, knobs):
         hm.unified_forward([(i, [7 + i, 300, 21], 0, True) for i in range(c)], greedy=True)
         forms.reset()
         out[chain] = [hm.unified_forward([(i, [50 + i + s], 3 + s, pick(i)) for i in range(c)], greedy=True, want_logits=True)[1] for s, pick in enumerate(picks)]
-        assert (forms.hits().get("decode_chain", 0) > 0) == bool(chain), forms.hits()
+        n, s = forms.hits().get("decode_chain", 0), len(picks)
+        listed = hm.forward_rows([(i, [50 + i + s], 3 + s) for i in range(c)], [c - 1, 0, c // 2] + list(range(c)))
+        assert (n > 0) == bool(chain) and forms.hits().get("decode_chain", 0) == n + n // s, forms.hits()
+        out[chain].append(listed)
         del hm
+    assert np.abs(out[1][-1] - out[0][-1]).max() < 0.02 * np.abs(out[0][-1]).max()
+    assert np.abs(out[1][-1][[1, 0]] - out[1][-1][[3, c + 2]]).max() < 1e-4 * np.abs(out[0][-1]).max()         # (heads of other row counts: fp32 sums in another order)
     for s, (mine, other, pick) in enumerate(zip(out[1], out[0], picks)):
         n = sum(bool(pick(i)) for i in range(c))
         if n:
