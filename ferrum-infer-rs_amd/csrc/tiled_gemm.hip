@@ -555,6 +555,7 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
 //   4096 × 4096 × 4096   112 (2) | 98.8 (1)     4096 × 10240 × 2048   148 (5) | 146 (3)      7000 × 8192 × 1024   109 (7) | 111 (4)
 //   3000 × 8192 × 4096   164 (3) | 173 (2)      4096 × 6144 × 1024    57 (3) | 67 (2)        5000 × 3072 × 512    22.9 (2) | 23.4 (1)
 // so wherever its rounds are half as many as the other's, but for short K.
+// A wave with columns of several kinds, or rare ones, finishes its tile 26 µs later (1000 × 9472 × 2048 with several sections 57 | 78, 600 × 20224 × 2048 64 | 80).
 static long big_tiles(const GemmRows& rows, int m, int n, int groups, int r, int c) { return (long)(rows.id ? rows.max_blocks * (rows.block / r) : cdiv(m, r)) * cdiv(n, c) * groups; }
 template <typename E>
 bool tiled_gemm_takes_256(const TiledGemm<E>& g) {
@@ -565,7 +566,9 @@ bool tiled_gemm_takes_256(const TiledGemm<E>& g) {
         if (knobs().tiled_256 == 0) {
             if (knobs().tiled_wide_min_tiles >= 0) return false;        // (a forced size of the tiles below stays what it is)
             const long halves = cdiv(big_tiles(g.rows, g.m, g.n, g.groups, 128, 256), 256), rounds = cdiv(big_tiles(g.rows, g.m, g.n, g.groups, 256, 256), 256);
-            if (halves <= 1 || rounds * (11.6f + 0.0201f * g.k) >= (g.k > 512 ? 0.97f : 0.93f) * halves * (5.5f + 0.01185f * g.k)) return false;
+            bool mixed = false;
+            for (int i = 0; i < g.nsec; i++) mixed |= gemm_rare_act(g.sec[i].act) || g.sec[i].begin % 128;
+            if (halves <= 1 || rounds * (11.6f + 0.0201f * g.k) + (mixed ? 26.f : 0.f) >= (g.k > 512 ? 0.97f : 0.93f) * halves * (5.5f + 0.01185f * g.k)) return false;
         }
         return tiled_gemm_wide_supports(g);
     }

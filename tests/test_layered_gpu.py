@@ -548,8 +548,8 @@ def test_projections_in_tiles_of_256_x_256(pkg, tmp_path, knobs, forms, name):
 @pytest.mark.parametrize("ff,n,forced,taken", [(2048, 32, None, 1), (2048, 31, None, 0), (256, 32, None, 0), (2048, 32, 257, 0)])
 def test_blocks_of_256_sorted_rows(pkg, tmp_path, knobs, forms, ff, n, forced, taken):
     """Two experts of which each token takes one: blocks of 256 rows from a mean of 2048 (128 tokens a sequence, and one more), where one of the two projections runs in
-    tiles of as many rows (2048 columns of K 1024), not where neither does (256 columns, K of 256) or another size is asked for; against blocks of 128."""
-    cfg = G.safolorn(1024, 260, 40, [G.sink_attention(4, 64, 32, 32, 256, 1e5, G.LONG, mlp=G.experts(2, 1, ff))])
+    tiles of as many rows (2048 columns of K 2048), not where neither does (256 columns, K of 256) or another size is asked for; against blocks of 128."""
+    cfg = G.safolorn(2048, 260, 40, [G.sink_attention(4, 64, 32, 32, 256, 1e5, G.LONG, mlp=G.experts(2, 1, ff))])
     path = G.write_checkpoint(tmp_path, cfg, G.weights(cfg, 33))
     items = [(i, toks(cfg, 129, i), 0) for i in range(n)]
     at = [129 * i + j for i in range(n) for j in (0, 64, 128)]
@@ -563,6 +563,23 @@ def test_blocks_of_256_sorted_rows(pkg, tmp_path, knobs, forms, ff, n, forced, t
             assert forms.hits().get("moe_rows_256", 0) == taken, forms.hits()
         del m
     assert rel(out[None], out[128]) < 4e-3        # (both sum K in steps of 32 in fp32: equal but for the order, 16-bit results of one layer)
+
+
+def test_columns_of_several_kinds_in_one_round(pkg, tmp_path, knobs, forms):
+    """An input projection of one round of 256 x 256 whose sections begin within a wave's columns: those are finished slowly there, so it runs in tiles of 128 x 256."""
+    cfg = G.safolorn(1152, 260, 40, [G.sink_attention(16, 64, 32, 32, 256, 1e5, G.LONG, mlp=G.glu(1552, 1.5))])
+    path = G.write_checkpoint(tmp_path, cfg, G.weights(cfg, 35))
+    items = [(i, toks(cfg, 128, i), 0) for i in range(13)]
+    out = {}
+    for forced in (None, 1):
+        knobs.set(TILED_256=forced)
+        m = load(pkg, path, "bfloat16", tokens=128 * 13, seqs=13, blocks=8 * 13 + 2, max_len=256)
+        forms.reset()
+        out[forced] = m.forward_rows(items, [128 * i + 127 for i in range(13)])
+        h = forms.hits()
+        assert bool(h.get("tiled_gemm_256x256")) == bool(forced) and bool(h.get("tiled_gemm_128x256")) != bool(forced), h
+        del m
+    assert rel(out[None], out[1]) < 4e-3
 
 
 @pytest.mark.parametrize("name", ["wide", "shared", "sinks", "loop", "talks"])

@@ -490,12 +490,13 @@ def test_tiles_of_256_x_256(env, m, n, k, f32, knobs, forms):
     forms.require("tiled_gemm_256x256")
 
 
-@pytest.mark.parametrize("n,forced,taken", [(8192, None, True), (8224, None, False), (8192, 257, False), (8192, 256, False), (8192, -1, True)])
-def test_rule_of_tiles_of_256_x_256(env, n, forced, taken, knobs, forms):
-    """2001 rows, K of 1024: one round of them where two of 128 x 256 fill the card, two where three do; a number of the latter asked for, their own line's among
-    them, is what runs."""
+@pytest.mark.parametrize("m,n,k,forced,taken", [
+    (2001, 8192, 2048, None, True), (2001, 8224, 2048, None, False), (2001, 8192, 2048, 257, False), (2001, 8192, 2048, 256, False), (2001, 8192, 2048, -1, True)])
+def test_rule_of_tiles_of_256_x_256(env, m, n, k, forced, taken, knobs, forms):
+    """One round of them where two of 128 x 256 fill the card, not two where three do; a number of the smaller tiles asked for, their own
+    line's among them, is what runs."""
     knobs.set(TILED_WIDE_MIN_TILES=forced)
-    _few_rows(env, 2001, n, 1024)
+    _few_rows(env, m, n, k)
     hits = forms.hits()
     assert bool(hits.get("tiled_gemm_256x256")) == taken and bool(hits.get("tiled_gemm_128x256")) != taken, hits
 
