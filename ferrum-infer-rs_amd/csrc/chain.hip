@@ -1,16 +1,19 @@
-// The attention half of a decode layer as ONE launch (gfx950).
+// The attention half of a decode layer as ONE launch, and the MLP of a dense layer of few rows with it (gfx950).
 //
-// A decode step of ≤ 32 rows is a chain of small dependent ops (qwen3_moe_forward_unified_layer.rs:46-455 issues them one
+// A decode step of few rows is a chain of small dependent ops (qwen3_moe_forward_unified_layer.rs:46-455 issues them one
 // launch at a time): [tail of the previous layer: combine + add + norm] → q|k|v GEMM → QK-norm + RoPE + paged-KV write +
 // attention → o_proj GEMM → add + norm + router + top-k.  As five launches every link pays its own ramp, its first memory
 // round trips and its drain (≈ 4–5 µs each even when trivial) on top of the kernel boundary, while HBM idles.  Here the five
 // links are ROLES of one grid, laid out in dependency order (blocks of role A first, …): every workgroup requests what does
-// not depend on its predecessor — its INT4 weights (all of them: a wave's K slice is 2–4 quant groups), its block table and
+// not depend on its predecessor — its weights (all of them: a wave's K slice is 1–4 quant groups), its block table and
 // first K/V tiles, its norm and router weights — and only then waits for the predecessor's rows.  What is left on the
 // critical path of a link is: activations in, arithmetic, result out.  One 512-thread workgroup per CU is resident (the
-// attention role holds two K/V fragment sets, 232 registers): at 32 rows the tail (32 workgroups), the q|k|v projection (80)
+// attention role holds two K/V fragment sets, 225 – 229 registers): at 32 rows the tail (32 workgroups), the q|k|v projection (80)
 // and attention (128) are all there from the start, the o projection's workgroups move in as the tail's and q|k|v's leave
 // (long before attention is done) and the router's as attention's leave — each early enough to have its weights on the way.
+// Layers that take it: head_dim 128, at most 14 query heads a kv head, no biases, act order, zero points, sandwich norms or tensor parallelism; INT4 of 2048 or 4096
+// columns with o_proj of K 4096, experts or dense; unquantised dense layers of 1024 columns with K 2048, or of 2048 with K 2048 or 4096.  Their MLP goes in where its
+// width is whole 2048s (INT4) or 1024s (fp16), eight at most.  Others (2560, 3072, 3584, 5120 columns, …) run launches of their own.
 //
 // Hand-offs: the rows are their own flags.  A row that crosses workgroups inside the launch is all ones on entry (NOT_YET); its producer
 // stores it write-through (sc1, 8- or 16-byte stores) and is done; a consumer's wave asks for just what it needs (sc1 loads, the GEMM roles
@@ -20,8 +23,8 @@
 // a role's work to its consumer's first product, now 0.6 – 1.0; a launch of one row of 2048 columns 17.0 → 15.05 µs, 8 rows 19.7 → 18.05; a step
 // of one sequence through 8 expert layers, 32 steps and the prompt: 13.34 → 12.59 ms, of 12 through 32 layers of 4096 75.6 → 72.3).  No role
 // waits before all its predecessors' workgroups have been dispatched (dependency order = dispatch order, and nothing that waits comes before
-// something it waits for); every wait is bounded (≈ 20 ms) and a give-up is counted in a host-visible word, so a missing producer costs a wrong
-// result that the runner reports, never a hang.  The rows are double-buffered: the q|k|v workgroups, behind their own result, make the OTHER
+// something it waits for), so one launch cannot starve itself.  Two at once, on two streams or in two processes, can: every wait is bounded (≈ 20 ms), a
+// give-up is counted in a host-visible word, and the runner does the call again in separate launches.  The rows are double-buffered: the q|k|v workgroups, behind their own result, make the OTHER
 // half all ones for the next launch, which nobody reads any more (no fill node per layer; the forward's head kernel does it for its first launch).
 //
 // Dense layers of few rows go on behind role B (decode_chain_mlp_supports): gate_up and its activation (G), then down in K parts (D), as roles in
@@ -31,10 +34,11 @@
 // after 15 µs, G's rows seen 16.5 – 18.5, done 22 – 25, D's act seen 24 – 29, done 31.  (G workgroups that load D's weights through the XCD's cache under
 // their products: those took 2 µs longer, and D began no earlier.)
 //
-// Arithmetic: each role is the arithmetic of the stand-alone kernel it replaces, operation for operation —
+// Arithmetic: in an INT4 expert layer each role is the arithmetic of the stand-alone kernel it replaces, operation for operation —
 // moe_combine_add_rmsnorm_kernel, w4_gemm_wgsplit_kernel<MT, 2> (K split over the 8 waves, LDS reduction in wave order),
 // paged_attn_kernel<128, true, 8> (fused QK-norm / RoPE / KV write, 8 KV-splitting waves merged in wave order),
-// add_rmsnorm_route_part_kernel (Q expert parts per token, in-launch ticket merge) — so the results are the same bits.
+// add_rmsnorm_route_part_kernel (Q expert parts per token, in-launch ticket merge) — but for o_proj's two parts of K.  fp16 projections and the MLP's roles have
+// the products, roundings and fp32 sums of theirs and add K in another order (over the 8 waves, in parts of their own).
 #include "common.h"
 #include "handed_off.h"
 #include "kernels.h"
@@ -55,7 +59,7 @@ constexpr int CH_GRAN = 10;              // granules per (token, router part): 8
 constexpr int CH_O_KS = 2;                // o_proj: K parts per block, each a workgroup of its own (fp32 partial rows, role B adds them)
 constexpr int CH_MAX_SPLITS = 16;          // KV ranges per (sequence, kv head) in the attention role
 constexpr int CH_MAX_T = CHAIN_MAX_ROWS;
-constexpr int CH_GRAN_WORDS = CH_MAX_T * 4 * CH_GRAN * 2;      // T ≤ 64 tokens × Q ≤ 4 parts, 8-byte granules
+constexpr int CH_GRAN_WORDS = CH_MAX_T * 4 * CH_GRAN * 2;      // tokens × Q ≤ 4 parts, 8-byte granules
 constexpr int CH_SMEM = 8 * 16 * (128 + 4) * 4 + 2 * 8 * 16 * 4 + 16 * 128 * 2 + 2 * 128 * 2;     // the attention role's arena: 73,216 B
 
 constexpr int CH_QKV_NST = 1, CH_O_NST = 1;     // 64-column supertiles per workgroup: one head (128 columns) for q|k|v, 64 columns for o_proj; 16 rows each
@@ -183,7 +187,7 @@ __device__ __forceinline__ void chain_role_a(const ChainArgs& p, int row, unsign
     for (int c = 0; c < CH; c++) {
         const int i = threadIdx.x + c * 512;
         if (i < nvec && p.has_a == 3) {
-            // dense model, the MLP's output as fp16 rows (≤ 16 or > 32 rows: no slabs): residual add, as fused_add_rms_norm
+            // dense model, the MLP's output as fp16 rows (no slabs): residual add, as fused_add_rms_norm
             const half8 xv = *reinterpret_cast<const half8*>(p.a_x + (long)row * H + i * 8);
             half8 rv = *reinterpret_cast<const half8*>(p.res_in + (long)row * H + i * 8);
 #pragma unroll
@@ -513,7 +517,7 @@ __device__ __forceinline__ void chain_role_gemm(const ChainGemm& w, int cb, int 
 }
 
 // ── attention role: paged_attn_kernel<128, true, 8> (decode, one new token per sequence) ────────────────────────────────
-template <bool KVS, bool WIDE>
+template <bool KVS>
 __device__ __forceinline__ void chain_role_attn(const ChainArgs& p, int wg, unsigned char* smem) {
     constexpr int HD = 128, NW = CH_W, DT = HD / 16, KS = HD / 32, OSTRIDE = HD + 4;
     float* lds_o = reinterpret_cast<float*>(smem);                    // [NW·16][OSTRIDE]
@@ -1119,7 +1123,7 @@ __global__ __launch_bounds__(512, 2) void decode_chain_kernel(ChainArgs p) {
         return;
     }
     wg -= n_qkv;
-    if (wg < n_attn) { chain_role_attn<KVS, WIDE>(p, wg, smem); return; }
+    if (wg < n_attn) { chain_role_attn<KVS>(p, wg, smem); return; }
     wg -= n_attn;
     if (wg < n_o) {
         // (K part fastest: the two workgroups of a block are neighbours)
@@ -1198,11 +1202,11 @@ bool decode_chain_mlp_supports(const W4Device& qkv, const W4Device& gu, const W4
     return inter % 128 == 0 && gu.k == qkv.k && gu.n == 2 * inter && dn.k == inter && dn.n == qkv.k && dn.G % per == 0 && dn.G / per <= 8 &&
            (size_t)(dn.G / per) * rows * dn.n * 4 <= slab_bytes;
 }
-// Rows up to which the launch takes the MLP: one block of them, and two of the smallest layers (µs of a step, the MLP's two launches behind the chain
-// | in it.  32 INT4 layers of 4096, inter 14336: 1 row 1393 | 1273, 4 rows 1430 | 1315, 12 of 120 keys 1568 | 1430, 16 1623 | 1483, 17 2096 | 2333, 1 of 8000
-// keys 1591 | 1437.  8 of 4096, 12288, GELU: 1 376 | 344, 8 393 | 362, 16 436 | 402, 17 550 | 557.  8 of 2048, 8192: 1 260 | 230, 8 287 | 246, 16 338 | 271, 17
-// 407 | 404, 32 428 | 428.  14 fp16 layers of 1024, 3072: 1 371 | 302, 8 418 | 330, 16 441 | 350, 17 488 | 439, 32 523 | 475, 64 707 | 751.  8 of 2048,
-// 6144: 1 310 | 268, 8 339 | 304, 16 368 | 321, 17 420 | 457, 32 450 | 492.)
+// Rows up to which the launch takes the MLP: one block of them, and two of the smallest layers.  µs of a step without its vocabulary, the MLP's two launches behind the
+// chain | in it.  32 INT4 layers of 4096, inter 14336: 1 row 1228 | 1091, 4 rows 1293 | 1145, 8 1312 | 1181, 12 of 120 keys 1453 | 1282, 16 1454 | 1289, 1 of 8000 keys
+// 1417 | 1267.  8 of 4096, 12288, GELU: 1 332 | 282, 8 357 | 310, 16 390 | 337.  8 of 2048, 8192: 1 222 | 186, 8 247 | 205, 16 292 | 228.  14 fp16 layers of 1024, 3072:
+// 1 307 | 233, 8 339 | 260, 16 368 | 279, 17 418 | 369, 32 450 | 400.  8 of 2048, 6144: 1 272 | 227, 8 297 | 262, 16 325 | 276.
+// Past the line, when it was drawn (vocabularies included): 17 rows of those layers 2096 | 2333, 550 | 557, 407 | 404 (32: 428 | 428), fp16 of 2048 420 | 457, of 1024 64 rows 707 | 751.
 int decode_chain_mlp_max_rows(const W4Device& qkv) { return qkv.f16t && qkv.G == 8 ? 32 : 16; }
 // Rows up to which a dense layer takes the launch: beyond 64 the 64-row GEMM tiles win (INT4 of 4096 × 14336, 96 rows: 5.56 ms a step against 5.61), and through
 // fp16 layers of 2048 columns the fourth block of rows costs more than the launches of their own (µs of a step of 6 layers, those | this one: 32 heads on 8, 48 rows

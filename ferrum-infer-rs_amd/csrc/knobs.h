@@ -41,7 +41,7 @@ struct Knobs {
     int route_gemm_topk = 1;          // prefill router GEMM + top-k as one launch (E = 128)
     int chain_attn_splits = 0;        // > 0: that many KV ranges whatever the context (experiments)
     int chain_max_keys = 4096;        // decode chain only up to this many keys per attention workgroup (× T·nkv / 128)
-    int dense_chain = 1;              // dense models at ≤ 64 rows: the attention half of the layer as the chain launch too (0 = launches of its own)
+    int dense_chain = 1;              // dense models at ≤ 64 rows (fp16 of 2048 columns: 48): the attention half of the layer as the chain launch too (0 = launches of its own)
     int chain_mlp_rows = 32;          // … and its MLP in that launch, up to this many rows (0 = its own two launches)
     int moe_em2 = 1;                  // decode: gate_up → down as one expert-major launch (0 = two launches)
     int moe_bm2 = 0;                  // decode at ≤ 64 pairs: gate_up → down as one block-major launch — measured slower than the two launches (profiles/r03_moe_bm2_timeline.txt): off

@@ -1561,8 +1561,8 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
     RUN(embed_rms_norm_f16(m->embed, tokens, c.embed_scale, m->residual, sandwich ? m->residual_f32 : nullptr, m->layers[0].input_ln,
                            c.rms_eps, m->norm_out, T, H, counters ? m->route_arrive : nullptr, counters ? 64 + (int)m->arrive_half_words : 0,
                            chain_rows ? reinterpret_cast<unsigned*>(m->chain_rows) : nullptr, chain_rows ? (int)(T * decode_chain_row_bytes(H, nq, nkv, chain_inter) / 4) : 0, s, m->layers[0].qkv.perm));
-    // dense models at 17–32 rows: the same launch for the attention half (tail of the previous layer's MLP — its down slabs +
-    // residual + norm — q|k|v, attention, o_proj, add + norm), then gate_up slabs → gated activation → down slabs
+    // dense models: the same launch (tail of the previous layer's MLP — its down slabs or fp16 rows + residual + norm — q|k|v, attention, o_proj, add + norm), with gate_up,
+    // activation and down in it (chain_inter) or behind it
     bool pending_dense_tail = false, tail_mlp = false;      // (tail_mlp: the slabs are the launch's own)
     int tail_S = 0, tail_rows_pad = 0, tail_n_pad = 0;
     auto dense_tail = [&](DecodeChainDesc& d) {
