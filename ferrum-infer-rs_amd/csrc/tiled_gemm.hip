@@ -554,8 +554,9 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
 //   2001 × 8192 × 1024  35.6 (2) | 34.3 (1)     3500 × 8192 × 2048    110 (4) | 100 (2)      8192 × 10240 × 4096  539 (10) | 463 (5)
 //   4096 × 4096 × 4096   112 (2) | 98.8 (1)     4096 × 10240 × 2048   148 (5) | 146 (3)      7000 × 8192 × 1024   109 (7) | 111 (4)
 //   3000 × 8192 × 4096   164 (3) | 173 (2)      4096 × 6144 × 1024    57 (3) | 67 (2)        5000 × 3072 × 512    22.9 (2) | 23.4 (1)
-// so wherever its rounds are half as many as the other's, but for short K: up to 1024 from four rounds on, since less than that is saved by the launch and lost by its
-// neighbours, whose clock falls (four layers of 1024 columns, ms of a prompt in 128 × 256 | in these: one of 8192 tokens 2.78 | 2.89, of 7000 2.41 | 2.49, 64 of 256 3.05 | 2.85).
+// so wherever its rounds are half as many as the other's, but for short K: up to 1024 not in two or three rounds, which save the launch 3 µs and cost its neighbours, whose
+// clock falls, more (four layers of 1024 columns, ms of a prompt in 128 × 256 | in these: one of 2300 tokens 0.89 | 0.87, of 7000 2.41 | 2.49, of 8192 2.78 | 2.89, 64 of 256
+// 3.05 | 2.85).
 // A wave with columns of several kinds, or rare ones, finishes its tile 20 – 26 µs later, which four rounds make up for (K = 2048, µs of the latter | of the former: 9472 columns
 // with several sections, 1000 rows 55 | 75, 3000 108 | 125, 5000 163 | 176, 8192 281 | 277, 12000 380 | 372; 20224 columns, 600 rows 62 | 75, 3000 219 | 209, 8192 563 | 485).
 static long big_tiles(const GemmRows& rows, int m, int n, int groups, int r, int c) { return (long)(rows.id ? rows.max_blocks * (rows.block / r) : cdiv(m, r)) * cdiv(n, c) * groups; }
@@ -570,7 +571,7 @@ bool tiled_gemm_takes_256(const TiledGemm<E>& g) {
             const long halves = cdiv(big_tiles(g.rows, g.m, g.n, g.groups, 128, 256), 256), rounds = cdiv(big_tiles(g.rows, g.m, g.n, g.groups, 256, 256), 256);
             bool mixed = false;
             for (int i = 0; i < g.nsec; i++) mixed |= gemm_rare_act(g.sec[i].act) || g.sec[i].begin % 128;
-            if (halves <= 1 || (mixed && rounds < 4) || (g.k <= 1024 && rounds < 4) || rounds * (11.6f + 0.0201f * g.k) >= (g.k > 512 ? 0.97f : 0.93f) * halves * (5.5f + 0.01185f * g.k)) return false;
+            if (halves <= 1 || (mixed && rounds < 4) || (g.k <= 1024 && (rounds == 2 || rounds == 3)) || rounds * (11.6f + 0.0201f * g.k) >= (g.k > 512 ? 0.97f : 0.93f) * halves * (5.5f + 0.01185f * g.k)) return false;
         }
         return tiled_gemm_wide_supports(g);
     }

@@ -492,9 +492,9 @@ def test_tiles_of_256_x_256(env, m, n, k, f32, knobs, forms):
 
 @pytest.mark.parametrize("m,n,k,forced,taken", [
     (2001, 8192, 2048, None, True), (2001, 8224, 2048, None, False), (2001, 8192, 2048, 257, False), (2001, 8192, 2048, 256, False), (2001, 8192, 2048, -1, True),
-    (2001, 8192, 1024, None, False), (3072, 16384, 1024, None, False), (4096, 16384, 1024, None, True)])
+    (2001, 8192, 1024, None, True), (2048, 16384, 1024, None, False), (3072, 16384, 1024, None, False), (4096, 16384, 1024, None, True)])
 def test_rule_of_tiles_of_256_x_256(env, m, n, k, forced, taken, knobs, forms):
-    """One round of them where two of 128 x 256 fill the card, not two where three do; with K of 1024 from four rounds on; a number of the smaller tiles asked for, their own
+    """One round of them where two of 128 x 256 fill the card, not two where three do; with K of 1024 one or four, not two or three; a number of the smaller tiles asked for, their own
     line's among them, is what runs."""
     knobs.set(TILED_WIDE_MIN_TILES=forced)
     _few_rows(env, m, n, k)
