@@ -22,6 +22,7 @@
 //    walks its whole KV range — no cross-wave merge, a loop long enough to amortise the prologue (at 256-token prompts
 //    the KV-split form gives a wave 1–2 block pairs), and the four waves request the same K/V lines at about the same
 //    time (L1 hits instead of 4× the L2 traffic).
+#include "attention_device.h"
 #include "common.h"
 #include "kernels.h"
 #include "knobs.h"
@@ -29,34 +30,6 @@
 #include "rope_rows.h"
 
 namespace fh {
-
-struct AttnArgs {
-    const __half* q;        // [total_q, nq, hd]
-    const __half* k_pool;   // [blocks, nkv, tile]
-    const __half* v_pool;
-    __half* out;            // [total_q, nq, hd]
-    const uint32_t* cu_seqlens_q;   // [num_seqs+1] or null (decode: token i ↔ seq i)
-    const uint32_t* pos_offsets;    // [num_seqs] kv position of each seq's first q token
-    const uint32_t* kv_lens;        // decode form: [num_seqs] kv length incl. the new token (pos = len-1)
-    const int32_t* block_tables;    // [num_seqs, max_blocks]
-    float* partial;         // [tiles][nsplit][16][hd+2] when nsplit > 1
-    int num_seqs, nq, nkv, tiles_per_seq, max_blocks, sliding_window, nsplit, units;
-    int compact;            // grid.x enumerates real work units of a ragged batch (see the kernel), not num_seqs × tiles_per_seq
-    float scale;
-    // fused decode form (FUSED_QKV): q / new K / new V come straight from the qkv projection output
-    const __half* qkv;      // [num_seqs, (nq + 2·nkv)·hd]
-    const __half* q_norm_w;
-    const __half* k_norm_w;
-    const float* cos_t;
-    const float* sin_t;
-    __half* k_pool_w;
-    __half* v_pool_w;
-    float eps;
-    int qk_mode;
-    // decode forms: the consumer is an act-order o_proj — channel c of a row is stored at out_scatter[c] (inverse of the
-    // projection's row permutation), so no gather launch sits between attention and the GEMM
-    const int32_t* out_scatter;
-};
 
 // a·b rounded to fp32, then to fp16: without the barrier the compiler rounds once (v_fma_mixlo_f16) in some instantiations and twice
 // in others, and forms that promise the same bits differ in the last one
@@ -664,61 +637,16 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void paged_prefill_attn_ker
 // operand against Pᵀ: every lane's accumulator then holds Σ_keys P of its query row, rescaled by α like O), and steps whose 64
 // keys are visible to every row of a tile (all but the diagonal ones) run a mask-free body.  Same staging, tile layout and
 // per-row arithmetic otherwise (Sᵀ = K·Qᵀ, lane-local exp2, Oᵀ += Vᵀ·Pᵀ); l is the sum of the fp16 P the numerator uses.
-template <int HD, int MT>
+template <int HD>
 __global__ __launch_bounds__(256, 2) void paged_prefill_attn64_kernel(AttnArgs p) {
-    constexpr int NW = 4, DT = HD / 16, KS = HD / 32, TILE = 16 * HD;
+    constexpr int NW = 4, MT = 2, DT = HD / 16, KS = HD / 32, TILE = 16 * HD;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     __half* lds_kv = reinterpret_cast<__half*>(smem);          // [2 stages][2 pairs][K0, K1, V0, V1][TILE]; reused by the epilogue
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int a = lane >> 4, b = lane & 15;
-    // workgroup → (kv head, unit): workgroups go to the XCDs in turn, and a head's units are taken on one XCD (on 8 / nkv of them with fewer
-    // heads), whose L2 holds the keys of 8000 tokens.  Dealt over all XCDs every L2 saw every head, and a step waited for the last-level
-    // cache (8100 tokens of 32 heads on 8 705 → 590 µs, 2048 76 → 62; 1500 and 548 of 16 on 8 47.6 → 42.5).
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    int kvh, from_last;
-    if ((p.nkv & 7) == 0) {
-        kvh = xcd + 8 * (slot / p.units);
-        from_last = slot % p.units;
-    } else if ((8 % p.nkv) == 0) {
-        kvh = xcd % p.nkv;
-        from_last = slot * (8 / p.nkv) + xcd / p.nkv;
-    } else {
-        kvh = blockIdx.x / p.units;
-        from_last = blockIdx.x % p.units;
-    }
-    if (from_last >= p.units) return;
-    const int G = p.nq / p.nkv;
-    int seq = -1, unit = 0;
-    {
-        const int w = p.units - 1 - from_last;       // launch order reversed: the longest key ranges (last units of a causal prompt) start first
-        int base = 0;
-        for (int s0 = 0; s0 < p.num_seqs; s0 += 64) {
-            const int s = s0 + lane;
-            int units = 0;
-            if (s < p.num_seqs) {
-                const int tiles = ((int)(p.cu_seqlens_q[s + 1] - p.cu_seqlens_q[s]) * G + 15) >> 4;
-                units = (tiles + NW * MT - 1) / (NW * MT);
-            }
-            int incl = units;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                const int t = __shfl_up(incl, off, 64);
-                if (lane >= off) incl += t;
-            }
-            const int total = __shfl(incl, 63, 64);
-            if (w < base + total) {
-                const unsigned long long hit = __ballot(w < base + incl);
-                const int src = __ffsll((long long)hit) - 1;
-                seq = s0 + src;
-                unit = w - (base + __shfl(incl - units, src, 64));
-                break;
-            }
-            base += total;
-        }
-        if (seq < 0) return;
-        seq = __builtin_amdgcn_readfirstlane(seq);          // wave-uniform by construction: scalar table reads below
-        unit = __builtin_amdgcn_readfirstlane(unit);
-    }
+    PrefillUnit u;
+    if (!prefill_unit(p, NW * MT, lane, &u)) return;
+    const int kvh = u.kvh, seq = u.seq, unit = u.unit, G = p.nq / p.nkv;
     const int tok0 = (int)p.cu_seqlens_q[seq];
     const int q_len = (int)p.cu_seqlens_q[seq + 1] - tok0;
     const int rows_total = q_len * G, tiles_s = (rows_total + 15) >> 4;
@@ -1239,23 +1167,22 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
         form_hit(FORM_ATTN_RESIDENT);
         return 0;
     }
-    // head_dim 128 has two sizes of workgroup.  128 rows read K/V from LDS half as often, 64 rows make twice the workgroups and half of a step's
-    // vector work in each; two workgroups of either share a CU.  The longest keys of a prompt are a workgroup's alone, and 64 rows pass them
-    // in 0.65 of the time, until there are rounds enough to hide that: 64 rows below 620 workgroups of 128.  Where a window or a context of
-    // more than 1.5 times the new tokens leaves every workgroup about as many keys, below 360.  Over 229 batches between 256 and 2300 that
-    // choice is 0.6 % from the faster of the two, always 128 rows 7, always 64 rows 11 (128 rows take up to 1.7 times as long below 360, 64 rows 1.4 times from 1000 on).
+    // head_dim 128 has two forms.  Workgroups of 128 rows share keys in LDS; in those of 64 rows each wave reads keys of its own (attention_keys.hip).  A workgroup
+    // passes the longest keys of a prompt alone, and 64 rows pass them in half the time: that form below 720 workgroups of 128.  Where a window or a context of
+    // more than 1.5 times the new tokens leaves every workgroup about as many keys, below 900.  Beyond that 128 rows take the caches half as often, at a higher clock.
     // µs, row-split or KV-split form / 64 rows / 128 rows (workgroups of 128 rows × kv heads)
-    //   8B heads (32 on 8)    1 × 8100 (2024)      2372 / 789 / 606      1 × 2048 (512)        196 / 66 / 65     1 × 1024 (256)         62 / 27 / 34
-    //                         1 × 2180 (545)            - / 75 / 92      1 × 700 (175)          32 / 21 / 31     1 × 500 (125)          19 / 16 / 19
-    //   16 on 8               1500 and 548 (256)     82 / 43 / 61        293, 1389, 366 (256)   87 / 40 / 56     1 × 986 at 366 (123)   49 / 36 / 51
-    //                         6 × 100, 1400 (250)    80 / 37 / 82        1 × 500 (62)           14 / 14 / 15     32 on 8, 1 × 4360 (1090)  - / 246 / 199
+    //   8B heads (32 on 8)    1 × 8100 (2024)      2372 / 654 / 578      1 × 2800 (700)          - / 96 / 114    1 × 2048 (512)          196 / 59 / 65
+    //                         1 × 3200 (800)           - / 119 / 113     1 × 1200 (300)          - / 28 / 50     [1600, 1600] (800)        - / 73 / 66
+    //                         2400 at 5800 (600)       - / 340 / 382     3200 at 7400 (800)      - / 588 / 588   4000 at 9000 (1000)       - / 840 / 777
+    //                         500 at 1000 (128)       57 / 24 / -        256 at 6000 (64)      146 / 60 / -      64 at 6000 (16)          54 / 56 / -
+    //   16 on 8               1500 and 548 (256)      82 / 28 / 61       293, 1389, 366 (256)   87 / 34 / 56     1 × 986 at 366 (123)     49 / 22 / 51
     // A batch qualifies where most of its sequences bring many rows, or they bring 256 on average.
     const long rows_heads = (long)total_q_tokens * G * num_kv_heads;
     const bool two_sizes = head_dim == 128 && !kn.attn_flash32, even = (sliding_window > 0 && max_kv_len > sliding_window) || (long)max_kv_len * 2 >= (long)max_q_len * 5;
-    const bool half_units = two_sizes && (kn.attn_flash_rows ? kn.attn_flash_rows == 64 : rows_heads < (even ? 360 : 620) * 128);
+    const bool half_units = two_sizes && (kn.attn_flash_rows ? kn.attn_flash_rows == 64 : rows_heads < (even ? 900 : 720) * 128);
     const bool flash_fits = (long)total_q_tokens * 2 >= (long)num_seqs * max_q_len || (two_sizes && (long)total_q_tokens * G >= (long)num_seqs * 256);
     if (!fq && cu_seqlens_q && !flash_off && (long)max_q_len * G >= flash_min_rows && flash_fits &&
-        rows_heads / (half_units || head_dim == 256 ? 64 : 128) >= (half_units && !kn.attn_flash_min_rows_set ? 192 : flash_min_wgs)) {
+        rows_heads / (half_units || head_dim == 256 ? 64 : 128) >= (half_units && !kn.attn_flash_min_rows_set ? (even ? 64 : 192) : flash_min_wgs)) {
         const int mt = half_units || head_dim == 256 ? 1 : 2, unit_tiles = 4 * mt;
         const long tiles_bound = ((long)total_q_tokens * G) / 16 + num_seqs;
         const long units = cdiv(tiles_bound, (long)unit_tiles) + num_seqs;
@@ -1271,18 +1198,24 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
             }                                                                                                          \
             hipLaunchKernelGGL((paged_prefill_attn_kernel<HDV, MTV>), grid, dim3(256), lds, s, a);                     \
         }
-        if (head_dim == 128 && !kn.attn_flash32) {           // 64 keys per step: two pairs per stage
-            const size_t lds64 = 2 * lds;
-            static bool attr64 = false;
-            if (!attr64) {
-                FH_CHECK_HIP(hipFuncSetAttribute((const void*)paged_prefill_attn64_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64));
-                FH_CHECK_HIP(hipFuncSetAttribute((const void*)paged_prefill_attn64_kernel<128, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64));
-                attr64 = true;
-            }
+        if (two_sizes) {
             a.units = (int)units;
             const dim3 flat((unsigned)(num_kv_heads < 8 && 8 % num_kv_heads == 0 ? 8 * cdiv(units, 8 / num_kv_heads) : units * num_kv_heads));
-            if (mt == 1) hipLaunchKernelGGL((paged_prefill_attn64_kernel<128, 1>), flat, dim3(256), lds64, s, a);
-            else hipLaunchKernelGGL((paged_prefill_attn64_kernel<128, 2>), flat, dim3(256), lds64, s, a);
+            if (mt == 1) {
+                // Eight waves where no workgroup shares its CU with another and the keys are many enough to pay for the larger merge
+                // (256 at 6000: 67 → 58 µs, 986 at 366 25 → 22; three of 170 at 300, 264 workgroups, 16 → 24; 256 at 0 11 → 12)
+                const long wgs = ((long)total_q_tokens * G + 63L * num_seqs) / 64 * num_kv_heads;
+                const bool eight = kn.attn_key_waves ? kn.attn_key_waves == 8 : wgs <= 256 && max_kv_len >= 512;
+                if (int rc = paged_prefill_attn_keys(a, eight, flat, s)) return rc;
+            } else {                                         // 64 keys per step: two pairs per stage
+                const size_t lds64 = 2 * lds;
+                static bool attr64 = false;
+                if (!attr64) {
+                    FH_CHECK_HIP(hipFuncSetAttribute((const void*)paged_prefill_attn64_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64));
+                    attr64 = true;
+                }
+                hipLaunchKernelGGL((paged_prefill_attn64_kernel<128>), flat, dim3(256), lds64, s, a);
+            }
         } else if (head_dim == 128) FH_FLASH(128, 2) else if (head_dim == 64) FH_FLASH(64, 2) else FH_FLASH(256, 1)
 #undef FH_FLASH
         FH_CHECK_LAUNCH();

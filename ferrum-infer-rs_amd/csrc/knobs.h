@@ -24,7 +24,8 @@ struct Knobs {
     bool attn_narrow = false;
     bool attn_no_resident = false;    // never take the resident-K/V short-prompt prefill form
     long attn_resident_min_wgs = 128; // … and only from this many workgroups (tests lower it)
-    int attn_flash_rows = 0;          // 64 / 128: forced rows per workgroup of the 64-key form
+    int attn_flash_rows = 0;          // 64 / 128: forced rows per workgroup of prompt attention (64: each wave on keys of its own)
+    int attn_key_waves = 0;           // 4 / 8: forced waves per workgroup of the 64-row form
     bool attn_flash32 = false;        // the flash form with 32-key steps (paged_prefill_attn_kernel) for head_dim 128 too
     int rope_quad_rows = 8192;        // split q|k|v, norm, rotation, cache write: four tokens of a head a wave from this many rows of a head
     // INT4 GEMMs (w4_gemm.hip)
@@ -172,6 +173,8 @@ enum Form : int {
     FORM_CHAIN_ROWS,            // decode chain: a forward's head made its rows ready
     FORM_MOE_ROWS_256,          // layered experts: sorted rows in blocks of 256
     FORM_DONE_AGAIN,            // a call whose in-launch waits gave up was done again in separate launches
+    FORM_ATTN_KEYS,             // prompt attention, each wave of a 64-row workgroup on keys of its own: four waves
+    FORM_ATTN_KEYS_WIDE,        // … eight
     FORM_COUNT
 };
 

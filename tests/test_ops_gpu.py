@@ -1033,6 +1033,34 @@ def test_paged_prefill_attention_in_both_unit_sizes(env, window, nq, nkv, rows, 
     test_paged_prefill_attention_lds_shared_kv(env, window, nq, nkv, 128, knobs, forms)
 
 
+@pytest.mark.parametrize("waves", [4, 8])
+@pytest.mark.parametrize("q_lens,pos,window,nq,nkv", [
+    ([9], [0], 0, 8, 8), ([64], [0], 0, 1, 1), ([65, 31], [0, 97], 0, 2, 2), ([16, 17], [15, 16], 0, 8, 2), ([128, 9], [129, 1000], 0, 14, 2),
+    ([300], [0], 33, 4, 2), ([40, 200], [700, 31], 64, 6, 6), ([22, 5, 70], [490, 3, 256], 1, 32, 4), ([258], [511], 0, 16, 8)])
+def test_prompt_attention_with_keys_by_wave(env, q_lens, pos, window, nq, nkv, waves, knobs, forms):
+    """Keys split over the waves of a workgroup: waves without any, rows and keys that do not fill a tile, a page or a step, groups that do not divide a tile, windows
+    that begin inside a step and leave waves nothing.  Against float32: probabilities and results are rounded by at most 2^-11 of themselves, (2 x 2^-11)^2 squared."""
+    pkg, B, ctx, O, torch = env
+    knobs.set(ATTN_FLASH_ROWS=64, ATTN_FLASH_MIN_ROWS=1, ATTN_KEY_WAVES=waves, ATTN_NO_RESIDENT=1)
+    S, total, kv = len(q_lens), sum(q_lens), [p + t for p, t in zip(pos, q_lens)]
+    mb = (max(kv) + 15) // 16
+    gen = torch.Generator("cuda").manual_seed(total)
+    rand = lambda *n: torch.randn(*n, generator=gen, device="cuda").half()
+    K, V, q = [rand(n, nkv, 128) for n in kv], [rand(n, nkv, 128) for n in kv], rand(total, nq, 128)
+    tables = torch.randperm(S * mb, generator=gen, device="cuda").to(torch.int32).reshape(S, mb)
+    ck, cv = _fill_pool(env, [host(x) for x in K], [host(x) for x in V], tables.cpu().numpy(), kv, nkv, 128, S * mb)
+    cu = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+    out = torch.full((total + 1, nq, 128), 9.0, dtype=torch.float16, device="cuda")
+    B.paged_varlen_attention(ctx, q, ck, cv, out, torch.from_numpy(cu).cuda(), torch.tensor(pos, dtype=torch.int32, device="cuda"), tables, S, total, max(kv), nq, nkv, 128,
+                             window, 16, mb, max(q_lens))
+    ctx.sync()
+    forms.require("attn_keys" if waves == 4 else "attn_keys_wide", absent=("attn_row_split", "attn_kv_narrow"))
+    assert bool((out[total] == 9.0).all())
+    for s in range(S):
+        ref = _ref_attention(O, host(q[cu[s]:cu[s + 1]]), host(K[s]), host(V[s]), pos[s], nq, nkv, 128, window)
+        assert nmse(ref, host(out[cu[s]:cu[s + 1]])) < 4 * 2.0 ** -22, s
+
+
 @pytest.mark.parametrize("nq,nkv,q_lens,pos,flash", [
     (16, 8, [1500, 548], [0, 0], True), (16, 8, [293, 1389, 366], [1133, 0, 0], True), (16, 8, [100] * 6 + [1400], [0] * 7, True),
     (16, 8, [986], [366], True), (16, 8, [767], [0], False), (16, 8, [769], [0], True), (32, 8, [384], [0], True), (32, 8, [383], [1], False),
