@@ -143,6 +143,8 @@ struct FerrumHipModel {
     fh::IndexLayout il{};
     uint8_t* idx_host = nullptr;   // pinned
     uint8_t* idx_dev = nullptr;
+    uint8_t* results = nullptr;    // pinned: logits on their way to the caller, in portions, and sampled ids behind them
+    hipEvent_t results_done[3] = {};
 
     // decode-steps state
     uint32_t* history = nullptr;   // [steps, sequences] sampled ids, pinned: written by the steps, read by the host

@@ -398,7 +398,7 @@ class HipModel:
             arr[i] = BatchItem(sid, keep[i].ctypes.data_as(C.POINTER(C.c_uint32)), len(keep[i]), pos, int(fin), 0)
             n_final += int(bool(fin))
         toks = np.zeros(max(n_final, 1), np.uint32)
-        logits = np.zeros((max(n_final, 1), self.local_vocab()[1]), np.float32) if want_logits else None   # this rank's slice when vocab_parallel
+        logits = np.empty((max(n_final, 1), self.local_vocab()[1]), np.float32) if want_logits else None   # this rank's slice when vocab_parallel
         opts, hold = None, []
         if token_mask is not None or repetition_penalties is not None:
             opts = GreedyOptions()
@@ -431,7 +431,7 @@ class HipModel:
         for i, (sid, _, pos) in enumerate(items):
             arr[i] = BatchItem(sid, keep[i].ctypes.data_as(C.POINTER(C.c_uint32)), len(keep[i]), pos, 0, 0)
         r = _i32(rows)
-        out = np.zeros((max(len(r), 1), self.local_vocab()[1]), np.float32)
+        out = np.empty((max(len(r), 1), self.local_vocab()[1]), np.float32)
         _check(self.lib.ferrum_hip_model_unified_forward_rows(self.h, arr, len(items), r.ctypes.data_as(C.POINTER(C.c_int32)), len(r),
                                                               out.ctypes.data_as(C.POINTER(C.c_float))), "unified_forward_rows")
         return out[:len(r)]

@@ -172,6 +172,33 @@ def test_long_block_tables_are_handed_over_at_once(pkg):
     assert best[32768] - best[512] < 110e-6, best
 
 
+@pytest.mark.parametrize("rows", [1, 8, 9, 40])
+def test_logits_by_way_of_pinned_portions(pkg, rows):
+    """4 MiB at a time, three on their way: a part of one, one whole, a little more, more than the ring holds; bit for bit what a copy into pinned memory gives."""
+    import ctypes as C
+    import torch
+    from ferrum_infer_rs_amd.executor import BatchItem
+    vocab = 131072
+    m = pkg.HipModel(group_size=128, num_layers=1, hidden=256, num_heads=4, num_kv_heads=2, head_dim=128, intermediate=256, vocab=vocab, has_qk_norm=1, activation=0,
+                     rms_eps=1e-6, rope_theta=1e6, max_seq_len=64, kv_num_blocks=2 * rows + 1, max_seqs=rows, max_tokens=rows * 3)
+    m.init_synthetic(3)
+    m.finalize()
+    tokens = [np.array([7 + i, 90 + i, 5], np.uint32) for i in range(rows)]
+    ids, logits = m.unified_forward([(i, tokens[i], 0, True) for i in range(rows)], want_logits=True)
+    for i in range(rows):
+        m.release(i)
+    pinned = torch.full((rows, vocab), 9.0, pin_memory=True)
+    items = (BatchItem * rows)(*[BatchItem(i, t.ctypes.data_as(C.POINTER(C.c_uint32)), 3, 0, 1, 0) for i, t in enumerate(tokens)])
+    got = np.zeros(rows, np.uint32)
+    assert m.lib.ferrum_hip_model_unified_forward_ex(m.h, items, rows, 1, None, got.ctypes.data_as(C.POINTER(C.c_uint32)),
+                                                     C.cast(pinned.data_ptr(), C.POINTER(C.c_float))) == 0
+    assert np.array_equal(pinned.numpy(), logits) and np.array_equal(got, ids) and np.array_equal(ids, logits.argmax(1))
+    for i in range(rows):
+        m.release(i)
+    every = m.forward_rows([(i, t, 0) for i, t in enumerate(tokens)], list(range(3 * rows)))
+    assert np.array_equal(every[2::3], logits)
+
+
 @pytest.mark.parametrize("big,prompt_len", [(6, 97), (8, 200), (16, 256), (16, 300)])
 @pytest.mark.parametrize("inter,activation,asym", [(384, 0, False), (640, 1, False), (128, 0, True), (1152, 1, True)])
 def test_prompt_gate_up_with_its_activation(pkg, big, prompt_len, inter, activation, asym, knobs, forms):
