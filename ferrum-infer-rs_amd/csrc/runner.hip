@@ -908,6 +908,11 @@ static int finalize_batch_buffers(FerrumHipModel* m) {
     FH_CHECK_HIP(hipHostMalloc((void**)&m->results, RESULT_RING * RESULT_PORTION + S * 4, hipHostMallocDefault));
     for (hipEvent_t& e : m->results_done) FH_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     if (int r = dev_alloc(&m->step_counter, (size_t)4)) return r;
+    // the pages of the results and the copy engine, once, ahead of the first call that waits for them (4 ms of it)
+    memset(m->results, 0, RESULT_RING * RESULT_PORTION + S * 4);
+    FH_CHECK_HIP(hipMemcpyAsync(m->results, m->idx_dev, std::min(off, RESULT_PORTION), hipMemcpyDeviceToHost, m->stream));
+    FH_CHECK_HIP(hipEventRecord(m->results_done[0], m->stream));
+    FH_CHECK_HIP(hipStreamSynchronize(m->stream));
     FH_CHECK_HIP(device_zero(m->idx_dev, off));      // with the fills queued before it, those of model_finalize among them: this is its last step
     return 0;
 }
