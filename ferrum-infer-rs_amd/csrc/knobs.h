@@ -25,6 +25,7 @@ struct Knobs {
     bool attn_no_resident = false;    // never take the resident-K/V short-prompt prefill form
     long attn_resident_min_wgs = 128; // … and only from this many workgroups (tests lower it)
     int attn_flash_rows = 0;          // 64 / 128: forced rows per workgroup of prompt attention (64: each wave on keys of its own)
+    bool no_stream_route = false;     // layered experts: update, router and sorted list in launches of their own
     int attn_key_waves = 0;           // 4 / 8: forced waves per workgroup of the 64-row form
     bool attn_flash32 = false;        // the flash form with 32-key steps (paged_prefill_attn_kernel) for head_dim 128 too
     int rope_quad_rows = 8192;        // split q|k|v, norm, rotation, cache write: four tokens of a head a wave from this many rows of a head
@@ -175,6 +176,7 @@ enum Form : int {
     FORM_DONE_AGAIN,            // a call whose in-launch waits gave up was done again in separate launches
     FORM_ATTN_KEYS,             // prompt attention, each wave of a 64-row workgroup on keys of its own: four waves
     FORM_ATTN_KEYS_WIDE,        // … eight
+    FORM_STREAM_ROUTE,          // layered experts: the update ahead of them, their router and the sorted list in one launch
     FORM_COUNT
 };
 

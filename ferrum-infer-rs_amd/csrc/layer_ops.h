@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <initializer_list>
 
+#include "kernels.h"
 #include "tiled_gemm.h"
 
 namespace fh {
@@ -68,6 +69,20 @@ struct StreamUpdate {
     int rows = 0, dim = 0;
 };
 template <typename E> int stream_update(const StreamUpdate<E>& u, hipStream_t s);
+// A router behind an update of few rows (out is what it reads): logits mul · out · Wᵀ + bias, each row's `top` of the first `experts`, and the pairs sorted by expert, as
+// moe_route_sort_f32 (kernels.h) lists them.
+constexpr int STREAM_ROUTE_MAX = 64;
+template <typename E>
+struct StreamRoute {
+    const E* w = nullptr; const float* bias = nullptr; int n = 0, k = 0, experts = 0, top = 0, block = 0;
+    float mul = 1.f;
+    MoeCorrectedRule rule{};
+    int32_t* ids = nullptr; float* weights = nullptr;
+    int32_t *sorted = nullptr, *block_ids = nullptr, *total = nullptr;
+    unsigned* ticket = nullptr;                   // zero between launches
+};
+template <typename E> bool stream_update_route_supports(const StreamUpdate<E>& u, const StreamRoute<E>& r);
+template <typename E> int stream_update_route(const StreamUpdate<E>& u, const StreamRoute<E>& r, bool corrected, hipStream_t s);
 template <typename E> int copy_rows(const E* x, long ldx, E* out, long ldo, int rows, int cols, hipStream_t s);
 // out[i] = E(rms(x[row_idx[i]]) · w); row_idx null: row i; w null: ones
 template <typename E>

@@ -302,6 +302,7 @@ public:
         FH_TRY(arena_.alloc(&sorted_, sorted));
         FH_TRY(arena_.alloc(&sorted_expert_, pairs));
         FH_TRY(arena_.alloc(&sorted_total_, pairs ? 4 : 0));
+        FH_TRY(arena_.alloc(&route_ticket_, pairs ? 4 : 0));
         FH_TRY(arena_.alloc(&expert_h_, expert_cols));
         FH_TRY(arena_.alloc(&expert_y_, pairs * Dp_));
         FH_TRY(arena_.alloc(&head_in_, (size_t)c_.max_seqs * Dp_));
@@ -497,14 +498,20 @@ private:
                 u.sub2 = sub2_; u.w = L.out1; u.w2 = L.out2;
             }
         }
-        RUN(stream_update(u, s));
+        bool routed = false;
+        if (ff && moe(L.s) && moe_route_sort_supports(T, L.s.experts + L.s.identity_experts, L.s.top)) {
+            const StreamRoute<E> r = stream_route(L, T);
+            routed = !knobs().no_stream_route && stream_update_route_supports(u, r);
+            if (routed) RUN(stream_update_route(u, r, corrected_route(L.s), s));
+        }
+        if (!routed) RUN(stream_update(u, s));
         if (!ff) return 0;
         StreamUpdate<E> f = next;
         if (post_norm()) { f.post_w = L.norm2; f.keep = lc_.stream_mult; }
         if (moe(L.s)) {
             // few tokens: the experts beside the shared one
             const bool shared = L.s.shared_width > 0, beside = shared && few_tokens(run);
-            FH_TRY(beside ? experts_beside(L, run) : experts(L, run));
+            FH_TRY(beside ? experts_beside(L, run, routed) : experts(L, run, routed));
             f.sub = nullptr;
             f.pairs = expert_y_; f.weights = expert_weights_; f.top = L.s.top;
             if (L.s.identity_experts) { f.pair_ids = expert_ids_; f.pair_limit = L.s.experts; }
@@ -560,12 +567,12 @@ private:
 
     bool few_tokens(const Run& run) const { return run.v.T <= knobs().layer_overlap_max_tokens && !run.trace; }
     // the experts on a stream of their own; join_ is recorded behind them
-    int experts_beside(Layer& L, const Run& run) {
+    int experts_beside(Layer& L, const Run& run, bool routed = false) {
         Run other = run;
         other.s = side_stream_;
         FH_CHECK_HIP(hipEventRecord(fork_, run.s));
         FH_CHECK_HIP(hipStreamWaitEvent(side_stream_, fork_, 0));
-        FH_TRY(experts(L, other));
+        FH_TRY(experts(L, other, routed));
         FH_CHECK_HIP(hipEventRecord(join_, side_stream_));
         return 0;
     }
@@ -576,42 +583,64 @@ private:
         r.unlisted = s.identity_experts;
         return r;
     }
-    // expert_y_ [T·top][Dp], expert_weights_ and expert_ids_ [T·top] of the chosen experts
-    int experts(Layer& L, const Run& run) {
-        const int T = run.v.T, E_ = L.s.experts, routed = E_ + L.s.identity_experts, pairs = T * L.s.top;
-        hipStream_t s = run.s;
-        TiledGemm<E> z = linear_f32(L.router, xb_, Dp_, T, router_logits_, routed);
-        z.n_store = routed; z.nsec = 1; z.sec[0] = {0, GEMM_ACT_NONE, 0, 0, L.g2};
-        RUN(tiled_gemm(z, s));
-        auto sorted_rows = [&](int block, int div) {
-            GemmRows r;
-            r.block = block;
-            r.max_blocks = std::min(pairs, pairs / block + std::min(E_, pairs));
-            r.id = sorted_; r.group = sorted_expert_; r.total = sorted_total_;
-            r.div = div;
-            return r;
-        };
+    GemmRows sorted_rows(const Layer& L, int pairs, int block, int div) const {
+        GemmRows r;
+        r.block = block;
+        r.max_blocks = std::min(pairs, pairs / block + std::min(L.s.experts, pairs));
+        r.id = sorted_; r.group = sorted_expert_; r.total = sorted_total_;
+        r.div = div;
+        return r;
+    }
+    // the experts' projections, on sorted rows
+    struct Experts { TiledGemm<E> up, down; };
+    Experts expert_projections(const Layer& L, int T) const {
+        const int pairs = T * L.s.top;
         TiledGemm<E> u = linear(L.up, xb_, Dp_, pairs, expert_h_, L.down.k), y = linear(L.down, expert_h_, L.down.k, pairs, expert_y_, Dp_);
         u.groups = y.groups = 1;
         u.nsec = 1; u.sec[0] = L.ff_sec[0];
-        u.rows = sorted_rows(256, L.s.top); y.rows = sorted_rows(256, 1);
-        const GemmRows rows = sorted_rows(moe_block(pairs, E_, tiled_gemm_takes_256(u) || tiled_gemm_takes_256(y)), 1);
-        u.rows = y.rows = rows;
+        u.rows = sorted_rows(L, pairs, 256, L.s.top); y.rows = sorted_rows(L, pairs, 256, 1);
+        y.rows = u.rows = sorted_rows(L, pairs, moe_block(pairs, L.s.experts, tiled_gemm_takes_256(u) || tiled_gemm_takes_256(y)), 1);
         u.rows.div = L.s.top;
+        return {u, y};
+    }
+    static bool corrected_route(const FerrumHipLayerSpec& s) { return s.ff != FERRUM_HIP_FF_MOE_RELU2; }
+    // the router of a layer's experts behind the update ahead of them
+    StreamRoute<E> stream_route(const Layer& L, int T) const {
+        StreamRoute<E> r;
+        r.w = L.router.w; r.bias = L.router.bias; r.n = L.router.n; r.k = L.router.k; r.mul = L.g2;
+        r.experts = L.s.experts + L.s.identity_experts; r.top = L.s.top;
+        r.block = expert_projections(L, T).up.rows.block;
+        if (corrected_route(L.s)) r.rule = route_rule(L.s, L.correction);
+        r.ids = expert_ids_; r.weights = expert_weights_;
+        r.sorted = sorted_; r.block_ids = sorted_expert_; r.total = sorted_total_;
+        r.ticket = route_ticket_;
+        return r;
+    }
+    // expert_y_ [T·top][Dp], expert_weights_ and expert_ids_ [T·top] of the chosen experts; routed: they have been chosen
+    int experts(Layer& L, const Run& run, bool routed = false) {
+        const int T = run.v.T, E_ = L.s.experts, all = E_ + L.s.identity_experts, pairs = T * L.s.top;
+        hipStream_t s = run.s;
+        const Experts x = expert_projections(L, T);
+        const GemmRows& rows = x.up.rows;
         if (rows.block == 256) form_hit(FORM_MOE_ROWS_256);
-        const bool corrected = L.s.ff != FERRUM_HIP_FF_MOE_RELU2;
-        const MoeCorrectedRule rule = route_rule(L.s, L.correction);
-        if (moe_route_sort_supports(T, routed, L.s.top)) {
-            RUN(moe_route_sort_f32(router_logits_, expert_ids_, expert_weights_, sorted_, sorted_expert_, sorted_total_, T, routed, L.s.top, 1, rows.block, s, corrected ? &rule : nullptr));
-        } else if (corrected) {
-            RUN(moe_route_corrected_f32(router_logits_, rule, expert_ids_, expert_weights_, T, routed, L.s.top, s));
-            RUN(moe_align_block_size(expert_ids_, sorted_, sorted_expert_, sorted_total_, pairs, E_, rows.block, rows.max_blocks * rows.block, s));
-        } else {
-            RUN(moe_route_topk_softmax_f32(router_logits_, expert_ids_, expert_weights_, T, E_, L.s.top, 1, s));
-            RUN(moe_align_block_size(expert_ids_, sorted_, sorted_expert_, sorted_total_, pairs, E_, rows.block, rows.max_blocks * rows.block, s));
+        if (!routed) {
+            TiledGemm<E> z = linear_f32(L.router, xb_, Dp_, T, router_logits_, all);
+            z.n_store = all; z.nsec = 1; z.sec[0] = {0, GEMM_ACT_NONE, 0, 0, L.g2};
+            RUN(tiled_gemm(z, s));
+            const bool corrected = corrected_route(L.s);
+            const MoeCorrectedRule rule = route_rule(L.s, L.correction);
+            if (moe_route_sort_supports(T, all, L.s.top)) {
+                RUN(moe_route_sort_f32(router_logits_, expert_ids_, expert_weights_, sorted_, sorted_expert_, sorted_total_, T, all, L.s.top, 1, rows.block, s, corrected ? &rule : nullptr));
+            } else if (corrected) {
+                RUN(moe_route_corrected_f32(router_logits_, rule, expert_ids_, expert_weights_, T, all, L.s.top, s));
+                RUN(moe_align_block_size(expert_ids_, sorted_, sorted_expert_, sorted_total_, pairs, E_, rows.block, rows.max_blocks * rows.block, s));
+            } else {
+                RUN(moe_route_topk_softmax_f32(router_logits_, expert_ids_, expert_weights_, T, E_, L.s.top, 1, s));
+                RUN(moe_align_block_size(expert_ids_, sorted_, sorted_expert_, sorted_total_, pairs, E_, rows.block, rows.max_blocks * rows.block, s));
+            }
         }
-        RUN(tiled_gemm(u, s));
-        RUN(tiled_gemm(y, s));
+        RUN(tiled_gemm(x.up, s));
+        RUN(tiled_gemm(x.down, s));
         return 0;
     }
     // rows per block of the sorted list: a large block shares an expert's weights between more rows, a small one pads less
@@ -1329,6 +1358,7 @@ private:
       *rnn_out_ = nullptr, *head_in_ = nullptr, *side_ = nullptr, *expert_h_ = nullptr, *expert_y_ = nullptr;
     float *router_logits_ = nullptr, *expert_weights_ = nullptr;
     int32_t *expert_ids_ = nullptr, *sorted_ = nullptr, *sorted_expert_ = nullptr, *sorted_total_ = nullptr;
+    unsigned* route_ticket_ = nullptr;       // zero between launches
     size_t partial_bytes_ = 0;
     // expansion of keys and values: one plan per distinct window
     std::vector<Plan> plans_;

@@ -1,6 +1,8 @@
 // Residual stream of the layered models: fp32 throughout, with a copy in the projections' number format written by whoever changes it.
 #include "common.h"
+#include "knobs.h"
 #include "layer_ops.h"
+#include "route_device.h"
 
 namespace fh {
 
@@ -291,9 +293,9 @@ int rms_norm_rows(const float* x, const int32_t* row_idx, const float* w, float 
 }
 
 // One workgroup per row; a thread holds VEC quads of the row in registers (0: any length, from memory).  POST: the sum itself is normed.
+// `copy`: the row in the number format goes there, too.
 template <typename E, int VEC, bool POST>
-__global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) {
-    __shared__ float red[64];
+__device__ __forceinline__ void stream_update_row(const StreamUpdate<E>& u, float* red, E* copy) {
     const long row = blockIdx.x;
     const int dim = u.dim, nt = blockDim.x;
     const float *s1 = u.sub + row * u.ld_sub, *s2 = u.sub2 + row * u.ld_sub;
@@ -431,6 +433,7 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
 #pragma unroll
                 for (int k = 0; k < 4; k++) o[k] = (E)(xv[c][k] * unit * wn[c][k]);
                 *reinterpret_cast<e4*>(out + i) = o;
+                if (copy) *reinterpret_cast<e4*>(copy + i) = o;
             }
         }
         return;
@@ -481,17 +484,131 @@ __global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) 
     const float unit = u.next_w ? 1.0f / sqrtf(block_sum<VEC == 1>(n, red + 32) / (float)dim + u.eps) : 1.0f;
     for (int i = threadIdx.x; i < dim; i += nt) out[i] = (E)(u.next_w ? xr[i] * unit * u.next_w[i] : xr[i]);
 }
+template <typename E, int VEC, bool POST>
+__global__ __launch_bounds__(1024) void stream_update_kernel(StreamUpdate<E> u) {
+    __shared__ float red[64];
+    stream_update_row<E, VEC, POST>(u, red, nullptr);
+}
+
+// An update whose rows a router reads next, the router's logits, each row's choice of experts, and by the workgroup that comes last the sorted list of the pairs: one
+// launch for three.  A workgroup has its row in LDS and the first of the router's weights, requested ahead of the row, in registers; a wave takes every nw-th step of K
+// of all experts as the first operand of the matrix instruction (the row's numbers are alike in all columns), and the waves' sums meet in LDS.
+// The ids cross workgroups within the launch: written and read past the caches, behind a ticket that the last one puts back.
+// Bound by latency: update, router and list of 32 rows of 2048 on 24 experts 4.8 + 5 + 10.5 µs in launches of their own, of which two of three are on the way to the first
+// load of each; a step of four such layers 665 → 628 µs, of two layers of 2 rows on 30 experts 226 → 221.
+template <typename E, bool POST, bool CORRECTED>
+__global__ __launch_bounds__(1024) void stream_update_route_kernel(StreamUpdate<E> u, StreamRoute<E> r) {
+    constexpr int EP = 16 / sizeof(E), SK = 4 * EP, AHEAD = 4, N = STREAM_ROUTE_MAX;
+    typedef E piece __attribute__((ext_vector_type(EP)));
+    __shared__ __attribute__((aligned(16))) E row_lds[4096];
+    __shared__ float red[64], part[16][N], logits[N];
+    __shared__ int16_t hist[16][N];
+    __shared__ int32_t offset[N];
+    __shared__ int last;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+    const int a = lane >> 4, b = lane & 15, steps = r.k / SK, tiles = r.n >> 4;
+    auto weights = [&](int t, int s) { return *reinterpret_cast<const piece*>(r.w + ((long)t * steps + s) * (64 * EP) + lane * EP); };
+    piece ahead[2][AHEAD];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) ahead[t][j] = weights(t, min(wave + j * nw, steps - 1));
+    for (int i = u.dim + threadIdx.x; i < r.k; i += blockDim.x) row_lds[i] = (E)0.f;
+    stream_update_row<E, 1, POST>(u, red, row_lds);
+    __syncthreads();
+    floatx4 acc[N / 16];
+#pragma unroll
+    for (int t = 0; t < N / 16; t++) acc[t] = (floatx4){0.f, 0.f, 0.f, 0.f};
+    auto numbers = [&](int s) { return *reinterpret_cast<const piece*>(row_lds + s * SK + a * EP); };
+#pragma unroll
+    for (int j = 0; j < AHEAD; j++) {
+        const int s = wave + j * nw;
+        if (s >= steps) continue;
+        const piece x = numbers(s);
+#pragma unroll
+        for (int t = 0; t < N / 16; t++)
+            if (t < 2) acc[t] = Frag<E>::mma(ahead[t < 2 ? t : 0][j], x, acc[t]);
+            else if (t < tiles) acc[t] = Frag<E>::mma(weights(t, s), x, acc[t]);
+    }
+    for (int s = wave + AHEAD * nw; s < steps; s += nw) {
+        const piece x = numbers(s);
+#pragma unroll
+        for (int t = 0; t < N / 16; t++)
+            if (t < tiles) acc[t] = Frag<E>::mma(weights(t, s), x, acc[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < N / 16; t++)
+        if (b == 0 && t < tiles) *reinterpret_cast<floatx4*>(&part[wave][16 * t + 4 * a]) = acc[t];
+    __syncthreads();
+    const long row = blockIdx.x;
+    if (wave == 0) {
+        if (lane < r.experts) {
+            float sum = 0.f;
+            for (int w = 0; w < nw; w++) sum += part[w][lane];
+            logits[lane] = sum * r.mul + (r.bias ? r.bias[lane] : 0.f);
+        }
+        __builtin_amdgcn_wave_barrier();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        int id;
+        float w;
+        if (CORRECTED) route_token_corrected<1>(logits, lane, r.experts, r.top, r.rule, id, w);
+        else route_token<1>(logits, lane, r.experts, r.top, 1, id, w);
+        if (lane < r.top) {
+            __hip_atomic_store(r.ids + row * r.top + lane, id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            r.weights[row * r.top + lane] = w;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (lane == 0) {
+            last = __hip_atomic_fetch_add(r.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+            if (last) __hip_atomic_store(r.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    __syncthreads();
+    if (!last) return;
+    const int pairs = u.rows * r.top, listed = r.experts - (CORRECTED ? r.rule.unlisted : 0);
+    route_sort_pairs<N>([&] { return (int)threadIdx.x < pairs ? __hip_atomic_load(r.ids + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : -1; }, pairs, listed,
+                        r.block, r.sorted, r.block_ids, r.total, hist, offset);
+}
+template <typename E>
+static int update_threads(const StreamUpdate<E>& u) { return u.rows <= 512 && u.dim >= 2048 ? 1024 : 256; }
+template <typename E>
+static int update_quads(const StreamUpdate<E>& u) {
+    const int threads = update_threads(u);
+    const bool vec = u.dim % 4 == 0 && u.dim <= threads * 16 && u.ld_sub % 4 == 0 && u.ld_pair % 4 == 0 && u.ldo % 4 == 0 && u.slab_stride % 4 == 0 && u.slab_stride2 % 4 == 0;
+    return !vec ? 0 : u.dim <= threads * 4 ? 1 : u.dim <= threads * 8 ? 2 : 4;
+}
 template <typename E>
 int stream_update(const StreamUpdate<E>& u, hipStream_t s) {
     FH_REQUIRE(!u.sub2 || (u.sub && u.w && u.w2 && !u.top), "stream update: a second branch needs both norms");
     FH_REQUIRE(u.sub || u.slabs == 1, "stream update: slabs of nothing");
     FH_REQUIRE(u.post_w ? !u.sub2 : u.keep == 1.f && !u.pair_ids && !u.sub_scale && !u.gate, "stream update: factors and the stream's own pairs belong to a normed sum of one branch");
-    const int threads = u.rows <= 512 && u.dim >= 2048 ? 1024 : 256;
-    const bool vec = u.dim % 4 == 0 && u.dim <= threads * 16 && u.ld_sub % 4 == 0 && u.ld_pair % 4 == 0 && u.ldo % 4 == 0 && u.slab_stride % 4 == 0 && u.slab_stride2 % 4 == 0;
-    const int quads = !vec ? 0 : u.dim <= threads * 4 ? 1 : u.dim <= threads * 8 ? 2 : 4;
+    const int threads = update_threads(u), quads = update_quads(u);
 #define UPDATE(V, P) hipLaunchKernelGGL((stream_update_kernel<E, V, P>), dim3(u.rows), dim3(threads), 0, s, u)
     if (u.post_w) { if (quads == 1) UPDATE(1, true); else if (quads == 2) UPDATE(2, true); else if (quads) UPDATE(4, true); else UPDATE(0, true); }
     else { if (quads == 1) UPDATE(1, false); else if (quads == 2) UPDATE(2, false); else if (quads) UPDATE(4, false); else UPDATE(0, false); }
+#undef UPDATE
+    FH_CHECK_LAUNCH();
+    return 0;
+}
+
+// (a quad of the row a thread, a thread a pair)
+template <typename E>
+bool stream_update_route_supports(const StreamUpdate<E>& u, const StreamRoute<E>& r) {
+    return update_quads(u) == 1 && u.out && u.dim <= r.k && r.k <= 4096 && r.k % 32 == 0 && r.n <= STREAM_ROUTE_MAX && r.n % 32 == 0 && r.experts <= r.n && u.rows * r.top <= update_threads(u);
+}
+template <typename E>
+int stream_update_route(const StreamUpdate<E>& u, const StreamRoute<E>& r, bool corrected, hipStream_t s) {
+    FH_REQUIRE(stream_update_route_supports(u, r) && u.rows > 0 && r.top > 0 && r.top <= r.experts && r.block > 0 && r.ticket, "stream update with a router: %d rows of %d, %d of %d experts",
+               u.rows, u.dim, r.top, r.experts);
+    FH_REQUIRE(!corrected || moe_route_corrected_supports(r.experts, r.top, r.rule), "stream update with a router: %d groups, %d kept", r.rule.groups, r.rule.keep);
+    FH_REQUIRE(!u.sub2 || (u.sub && u.w && u.w2 && !u.top), "stream update: a second branch needs both norms");
+    FH_REQUIRE(u.sub || u.slabs == 1, "stream update: slabs of nothing");
+    FH_REQUIRE(u.post_w ? !u.sub2 : u.keep == 1.f && !u.pair_ids && !u.sub_scale && !u.gate, "stream update: factors and the stream's own pairs belong to a normed sum of one branch");
+    form_hit(FORM_STREAM_ROUTE);
+    form_hit(FORM_MOE_ROUTE_SORT);
+#define UPDATE(P, C) hipLaunchKernelGGL((stream_update_route_kernel<E, P, C>), dim3(u.rows), dim3(update_threads(u)), 0, s, u, r)
+    if (u.post_w) { if (corrected) UPDATE(true, true); else UPDATE(true, false); }
+    else { if (corrected) UPDATE(false, true); else UPDATE(false, false); }
 #undef UPDATE
     FH_CHECK_LAUNCH();
     return 0;
@@ -504,6 +621,8 @@ int stream_update(const StreamUpdate<E>& u, hipStream_t s) {
                                   int, hipStream_t);                                                                                    \
     template int copy_rows<E>(const E*, long, E*, long, int, int, hipStream_t);                                                          \
     template int stream_update<E>(const StreamUpdate<E>&, hipStream_t);                                                                  \
+    template bool stream_update_route_supports<E>(const StreamUpdate<E>&, const StreamRoute<E>&);                                        \
+    template int stream_update_route<E>(const StreamUpdate<E>&, const StreamRoute<E>&, bool, hipStream_t);                               \
     template int rms_norm_rows<E>(const float*, const int32_t*, const float*, float, E*, int, int, int, hipStream_t);
 INSTANTIATE(bf16)
 INSTANTIATE(float)

@@ -338,6 +338,24 @@ def test_grouped_experts_alone(pkg, tmp_path, forms, dtype, n, top, ff, groups, 
     assert bool(h.get("moe_route_sort")) == (tokens * top <= 1024) and bool(h.get("route_grouped")) == (tokens * top > 1024)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,n,top,groups,keep,tokens,fused", [(2080, 24, 8, 8, 4, 32, True), (4096, 33, 3, 3, 2, 128, True), (72, 64, 2, 4, 2, 128, True), (1024, 7, 4, 1, 1, 64, True),
+                                                                  (1024, 7, 4, 1, 1, 65, False), (4100, 16, 2, 2, 1, 5, False), (512, 66, 2, 6, 3, 9, False)])
+def test_update_router_and_sorted_list_in_one_launch(pkg, tmp_path, knobs, forms, dtype, width, n, top, groups, keep, tokens, fused):
+    """4 and 16 waves, rows that end inside a step, two and four tiles of experts, as many pairs as threads; against the same in launches of their own.  Choices with a margin, so
+    that the logits' order of summation (32-bit sums of `width` products: 1e-6 of their size) decides none; the stream then differs by the rounding of weights."""
+    cfg = model([G.scan(8, 2, 2, 2, mlp=G.grouped_experts(n, top, 32, groups, keep, 1.4))], width=width)
+    w = G.weights(cfg, 91, clear_routes=False)
+    w["l0.mlp.correction"] = G.bf16(8.0 * np.random.default_rng(5).permutation(n) - 4.0 * n)
+    taps = []
+    for off in (None, 1):
+        knobs.set(NO_STREAM_ROUTE=off)
+        forms.reset()
+        taps.append(taps_of(pkg, tmp_path, cfg, w, dtype, toks(cfg, tokens, 6)))
+        assert bool(forms.hits().get("stream_route")) == (fused and not off)
+    assert rel(taps[0], taps[1]) < {"float32": 2e-6, "bfloat16": 2.0 ** -9}[dtype]
+
+
 MISTAKES = {"weights read the correction": lambda s, c: s + c, "excluded choices are 0": None, "a group counts by its best": None, "choice without the correction": None}
 
 
