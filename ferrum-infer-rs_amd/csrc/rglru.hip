@@ -5,7 +5,7 @@
 //
 // The two gate projections of a channel are computed side by side on the matrix cores (tiles interleaved ra, ri), so one lane holds
 // both gates of its (token, channel) and everything from the sigmoids to the state update stays in fp32 registers.  1 − a² is taken as
-// 1 − e^(2 log a) by a series where it would cancel.  One token per sequence: that launch also updates the state and writes the output.  Portions: decay and drive go to
+// 1 − e^(2 log a) by a series where it would cancel.  One token per sequence: that launch also updates the state and writes the output, for blocks of up to 128 channels behind the convolution too.  Portions: decay and drive go to
 // memory and a chunked scan (64 tokens per workgroup; chunk totals, carry over chunks, final pass) produces the output.
 // A sequence's first token starts from zero whatever its slot holds, so slots are reused without clearing.
 #include "common.h"
@@ -80,6 +80,86 @@ __global__ __launch_bounds__(256) void rglru_gates_kernel(RglruDims d, RglruBuff
         }
 }
 
+// One token a sequence: convolution, gates, state and output of 16 rows × a block of up to 128 channels in a workgroup, which is the only one to touch these channels' stored
+// inputs.  The gates' weights (64 KiB, in 32 bits 128) are requested ahead of the convolution, whose results its waves, a 16-channel tile each, read from LDS.
+// Bound by latency: one row of 2048 channels in 16 blocks 3.7 + 4.0 µs in two launches → 4.4, four rows in 32 bits 4.6 + 8.0 → 7.1; a step of six layers, four of them such, 314 → 299 µs,
+// of three in 32 bits with two 291 → 280; 32 rows of three layers 230 → 213 and 387 → 366.
+constexpr int STEP_BLOCK = 128, STEP_TAPS = 4;
+template <typename E>
+__global__ __launch_bounds__(512) void rglru_step_kernel(RglruDims d, RglruBuffers<E> p, BatchView v) {
+    constexpr int EP = 16 / sizeof(E), SK = 4 * EP, KS = STEP_BLOCK / SK, PITCH = STEP_BLOCK + EP;
+    typedef E piece_t __attribute__((ext_vector_type(EP)));
+    typedef typename Frag<E>::v8 v8;
+    __shared__ __attribute__((aligned(16))) E u_lds[16 * PITCH];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, a = lane >> 4, b = lane & 15;
+    const int g = blockIdx.x, row0 = blockIdx.y * 16, ksteps = d.bp / SK;       // (a wave for each 16 channels)
+    const E* wr = p.gate_w + ((long)(g * (d.bp >> 4) + wave) * 2) * ksteps * (64 * EP) + lane * EP;
+    piece_t w[2][KS];
+#pragma unroll
+    for (int s = 0; s < KS; s++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) w[h][s] = *reinterpret_cast<const piece_t*>(wr + (long)(h * ksteps + min(s, ksteps - 1)) * (64 * EP));
+    const int c = g * d.bp + wave * 16 + b;
+    const float bra = p.ra_b[c], bri = p.ri_b[c], sp = p.lam[c];
+    float state[4], y[4];
+    float* at[4];
+    bool first[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int row = min(row0 + 4 * a + q, v.T - 1);                        // (token i belongs to sequence i)
+        at[q] = p.state + (long)v.slots[row] * d.wp + c;
+        first[q] = v.pos[row] == 0;
+        state[q] = *at[q];
+        y[q] = (float)p.y[(long)row * p.ld + c];
+    }
+    const ShortConv<E> conv = rglru_conv(d, p);
+    const int per = d.bp >> 3;
+    for (int i = threadIdx.x; i < 16 * per; i += blockDim.x) {
+        const int r = i / per, cc = (i - r * per) * 8, ch = g * d.bp + cc, tok = row0 + r;
+        if (tok >= v.T) break;
+        const int slot = v.slots[tok];
+        const bool fresh = v.pos[tok] == 0;
+        v8 in[STEP_TAPS];                                                      // (of the token `back` ago; 0: this one)
+#pragma unroll
+        for (int back = 0; back < STEP_TAPS; back++) in[back] = conv_input(conv, tok, 0, min(back, conv.taps - 1), slot, fresh, ch);
+        float acc[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) acc[k] = conv.b[ch + k];
+#pragma unroll
+        for (int back = STEP_TAPS - 1; back >= 0; back--)
+            if (back < conv.taps)
+#pragma unroll
+                for (int k = 0; k < 8; k++) acc[k] += conv.w[(long)(conv.taps - 1 - back) * conv.wp + ch + k] * (float)in[back][k];
+        v8 o;
+#pragma unroll
+        for (int k = 0; k < 8; k++) o[k] = (E)acc[k];
+        *reinterpret_cast<v8*>(u_lds + r * PITCH + cc) = o;
+#pragma unroll
+        for (int back = 0; back < STEP_TAPS - 1; back++)                       // (entry j: the input taps − 2 − j tokens back)
+            if (back < conv.taps - 1) *reinterpret_cast<v8*>(conv.state + ((long)slot * (conv.taps - 1) + conv.taps - 2 - back) * conv.wp + ch) = in[back];
+    }
+    __syncthreads();
+    floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int s = 0; s < KS; s++) {
+        if (s >= ksteps) break;
+        const piece_t ax = *reinterpret_cast<const piece_t*>(u_lds + b * PITCH + s * SK + EP * a);
+#pragma unroll
+        for (int h = 0; h < 2; h++) acc[h] = Frag<E>::mma(ax, w[h][s], acc[h]);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+        const int r = 4 * a + q, row = row0 + r;
+        if (row >= v.T) continue;
+        const float gate = gate_sigmoid(acc[0][q] + bra), in = gate_sigmoid(acc[1][q] + bri);
+        const float log_a = -8.0f * gate * sp, decay = __expf(log_a);
+        const float drive = __builtin_amdgcn_sqrtf(one_minus_exp(2.0f * log_a)) * in * (float)u_lds[r * PITCH + wave * 16 + b];
+        const float h = first[q] ? drive : decay * state[q] + drive;
+        *at[q] = h;
+        p.out[(long)row * d.wp + c] = (E)(h * y[q]);
+    }
+}
+
 // totals of every chunk that another chunk of its sequence follows: Π decay and the state it would reach from zero
 template <typename E>
 __global__ __launch_bounds__(256) void rglru_chunk_totals_kernel(RglruDims d, RglruBuffers<E> p, BatchView v) {
@@ -143,6 +223,13 @@ __global__ __launch_bounds__(256) void rglru_apply_kernel(RglruDims d, RglruBuff
 template <typename E>
 int rglru_forward(const RglruDims& d, const RglruBuffers<E>& b, const BatchView& v, hipStream_t s) {
     const int cb = cdiv(d.wp, 256);
+    // a wave for every 16 channels and the inputs in registers: wider blocks and longer convolutions take the two launches
+    if (v.single && d.bp <= STEP_BLOCK && d.taps <= STEP_TAPS) {
+        form_hit(FORM_RGLRU_STEP);
+        hipLaunchKernelGGL(rglru_step_kernel<E>, dim3(d.blocks, cdiv(v.T, 16)), dim3(4 * d.bp), 0, s, d, b, v);
+        FH_CHECK_LAUNCH();
+        return 0;
+    }
     if (int rc = short_conv(rglru_conv(d, b), v, s)) return rc;
     const int mt = v.T <= 16 ? 1 : (v.T <= 32 ? 2 : 4);
     // prompts: the waves of a workgroup share the rows they read; steps: one wave per workgroup, spread over the CUs

@@ -143,6 +143,26 @@ def test_recurrence_alone(pkg, tmp_path, dtype, i):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width,blocks,conv,rows", [(96, 3, 1, 1), (128, 1, 2, 15), (256, 2, 4, 16), (200, 2, 3, 17), (129, 1, 4, 33), (32, 1, 5, 17)])
+def test_recurrence_a_token_at_a_time(pkg, tmp_path, dtype, width, blocks, conv, rows):
+    """Sequences from their first token on, longer than the convolution and at unequal positions: blocks of 32, 64 and 128 channels (one launch) and of more, 1 to 4 taps and 5,
+    rows that end on either side of a tile.  Logits round as those of whole models do; the slots were used before."""
+    cfg = one_layer(G.recurrent(width, blocks, conv))
+    w, n = G.weights(cfg, 34), 7
+    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), dtype, seqs=rows)
+    for turn in range(2):
+        t = [toks(cfg, n, 40 + 64 * turn + i) for i in range(rows)]
+        got = [[] for _ in t]
+        for s in range(n + 2):
+            on = [i for i in range(rows) if 0 <= s - i % 3 < n]
+            for i, lg in zip(on, m.forward_rows([(i, t[i][s - i % 3:s - i % 3 + 1], s - i % 3) for i in on], list(range(len(on)))) if on else []):
+                got[i].append(lg)
+        assert all(rel(got[i], L.forward(cfg, w, t[i])) < TOL[dtype] for i in range(rows))
+        for i in range(rows):
+            m.release(i)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("ff", [41, 160])
 def test_feed_forward_alone(pkg, tmp_path, dtype, ff):
     """norm1 = −1 erases the mixer's contribution: what remains is the gated, normed feed-forward with its piecewise activation."""
