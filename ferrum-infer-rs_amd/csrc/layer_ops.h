@@ -15,6 +15,7 @@ struct BatchView {
     int T = 0, num_seqs = 0, max_blocks = 0;
     int max_keys = 0;                            // longest context of the batch, new tokens included (upper bound)
     bool single = false;                         // every sequence brings one token
+    bool all_sampled = false;                    // … and the head takes every row, in order
     const uint32_t* tokens = nullptr;            // [T]
     const uint32_t* cu = nullptr;                // [num_seqs + 1]
     const uint32_t* pos = nullptr;               // [num_seqs] position of a sequence's first new token
@@ -31,23 +32,26 @@ struct BatchView {
 
 // ── residual stream (residual_stream.hip) ──
 // x = factor · embed[token] (+ bigram[(prev·mul_prev + token·mul_cur) mod buckets], or the extra row for a first token) (+ positions[position]),
-// fp32; xb = E(x)
+// fp32; xb = E(x), with norm E(rms(x) · norm_w) (norm_w null: ones) and E(x) to raw where it is given
 template <typename E>
 struct Embedding {
     const E *table = nullptr, *bigram = nullptr, *positions = nullptr;
     int buckets = 0;
     int64_t mul_prev = 0, mul_cur = 0;
-    float factor = 1.f;
+    float factor = 1.f, eps = 0.f;
+    bool norm = false;
+    const float* norm_w = nullptr;
+    E* raw = nullptr; long ld_raw = 0;
 };
 template <typename E> int embed_tokens(const Embedding<E>& e, const BatchView& v, float* x, E* xb, int dim, int ldb, hipStream_t s);
 // x += sub + Σ_j weights[row][j] · pairs[row·top + j] (top 0: none); xb = E(x); sub is the sum of `slabs` partial sums
 template <typename E>
 int branch_add(const float* sub, long ld_sub, int slabs, long slab_stride, const E* pairs, long ld_pair, const float* weights, int top, float* x, E* xb,
                int rows, int dim, int ldb, hipStream_t s);
-// x += mult · rms(sub · gate) · w (gate null: none); xb = E(x), with next_norm E(rms(x)); sub is the sum of `slabs` partial sums
+// x += mult · rms(sub · gate) · w (gate null: none); xb = E(x), with next_norm E(rms(x) · next_w) (next_w null: ones); sub is the sum of `slabs` partial sums
 template <typename E>
 int post_norm_add(const float* sub, long ld_sub, int slabs, long slab_stride, const E* gate, long ld_gate, const float* w, float mult, float eps, bool next_norm,
-                  float* x, E* xb, int rows, int dim, int ldb, hipStream_t s);
+                  const float* next_w, float* x, E* xb, int rows, int dim, int ldb, hipStream_t s);
 // Blocks whose sublayers follow one another: x ← [keep · x +] branch + add + Σ_j weights[row][j] · pairs[row·top + j], where the branch is sub, or with a second one the mean
 // (sub·rms⁻¹·w + sub2·rms⁻¹·w2) / 2; with post_w x ← rms(x) · post_w; then out = E(rms(x) · next_w), or E(x) without next_w.  sub and sub2 are sums
 // of `slabs` partial sums.  With post_w only: sub is taken times sub_scale[row], pairs with an id of pair_limit or more stand for the stream itself,
@@ -83,7 +87,6 @@ struct StreamRoute {
 };
 template <typename E> bool stream_update_route_supports(const StreamUpdate<E>& u, const StreamRoute<E>& r);
 template <typename E> int stream_update_route(const StreamUpdate<E>& u, const StreamRoute<E>& r, bool corrected, hipStream_t s);
-template <typename E> int copy_rows(const E* x, long ldx, E* out, long ldo, int rows, int cols, hipStream_t s);
 // out[i] = E(rms(x[row_idx[i]]) · w); row_idx null: row i; w null: ones
 template <typename E>
 int rms_norm_rows(const float* x, const int32_t* row_idx, const float* w, float eps, E* out, int rows, int dim, int ldo, hipStream_t s);

@@ -21,7 +21,7 @@ public:
     virtual int layer_runs() const = 0;           // layers in the order they run, looped ones once per pass
     // embedding and every layer; taps: [layer_runs()][max_tokens][hidden] or null
     virtual int forward(const BatchView& v, float* taps, bool trace, hipStream_t s) = 0;
-    // final norm + vocabulary projection of `rows` rows of the last forward
+    // final norm + vocabulary projection of `rows` rows of the last forward; row_idx null: all of them, in order, of a forward with all_sampled
     virtual int head(const int32_t* row_idx, int rows, float* logits, hipStream_t s) = 0;
     virtual bool has_state() const = 0;           // some layer carries recurrent state
     virtual bool reads_previous_token() const = 0;

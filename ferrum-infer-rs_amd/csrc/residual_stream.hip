@@ -6,56 +6,6 @@
 
 namespace fh {
 
-template <typename E, bool VEC>
-__global__ __launch_bounds__(256) void embed_kernel(Embedding<E> p, BatchView v, float* __restrict__ x, E* __restrict__ xb, int dim, int ldb) {
-    const int t = blockIdx.x;
-    const uint32_t tok = v.tokens[t];
-    const E *own = p.table + (long)tok * dim, *bigram = nullptr, *place = nullptr;
-    if (p.bigram || p.positions) {
-        const int seq = v.tok_seq[t], at = t - (int)v.cu[seq];
-        if (p.bigram) {
-            const int64_t prev = at == 0 ? (int64_t)v.prev[seq] : (int64_t)v.tokens[t - 1];
-            bigram = p.bigram + dim * (prev < 0 ? (long)p.buckets : (long)(((uint64_t)prev * (uint64_t)p.mul_prev + (uint64_t)tok * (uint64_t)p.mul_cur) % (uint64_t)p.buckets));
-        }
-        if (p.positions) place = p.positions + (long)(v.pos[seq] + at) * dim;
-    }
-    if (VEC) {
-        typedef typename Frag<E>::v8 v8;
-        for (int i = threadIdx.x * 8; i < dim; i += 2048) {
-            const v8 e = *reinterpret_cast<const v8*>(own + i);
-            v8 g = e, l = e, o;
-            if (bigram) g = *reinterpret_cast<const v8*>(bigram + i);
-            if (place) l = *reinterpret_cast<const v8*>(place + i);
-            floatx4 f[2];
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const float y = (float)e[j] * p.factor + (bigram ? (float)g[j] : 0.f) + (place ? (float)l[j] : 0.f);
-                f[j >> 2][j & 3] = y;
-                o[j] = (E)y;
-            }
-            *reinterpret_cast<floatx4*>(x + (long)t * dim + i) = f[0];
-            *reinterpret_cast<floatx4*>(x + (long)t * dim + i + 4) = f[1];
-            *reinterpret_cast<v8*>(xb + (long)t * ldb + i) = o;
-        }
-        return;
-    }
-    for (int i = threadIdx.x; i < dim; i += 256) {
-        float e = (float)own[i] * p.factor;
-        if (bigram) e += (float)bigram[i];
-        if (place) e += (float)place[i];
-        x[(long)t * dim + i] = e;
-        xb[(long)t * ldb + i] = (E)e;
-    }
-}
-
-template <typename E>
-int embed_tokens(const Embedding<E>& e, const BatchView& v, float* x, E* xb, int dim, int ldb, hipStream_t s) {
-    if (dim % 8 == 0) hipLaunchKernelGGL((embed_kernel<E, true>), dim3(v.T), dim3(256), 0, s, e, v, x, xb, dim, ldb);
-    else hipLaunchKernelGGL((embed_kernel<E, false>), dim3(v.T), dim3(256), 0, s, e, v, x, xb, dim, ldb);
-    FH_CHECK_LAUNCH();
-    return 0;
-}
-
 // AT_ONCE: the waves' sums read together, for launches whose time is latency; of many rows the loop is no slower and leaves 16 registers (2048 × 2048 9.1, not 10.4 µs)
 template <bool AT_ONCE = true>
 __device__ __forceinline__ float block_sum(float q, float* red) {
@@ -74,6 +24,94 @@ __device__ __forceinline__ float block_sum(float q, float* red) {
     for (int i = 0; i < 16; i++) t += i < (int)(blockDim.x >> 6) ? r[i] : 0.f;
     return t;
 }
+
+// One workgroup per token.  VEC 1: a thread's 8 numbers stay in registers for the norm of the first block's input; 2: several such pieces, read back from x; 0: any length.
+template <typename E, int VEC>
+__global__ __launch_bounds__(256) void embed_kernel(Embedding<E> p, BatchView v, float* __restrict__ x, E* __restrict__ xb, int dim, int ldb) {
+    __shared__ float red[16];
+    const int t = blockIdx.x;
+    float* xr = x + (long)t * dim;
+    E *br = xb + (long)t * ldb, *raw = p.raw + (long)t * p.ld_raw;
+    const uint32_t tok = v.tokens[t];
+    const E *own = p.table + (long)tok * dim, *bigram = nullptr, *place = nullptr;
+    if (p.bigram || p.positions) {
+        const int seq = v.tok_seq[t], at = t - (int)v.cu[seq];
+        if (p.bigram) {
+            const int64_t prev = at == 0 ? (int64_t)v.prev[seq] : (int64_t)v.tokens[t - 1];
+            bigram = p.bigram + dim * (prev < 0 ? (long)p.buckets : (long)(((uint64_t)prev * (uint64_t)p.mul_prev + (uint64_t)tok * (uint64_t)p.mul_cur) % (uint64_t)p.buckets));
+        }
+        if (p.positions) place = p.positions + (long)(v.pos[seq] + at) * dim;
+    }
+    float q = 0.f;
+    if constexpr (VEC > 0) {
+        typedef typename Frag<E>::v8 v8;
+        floatx4 f[2], w[2] = {{1.f, 1.f, 1.f, 1.f}, {1.f, 1.f, 1.f, 1.f}};
+        const int mine = threadIdx.x * 8;
+        if (VEC == 1 && p.norm_w && mine < dim) {
+            w[0] = *reinterpret_cast<const floatx4*>(p.norm_w + mine);
+            w[1] = *reinterpret_cast<const floatx4*>(p.norm_w + mine + 4);
+        }
+        for (int i = mine; i < dim; i += 2048) {
+            const v8 e = *reinterpret_cast<const v8*>(own + i);
+            v8 g = e, l = e, o;
+            if (bigram) g = *reinterpret_cast<const v8*>(bigram + i);
+            if (place) l = *reinterpret_cast<const v8*>(place + i);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const float y = (float)e[j] * p.factor + (bigram ? (float)g[j] : 0.f) + (place ? (float)l[j] : 0.f);
+                f[j >> 2][j & 3] = y;
+                q += y * y;
+                o[j] = (E)y;
+            }
+            *reinterpret_cast<floatx4*>(xr + i) = f[0];
+            *reinterpret_cast<floatx4*>(xr + i + 4) = f[1];
+            if (p.raw) *reinterpret_cast<v8*>(raw + i) = o;
+            if (!p.norm) *reinterpret_cast<v8*>(br + i) = o;
+            if (VEC == 1) break;
+        }
+        if (!p.norm) return;
+        const float inv = 1.0f / sqrtf(block_sum<VEC == 1>(q, red) / (float)dim + p.eps);
+        for (int i = mine; i < dim; i += 2048) {
+            if (VEC != 1) {                                       // (a thread's own numbers)
+                f[0] = *reinterpret_cast<const floatx4*>(xr + i);
+                f[1] = *reinterpret_cast<const floatx4*>(xr + i + 4);
+                if (p.norm_w) {
+                    w[0] = *reinterpret_cast<const floatx4*>(p.norm_w + i);
+                    w[1] = *reinterpret_cast<const floatx4*>(p.norm_w + i + 4);
+                }
+            }
+            v8 o;
+#pragma unroll
+            for (int j = 0; j < 8; j++) o[j] = (E)(f[j >> 2][j & 3] * inv * w[j >> 2][j & 3]);
+            *reinterpret_cast<v8*>(br + i) = o;
+            if (VEC == 1) break;
+        }
+        return;
+    }
+    for (int i = threadIdx.x; i < dim; i += 256) {
+        float e = (float)own[i] * p.factor;
+        if (bigram) e += (float)bigram[i];
+        if (place) e += (float)place[i];
+        xr[i] = e;
+        q += e * e;
+        if (p.raw) raw[i] = (E)e;
+        if (!p.norm) br[i] = (E)e;
+    }
+    if (!p.norm) return;
+    const float inv = 1.0f / sqrtf(block_sum<false>(q, red) / (float)dim + p.eps);
+    for (int i = threadIdx.x; i < dim; i += 256) br[i] = (E)(p.norm_w ? xr[i] * inv * p.norm_w[i] : xr[i] * inv);
+}
+
+template <typename E>
+int embed_tokens(const Embedding<E>& e, const BatchView& v, float* x, E* xb, int dim, int ldb, hipStream_t s) {
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(v.T), dim3(256), 0, s, e, v, x, xb, dim, ldb); };
+    if (dim % 8) go(embed_kernel<E, 0>);
+    else if (dim <= 2048) go(embed_kernel<E, 1>);
+    else go(embed_kernel<E, 2>);
+    FH_CHECK_LAUNCH();
+    return 0;
+}
+
 // Σ over the slabs of a branch, in their order; TOGETHER: two, or up to four, are under way at once (one after the other each cost a round trip, 0.7 µs)
 template <bool TOGETHER = true>
 __device__ __forceinline__ floatx4 sum_slabs(const float* p, int slabs, long stride) {
@@ -147,14 +185,14 @@ int branch_add(const float* sub, long ld_sub, int slabs, long slab_stride, const
 }
 
 // One workgroup per row; a thread holds VEC quads of the row in registers (0: any length, from memory), so the branch is read once.  NEXT: the copy is the row
-// divided by its root mean square, the input of a block that norms ahead of its sublayers.
+// divided by its root mean square, times next_w where there is one: the input of a block that norms ahead of its sublayers, or of the head.
 // One quad a thread (decode, and narrow rows): latency alone, so everything is requested at once, what the first sum does not need ahead of it.  Of
 // several quads the row's own are requested first, and what is not needed yet does not take registers (all at once: rows of 6144 in two slabs
 // 3.6 → 4.2 µs, 512 of them 7.7 → 9.1; the update below 1024 × 4096 8.5 → 15.5, 8192 × 2880 43 → 100).
 template <typename E, int VEC, bool GATE, bool NEXT>
 __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __restrict__ sub, long ld_sub, int slabs, long slab_stride, const E* __restrict__ gate,
                                                              long ld_gate, const float* __restrict__ w, float mult, float eps,
-                                                             float* __restrict__ x, E* __restrict__ xb, int dim, int ldb) {
+                                                             const float* __restrict__ next_w, float* __restrict__ x, E* __restrict__ xb, int dim, int ldb) {
     __shared__ float red[32];
     const long row = blockIdx.x;
     const float* sr = sub + row * ld_sub;
@@ -164,7 +202,7 @@ __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __rest
     float q = 0.f, n = 0.f;
     if constexpr (VEC > 0) {
         typedef E e4 __attribute__((ext_vector_type(4)));
-        floatx4 v[VEC ? VEC : 1], xv[VEC ? VEC : 1], wv[VEC ? VEC : 1];
+        floatx4 v[VEC ? VEC : 1], xv[VEC ? VEC : 1], wv[VEC ? VEC : 1], wn = {1.f, 1.f, 1.f, 1.f};
 #pragma unroll
         for (int c = 0; c < VEC; c++) {
             const int i = (c * blockDim.x + threadIdx.x) * 4;
@@ -174,6 +212,7 @@ __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __rest
                     wv[c] = *reinterpret_cast<const floatx4*>(w + i);
                 };
                 if (VEC == 1) rest();
+                if (VEC == 1 && NEXT && next_w) wn = *reinterpret_cast<const floatx4*>(next_w + i);
                 e4 gv = {};
                 if (GATE && VEC == 1) gv = *reinterpret_cast<const e4*>(gr + i);
                 v[c] = sum_slabs<VEC == 1>(sr + i, slabs, slab_stride);
@@ -198,9 +237,10 @@ __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __rest
         for (int c = 0; c < VEC; c++) {
             const int i = (c * blockDim.x + threadIdx.x) * 4;
             if (i < dim) {
+                if (VEC != 1 && NEXT && next_w) wn = *reinterpret_cast<const floatx4*>(next_w + i);
                 e4 o;
 #pragma unroll
-                for (int j = 0; j < 4; j++) o[j] = (E)(xv[c][j] * unit);
+                for (int j = 0; j < 4; j++) o[j] = (E)(NEXT ? xv[c][j] * unit * wn[j] : xv[c][j]);
                 *reinterpret_cast<e4*>(br + i) = o;
             }
         }
@@ -221,35 +261,24 @@ __global__ __launch_bounds__(1024) void post_norm_add_kernel(const float* __rest
     }
     if (NEXT) {
         const float unit = 1.0f / sqrtf(block_sum<VEC == 1>(n, red + 16) / (float)dim + eps);
-        for (int i = threadIdx.x; i < dim; i += blockDim.x) br[i] = (E)(xr[i] * unit);
+        for (int i = threadIdx.x; i < dim; i += blockDim.x) br[i] = (E)(next_w ? xr[i] * unit * next_w[i] : xr[i] * unit);
     }
 }
 
 template <typename E>
 int post_norm_add(const float* sub, long ld_sub, int slabs, long slab_stride, const E* gate, long ld_gate, const float* w, float mult, float eps, bool next_norm,
-                  float* x, E* xb, int rows, int dim, int ldb, hipStream_t s) {
+                  const float* next_w, float* x, E* xb, int rows, int dim, int ldb, hipStream_t s) {
     const int threads = rows <= 512 && dim >= 2048 ? 1024 : 256;
     const bool vec = dim % 4 == 0 && dim <= threads * 16 && ld_sub % 4 == 0 && ld_gate % 4 == 0 && ldb % 4 == 0 && slab_stride % 4 == 0;
     auto go = [&](auto v, auto g, auto n) {
         hipLaunchKernelGGL((post_norm_add_kernel<E, decltype(v)::value, decltype(g)::value, decltype(n)::value>), dim3(rows), dim3(threads), 0, s, sub, ld_sub, slabs,
-                           slab_stride, gate, ld_gate, w, mult, eps, x, xb, dim, ldb);
+                           slab_stride, gate, ld_gate, w, mult, eps, next_w, x, xb, dim, ldb);
     };
     auto with_next = [&](auto v, auto g) { next_norm ? go(v, g, std::true_type{}) : go(v, g, std::false_type{}); };
     auto with_gate = [&](auto v) { gate ? with_next(v, std::true_type{}) : with_next(v, std::false_type{}); };
     if (!vec) with_gate(std::integral_constant<int, 0>{});
     else if (dim <= threads * 4) with_gate(std::integral_constant<int, 1>{});
     else with_gate(std::integral_constant<int, 4>{});
-    FH_CHECK_LAUNCH();
-    return 0;
-}
-
-template <typename E>
-__global__ __launch_bounds__(256) void copy_rows_kernel(const E* __restrict__ x, long ldx, E* __restrict__ out, long ldo, int cols) {
-    for (int i = threadIdx.x; i < cols; i += 256) out[blockIdx.x * ldo + i] = x[blockIdx.x * ldx + i];
-}
-template <typename E>
-int copy_rows(const E* x, long ldx, E* out, long ldo, int rows, int cols, hipStream_t s) {
-    hipLaunchKernelGGL(copy_rows_kernel<E>, dim3(rows), dim3(256), 0, s, x, ldx, out, ldo, cols);
     FH_CHECK_LAUNCH();
     return 0;
 }
@@ -617,9 +646,8 @@ int stream_update_route(const StreamUpdate<E>& u, const StreamRoute<E>& r, bool 
 #define INSTANTIATE(E)                                                                                                                  \
     template int embed_tokens<E>(const Embedding<E>&, const BatchView&, float*, E*, int, int, hipStream_t);                              \
     template int branch_add<E>(const float*, long, int, long, const E*, long, const float*, int, float*, E*, int, int, int, hipStream_t); \
-    template int post_norm_add<E>(const float*, long, int, long, const E*, long, const float*, float, float, bool, float*, E*, int, int, \
-                                  int, hipStream_t);                                                                                    \
-    template int copy_rows<E>(const E*, long, E*, long, int, int, hipStream_t);                                                          \
+    template int post_norm_add<E>(const float*, long, int, long, const E*, long, const float*, float, float, bool, const float*, float*, \
+                                  E*, int, int, int, hipStream_t);                                                                      \
     template int stream_update<E>(const StreamUpdate<E>&, hipStream_t);                                                                  \
     template bool stream_update_route_supports<E>(const StreamUpdate<E>&, const StreamRoute<E>&);                                        \
     template int stream_update_route<E>(const StreamUpdate<E>&, const StreamRoute<E>&, bool, hipStream_t);                               \

@@ -1499,6 +1499,7 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
     if (m->layered) {
         BatchView v;
         v.T = sh.m_total; v.num_seqs = sh.num_seqs; v.max_blocks = m->max_blocks_per_seq; v.max_keys = sh.max_kv_len; v.single = sh.all_single_token;
+        v.all_sampled = sh.num_sampled == sh.m_total;            // (of sequences of several tokens no more than one is)
         v.tokens = idx<uint32_t>(m, m->il.tokens); v.cu = idx<uint32_t>(m, m->il.cu_seqlens); v.pos = idx<uint32_t>(m, m->il.pos_offsets);
         v.bt = idx<int32_t>(m, m->il.block_tables); v.tok_seq = idx<int32_t>(m, m->il.tok_seq); v.prev = idx<int32_t>(m, m->il.prev_tokens);
         v.slots = idx<int32_t>(m, m->il.state_slots); v.units = idx<int32_t>(m, m->il.scan_units); v.num_units = m->batch_units;
@@ -2008,13 +2009,13 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
     return 0;
 }
 
-// final norm + lm_head on the rows listed in the index block (same rows the reference packs, qwen3_moe_forward_unified.rs:365-392)
-int enqueue_head(FerrumHipModel* m, int rows) {
+// final norm + lm_head on the rows listed in the index block (same rows the reference packs, qwen3_moe_forward_unified.rs:365-392); all: they are every row of the forward, in order
+int enqueue_head(FerrumHipModel* m, int rows, bool all) {
     const FerrumHipModelConfig& c = m->cfg;
     hipStream_t s = m->stream;
     const int32_t* sampled_idx = idx<int32_t>(m, m->il.sampled_idx);
     if (knobs().trace_launches) fprintf(stderr, "[ferrum_hip] head rows=%d\n", rows);
-    if (m->layered) return m->layered->head(sampled_idx, rows, m->logits, s);
+    if (m->layered) return m->layered->head(all ? nullptr : sampled_idx, rows, m->logits, s);
     if (c.sandwich_norms) {
         if (int rc = rms_norm_f32_to_f16(m->residual_f32, sampled_idx, m->final_norm, c.rms_eps, m->sampled_hidden, rows, c.hidden, s)) return rc;
     } else {
@@ -2034,7 +2035,7 @@ int enqueue_forward(FerrumHipModel* m, const StepShape& sh, bool greedy, const G
     hipStream_t s = m->stream;
     if (int rc = enqueue_body(m, sh)) return rc;
     if (sh.num_sampled > 0) {
-        if (int rc = enqueue_head(m, sh.num_sampled)) return rc;
+        if (int rc = enqueue_head(m, sh.num_sampled, sh.num_sampled == sh.m_total)) return rc;
         int rc;
         const bool trace = knobs().trace_launches;
 #define RUN(x)                                                                       \
@@ -2215,7 +2216,7 @@ static int forward_batch(FerrumHipModel* m, const FerrumHipBatchItem* items, int
             const int n = std::min(c.max_seqs, num_rows - r0);
             memcpy(h_samp, rows + r0, (size_t)n * 4);
             FH_CHECK_HIP(hipMemcpyAsync(m->idx_dev + m->il.sampled_idx, h_samp, (size_t)n * 4, hipMemcpyHostToDevice, m->stream));
-            if (int rc = enqueue_head(m, n)) return rc;
+            if (int rc = enqueue_head(m, n, false)) return rc;
             if (int rc = copy_results(m, logits_out + (size_t)r0 * m->vp_n, m->logits, (size_t)n * m->vp_n * 4)) return rc;
         }
         uint8_t* ids = m->results + RESULT_RING * RESULT_PORTION;

@@ -114,6 +114,30 @@ def test_rows_of_several_quads_a_thread(pkg, tmp_path, dtype, width, n):
     assert rel(taps_of(pkg, tmp_path, cfg, w, dtype, t), taps) < TOL[dtype]
 
 
+ENDS = {"nerenex": lambda w: G.config(w, 50, [G.recurrent(24, 2, 2, ff=33), G.attention(2, 8, 4, 8, 16, 24, 7)]),
+        "nerenex with a feed-forward": lambda w: G.config(w, 50, [G.attention(2, 8, 4, 8, 16, 24, 7), G.recurrent(24, 2, 2, ff=33)]),
+        "safolorn": lambda w: G.safolorn(w, 50, 12, [G.sink_attention(2, 8, 4, 8, 24, mlp=G.glu(30, 0.7))]),
+        "segetar": lambda w: G.segetar(w, 50, [G.scan(24, 2, 1, 2, mlp=G.dense(30))]),
+        "a loop behind a layer": lambda w: G.segetar(w, 50, [G.scan(24, 2, 1, 2, mlp=G.dense(30)), G.scan(16, 2, 1, 2)], (1, 2, 2)),
+        "a loop": lambda w: G.segetar(w, 50, [G.scan(24, 2, 1, 2, mlp=G.dense(30)), G.scan(16, 2, 1, 2)], (0, 1, 2)),
+        "fororax": lambda w: G.fororax(w, 50, [G.far_attention(2, 1, 8, 8, mlp=G.identity_experts(3, 1, 2, 9, 33))])}
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [72, 45, 2056])
+@pytest.mark.parametrize("name", list(ENDS))
+def test_norms_of_the_first_layer_and_of_the_head(pkg, tmp_path, name, width, dtype):
+    """Steps whose rows all go to the head, which the last update norms, against the same steps with listed rows, which the head norms itself: numbers of the format that differ
+    by their last place where 32-bit sums do, so logits by no more than two of its roundings; and both against the oracle.  Rows of one piece a thread, of none and of several."""
+    cfg = ENDS[name](width)
+    w, t = G.weights(cfg, 23), toks(cfg, 9, 8)
+    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), dtype)
+    got = [np.concatenate([m.unified_forward([(s, t[i:i + 1], i, True) for s in (1, 2)], want_logits=True)[1] for i in range(len(t))])]
+    got.append(np.concatenate([m.forward_rows([(s, t[i:i + 1], i) for s in (3, 4)], [0, 1]) for i in range(len(t))]))
+    assert rel(got[0], got[1]) < {"float32": 2e-6, "bfloat16": 2.0 ** -7}[dtype]
+    assert rel(got[0], np.repeat(L.forward(cfg, w, t), 2, axis=0)) < TOL[dtype]
+
+
 ATTN = [G.attention(3, 20, 6, 36, 44, 52, 9, base=300.0), G.attention(16, 32, 16, 32, 32, 64, 40), G.attention(5, 64, 34, 17, 33, 130, 25, scale=0.3),
         G.attention(1, 5, 2, 3, 4, 7, 2), G.attention(33, 16, 8, 24, 20, 385, 64), G.attention(2, 130, 70, 140, 16, 520, 30)]
 
