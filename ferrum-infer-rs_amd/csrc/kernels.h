@@ -56,6 +56,10 @@ int w4_gemm_rows_splits(const W4Device& w, int m, size_t slab_bytes);
 int w4_gemm_rows(const W4Device& w, const __half* x, float* slabs, size_t slab_bytes, int m, int* S_out, int* rows_pad_out, int* n_pad_out,
                  hipStream_t stream);
 bool f16t_gemm_gated_supports(const W4Device& w, int im);
+// a prompt's q|k|v that norms, rotates and stores its rows itself (qkv_rows.h)
+struct QkvRows;
+bool f16t_gemm_qkv_supports(const W4Device& w, const __half* x, const QkvRows& to);
+int f16t_gemm_qkv(const W4Device& w, const __half* x, const QkvRows& to, hipStream_t stream);
 int f16t_gemm_gated(const W4Device& w, const __half* x, __half* out, int m, int im, int gelu, hipStream_t stream);
 bool w4_gemm_gated_supports(const W4Device& w, int m, int im);
 int w4_gemm_gated(const W4Device& w, const __half* x, __half* out, int m, int im, int gelu, hipStream_t stream);

@@ -28,6 +28,7 @@ struct Knobs {
     bool no_stream_route = false;     // layered experts: update, router and sorted list in launches of their own
     int attn_key_waves = 0;           // 4 / 8: forced waves per workgroup of the 64-row form
     bool attn_flash32 = false;        // the flash form with 32-key steps (paged_prefill_attn_kernel) for head_dim 128 too
+    int qkv_min_tiles = 256;           // unquantised q|k|v of a prompt with norm, rotation and cache write in its launch from this many tiles of 128 × 128
     int rope_quad_rows = 8192;        // split q|k|v, norm, rotation, cache write: four tokens of a head a wave from this many rows of a head
     // INT4 GEMMs (w4_gemm.hip)
     int moe_kw_pairs = 16;
@@ -176,6 +177,7 @@ enum Form : int {
     FORM_DONE_AGAIN,            // a call whose in-launch waits gave up was done again in separate launches
     FORM_ATTN_KEYS,             // prompt attention, each wave of a 64-row workgroup on keys of its own: four waves
     FORM_ATTN_KEYS_WIDE,        // … eight
+    FORM_F16_QKV,               // unquantised q|k|v of a prompt, normed, rotated and stored by its launch
     FORM_STREAM_ROUTE,          // layered experts: the update ahead of them, their router and the sorted list in one launch
     FORM_COUNT
 };

@@ -8,8 +8,7 @@
 #include "common.h"
 #include "kernels.h"
 #include "knobs.h"
-#include "kv_layout.h"
-#include "rope_rows.h"
+#include "qkv_rows.h"
 
 namespace fh {
 
@@ -23,95 +22,50 @@ namespace fh {
 //   (32 + 2·8) × 256    8: 4.7 | 3.3    128: 5.6 | 4.8    192: 6.2 | 5.8    256: 6.6 | 7.0    1024: 15.7 | 17.5
 //   (8 + 2·2) × 128     8: 3.3 | 2.7    512: 3.8 | 3.8    768: 4.3 | 4.3   1024: 4.3 | 4.9
 template <int HD, bool QUADS>
-__global__ __launch_bounds__(QUADS ? 256 : 64) void split_qkv_norm_rope_paged_kernel(
-    const __half* __restrict__ qkv, const __half* __restrict__ q_norm_w, const __half* __restrict__ k_norm_w,
-    const float* __restrict__ cos_t, const float* __restrict__ sin_t, __half* __restrict__ q_out,
-    __half* __restrict__ cache_k, __half* __restrict__ cache_v, const uint32_t* __restrict__ cu_seqlens_q,
-    const uint32_t* __restrict__ pos_offsets, const int32_t* __restrict__ block_tables, int num_seqs, int m_total,
-    int q_heads, int kv_heads, float eps, int qk_mode, int max_blocks_per_seq) {
-    constexpr int PPL = HD / 32, HALF = HD / 2;
+__global__ __launch_bounds__(QUADS ? 256 : 64) void split_qkv_norm_rope_paged_kernel(const __half* __restrict__ qkv, QkvRows p) {
+    constexpr int HALF = HD / 2;
     constexpr int TOKENS = QUADS ? 4 : 1;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, q16 = lane & 15, quarter = lane >> 4;
-    const int heads = q_heads + 2 * kv_heads, head_raw = blockIdx.y * 4 + (QUADS ? wave : quarter), head = min(head_raw, heads - 1);
+    const int heads = p.q_heads + 2 * p.kv_heads, head_raw = blockIdx.y * 4 + (QUADS ? wave : quarter), head = min(head_raw, heads - 1);
     if (QUADS && head_raw >= heads) return;
-    const int tok0 = blockIdx.x * TOKENS, tok = QUADS ? min(tok0 + quarter, m_total - 1) : tok0;         // clamped: loads stay unconditional
-    const bool act = QUADS ? tok0 + quarter < m_total : head_raw < heads;
-    const int q_dim = q_heads * HD, kv_dim = kv_heads * HD;
+    const int tok0 = blockIdx.x * TOKENS, tok = QUADS ? min(tok0 + quarter, p.m_total - 1) : tok0;         // clamped: loads stay unconditional
+    const bool act = QUADS ? tok0 + quarter < p.m_total : head_raw < heads;
+    const int q_dim = p.q_heads * HD, kv_dim = p.kv_heads * HD;
     const __half* row = qkv + (long)tok * (q_dim + 2 * kv_dim);
 
     // locate the sequences: the last s with cu_seqlens_q[s] ≤ tok (what the reference kernel's linear scan returns), found
     // 64 sequences per memory round trip — a serial scan costs the tokens of the 32nd prompt 31 dependent loads
     int seq4[4] = {0, 0, 0, 0};
-    for (int s0 = 0; s0 < num_seqs; s0 += 64) {
+    for (int s0 = 0; s0 < p.num_seqs; s0 += 64) {
         const int s = s0 + lane;
-        const uint32_t first = s < num_seqs ? cu_seqlens_q[s] : 0xffffffffu;
+        const uint32_t first = s < p.num_seqs ? p.cu[s] : 0xffffffffu;
         unsigned long long le = 0;
 #pragma unroll
         for (int j = 0; j < TOKENS; j++) {
-            le = __ballot(first <= (uint32_t)min(tok0 + j, m_total - 1));
+            le = __ballot(first <= (uint32_t)min(tok0 + j, p.m_total - 1));
             if (le) seq4[j] = s0 + 63 - __clzll((long long)le);
         }
         if (le != ~0ull) break;                              // (the last token's is the largest set)
     }
     const int seq = !QUADS || quarter == 0 ? seq4[0] : quarter == 1 ? seq4[1] : quarter == 2 ? seq4[2] : seq4[3];
-    const int pos = (int)pos_offsets[seq] + (tok - (int)cu_seqlens_q[seq]);
+    const int pos = (int)p.pos_offsets[seq] + (tok - (int)p.cu[seq]);
 
-    const bool is_q = head < q_heads;
-    const bool is_k = !is_q && head < q_heads + kv_heads;
-    const int local_head = is_q ? head : is_k ? head - q_heads : head - q_heads - kv_heads;
+    const bool is_q = head < p.q_heads;
+    const bool is_k = !is_q && head < p.q_heads + p.kv_heads;
+    const int local_head = is_q ? head : is_k ? head - p.q_heads : head - p.q_heads - p.kv_heads;
     const __half* src = row + (is_q ? 0 : is_k ? q_dim : q_dim + kv_dim) + local_head * HD;
-    const int mode = (is_q || is_k) ? qk_mode : 0;
-    const RopeRow<HD> rr = rope_row16<HD>(src, is_q ? q_norm_w : k_norm_w, cos_t + (long)pos * HALF, sin_t + (long)pos * HALF,
-                                          mode, qk_mode == 1, qk_mode != 0, eps, q16);
-    using hv = typename RopeRow<HD>::hv;
-    if (is_q) {
-        if (!act) return;
-        __half* dst = q_out + ((long)tok * q_heads + local_head) * HD;
-        *reinterpret_cast<hv*>(dst + rr.off0) = rr.out0;
-        *reinterpret_cast<hv*>(dst + rr.off1) = rr.out1;
-        return;
-    }
-    const int logical = pos / KV_BLOCK, slot = pos % KV_BLOCK;
-    const long physical = block_tables[(long)seq * max_blocks_per_seq + logical];
-    __half* tile = (is_k ? cache_k : cache_v) + (physical * kv_heads + local_head) * kv_tile_elems(HD);
-    _Float16* t16 = reinterpret_cast<_Float16*>(tile);
-    if (is_k) {                                              // (PPL dimensions of a row lie within one chunk of eight)
-        if (!act) return;
-        *reinterpret_cast<hv*>(t16 + k_tile_off(slot, rr.off0)) = rr.out0;
-        *reinterpret_cast<hv*>(t16 + k_tile_off(slot, rr.off1)) = rr.out1;
-        return;
-    }
-    if constexpr (QUADS && HD == 128) {
-        const int pos_first = __builtin_amdgcn_readfirstlane(pos);
-        if (tok0 + 3 < m_total && seq4[0] == seq4[3] && pos_first % 4 == 0) {
-            // quarter t holds token t's dimensions off0 … + 3 and off1 … + 3, as four pairs; quarter r leaves with pair r of all four tokens
-            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-            const u32x2 lo = __builtin_bit_cast(u32x2, rr.out0), hi = __builtin_bit_cast(u32x2, rr.out1);
-            uint32_t from[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int pair = (quarter + i) & 3;          // quarter t sends the pair of quarter t + i
-                const uint32_t mine = pair == 0 ? lo[0] : pair == 1 ? lo[1] : pair == 2 ? hi[0] : hi[1];
-                from[i] = i == 0 ? mine : (uint32_t)__shfl((int)mine, ((quarter - i) & 3) * 16 + q16, 64);
-            }
-            uint32_t key[4];                                 // from[i] is of token (quarter − i) mod 4
-#pragma unroll
-            for (int t = 0; t < 4; t++) {
-                const int i = (quarter - t) & 3;
-                key[t] = i == 0 ? from[0] : i == 1 ? from[1] : i == 2 ? from[2] : from[3];
-            }
-            const int d = (quarter < 2 ? rr.off0 : rr.off1) + 2 * (quarter & 1);
-            *reinterpret_cast<u32x2*>(t16 + v_tile_off(slot & ~3, d)) = (u32x2){(key[0] & 0xffff) | key[1] << 16, (key[2] & 0xffff) | key[3] << 16};
-            *reinterpret_cast<u32x2*>(t16 + v_tile_off(slot & ~3, d + 1)) = (u32x2){key[0] >> 16 | (key[1] & 0xffff0000u), key[2] >> 16 | (key[3] & 0xffff0000u)};
-            return;
-        }
-    }
-    if (!act) return;
-#pragma unroll
-    for (int k = 0; k < PPL; k++) {
-        t16[v_tile_off(slot, rr.off0 + k)] = rr.out0[k];
-        t16[v_tile_off(slot, rr.off1 + k)] = rr.out1[k];
-    }
+    const int mode = (is_q || is_k) ? p.qk_mode : 0;
+    const bool quad = QUADS && tok0 + 3 < p.m_total && seq4[0] == seq4[3] && __builtin_amdgcn_readfirstlane(pos) % 4 == 0;
+    const long physical = is_q ? 0 : p.block_tables[(long)seq * p.max_blocks + pos / KV_BLOCK];
+    auto row_of = [&](auto m) {
+        constexpr int MODE = decltype(m)::value;
+        const RopeRow<HD> rr = rope_row16<HD>(src, is_q ? p.q_norm_w : p.k_norm_w, p.cos_t + (long)pos * HALF, p.sin_t + (long)pos * HALF,
+                                              MODE, MODE == 1, MODE != 0, p.eps, q16);
+        qkv_store_row<HD>(rr, p, is_q, is_k, local_head, tok, pos, physical, act, quad, q16, quarter);
+    };
+    if (QUADS) qkv_with_mode(mode, row_of);
+    else if (mode) qkv_with_mode(p.qk_mode, row_of);         // (heads of a wave differ: queries and keys, then values)
+    else row_of(std::integral_constant<int, 0>{});
 }
 
 int split_qkv_norm_rope_into_paged_cache_varlen_f16(
@@ -125,10 +79,9 @@ int split_qkv_norm_rope_into_paged_cache_varlen_f16(
     FH_REQUIRE(qk_mode >= 0 && qk_mode <= 3, "paged KV: qk_mode=%d out of range", qk_mode);
     const bool quads = (long)m_total * (q_heads + 2 * kv_heads) >= knobs().rope_quad_rows;
     const dim3 grid(quads ? cdiv(m_total, 4) : m_total, cdiv(q_heads + 2 * kv_heads, 4));
-#define FH_ROPE(HDV, QUADS)                                                                                            \
-    hipLaunchKernelGGL((split_qkv_norm_rope_paged_kernel<HDV, QUADS>), grid, dim3(QUADS ? 256 : 64), 0, s, qkv, q_norm_w, k_norm_w, cos_t, \
-                       sin_t, q_out, cache_k, cache_v, cu_seqlens_q, pos_offsets, block_tables, num_seqs, m_total, q_heads, kv_heads, eps, \
-                       qk_mode, max_blocks_per_seq)
+    const QkvRows p{q_norm_w, k_norm_w, cos_t, sin_t, q_out, cache_k, cache_v, cu_seqlens_q, pos_offsets, block_tables, num_seqs, m_total, q_heads, kv_heads, eps, qk_mode,
+                    max_blocks_per_seq};
+#define FH_ROPE(HDV, QUADS) hipLaunchKernelGGL((split_qkv_norm_rope_paged_kernel<HDV, QUADS>), grid, dim3(QUADS ? 256 : 64), 0, s, qkv, p)
     if (quads) { if (head_dim == 64) FH_ROPE(64, true); else if (head_dim == 128) FH_ROPE(128, true); else FH_ROPE(256, true); }
     else { if (head_dim == 64) FH_ROPE(64, false); else if (head_dim == 128) FH_ROPE(128, false); else FH_ROPE(256, false); }
 #undef FH_ROPE

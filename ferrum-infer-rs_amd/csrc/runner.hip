@@ -13,6 +13,7 @@
 
 #include "runner.h"
 #include "knobs.h"
+#include "qkv_rows.h"
 #include "tp_comm.h"
 
 #include <chrono>
@@ -1728,14 +1729,6 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
             }
             continue;
         }
-        if (pending_tail) {
-            RUN(w4_gemm_dense(L.qkv, nullptr, m->qkv_out, T, m->workspace, m->workspace_bytes, s, &tail));
-            pending_tail = false;
-        } else {
-            RUN(dense_linear(m, L.qkv, m->norm_out, m->qkv_out, T, s, qkv_in_perm));
-        }
-        qkv_in_perm = false;
-        bool attn_perm = false;          // attn_out holds the row in L.o's packed order
         // per-layer attention schedule (llama_layer_attention_schedule, llama_family.rs:1028-1045)
         const int pattern = c.sliding_window_pattern;
         const bool is_global = pattern == 0 || (li + 1) % pattern == 0;
@@ -1743,7 +1736,22 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
         const float* cos_l = (!is_global && m->cos_local) ? m->cos_local : m->cos_t;
         const float* sin_l = (!is_global && m->sin_local) ? m->sin_local : m->sin_t;
         const bool layer_decode = sh.pure_decode && layer_window == 0;
-        if (sh.all_single_token && m->fuse_rope_attn && nq / nkv <= 14) {
+        const bool fused_qkv = sh.all_single_token && m->fuse_rope_attn && nq / nkv <= 14;          // norm, rotation and cache write in the attention launch
+        const QkvRows rows{L.q_norm ? L.q_norm : dummy, L.k_norm ? L.k_norm : dummy, cos_l, sin_l, m->q_out, L.k_pool, L.v_pool, cu, pos, bt, sh.num_seqs, T, nq, nkv, c.rms_eps,
+                           qk_mode, m->max_blocks_per_seq};
+        bool split = fused_qkv;          // the rows of q|k|v are where they belong, or will be
+        if (pending_tail) {
+            RUN(w4_gemm_dense(L.qkv, nullptr, m->qkv_out, T, m->workspace, m->workspace_bytes, s, &tail));
+            pending_tail = false;
+        } else if (!split && hd == 128 && f16t_gemm_qkv_supports(L.qkv, m->norm_out, rows)) {
+            RUN(f16t_gemm_qkv(L.qkv, m->norm_out, rows, s));
+            split = true;
+        } else {
+            RUN(dense_linear(m, L.qkv, m->norm_out, m->qkv_out, T, s, qkv_in_perm));
+        }
+        qkv_in_perm = false;
+        bool attn_perm = false;          // attn_out holds the row in L.o's packed order
+        if (fused_qkv) {
             // decode: QK-norm + RoPE + KV write happen in the attention kernel's prologue (one launch fewer)
             RUN(paged_decode_attention_fused_qkv_f16(m->qkv_out, L.q_norm ? L.q_norm : dummy, L.k_norm ? L.k_norm : dummy,
                                                      cos_l, sin_l, c.rms_eps, qk_mode, L.k_pool, L.v_pool, m->attn_out,
@@ -1751,10 +1759,11 @@ int enqueue_body(FerrumHipModel* m, const StepShape& sh) {
                                                      m->max_blocks_per_seq, m->workspace, m->workspace_bytes, s, L.o.inv_perm));
             attn_perm = L.o.perm != nullptr;
         } else {
-            RUN(split_qkv_norm_rope_into_paged_cache_varlen_f16(m->qkv_out, L.q_norm ? L.q_norm : dummy,
-                                                                L.k_norm ? L.k_norm : dummy, cos_l, sin_l, m->q_out,
-                                                                L.k_pool, L.v_pool, cu, pos, bt, sh.num_seqs, T, nq, nkv, hd,
-                                                                c.rms_eps, qk_mode, KV_BLOCK, m->max_blocks_per_seq, s));
+            if (!split)
+                RUN(split_qkv_norm_rope_into_paged_cache_varlen_f16(m->qkv_out, L.q_norm ? L.q_norm : dummy,
+                                                                    L.k_norm ? L.k_norm : dummy, cos_l, sin_l, m->q_out,
+                                                                    L.k_pool, L.v_pool, cu, pos, bt, sh.num_seqs, T, nq, nkv, hd,
+                                                                    c.rms_eps, qk_mode, KV_BLOCK, m->max_blocks_per_seq, s));
             if (layer_decode) {
                 RUN(paged_batched_decode_attention_f16(m->q_out, L.k_pool, L.v_pool, m->attn_out, bt, kvl, sh.num_seqs,
                                                        sh.max_kv_len, nq, nkv, hd, KV_BLOCK, m->max_blocks_per_seq,

@@ -96,6 +96,10 @@ struct TiledGemm {
 template <typename E> int tiled_gemm(const TiledGemm<E>& g, hipStream_t s);
 // whether a launch of many rows runs in tiles of 256 × 256, which want blocks of 256 sorted rows
 template <typename E> bool tiled_gemm_takes_256(const TiledGemm<E>& g);
+// A prompt's q|k|v projection whose launch norms, rotates and stores the rows itself (heads of 128 columns; qkv_rows.h)
+struct QkvRows;
+bool tiled_gemm_qkv_supports(const TiledGemm<_Float16>& g, const QkvRows& to);
+int tiled_gemm_qkv(const TiledGemm<_Float16>& g, const QkvRows& to, hipStream_t s);
 // number of K parts worth making for a projection of m rows whose consumer sums slabs (≤ GEMM_MAX_SLABS)
 constexpr int GEMM_MAX_SLABS = 4;
 int tiled_gemm_slabs(int m, int n, int k);

@@ -6,6 +6,7 @@
 
 #include "common.h"
 #include "knobs.h"
+#include "qkv_rows.h"
 #include "tiled_gemm.h"
 #include "tiled_gemm_device.h"
 
@@ -258,8 +259,10 @@ struct BigTile {
     static_assert(MI % 2 == 0 && (NJ == 2 || NJ == 4 || NJ == 8), "every wave copies whole fragments");
     static_assert(LDS >= (size_t)4 * 32 * (16 * NJ + 4) * 4, "the epilogue's rows fit the stages");
 };
-template <typename E, int MI, int NJ, int G, int PER_CU>
-__global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E> p, int mtiles, int ntiles) {
+// Rows: what the launch does with its rows besides (RowsAsTheyAre: nothing; QkvRows: the q|k|v of heads of 128 columns, normed, rotated and stored).
+struct RowsAsTheyAre {};
+template <typename E, int MI, int NJ, int G, int PER_CU, typename Rows>
+__global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E> p, int mtiles, int ntiles, Rows to) {
     typedef BigTile<MI, NJ, G> T;
     typedef typename Frag<E>::v8 v8;
     constexpr bool F32 = sizeof(E) == 4;
@@ -391,6 +394,58 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     // complete in order), then a lane finishes 8 columns of a row: bias, activation and factors, and rows leave in 16-byte pieces.  In a
     // gated section the lanes of the up tiles have nothing to do, those of the gate tiles read both.
     __syncthreads();
+    if constexpr (std::is_same<Rows, QkvRows>::value) {
+        // The tile as fp16, which is what a launch of its own would read, in LDS, whole heads of it; where a row goes is found out once for all heads.  Four tokens of a head a
+        // wave and turn, as there.
+        constexpr int PITCH = T::COLS + 8, TURNS = T::ROWS / 16;
+        static_assert(!F32 && T::COLS % 128 == 0 && (size_t)T::ROWS * (PITCH * 2 + 12) <= T::LDS, "whole heads, and their rows fit the stages");
+        _Float16* tile = reinterpret_cast<_Float16*>(smem);
+        int *pos_of = reinterpret_cast<int*>(tile + T::ROWS * PITCH), *block_of = pos_of + T::ROWS, *seq_of = block_of + T::ROWS;
+#pragma unroll
+        for (int i = 0; i < MI; i++)
+#pragma unroll
+            for (int j = 0; j < NJ; j++) *reinterpret_cast<f16x4*>(tile + ((wm * MI + i) * 16 + b) * PITCH + (wn * NJ + j) * 16 + 4 * a) = __builtin_convertvector(acc[i][j] + 0.f, f16x4);      // (− 0 → 0, as the sum with a bias that is none)
+        if ((int)threadIdx.x < T::ROWS) {                                // (whole waves)
+            const int tok = min(m0 + (int)threadIdx.x, to.m_total - 1);
+            int seq = 0;                                                 // the last whose first token is not behind this one
+            for (int s0 = 0; s0 < to.num_seqs; s0 += 64) {
+                const int first = (int)to.cu[min(s0 + lane, to.num_seqs - 1)], some = min(64, to.num_seqs - s0);
+                for (int j = 0; j < some; j++)
+                    if (__builtin_amdgcn_readlane(first, j) <= tok) seq = s0 + j;
+            }
+            const int pos = (int)to.pos_offsets[seq] + (tok - (int)to.cu[seq]);
+            pos_of[threadIdx.x] = pos;
+            seq_of[threadIdx.x] = seq;
+            block_of[threadIdx.x] = to.block_tables[(long)seq * to.max_blocks + pos / KV_BLOCK];
+        }
+        __syncthreads();
+        const int row0 = wave * (T::ROWS / 4) + a;                       // a quarter's first row
+#pragma unroll 1
+        for (int h = 0; h < T::COLS / 128; h++) {
+            const int head = n0 / 128 + h;
+            if (head >= to.q_heads + 2 * to.kv_heads) break;
+            const bool is_q = head < to.q_heads, is_k = !is_q && head < to.q_heads + to.kv_heads;
+            const int local = is_q ? head : is_k ? head - to.q_heads : head - to.q_heads - to.kv_heads, mode = is_q || is_k ? to.qk_mode : 0;
+            qkv_with_mode(mode, [&](auto m) {
+                constexpr int MODE = decltype(m)::value;
+                RopeCoef<128> coef[TURNS];
+#pragma unroll
+                for (int u = 0; u < TURNS; u++) {
+                    const long at = (long)pos_of[row0 + 4 * u] * 64;
+                    coef[u] = rope_coef16<128>(is_q ? to.q_norm_w : to.k_norm_w, to.cos_t + at, to.sin_t + at, MODE, MODE == 1, MODE != 0, b);
+                }
+#pragma unroll
+                for (int u = 0; u < TURNS; u++) {
+                    const int r = row0 + 4 * u, r0 = __builtin_amdgcn_readfirstlane(r), tok = m0 + r;
+                    const RopeRow<128> rr = rope_row16<128>(rope_source16<128>(reinterpret_cast<const __half*>(tile + r * PITCH + h * 128), MODE, b), coef[u], MODE, to.eps, b);
+                    const int pos = pos_of[r];
+                    const bool quad = m0 + r0 + 3 < to.m_total && seq_of[r0] == seq_of[r0 + 3] && __builtin_amdgcn_readfirstlane(pos) % 4 == 0;
+                    qkv_store_row<128>(rr, to, is_q, is_k, local, tok, pos, block_of[r], tok < to.m_total, quad, b, a);
+                }
+            });
+        }
+        return;
+    }
     // Where the whole launch is one gated section, a row takes half as many lanes, none of them idle: an
     // expert model's up-projections 286 → 272 µs a launch.
     constexpr int LD = 16 * NJ + 4;
@@ -516,18 +571,18 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
     }
 }
 
-template <typename E, int MI, int NJ, int G, int PER_CU>
-static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
+template <typename E, int MI, int NJ, int G, int PER_CU, typename Rows = RowsAsTheyAre>
+static int launch_big(const TiledGemm<E>& g, hipStream_t s, const Rows& to = {}) {
     typedef BigTile<MI, NJ, G> T;
     static bool attr = false;
     if (!attr) {
-        FH_CHECK_HIP(hipFuncSetAttribute((const void*)tiled_gemm_big_kernel<E, MI, NJ, G, PER_CU>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::LDS));
+        FH_CHECK_HIP(hipFuncSetAttribute((const void*)tiled_gemm_big_kernel<E, MI, NJ, G, PER_CU, Rows>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)T::LDS));
         attr = true;
     }
     const int mtiles = g.rows.id ? g.rows.max_blocks * (g.rows.block / T::ROWS) : cdiv(g.m, T::ROWS), ntiles = cdiv(g.n, T::COLS);
     form_hit(g.rows.id ? FORM_TILED_GEMM_GROUPED_BIG : FORM_TILED_GEMM_BIG);
     form_hit(T::ROWS == 64 ? FORM_TILED_GEMM_64X64 : T::COLS == 256 ? FORM_TILED_GEMM_128X256 : T::COLS == 128 ? FORM_TILED_GEMM_128X128 : FORM_TILED_GEMM_128X64);
-    hipLaunchKernelGGL((tiled_gemm_big_kernel<E, MI, NJ, G, PER_CU>), dim3(mtiles * ntiles, 1, g.groups), dim3(256), T::LDS, s, g, mtiles, ntiles);
+    hipLaunchKernelGGL((tiled_gemm_big_kernel<E, MI, NJ, G, PER_CU, Rows>), dim3(mtiles * ntiles, 1, g.groups), dim3(256), T::LDS, s, g, mtiles, ntiles, to);
     FH_CHECK_LAUNCH();
     return 0;
 }
@@ -599,6 +654,18 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
         if (tiles(128, 128) > knobs().tiled_half_max_tiles) return launch_big<E, 4, 4, 2, 2>(g, s);
         return tiles(64, 64) > knobs().tiled_small_max_tiles ? launch_big<E, 4, 2, 3, 2>(g, s) : launch_big<E, 2, 2, 3, 3>(g, s);
     }
+}
+
+// The rows of a q|k|v projection by its own launch: 5.7 µs more of it at 2048 × 4096 × 1024 (23.8 → 29.5) for a launch of 11.7 that reads and writes them once more.  From a
+// tile of 128 × 128 for each CU on; µs of a prompt through 14 layers, launch of its own | this: 488 tokens (128 tiles) 1087 | 1149, 700 (192) 1566 | 1570, 986 (256) 1433 | 1408,
+// 1500 (384) 1998 | 1936, 2048 (512) 2034 | 1941, 4096 4146 | 4009, 8192 5932 | 5572.
+bool tiled_gemm_qkv_supports(const TiledGemm<_Float16>& g, const QkvRows& to) {
+    return big_tiles(g.rows, g.m, g.n, 1, 128, 128) >= knobs().qkv_min_tiles && g.m == to.m_total && g.n == (to.q_heads + 2 * to.kv_heads) * 128 && !g.bias && !g.nsec;
+}
+int tiled_gemm_qkv(const TiledGemm<_Float16>& g, const QkvRows& to, hipStream_t s) {
+    FH_REQUIRE(tiled_gemm_qkv_supports(g, to), "tiled_gemm_qkv: %d rows of %d + 2 × %d heads", g.m, to.q_heads, to.kv_heads);
+    form_hit(FORM_F16_QKV);
+    return big_tiles(g.rows, g.m, g.n, 1, 128, 256) >= (knobs().tiled_wide_min_tiles >= 0 ? knobs().tiled_wide_min_tiles : 257) ? launch_big<_Float16, 4, 8, 2, 2>(g, s, to) : launch_big<_Float16, 4, 4, 2, 2>(g, s, to);
 }
 
 int tiled_gemm_slabs(int m, int n, int k) {

@@ -21,6 +21,7 @@
 #include "kernels.h"
 #include "knobs.h"
 #include "route_merge.h"
+#include "qkv_rows.h"
 #include "tiled_gemm.h"
 #include "w4_device.h"
 
@@ -3517,6 +3518,22 @@ int f16t_gemm_gated(const W4Device& w, const __half* x, __half* out, int m, int 
     g.nsec = 1; g.sec[0].begin = 0; g.sec[0].act = gelu ? GEMM_ACT_GELU_GLU : GEMM_ACT_SILU_GLU;
     g.pair = im / 16;
     return tiled_gemm(g, stream);
+}
+
+// q|k|v of a prompt
+static TiledGemm<_Float16> f16t_qkv(const W4Device& w, const __half* x, const QkvRows& to) {
+    TiledGemm<_Float16> g;
+    g.x = reinterpret_cast<const _Float16*>(x); g.ldx = w.k; g.w = reinterpret_cast<const _Float16*>(w.f16t);
+    g.m = to.m_total; g.n = w.n; g.k = w.k;
+    return g;
+}
+bool f16t_gemm_qkv_supports(const W4Device& w, const __half* x, const QkvRows& to) {
+    return w.f16t && !w.bias && w.k % 32 == 0 && ((uintptr_t)x & 15) == 0 && tiled_gemm_qkv_supports(f16t_qkv(w, x, to), to);
+}
+int f16t_gemm_qkv(const W4Device& w, const __half* x, const QkvRows& to, hipStream_t stream) {
+    FH_REQUIRE(f16t_gemm_qkv_supports(w, x, to), "f16t_gemm_qkv: %d rows, N=%d K=%d", to.m_total, w.n, w.k);
+    form_hit(FORM_F16_DENSE_LINEAR);
+    return tiled_gemm_qkv(f16t_qkv(w, x, to), to, stream);
 }
 
 int f16t_gemm(const __half* x, const __half* wt, __half* out, int m, int n, int k, float* workspace,

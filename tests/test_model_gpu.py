@@ -284,6 +284,31 @@ def test_unquantised_gate_up_with_its_activation(pkg, prompt_len, inter, size, a
     _assert_parity(res)
 
 
+@pytest.mark.parametrize("nq,nkv,qk_norm", [(3, 1, True), (4, 2, False)])
+@pytest.mark.parametrize("size", ["128x128", "128x256"])
+def test_unquantised_qkv_with_its_rows(pkg, size, nq, nkv, qk_norm, knobs, forms):
+    """Norm, rotation and cache write in the projection's launch leave the bits that a launch of their own does: rows that end within a tile and with it, four tokens of several
+    sequences, positions at none of a value tile's fours, whole tiles of heads and half of one.  (Portions of more than 64 rows: fewer run in the few-row kernel without this,
+    whose sums over K have another order, so that one fp16 rounding in 2^11 may fall to the other side.)"""
+    from tests import modelgen, tile_sizes
+    tm = modelgen.TinyModel(False, layers=2, hidden=256, nq=nq, nkv=nkv, hd=128, inter=256, vocab=512, seed=177, max_seq_len=256, dense_proj=True, tied=True, qk_norm=qk_norm)
+    knobs.set(**tile_sizes.SIZES[size])
+    toks = np.random.default_rng(5).integers(0, 512, size=(4, 256)).astype(np.uint32)
+    got = []
+    for tiles in (10 ** 6, 1):
+        knobs.set(QKV_MIN_TILES=tiles)
+        forms.reset()
+        hm = tm.hip_model(pkg, kv_num_blocks=40, max_seqs=4, max_tokens=256)
+        at, out = [0] * 4, []
+        for portion in ([130, 61, 7, 1], [33, 90, 3, 2], [1, 1, 1, 1], [2, 1, 80, 5]):
+            out.append(hm.unified_forward([(i, toks[i, at[i]:at[i] + n], at[i], True) for i, n in enumerate(portion)], want_logits=True)[1])
+            at = [a + n for a, n in zip(at, portion)]
+        got.append(np.concatenate(out))
+        assert forms.hits().get("f16_qkv", 0) == (6 if tiles == 1 else 0)
+        del hm
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
 @pytest.mark.parametrize("tokens", [1, 100])
 @pytest.mark.parametrize("activation,lo,hi", [(1, -5.5, -2.0), (1, -2.0, 3.0), (0, -12.0, 12.0)])
 def test_unquantised_activation_errs_by_its_rounding(pkg, activation, lo, hi, tokens, knobs, forms):
