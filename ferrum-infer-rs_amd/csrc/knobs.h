@@ -69,7 +69,7 @@ struct Knobs {
     int tiled_half_max_tiles = 256;   // … its 128 × 64 and 64 × 64 forms up to this many tiles of 128 × 128
     int tiled_small_max_tiles = 256;  // … the latter up to this many of them
     int moe_rows_block = 0;           // > 0: forced rows per block of the sorted expert rows
-    int tiled_nw = 0, tiled_kw = 0, tiled_j = 0;      // > 0: forced waves per workgroup, K parts, 16-column tiles per wave of the few-row kernel (1, 2; 4 with two row tiles)
+    int tiled_nw = 0, tiled_kw = 0, tiled_j = 0;      // > 0: forced waves per workgroup, K parts, 16-column tiles per wave of the few-row kernel (1, 2; 3, 4 with two row tiles)
     int layer_overlap_max_tokens = 64;   // parallel blocks: experts on a stream of their own beside the mixer up to this many tokens (0 = never)
     int latent_tiles = 0;             // 1 / 2: forced 16-row tiles per workgroup of the latent attention
     int latent_splits = 0;            // > 0: forced KV split count of the latent attention
@@ -169,6 +169,7 @@ enum Form : int {
     FORM_W4_ROWS,               // ≤ 16 rows: a workgroup's share of the rows resident in LDS, K split over the grid into slabs
     FORM_W4_GATED,              // ≤ 16 rows: gate_up with its activation in the launch
     FORM_F16_GATED,             // unquantised gate_up with its activation in the launch
+    FORM_TILED_GEMM_COLS48,     // few-row projection with 48 columns a wave
     FORM_TILED_GEMM_COLS64,     // few-row projection with 64 columns a wave
     FORM_TILED_GEMM_256X256,    // prompts: tiles of 256 × 256, a workgroup's one after the other (tiled_gemm_wide.hip)
     FORM_CHAIN_MLP,             // decode chain: the MLP of a dense layer in the launch too

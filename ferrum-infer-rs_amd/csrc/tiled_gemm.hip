@@ -93,8 +93,11 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(FewRows f, TiledGemm<E>
     }
     const int spread = EXT && p.x_blocks ? 4 : 0;               // (log2 of the pieces between a row's pieces)
     const bool halves = PAIRED<E> && J == 2 && EXT && p.pair;
-    const unsigned char* wt = reinterpret_cast<const unsigned char*>(p.w) + ((long)g * (p.n >> 4) + (!live ? 0 : halves ? n0 >> 5 : n0 >> 4)) * loads * 1024 + lane * 16;
+    const int tile0 = !live ? 0 : halves ? n0 >> 5 : n0 >> 4;
+    const unsigned char* wt = reinterpret_cast<const unsigned char*>(p.w) + ((long)g * (p.n >> 4) + tile0) * loads * 1024 + lane * 16;
     const long next_tile = (long)(halves ? p.pair : 1) * loads * 1024;
+    // (past the last column of more than two tiles: the last once more)
+    auto tile = [&](int j) { return (J > 2 ? min(j, (p.n >> 4) - 1 - tile0) : j) * next_tile; };
     const int buffer = f.rows * PIECES * 16, region = max(2 * buffer, MT * J * 1024);
     unsigned char* const rows_buf = smem + wave * region;
     piece_t bw[2][U][J];
@@ -112,7 +115,7 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(FewRows f, TiledGemm<E>
 #pragma unroll
         for (int u = 0; u < U; u++)
 #pragma unroll
-            for (int j = 0; j < J; j++) bq[u][j] = __builtin_nontemporal_load(reinterpret_cast<const piece_t*>(wt + j * next_tile + (long)min(s + u, s1 - 1) * 1024));
+            for (int j = 0; j < J; j++) bq[u][j] = __builtin_nontemporal_load(reinterpret_cast<const piece_t*>(wt + tile(j) + (long)min(s + u, s1 - 1) * 1024));
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
@@ -123,12 +126,12 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(FewRows f, TiledGemm<E>
     const int turn = ((blockIdx.x * f.cw + cg + part + z) & ((chunks & -chunks) - 1)) * U;
     auto place = [&](int i) { i += turn; return s0 + (i < len ? i : i - len); };
     if (len > 0) load(bw[0], 0, place(0));
-    const GemmSection sec = gemm_section(p, n0);
+    const GemmSection first = gemm_section(p, n0);
     floatx4 bias[J], acc[MT][J];
 #pragma unroll
     for (int j = 0; j < J; j++) {
         bias[j] = (floatx4){0.f, 0.f, 0.f, 0.f};
-        if (p.bias && live) bias[j] = *reinterpret_cast<const floatx4*>(p.bias + (long)g * p.n + n0 + 16 * j + 4 * a);
+        if (p.bias && live) bias[j] = *reinterpret_cast<const floatx4*>(p.bias + (long)g * p.n + (J > 2 ? min(n0 + 16 * j, p.n - 16) : n0 + 16 * j) + 4 * a);
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) acc[mt][j] = (floatx4){0.f, 0.f, 0.f, 0.f};
     }
@@ -202,12 +205,13 @@ __global__ __launch_bounds__(512) void tiled_gemm_kernel(FewRows f, TiledGemm<E>
         return sum;
     };
     if (p.slabs > 1) p.out_f32 += z * p.slab_stride;
-    const bool gated = EXT && J == 2 && gemm_gated_act(sec.act);
+    const bool gated = EXT && J == 2 && gemm_gated_act(first.act);
     const bool vec = p.n_store % 4 == 0 && p.ldo % 4 == 0 && p.out_group % 4 == 0 && p.ld_col_scale % 4 == 0 && ((uintptr_t)p.out & 7) == 0 && ((uintptr_t)p.out_f32 & 15) == 0;
     const int tiles = gated ? J : 1;
 #pragma unroll 1
     for (int t = part * tiles; t < MT * J; t += kw * tiles) {
         const int mt = t / J, j = t % J;
+        const GemmSection sec = J > 2 ? gemm_section(p, min(n0 + 16 * j, p.n - 1)) : first;       // (sections begin at whole 32s)
         floatx4 v = bias[0];
 #pragma unroll
         for (int i = 1; i < J; i++) v = j == i ? bias[i] : v;
@@ -789,10 +793,23 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     const bool two_rounds = !rows.id && tiles16 > 256 && tiles16 <= 512;
     const bool ext = rows.id || g.x_blocks || g.col_scale || gated || rare, wide = !rows.id && tiles16 > 2048;
     int J = rows.id ? 2 : mt == 1 ? ((two_rounds && loads >= (tiles16 < 448 ? 48 : g.slabs > 1 ? 64 : 80)) || (wide && (g.m > 12 || (g.m > 8 && loads >= 48) || loads > 128)) ? 2 : 1) : tiles16 <= 256 || (two_rounds && loads <= (g.slabs > 1 ? 32 : 8)) ? 1 : 2;
-    if (mt == 2 && !ext && tiles16 >= 4096 && loads >= (g.m > 24 ? 48 : 96) && g.n % 64 == 0) J = 4;
-    if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : knobs().tiled_j == 4 && mt == 2 && !ext && g.n % 64 == 0 ? 4 : 2;
+    // Two row tiles, 32 columns and a little more than a workgroup for each CU: the CUs with two are what the launch waits for, at the 29 bytes a clock that a CU's loads
+    // get, half of them the rows once more.  48 columns bring it back to one, then 64, where the rows are many bytes and parts not too long (a step of
+    // segetar, 32 rows: 598 → 586 µs, of nerenex in 32 bits 363 → 345).  µs, 16 bits, 32 | 48 | 64 columns:
+    //                        K = 1024              2048                  4096                  8192
+    //   32 × 8192        6.7 |  7.2 |  7.7     9.1 | 10.2 | 11.0    15.1 | 16.8 | 19.1    25.4 | 29.5 | 35.4
+    //   32 × 8224        7.7 |  6.9 |  7.7    12.0 | 10.1 | 11.0    21.4 | 16.7 | 19.1    39.5 | 30.2 | 35.7
+    //   20 × 9280        7.8 |  7.3 |  7.8    11.9 |  9.9 | 10.7    20.9 | 16.3 | 18.4    37.2 | 28.2 | 34.5
+    //   32 × 12288       8.6 |  8.4 |  8.6    13.2 | 11.9 | 12.3    23.5 | 19.6 | 21.2    43.5 | 34.4 | 41.9
+    //   32 × 12320       8.6 | 10.0 |  8.6    13.2 | 16.3 | 12.3    23.5 | 28.9 | 21.1    43.6 | 52.5 | 41.8
+    //   32 × 14336       8.8 | 10.6 |  9.2    13.6 | 17.1 | 13.2    24.4 | 30.1 | 22.6    44.5 | 55.6 | 47.1
+    //   32 × 16384       9.3 | 10.8 |  9.8    14.5 | 17.3 | 14.5    26.4 | 30.6 | 24.9    46.3 | 57.1 | 53.7
+    if (mt == 2 && !ext && tiles16 > 512 && tiles16 <= 768) J = 3;
+    if (mt == 2 && !ext && tiles16 > 768 && tiles16 <= 896 && loads >= 64 && loads <= 128) J = 4;
+    if (mt == 2 && !ext && tiles16 >= 4096 && loads >= (g.m > 24 ? 48 : 96) && g.n % 64 == 0) J = 4;       // (a vocabulary)
+    if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : knobs().tiled_j > 2 && mt == 2 && !ext ? knobs().tiled_j : 2;
     if (gated) J = 2;
-    const long cols = g.n / (16 * J), blocks = (long)rbs * cols * zs;
+    const long cols = cdiv(g.n, 16 * J), blocks = (long)rbs * cols * zs;
     int nw = mt == 1 && !rows.id && ((blocks > 512 && loads >= 64 && (!wide || loads % 32 == 0)) || (blocks <= 256 && J == 1 && loads >= 96)) ? 8 : 4, kw = nw;
     if (J == 1 && two_rounds) kw = 2;
     // Sorted rows, 32 columns: K in as many parts as there are waves, until workgroups are so many that the parts' sums and their waits only add.  µs in
@@ -807,7 +824,7 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     if (rows.id && mt == 1 && loads >= 96) nw = kw = 8;
     else if (rows.id) kw = mt == 1 ? (blocks < 20000 ? 4 : 1) : mt == 2 ? (blocks < 4096 ? 4 : 1) : blocks < 512 ? 4 : blocks < 3000 ? 2 : 1;
     else if (mt == 4 && (long)rbs * cdiv(cols, 4) * zs > 128) kw = 1;
-    else if (mt == 4 || J == 4)
+    else if (mt == 4 || (J == 4 && tiles16 > 1024))
         for (int k : {2, 1}) {
             const int slots = mt == 4 ? 256 : 512;
             if (cdiv((long)rbs * cdiv(cols, 4 / k) * zs, slots) * kw <= cdiv((long)rbs * cdiv(cols, 4 / kw) * zs, slots) * k) kw = k;
@@ -821,6 +838,10 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
 #define SMALL(J_, EXT_) \
     (mt == 1 ? launch_small<E, 1, J_, EXT_>(g, grid, nw, kw, s) : mt == 2 ? launch_small<E, 2, J_, EXT_>(g, grid, nw, kw, s) : launch_small<E, 4, J_, EXT_>(g, grid, nw, kw, s))
     if (ext) return J == 1 ? SMALL(1, true) : SMALL(2, true);
+    if (J == 3) {
+        form_hit(FORM_TILED_GEMM_COLS48);
+        return launch_small<E, 2, 3, false>(g, grid, nw, kw, s);
+    }
     if (J == 4) {
         form_hit(FORM_TILED_GEMM_COLS64);
         return launch_small<E, 2, 4, false>(g, grid, nw, kw, s);

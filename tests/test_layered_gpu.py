@@ -568,6 +568,20 @@ def test_few_row_and_tile_projections_agree(pkg, cases, knobs, forms, name):
             assert h.get("tiled_gemm") and not h.get("tiled_gemm_big")
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("j", [3, 4])
+@pytest.mark.parametrize("name", ["wide", "shared", "loop", "all", "talks"])
+def test_sections_within_a_wave_s_columns(pkg, cases, knobs, forms, name, j, dtype):
+    """48 and 64 columns a wave where the projection's parts, of 32 columns and of more, each have an activation of their own, and the last wave's columns do not all exist."""
+    cfg, w, path = cases(name)
+    t = toks(cfg, 29, 13)
+    knobs.set(TILED_J=j, TILED_MIN_TILES=-1, TILED_BIG_MIN_TILES=10 ** 6)
+    m = load(pkg, path, dtype)
+    forms.reset()
+    assert rel(feed(m, 1, t, [29]), L.forward(cfg, w, t)) < TOL[dtype]
+    assert forms.hits().get(f"tiled_gemm_cols{16 * j}")
+
+
 EVEN = {"nerenex": lambda: G.config(256, 260, [G.recurrent(256, 2, 3, ff=384), G.attention(20, 64, 32, 48, 128, 256, 130, ff=640), G.recurrent(640, 5, 2, ff=128)], mult=0.6),
         "safolorn": lambda: G.safolorn(128, 260, 40, [G.sink_attention(8, 64, 32, 64, 256, 1e5, G.LONG, mlp=G.glu(384, 1.5)), G.sink_attention(4, 64, 32, 32, 256, 1e5, G.LONG, mlp=G.experts(5, 2, 256))]),
         "segetar": lambda: G.segetar(256, 260, [G.scan(256, 16, 128, 4, mlp=G.dense(384)), G.gated_pair(8, 2, 64, 64, 130, 4, 64, 64, mlp=G.grouped_experts(6, 2, 128, 2, 1))]),

@@ -473,6 +473,15 @@ def test_few_rows_of_several_row_tiles(env, m, n, k, j, kw, knobs, forms):
     forms.require("tiled_gemm", *(["tiled_gemm_cols64"] if j == 4 and m <= 32 else []))
 
 
+@pytest.mark.parametrize("m,n,k,form", [(17, 8224, 96, 48), (32, 8256, 2080, 48), (20, 12288, 64, 48), (32, 8192, 2048, None), (32, 12320, 2048, 64), (17, 14336, 4096, 64), (32, 12320, 1024, None),
+                                        (32, 14368, 2048, None), (16, 9280, 2048, None)])
+def test_columns_past_a_round_of_workgroups(env, m, n, k, form, knobs, forms):
+    """48 and 64 columns a wave on both sides of the lines where they begin and end; the last wave's columns there in whole and in parts."""
+    _few_rows(env, m, n, k)
+    h = forms.hits()
+    assert [c for c in (48, 64) if h.get(f"tiled_gemm_cols{c}")] == ([form] if form else []), h
+
+
 @pytest.mark.parametrize("m,n,k,form", [(30, 65600, 1568, "tiled_gemm_cols64"), (17, 65600, 3104, "tiled_gemm_cols64"), (20, 139328, 1056, None), (32, 139264, 1056, None), (12, 120960, 4128, None),
                                         (12, 120832, 4128, "tiled_gemm"), (32, 139008, 1056, "tiled_gemm"), (10, 65568, 2080, "tiled_gemm"), (15, 32800, 96, "tiled_gemm")])
 def test_vocabularies_on_both_sides_of_a_line(env, m, n, k, form, knobs, forms):
