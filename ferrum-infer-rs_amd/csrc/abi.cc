@@ -36,6 +36,7 @@ void reload_knobs() {
     k.attn_no_rs = env_flag("FERRUM_HIP_ATTN_NO_RS");
     k.attn_narrow = env_flag("FERRUM_HIP_ATTN_NARROW");
     k.attn_flash_rows = env_int("FERRUM_HIP_ATTN_FLASH_ROWS", 0);
+    k.no_grouped_step = env_flag("FERRUM_HIP_NO_GROUPED_STEP");
     k.no_stream_route = env_flag("FERRUM_HIP_NO_STREAM_ROUTE");
     k.attn_key_waves = env_int("FERRUM_HIP_ATTN_KEY_WAVES", 0);
     k.qkv_min_tiles = env_int("FERRUM_HIP_QKV_MIN_TILES", 256);
@@ -114,7 +115,7 @@ static const char* const g_form_names[FORM_COUNT] = {
     "tp_allreduce_loopback", "tp_allreduce_oneshot", "f16_dense_linear", "w4_fused_tail", "attn_resident", "w4_big", "w4_ldsk", "gather_columns",
     "perm_producer", "moe_expert_major_pair", "decode_chain", "moe_deferred_merge", "dense_chain", "tp_allreduce_norm_fused", "moe_block_major_pair", "chain_attn_kv_splits", "chain_qkv_wide", "route_gemm_topk",
     "tiled_gemm", "tiled_gemm_big", "tiled_gemm_128x256", "tiled_gemm_128x128", "tiled_gemm_128x64", "tiled_gemm_64x64", "tiled_gemm_grouped", "tiled_gemm_grouped_big", "moe_route_sort", "latent_attn_plain", "latent_attn", "latent_attn_pair", "latent_attn_split", "latent_attn_expanded", "rglru_step", "rglru_scan",
-    "grouped_attn_plain", "grouped_attn_keys", "grouped_attn_split", "grouped_attn_tile", "linear_step", "linear_chunk", "scan_step", "scan_chunk", "route_grouped",
+    "grouped_attn_plain", "grouped_attn_keys", "grouped_attn_step", "grouped_attn_split", "grouped_attn_tile", "linear_step", "linear_chunk", "scan_step", "scan_chunk", "route_grouped",
     "route_softmax", "talk_attn_plain", "talk_attn_keys", "talk_attn_tile", "talk_attn_tile_split", "w4_rows", "w4_gated", "f16_gated", "tiled_gemm_cols48", "tiled_gemm_cols64", "tiled_gemm_256x256", "chain_mlp", "chain_rows", "moe_rows_256", "done_again", "attn_keys", "attn_keys_wide", "f16_qkv", "stream_route"};
 const char* form_name(int f) { return f >= 0 && f < FORM_COUNT ? g_form_names[f] : nullptr; }
 }  // namespace fh

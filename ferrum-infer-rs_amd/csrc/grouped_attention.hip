@@ -195,13 +195,23 @@ __device__ __forceinline__ void grouped_store4(const GroupedBuffers<E>& p, long 
     *reinterpret_cast<v4*>(p.out + tok * p.ldo + col) = y;
 }
 
+// for what crosses waves in LDS alone: loads under way stay so
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // Few rows per sequence.  grid (16-row tiles × KV splits, kv_heads): the four waves take 32-key steps of the range in turn, straight from
 // the cache into registers (the next step is requested before this one is used), and merge through LDS.  32-bit models take it for prompts too: 16
 // (token, head) rows share a read of the cache that the plain form makes for each of them (16 heads of 128 dimensions on 4, a prompt of 1000 tokens
 // and 8 decoded: 3.61 -> 0.20 ms).  One set of operand registers there: keys are requested behind the scores, values behind their product.
 // FAR: scores fall with the logarithm of the distance.
-template <typename E, int DS, bool FAR>
-__global__ __launch_bounds__(256) void grouped_attn_keys_kernel(GroupedDims d, GroupedBuffers<E> p, BatchView v, int nsplit) {
+// STEP, one token a sequence: what grouped_prepare does too.  A workgroup norms and rotates its queries and the token's key while its first keys are under way (a step of
+// segetar, 32 rows, four such layers: 586 → 576 µs, of fororax, one, 212.7 → 207.5; every wave for itself: 64 times the loads, 606); the wave whose keys end with the token's block puts the token's key and value into its operands, and
+// the first tile's into the cache.
+template <typename E, int DS, bool FAR, bool STEP>
+__global__ __launch_bounds__(256, STEP && sizeof(E) == 2 ? 2 : 1) void grouped_attn_keys_kernel(GroupedDims d, GroupedBuffers<E> p, BatchView v, int nsplit) {
     typedef typename Frag<E>::v8 v8;
     constexpr int DT = 2 * DS, D = 32 * DS, LD = D + 4, NB = sizeof(E) == 2 ? 2 : 1;
     extern __shared__ __attribute__((aligned(16))) float lds_o[];              // [4][16][LD]
@@ -229,8 +239,127 @@ __global__ __launch_bounds__(256) void grouped_attn_keys_kernel(GroupedDims d, G
             for (int s = 0; s < DS; s++) f[i][s] = *reinterpret_cast<const v8*>(pool + blk * kd + off + s * 512);
         }
     };
+    // STEP: a thread's 8 numbers of the tile's query rows and, behind them, of the token's key, all requested ahead of the keys
+    constexpr int PR = 4 * DS;                                                  // pieces of a row
+    __shared__ __attribute__((aligned(16))) E rows_lds[STEP ? 17 * D : 8];
+    __shared__ float red[STEP ? 17 * PR : 1];
+    const int slot = w.pos0 & 15;
+    const bool own = STEP && p.k_in != nullptr, owner = own && st_hi == nstep && st_lo + wave < st_hi && (nstep - 1 - st_lo - wave) % 4 == 0;       // (wave: of the last step)
+    E v_new[STEP ? DS : 1][2];
+    if constexpr (STEP) {
+        const E *q_row = p.q_in + tok * p.ld, *k_row = own ? p.k_in + tok * p.ld : q_row;
+        const int tile_rows = min(16, rows - w.tile * 16), pieces = (tile_rows + (own ? 1 : 0)) * PR, h0 = kvh * G + w.tile * 16;
+        struct Piece { v8 x; float c[4], s[4]; floatx8 w; };
+        // (as rot_load, but with nothing between its loads: without a rotation they are any numbers)
+        const int half = d.rot_dims >> 1;
+        const float *cos_t = half ? p.cos_t + (long)row_pos * half : p.q_norm, *sin_t = half ? p.sin_t + (long)row_pos * half : p.q_norm;
+        auto fetch = [&](int i) {
+            const int r = min(i, pieces - 1) / PR, c = (min(i, pieces - 1) - r * PR) * 8;
+            const bool key = r == tile_rows;
+            Piece f;
+            f.x = *reinterpret_cast<const v8*>((key ? k_row + kvh * D : q_row + (h0 + r) * D) + c);
+            f.w = *reinterpret_cast<const floatx8*>((key ? p.k_norm : p.q_norm) + (p.head_norm ? 0 : (key ? kvh : h0 + r) * D) + c);
 #pragma unroll
-    for (int s = 0; s < DS; s++) qf[s] = *reinterpret_cast<const v8*>(p.q + (tok * d.heads + head) * D + 32 * s + 8 * a);
+            for (int j = 0; j < 4; j++) {
+                const int at = max(0, min((c >> 1) + j, half - 1));
+                f.c[j] = cos_t[at];
+                f.s[j] = sin_t[at];
+            }
+            return f;
+        };
+        auto squares = [&](const v8& x) {
+            float t = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) t += (float)x[j] * (float)x[j];        // (padded columns are zero)
+            return t;
+        };
+        const int i0 = threadIdx.x, nq = d.heads * D, nk = own ? d.kv_heads * D : 0;
+        Piece f0 = fetch(i0);
+        float sq = 0.f, sk = 0.f;
+        if (!p.head_norm)
+            for (int i = i0 * 8; i < nq + nk; i += 4096) {
+                const int i2 = i + 2048, at2 = min(i2, nq + nk - 8);           // (two at once)
+                const v8 x = *reinterpret_cast<const v8*>(i < nq ? q_row + i : k_row + (i - nq)), x2 = *reinterpret_cast<const v8*>(at2 < nq ? q_row + at2 : k_row + (at2 - nq));
+                const float t = squares(x), t2 = i2 < nq + nk ? squares(x2) : 0.f;
+                if (i < nq) sq += t; else sk += t;
+                if (i2 < nq) sq += t2; else sk += t2;
+            }
+        if (owner)
+#pragma unroll
+            for (int s = 0; s < DS; s++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) v_new[s][h] = p.v_in[tok * p.ld + kvh * D + 32 * s + 16 * h + b];
+        asm volatile("" ::: "memory");
+        load(kf[0], p.k_pool, st_lo + wave);
+        load(vf[0], p.v_pool, st_lo + wave);
+        if (p.head_norm) {
+            for (int i = i0; i < pieces; i += 256) red[i] = squares(i == i0 ? f0.x : fetch(i).x);
+        } else {
+            sq = wave_reduce_sum(sq);
+            sk = wave_reduce_sum(sk);
+            if (lane == 0) { red[wave] = sq; red[4 + wave] = sk; }
+        }
+        lds_barrier();
+        for (int i = i0; i < pieces; i += 256) {
+            const Piece f = i == i0 ? f0 : fetch(i);
+            const int r = i / PR;
+            const bool key = r == tile_rows;
+            float sum = 0.f;
+            if (p.head_norm)
+#pragma unroll
+                for (int j = 0; j < PR; j++) sum += red[r * PR + j];
+            else
+                sum = key ? red[4] + red[5] + red[6] + red[7] : red[0] + red[1] + red[2] + red[3];
+            const float inv = 1.0f / sqrtf(sum / (float)(p.head_norm ? d.dim : (key ? d.kv_heads : d.heads) * d.dim) + p.eps);
+            floatx8 y;
+#pragma unroll
+            for (int j = 0; j < 8; j++) y[j] = (float)f.x[j] * inv * f.w[j];
+            Rot4 rot;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const bool turns = (((i - r * PR) * 8) >> 1) + j < half;
+                rot.c[j] = turns ? f.c[j] : 1.f;
+                rot.s[j] = turns ? f.s[j] : 0.f;
+            }
+            y = rot_apply(y, rot);
+            v8 o;
+#pragma unroll
+            for (int j = 0; j < 8; j++) o[j] = (E)y[j];
+            *reinterpret_cast<v8*>(rows_lds + (key ? 16 : r) * D + (i - r * PR) * 8) = o;
+        }
+        lds_barrier();
+#pragma unroll
+        for (int s = 0; s < DS; s++) qf[s] = *reinterpret_cast<const v8*>(rows_lds + min(b, tile_rows - 1) * D + 32 * s + 8 * a);
+    } else {
+#pragma unroll
+        for (int s = 0; s < DS; s++) qf[s] = *reinterpret_cast<const v8*>(p.q + (tok * d.heads + head) * D + 32 * s + 8 * a);
+    }
+    // the token's key and value in the operands of its block (twice there where the block is the last step's only one); in a block that it opens nothing else is
+    auto place = [&](v8 (&kq)[2][DS], v8 (&vq)[2][DS], int st) {
+        if (!STEP || !owner || st != nstep - 1) return;
+        const long at = (long)__builtin_amdgcn_readfirstlane(bt[blk_hi - 1]) * kd + off;
+#pragma unroll
+        for (int s = 0; s < DS; s++) {
+            const v8 k_new = *reinterpret_cast<const v8*>(rows_lds + (STEP ? 16 * D + 32 * s + 8 * a : 0));
+            const E v0 = v_new[STEP ? s : 0][0], v1 = v_new[STEP ? s : 0][1];
+            v8 v_put;
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+                if (blk_lo + 2 * st + i >= blk_hi - 1) {
+                    kq[i][s] = b == slot ? k_new : kq[i][s];
+#pragma unroll
+                    for (int j = 0; j < 8; j++) vq[i][s][j] = 4 * a + (j & 3) == slot ? (j < 4 ? v0 : v1) : slot == 0 ? (E)0.f : vq[i][s][j];
+                    v_put = vq[i][s];
+                }
+            if (w.tile) continue;
+            if (b == slot) *reinterpret_cast<v8*>(p.k_pool + at + s * 512) = k_new;
+            if (slot == 0) *reinterpret_cast<v8*>(p.v_pool + at + s * 512) = v_put;
+            else if (a == slot >> 2) {
+                p.v_pool[at + s * 512 + (slot & 3)] = v0;
+                p.v_pool[at + s * 512 + 4 + (slot & 3)] = v1;
+            }
+        }
+    };
     float m_run = -INFINITY, l_run = 0.f;
     floatx4 o[DT];
 #pragma unroll
@@ -271,21 +400,26 @@ __global__ __launch_bounds__(256) void grouped_attn_keys_kernel(GroupedDims d, G
     if (st_lo + wave < st_hi) {
         int st = st_lo + wave;
         float sc[8];
-        load(kf[0], p.k_pool, st);
-        load(vf[0], p.v_pool, st);
+        if (!STEP) {
+            load(kf[0], p.k_pool, st);
+            load(vf[0], p.v_pool, st);
+        }
         while (true) {
             if constexpr (NB == 2) {
                 load(kf[1], p.k_pool, st + 4);
                 load(vf[1], p.v_pool, st + 4);
+                place(kf[0], vf[0], st);
                 scores(kf[0], st, sc);
                 weigh(vf[0], sc);
                 st += 4;
                 if (st >= st_hi) break;
                 load(kf[0], p.k_pool, st + 4);
                 load(vf[0], p.v_pool, st + 4);
+                place(kf[1], vf[1], st);
                 scores(kf[1], st, sc);
                 weigh(vf[1], sc);
             } else {
+                place(kf[0], vf[0], st);
                 scores(kf[0], st, sc);
                 load(kf[0], p.k_pool, st + 4);
                 weigh(vf[0], sc);
@@ -502,9 +636,15 @@ __global__ __launch_bounds__(256, DS <= 4 ? 2 : 1) void grouped_attn_tile_kernel
     }
 }
 
+// Steps whose attention prepares its rows itself; heads of more than 128 dimensions would need more registers than there are
+template <typename E>
+static bool grouped_step(const GroupedDims& d, const GroupedBuffers<E>& b, const BatchView& v) {
+    return v.single && !b.talk && !knobs().grouped_plain && !knobs().no_grouped_step && d.dp == d.vp && d.dp <= 128 && d.scale > 0.f;
+}
 template <typename E>
 int grouped_prepare(const GroupedDims& d, const GroupedBuffers<E>& b, const BatchView& v, hipStream_t s) {
     FH_REQUIRE(b.k_in || b.head_norm, "grouped attention: keys and values of another layer take norms of one head each");
+    if (grouped_step(d, b, v)) return 0;
     int sub = 1;
     while (sub < 64 && sub * 8 < d.dp) sub *= 2;
     if (b.head_norm) hipLaunchKernelGGL(grouped_prepare_heads_kernel<E>, dim3(v.T), dim3(256), 0, s, d, b, v, sub);
@@ -537,7 +677,13 @@ template <int DS, bool FAR, typename E>
 static int grouped_keys(const GroupedDims& d, const GroupedBuffers<E>& b, const BatchView& v, hipStream_t s) {
     constexpr size_t lds = (size_t)64 * (32 * DS + 4) * 4;
     static bool attr = false;
-    if (!attr) { FH_CHECK_HIP(hipFuncSetAttribute((const void*)grouped_attn_keys_kernel<E, DS, FAR>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)); attr = true; }
+    constexpr bool MAY = DS <= 4;
+    const bool step = MAY && grouped_step(d, b, v);
+    if (!attr) {
+        FH_CHECK_HIP(hipFuncSetAttribute((const void*)grouped_attn_keys_kernel<E, DS, FAR, false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        FH_CHECK_HIP(hipFuncSetAttribute((const void*)grouped_attn_keys_kernel<E, DS, FAR, MAY>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        attr = true;
+    }
     const int G = d.heads / d.kv_heads, tiles = v.single ? v.num_seqs * cdiv(G, 16) : (int)((long)v.T * G / 16) + v.num_seqs;
     // split the keys while the launch has fewer workgroups than stay resident and a split keeps ≥ 128 keys
     const int keys = (int)std::min<long>(v.max_keys, (long)d.window + 16);
@@ -546,7 +692,9 @@ static int grouped_keys(const GroupedDims& d, const GroupedBuffers<E>& b, const 
     if (knobs().grouped_splits > 0) ns = std::min(16, knobs().grouped_splits);
     while (ns > 1 && (size_t)tiles * d.kv_heads * ns * 16 * (d.vp + GROUPED_PARTIAL_PAD) * 4 > b.partial_bytes) ns /= 2;
     form_hit(ns > 1 ? FORM_GROUPED_ATTN_SPLIT : FORM_GROUPED_ATTN_KEYS);
-    hipLaunchKernelGGL((grouped_attn_keys_kernel<E, DS, FAR>), dim3(tiles * ns, d.kv_heads), dim3(256), lds, s, d, b, v, ns);
+    if (step) form_hit(FORM_GROUPED_ATTN_STEP);
+    if (step) hipLaunchKernelGGL((grouped_attn_keys_kernel<E, DS, FAR, MAY>), dim3(tiles * ns, d.kv_heads), dim3(256), lds, s, d, b, v, ns);
+    else hipLaunchKernelGGL((grouped_attn_keys_kernel<E, DS, FAR, false>), dim3(tiles * ns, d.kv_heads), dim3(256), lds, s, d, b, v, ns);
     FH_CHECK_LAUNCH();
     if (ns > 1) {
         hipLaunchKernelGGL(grouped_attn_reduce_kernel<E>, dim3(tiles, d.kv_heads), dim3(256), 0, s, d, b, v, ns);

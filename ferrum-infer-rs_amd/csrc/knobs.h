@@ -25,6 +25,7 @@ struct Knobs {
     bool attn_no_resident = false;    // never take the resident-K/V short-prompt prefill form
     long attn_resident_min_wgs = 128; // … and only from this many workgroups (tests lower it)
     int attn_flash_rows = 0;          // 64 / 128: forced rows per workgroup of prompt attention (64: each wave on keys of its own)
+    bool no_grouped_step = false;     // layered grouped attention: norms, rotation and cache write of steps in a launch of their own
     bool no_stream_route = false;     // layered experts: update, router and sorted list in launches of their own
     int attn_key_waves = 0;           // 4 / 8: forced waves per workgroup of the 64-row form
     bool attn_flash32 = false;        // the flash form with 32-key steps (paged_prefill_attn_kernel) for head_dim 128 too
@@ -154,6 +155,7 @@ enum Form : int {
     FORM_RGLRU_SCAN,            // … prompt portions: chunked scan
     FORM_GROUPED_ATTN_PLAIN,    // grouped attention, one workgroup per (token, head), any size and number format
     FORM_GROUPED_ATTN_KEYS,     // … few rows: the waves of a workgroup split the keys
+    FORM_GROUPED_ATTN_STEP,     // … a step of one token a sequence, with its norms, rotation and cache write
     FORM_GROUPED_ATTN_SPLIT,    // … and several workgroups do
     FORM_GROUPED_ATTN_TILE,     // … prompts: 128 rows, keys and values shared through LDS
     FORM_LINEAR_STEP,           // linear attention token by token, the state in registers

@@ -163,7 +163,7 @@ struct GroupedBuffers {
     E* out = nullptr; long ldo = 0;
     float* partial = nullptr; size_t partial_bytes = 0;
 };
-// norms, rotation, cache write (k_in null: another layer caches the keys and values)
+// norms, rotation, cache write (k_in null: another layer caches the keys and values), where grouped_attention does not do them itself: of steps of one token a sequence
 template <typename E> int grouped_prepare(const GroupedDims& d, const GroupedBuffers<E>& b, const BatchView& v, hipStream_t s);
 template <typename E> int grouped_attention(const GroupedDims& d, const GroupedBuffers<E>& b, const BatchView& v, hipStream_t s);
 // … with mixed heads (talk); grouped_attention takes these launches there

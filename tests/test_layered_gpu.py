@@ -399,6 +399,36 @@ def test_far_key_among_hundreds_at_page_borders(pkg, tmp_path, dtype):
 
 
 # ── decoding loop, graph, sampling ────────────────────────────────────────────────────────────────────────────────────────
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("splits", [1, 4])
+@pytest.mark.parametrize("name", ["all", "loop", "bare", "far", "uneven"])
+def test_grouped_steps_prepare_their_rows(pkg, cases, knobs, forms, name, splits, dtype):
+    """Single tokens from the first one on, over the starts of blocks, at unequal positions, then a portion that reads what they cached: heads of 1 to 4 pieces of 32, one norm
+    for all heads and one each, more heads than a tile holds, another layer's cache.  Against a launch of its own: the roots' sums run in another order, so numbers of the
+    format differ by a place now and then, logits by no more than four of its roundings; and against the oracle."""
+    cfg, w, path = cases(name)
+    t = toks(cfg, 41, 14)
+    got = []
+    knobs.set(GROUPED_SPLITS=splits)
+    for off in (None, 1):
+        knobs.set(NO_GROUPED_STEP=off)
+        forms.reset()
+        m = load(pkg, path, dtype)
+        rows = []
+        for i in range(36):
+            now = [(1, t[i:i + 1], i)] + ([(2, t[i - 5:i - 4], i - 5)] if i >= 5 else [])
+            rows.append(m.forward_rows(now, list(range(len(now)))))
+        rows.append(m.forward_rows([(1, t[36:], 36)], list(range(5))))
+        got.append(np.concatenate(rows))
+        assert bool(forms.hits().get("grouped_attn_step")) == (not off)
+    want = L.forward(cfg, w, t)
+    wanted = np.concatenate([np.stack([want[i]] + ([want[i - 5]] if i >= 5 else [])) for i in range(36)] + [want[36:]])
+    assert rel(got[0], got[1]) < {"float32": 2e-6, "bfloat16": 2.0 ** -6}[dtype]
+    # (in 16 bits 36 steps of these tokens take either way to the edge of TOL, 0.04 of the oracle: there the two errors have to be alike, by as much as the results may differ)
+    err = [rel(g, wanted) for g in got]
+    assert err[0] < TOL[dtype] if dtype == "float32" else err[0] < err[1] + 2.0 ** -6, err
+
+
 def near_greedy(cfg, w, prompt, out, slack):
     """Every generated token's oracle logit is within `slack` (relative to the logits' rms) of the best one."""
     full = np.concatenate([prompt, out]).astype(np.uint32)
