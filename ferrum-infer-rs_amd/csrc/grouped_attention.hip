@@ -685,10 +685,19 @@ static int grouped_keys(const GroupedDims& d, const GroupedBuffers<E>& b, const 
         attr = true;
     }
     const int G = d.heads / d.kv_heads, tiles = v.single ? v.num_seqs * cdiv(G, 16) : (int)((long)v.T * G / 16) + v.num_seqs;
-    // split the keys while the launch has fewer workgroups than stay resident and a split keeps ≥ 128 keys
-    const int keys = (int)std::min<long>(v.max_keys, (long)d.window + 16);
+    // Split the keys while the launch has fewer workgroups than stay resident and a split keeps ≥ 128 keys.  Steps in 16 bits that prepare their rows themselves: a launch for the
+    // splits costs as much as three rounds of 128 keys, so more than 512 a split, and up to 128 workgroups, which pull what the memory gives.  µs of a step with 1 | 2 | 4 | 8
+    // splits (fororax, a layer with 4 heads of keys; segetar, four of them):
+    //   fororax   1 × 200 keys   181 | 184 | 184 | 186     1 × 1000   193 | 190 | 188 | 190     1 × 2000   208 | 199 | 195 | 194     1 × 4000   236 | 218 | 208 | 203
+    //             8 × 200        211 | 214 | 215 | 219     8 × 1000   223 | 225 | 221 | 224     8 × 2000   237 | 230 | 227 | 227
+    //            24 × 200        238 | 242 | 246 | 253    24 × 1000   249 | 251 | 254 | 260    24 × 2000   273 | 270 | 273 | 279
+    //   segetar   1 × 90         363 | 374 | 377 | 389     1 × 1000   407 | 396 | 397 | 404    32 × 90     552 | 565 | 573 | 604    32 × 1000   615 | 624 | 632 | 661
+    const int keys = (int)std::min<long>(v.max_keys, (long)d.window + 16), wgs = tiles * d.kv_heads;
     int ns = 1;
-    while (ns < 16 && tiles * d.kv_heads * ns < 512 && keys >= 2 * ns * 128) ns *= 2;
+    if (step && sizeof(E) == 2)
+        while (ns < 16 && wgs * ns < 128 && keys > ns * 512) ns *= 2;
+    else
+        while (ns < 16 && wgs * ns < 512 && keys >= 2 * ns * 128) ns *= 2;
     if (knobs().grouped_splits > 0) ns = std::min(16, knobs().grouped_splits);
     while (ns > 1 && (size_t)tiles * d.kv_heads * ns * 16 * (d.vp + GROUPED_PARTIAL_PAD) * 4 > b.partial_bytes) ns /= 2;
     form_hit(ns > 1 ? FORM_GROUPED_ATTN_SPLIT : FORM_GROUPED_ATTN_KEYS);

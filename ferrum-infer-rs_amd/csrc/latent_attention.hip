@@ -723,9 +723,9 @@ static int latent_mfma(const LatentDims& d, const LatentBuffers<bf16>& b, const 
     const int tiles = v.single ? v.num_seqs * cdiv(d.heads, rows) : (int)(((long)v.T * d.heads) / rows) + v.num_seqs;      // upper bound of Σ ceil(rows of a sequence / rows)
     const int keys = (int)std::min<long>(v.max_keys, (long)d.window + 16);
     // split the keys while the launch has fewer workgroups than stay resident (2 per CU, 1 with two tiles) and a split keeps ≥ 128
-    // keys (two steps)
+    // keys (two steps); up to 256 keys the second launch costs more than it saves (a step of safolorn, one layer's cache of 120 keys, 32 rows: 206 µs whole, 210 in two)
     int ns = 1;
-    while (ns < 16 && tiles * ns < 512 / mt && keys >= 2 * ns * 128) ns *= 2;
+    while (ns < 16 && tiles * ns < 512 / mt && keys > 256 && keys >= 2 * ns * 128) ns *= 2;
     if (knobs().latent_splits > 0)
         for (ns = 1; ns < std::min(16, knobs().latent_splits); ns *= 2) {}
     while (ns > 1 && (size_t)tiles * ns * rows * (d.kp + LATENT_PARTIAL_PAD) * 4 > b.partial_bytes) ns /= 2;
@@ -758,9 +758,11 @@ static int latent_mfma(const LatentDims& d, const LatentBuffers<bf16>& b, const 
 static int latent_mfma(const LatentDims& d, const LatentBuffers<float>& b, const BatchView& v, hipStream_t s) {
     const int tiles = v.single ? v.num_seqs * cdiv(d.heads, 16) : (int)(((long)v.T * d.heads) / 16) + v.num_seqs;
     const int keys = (int)std::min<long>(v.max_keys, (long)d.window + 16);
-    // split the keys while there is less than a workgroup per CU and a split keeps ≥ 128 keys (two steps, 4 µs of products each)
+    // Split the keys while there is less than a workgroup per CU and a split keeps ≥ 64 keys (a step, 4 µs of products, as much as the launch that joins them).  µs of a step of
+    // nerenex, one such layer, with 1 | 2 | 4 | 8 splits: 1 × 120 keys 272 | 266 | 261 | 262, 1 × 200 285 | 270 | 260 | 261, 1 × 400 312 | 288 | 269 | 261,
+    // 16 × 60 300 | 294 | 295 | 298, 16 × 200 321 | 305 | 295 | 298, 16 × 400 351 | 324 | 304 | 297.
     int ns = 1;
-    while (ns < 16 && tiles * ns < 256 && keys >= 2 * ns * 128) ns *= 2;
+    while (ns < 16 && tiles * ns < 256 && keys >= 2 * ns * 64) ns *= 2;
     if (knobs().latent_splits > 0)
         for (ns = 1; ns < std::min(16, knobs().latent_splits); ns *= 2) {}
     while (ns > 1 && (size_t)tiles * ns * 16 * (d.kp + LATENT_PARTIAL_PAD) * 4 > b.partial_bytes) ns /= 2;
