@@ -144,6 +144,7 @@ struct FerrumHipModel {
     uint8_t* idx_host = nullptr;   // pinned
     uint8_t* idx_dev = nullptr;
     uint8_t* results = nullptr;    // pinned: logits on their way to the caller, in portions, and sampled ids behind them
+    size_t results_ids = 0;        // (where those begin)
     hipEvent_t results_done[3] = {};
 
     // decode-steps state

@@ -906,12 +906,14 @@ static int finalize_batch_buffers(FerrumHipModel* m) {
     m->il.total = off;
     FH_CHECK_HIP(hipHostMalloc((void**)&m->idx_host, off, hipHostMallocDefault));
     FH_CHECK_HIP(hipMalloc((void**)&m->idx_dev, off));
-    FH_CHECK_HIP(hipHostMalloc((void**)&m->results, RESULT_RING * RESULT_PORTION + S * 4, hipHostMallocDefault));
+    // (a ring of portions, or the largest result where that is less: pages that no call would use take as long to pin: 0.5 ms a MiB, of a model with one sequence 35.9 ms of preparation → 30.3)
+    m->results_ids = std::min<size_t>(RESULT_RING * RESULT_PORTION, S * (size_t)m->cfg.vocab * 4 + 255) / 256 * 256;
+    FH_CHECK_HIP(hipHostMalloc((void**)&m->results, m->results_ids + S * 4, hipHostMallocDefault));
     for (hipEvent_t& e : m->results_done) FH_CHECK_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     if (int r = dev_alloc(&m->step_counter, (size_t)4)) return r;
     // the pages of the results and the copy engine, once, ahead of the first call that waits for them (4 ms of it)
-    memset(m->results, 0, RESULT_RING * RESULT_PORTION + S * 4);
-    FH_CHECK_HIP(hipMemcpyAsync(m->results, m->idx_dev, std::min(off, RESULT_PORTION), hipMemcpyDeviceToHost, m->stream));
+    memset(m->results, 0, m->results_ids + S * 4);
+    FH_CHECK_HIP(hipMemcpyAsync(m->results, m->idx_dev, std::min(off, m->results_ids), hipMemcpyDeviceToHost, m->stream));
     FH_CHECK_HIP(hipEventRecord(m->results_done[0], m->stream));
     FH_CHECK_HIP(hipStreamSynchronize(m->stream));
     FH_CHECK_HIP(device_zero(m->idx_dev, off));      // with the fills queued before it, those of model_finalize among them: this is its last step
@@ -2228,7 +2230,7 @@ static int forward_batch(FerrumHipModel* m, const FerrumHipBatchItem* items, int
             if (int rc = enqueue_head(m, n, false)) return rc;
             if (int rc = copy_results(m, logits_out + (size_t)r0 * m->vp_n, m->logits, (size_t)n * m->vp_n * 4)) return rc;
         }
-        uint8_t* ids = m->results + RESULT_RING * RESULT_PORTION;
+        uint8_t* ids = m->results + m->results_ids;
         const size_t id_bytes = greedy && out_tokens ? (size_t)sh.num_sampled * 4 : 0;
         if (id_bytes) FH_CHECK_HIP(hipMemcpyAsync(ids, m->out_tokens, id_bytes, hipMemcpyDeviceToHost, m->stream));
         if (sh.num_sampled > 0 && logits_out) {
