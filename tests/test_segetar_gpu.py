@@ -356,6 +356,47 @@ def test_update_router_and_sorted_list_in_one_launch(pkg, tmp_path, knobs, forms
     assert rel(taps[0], taps[1]) < {"float32": 2e-6, "bfloat16": 2.0 ** -9}[dtype]
 
 
+@pytest.mark.parametrize("width", [1024, 4096])
+def test_routers_of_32_bits_sum_in_parts(pkg, tmp_path, knobs, forms, width):
+    """A row's two logits are of 12 and nearly alike, their experts' results opposite: what the layer adds is half of their difference, so the errors of the logits' sums are what the
+    stream shows.  In one launch with the update and in launches of their own, against 64 bits.  Emulated, relative to the logits: sums of 128 products and sums of those 2.1 to 2.2e-7,
+    sums of 256 2.9e-7; the ratio of two such errors over 1024 rows scatters by 0.03, so 1.2 lies four deviations from either."""
+    cfg = model([G.scan(8, 2, 2, 2, mlp=G.grouped_experts(2, 2, 32))], width=width, vocab=1024)
+    w, rng = G.weights(cfg, 92, clear_routes=False), np.random.default_rng(7)
+    silence(w, "o")
+    w["l0.norm2"][:], w["l0.mlp.correction"][:] = 1.0, 0.0
+    w["l0.mlp.router"] = G.bf16(rng.standard_normal((2, width)) * 17.0 * width ** -0.5)
+    r, rows = w["l0.mlp.router"].astype(np.float64), []
+    while len(rows) < 1024:
+        x = rng.standard_normal(width)
+        x = G.bf16(x - (r[0] - r[1]) * ((r[0] - r[1]) @ x / ((r[0] - r[1]) @ (r[0] - r[1]))))
+        level = r[0] @ x / np.sqrt(np.mean(x.astype(np.float64) ** 2))
+        if 4.0 < abs(level) < 28.0:                                           # (negative, where weights follow the logits)
+            rows.append(-x if level > 0 else x)
+    w["embed"] = np.array(rows, np.float32)
+    for part in ("gate", "up"):
+        w["l0.mlp.e1." + part] = w["l0.mlp.e0." + part]
+    w["l0.mlp.e1.down"] = -w["l0.mlp.e0.down"]
+    x = w["embed"].astype(np.float64)
+    h = L.unit_rms(x, cfg["norm"]["eps"])
+    y = (L.silu(h @ w["l0.mlp.e0.gate"].T.astype(np.float64)) * (h @ w["l0.mlp.e0.up"].T.astype(np.float64))) @ w["l0.mlp.e0.down"].T.astype(np.float64)
+    s = L.sigmoid(h @ r.T)
+    want, path, errors = (s[:, 0] - s[:, 1]) / s.sum(axis=1), G.write_checkpoint(tmp_path, cfg, w), []
+    for off in (None, 1):
+        knobs.set(NO_STREAM_ROUTE=off)
+        forms.reset()
+        m, got = load(pkg, path, "float32"), []
+        m.enable_taps()
+        for i in range(0, 1024, 128):
+            m.forward_rows([(1, np.arange(i, i + 128, dtype=np.uint32), 0)], [127])
+            got.append(m.read_taps(128)[0].astype(np.float64))
+            m.release(1)
+        assert bool(forms.hits().get("stream_route")) == (not off)
+        got = ((np.concatenate(got) - x) * y).sum(axis=1) / (y * y).sum(axis=1)
+        errors.append(np.sqrt(np.mean((got - want) ** 2)))
+    assert errors[0] < 1.2 * errors[1], errors
+
+
 MISTAKES = {"weights read the correction": lambda s, c: s + c, "excluded choices are 0": None, "a group counts by its best": None, "choice without the correction": None}
 
 
