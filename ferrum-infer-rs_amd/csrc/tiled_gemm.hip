@@ -807,7 +807,7 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     if (mt == 2 && !ext && tiles16 > 512 && tiles16 <= 768) J = 3;
     if (mt == 2 && !ext && tiles16 > 768 && tiles16 <= 896 && loads >= 64 && loads <= 128) J = 4;
     if (mt == 2 && !ext && tiles16 >= 4096 && loads >= (g.m > 24 ? 48 : 96) && g.n % 64 == 0) J = 4;       // (a vocabulary)
-    if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : knobs().tiled_j > 2 && mt == 2 && !ext ? knobs().tiled_j : 2;
+    if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : (knobs().tiled_j == 3 || knobs().tiled_j == 4) && mt == 2 && !ext ? knobs().tiled_j : 2;
     if (gated) J = 2;
     const long cols = cdiv(g.n, 16 * J), blocks = (long)rbs * cols * zs;
     int nw = mt == 1 && !rows.id && ((blocks > 512 && loads >= 64 && (!wide || loads % 32 == 0)) || (blocks <= 256 && J == 1 && loads >= 96)) ? 8 : 4, kw = nw;

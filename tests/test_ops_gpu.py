@@ -473,6 +473,15 @@ def test_few_rows_of_several_row_tiles(env, m, n, k, j, kw, knobs, forms):
     forms.require("tiled_gemm", *(["tiled_gemm_cols64"] if j == 4 and m <= 32 else []))
 
 
+@pytest.mark.parametrize("j", [3, 5, 6])
+def test_forced_columns_that_no_form_has(env, j, knobs, forms):
+    """A forced number of 16-column tiles for which there is no kernel is 2, as it is with one and four row tiles: every column is written."""
+    knobs.set(TILED_J=j, TILED_BIG_MIN_TILES=10 ** 6, TILED_MIN_TILES=-1)
+    for m in (10, 20, 50):
+        _few_rows(env, m, 320, 96)
+    assert bool(forms.hits().get("tiled_gemm_cols48")) == (j == 3)
+
+
 @pytest.mark.parametrize("m,n,k,form", [(17, 8224, 96, 48), (32, 8256, 2080, 48), (20, 12288, 64, 48), (32, 8192, 2048, None), (32, 12320, 2048, 64), (17, 14336, 4096, 64), (32, 12320, 1024, None),
                                         (32, 14368, 2048, None), (16, 9280, 2048, None)])
 def test_columns_past_a_round_of_workgroups(env, m, n, k, form, knobs, forms):
