@@ -804,8 +804,11 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     //   32 × 12320       8.6 | 10.0 |  8.6    13.2 | 16.3 | 12.3    23.5 | 28.9 | 21.1    43.6 | 52.5 | 41.8
     //   32 × 14336       8.8 | 10.6 |  9.2    13.6 | 17.1 | 13.2    24.4 | 30.1 | 22.6    44.5 | 55.6 | 47.1
     //   32 × 16384       9.3 | 10.8 |  9.8    14.5 | 17.3 | 14.5    26.4 | 30.6 | 24.9    46.3 | 57.1 | 53.7
-    if (mt == 2 && !ext && tiles16 > 512 && tiles16 <= 768) J = 3;
-    if (mt == 2 && !ext && tiles16 > 768 && tiles16 <= 896 && loads >= 64 && loads <= 128) J = 4;
+    // Slabs of K gain by 48 columns as one slab does, by 64 nothing; groups, the heads' own short columns, by neither.  32 rows, 32 | 48 | 64 columns:
+    //   2112 × 8192 in 4 slabs  10.8 |  9.1 |  9.5     3072, 4  11.6 | 11.2 | 12.1     3584, 4  12.3 | 14.5 | 12.8     5120, 2  18.0 | 15.6 | 17.1     7168, 2  21.0 | 25.1 | 21.4
+    //   23 groups of 512 × 128   4.0 |  4.8 |  5.9     24 of 512 × 128  4.4 | 5.3 | 7.0     72 of 128 × 512  6.8 | 6.8 | 6.8     96 of 128 × 512  7.0 | 8.2 | 7.2
+    if (mt == 2 && !ext && g.groups == 1 && tiles16 > 512 && tiles16 <= 768) J = 3;
+    if (mt == 2 && !ext && zs == 1 && tiles16 > 768 && tiles16 <= 896 && loads >= 64 && loads <= 128) J = 4;
     if (mt == 2 && !ext && tiles16 >= 4096 && loads >= (g.m > 24 ? 48 : 96) && g.n % 64 == 0) J = 4;       // (a vocabulary)
     if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : (knobs().tiled_j == 3 || knobs().tiled_j == 4) && mt == 2 && !ext ? knobs().tiled_j : 2;
     if (gated) J = 2;

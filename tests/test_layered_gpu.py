@@ -627,6 +627,19 @@ def test_sections_within_a_wave_s_columns(pkg, cases, knobs, forms, name, j, dty
     assert forms.hits().get(f"tiled_gemm_cols{16 * j}")
 
 
+@pytest.mark.parametrize("layer,width", [(G.attention(20, 32, 16, 32, 32, 512, 40), 72), (G.attention(24, 32, 16, 32, 32, 512, 40), 72), (G.recurrent(24, 2, 2, ff=8192), 3104)])
+def test_groups_and_slabs_past_a_round_of_workgroups(pkg, tmp_path, layer, width, forms):
+    """As many 16-column tiles as make a wave of one projection take 48 or 64 columns, but in groups (the heads' own projections to 512 latents) or in four slabs of K: 32 columns,
+    the faster form there."""
+    cfg = one_layer(layer, width=width)
+    w, t = G.weights(cfg, 41), toks(cfg, 24, 16)
+    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), "bfloat16", seqs=24)
+    forms.reset()
+    got = m.forward_rows([(i, t[i:i + 1], 0) for i in range(24)], list(range(24)))
+    assert not forms.hits().get("tiled_gemm_cols48" if width == 72 else "tiled_gemm_cols64"), forms.hits()
+    assert rel(got, np.concatenate([L.forward(cfg, w, t[i:i + 1]) for i in range(24)])) < TOL["bfloat16"]
+
+
 EVEN = {"nerenex": lambda: G.config(256, 260, [G.recurrent(256, 2, 3, ff=384), G.attention(20, 64, 32, 48, 128, 256, 130, ff=640), G.recurrent(640, 5, 2, ff=128)], mult=0.6),
         "safolorn": lambda: G.safolorn(128, 260, 40, [G.sink_attention(8, 64, 32, 64, 256, 1e5, G.LONG, mlp=G.glu(384, 1.5)), G.sink_attention(4, 64, 32, 32, 256, 1e5, G.LONG, mlp=G.experts(5, 2, 256))]),
         "segetar": lambda: G.segetar(256, 260, [G.scan(256, 16, 128, 4, mlp=G.dense(384)), G.gated_pair(8, 2, 64, 64, 130, 4, 64, 64, mlp=G.grouped_experts(6, 2, 128, 2, 1))]),
