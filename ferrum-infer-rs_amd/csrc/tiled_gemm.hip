@@ -411,11 +411,20 @@ __global__ __launch_bounds__(256, PER_CU) void tiled_gemm_big_kernel(TiledGemm<E
             for (int j = 0; j < NJ; j++) *reinterpret_cast<f16x4*>(tile + ((wm * MI + i) * 16 + b) * PITCH + (wn * NJ + j) * 16 + 4 * a) = __builtin_convertvector(acc[i][j] + 0.f, f16x4);      // (− 0 → 0, as the sum with a bias that is none)
         if ((int)threadIdx.x < T::ROWS) {                                // (whole waves)
             const int tok = min(m0 + (int)threadIdx.x, to.m_total - 1);
-            int seq = 0;                                                 // the last whose first token is not behind this one
-            for (int s0 = 0; s0 < to.num_seqs; s0 += 64) {
-                const int first = (int)to.cu[min(s0 + lane, to.num_seqs - 1)], some = min(64, to.num_seqs - s0);
-                for (int j = 0; j < some; j++)
-                    if (__builtin_amdgcn_readlane(first, j) <= tok) seq = s0 + j;
+            // The last sequence that begins no later than a row's token: of 64 sequences at a time, from the 64 on that hold the tile's first token, one ballot for all rows and a step
+            // for each that begins among the wave's (a step for each of all sequences: 8192 × 4096 × 1024 with 512 of them 43 µs longer)
+            const uint32_t from = (uint32_t)min(m0 + wave * 64, to.m_total - 1), upto = (uint32_t)min(m0 + wave * 64 + 63, to.m_total - 1);
+            int seq = 0, s0 = 0;
+            if (to.num_seqs > 64) s0 = 64 * (63 - __clzll((long long)__ballot(lane * 64 < to.num_seqs && to.cu[min(lane * 64, to.num_seqs - 1)] <= from)));
+            for (; s0 < to.num_seqs; s0 += 64) {
+                const uint32_t first = s0 + lane < to.num_seqs ? to.cu[s0 + lane] : 0xffffffffu;
+                const unsigned long long before = __ballot(first <= from), among = __ballot(first <= upto);
+                if (before) seq = s0 + 63 - __clzll((long long)before);
+                for (unsigned long long rest = among & ~before; rest; rest &= rest - 1) {
+                    const int j = __builtin_ctzll(rest);
+                    if (__builtin_amdgcn_readlane((int)first, j) <= tok) seq = s0 + j;
+                }
+                if (among != ~0ull) break;
             }
             const int pos = (int)to.pos_offsets[seq] + (tok - (int)to.cu[seq]);
             pos_of[threadIdx.x] = pos;

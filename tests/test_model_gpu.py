@@ -309,6 +309,44 @@ def test_unquantised_qkv_with_its_rows(pkg, size, nq, nkv, qk_norm, knobs, forms
     assert np.isfinite(got[0]).all() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
 
 
+@pytest.mark.parametrize("seqs", [63, 64, 65, 130])
+def test_unquantised_qkv_of_many_sequences(pkg, seqs, knobs, forms):
+    """Where a tile's rows go, with its sequences on both sides of a 64th one and up to 40 of them beginning in a wave's rows: the bits that a launch of its own leaves."""
+    from tests import modelgen
+    tm = modelgen.TinyModel(False, layers=2, hidden=256, nq=4, nkv=2, hd=128, inter=256, vocab=512, seed=178, max_seq_len=256, dense_proj=True, tied=True)
+    lens = [[1 + i * 7 % 5 if i != 40 else 150 for i in range(seqs)], [1 if i % 64 > 20 else 4 for i in range(seqs)]]
+    toks = np.random.default_rng(6).integers(0, 512, size=(seqs, 160)).astype(np.uint32)
+    got = []
+    for tiles in (10 ** 6, 1):
+        knobs.set(QKV_MIN_TILES=tiles, TILED_BIG_MIN_TILES=1, TILED_WIDE_MIN_TILES=10 ** 6, TILED_HALF_MAX_TILES=0)
+        forms.reset()
+        hm = tm.hip_model(pkg, kv_num_blocks=2 * seqs + 16, max_seqs=seqs, max_tokens=640)
+        out = [hm.unified_forward([(i, toks[i, at:at + n], at, True) for i, (at, n) in enumerate(zip(ats, ns))], want_logits=True)[1] for ats, ns in ((seqs * [0], lens[0]), lens)]
+        got.append(np.concatenate(out))
+        assert forms.hits().get("f16_qkv", 0) == (4 if tiles == 1 else 0)
+        del hm
+    assert np.isfinite(got[0]).all() and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
+def test_unquantised_qkv_of_many_sequences_costs_no_search(pkg, knobs):
+    """8192 tokens of 512 sequences through four layers of 1024 columns: 100 us less than with a launch of its own; a step for each sequence in each tile made it 85 us more."""
+    import time
+    from tests import modelgen
+    tm = modelgen.TinyModel(False, layers=4, hidden=1024, nq=16, nkv=8, hd=128, inter=256, vocab=512, seed=179, max_seq_len=256, dense_proj=True, tied=True)
+    hm = tm.hip_model(pkg, kv_num_blocks=600, max_seqs=512, max_tokens=8192)
+    toks = np.random.default_rng(7).integers(0, 512, size=(512, 16)).astype(np.uint32)
+    best = {}
+    for turn in range(12):
+        for tiles in (10 ** 6, 256):
+            knobs.set(QKV_MIN_TILES=tiles)
+            t = time.perf_counter()
+            hm.unified_forward([(i, toks[i], 0, i == 0) for i in range(512)])
+            best[tiles] = min(best.get(tiles, 1.0), time.perf_counter() - t)
+            for i in range(512):
+                hm.release(i)
+    assert best[256] < best[10 ** 6], best
+
+
 @pytest.mark.parametrize("tokens", [1, 100])
 @pytest.mark.parametrize("activation,lo,hi", [(1, -5.5, -2.0), (1, -2.0, 3.0), (0, -12.0, 12.0)])
 def test_unquantised_activation_errs_by_its_rounding(pkg, activation, lo, hi, tokens, knobs, forms):
