@@ -628,6 +628,13 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s, const Rows& to = {})
 // A wave with columns of several kinds, or rare ones, finishes its tile 20 – 26 µs later, which four rounds make up for (K = 2048, µs of the latter | of the former: 9472 columns
 // with several sections, 1000 rows 55 | 75, 3000 108 | 125, 5000 163 | 176, 8192 281 | 277, 12000 380 | 372; 20224 columns, 600 rows 62 | 75, 3000 219 | 209, 8192 563 | 485).
 static long big_tiles(const GemmRows& rows, int m, int n, int groups, int r, int c) { return (long)(rows.id ? rows.max_blocks * (rows.block / r) : cdiv(m, r)) * cdiv(n, c) * groups; }
+// rounds of 128 × 256 and of 256 × 256, and the time of either
+struct BigRounds { long halves, wholes; float half_us, whole_us; };
+template <typename E>
+static BigRounds big_rounds(const TiledGemm<E>& g) {
+    const long halves = cdiv(big_tiles(g.rows, g.m, g.n, g.groups, 128, 256), 256), wholes = cdiv(big_tiles(g.rows, g.m, g.n, g.groups, 256, 256), 256);
+    return {halves, wholes, halves * (5.5f + 0.01185f * g.k), wholes * (11.6f + 0.0201f * g.k)};
+}
 template <typename E>
 bool tiled_gemm_takes_256(const TiledGemm<E>& g) {
     if constexpr (sizeof(E) == 4) {
@@ -636,10 +643,10 @@ bool tiled_gemm_takes_256(const TiledGemm<E>& g) {
         if (knobs().tiled_256 < 0 || (g.rows.id && g.rows.block % 256)) return false;
         if (knobs().tiled_256 == 0) {
             if (knobs().tiled_wide_min_tiles >= 0) return false;        // (a forced size of the tiles below stays what it is)
-            const long halves = cdiv(big_tiles(g.rows, g.m, g.n, g.groups, 128, 256), 256), rounds = cdiv(big_tiles(g.rows, g.m, g.n, g.groups, 256, 256), 256);
+            const BigRounds r = big_rounds(g);
             bool mixed = false;
             for (int i = 0; i < g.nsec; i++) mixed |= gemm_rare_act(g.sec[i].act) || g.sec[i].begin % 128;
-            if (halves <= 1 || (mixed && rounds < 4) || (g.k <= 1024 && (rounds == 2 || rounds == 3)) || rounds * (11.6f + 0.0201f * g.k) >= (g.k > 512 ? 0.97f : 0.93f) * halves * (5.5f + 0.01185f * g.k)) return false;
+            if (r.halves <= 1 || (mixed && r.wholes < 4) || (g.k <= 1024 && (r.wholes == 2 || r.wholes == 3)) || r.whole_us >= (g.k > 512 ? 0.97f : 0.93f) * r.half_us) return false;
         }
         return tiled_gemm_wide_supports(g);
     }
@@ -672,8 +679,16 @@ static int launch_big(const TiledGemm<E>& g, hipStream_t s) {
 // The rows of a q|k|v projection by its own launch: 5.7 µs more of it at 2048 × 4096 × 1024 (23.8 → 29.5) for a launch of 11.7 that reads and writes them once more.  From a
 // tile of 128 × 128 for each CU on; µs of a prompt through 14 layers, launch of its own | this: 488 tokens (128 tiles) 1087 | 1149, 700 (192) 1566 | 1570, 986 (256) 1433 | 1408,
 // 1500 (384) 1998 | 1936, 2048 (512) 2034 | 1941, 4096 4146 | 4009, 8192 5932 | 5572.
+// Where the projection alone would run in tiles of 256 × 256, only if these are faster by less than what the launch saves, 0.65 µs for a million numbers.  µs that a layer takes
+// longer with this (four layers of it, 128 tokens a sequence and more):
+//   tiles of 256 × 256:    K = 1024, 4096 columns   3000 tokens − 3, 4096 − 8            2048, 4096    3000 + 0, 4096 − 7, 8192 − 10     2048, 5120    2048 + 2, 3000 − 3
+//                             3072, 5120            2048 + 10, 3000 + 5                  4096, 6144    1400 + 10, 2048 + 13, 8192 + 6
+//   smaller ones:             1024, 4096            1024 − 2, 2048 − 6, 8192 − 26        2048, 5120    1024 − 3, 4096 − 8, 8192 − 28
+//                             3072, 5120            1024 − 5, 4096 − 6, 8192 − 37        4096, 6144    700 − 3, 3000 − 10, 4096 − 17
 bool tiled_gemm_qkv_supports(const TiledGemm<_Float16>& g, const QkvRows& to) {
-    return big_tiles(g.rows, g.m, g.n, 1, 128, 128) >= knobs().qkv_min_tiles && g.m == to.m_total && g.n == (to.q_heads + 2 * to.kv_heads) * 128 && !g.bias && !g.nsec;
+    if (big_tiles(g.rows, g.m, g.n, 1, 128, 128) < knobs().qkv_min_tiles || g.m != to.m_total || g.n != (to.q_heads + 2 * to.kv_heads) * 128 || g.bias || g.nsec) return false;
+    const BigRounds r = big_rounds(g);
+    return !tiled_gemm_takes_256(g) || r.half_us - r.whole_us + 2.f <= 0.65e-6f * g.m * g.n;
 }
 int tiled_gemm_qkv(const TiledGemm<_Float16>& g, const QkvRows& to, hipStream_t s) {
     FH_REQUIRE(tiled_gemm_qkv_supports(g, to), "tiled_gemm_qkv: %d rows of %d + 2 × %d heads", g.m, to.q_heads, to.kv_heads);

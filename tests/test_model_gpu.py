@@ -347,6 +347,20 @@ def test_unquantised_qkv_of_many_sequences_costs_no_search(pkg, knobs):
     assert best[256] < best[10 ** 6], best
 
 
+@pytest.mark.parametrize("hidden,nq,nkv,tokens,fused", [(1024, 16, 8, 896, False), (1024, 16, 8, 1024, True), (1024, 16, 8, 4096, True), (2048, 16, 8, 3000, False), (2048, 16, 8, 4096, True),
+                                                         (2048, 32, 4, 2048, False), (2048, 32, 4, 3000, True), (4096, 32, 8, 1024, True), (4096, 32, 8, 2048, False), (4096, 32, 8, 3000, True)])
+def test_unquantised_qkv_takes_its_rows_along_where_that_is_faster(pkg, hidden, nq, nkv, tokens, fused, forms):
+    """Where tiles of 256 x 256 are faster by more than the launch that places the rows takes, they are kept (2048 tokens of 6144 columns, K = 4096: 12 us a layer)."""
+    from tests import modelgen
+    tm = modelgen.TinyModel(False, layers=1, hidden=hidden, nq=nq, nkv=nkv, hd=128, inter=256, vocab=512, seed=180, max_seq_len=4096, dense_proj=True, tied=True)
+    hm = tm.hip_model(pkg, kv_num_blocks=260, max_seqs=1, max_tokens=4096)
+    forms.reset()
+    logits = hm.unified_forward([(0, np.arange(tokens, dtype=np.uint32) % 512, 0, True)], want_logits=True)[1]
+    h = forms.hits()
+    assert bool(h.get("f16_qkv")) == fused and (fused or hidden == 1024 or h.get("tiled_gemm_256x256")), h
+    assert np.isfinite(logits).all()
+
+
 @pytest.mark.parametrize("tokens", [1, 100])
 @pytest.mark.parametrize("activation,lo,hi", [(1, -5.5, -2.0), (1, -2.0, 3.0), (0, -12.0, 12.0)])
 def test_unquantised_activation_errs_by_its_rounding(pkg, activation, lo, hi, tokens, knobs, forms):
