@@ -685,17 +685,20 @@ static int grouped_keys(const GroupedDims& d, const GroupedBuffers<E>& b, const 
         attr = true;
     }
     const int G = d.heads / d.kv_heads, tiles = v.single ? v.num_seqs * cdiv(G, 16) : (int)((long)v.T * G / 16) + v.num_seqs;
-    // Split the keys while the launch has fewer workgroups than stay resident and a split keeps ≥ 128 keys.  Steps in 16 bits that prepare their rows themselves: a launch for the
-    // splits costs as much as three rounds of 128 keys, so more than 512 a split, and up to 128 workgroups, which pull what the memory gives.  µs of a step with 1 | 2 | 4 | 8
-    // splits (fororax, a layer with 4 heads of keys; segetar, four of them):
-    //   fororax   1 × 200 keys   181 | 184 | 184 | 186     1 × 1000   193 | 190 | 188 | 190     1 × 2000   208 | 199 | 195 | 194     1 × 4000   236 | 218 | 208 | 203
-    //             8 × 200        211 | 214 | 215 | 219     8 × 1000   223 | 225 | 221 | 224     8 × 2000   237 | 230 | 227 | 227
-    //            24 × 200        238 | 242 | 246 | 253    24 × 1000   249 | 251 | 254 | 260    24 × 2000   273 | 270 | 273 | 279
-    //   segetar   1 × 90         363 | 374 | 377 | 389     1 × 1000   407 | 396 | 397 | 404    32 × 90     552 | 565 | 573 | 604    32 × 1000   615 | 624 | 632 | 661
+    // Split the keys while the launch has fewer workgroups than stay resident and a split keeps ≥ 128 keys.  Steps in 16 bits that prepare their rows themselves: the launch that joins
+    // the splits costs as much as three rounds of 128 keys, so none up to 512 keys, then four, and more where a split keeps more than 512.  128 workgroups pull
+    // what the memory gives: beyond 64 only from 1536 keys on.  µs of a step with 1 | 2 | 4 | 8 splits (captured for up to as many keys as the next multiple of 256;
+    // two layers with 4 heads of keys at fororax's sizes, and segetar's three):
+    //   fororax   1 × 450 keys   174 | 178 | 177 | 180     1 × 700    181 | 181 | 179 | 180     1 × 960   185 | 182 | 177 | 179     1 × 1950   207 | 193 | 183 | 183     1 × 3950   255 | 218 | 197 | 191
+    //             8 × 450        204 | 208 | 206 | 212     8 × 700    211 | 211 | 210 | 213     8 × 960   210 | 209 | 205 | 208     8 × 1950   233 | 220 | 211 | 213
+    //            16 × 450        217 | 221 | 221 | 230    16 × 960    221 | 222 | 220 | 229    16 × 1950  246 | 234 | 230 | 239
+    //            24 × 450        228 | 233 | 238 | 252    24 × 960    233 | 235 | 240 | 252    24 × 1950  256 | 249 | 254 | 266    31 × 960     241 | 246 | 252 | 265
+    //            31 × 1950       266 | 262 | 268 | 282
+    //   segetar   1 × 450        386 | 385 | 388 | 397     1 × 960    410 | 409 | 396 | 405     4 × 960   463 | 459 | 454 | 458     8 × 960    484 | 480 | 478 | 483
     const int keys = (int)std::min<long>(v.max_keys, (long)d.window + 16), wgs = tiles * d.kv_heads;
     int ns = 1;
     if (step && sizeof(E) == 2)
-        while (ns < 16 && wgs * ns < 128 && keys > ns * 512) ns *= 2;
+        while (ns < 16 && wgs * ns <= 128 && keys > std::max(ns < 4 ? 512 : ns * 512, wgs * ns > 64 ? 1536 : 0)) ns *= 2;
     else
         while (ns < 16 && wgs * ns < 512 && keys >= 2 * ns * 128) ns *= 2;
     if (knobs().grouped_splits > 0) ns = std::min(16, knobs().grouped_splits);

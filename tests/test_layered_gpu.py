@@ -429,17 +429,19 @@ def test_grouped_steps_prepare_their_rows(pkg, cases, knobs, forms, name, splits
     assert err[0] < TOL[dtype] if dtype == "float32" else err[0] < err[1] + 2.0 ** -6, err
 
 
-@pytest.mark.parametrize("name,dtype,keys,form", [("grouped", "bfloat16", 512, "grouped_attn_keys"), ("grouped", "bfloat16", 513, "grouped_attn_split"),
-                                                  ("grouped", "bfloat16", 1025, "grouped_attn_split"), ("latent", "float32", 127, "latent_attn"), ("latent", "float32", 128, "latent_attn_split"),
-                                                  ("latent", "bfloat16", 256, "latent_attn"), ("latent", "bfloat16", 257, "latent_attn_split")])
-def test_keys_of_a_step_on_both_sides_of_a_split(pkg, tmp_path, name, dtype, keys, form, forms):
-    """A step over as many keys as one split takes, and over one more, against the oracle."""
-    cfg = G.segetar(72, 50, [G.gated_pair(8, 4, 24, 32, 2000, 2, 16, 16)]) if name == "grouped" else one_layer(G.attention(8, 32, 16, 32, 32, 64, 2000))
+@pytest.mark.parametrize("name,dtype,rows,keys,form", [("grouped", "bfloat16", 1, 512, "grouped_attn_keys"), ("grouped", "bfloat16", 1, 513, "grouped_attn_split"),
+                                                       ("grouped", "bfloat16", 1, 1025, "grouped_attn_split"), ("grouped", "bfloat16", 33, 1025, "grouped_attn_keys"),
+                                                       ("grouped", "bfloat16", 33, 1537, "grouped_attn_split"), ("latent", "float32", 1, 127, "latent_attn"),
+                                                       ("latent", "float32", 1, 128, "latent_attn_split"), ("latent", "bfloat16", 1, 256, "latent_attn"),
+                                                       ("latent", "bfloat16", 1, 257, "latent_attn_split")])
+def test_keys_of_a_step_on_both_sides_of_a_split(pkg, tmp_path, name, dtype, rows, keys, form, forms):
+    """A step over as many keys as one split takes, and over one more, against the oracle; with 66 workgroups a split takes more.  (Of several rows the others are of one token.)"""
+    cfg = G.segetar(72, 50, [G.gated_pair(8, 4 if rows == 1 else 2, 24, 32, 2000, 2, 16, 16)]) if name == "grouped" else one_layer(G.attention(8, 32, 16, 32, 32, 64, 2000))
     w, t = G.weights(cfg, 37), toks(cfg, keys, 15)
-    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), dtype, tokens=1100)
+    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), dtype, seqs=max(rows, 4), tokens=1600)
     m.forward_rows([(1, t[:-1], 0)], [])
     forms.reset()
-    got = m.forward_rows([(1, t[-1:], keys - 1)], [0])
+    got = m.forward_rows([(1, t[-1:], keys - 1)] + [(2 + i, t[i:i + 1], 0) for i in range(rows - 1)], [0])
     assert forms.hits().get(form) == 1, forms.hits()
     assert rel(got, L.forward(cfg, w, t)[-1:]) < TOL[dtype]
 
