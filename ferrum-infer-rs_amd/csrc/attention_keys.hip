@@ -51,7 +51,7 @@ __global__ __launch_bounds__(64 * NW_, 2) void paged_prefill_attn_keys_kernel(At
     const int kv_end = __builtin_amdgcn_readfirstlane(pos0 + t_last + 1);
     const int kv_begin = __builtin_amdgcn_readfirstlane(p.sliding_window > 0 ? max(0, pos0 + t_first + 1 - p.sliding_window) : 0);
     const int nblocks = cdiv_dev(kv_end, KV_BLOCK);
-    const int first = kv_begin / (NB * KV_BLOCK) + wave, pairs = (nblocks + NB - 1) / NB;      // steps of two blocks: this wave's are first, first + 4, …
+    const int first = kv_begin / (NB * KV_BLOCK) + wave, pairs = (nblocks + NB - 1) / NB;      // steps of two blocks: this wave's are first, first + NW, …
 
     typedef const int32_t __attribute__((address_space(4))) Table;           // (not written in this launch: scalar loads)
     Table* bt = (Table*)(uintptr_t)(p.block_tables + (long)seq * p.max_blocks);

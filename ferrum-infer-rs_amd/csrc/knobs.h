@@ -178,6 +178,7 @@ enum Form : int {
     FORM_CHAIN_ROWS,            // decode chain: a forward's head made its rows ready
     FORM_MOE_ROWS_256,          // layered experts: sorted rows in blocks of 256
     FORM_DONE_AGAIN,            // a call whose in-launch waits gave up was done again in separate launches
+    FORM_IDS_LATE,              // a decode call whose ids did not come while they were watched for: the stream's end was waited for
     FORM_ATTN_KEYS,             // prompt attention, each wave of a 64-row workgroup on keys of its own: four waves
     FORM_ATTN_KEYS_WIDE,        // … eight
     FORM_F16_QKV,               // unquantised q|k|v of a prompt, normed, rotated and stored by its launch

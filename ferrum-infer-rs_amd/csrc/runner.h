@@ -99,7 +99,7 @@ struct FerrumHipModel {
     int chain_parity = 0;                 // … and of the decode chain launch (chain.hip)
     int em2_parity = 0;                   // which half the next merged launch counts in (enqueue order = stream order)
     bool em2_failed = false;              // a bounded in-launch wait gave up once: the two-launch form from then on
-    unsigned* inlaunch_timeouts = nullptr; // pinned host word (device-visible): bumped by any in-launch wait that gave up; read after every host sync
+    unsigned* inlaunch_timeouts = nullptr; // pinned host word (device-visible): bumped by any in-launch wait that gave up; read when a call's results are in host memory
     unsigned inlaunch_timeouts_seen = 0;
     int route_parts = 4;                  // expert parts per token in the decode route kernel (1 = single-workgroup kernel)
     bool fuse_rope_attn = true;           // decode: QK-norm + RoPE + KV write inside the attention launch
@@ -150,6 +150,7 @@ struct FerrumHipModel {
     // decode-steps state
     uint32_t* history = nullptr;   // [steps, sequences] sampled ids, pinned: written by the steps, read by the host
     int history_cap = 0;
+    bool steps_queued = false;     // a call's steps may still write there
     int32_t* step_counter = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;

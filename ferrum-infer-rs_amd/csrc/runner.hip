@@ -300,7 +300,7 @@ static void drop_graph(FerrumHipModel* m) {
 }
 
 // Tensor / expert / vocabulary parallel: a one-shot all-reduce or all-gather whose wait for a peer gave up left the rank's un-reduced partial in
-// the output — ids sampled from it must not be handed back as a success.  Called after every host synchronisation of a forward.
+// the output — ids sampled from it must not be handed back as a success.  Called when a forward's results are in host memory, which is behind every wait of it.
 static int check_peer_waits(FerrumHipModel* m) {
     if (const unsigned n = comm_take_timeouts(m->comm)) {
         drop_graph(m);
@@ -346,11 +346,13 @@ static int copy_results(FerrumHipModel* m, void* dst, const void* src, size_t by
 // Sampled ids in pinned memory, which a step's last kernel writes last: the host watches for them (a stream's synchronisation wakes up 10 – 18 µs later: a call of one
 // step through 6 layers 355 → 339 µs, 8 expert layers 356 → 345).  The kernel may still be leaving then, so the stream is waited for
 // where something is taken away that it was launched with.  false: none after some milliseconds, and the stream's end has to be waited for.
+// What earlier kernels of the stream wrote to host memory (ids of the steps before, waits that gave up) is there when an id of the last one is: these are writes of
+// system scope, a kernel has ended with all its writes done before the next begins, and the id is read with acquire order.
 constexpr uint32_t NO_ID = 0xFFFFFFFFu;
 static bool ids_there(const uint32_t* ids, int n) {
     const auto t0 = std::chrono::steady_clock::now();
     for (int i = 0; i < n; i++)
-        for (unsigned spins = 1; *reinterpret_cast<const volatile uint32_t*>(ids + i) == NO_ID; spins++) {
+        for (unsigned spins = 1; __atomic_load_n(ids + i, __ATOMIC_ACQUIRE) == NO_ID; spins++) {
             __builtin_ia32_pause();
             if (spins % 256 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(4)) return false;
         }
@@ -2387,7 +2389,9 @@ int ferrum_hip_model_decode_steps(FerrumHipModel* m, const uint64_t* seq_ids, co
                 m->graph_max_kv = kv_bucket;
             }
         }
+        if (m->steps_queued) FH_CHECK_HIP(hipStreamSynchronize(m->stream));      // (a call that failed behind its first launch: its ids are none of this one's)
         std::fill_n(m->history + (size_t)(steps - 1) * n, n, NO_ID);
+        m->steps_queued = true;
         const int most = *std::max_element(parts.words, parts.words + parts.n);
         hipLaunchKernelGGL(decode_begin_kernel, dim3(cdiv(most, BEGIN_WORDS), parts.n), dim3(256), 0, m->stream, reinterpret_cast<const uint32_t*>(m->idx_host),
                            reinterpret_cast<uint32_t*>(m->idx_dev), parts, m->step_counter);
@@ -2398,7 +2402,11 @@ int ferrum_hip_model_decode_steps(FerrumHipModel* m, const uint64_t* seq_ids, co
             for (int st = 0; st < steps; st++)
                 if (int rc = enqueue_step()) return rc;
         }
-        if (!ids_there(m->history + (size_t)(steps - 1) * n, n)) FH_CHECK_HIP(hipStreamSynchronize(m->stream));
+        if (!ids_there(m->history + (size_t)(steps - 1) * n, n)) {
+            form_hit(FORM_IDS_LATE);
+            FH_CHECK_HIP(hipStreamSynchronize(m->stream));
+        }
+        m->steps_queued = false;
         return 0;
     })) return rc;
     if (out_tokens) memcpy(out_tokens, m->history, (size_t)steps * n * 4);

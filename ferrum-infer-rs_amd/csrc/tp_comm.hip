@@ -352,7 +352,7 @@ struct FerrumHipComm {
     bool peer_imported[8] = {};
     uint8_t** peers_dev = nullptr;        // device copy of peer_ptrs
     unsigned* state = nullptr;            // device: epoch, tickets, timeouts
-    unsigned* timeouts_host = nullptr;    // pinned host word bumped by a one-shot wait that gave up (read by the runner after every host sync)
+    unsigned* timeouts_host = nullptr;    // pinned host word bumped by a one-shot wait that gave up (read by the runner when a call's results are in host memory)
     unsigned timeouts_seen = 0;
     bool oneshot_failed = false;          // a one-shot call timed out: its output was the rank's un-reduced partial and the epochs may have diverged — the transport stays off
     bool finegrained = false;             // the comm buffer is fine-grained device memory (hipExtMallocWithFlags)
@@ -430,7 +430,7 @@ int comm_all_gather_bytes(FerrumHipComm* c, const void* in, void* out, size_t by
     return 0;
 }
 
-// Called by the runner after every host synchronisation of a forward: a one-shot wait that gave up skipped its reduction
+// Called by the runner when a forward's results are in host memory: a one-shot wait that gave up skipped its reduction
 // (the output kept the rank's partial).  Returns the number of new give-ups and turns the transport off for good.
 unsigned comm_take_timeouts(FerrumHipComm* c) {
     if (!c || !c->timeouts_host) return 0;

@@ -172,6 +172,34 @@ def test_long_block_tables_are_handed_over_at_once(pkg):
     assert best[32768] - best[512] < 110e-6, best
 
 
+def test_ids_that_come_late(pkg, forms):
+    """A call of 216 steps outlasts the milliseconds for which ids are watched for, and waits for the stream's end; calls of 8 steps do not.  The same ids, and a call goes on
+    behind either."""
+    m = pkg.HipModel(group_size=128, num_layers=4, hidden=1024, num_heads=8, num_kv_heads=4, head_dim=128, intermediate=2048, vocab=32768, has_qk_norm=1, activation=0, rms_eps=1e-6,
+                     rope_theta=1e6, max_seq_len=512, kv_num_blocks=3 * 33, max_seqs=3, max_tokens=64)
+    m.init_synthetic(3)
+    m.finalize()
+    prompt, got = [np.random.default_rng(i).integers(0, 32768, 9 + i).astype(np.uint32) for i in range(3)], []
+    for cuts in ([8] * 28, [216, 8]):
+        first, _ = m.unified_forward([(i, prompt[i], 0, True) for i in range(3)])
+        m.decode_steps([0, 1, 2], first, 1)                 # (captures the step)
+        for i in range(3):
+            m.release(i)
+        last, _ = m.unified_forward([(i, prompt[i], 0, True) for i in range(3)])
+        out, late = [], []
+        for n in cuts:
+            forms.reset()
+            ids = m.decode_steps([0, 1, 2], last, n)
+            late.append(forms.hits().get("ids_late", 0))
+            out.append(ids)
+            last = ids[-1]
+        got.append(np.concatenate(out))
+        for i in range(3):
+            m.release(i)
+        assert late[0] == (1 if cuts[0] == 216 else 0) and late[-1] == 0, late
+    assert np.array_equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("rows", [1, 8, 9, 40])
 def test_logits_by_way_of_pinned_portions(pkg, rows):
     """4 MiB at a time, three on their way: a part of one, one whole, a little more, more than the ring holds; bit for bit what a copy into pinned memory gives."""
