@@ -831,7 +831,9 @@ int tiled_gemm(const TiledGemm<E>& gin, hipStream_t s) {
     // Slabs of K gain by 48 columns as one slab does, by 64 nothing; groups, the heads' own short columns, by neither.  32 rows, 32 | 48 | 64 columns:
     //   2112 × 8192 in 4 slabs  10.8 |  9.1 |  9.5     3072, 4  11.6 | 11.2 | 12.1     3584, 4  12.3 | 14.5 | 12.8     5120, 2  18.0 | 15.6 | 17.1     7168, 2  21.0 | 25.1 | 21.4
     //   23 groups of 512 × 128   4.0 |  4.8 |  5.9     24 of 512 × 128  4.4 | 5.3 | 7.0     72 of 128 × 512  6.8 | 6.8 | 6.8     96 of 128 × 512  7.0 | 8.2 | 7.2
-    if (mt == 2 && !ext && g.groups == 1 && tiles16 > 512 && tiles16 <= 768) J = 3;
+    // A short K is over before workgroups are waited for, and what a wave does behind it for three tiles counts (32 | 48 columns):
+    //   17 × 8224 × 64   4.4 | 5.7     32 × 9280 × 128  4.3 | 5.1     17 × 12288 × 256  4.8 | 5.0     17 × 8224 × 512  5.0 | 5.3     32 × 9280 × 512  5.8 | 5.6     17 × 8224 × 768  6.3 | 6.1
+    if (mt == 2 && !ext && g.groups == 1 && tiles16 > 512 && tiles16 <= 768 && loads > 16) J = 3;
     if (mt == 2 && !ext && zs == 1 && tiles16 > 768 && tiles16 <= 896 && loads >= 64 && loads <= 128) J = 4;
     if (mt == 2 && !ext && tiles16 >= 4096 && loads >= (g.m > 24 ? 48 : 96) && g.n % 64 == 0) J = 4;       // (a vocabulary)
     if (knobs().tiled_j > 0) J = knobs().tiled_j == 1 ? 1 : (knobs().tiled_j == 3 || knobs().tiled_j == 4) && mt == 2 && !ext ? knobs().tiled_j : 2;

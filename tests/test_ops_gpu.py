@@ -482,7 +482,7 @@ def test_forced_columns_that_no_form_has(env, j, knobs, forms):
     assert bool(forms.hits().get("tiled_gemm_cols48")) == (j == 3)
 
 
-@pytest.mark.parametrize("m,n,k,form", [(17, 8224, 96, 48), (32, 8256, 2080, 48), (20, 12288, 64, 48), (32, 8192, 2048, None), (32, 12320, 2048, 64), (17, 14336, 4096, 64), (32, 12320, 1024, None),
+@pytest.mark.parametrize("m,n,k,form", [(17, 8224, 96, None), (17, 8224, 544, 48), (32, 8256, 2080, 48), (20, 12288, 64, None), (32, 9280, 512, None), (20, 12288, 576, 48), (32, 8192, 2048, None), (32, 12320, 2048, 64), (17, 14336, 4096, 64), (32, 12320, 1024, None),
                                         (32, 14368, 2048, None), (16, 9280, 2048, None)])
 def test_columns_past_a_round_of_workgroups(env, m, n, k, form, knobs, forms):
     """48 and 64 columns a wave on both sides of the lines where they begin and end; the last wave's columns there in whole and in parts."""
