@@ -636,10 +636,15 @@ __global__ __launch_bounds__(256, DS <= 4 ? 2 : 1) void grouped_attn_tile_kernel
     }
 }
 
-// Steps whose attention prepares its rows itself; heads of more than 128 dimensions would need more registers than there are
+// Steps whose attention prepares its rows itself; heads of more than 128 dimensions would need more registers than there are.  In 32 bits, where a CU holds one workgroup, only as
+// many as run at once: those behind them would wait for the rows' preparation, too.  µs of a step, prepared by a launch of its own | so (segetar, four such layers with 4 heads of keys):
+//   rows      16          32          64            128           256           400
+//   32 bits   789 | 782   971 | 961   1452 | 1452   2343 | 2348   3613 | 3656   5373 | 5458
+//   16 bits   510 | 484   580 | 554    714 |  683   1038 | 1018   1286 | 1291   1775 | 1778     (runs of one side differ by 10 in the last two)
 template <typename E>
 static bool grouped_step(const GroupedDims& d, const GroupedBuffers<E>& b, const BatchView& v) {
-    return v.single && !b.talk && !knobs().grouped_plain && !knobs().no_grouped_step && d.dp == d.vp && d.dp <= 128 && d.scale > 0.f;
+    return v.single && !b.talk && !knobs().grouped_plain && !knobs().no_grouped_step && d.dp == d.vp && d.dp <= 128 && d.scale > 0.f &&
+           (sizeof(E) == 2 || (long)v.num_seqs * cdiv(d.heads / d.kv_heads, 16) * d.kv_heads <= 256);
 }
 template <typename E>
 int grouped_prepare(const GroupedDims& d, const GroupedBuffers<E>& b, const BatchView& v, hipStream_t s) {

@@ -446,6 +446,20 @@ def test_keys_of_a_step_on_both_sides_of_a_split(pkg, tmp_path, name, dtype, row
     assert rel(got, L.forward(cfg, w, t)[-1:]) < TOL[dtype]
 
 
+@pytest.mark.parametrize("dtype,rows,alone", [("float32", 64, False), ("float32", 65, True), ("bfloat16", 65, False)])
+def test_rows_of_a_round_of_workgroups_prepare_themselves(pkg, tmp_path, dtype, rows, alone, forms):
+    """32 bits, 4 heads of keys: 256 workgroups run at once, and with more of them a launch of its own prepares the rows.  Second tokens, against the oracle."""
+    cfg = G.segetar(72, 50, [G.gated_pair(8, 4, 24, 32, 40, 2, 16, 16)])
+    w = G.weights(cfg, 43)
+    t = [toks(cfg, 2, 50 + i) for i in range(rows)]
+    m = load(pkg, G.write_checkpoint(tmp_path, cfg, w), dtype, seqs=rows)
+    m.forward_rows([(i, t[i][:1], 0) for i in range(rows)], [])
+    forms.reset()
+    got = m.forward_rows([(i, t[i][1:], 1) for i in range(rows)], list(range(rows)))
+    assert bool(forms.hits().get("grouped_attn_step")) != alone, forms.hits()
+    assert rel(got, np.stack([L.forward(cfg, w, t[i])[1] for i in range(rows)])) < TOL[dtype]
+
+
 def near_greedy(cfg, w, prompt, out, slack):
     """Every generated token's oracle logit is within `slack` (relative to the logits' rms) of the best one."""
     full = np.concatenate([prompt, out]).astype(np.uint32)
