@@ -116,7 +116,7 @@ static const char* const g_form_names[FORM_COUNT] = {
     "perm_producer", "moe_expert_major_pair", "decode_chain", "moe_deferred_merge", "dense_chain", "tp_allreduce_norm_fused", "moe_block_major_pair", "chain_attn_kv_splits", "chain_qkv_wide", "route_gemm_topk",
     "tiled_gemm", "tiled_gemm_big", "tiled_gemm_128x256", "tiled_gemm_128x128", "tiled_gemm_128x64", "tiled_gemm_64x64", "tiled_gemm_grouped", "tiled_gemm_grouped_big", "moe_route_sort", "latent_attn_plain", "latent_attn", "latent_attn_pair", "latent_attn_split", "latent_attn_expanded", "rglru_step", "rglru_scan",
     "grouped_attn_plain", "grouped_attn_keys", "grouped_attn_step", "grouped_attn_split", "grouped_attn_tile", "linear_step", "linear_chunk", "scan_step", "scan_chunk", "route_grouped",
-    "route_softmax", "talk_attn_plain", "talk_attn_keys", "talk_attn_tile", "talk_attn_tile_split", "w4_rows", "w4_gated", "f16_gated", "tiled_gemm_cols48", "tiled_gemm_cols64", "tiled_gemm_256x256", "chain_mlp", "chain_rows", "moe_rows_256", "done_again", "ids_late", "attn_keys", "attn_keys_wide", "f16_qkv", "stream_route"};
+    "route_softmax", "talk_attn_plain", "talk_attn_keys", "talk_attn_tile", "talk_attn_tile_split", "w4_rows", "w4_gated", "f16_gated", "tiled_gemm_cols48", "tiled_gemm_cols64", "tiled_gemm_256x256", "chain_mlp", "chain_rows", "moe_rows_256", "done_again", "ids_late", "attn_flash_64", "attn_keys", "attn_keys_wide", "f16_qkv", "stream_route"};
 const char* form_name(int f) { return f >= 0 && f < FORM_COUNT ? g_form_names[f] : nullptr; }
 }  // namespace fh
 

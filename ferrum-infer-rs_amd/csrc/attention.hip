@@ -637,9 +637,9 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void paged_prefill_attn_ker
 // operand against Pᵀ: every lane's accumulator then holds Σ_keys P of its query row, rescaled by α like O), and steps whose 64
 // keys are visible to every row of a tile (all but the diagonal ones) run a mask-free body.  Same staging, tile layout and
 // per-row arithmetic otherwise (Sᵀ = K·Qᵀ, lane-local exp2, Oᵀ += Vᵀ·Pᵀ); l is the sum of the fp16 P the numerator uses.
-template <int HD>
+template <int HD, int MT>
 __global__ __launch_bounds__(256, 2) void paged_prefill_attn64_kernel(AttnArgs p) {
-    constexpr int NW = 4, MT = 2, DT = HD / 16, KS = HD / 32, TILE = 16 * HD;
+    constexpr int NW = 4, DT = HD / 16, KS = HD / 32, TILE = 16 * HD;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     __half* lds_kv = reinterpret_cast<__half*>(smem);          // [2 stages][2 pairs][K0, K1, V0, V1][TILE]; reused by the epilogue
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -1167,22 +1167,41 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
         form_hit(FORM_ATTN_RESIDENT);
         return 0;
     }
-    // head_dim 128 has two forms.  Workgroups of 128 rows share keys in LDS; in those of 64 rows each wave reads keys of its own (attention_keys.hip).  A workgroup
-    // passes the longest keys of a prompt alone, and 64 rows pass them in half the time: that form below 720 workgroups of 128.  Where a window or a context of
-    // more than 1.5 times the new tokens leaves every workgroup about as many keys, below 900.  Beyond that 128 rows take the caches half as often, at a higher clock.
+    // head_dim 128 has three forms.  Workgroups of 128 rows share keys in LDS; in those of 64 rows each wave reads keys of its own (attention_keys.hip), or they share them, too.  A
+    // workgroup passes the longest keys of a prompt alone, and 64 rows pass them in half the time: they are taken below 720 workgroups of 128 (640 with fewer than eight kv
+    // heads, whose keys are in several L2).  Where a context of more than 1.5 times the new tokens leaves every workgroup about as many keys, below 900, and where a
+    // window does, below 360: its few keys do not outweigh what 64 rows do once a workgroup.  Beyond that 128 rows take the caches half as often, at a higher clock.
     // µs, row-split or KV-split form / 64 rows / 128 rows (workgroups of 128 rows × kv heads)
     //   8B heads (32 on 8)    1 × 8100 (2024)      2372 / 654 / 578      1 × 2800 (700)          - / 96 / 114    1 × 2048 (512)          196 / 59 / 65
     //                         1 × 3200 (800)           - / 119 / 113     1 × 1200 (300)          - / 28 / 50     [1600, 1600] (800)        - / 73 / 66
     //                         2400 at 5800 (600)       - / 340 / 382     3200 at 7400 (800)      - / 588 / 588   4000 at 9000 (1000)       - / 840 / 777
     //                         500 at 1000 (128)       57 / 24 / -        256 at 6000 (64)      146 / 60 / -      64 at 6000 (16)          54 / 56 / -
+    //     windows 256 | 1024  1 × 1360 (340)         - / 24 | 36 / 24 | 47       1 × 1920 (480)   - / 29 | 46 / 25 | 45      1 × 3000 (750)   - / 45 | 74 / 39 | 78
     //   16 on 8               1500 and 548 (256)      82 / 28 / 61       293, 1389, 366 (256)   87 / 34 / 56     1 × 986 at 366 (123)     49 / 22 / 51
+    //   32 on 4               1 × 2800 (700)           - / 93 / 86
+    // The waves' sums cost a workgroup 1 µs at its end, which few keys do not pay for: up to 256, and up to 512 where workgroups are more than the two a CU that run at once, they are
+    // shared (720 where eight heads or more share a kv head, so that nearly all workgroups have the longest keys).  µs of 64 rows, shared / by wave (workgroups of 64 rows; 367
+    // batches, of which three are more than 3 % slower so than with keys shared):
+    //   64 on 8   1 × 250 (250)  11.7 / 11.9     2 × 300 (600)  17.2 / 19.8     1 × 560 (560)  18.9 / 21.7     1 × 800 (800)  29.3 / 28.9
+    //   32 on 8   4 × 110 (220)  10.4 / 10.8     1 × 400 (200)  13.5 / 13.2     3 × 400 (600)  19.6 / 20.7     1 × 1200, window 128  20.2 / 21.6     … at 600  22.9 / 21.5
+    // Of 990 prompts between 60 and 8000 tokens, eight kinds of heads, with and without windows and contexts, the choice takes 0.90 of the time that 64 rows of shared keys and
+    // 128 rows took alone; 10 are more than 4 % slower, the most by 10 % (1200 tokens of 32 heads on 8 with a window of 768, little more than a round of workgroups).
     // A batch qualifies where most of its sequences bring many rows, or they bring 256 on average.
-    const long rows_heads = (long)total_q_tokens * G * num_kv_heads;
-    const bool two_sizes = head_dim == 128 && !kn.attn_flash32, even = (sliding_window > 0 && max_kv_len > sliding_window) || (long)max_kv_len * 2 >= (long)max_q_len * 5;
-    const bool half_units = two_sizes && (kn.attn_flash_rows ? kn.attn_flash_rows == 64 : rows_heads < (even ? 900 : 720) * 128);
+    const long rows_heads = (long)total_q_tokens * G * num_kv_heads, wgs64 = rows_heads / 64;
+    const bool windowed = sliding_window > 0 && max_kv_len > sliding_window, even = windowed || (long)max_kv_len * 2 >= (long)max_q_len * 5;
+    const bool two_sizes = head_dim == 128 && !kn.attn_flash32;
+    const int keys_seen = windowed ? sliding_window : max_kv_len;
+    const long half_below = windowed ? 360 : even ? 900 : num_kv_heads >= 8 ? 720 : 640;
+    const bool half_units = two_sizes && (kn.attn_flash_rows ? kn.attn_flash_rows == 64 : rows_heads < half_below * 128);
+    const bool few_keys = max_kv_len <= 256 || (wgs64 > 512 && max_kv_len <= (G >= 8 && wgs64 <= 720 ? 720 : 512)) || (windowed && sliding_window <= 128 && max_kv_len < 2 * max_q_len);
+    const bool shared = kn.attn_key_waves ? kn.attn_key_waves == 1 : !kn.attn_flash_rows && wgs64 >= 192 && few_keys;
+    // Below 192 workgroups only with keys enough, alike for all: the KV-split form has more workgroups, and with few kv heads more of them on a key's L2.  µs, that form / 64 rows (32 on 8):
+    //   132 at 396  12.1 / 13.6     132 at 924  22.7 / 17.3     200 at 300  13.0 / 13.3     200 at 600  19.3 / 15.7     280 at 420  22.8 / 15.7
+    //   (14 on 2)   301 at 903  18.9 / 19.4     457 at 1371  26.0 / 24.2     (32 on 4)   200 at 600  15.5 / 15.8     280 at 840  28.2 / 18.3
+    const bool keys_enough = even && wgs64 >= 64 && wgs64 * keys_seen >= (num_kv_heads >= 8 ? 60000 : 96000);
     const bool flash_fits = (long)total_q_tokens * 2 >= (long)num_seqs * max_q_len || (two_sizes && (long)total_q_tokens * G >= (long)num_seqs * 256);
-    if (!fq && cu_seqlens_q && !flash_off && (long)max_q_len * G >= flash_min_rows && flash_fits &&
-        rows_heads / (half_units || head_dim == 256 ? 64 : 128) >= (half_units && !kn.attn_flash_min_rows_set ? (even ? 64 : 192) : flash_min_wgs)) {
+    const bool covers = half_units && !kn.attn_flash_min_rows_set ? wgs64 >= 192 || keys_enough : rows_heads / (half_units || head_dim == 256 ? 64 : 128) >= flash_min_wgs;
+    if (!fq && cu_seqlens_q && !flash_off && (long)max_q_len * G >= flash_min_rows && flash_fits && covers) {
         const int mt = half_units || head_dim == 256 ? 1 : 2, unit_tiles = 4 * mt;
         const long tiles_bound = ((long)total_q_tokens * G) / 16 + num_seqs;
         const long units = cdiv(tiles_bound, (long)unit_tiles) + num_seqs;
@@ -1201,20 +1220,26 @@ static int paged_attention_launch(const __half* q, const __half* k_pool, const _
         if (two_sizes) {
             a.units = (int)units;
             const dim3 flat((unsigned)(num_kv_heads < 8 && 8 % num_kv_heads == 0 ? 8 * cdiv(units, 8 / num_kv_heads) : units * num_kv_heads));
-            if (mt == 1) {
+            if (mt == 1 && !shared) {
                 // Eight waves where no workgroup shares its CU with another and the keys are many enough to pay for the larger merge
                 // (256 at 6000: 67 → 58 µs, 986 at 366 25 → 22; three of 170 at 300, 264 workgroups, 16 → 24; 256 at 0 11 → 12)
                 const long wgs = ((long)total_q_tokens * G + 63L * num_seqs) / 64 * num_kv_heads;
-                const bool eight = kn.attn_key_waves ? kn.attn_key_waves == 8 : wgs <= 256 && max_kv_len >= 512;
+                const bool eight = kn.attn_key_waves ? kn.attn_key_waves == 8 : wgs <= 256 && keys_seen >= 512;
                 if (int rc = paged_prefill_attn_keys(a, eight, flat, s)) return rc;
             } else {                                         // 64 keys per step: two pairs per stage
                 const size_t lds64 = 2 * lds;
                 static bool attr64 = false;
                 if (!attr64) {
-                    FH_CHECK_HIP(hipFuncSetAttribute((const void*)paged_prefill_attn64_kernel<128>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64));
+                    FH_CHECK_HIP(hipFuncSetAttribute((const void*)paged_prefill_attn64_kernel<128, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64));
+                    FH_CHECK_HIP(hipFuncSetAttribute((const void*)paged_prefill_attn64_kernel<128, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds64));
                     attr64 = true;
                 }
-                hipLaunchKernelGGL((paged_prefill_attn64_kernel<128>), flat, dim3(256), lds64, s, a);
+                if (mt == 1) {
+                    form_hit(FORM_ATTN_FLASH_64);
+                    hipLaunchKernelGGL((paged_prefill_attn64_kernel<128, 1>), flat, dim3(256), lds64, s, a);
+                } else {
+                    hipLaunchKernelGGL((paged_prefill_attn64_kernel<128, 2>), flat, dim3(256), lds64, s, a);
+                }
             }
         } else if (head_dim == 128) FH_FLASH(128, 2) else if (head_dim == 64) FH_FLASH(64, 2) else FH_FLASH(256, 1)
 #undef FH_FLASH

@@ -27,7 +27,7 @@ struct Knobs {
     int attn_flash_rows = 0;          // 64 / 128: forced rows per workgroup of prompt attention (64: each wave on keys of its own)
     bool no_grouped_step = false;     // layered grouped attention: norms, rotation and cache write of steps in a launch of their own
     bool no_stream_route = false;     // layered experts: update, router and sorted list in launches of their own
-    int attn_key_waves = 0;           // 4 / 8: forced waves per workgroup of the 64-row form
+    int attn_key_waves = 0;           // 4 / 8: forced waves per workgroup of the 64-row form; 1: workgroups of 64 rows share keys in LDS
     bool attn_flash32 = false;        // the flash form with 32-key steps (paged_prefill_attn_kernel) for head_dim 128 too
     int qkv_min_tiles = 256;           // unquantised q|k|v of a prompt with norm, rotation and cache write in its launch from this many tiles of 128 × 128
     int rope_quad_rows = 8192;        // split q|k|v, norm, rotation, cache write: four tokens of a head a wave from this many rows of a head
@@ -179,6 +179,7 @@ enum Form : int {
     FORM_MOE_ROWS_256,          // layered experts: sorted rows in blocks of 256
     FORM_DONE_AGAIN,            // a call whose in-launch waits gave up was done again in separate launches
     FORM_IDS_LATE,              // a decode call whose ids did not come while they were watched for: the stream's end was waited for
+    FORM_ATTN_FLASH_64,         // prompt attention, workgroups of 64 rows share keys in LDS
     FORM_ATTN_KEYS,             // prompt attention, each wave of a 64-row workgroup on keys of its own: four waves
     FORM_ATTN_KEYS_WIDE,        // … eight
     FORM_F16_QKV,               // unquantised q|k|v of a prompt, normed, rotated and stored by its launch

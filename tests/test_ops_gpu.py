@@ -1051,6 +1051,38 @@ def test_paged_prefill_attention_in_both_unit_sizes(env, window, nq, nkv, rows, 
     test_paged_prefill_attention_lds_shared_kv(env, window, nq, nkv, 128, knobs, forms)
 
 
+KEYS, WIDE, SHARED, BROAD, OTHER = "attn_keys", "attn_keys_wide", "attn_flash_64", "attn_flash", "attn_kv_narrow"
+
+
+@pytest.mark.parametrize("q_lens,pos,window,nq,nkv,form", [
+    ([250], 0, 0, 64, 8, SHARED), ([300], 0, 0, 64, 8, KEYS), ([300, 260], 0, 0, 64, 8, SHARED), ([700], 0, 0, 64, 8, SHARED), ([740], 0, 0, 64, 8, KEYS), ([500] * 3, 0, 0, 32, 8, SHARED),
+    ([513] * 3, 0, 0, 32, 8, KEYS), ([400], 0, 100, 32, 4, SHARED), ([400], 500, 100, 32, 4, KEYS), ([400], 0, 129, 32, 4, KEYS), ([132], 396, 0, 32, 8, OTHER), ([132], 924, 0, 32, 8, WIDE),
+    ([264], 800, 0, 16, 2, OTHER), ([500], 800, 0, 16, 2, WIDE), ([1439], 0, 256, 32, 8, KEYS), ([1440], 0, 256, 32, 8, BROAD), ([719], 0, 0, 128, 8, KEYS), ([720], 0, 0, 128, 8, BROAD),
+    ([1279], 0, 0, 64, 4, KEYS), ([1280], 0, 0, 64, 4, BROAD)])
+def test_form_of_a_prompt_by_its_workgroups_and_keys(env, q_lens, pos, window, nq, nkv, form, forms):
+    """Which form a prompt takes on either side of each line; up to 600 tokens its results, too, against float32 (bound: see the test below)."""
+    pkg, B, ctx, O, torch = env
+    S, total, kv = len(q_lens), sum(q_lens), [pos + t for t in q_lens]
+    mb = (max(kv) + 15) // 16
+    gen = torch.Generator("cuda").manual_seed(total)
+    rand = lambda *n: torch.randn(*n, generator=gen, device="cuda").half()
+    K, V, q = [rand(n, nkv, 128) for n in kv], [rand(n, nkv, 128) for n in kv], rand(total, nq, 128)
+    tables = torch.randperm(S * mb, generator=gen, device="cuda").to(torch.int32).reshape(S, mb)
+    ck, cv = _fill_pool(env, [host(x) for x in K], [host(x) for x in V], tables.cpu().numpy(), kv, nkv, 128, S * mb)
+    cu = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+    out = torch.full((total + 1, nq, 128), 9.0, dtype=torch.float16, device="cuda")
+    forms.reset()
+    B.paged_varlen_attention(ctx, q, ck, cv, out, torch.from_numpy(cu).cuda(), torch.full((S,), pos, dtype=torch.int32, device="cuda"), tables, S, total, max(kv), nq, nkv, 128,
+                             window, 16, mb, max(q_lens))
+    ctx.sync()
+    h = forms.hits()
+    assert h.get(form) and not any(h.get(f) for f in (KEYS, WIDE, SHARED, OTHER) if f != form), h
+    assert bool((out[total] == 9.0).all()) and bool(torch.isfinite(out).all())
+    for s in range(S if total <= 600 else 0):
+        ref = _ref_attention(O, host(q[cu[s]:cu[s + 1]]), host(K[s]), host(V[s]), pos, nq, nkv, 128, window)
+        assert nmse(ref, host(out[cu[s]:cu[s + 1]])) < 4 * 2.0 ** -22, s
+
+
 @pytest.mark.parametrize("waves", [4, 8])
 @pytest.mark.parametrize("q_lens,pos,window,nq,nkv", [
     ([9], [0], 0, 8, 8), ([64], [0], 0, 1, 1), ([65, 31], [0, 97], 0, 2, 2), ([16, 17], [15, 16], 0, 8, 2), ([128, 9], [129, 1000], 0, 14, 2),
